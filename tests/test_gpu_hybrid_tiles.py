@@ -1,0 +1,64 @@
+"""Products of more than 16 rows on the hybrid engine's bf16 path: every tile form at its edges.
+
+The tile forms add an output's products in the same order, so the logits of a row have to be the same bits whichever form the number of
+rows and columns picks; the smallest form is held to the float64 restatement by the design's own tests.  Gate and up products with their
+activation behind them, dense and routed, are held to the restatement at sizes that pick each form."""
+import pytest
+import torch
+
+from oracle import kazozen_ref as KR
+from tests import hybrid_util as U
+from tests import kazozen_util as P
+from vox_serve_amd.engine_hybrid import HybridEngine
+from vox_serve_amd.model import kazozen
+
+pytestmark = pytest.mark.gpu
+
+BF16_BAR = 4e-2     # relative RMS over the vocabulary, as in the design's tests
+
+
+@pytest.fixture(scope="module", autouse=True)
+def _gpu():
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+
+
+# (rows, vocabulary): 128 x 128 on four waves (with remainders of 2 rows and 1 column), on eight waves, 64 x 64 with two stages, and one k-tile
+@pytest.mark.parametrize("rows,vocab,width", [(130, 16769, 128), (255, 14400, 192), (65, 19201, 128), (129, 28673, 64)])
+def test_a_row_has_the_same_logits_in_every_tile_form(rows, vocab, width):
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2)], width=width, vocab=vocab, bigram=None)
+    d = kazozen.config_from_dict(cfg)
+    eng = HybridEngine(d, kazozen.pack_weights(P.random_checkpoint(cfg, seed=rows), d), dtype=torch.bfloat16, max_batch=1, page_size=16, max_pages=20,
+                       max_seq_len=320, max_prefill_rows=rows, max_out=rows)
+    toks = torch.randint(0, vocab, (rows,), generator=torch.Generator().manual_seed(7), dtype=torch.int32)
+    eng.row_ids[:rows, 0] = toks.cuda()
+
+    def logits(out):
+        npg = (rows + 15) // 16
+        eng.upload_plan(pos=range(rows), kvlen=range(1, rows + 1), page=[t // 16 for t in range(rows)], slot=[t % 16 for t in range(rows)], q_req=[0] * rows,
+                        last_rows=out, indptr=[0, npg], indices=range(npg), req_rows=[0, rows], state=[0])
+        eng.step(rows, 1, len(out), sample=False, max_kvlen=rows)
+        return eng.out_logits[: len(out)].clone()
+    try:
+        whole = logits(list(range(rows)))
+        for a in range(0, rows, 17):
+            part = list(range(min(a, rows - 17), min(a, rows - 17) + 17))      # 17 rows: tiles of 64
+            assert torch.equal(logits(part), whole[part]), (rows, vocab, a)
+    finally:
+        eng.close()
+
+
+@pytest.mark.parametrize("rows,mlp", [(130, P.dense(8384)), (129, P.dense(7424)), (65, P.dense(9600)), (17, P.dense(64)), (70, P.moe(4, 4, 3840, 0, 0)),
+                                      (131, P.moe(4, 4, 2176, 2, 2)), (67, P.moe(6, 2, 2560, 3, 2)), (33, P.moe(3, 1, 64, 0, 0))])
+def test_activation_behind_both_products(rows, mlp):
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=mlp)], width=64, vocab=50)
+    S = P.random_checkpoint(cfg, seed=3)
+    toks = torch.randint(0, 50, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
+    d = U.Driver(cfg, S, dtype=torch.bfloat16, page_size=16, pages=20, max_rows=rows)
+    try:
+        got = d.run_cut("r", toks, [rows])
+    finally:
+        d.close()
+    # (a routed layer: a choice that bf16 rounding flips moves a whole row, so the bar holds for nine rows of ten)
+    err = U.rel_err(got, KR.forward(cfg, S, toks), None if mlp["kind"] == "dense" else 0.9)
+    assert err < BF16_BAR, err

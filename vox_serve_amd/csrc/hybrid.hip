@@ -186,8 +186,9 @@ struct hb_rowmap {
     float epi_arg;
     const float* col_scale;     // HB_EPI_RESID_SCALED: [N] fp32
     hb_join join;               // HB_EPI_JOIN
+    const bf16_t* a16;          // the rows of A as bf16, lda apart (A itself is not read), or NULL
 };
-static inline hb_rowmap hb_plain() { return hb_rowmap{nullptr, nullptr, 0, 1, 0, 0, 0, 0, nullptr, 0.f, nullptr, {}}; }
+static inline hb_rowmap hb_plain() { return hb_rowmap{nullptr, nullptr, 0, 1, 0, 0, 0, 0, nullptr, 0.f, nullptr, {}, nullptr}; }
 template <int EPI> __device__ __forceinline__ float hb_epi_arg(const hb_rowmap& rm, int col) {
     if (EPI == HB_EPI_RELU2) return col < (int)rm.epi_arg ? 1.0f : 0.0f;
     return EPI == HB_EPI_RESID_SCALED ? rm.col_scale[col] : rm.epi_arg;
@@ -490,6 +491,7 @@ __global__ __launch_bounds__(256) void k_hb_rms_row(const float* x, long ldx, co
 // ---- GEMM  C[M,N] (+)= A[M,K] . W[N,K]^T + bias ---------------------------------------------------------------------------
 // bf16: both operands staged in LDS as bf16 (activations rounded once), v_mfma_f32_16x16x32_bf16; four waves, 64 output columns
 // per block, BM = 64 (2 x 2 tiles per wave) or BM = 16 (one tile per wave).  Every edge (M, N, K) is guarded at the LDS fill.
+// More than 16 rows take k_hb_gemm_dma below; this form is for odd K, unaligned operands, strided batches and scaled rows.
 template <int BM, int EPI>
 __global__ __launch_bounds__(256) void k_hb_gemm_bf16(const float* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
                                                       int N, int K, hb_rowmap rm) {
@@ -619,6 +621,137 @@ __global__ __launch_bounds__(256) void k_hb_gemm_bf16(const float* A, long lda, 
                 if (gm < M) hb_finish<EPI>(rm, C, ldc, lst ? lst[gm] : gm, gn, acc[i][j][r], b);
             }
         }
+}
+
+// More than 16 rows, both operands bf16 in memory, K a multiple of 64: BM x BN outputs per block, WM x WN waves.  k-tiles of 64 go from memory
+// straight into LDS (global_load_lds, 1 KB per wave instruction = eight 128-byte rows) and S stages of them are kept in flight: a tile's
+// requests are S - 1 tiles old when it is multiplied, and no register holds them.  One wait + barrier per k-tile: it says that every wave's
+// part of tile t has landed and that nobody reads the stage of tile t - 1 any more, which is then requested anew.  The 16-byte pieces of a
+// row lie at piece ^ (row & 7) (the swizzle is in the address each lane reads), so the fragment reads of 16 rows do not meet in a bank.
+// Per output the products are added as in k_hb_gemm_bf16 (k ascending in steps of 32): the same bits.
+// The blocks of one XCD (block id modulo 8) take neighbouring tiles, 512 rows deep, so that its L2 holds what they share.
+// Bound by the L2 -> LDS path (one k-tile of 128 x 128 moves 32 KB for 515 matrix clocks) and, for wide outputs, by their stores.
+// Measured against k_hb_gemm_bf16<64> (2048 rows; us): 2048 x 2048 64.7 -> 25.1, 2048 x 5632 (N x K) 160 -> 51, 11264 x 2048 305 -> 118;
+// 200 rows: 2048 x 2048 31.4 -> 11.6; 64 rows: 31.0 -> 11.2.  Staged through registers instead the same tiles took 34.7 / 74.6 / 151.
+// GLU: the block's columns are BN / 2 gate rows and the BN / 2 up rows beside them, interleaved so that a lane owns both; what is stored is
+// hb_glu of the two, rounded to bf16 as the product behind it reads it (C: bf16 [.][ff], N = ff): neither product is written to memory.
+struct hb_glu_args {
+    float limit, alpha, up_offset;
+    int gelu;
+};
+// (m0 holds the LDS address of the instruction; nothing else in this kernel uses it)
+__device__ __forceinline__ void hb_dma16(const void* base, unsigned off, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
+}
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool GLU, bool LIST>
+__global__ __launch_bounds__(WM * WN * 64) void k_hb_gemm_dma(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
+                                                              int N, int K, hb_rowmap rm, hb_glu_args glu) {
+    constexpr int BK = 64, NWV = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16, CN = GLU ? BN / 2 : BN, NA = BM / 8 / NWV, NW = BN / 8 / NWV;
+    constexpr int STAGE = (BM + BN) * BK, U = NT * 8;       // U: gate (up) columns of a wave
+    static_assert(BM % (8 * NWV) == 0 && BN % (8 * NWV) == 0 && (!GLU || NT % 2 == 0), "whole wave instructions");
+    extern __shared__ __attribute__((aligned(1024))) bf16_t smem[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int* lst = nullptr;
+    Wt += (size_t)blockIdx.y * rm.w_stride;
+    if (bias) bias += (size_t)blockIdx.y * rm.b_stride;
+    if (LIST) {
+        M = rm.count[blockIdx.y];
+        lst = rm.list + (size_t)blockIdx.y * rm.cap;
+    }
+    const int tm = (M + BM - 1) / BM, tn = (N + CN - 1) / CN, total = tm * tn, per = (total + 7) >> 3;
+    const int in_xcd = (int)blockIdx.x >> 3, t = ((int)blockIdx.x & 7) * per + in_xcd;
+    if (in_xcd >= per || t >= total) return;
+    constexpr int GM = 512 / BM;
+    const int g0 = t / (GM * tn) * GM, gh = tm - g0 < GM ? tm - g0 : GM, tg = t - g0 * tn;
+    const int m0 = (g0 + tg % gh) * BM, n0 = tg / gh * CN;
+    const int wm = wv / WN, wn = wv % WN, fr = lane & 15, fk = lane >> 4;
+    // byte offsets of this lane's 16 bytes of each of its rows (rows past the end repeat the last one: nothing of them is stored)
+    const unsigned pc = ((lane & 7) ^ (lane >> 3)) * 16;
+    unsigned ao[NA], wo[NW];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        int gm = m0 + (wv + i * NWV) * 8 + (lane >> 3);
+        gm = gm < M ? gm : M - 1;
+        if (LIST) gm = lst[gm] / rm.a_div;
+        ao[i] = (unsigned)gm * (unsigned)(lda * 2) + pc;
+    }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int r = (wv + i * NWV) * 8 + (lane >> 3);
+        int gn = GLU ? n0 + r / (2 * U) * U + r % U : n0 + r;
+        gn = gn < N ? gn : N - 1;
+        if (GLU && r % (2 * U) >= U) gn += N;
+        wo[i] = (unsigned)gn * (unsigned)(K * 2) + pc;
+    }
+    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)smem + wv * 1024;
+    auto request = [&](int stage, int k0) {
+        const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * (STAGE * 2));
+#pragma unroll
+        for (int i = 0; i < NA; ++i) hb_dma16(A, ao[i] + k0 * 2, ls + i * NWV * 1024);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) hb_dma16(Wt, wo[i] + k0 * 2, ls + BM * 128 + i * NWV * 1024);
+    };
+    hb_f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+    const int nt = K / BK, klast = K - BK;
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) request(s, s * BK < klast ? s * BK : klast);
+    int stage = 0;
+    for (int kt = 0; kt < nt; ++kt) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
+        const int kn = (kt + S - 1) * BK;
+        request(stage == 0 ? S - 1 : stage - 1, kn < klast ? kn : klast);
+        const bf16_t *as = smem + stage * STAGE + (wm * MT * 16 + fr) * BK, *ws = smem + stage * STAGE + BM * BK + (wn * NT * 16 + fr) * BK;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks) {
+            const int piece = ((ks * 4 + fk) ^ (fr & 7)) << 3;
+            hb_bf16x8 af[MT], wf[NT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) af[i] = *(const hb_bf16x8*)(as + i * 16 * BK + piece);
+#pragma unroll
+            for (int j = 0; j < NT; ++j) wf[j] = *(const hb_bf16x8*)(ws + j * 16 * BK + piece);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], wf[j], acc[i][j], 0, 0, 0);
+        }
+        stage = stage == S - 1 ? 0 : stage + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (the repeated last tiles: nothing may land after the block has ended)
+    if constexpr (GLU) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT / 2; ++j) {
+                const int gn = n0 + wn * U + j * 16 + fr;
+                if (gn >= N) continue;
+                const float bg = bias ? bias[gn] : 0.f, bu = bias ? bias[N + gn] : 0.f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int gm = m0 + (wm * MT + i) * 16 + fk * 4 + r;
+                    if (gm < M)
+                        ((bf16_t*)C)[(size_t)(LIST ? lst[gm] : gm) * ldc + gn] =
+                            f2bf(hb_glu(acc[i][j][r] + bg, acc[i][j + NT / 2][r] + bu, glu.limit, glu.alpha, glu.up_offset, glu.gelu));
+                }
+            }
+    } else {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int gn = n0 + (wn * NT + j) * 16 + fr;
+                if (gn >= N) continue;
+                const float b = bias ? bias[gn] : 0.f;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int gm = m0 + (wm * MT + i) * 16 + fk * 4 + r;
+                    if (gm < M) hb_finish<EPI>(rm, C, ldc, LIST ? lst[gm] : gm, gn, acc[i][j][r], b);
+                }
+            }
+    }
 }
 
 // fp32: LDS-tiled FMA, 64 output columns per block, BM = 64 (4 x 4 per thread) or 16 (1 x 4 per thread); k ascending per element.
@@ -1081,24 +1214,98 @@ bool hb_try_rows16(hipStream_t st, const float* A, long lda, const bf16_t* W, co
 template <int EPI>
 bool hb_try_rows16(hipStream_t, const float*, long, const float*, const float*, float*, long, int, int, int, const hb_rowmap&, int) { return false; }
 
-// rm.count != NULL: `groups` gathered GEMMs of at most M rows each in one launch (see hb_rowmap)
+static inline int hb_tile_count(int M, int N, int bm, int bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); }
+// room for the rows of a product rounded to bf16
+struct hb_ws16 {
+    bf16_t* p;
+    size_t n;
+};
+__global__ __launch_bounds__(256) void k_hb_to_bf16(const float* A, long lda, bf16_t* out, int K8, size_t n8) {
+    for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (size_t)gridDim.x * 256) {
+        const size_t row = i / K8, c = (i - row * K8) * 8;
+        const float4 a = *(const float4*)(A + row * lda + c), b = *(const float4*)(A + row * lda + c + 4);
+        *(uint4*)(out + i * 8) = make_uint4(pack_bf2(a.x, a.y), pack_bf2(a.z, a.w), pack_bf2(b.x, b.y), pack_bf2(b.z, b.w));
+    }
+}
+// what k_hb_gemm_dma reads in whole 16-byte pieces and addresses in 32 bits
+static inline bool hb_dma_ok(const bf16_t* W, size_t a_rows, size_t N, int K, const hb_rowmap& rm) {
+    return K > 0 && K % 64 == 0 && ((size_t)W & 15) == 0 && (rm.w_stride & 7) == 0 && a_rows * K < (1ull << 31) && N * K < (1ull << 31);
+}
+// Tiles by how many blocks they leave for 256 compute units (`rows`: rows of a product as far as the host knows; a gathered one has fewer
+// than M).  2048 rows, N x K = 2560 x 2048: 128 x 128 / four waves, two blocks per CU 38.1 us, eight waves, four stages, one block 44.8; at
+// exactly one tile per CU (2048 x 2048) 32.3 and 25.1.  Below 224 tiles of 128: 64 x 64 (1024 rows, 2048 x 2048: 17.1 against 24.0), with
+// four stages while there are at most two blocks per CU (512 rows, 2048 x 5632: 25.6 against 42.0 with two stages; 200 rows, 11264 x 2048,
+// 704 tiles: 27.0 against 20.6).
+template <int EPI, bool GLU, bool LIST>
+void hb_launch_dma(hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
+                   const hb_rowmap& rm, int groups, int rows, hb_glu_args glu = hb_glu_args{}) {
+    constexpr int G = GLU ? 2 : 1;
+    const int t128 = hb_tile_count(rows, N, 128, 128 / G) * groups, t64 = hb_tile_count(rows, N, 64, 64 / G) * groups;
+#define HB_DMA(BM_, BN_, WM_, WN_, S_) \
+    do { \
+        constexpr int lds = S_ * (BM_ + BN_) * 128; \
+        const auto kern = k_hb_gemm_dma<BM_, BN_, WM_, WN_, S_, EPI, GLU, LIST>; \
+        if (lds > 64 * 1024) (void)hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds); \
+        hipLaunchKernelGGL(kern, dim3((hb_tile_count(M, N, BM_, BN_ / G) + 7) & ~7, groups), dim3(WM_ * WN_ * 64), lds, st, A, lda, W, bias, C, ldc, M, N, K, \
+                           rm, glu); \
+    } while (0)
+    if (t128 > 256) HB_DMA(128, 128, 2, 2, 2);
+    else if (t128 >= 224) HB_DMA(128, 128, 4, 2, 4);
+    else if (t64 <= 512) HB_DMA(64, 64, 2, 2, 4);
+    else HB_DMA(64, 64, 2, 2, 2);
+#undef HB_DMA
+}
+// the rows of A as bf16: rm.a16 when the kernel before has left them so, else rounded into the workspace (NULL: neither is possible)
+static const bf16_t* hb_rows16(hipStream_t st, hb_ws16 ws, const hb_rowmap& rm, const float* A, long& lda, int a_rows, int K) {
+    if (rm.a16) return rm.a16;
+    if (rm.a_scale || (lda & 3) || ((size_t)A & 15) || (size_t)a_rows * K > ws.n) return nullptr;
+    const size_t n8 = (size_t)a_rows * (K / 8), blocks = (n8 + 255) / 256;
+    hipLaunchKernelGGL(k_hb_to_bf16, dim3((unsigned)(blocks < 2048 ? blocks : 2048)), dim3(256), 0, st, A, lda, ws.p, K / 8, n8);
+    lda = K;
+    return ws.p;
+}
+// rm.count != NULL: `groups` gathered GEMMs of at most M rows each (about `rows`) in one launch (see hb_rowmap), their rows among the first
+// a_rows of A
 template <int EPI>
-int hb_gemm_tiles(hipStream_t st, const float* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
-                  hb_rowmap rm = hb_plain(), int groups = 1) {
+int hb_gemm_tiles(hb_ws16 ws, hipStream_t st, const float* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
+                  const hb_rowmap& rm, int groups = 1, int rows = 0, int a_rows = 0) {
+    if (!a_rows) a_rows = M;
+    if (!rows) rows = M;
+    if (M > 16 && (groups == 1 || (rm.count && EPI == HB_EPI_STORE)) && hb_dma_ok(W, a_rows, N, K, rm)) {
+        long ld16 = lda;
+        if (const bf16_t* a16 = hb_rows16(st, ws, rm, A, ld16, a_rows, K)) {
+            if (!rm.count) hb_launch_dma<EPI, false, false>(st, a16, ld16, W, bias, C, ldc, M, N, K, rm, 1, rows);
+            else if constexpr (EPI == HB_EPI_STORE) hb_launch_dma<EPI, false, true>(st, a16, ld16, W, bias, C, ldc, M, N, K, rm, groups, rows);
+            return VOX_OK;
+        }
+    }
     if (M <= 16) hipLaunchKernelGGL((k_hb_gemm_bf16<16, EPI>), dim3((N + 63) / 64, 1, groups), dim3(256), 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
     else hipLaunchKernelGGL((k_hb_gemm_bf16<64, EPI>), dim3((N + 63) / 64, (M + 63) / 64, groups), dim3(256), 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
     return VOX_OK;
 }
 template <int EPI>
-int hb_gemm_tiles(hipStream_t st, const float* A, long lda, const float* W, const float* bias, float* C, long ldc, int M, int N, int K,
-                  hb_rowmap rm = hb_plain(), int groups = 1) {
+int hb_gemm_tiles(hb_ws16, hipStream_t st, const float* A, long lda, const float* W, const float* bias, float* C, long ldc, int M, int N, int K,
+                  const hb_rowmap& rm, int groups = 1, int = 0, int = 0) {
     if (M <= 16) hipLaunchKernelGGL((k_hb_gemm_f32<16, EPI>), dim3((N + 63) / 64, 1, groups), dim3(256), 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
     else hipLaunchKernelGGL((k_hb_gemm_f32<64, EPI>), dim3((N + 63) / 64, (M + 63) / 64, groups), dim3(256), 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
     return VOX_OK;
 }
+// Gate and up products with their activation behind them in one launch: y[.][ff] bf16 = hb_glu(A . Wg^T + b, A . Wu^T + b), Wg = the first ff rows
+// of W, Wu = the next.  false: these operands do not allow it (the two steps are the caller's).  K_next: columns of the product that reads y.
+static bool hb_try_glu(hb_ws16 ws, hipStream_t st, const float* A, long lda, int a_rows, const bf16_t* W, const float* bias, void* y, int M, int ff, int K,
+                       const bf16_t* w_next, int n_next, const hb_rowmap& rm, int groups, int rows, size_t y_rows, hb_glu_args glu) {
+    if (M <= 16 || !hb_dma_ok(W, a_rows, 2 * (size_t)ff, K, rm) || !hb_dma_ok(w_next, y_rows, n_next, ff, rm)) return false;
+    const bf16_t* a16 = hb_rows16(st, ws, rm, A, lda, a_rows, K);
+    if (!a16) return false;
+    if (rm.count) hb_launch_dma<HB_EPI_STORE, true, true>(st, a16, lda, W, bias, (float*)y, ff, M, ff, K, rm, groups, rows, glu);
+    else hb_launch_dma<HB_EPI_STORE, true, false>(st, a16, lda, W, bias, (float*)y, ff, M, ff, K, rm, 1, rows, glu);
+    return true;
+}
+static bool hb_try_glu(hb_ws16, hipStream_t, const float*, long, int, const float*, const float*, void*, int, int, int, const float*, int, const hb_rowmap&, int,
+                       int, size_t, hb_glu_args) { return false; }
 // nz > 1: a strided batch of nz products (rm gives the strides) in one launch
 template <typename T, int EPI>
-int hb_gemm_epi(hipStream_t st, const float* A, long lda, const T* W, const float* bias, float* C, long ldc, int M, int N, int K,
+int hb_gemm_epi(hb_ws16 ws, hipStream_t st, const float* A, long lda, const T* W, const float* bias, float* C, long ldc, int M, int N, int K,
                 const hb_rowmap& rm, int nz) {
     if (M <= 0 || N <= 0) return VOX_OK;
     // four columns per wave once that still leaves a block for every compute unit several times over
@@ -1115,21 +1322,21 @@ int hb_gemm_epi(hipStream_t st, const float* A, long lda, const T* W, const floa
     else if (M <= 4) HB_GEMV(4);
     else if (M <= 8) HB_GEMV(8);
 #undef HB_GEMV
-    else return hb_gemm_tiles<EPI>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    else return hb_gemm_tiles<EPI>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
     return VOX_OK;
 }
 template <typename T>
-int hb_gemm(hipStream_t st, int epi, const float* A, long lda, const T* W, const float* bias, float* C, long ldc, int M, int N, int K,
+int hb_gemm(hb_ws16 ws, hipStream_t st, int epi, const float* A, long lda, const T* W, const float* bias, float* C, long ldc, int M, int N, int K,
             const hb_rowmap& rm = hb_plain(), int nz = 1) {
-    if (epi == HB_EPI_GELU) return hb_gemm_epi<T, HB_EPI_GELU>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_RESID) return hb_gemm_epi<T, HB_EPI_RESID>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_TANH) return hb_gemm_epi<T, HB_EPI_TANH>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_SOFTCAP) return hb_gemm_epi<T, HB_EPI_SOFTCAP>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_RESID_SCALED) return hb_gemm_epi<T, HB_EPI_RESID_SCALED>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_SCALE) return hb_gemm_epi<T, HB_EPI_SCALE>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_RELU2) return hb_gemm_epi<T, HB_EPI_RELU2>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    if (epi == HB_EPI_JOIN) return hb_gemm_epi<T, HB_EPI_JOIN>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
-    return hb_gemm_epi<T, HB_EPI_STORE>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_GELU) return hb_gemm_epi<T, HB_EPI_GELU>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_RESID) return hb_gemm_epi<T, HB_EPI_RESID>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_TANH) return hb_gemm_epi<T, HB_EPI_TANH>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_SOFTCAP) return hb_gemm_epi<T, HB_EPI_SOFTCAP>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_RESID_SCALED) return hb_gemm_epi<T, HB_EPI_RESID_SCALED>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_SCALE) return hb_gemm_epi<T, HB_EPI_SCALE>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_RELU2) return hb_gemm_epi<T, HB_EPI_RELU2>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    if (epi == HB_EPI_JOIN) return hb_gemm_epi<T, HB_EPI_JOIN>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
+    return hb_gemm_epi<T, HB_EPI_STORE>(ws, st, A, lda, W, bias, C, ldc, M, N, K, rm, nz);
 }
 
 // ---- linear recurrences ------------------------------------------------------------------------------------------------------
@@ -4434,6 +4641,7 @@ struct vox_hybrid {
     float *moe_wgt = nullptr, *moe_act = nullptr, *moe_out = nullptr;
     int *moe_sel = nullptr, *moe_list = nullptr, *moe_count = nullptr;
     bf16_t* logits16 = nullptr;
+    hb_ws16 ws16{nullptr, 0};               // [max_rows][widest operand]: rows of a product rounded to bf16
     float* attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
     int max_in = 0, max_mix = 0, max_ff = 0;
@@ -4710,13 +4918,14 @@ static int hb_win_attention(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* 
 
 // cur joins (A . W^T + bias)
 template <typename T>
-static int hb_gemm_resid(hipStream_t st, const float* A, long lda, const T* W, const float* bias, float* cur, long ldx, int n, int N, int K,
-                         const hb_join& j) {
+static int hb_gemm_resid(hb_ws16 ws, hipStream_t st, const float* A, long lda, const T* W, const float* bias, float* cur, long ldx, int n, int N, int K,
+                         const hb_join& j, const bf16_t* a16 = nullptr) {
     hb_rowmap rm = hb_plain();
     rm.col_scale = j.scale;
     rm.join = j;
+    rm.a16 = a16;
     const int epi = j.store ? HB_EPI_STORE : j.gate || j.streams > 0 ? HB_EPI_JOIN : (j.scale ? HB_EPI_RESID_SCALED : HB_EPI_RESID);
-    return hb_gemm<T>(st, epi, A, lda, W, bias, cur, ldx, n, N, K, rm);
+    return hb_gemm<T>(ws, st, epi, A, lda, W, bias, cur, ldx, n, N, K, rm);
 }
 // One mixer: reads the rows hn (!= NULL, ldh apart: normed already, or read as they are) or norms src (rows lds apart) itself with L.norm1; out_scale * mixer(.) joins cur as `jn`
 // says; pd != NULL: the rows are pd->x, with whatever is pending on it (the layer's residual gate, when it has one, is added to it here: its logits are the last columns of the input projection).
@@ -4750,11 +4959,11 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
             hipLaunchKernelGGL(k_hb_shift_mix, dim3(n, n <= 64 ? (W + 255) / 256 : 1), dim3(256), 0, st, hn, (long)W, L.shift_mu, m->shift, rows_stride,
                                state, per_slot, (long)HD * L.dim, io->pos, io->row_req, io->req_rows, io->req_state, W);
             // r, k, v, g: four products of one shape, each on its own mix, in one launch
-            VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, m->shift, W, wi, L.b_in, m->proj, n_proj, n, HD, W,
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, m->shift, W, wi, L.b_in, m->proj, n_proj, n, HD, W,
                                hb_rowmap{nullptr, nullptr, 0, 1, (long)HD * W, rows_stride, (long)HD, (long)HD}, 4));
-            VOX_TRY(hb_gemm<T>(st, HB_EPI_TANH, m->shift + 4 * rows_stride, W, wi + (size_t)4 * HD * W, nullptr, m->proj + 4 * HD, n_proj, n, L.lora, W));
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_TANH, m->shift + 4 * rows_stride, W, wi + (size_t)4 * HD * W, nullptr, m->proj + 4 * HD, n_proj, n, L.lora, W));
         }
-        VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, m->proj + 4 * HD, n_proj, (const T*)L.w_decay2, L.decay0, m->proj + 4 * HD + L.lora, n_proj, n, HD, L.lora));
+        VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, m->proj + 4 * HD, n_proj, (const T*)L.w_decay2, L.decay0, m->proj + 4 * HD + L.lora, n_proj, n, HD, L.lora));
         const int dpw = L.dim <= 16 * HB_SCAN_MAX_WAVES ? 16 : (L.dim <= 32 * HB_SCAN_MAX_WAVES ? 32 : 64);
         const int nwv = (L.dim + dpw - 1) / dpw, dpad = nwv * dpw;
         const int tt = 4096 / dpad >= 16 ? 16 : (4096 / dpad >= 1 ? 4096 / dpad : 1);
@@ -4784,7 +4993,7 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
         if (!fused_norm)
             hipLaunchKernelGGL(k_hb_head_norm, dim3(n, L.heads), dim3(64), 0, st, m->mix, (long)n_mix, L.head_norm, 1, m->proj, (long)n_proj, 3 * HD,
                                (int)HB_GATE_SILU, L.vdim, c.eps, L.out_scale);
-        return hb_gemm_resid<T>(st, m->mix, n_mix, (const T*)L.w_out, nullptr, cur, ldx, n, W, n_mix, jn);
+        return hb_gemm_resid<T>(m->ws16, st, m->mix, n_mix, (const T*)L.w_out, nullptr, cur, ldx, n, W, n_mix, jn);
     }
     if (pd) {
         // (post-normed layer: the rows are the stream itself, a norm may still be pending on it)
@@ -4796,7 +5005,7 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
         hn = m->h;
         ldh = W;
     }
-    if (hn) VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, hn, ldh, (const T*)L.w_in, L.b_in, m->proj, n_proj, n, n_in, W));
+    if (hn) VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, hn, ldh, (const T*)L.w_in, L.b_in, m->proj, n_proj, n, n_in, W));
     const int vt = (L.vdim + 63) / 64;
     // dims per wave of the scans: the smallest of 16 / 32 / 64 that covers dim with at most 16 waves
     const int dpw = L.dim <= 16 * HB_SCAN_MAX_WAVES ? 16 : (L.dim <= 32 * HB_SCAN_MAX_WAVES ? 32 : 64);
@@ -4846,9 +5055,9 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
         const int H = L.heads, G = L.kv_heads, nv = H * L.vdim;
         const long per_slot = (long)H * L.dim * L.vdim + (long)(L.conv_taps - 1) * y.nqkv, hist_off = (long)H * L.dim * L.vdim;
         if (L.lora > 0)
-            VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, m->proj + y.off_din, n_proj, (const T*)L.w_decay2, nullptr, m->proj + y.off_dec, n_proj, n, y.ndec, L.lora));
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, m->proj + y.off_din, n_proj, (const T*)L.w_decay2, nullptr, m->proj + y.off_dec, n_proj, n, y.ndec, L.lora));
         if (L.gate_rank > 0)
-            VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, m->proj + y.off_gin, n_proj, (const T*)L.w_gate2, nullptr, m->proj + y.off_gate, n_proj, n, nv, L.gate_rank));
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, m->proj + y.off_gin, n_proj, (const T*)L.w_gate2, nullptr, m->proj + y.off_gate, n_proj, n, nv, L.gate_rank));
         hipLaunchKernelGGL(k_hb_delta_conv, dim3(n, (y.nqkv + y.ndec + H + 255) / 256), dim3(256), 0, st, m->proj, (long)n_proj, L.conv_w, state,
                            per_slot, hist_off, L.a_log, L.dt_bias, io->pos, io->row_req, io->req_rows, io->req_state, y, H, L.dim, L.conv_taps,
                            L.decay_channels);
@@ -4895,9 +5104,9 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
         hipLaunchKernelGGL((k_hb_latent_prep<T>), dim3(n, prep_y), dim3(256), 0, st, m->proj, (long)n_proj, (T*)cache, L.q_lat_norm, L.kv_lat_norm,
                            L.inv_freq, io->pos, io->page, io->slot, L.q_rank, y.off_kv, R, r, L.rot_dims, ps, c.eps, mag, H, L.dim, y.off_qa);
         if (L.q_rank > 0)
-            VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, m->proj, n_proj, (const T*)L.w_uq, nullptr, q, n_proj, n, H * dq, L.q_rank));
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, m->proj, n_proj, (const T*)L.w_uq, nullptr, q, n_proj, n, H * dq, L.q_rank));
         // every head's plain query part times its key expansion: the query against the cached latent
-        VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, q, n_proj, (const T*)L.w_ukT, nullptr, qa, n_proj, n, R, L.dim,
+        VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, q, n_proj, (const T*)L.w_ukT, nullptr, qa, n_proj, n, R, L.dim,
                            hb_rowmap{nullptr, nullptr, 0, 1, (long)R * L.dim, (long)dq, (long)D, 0, nullptr, 0.f}, H));
         if (r > 0 && L.q_rank > 0)
             hipLaunchKernelGGL(k_hb_latent_qrot, dim3(n, H), dim3(64), 0, st, q, (long)n_proj, qa, (long)n_proj, L.inv_freq, io->pos, L.dim, R, r,
@@ -4949,14 +5158,14 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
                                HB_ATTN_SEG, gate, (long)n_proj, L.out_scale, 64, sink, 0, 0);
         }
         // every head's weighted latent times its value expansion
-        VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, o, n_proj, (const T*)L.w_uv, nullptr, m->mix, n_mix, n, L.vdim, R,
+        VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, o, n_proj, (const T*)L.w_uv, nullptr, m->mix, n_mix, n, L.vdim, R,
                            hb_rowmap{nullptr, nullptr, 0, 1, (long)L.vdim * R, (long)R, (long)L.vdim, 0, nullptr, 0.f}, H));
     } else if (L.kind == VOX_MIXER_RGLRU) {
         const int C = L.heads * L.dim, bs = L.dim;
         hipLaunchKernelGGL(k_hb_conv_causal, dim3(n, (C + 255) / 256), dim3(256), 0, st, m->proj, (long)n_proj, L.conv_w, L.conv_b, state, io->pos,
                            io->row_req, io->req_rows, io->req_state, C, L.conv_taps);
         // block-diagonal gates: block b's 2*bs outputs (r rows, then i rows) from its bs channels of the convolution's output
-        VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, m->proj + 2 * C, n_proj, (const T*)L.w_gates, L.b_gates, m->proj + 3 * C, n_proj, n, 2 * bs, bs,
+        VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, m->proj + 2 * C, n_proj, (const T*)L.w_gates, L.b_gates, m->proj + 3 * C, n_proj, n, 2 * bs, bs,
                            hb_rowmap{nullptr, nullptr, 0, 1, (long)2 * bs * bs, (long)bs, (long)2 * bs, (long)2 * bs}, L.heads));
         // steps of many rows cut every request's rows into chunks that run side by side; the chunked form replays the same recurrence
         // from carries that were pushed through whole chunks, which differs from the plain form by rounding only
@@ -5032,7 +5241,7 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
             hipLaunchKernelGGL(hb_merge_kernel(L.vdim), dim3(n, H), dim3(64), 0, st, m->attn_ws, nseg, m->mix, (long)n_mix, io->pos, H, L.vdim, window, P,
                                HB_ATTN_SEG, gate, (long)n_proj, L.out_scale, 64, sink, 0, 0);
     }
-    return hb_gemm_resid<T>(st, m->mix, n_mix, (const T*)L.w_out, nullptr, cur, ldx, n, W, n_mix, jn);
+    return hb_gemm_resid<T>(m->ws16, st, m->mix, n_mix, (const T*)L.w_out, nullptr, cur, ldx, n, W, n_mix, jn);
 }
 
 // Routed feed-forward of the rows h2 (first completed by `post` when it names a sublayer's output), added to cur.  Few rows: one GEMV pair per routed entry; more: the entries are
@@ -5061,27 +5270,36 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
                            (const T*)E.shared_down, m->moe_act, cur, ldx, W, q);
         return VOX_OK;
     }
-    if (L.res_gate) VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, h2, ldh, (const T*)L.w_gate_ff, L.b_gate_ff, m->rgate, W, n, W, W));
+    if (L.res_gate) VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, h2, ldh, (const T*)L.w_gate_ff, L.b_gate_ff, m->rgate, W, n, W, W));
     if (E.experts > 0) {
         const int cap = m->cfg.max_rows;
         hipLaunchKernelGGL(k_hb_moe_group, dim3(E.experts), dim3(256), 0, st, m->moe_sel, ne, cap, m->moe_list, m->moe_count);
-        VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(st, h2, ldh, (const T*)E.w_gate_up, nullptr, m->ff, (long)nf * ff, n, nf * ff, W,
-                                            hb_rowmap{m->moe_count, m->moe_list, cap, top, (long)nf * ff * W, 0, 0, 0,
-                                                      E.scale_input ? m->moe_wgt : (const float*)nullptr, 0.f}, E.experts));
-        hipLaunchKernelGGL(k_hb_glu_clamp, dim3(ne, (ff + 1023) / 1024), dim3(256), 0, st, m->ff, m->moe_act, ff, E.limit, E.act_alpha,
-                           m->moe_sel, E.experts, E.up_offset, 0, up_down, relu2);
-        VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(st, m->moe_act, (long)ff, (const T*)E.w_down, nullptr, m->moe_out, (long)W, n, W, ff,
-                                            hb_rowmap{m->moe_count, m->moe_list, cap, 1, (long)W * ff, 0, 0, 0}, E.experts));
+        const int rows = (int)(((size_t)ne + E.experts - 1) / E.experts);        // of an expert, were they all alike
+        const hb_rowmap up{m->moe_count, m->moe_list, cap, top, (long)nf * ff * W, 0, 0, 0, E.scale_input ? m->moe_wgt : (const float*)nullptr, 0.f};
+        hb_rowmap down{m->moe_count, m->moe_list, cap, 1, (long)W * ff, 0, 0, 0};
+        if (!up_down && !E.scale_input && hb_try_glu(m->ws16, st, h2, ldh, n, (const T*)E.w_gate_up, nullptr, m->moe_act, n, ff, W, (const T*)E.w_down, W, up,
+                                                     E.experts, rows, (size_t)ne, hb_glu_args{E.limit, E.act_alpha, E.up_offset, 0}))
+            down.a16 = (const bf16_t*)m->moe_act;
+        else {
+            VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(m->ws16, st, h2, ldh, (const T*)E.w_gate_up, nullptr, m->ff, (long)nf * ff, n, nf * ff, W, up, E.experts, rows, n));
+            hipLaunchKernelGGL(k_hb_glu_clamp, dim3(ne, (ff + 1023) / 1024), dim3(256), 0, st, m->ff, m->moe_act, ff, E.limit, E.act_alpha,
+                               m->moe_sel, E.experts, E.up_offset, 0, up_down, relu2);
+        }
+        VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(m->ws16, st, m->moe_act, (long)ff, (const T*)E.w_down, nullptr, m->moe_out, (long)W, n, W, ff, down, E.experts, rows, ne));
     }
     hipLaunchKernelGGL(k_hb_moe_combine, dim3(n), dim3(256), 0, st, cur, ldx, h2, ldh, m->moe_out, m->moe_sel, m->moe_wgt, top, E.experts, W,
                        E.scale_input, jn);
     if (E.shared_ff > 0) {
         const int sf = E.shared_ff;
-        VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, h2, ldh, (const T*)E.shared_gate_up, nullptr, m->ff, nf * sf, n, nf * sf, W));
-        hipLaunchKernelGGL(k_hb_glu_clamp, dim3(n, (sf + 1023) / 1024), dim3(256), 0, st, m->ff, m->moe_act, sf, E.shared_limit, E.act_alpha,
-                           (const int*)nullptr, 0, E.up_offset, 0, up_down, relu2);
+        const bool fused = !up_down && hb_try_glu(m->ws16, st, h2, ldh, n, (const T*)E.shared_gate_up, nullptr, m->moe_act, n, sf, W, (const T*)E.shared_down, W,
+                                                  hb_plain(), 1, n, (size_t)n, hb_glu_args{E.shared_limit, E.act_alpha, E.up_offset, 0});
+        if (!fused) {
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, h2, ldh, (const T*)E.shared_gate_up, nullptr, m->ff, nf * sf, n, nf * sf, W));
+            hipLaunchKernelGGL(k_hb_glu_clamp, dim3(n, (sf + 1023) / 1024), dim3(256), 0, st, m->ff, m->moe_act, sf, E.shared_limit, E.act_alpha,
+                               (const int*)nullptr, 0, E.up_offset, 0, up_down, relu2);
+        }
         jn.store = 0;      // (the routed sum is there already)
-        VOX_TRY(hb_gemm_resid<T>(st, m->moe_act, sf, (const T*)E.shared_down, nullptr, cur, ldx, n, W, sf, jn));
+        VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->moe_act, sf, (const T*)E.shared_down, nullptr, cur, ldx, n, W, sf, jn, fused ? (const bf16_t*)m->moe_act : nullptr));
     }
     return VOX_OK;
 }
@@ -5106,7 +5324,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
         const vox_hybrid_layer& L = m->layers[run.layer];
         if (run.loop_in) {
             hb_settle(st, pd, n, W);
-            VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, cur, ldx, (const T*)m->w.loop_in, nullptr, other, ldx, n, W, 2 * W));
+            VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, cur, ldx, (const T*)m->w.loop_in, nullptr, other, ldx, n, W, 2 * W));
             float* t = cur; cur = other; other = t;
         }
         const bool has_ff = L.ff > 0 || L.moe;
@@ -5160,6 +5378,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             if (!parallel && !post) hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h2, nullptr, nullptr, (long)W, L.norm2_b);
             const float* hd = parallel ? hf : m->h2;
             const float limit = L.ff_limit > 0.f ? L.ff_limit : INFINITY, alpha = L.ff_alpha != 0.f ? L.ff_alpha : 1.0f;
+            const bf16_t* act16 = nullptr;      // the activations as bf16, when the products behind them left them so
             if (post && n == 1 && hb_try_post_gemv<T>(st, pd, true, (const T*)L.w_up, L.b_up, m->ff_act, L.ff, W, limit, alpha, L.ff_up_offset,
                                                       L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0)) {
                 // (one row of a post-normed layer: norm, both products and the activation in one launch)
@@ -5174,24 +5393,30 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
                                    m->ff_act, W, q);
             } else {
                 if (post) hd = pd.x;
-                VOX_TRY(hb_gemm<T>(st, HB_EPI_STORE, hd, ldf, (const T*)L.w_up, L.b_up, m->ff, 2 * L.ff, n, 2 * L.ff, W));
-                hipLaunchKernelGGL(k_hb_glu_clamp, dim3(n, (L.ff + 1023) / 1024), dim3(256), 0, st, m->ff, m->ff_act, L.ff, limit, alpha,
-                                   (const int*)nullptr, 0, L.ff_up_offset, L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0, 0, 0);
+                const int gelu = L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0;
+                if (hb_try_glu(m->ws16, st, hd, ldf, n, (const T*)L.w_up, L.b_up, m->ff_act, n, L.ff, W, (const T*)L.w_down, W, hb_plain(), 1, n, (size_t)n,
+                               hb_glu_args{limit, alpha, L.ff_up_offset, gelu}))
+                    act16 = (const bf16_t*)m->ff_act;
+                else {
+                    VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, hd, ldf, (const T*)L.w_up, L.b_up, m->ff, 2 * L.ff, n, 2 * L.ff, W));
+                    hipLaunchKernelGGL(k_hb_glu_clamp, dim3(n, (L.ff + 1023) / 1024), dim3(256), 0, st, m->ff, m->ff_act, L.ff, limit, alpha,
+                                       (const int*)nullptr, 0, L.ff_up_offset, gelu, 0, 0);
+                }
             }
-            VOX_TRY(hb_gemm_resid<T>(st, m->ff_act, L.ff, (const T*)L.w_down, L.b_down, dst, ldd, n, W, L.ff, j2));
+            VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->ff_act, L.ff, (const T*)L.w_down, L.b_down, dst, ldd, n, W, L.ff, j2, act16));
         } else if (L.ff > 0) {
             // up rows with their activation, then (a residual gate) its rows, as one product
             const int nf = L.ff + L.res_gate, epi = L.ff_act == VOX_ACT_RELU2 ? HB_EPI_RELU2 : HB_EPI_GELU;
             hb_rowmap rm = hb_plain();
             rm.epi_arg = (float)L.ff;
             if (parallel || post) {
-                VOX_TRY(hb_gemm<T>(st, epi, post ? pd.x : hf, ldf, (const T*)L.w_up, L.b_up, m->ff, nf, n, nf, W, rm));
+                VOX_TRY(hb_gemm<T>(m->ws16, st, epi, post ? pd.x : hf, ldf, (const T*)L.w_up, L.b_up, m->ff, nf, n, nf, W, rm));
             } else if (!(n == 1 && hb_try_norm_gemv<T>(m, st, epi, src, lds_x, nullptr, L.norm2, (const T*)L.w_up, L.b_up, m->ff, nf, W, rm.epi_arg, L.norm2_b))) {
                 hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h, nullptr, nullptr, (long)W, L.norm2_b);
-                VOX_TRY(hb_gemm<T>(st, epi, m->h, W, (const T*)L.w_up, L.b_up, m->ff, nf, n, nf, W, rm));
+                VOX_TRY(hb_gemm<T>(m->ws16, st, epi, m->h, W, (const T*)L.w_up, L.b_up, m->ff, nf, n, nf, W, rm));
             }
             if (L.res_gate) { j2.gate = m->ff + L.ff; j2.ldg = nf; }
-            VOX_TRY(hb_gemm_resid<T>(st, m->ff, nf, (const T*)L.w_down, nullptr, dst, ldd, n, W, L.ff, j2));
+            VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->ff, nf, (const T*)L.w_down, nullptr, dst, ldd, n, W, L.ff, j2));
         }
         if (post) {
             if (has_ff) pd.p = post2;
@@ -5216,7 +5441,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
         if (!(n_out == 1 && hb_try_norm_gemv<T>(m, st, epi, last, ld_last, io->out_rows, m->w.final_norm, (const T*)m->w.head, nullptr, io->logits, c.vocab,
                                                 W, rm.epi_arg, m->w.final_norm_b))) {
             hb_norm(m, st, n_out, last, ld_last, io->out_rows, m->w.final_norm, m->hout, nullptr, nullptr, (long)W, m->w.final_norm_b);
-            VOX_TRY(hb_gemm<T>(st, epi, m->hout, W, (const T*)m->w.head, nullptr, io->logits, c.vocab, n_out, c.vocab, W, rm));
+            VOX_TRY(hb_gemm<T>(m->ws16, st, epi, m->hout, W, (const T*)m->w.head, nullptr, io->logits, c.vocab, n_out, c.vocab, W, rm));
         }
     }
     VOX_HIP(hipGetLastError());
@@ -5385,6 +5610,14 @@ int vox_hybrid_create(vox_ctx* ctx, const vox_hybrid_config* cfg, const vox_hybr
               hipMalloc((void**)&m->ff, R * (size_t)(m->max_ff > 0 ? m->max_ff : 1) * 4) == hipSuccess &&
               hipMalloc((void**)&m->hout, (size_t)cfg->max_out * W * 4) == hipSuccess &&
               hipMalloc((void**)&m->logits16, (size_t)cfg->max_batch * cfg->vocab * 2) == hipSuccess;
+    if (ok && cfg->dtype == VOX_HYBRID_BF16 && R > 16) {
+        size_t k = 2 * W;
+        if ((size_t)m->max_mix > k) k = m->max_mix;
+        for (const vox_hybrid_layer& L : m->layers)
+            if ((size_t)L.ff > k) k = L.ff;
+        m->ws16.n = R * k;
+        ok = hipMalloc((void**)&m->ws16.p, m->ws16.n * 2) == hipSuccess;
+    }
     if (ok && cfg->streams > 0) {
         float one[HB_MAX_STREAMS];
         for (float& v : one) v = 1.0f;
@@ -5434,7 +5667,7 @@ int vox_hybrid_create(vox_ctx* ctx, const vox_hybrid_config* cfg, const vox_hybr
 void vox_hybrid_destroy(vox_hybrid* m) {
     if (!m) return;
     (void)hipFree(m->xa); (void)hipFree(m->xb); (void)hipFree(m->h); (void)hipFree(m->h2); (void)hipFree(m->proj); (void)hipFree(m->mix);
-    (void)hipFree(m->ff); (void)hipFree(m->ff_act); (void)hipFree(m->u); (void)hipFree(m->y); (void)hipFree(m->ones); (void)hipFree(m->rgate); (void)hipFree(m->hout); (void)hipFree(m->logits16); (void)hipFree(m->attn_ws); (void)hipFree(m->shift); (void)hipFree(m->scan_ws);
+    (void)hipFree(m->ff); (void)hipFree(m->ff_act); (void)hipFree(m->u); (void)hipFree(m->y); (void)hipFree(m->ones); (void)hipFree(m->rgate); (void)hipFree(m->hout); (void)hipFree(m->logits16); (void)hipFree(m->ws16.p); (void)hipFree(m->attn_ws); (void)hipFree(m->shift); (void)hipFree(m->scan_ws);
     (void)hipFree(m->moe_wgt); (void)hipFree(m->moe_sel); (void)hipFree(m->moe_act); (void)hipFree(m->moe_out);
     (void)hipFree(m->moe_list); (void)hipFree(m->moe_count);
     delete m;
