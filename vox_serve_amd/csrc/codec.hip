@@ -3446,6 +3446,261 @@ __global__ void k_flow_slots(int* slots, int N, int B) {
     if (i < N) slots[i] = i / B;
 }
 
+// ---- estimator transformer block at 256 channels, 8 heads of 64, feed-forward 1024: two launches beside the attention ------------------
+// Everything but the attention is row-local, so a block keeps 16 rows in LDS and walks its products there: the operands of a product are the
+// rows' three bf16 terms in the order an MFMA operand is read (one 16-byte read per lane, no conflicts), the weights come from a
+// fragment-major copy (1 KB per wave request, whole lines) straight into registers.  Products are taken transposed (weight rows x
+// activation rows): a lane then holds four neighbouring columns of one row, which is what it stores, normalises and splits.
+//   k_tb_qkv   rows = residual + feed-forward parts of the block before, LayerNorm, q | k | v: grid (row tiles, 256-column groups)
+//   k_tb_ff    attention out + residual, LayerNorm, GELU feed-forward: grid (row tiles, 4); block y owns a quarter of the hidden columns from
+//              ff1 to its part of ff2 (parts [4] + the residual rows are added by whoever reads them, in a fixed order); the out product is
+//              done by all four
+// What one of these leaves for another (parts, the residual rows) lies in the order of the lanes, [row tile][wave][tile][lane] x 4 floats:
+// whole lines per request (as [row][256] every request touched 16 lines: k_tb_qkv 12.8 us against 8.3 with plain rows to read).
+// Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 8.2 /
+// 10.3 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 12.7; a window of 8 requests 45.9 -> 31.6 ms.  A row's result depends on that row only.
+#define TB_C 256
+#define TB_IN 512
+#define TB_FF 1024
+struct FlowPacked {
+    const bf16_t *qkv = nullptr, *out = nullptr, *ff1 = nullptr, *ff2 = nullptr;
+};
+// w [N][K] bf16 -> tiles of 16 rows x 32 columns (row tile major), each as the 64 lanes of an MFMA operand hold it
+__global__ __launch_bounds__(256) void k_pack_frag(const bf16_t* w, bf16_t* out, int K, size_t chunks) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= chunks) return;
+    const int kb_n = K >> 5, lane = (int)(i & 63);
+    const size_t tile = i >> 6, kb = tile % kb_n, rt = tile / kb_n;
+    *reinterpret_cast<uint4*>(out + i * 8) = *reinterpret_cast<const uint4*>(w + (rt * 16 + (lane & 15)) * K + kb * 32 + (lane >> 4) * 8);
+}
+struct tb_split {
+    uint2 t[3];      // four values' leading, second and third bf16 terms
+};
+__device__ __forceinline__ tb_split tb_split3(float4 v) {
+    tb_split s;
+    s.t[0] = make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
+    const float4 r = make_float4(v.x - bflo(s.t[0].x), v.y - bfhi(s.t[0].x), v.z - bflo(s.t[0].y), v.w - bfhi(s.t[0].y));
+    s.t[1] = make_uint2(pack_bf2(r.x, r.y), pack_bf2(r.z, r.w));
+    s.t[2] = make_uint2(pack_bf2(r.x - bflo(s.t[1].x), r.y - bfhi(s.t[1].x)), pack_bf2(r.z - bflo(s.t[1].y), r.w - bfhi(s.t[1].y)));
+    return s;
+}
+__device__ __forceinline__ float4 tb_add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+// Column tile 2 wave + t of 256 columns as an operand of the next product: k-block `wave`, k group 2 t + kq / 2
+__device__ __forceinline__ void tb_put(uint4* pl, int kb_n, int wave, int t, int lane, float4 v) {
+    const tb_split s = tb_split3(v);
+    const int fr = lane & 15, kq = lane >> 4;
+    uint2* d = reinterpret_cast<uint2*>(pl + wave * 64 + (2 * t + (kq >> 1)) * 16 + fr) + (kq & 1);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) d[p * kb_n * 128] = s.t[p];
+}
+// LayerNorm of the rows whose columns lie 8 to a lane (two tiles of four) over the block's eight waves; red: [2][8][16]
+__device__ __forceinline__ void tb_layernorm(float4 (&v)[2], const float4 (&w)[2], const float4 (&b)[2], float* red, int wave, int lane) {
+    const int fr = lane & 15;
+    float s = ((v[0].x + v[0].y) + (v[0].z + v[0].w)) + ((v[1].x + v[1].y) + (v[1].z + v[1].w));
+    s += __shfl_xor(s, 16, 64); s += __shfl_xor(s, 32, 64);
+    if (lane < 16) red[wave * 16 + fr] = s;
+    __syncthreads();
+    float tot = red[fr];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) tot += red[i * 16 + fr];
+    const float mean = tot / (float)TB_C;
+    float q = 0.0f;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        v[t] = make_float4(v[t].x - mean, v[t].y - mean, v[t].z - mean, v[t].w - mean);
+        q += (v[t].x * v[t].x + v[t].y * v[t].y) + (v[t].z * v[t].z + v[t].w * v[t].w);
+    }
+    q += __shfl_xor(q, 16, 64); q += __shfl_xor(q, 32, 64);
+    if (lane < 16) red[128 + wave * 16 + fr] = q;
+    __syncthreads();
+    float var = red[128 + fr];
+#pragma unroll
+    for (int i = 1; i < 8; ++i) var += red[128 + i * 16 + fr];
+    const float rstd = rsqrtf(var / (float)TB_C + 1e-5f);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+        v[t] = make_float4(v[t].x * rstd * w[t].x + b[t].x, v[t].y * rstd * w[t].y + b[t].y, v[t].z * rstd * w[t].z + b[t].z, v[t].w * rstd * w[t].w + b[t].w);
+}
+// two column tiles against the rows in pl (KB k-blocks, three terms, low terms first)
+template <int KB>
+__device__ __forceinline__ void tb_product(const uint4 (&wf)[2][KB], const uint4* pl, int lane, f32x4 (&acc)[2]) {
+    acc[0] = acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+        for (int p = 2; p >= 0; --p) {
+            const uint4 x = pl[(p * KB + kb) * 64 + lane];
+#pragma unroll
+            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[t], 0, 0, 0);
+        }
+}
+template <int KB>
+__device__ __forceinline__ void tb_weights(uint4 (&wf)[2][KB], const bf16_t* w, int tile, int kb_all, int kb0, int lane) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) wf[t][kb] = *reinterpret_cast<const uint4*>(w + ((size_t)(tile + t) * kb_all + kb0 + kb) * 512 + lane * 8);
+}
+// floats of column tile 2 wave + t of row tile `rt` in lane order
+__device__ __forceinline__ size_t tb_at(int rt, int wave, int t, int lane) { return ((((size_t)rt * 8 + wave) * 2 + t) * 64 + lane) * 4; }
+// rows [.][256] = parts[4] + (((parts[0] + parts[1]) + parts[2]) + parts[3]), ps floats apart
+__device__ __forceinline__ float4 tb_sum(const float* p, size_t ps) {
+    float4 v[5];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) v[i] = *reinterpret_cast<const float4*>(p + i * ps);
+    return tb_add(v[4], tb_add(tb_add(tb_add(v[0], v[1]), v[2]), v[3]));
+}
+template <bool PARTS>
+__global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* parts, size_t ps, const bf16_t* w, const float* lnw, const float* lnb,
+                                                float* qkv, float* h_out, int M, int N) {
+    __shared__ uint4 pl[3 * 8 * 64];
+    __shared__ float red[256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4;
+    const int m = blockIdx.x * 16 + fr, row = m < M ? m : M - 1, tile = (blockIdx.y * 8 + wave) * 2;
+    float4 v[2], lw[2], lb[2];
+    uint4 wf[2][8];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int c = (wave * 2 + t) * 16 + kq * 4;
+        v[t] = PARTS ? tb_sum(parts + tb_at(blockIdx.x, wave, t, lane), ps) : *reinterpret_cast<const float4*>(h + (size_t)row * TB_C + c);
+        lw[t] = *reinterpret_cast<const float4*>(lnw + c);
+        lb[t] = *reinterpret_cast<const float4*>(lnb + c);
+    }
+    tb_weights<8>(wf, w, tile, 8, 0, lane);
+    if (PARTS && blockIdx.y == 0)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) *reinterpret_cast<float4*>(h_out + tb_at(blockIdx.x, wave, t, lane)) = v[t];
+    tb_layernorm(v, lw, lb, red, wave, lane);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, v[t]);
+    __syncthreads();
+    f32x4 acc[2];
+    tb_product<8>(wf, pl, lane, acc);
+    if (m < M)
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+            *reinterpret_cast<float4*>(qkv + (size_t)m * N + (tile + t) * 16 + kq * 4) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+}
+// lane_h: h lies in lane order
+__global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h, int lane_h, FlowPacked w, const float* b_out, const float* lnw, const float* lnb,
+                                               const float* b1, const float* b2, float* parts, size_t ps, int M) {
+    __shared__ uint4 pl[3 * 16 * 64];
+    __shared__ float red[256];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4, q = blockIdx.y;
+    const int m0 = blockIdx.x * 16, m = m0 + fr, row = m < M ? m : M - 1;
+    float4 a[2][2], res[2], bo[2], lw[2], lb[2], bh[2], by[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {      // the attention rows: thread = (row, 8 columns)
+        const float* s = att + (size_t)(m0 + (tid & 15) < M ? m0 + (tid & 15) : M - 1) * TB_IN + ((tid >> 4) + 32 * i) * 8;
+        a[i][0] = *reinterpret_cast<const float4*>(s);
+        a[i][1] = *reinterpret_cast<const float4*>(s + 4);
+    }
+    uint4 wo[2][16];
+    tb_weights<16>(wo, w.out, wave * 2, 16, 0, lane);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const int c = (wave * 2 + t) * 16 + kq * 4;
+        res[t] = *reinterpret_cast<const float4*>(h + (lane_h ? tb_at(blockIdx.x, wave, t, lane) : (size_t)row * TB_C + c));
+        bo[t] = *reinterpret_cast<const float4*>(b_out + c);
+        lw[t] = *reinterpret_cast<const float4*>(lnw + c);
+        lb[t] = *reinterpret_cast<const float4*>(lnb + c);
+        bh[t] = *reinterpret_cast<const float4*>(b1 + q * 256 + c);
+        by[t] = *reinterpret_cast<const float4*>(b2 + c);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const tb_split s0 = tb_split3(a[i][0]), s1 = tb_split3(a[i][1]);
+        const int k8 = (tid >> 4) + 32 * i;
+#pragma unroll
+        for (int p = 0; p < 3; ++p) pl[(p * 16 + (k8 >> 2)) * 64 + (k8 & 3) * 16 + (tid & 15)] = make_uint4(s0.t[p].x, s0.t[p].y, s1.t[p].x, s1.t[p].y);
+    }
+    __syncthreads();
+    f32x4 acc[2];
+    tb_product<16>(wo, pl, lane, acc);
+    uint4 w1[2][8], w2[2][8];
+    tb_weights<8>(w1, w.ff1, q * 16 + wave * 2, 8, 0, lane);
+    float4 x[2], n[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) n[t] = x[t] = tb_add(res[t], tb_add(make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]), bo[t]));
+    tb_layernorm(n, lw, lb, red, wave, lane);      // (its barriers: every wave has read the attention rows)
+#pragma unroll
+    for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, n[t]);
+    __syncthreads();
+    tb_product<8>(w1, pl, lane, acc);
+    tb_weights<8>(w2, w.ff2, wave * 2, 32, q * 8, lane);
+    uint4* const hid = pl + 3 * 8 * 64;
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        float g[4];
+        const float bb[4] = {bh[t].x, bh[t].y, bh[t].z, bh[t].w};
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float z = acc[t][r] + bb[r];
+            g[r] = 0.5f * z * (1.0f + erff(z * 0.70710678118654752440f));
+        }
+        tb_put(hid, 8, wave, t, lane, make_float4(g[0], g[1], g[2], g[3]));
+    }
+    __syncthreads();
+    tb_product<8>(w2, hid, lane, acc);
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        float4 y = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
+        const size_t o = tb_at(blockIdx.x, wave, t, lane);
+        if (q == 0) {
+            y = tb_add(y, by[t]);
+            *reinterpret_cast<float4*>(parts + 4 * ps + o) = x[t];
+        }
+        *reinterpret_cast<float4*>(parts + (size_t)q * ps + o) = y;
+    }
+}
+__global__ __launch_bounds__(256) void k_tb_join(const float* parts, size_t ps, float* h, int M) {
+    const int i = blockIdx.x * 256 + threadIdx.x, lane = i & 63, col = (i >> 6 & 15) * 16 + (lane >> 4) * 4, m = (i >> 10) * 16 + (lane & 15);
+    if (m < M) *reinterpret_cast<float4*>(h + (size_t)m * TB_C + col) = tb_sum(parts + (size_t)i * 4, ps);
+}
+// fragment-major copies of every transformer block's weights, or an empty list where a block has other sizes (then the general launches run)
+static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, std::vector<FlowPacked>& out, void** mem) {
+    if (C != TB_C || inner != TB_IN || tb.empty()) return true;
+    const vox_conv_w vox_flow_tblock_w::*const which[4] = {&vox_flow_tblock_w::qkv, &vox_flow_tblock_w::out, &vox_flow_tblock_w::ff1, &vox_flow_tblock_w::ff2};
+    const int n_of[4] = {3 * TB_IN, TB_C, TB_FF, TB_C}, k_of[4] = {TB_C, TB_IN, TB_C, TB_FF};
+    size_t per = 0;
+    for (int i = 0; i < 4; ++i) per += (size_t)n_of[i] * k_of[i];
+    for (const vox_flow_tblock_w& t : tb)
+        for (int i = 0; i < 4; ++i) {
+            const vox_conv_w& w = t.*which[i];
+            if (w.n_taps != 1 || w.n != n_of[i] || w.cin != k_of[i] || (i == 0) == (w.bias != nullptr) || ((size_t)w.w & 15) || ((size_t)w.bias & 15) ||
+                ((size_t)t.ln1_w & 15) || ((size_t)t.ln1_b & 15) || ((size_t)t.ln3_w & 15) || ((size_t)t.ln3_b & 15)) return true;
+        }
+    if (hipMalloc(mem, per * tb.size() * 2) != hipSuccess) return false;
+    bf16_t* p = (bf16_t*)*mem;
+    for (const vox_flow_tblock_w& t : tb) {
+        FlowPacked f;
+        const bf16_t** const to[4] = {&f.qkv, &f.out, &f.ff1, &f.ff2};
+        for (int i = 0; i < 4; ++i) {
+            const size_t chunks = (size_t)n_of[i] * k_of[i] / 8;
+            hipLaunchKernelGGL(k_pack_frag, dim3((unsigned)((chunks + 255) / 256)), dim3(256), 0, (hipStream_t) nullptr, (const bf16_t*)(t.*which[i]).w, p, k_of[i], chunks);
+            *to[i] = p;
+            p += chunks * 8;
+        }
+        out.push_back(f);
+    }
+    return hipGetLastError() == hipSuccess;
+}
+// floats of scratch for M rows: four parts, the residual rows of the block before and of this one
+static size_t tb_room(int M) { return (size_t)((M + 15) / 16) * 16 * TB_C * 6; }
+// q | k | v of the rows into qkv (first: of h itself; else of what the block before has left in ws)
+static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* h, float* ws, bool first, float* qkv, int M) {
+    const dim3 g((M + 15) / 16, 3 * TB_IN / 256);
+    const size_t ps = tb_room(M) / 6;
+    if (first) hipLaunchKernelGGL(k_tb_qkv<false>, g, dim3(512), 0, st, h, ws, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN);
+    else hipLaunchKernelGGL(k_tb_qkv<true>, g, dim3(512), 0, st, h, ws, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws + 5 * ps, M, 3 * TB_IN);
+}
+static void tb_ff(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* att, float* h, float* ws, bool first, bool last, int M) {
+    const size_t ps = tb_room(M) / 6;
+    hipLaunchKernelGGL(k_tb_ff, dim3((M + 15) / 16, 4), dim3(512), 0, st, att, first ? h : ws + 5 * ps, first ? 0 : 1, f, w.out.bias, w.ln3_w, w.ln3_b,
+                       w.ff1.bias, w.ff2.bias, ws, ps, M);
+    if (last) hipLaunchKernelGGL(k_tb_join, dim3((unsigned)((M + 15) / 16 * 4)), dim3(256), 0, st, ws, ps, h, M);
+}
+
 struct vox_flow {
     vox_ctx* ctx;
     vox_flow_config cfg;
@@ -3453,6 +3708,8 @@ struct vox_flow {
     std::vector<vox_flow_conformer_w> enc;
     std::vector<vox_flow_resnet_w> resnets;
     std::vector<vox_flow_tblock_w> tblocks;
+    std::vector<FlowPacked> packed;         // per transformer block, or empty
+    void* packed_mem = nullptr;
     int max_batch, max_T, max_prompt_T, n_res, n_att;
     std::vector<float> dt;                  // host: Euler step sizes
     float* tb = nullptr;                    // [n_steps][n_res][C]: mlp_r(Mish(time_mlp(emb_s)))
@@ -3489,6 +3746,7 @@ void vox_flow_destroy(vox_flow* m) {
     (void)hipFree(m->s_enc); (void)hipFree(m->s_up); (void)hipFree(m->s_att); (void)hipFree(m->s_cnn1); (void)hipFree(m->s_cnn2);
     (void)hipFree(m->s_eidx); (void)hipFree(m->s_cidx);
     for (void* p : m->conv1x_mem) (void)hipFree(p);
+    (void)hipFree(m->packed_mem);
     delete m;
 }
 
@@ -3645,7 +3903,9 @@ static int flow_run(vox_flow* m, hipStream_t st, const int32_t* tokens, int B, i
             for (int j = 0; j < c.est_blocks; ++j, ++li) {
                 const vox_flow_tblock_w& tw = m->tblocks[li];
                 float* kv = (evolve ? m->s_att : m->att_kv) + ((size_t)s * m->n_att + li) * att_layer;
-                VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, T2, a2, 0));
+                const FlowPacked* pk = m->packed.empty() || tb_room(N * T2) > m->buf_floats ? nullptr : &m->packed[li];
+                if (pk) tb_qkv(st, *pk, tw, h, a1, j == 0, a2, N * T2);
+                else VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, T2, a2, 0));
                 FlowAttn a{a2, init ? nullptr : kv, nullptr, nullptr, nullptr, a3, T2, HE, hd, Tc, capA, B, att_half, 1.0f / sqrtf((float)hd)};
                 if (evolve) { a.cidx = m->s_cidx; a.prefix = c.prefix; a.ring_head = evolve->att_head; }
                 launch_flow_attn(st, a, T2, HE, N);
@@ -3655,6 +3915,7 @@ static int flow_run(vox_flow* m, hipStream_t st, const int32_t* tokens, int B, i
                 if (init)
                     hipLaunchKernelGGL(k_flow_cache_store, dim3(ew_grid((size_t)N * HE * capA * 2 * hd)), dim3(256), 0, st, a2, kv, T2, HE, hd, capA,
                                        c.prefix, att_half, N);
+                if (pk) { tb_ff(st, *pk, tw, a3, h, a1, j == 0, j + 1 == c.est_blocks, N * T2); continue; }
                 VOX_TRY(conv_gemm(st, tw.out, a3, nullptr, nullptr, N, T2, 0, FLOW_OFF0, h, h, nullptr, 0));
                 VOX_TRY(ln_gemm(st, tw.ff1, h, tw.ln3_w, tw.ln3_b, 1e-5f, a1, N, T2, a2, 1));
                 VOX_TRY(conv_gemm(st, tw.ff2, a2, nullptr, nullptr, N, T2, 0, FLOW_OFF0, h, h, nullptr, 0));
@@ -3735,6 +3996,7 @@ int vox_flow_create(vox_ctx* ctx, const vox_flow_config* cfg, const vox_flow_wei
         cx.w = wx; cx.bias = bx; cx.n = 2 * C; cx.bias_mod = 0;
         m->conv1x.push_back(cx);
     }
+    ok = ok && tb_pack(m->tblocks, C, inner, m->packed, &m->packed_mem);
     if (!ok) { vox_flow_destroy(m); return vox_fail(VOX_ERR_NOMEM, "flow_create: hipMalloc failed"); }
     // time projections of every Euler step and resnet, once: tb[s][r] = mlp_r(Mish(linear_2(SiLU(linear_1(emb_s)))))
     hipStream_t st = nullptr;
@@ -4075,6 +4337,8 @@ struct vox_glmflow {
     std::vector<vox_flow_conformer_w> enc;
     std::vector<vox_flow_resnet_w> resnets;
     std::vector<vox_flow_tblock_w> tblocks;
+    std::vector<FlowPacked> packed;         // per transformer block, or empty
+    void* packed_mem = nullptr;
     int max_batch, max_T, max_mel, n_res, n_att;
     std::vector<float> dt;
     float* tb = nullptr;
@@ -4090,7 +4354,7 @@ extern "C" {
 void vox_glmflow_destroy(vox_glmflow* m) {
     if (!m) return;
     for (int i = 0; i < 10; ++i) (void)hipFree(m->buf[i]);
-    (void)hipFree(m->tb); (void)hipFree(m->spk); (void)hipFree(m->pe); (void)hipFree(m->pp);
+    (void)hipFree(m->tb); (void)hipFree(m->spk); (void)hipFree(m->pe); (void)hipFree(m->pp); (void)hipFree(m->packed_mem);
     delete m;
 }
 
@@ -4123,6 +4387,7 @@ int vox_glmflow_create(vox_ctx* ctx, const vox_glmflow_config* cfg, const vox_gl
     alloc(&m->spk, (size_t)max_batch * c.mel);
     alloc(&m->pe, (size_t)2 * FLOW_MAXKEYS * D);
     alloc(&m->pp, (size_t)2 * FLOW_MAXKEYS * D);
+    ok = ok && tb_pack(m->tblocks, C, inner, m->packed, &m->packed_mem);
     if (!ok) { vox_glmflow_destroy(m); return vox_fail(VOX_ERR_NOMEM, "glmflow_create: hipMalloc failed"); }
     hipStream_t st = nullptr;
     g_conv_planes = 3;
@@ -4196,9 +4461,12 @@ int vox_glmflow_decode(vox_glmflow* m, void* stream, const int32_t* tokens, int 
     auto tblocks = [&](float* h, int rows_T, int& li, float* a1, float* a2, float* a3) -> int {
         for (int j = 0; j < c.est_blocks; ++j, ++li) {
             const vox_flow_tblock_w& tw = m->tblocks[li];
-            VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, rows_T, a2, 0));
+            const FlowPacked* pk = m->packed.empty() || tb_room(N * rows_T) > m->buf_floats ? nullptr : &m->packed[li];
+            if (pk) tb_qkv(st, *pk, tw, h, a1, j == 0, a2, N * rows_T);
+            else VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, rows_T, a2, 0));
             FlowAttn a{a2, nullptr, nullptr, nullptr, nullptr, a3, rows_T, HE, hd, 0, 0, 0, 0, 1.0f / sqrtf((float)hd), 0};
             launch_flow_attn(st, a, rows_T, HE, N);
+            if (pk) { tb_ff(st, *pk, tw, a3, h, a1, j == 0, j + 1 == c.est_blocks, N * rows_T); continue; }
             VOX_TRY(conv_gemm(st, tw.out, a3, nullptr, nullptr, N, rows_T, 0, FLOW_OFF0, h, h, nullptr, 0));
             VOX_TRY(ln_gemm(st, tw.ff1, h, tw.ln3_w, tw.ln3_b, 1e-5f, a1, N, rows_T, a2, 1));
             VOX_TRY(conv_gemm(st, tw.ff2, a2, nullptr, nullptr, N, rows_T, 0, FLOW_OFF0, h, h, nullptr, 0));
