@@ -1,0 +1,52 @@
+"""The LDS-DMA convolutions of the Qwen3 codec (k_conv_dma) at the shapes where their tiles can go wrong, against the CPU oracle in fp32.
+
+Channel counts that are multiples of 32, 64, 128 and 256 only (the k-steps of the tiles), fewer rows than one tile and rows that do not
+fill the last one, intermediate sizes that end inside a gate / up pair, chunks shorter than a conv's look-back (the history shifts in
+place) and a batch whose requests end inside a tile.
+
+Tolerance: the waveform bar of the decoder, RMS <= 1e-4 against fp32 (two bf16 terms keep 16 significand bits of every operand: relative
+2^-17 per product, and the sums are fp32).  In the bf16 operand mode one term keeps 8 bits, 2^-9 per operand.  That mode rounds where the
+staged kernels rounded, so it is held to the same multiple of its own rounding: 2^8 times the bar."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import qwen3_codec_ref as CR
+from .test_gpu_codec import dev, oracle_exact, rms  # noqa: F401  (dev: fixture)
+
+pytestmark = pytest.mark.gpu
+
+
+def cfg_of(codebook_dim, latent, hidden, inter, heads, head_dim, decoder, rates):
+    return CR.CodecCfg(codebook_size=64, codebook_dim=codebook_dim, latent_dim=latent, decoder_dim=decoder, hidden_size=hidden,
+                       intermediate_size=inter, head_dim=head_dim, num_heads=heads, num_layers=2, num_quantizers=3, sliding_window=12,
+                       upsample_rates=rates, upsampling_ratios=[2, 2])
+
+
+CASES = [
+    # codebook, latent, hidden, intermediate, heads, head_dim, decoder, rates, requests, frames per chunk
+    ((64, 96, 96, 96, 2, 16, 512, [2, 2, 2, 2]), 1, 1),        # 32-channel steps, one row, look-back longer than the chunk
+    ((64, 96, 32, 160, 2, 16, 1536, [3, 2, 2, 2]), 3, 2),      # 1536 -> 768 ... 96 channels, gate / up pairs ending inside a column tile
+    ((128, 64, 64, 96, 4, 16, 512, [4, 2, 2, 2]), 5, 3),       # 64-channel steps, 15 rows of a 16-row tile
+    ((256, 128, 128, 128, 2, 64, 512, [2, 3, 2, 2]), 17, 1),   # 128-channel steps, 17 rows: one into a second tile; head dim 64
+    ((512, 384, 384, 640, 6, 64, 1024, [2, 2, 2, 3]), 2, 4),   # 128-channel steps only
+    ((512, 256, 512, 768, 8, 64, 512, [8, 5, 4, 3]), 4, 2),    # 256-channel steps, the last block's 32 channels over many rows
+]
+
+
+@pytest.mark.parametrize("shape,n,chunk", CASES)
+@pytest.mark.parametrize("precision", ["fp32", "bf16"])
+def test_conv_tiles_against_fp32(dev, shape, n, chunk, precision):  # noqa: F811
+    from vox_serve_amd.tokenizer.qwen3_codec import Qwen3CodecConfig, Qwen3TTSDecoder
+    cfg = cfg_of(*shape)
+    W = CR.random_codec_weights(cfg, seed=7)
+    g = torch.Generator().manual_seed(5)
+    codes = torch.randint(0, cfg.codebook_size, (n, cfg.num_quantizers, 3 * chunk), generator=g)
+    ref = oracle_exact(cfg, W, codes, chunk)
+    pc = Qwen3CodecConfig(**{k: getattr(cfg, k) for k in Qwen3CodecConfig.__dataclass_fields__})
+    dec = Qwen3TTSDecoder(W, pc, device=dev, max_batch=n, max_slots=n, detokenize_interval=chunk, operand_precision=precision)
+    cache = dec.init_cache(n)
+    got = torch.cat([dec.decode_chunk(codes[:, :, t:t + chunk], cache)[0].cpu().clone() for t in range(0, 3 * chunk, chunk)], -1).numpy()
+    assert got.shape == ref.shape and rms(ref) > 1e-3
+    assert rms(got - ref) < (1e-4 if precision == "fp32" else 2 ** 8 * 1e-4), (rms(got - ref), rms(ref))
+    dec.close()

@@ -211,11 +211,7 @@ __global__ __launch_bounds__(256, (WM * WN > 12 ? 3 : 4)) void k_conv_gemm(ConvG
                 if (st >= a.L) arow = nullptr;
                 else if (st >= 0) arow = a.x + ((size_t)a_b[i] * a.L + st) * a.Cin;
                 else if (a.state && a.P + st >= 0) arow = a.state + ((size_t)a.slots[a_b[i]] * a.P + (a.P + st)) * a.Cin;
-                if (arow && a.x_s2) {          // (v0, v1) = the 8 h terms and the 8 m terms
-                    const bf16_t* r16 = reinterpret_cast<const bf16_t*>(arow);
-                    v0[i] = *reinterpret_cast<const float4*>(r16 + c0 + seg * 8);
-                    v1[i] = *reinterpret_cast<const float4*>(r16 + a.Cin + c0 + seg * 8);
-                } else if (arow) {
+                if (arow) {
                     v0[i] = *reinterpret_cast<const float4*>(arow + c0 + seg * 8);
                     v1[i] = *reinterpret_cast<const float4*>(arow + c0 + seg * 8 + 4);
                 }
@@ -244,16 +240,11 @@ __global__ __launch_bounds__(256, (WM * WN > 12 ? 3 : 4)) void k_conv_gemm(ConvG
             const int idx = tid + 256 * i;
             if (idx < BM * SEG) {
                 const int o = (idx / SEG) * LD + (idx % SEG) * 8;
-                if (a.x_s2) {
-                    *reinterpret_cast<float4*>(&As[0][o]) = v0[i];
-                    *reinterpret_cast<float4*>(&As[1][o]) = v1[i];
-                } else {
-                    uint4 h, m, l;
-                    split3(v0[i], v1[i], h, m, l);
-                    *reinterpret_cast<uint4*>(&As[0][o]) = h;
-                    if ((NP ? NP : a.planes) > 1) *reinterpret_cast<uint4*>(&As[1][o]) = m;
-                    if ((NP ? NP : a.planes) > 2) *reinterpret_cast<uint4*>(&As[2][o]) = l;
-                }
+                uint4 h, m, l;
+                split3(v0[i], v1[i], h, m, l);
+                *reinterpret_cast<uint4*>(&As[0][o]) = h;
+                if ((NP ? NP : a.planes) > 1) *reinterpret_cast<uint4*>(&As[1][o]) = m;
+                if ((NP ? NP : a.planes) > 2) *reinterpret_cast<uint4*>(&As[2][o]) = l;
             }
         }
 #pragma unroll
@@ -402,20 +393,8 @@ __device__ __forceinline__ void conv_taps_kloop(const ConvGemmArgs& a, int H, un
     }
 }
 
-template <int WM, int WN>
-__global__ __launch_bounds__(256, (WM * WN >= 12 ? 3 : 4)) void k_conv_taps(ConvGemmArgs a, int H) {
-    constexpr int BM = 32 * WM, BN = 32 * WN;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
-    const int wm = (wave >> 1) * 16 * WM, wn = (wave & 1) * 16 * WN;
-    f32x4 acc[WM][WN];
-    conv_taps_kloop<WM, WN>(a, H, smem_raw, acc, m0, n0);
-    conv_epilogue<WM, WN>(a, acc, m0, n0, wm, wn, lane);
-}
-
 // A whole residual unit of the decoder in ONE kernel:  h += conv2(act2(conv1(x)))  and  out2 = act_next(h)  — conv1 = the dilated 7-tap
-// conv over S2 rows (k_conv_taps' K loop), conv2 = the 1-tap C -> C conv.  The block's tile covers ALL C output channels of conv1, so the
+// conv over S2 rows (conv_taps_kloop), conv2 = the 1-tap C -> C conv.  The block's tile covers ALL C output channels of conv1, so the
 // activated intermediate (the whole K of conv2) is on chip: it goes from the accumulators through Snake + the two-term split into LDS
 // as the A operand of the second GEMM instead of to HBM and back (per unit at 614 k rows x 96 channels: 236 MB written + 236 MB read).
 // Accumulation orders are those of the two kernels it replaces (conv2: 32-channel chunks in order, the m term before the h term), so the
@@ -521,6 +500,313 @@ __device__ __forceinline__ void ln_row_stats(const float* row, int C, int l16, f
     rstd = rsqrtf(vs / (float)C + eps);
 }
 
+// ================================================================================================
+// Convolutions over S2 rows through LDS DMA.  BM x BN outputs per block of WM x WN x WK waves; K is walked tap by tap in steps of BK
+// channels.  A step's NP x BM activation rows (a row may lie in the chunk, in the history or in neither) and BN weight rows go from memory
+// straight into one of S LDS stages (global_load_lds, 1 KB per wave instruction); S - 1 steps are in flight and no register holds them.
+// One wait + barrier per step: every wave's part of the step has landed, and nobody reads the stage of the step before any more.  16-byte
+// pieces lie swizzled by row (in the address that each lane reads), so the fragment reads of 16 rows do not meet in a bank.
+// WK > 1: the waves share the 32-channel slices of a step and add their sums through LDS at the end — a call of a few rows then has
+// every wave of a CU at work on one small tile.
+// EPI: 0, CONV_GELU, or CONV_GLU: columns come in pairs (n, N + n) of w, out2 <- S2 of silu(v[n]) * v[N + n], N columns.
+// The weights are the MFMA's first operand, so a lane ends with 4 (8) neighbouring channels of one row: the residual, the constants and both
+// outputs move in 16-byte accesses without a lane exchange.  With a lane per column the same epilogue cost more than the products of the
+// one-tap convs (us, rows x channels, residual + h + activation: 51 200 x 384 134 -> 67, 204 800 x 192 240 -> 175 = 3.6 TB/s).
+// Bound: few rows, the chain of steps (one L2 trip for the first, ~0.2 us for each further); many rows, the L2 -> LDS path beside the
+// matrix cores (1.27 PFLOP/s at 10 240 rows, 768 x 7 x 768, one 128 x 256 tile per CU).
+// Extra blocks behind the tiles write a history that an earlier launch was the last to read (ConvDmaArgs::job).
+// ================================================================================================
+struct ConvJob {           // history rows <- the last P rows of [history ++ x], n requests of L rows; C: floats per row
+    float* state;
+    const float* x;
+    int L, P, C, n;
+};
+struct ConvDmaArgs : ConvGemmArgs {
+    int tm, tn, tiles8, mfast;      // tiles along M and N; their number rounded up to 8; 1: the blocks of an XCD walk the rows first
+    const float* rms_x;    // fp32 rows [M, Cin] whose 1 / rms scales the sums of row m (the rows' RMSNorm, its weight already in x), or NULL
+    float rms_eps;
+    const float* nw;       // out2 <- S2 of v * nw[n] (no activation), or NULL
+    ConvJob job;
+};
+__device__ uint4 g_conv_zero_row[1];        // what a tap reads outside the chunk and its history
+// (m0 holds the LDS address of the instruction; nothing else in the kernels that use it does)
+__device__ __forceinline__ void conv_dma16(const char* p, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+}
+typedef f32x4 f32x4_a4 __attribute__((aligned(4)));       // (per-channel constants are where the caller's tensors have them)
+// W neighbouring channels of a row as its two terms
+template <int W>
+__device__ __forceinline__ void conv_put_s2(bf16_t* row, int width, int c, const float (&v)[W]) {
+    unsigned h[W / 2], m[W / 2];
+#pragma unroll
+    for (int e = 0; e < W / 2; ++e) {
+        h[e] = pack_bf2(v[2 * e], v[2 * e + 1]);
+        m[e] = pack_bf2(v[2 * e] - bflo(h[e]), v[2 * e + 1] - bfhi(h[e]));
+    }
+    if constexpr (W == 8) {
+        *reinterpret_cast<uint4*>(row + c) = make_uint4(h[0], h[1], h[2], h[3]);
+        *reinterpret_cast<uint4*>(row + width + c) = make_uint4(m[0], m[1], m[2], m[3]);
+    } else {
+        *reinterpret_cast<uint2*>(row + c) = make_uint2(h[0], h[1]);
+        *reinterpret_cast<uint2*>(row + width + c) = make_uint2(m[0], m[1]);
+    }
+}
+// The epilogue of W neighbouring channels (n ..) of MT rows (m, m + 16, ..) that one lane holds: constants once, every row's residual
+// requested ahead of the first store, 16-byte accesses throughout.
+template <bool GELU, int W, int MT>
+__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n) {
+    if (n >= a.N) return;          // (N and the group width are multiples of W)
+    float b[W], s[W], al[W], ib[W], nw[W], rs[MT][W];
+    const auto fetch = [](float (&d)[W], const float* p) {
+#pragma unroll
+        for (int q = 0; q < W / 4; ++q) {
+            const f32x4 t = *reinterpret_cast<const f32x4_a4*>(p + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
+        }
+    };
+    const int cj = a.out2 ? n / a.sn_mod : 0, cc = n - cj * a.sn_mod;      // (a transposed conv's N = r * sn_mod outputs: r consumer rows)
+    if (a.bias) fetch(b, a.bias + n % a.bias_mod);
+    if (a.scale) fetch(s, a.scale + n);
+    if (a.sn_alpha) { fetch(al, a.sn_alpha + cc); fetch(ib, a.sn_invb + cc); }
+    if (a.nw) fetch(nw, a.nw + n);
+    if (a.res)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+            if (m + 16 * i < a.M) fetch(rs[i], a.res + (size_t)(m + 16 * i) * a.N + n);
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const size_t o = (size_t)(m + 16 * i) * a.N + n;
+        if (m + 16 * i >= a.M) continue;
+        const float rr = rms ? rms[16 * i] : 1.0f;
+        float v[W];
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+            v[e] = acc[i][e / 4][e % 4];
+            if (rms) v[e] *= rr;
+            if (a.bias) v[e] += b[e];
+            if (GELU) v[e] = 0.5f * v[e] * (1.0f + erff(v[e] * 0.70710678118654752440f));
+            if (a.scale) v[e] = s[e] * v[e];
+            if (a.res) v[e] = rs[i][e] + v[e];
+        }
+        if (a.out)
+#pragma unroll
+            for (int q = 0; q < W / 4; ++q) *reinterpret_cast<float4*>(a.out + o + 4 * q) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        if (!a.out2) continue;
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+            if (a.sn_alpha) v[e] = snake_f(v[e], al[e], ib[e]);
+            else if (a.nw) v[e] *= nw[e];
+        }
+        if (a.out2_s2) {
+            conv_put_s2<W>(reinterpret_cast<bf16_t*>(a.out2 + (size_t)(m + 16 * i) * a.N) + (size_t)cj * 2 * a.sn_mod, a.sn_mod, cc, v);
+        } else {
+#pragma unroll
+            for (int q = 0; q < W / 4; ++q) *reinterpret_cast<float4*>(a.out2 + o + 4 * q) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
+        }
+    }
+}
+__device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x4 u, float rms, int m, int n) {
+    if (n >= a.N || m >= a.M) return;
+    float v[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const float gv = g[e] * rms, uv = u[e] * rms;
+        v[e] = (gv / (1.0f + expf(-gv))) * uv;
+    }
+    conv_put_s2<4>(reinterpret_cast<bf16_t*>(a.out2 + (size_t)m * a.N), a.N, n, v);
+}
+#define CONV_GELU 1
+#define CONV_GLU 2
+template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI>
+__global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
+    constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8;
+    constexpr int SA = NP * BM * BK * 2, SB = BN * BK * 2, ST = SA + SB, CA = SA / 1024, CB = SB / 1024;
+    constexpr bool PAIR = EPI != CONV_GLU && NT % 2 == 0;
+    constexpr int NA = (CA + NWV - 1) / NWV, NB = (CB + NWV - 1) / NWV;      // (where the waves do not divide them some chunks are asked for twice)
+    static_assert(SA % 1024 == 0 && SB % 1024 == 0 && KS % WK == 0 && (BM * PPR) % 64 == 0, "whole wave instructions");
+    static_assert(WK == 1 || NWV * MT * NT * 1024 <= S * ST, "partial sums");
+    static_assert((BK & (BK - 1)) == 0 && (EPI != CONV_GLU || NT % 2 == 0), "swizzle; gate and up columns in one lane");
+    extern __shared__ __attribute__((aligned(1024))) char conv_lds[];
+    __shared__ float rms_s[BM];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.x >= a.tiles8) {
+        // new history = last P rows of [history ++ x]; one thread per (request, channel), rows ascending (in place)
+        const ConvJob& j = a.job;
+        const int per = (j.C + 64 * NWV - 1) / (64 * NWV), e0 = (int)blockIdx.x - a.tiles8, b = e0 / per, c = (e0 % per) * 64 * NWV + tid;
+        if (c >= j.C) return;
+        float* s = j.state + (size_t)a.slots[b] * j.P * j.C + c;
+        const float* x = j.x + (size_t)b * j.L * j.C + c;
+#pragma unroll 6
+        for (int i = 0; i < j.P; ++i) {
+            const int e = j.L + i;
+            s[(size_t)i * j.C] = e < j.P ? s[(size_t)e * j.C] : x[(size_t)(e - j.P) * j.C];
+        }
+        return;
+    }
+    const int t = ((int)blockIdx.x & 7) * (a.tiles8 >> 3) + ((int)blockIdx.x >> 3);
+    if (t >= a.tm * a.tn) return;
+    const int m0 = (a.mfast ? t % a.tm : t / a.tn) * BM, n0 = (a.mfast ? t / a.tm : t % a.tn) * BN;      // (glu: n0 counts gate and up columns)
+    const int wk = wv % WK, wmn = wv / WK, wm = wmn / WN, wn = wmn % WN, fr = lane & 15, fk = lane >> 4;
+    const int rb = a.Cin * 4;
+    // The weights are the first operand of the MFMA: a lane's four sums are neighbouring channels of one row.  PAIR: tiles j and j + 1 take the
+    // weight rows 8 q + 0..3 and 8 q + 4..7 (q = 0..3), so that they hold eight neighbouring channels together.
+    const auto wswz = [](int r) {
+        if (PAIR) return BK == 32 ? ((r >> 1) & 1) | ((r >> 2) & 2) : (r & 3) | ((r >> 1) & 4);
+        return BK == 32 ? (r >> 1) & 3 : r & 7;
+    };
+    // per DMA instruction of the wave: the lane's row of the chunk (its time), that row in x and the row that time 0 would have in the history
+    const char *xp[NA], *sp[NA], *cur[NA], *wp[NB];
+    int ts[NA], step[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int q = (i * NWV + wv) % CA * 64 + lane, pl = q / (BM * PPR), r = q / PPR % BM, pc = (q % PPR) ^ (BK == 32 ? (r >> 1) & 3 : r & 7);
+        int m = m0 + r;
+        m = m < a.M ? m : a.M - 1;                  // (rows past the end repeat the last one: nothing of them is stored)
+        const int b = m / a.L;
+        ts[i] = m - b * a.L;
+        xp[i] = reinterpret_cast<const char*>(a.x) + (size_t)m * rb + pl * a.Cin * 2 + pc * 16;
+        sp[i] = a.state ? reinterpret_cast<const char*>(a.state) + ((size_t)a.slots[b] * a.P + a.P + ts[i]) * rb + pl * a.Cin * 2 + pc * 16 : nullptr;
+    }
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const int q = (i * NWV + wv) % CB * 64 + lane, r = q / PPR, pc = (q % PPR) ^ wswz(r);
+        int n = n0 + r;
+        if (EPI == CONV_GLU) {
+            n = (n0 >> 1) + (r >> 5) * 16 + (r & 15);
+            n = (n < a.N ? n : a.N - 1) + ((r >> 4) & 1) * a.N;
+        } else {
+            n = n < a.N ? n : a.N - 1;
+        }
+        wp[i] = reinterpret_cast<const char*>(a.w) + ((size_t)n * a.Cin + pc * 8) * 2;
+    }
+    const int nck = a.Cin / BK, nit = a.n_taps * nck;
+    const size_t wtap = (size_t)(EPI == CONV_GLU ? 2 * a.N : a.N) * a.Cin * 2 - (size_t)a.Cin * 2;      // from the end of one tap's row to the next tap's
+    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)conv_lds;
+    auto tap_rows = [&](int tap) {
+        const int off = a.off[tap];
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            const int e = ts[i] - off;
+            const bool in = e >= 0 && e < a.L, hist = e < 0 && a.state && a.P + e >= 0;
+            cur[i] = in ? xp[i] - (ptrdiff_t)off * rb : hist ? sp[i] - (ptrdiff_t)off * rb : reinterpret_cast<const char*>(g_conv_zero_row);
+            step[i] = in || hist ? BK * 2 : 0;
+        }
+    };
+    int rt = 0, rc = 0, rq = 0;      // tap, chunk and number of the next request
+    tap_rows(0);
+    auto request = [&](int stage) {
+        const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * ST);
+#pragma unroll
+        for (int i = 0; i < NA; ++i) conv_dma16(cur[i], ls + (i * NWV + wv) % CA * 1024);
+#pragma unroll
+        for (int i = 0; i < NB; ++i) conv_dma16(wp[i], ls + SA + (i * NWV + wv) % CB * 1024);
+        if (++rq >= nit) return;     // (past the last step the same one is asked for again: the count in flight stays the same)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) cur[i] += step[i];
+#pragma unroll
+        for (int i = 0; i < NB; ++i) wp[i] += BK * 2;
+        if (++rc == nck) {
+            rc = 0;
+            tap_rows(++rt);
+#pragma unroll
+            for (int i = 0; i < NB; ++i) wp[i] += wtap;
+        }
+    };
+#pragma unroll
+    for (int s = 0; s < S - 1; ++s) request(s);
+    if (a.rms_x) {
+        for (int r = wv; r < BM; r += NWV) {
+            const int m = m0 + r < a.M ? m0 + r : a.M - 1;
+            const float4* x4 = reinterpret_cast<const float4*>(a.rms_x + (size_t)m * a.Cin);
+            float s = 0.0f;
+            for (int c = lane; c < a.Cin / 4; c += 64) {
+                const float4 v = x4[c];
+                s += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+            }
+            for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
+            if (lane == 0) rms_s[r] = rsqrtf(s / (float)a.Cin + a.rms_eps);
+        }
+    }
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    const int wfr = PAIR ? (fr >> 2) * 8 + (fr & 3) : fr;
+    int stage = 0;
+    for (int it = 0; it < nit; ++it) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NB)) : "memory");
+        request(stage == 0 ? S - 1 : stage - 1);
+        const char *as = conv_lds + stage * ST + (wm * MT * 16 + fr) * BK * 2, *bs = conv_lds + stage * ST + SA + (wn * NT * 16 + wfr) * BK * 2;
+#pragma unroll
+        for (int k = 0; k < KS / WK; ++k) {
+            const int piece = (((wk * (KS / WK) + k) * 4 + fk) ^ (BK == 32 ? (fr >> 1) & 3 : fr & 7)) * 16;
+            const int wpiece = (((wk * (KS / WK) + k) * 4 + fk) ^ wswz(wfr)) * 16;
+            cbf16x8 bf[NT];
+#pragma unroll
+            for (int j = 0; j < NT; ++j) bf[j] = *reinterpret_cast<const cbf16x8*>(bs + (PAIR ? (j >> 1) * 32 + (j & 1) * 4 : j * 16) * BK * 2 + wpiece);
+#pragma unroll
+            for (int p = NP - 1; p >= 0; --p) {
+                cbf16x8 af[MT];
+#pragma unroll
+                for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const cbf16x8*>(as + (p * BM + i * 16) * BK * 2 + piece);
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
+            }
+        }
+        stage = stage == S - 1 ? 0 : stage + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");        // (the repeated last steps: nothing may land any more)
+    constexpr int FR = MT * NT;
+    f32x4* part = reinterpret_cast<f32x4*>(conv_lds) + (size_t)wmn * WK * FR * 64 + lane;
+    if (WK > 1) {
+#pragma unroll
+        for (int f = 0; f < FR; ++f) part[(wk * FR + f) * 64] = acc[f / NT][f % NT];
+        __syncthreads();
+    }
+    auto sum = [&](int f) {
+        if (WK == 1) return acc[f / NT][f % NT];
+        f32x4 v = part[f * 64];
+#pragma unroll
+        for (int k = 1; k < WK; ++k) v += part[(k * FR + f) * 64];
+        return v;
+    };
+    const int rl = wm * MT * 16 + fr, nl = n0 + wn * NT * 16;
+    if constexpr (EPI == CONV_GLU) {
+#pragma unroll
+        for (int f = 0; f < FR; f += 2)
+            if (WK == 1 || (f / 2) % WK == wk)
+                conv_dma_glu(a, sum(f), sum(f + 1), rms_s[rl + f / NT * 16], m0 + rl + f / NT * 16, (nl >> 1) + f % NT * 8 + fk * 4);
+    } else {
+        constexpr int P = PAIR ? 2 : 1;
+        const float* rms = a.rms_x ? rms_s + rl : nullptr;
+#pragma unroll
+        for (int j = 0; j < NT; j += P) {
+            const int n = nl + j * 16 + fk * 4 * P;
+            if constexpr (WK == 1) {
+                f32x4 v[MT][P];
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+#pragma unroll
+                    for (int q = 0; q < P; ++q) v[i][q] = acc[i][j + q];
+                conv_dma_out<EPI == CONV_GELU, 4 * P, MT>(a, v, rms, m0 + rl, n);
+            } else {
+#pragma unroll
+                for (int i = 0; i < MT; ++i)
+                    if ((i * (NT / P) + j / P) % WK == wk) {
+                        f32x4 v[1][P];
+#pragma unroll
+                        for (int q = 0; q < P; ++q) v[0][q] = sum(i * NT + j + q);
+                        conv_dma_out<EPI == CONV_GELU, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
+                    }
+            }
+        }
+    }
+}
+
 // Few-row variant (M <= 48: the transformer and the first upsampling stages of a single request's chunk): tile
 // 16(M) x 64(N), one n-tile per wave, K walked in BK-wide chunks (128 where Cin allows) with the same one-step
 // register prefetch.  These stages run a handful of blocks: time = number of dependent K steps, so the steps are wide.
@@ -551,14 +837,7 @@ __global__ __launch_bounds__(256) void k_conv_gemm_skinny(ConvGemmArgs a) {
                 if (st >= a.L) arow = nullptr;
                 else if (st >= 0) arow = a.x + ((size_t)ab * a.L + st) * a.Cin;
                 else if (a.state && a.P + st >= 0) arow = a.state + ((size_t)a.slots[ab] * a.P + (a.P + st)) * a.Cin;
-                if (arow && a.x_s2) {          // (xy, zw) = the 4 h terms and the 4 m terms
-                    const bf16_t* r16 = reinterpret_cast<const bf16_t*>(arow);
-                    const float2 h2 = *reinterpret_cast<const float2*>(r16 + c0 + seg * 4);
-                    const float2 m2 = *reinterpret_cast<const float2*>(r16 + a.Cin + c0 + seg * 4);
-                    av[i] = make_float4(h2.x, h2.y, m2.x, m2.y);
-                } else if (arow) {
-                    av[i] = *reinterpret_cast<const float4*>(arow + c0 + seg * 4);
-                }
+                if (arow) av[i] = *reinterpret_cast<const float4*>(arow + c0 + seg * 4);
             }
         }
 #pragma unroll
@@ -584,11 +863,7 @@ __global__ __launch_bounds__(256) void k_conv_gemm_skinny(ConvGemmArgs a) {
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int idx = tid + 256 * i;
-            if (idx < 16 * SEGA && a.x_s2 && !LN) {
-                const int o = (idx / SEGA) * LD + (idx % SEGA) * 4;
-                *reinterpret_cast<float2*>(&As[0][o]) = make_float2(av[i].x, av[i].y);
-                *reinterpret_cast<float2*>(&As[1][o]) = make_float2(av[i].z, av[i].w);
-            } else if (idx < 16 * SEGA) {      // 4 fp32 -> 4 bf16 per plane (8 bytes)
+            if (idx < 16 * SEGA) {      // 4 fp32 -> 4 bf16 per plane (8 bytes)
                 float x4[4] = {av[i].x, av[i].y, av[i].z, av[i].w};
                 if (LN) {
                     const int r = idx / SEGA, c = (it % nck) * BK + (idx % SEGA) * 4;
@@ -852,22 +1127,31 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
 // ================================================================================================
 // small kernels
 // ================================================================================================
+// element c of row `row` of a C-wide activation: fp32, or the two terms of an S2 row
+__device__ __forceinline__ void put_row(float* y, size_t row, int C, int c, float v, int s2) {
+    if (s2) {
+        bf16_t* r16 = reinterpret_cast<bf16_t*>(y + row * C);
+        split2(v, r16[c], r16[C + c]);
+    } else {
+        y[row * C + c] = v;
+    }
+}
 // RVQ decode: q0 = emb[0][code0], qr = sum_{k>=1} emb[k][code_k] (sequential in k)      qwen3_codec.py:1204-1210
 __global__ __launch_bounds__(256) void k_rvq(const int* codes, int code_stride, const float* emb, int Q, int bins, int vq,
-                                             float* q0, float* qr) {
+                                             float* q0, float* qr, int s2) {
     const int row = blockIdx.x;
     const int* cr = codes + (size_t)row * code_stride;
     for (int d = threadIdx.x; d < vq; d += 256) {
         int c0 = cr[0];
         c0 = c0 < 0 ? 0 : (c0 >= bins ? bins - 1 : c0);          // postprocess clamps to [0, bins-1] (qwen3_tts.py:2027)
-        q0[(size_t)row * vq + d] = emb[((size_t)c0) * vq + d];
+        put_row(q0, row, vq, d, emb[((size_t)c0) * vq + d], s2);
         float s = 0.0f;
         for (int k = 1; k < Q; ++k) {
             int c = cr[k];
             c = c < 0 ? 0 : (c >= bins ? bins - 1 : c);
             s = s + emb[((size_t)k * bins + c) * vq + d];
         }
-        qr[(size_t)row * vq + d] = s;
+        put_row(qr, row, vq, d, s, s2);
     }
 }
 
@@ -945,7 +1229,7 @@ __global__ __launch_bounds__(256) void k_codec_rope_kv(float* qkv, bf16_t* ring,
 // One block per (head, request): K/V ring tile in LDS (row stride D+1: conflict-free both for "lane = key" in the
 // scores and "lane = dim" in PV), the T queries of the chunk spread over the four waves.
 __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16_t* ring, const int* slots, const long* pos,
-                                                    float* out, int T, int H, int D, int Wn) {
+                                                    float* out, int T, int H, int D, int Wn, int s2) {
     extern __shared__ float sm[];   // K [Wn][D+1], V [Wn][D+1], Q [T][D], P [4][Wn]
     const int LD = D + 1;
     float* Ks = sm;
@@ -1000,7 +1284,7 @@ __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16
         for (int d = lane; d < D; d += 64) {
             float o = 0.0f;
             for (int j = 0; j < nvis; ++j) o = fmaf(P[j], Vs[j * LD + d], o);
-            out[((size_t)(b * T + i)) * HD + (size_t)h * D + d] = o / ls;
+            put_row(out, (size_t)(b * T + i), HD, h * D + d, o / ls, s2);
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
@@ -1017,7 +1301,7 @@ __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16
 // (profiles/round4_codec_attn_ab.txt).
 template <int D>
 __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* ring, const int* slots, const long* pos, float* out, int T,
-                                                     int H, int Wn, const float* inv_freq) {
+                                                     int H, int Wn, const float* inv_freq, int s2) {
     extern __shared__ float sm[];   // K [Wn][D+1], V [Wn][D+1], Q [T][D], P [T][Wn]
     constexpr int LD = D + 1, half = D / 2, CH = D / 8;
     float* Ks = sm;
@@ -1115,7 +1399,7 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
                 for (int u = 0; u < 8; ++u) o = fmaf(pv[u], vv[u], o);
             }
             for (; j < nvis; ++j) o = fmaf(P[j], Vs[j * LD + d], o);
-            out[((size_t)(b * T + i)) * HD + (size_t)h * D + d] = o / ls;
+            put_row(out, (size_t)(b * T + i), HD, h * D + d, o / ls, s2);
         }
     }
 }
@@ -1139,7 +1423,7 @@ __global__ __launch_bounds__(256) void k_silu_mul_f32(const float* gu, float* h,
 // ConvNeXt front: causal depthwise conv k=7 (+bias) then LayerNorm over channels.   qwen3_codec.py:447-450
 __global__ __launch_bounds__(256) void k_dwconv_ln(const float* x, const float* state, const int* slots, const float* w,
                                                    const float* wb, const float* lnw, const float* lnb, float* y, int L,
-                                                   int C, float eps) {
+                                                   int C, float eps, int s2) {
     __shared__ float red[4];
     extern __shared__ float ybuf[];   // [C]
     const int row = blockIdx.x, b = row / L, t = row % L;
@@ -1157,13 +1441,13 @@ __global__ __launch_bounds__(256) void k_dwconv_ln(const float* x, const float* 
         s1 += acc;
     }
     const float mean = block_sum(s1, red) / (float)C;
-    float s2 = 0.0f;
+    float sq = 0.0f;
     for (int c = threadIdx.x; c < C; c += 256) {
         const float d = ybuf[c] - mean;
-        s2 += d * d;
+        sq += d * d;
     }
-    const float rstd = rsqrtf(block_sum(s2, red) / (float)C + eps);
-    for (int c = threadIdx.x; c < C; c += 256) y[(size_t)row * C + c] = (ybuf[c] - mean) * rstd * lnw[c] + lnb[c];
+    const float rstd = rsqrtf(block_sum(sq, red) / (float)C + eps);
+    for (int c = threadIdx.x; c < C; c += 256) put_row(y, (size_t)row, C, c, (ybuf[c] - mean) * rstd * lnw[c] + lnb[c], s2);
 }
 
 // final causal conv k=7, C -> 1, + clamp(-1,1).  One wave per output sample group.
@@ -1290,31 +1574,23 @@ static int rows_nt_tiles(int which) {
     static const int v4 = [] { const char* e = getenv("VOX_ROWS_NT4"); return e ? atoi(e) : 2048; }();
     return which ? v4 : v2;
 }
-// VOX_CONV_TAPS=0: the per-tap staging kernel for every multi-tap conv (A/B timing)
-static bool conv_taps_on() {
-    static const bool on = [] { const char* e = getenv("VOX_CONV_TAPS"); return !(e && e[0] == '0'); }();
-    return on;
-}
 static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const float* state, const int* slots, int n,
                      int L, int P, const int* offs, float* out, const float* res, const float* scale, int gelu,
                      float* out2 = nullptr, const vox_snake_w* sn = nullptr, int sn_mod = 0, const float* rscale = nullptr,
-                     const float* ln_w = nullptr, const float* ln_b = nullptr, float ln_eps = 0.0f, int x_s2 = 0, int out2_s2 = 0) {
+                     const float* ln_w = nullptr, const float* ln_b = nullptr, float ln_eps = 0.0f) {
     if (w.cin % CG_BK) return vox_fail(VOX_ERR_INVALID, "codec gemm: Cin %d %% %d != 0", w.cin, CG_BK);
     if (w.n_taps > CG_MAXTAPS) return vox_fail(VOX_ERR_INVALID, "codec gemm: too many taps");
     ConvGemmArgs a{};
     a.x = x; a.state = state; a.slots = slots; a.w = (const bf16_t*)w.w; a.bias = w.bias; a.res = res; a.scale = scale;
     a.out = out; a.M = n * L; a.N = w.n; a.Cin = w.cin; a.L = L; a.P = P; a.n_taps = w.n_taps; a.rscale = rscale;
-    a.planes = x_s2 ? 2 : g_conv_planes;
-    a.x_s2 = x_s2; a.out2_s2 = (out2 && sn) ? out2_s2 : 0;
+    a.planes = g_conv_planes;
 #ifdef VOX_DEV_KNOBS
     { static const int dv = [] { const char* e = getenv("VOX_CODEC_DEV"); return e ? atoi(e) : 0; }(); a.dev = dv; }
 #endif
-    if (x_s2 && ln_w) return vox_fail(VOX_ERR_INVALID, "codec gemm: S2 rows with a fused LayerNorm");
-    if (a.out2_s2 && ((w.n & 1) || ((sn_mod > 0 ? sn_mod : w.n) & 1))) return vox_fail(VOX_ERR_INVALID, "codec gemm: S2 output needs an even channel count");
     a.bias_mod = w.bias_mod > 0 ? w.bias_mod : w.n; a.gelu = gelu;
     if (out2 && sn) { a.out2 = out2; a.sn_alpha = sn->alpha; a.sn_invb = sn->inv_beta; a.sn_mod = sn_mod > 0 ? sn_mod : w.n; }
     for (int k = 0; k < w.n_taps; ++k) a.off[k] = offs ? offs[k] : 0;
-    if (g_conv_rows_gemm && rows_gemm_on() && !x_s2 && a.M <= g_conv_skinny_rows && w.cin % 32 == 0 && (w.n_taps * w.cin) % 128 == 0 && (!ln_w || (w.n_taps == 1 && a.off[0] == 0))) {
+    if (g_conv_rows_gemm && rows_gemm_on() && a.M <= g_conv_skinny_rows && w.cin % 32 == 0 && (w.n_taps * w.cin) % 128 == 0 && (!ln_w || (w.n_taps == 1 && a.off[0] == 0))) {
         // every operand requested up front, K split over the block's waves (k_rows_gemm): 8 waves from K = 512 on
         const int K = w.n_taps * w.cin, wv = (K >= 512 && K % 256 == 0 && rows_wv8_on()) ? 8 : 4, kb = K / (32 * wv);
         const int tiles = ((w.n + 15) / 16) * ((a.M + 15) / 16);
@@ -1364,24 +1640,6 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
     // fragment read then feeds 3-4 MFMAs instead of 2 (the 64 x 64 tile is LDS-read bound with the 3-term split)
     {
         const int wnb = (w.n % 128 == 0 || w.n >= 256) ? 4 : ((w.n > 64 && w.n <= 96) || w.n % 96 == 0) ? 3 : 0;
-        // S2 rows and several taps: the activation tile is staged once per 32-channel chunk for all taps (k_conv_taps); 128-row tiles when
-        // they fill the chip and divide the request length, else 64-row tiles
-        if (wnb && x_s2 && w.n_taps > 1 && conv_taps_on()) {
-            int H = 0, omin = 0;
-            for (int k = 0; k < w.n_taps; ++k) { H = a.off[k] > H ? a.off[k] : H; omin = a.off[k] < omin ? a.off[k] : omin; }
-            const int ncb = (w.n + 32 * wnb - 1) / (32 * wnb);
-            // (below ~256 blocks the per-tap kernels' smaller tiles win: measured at 1 and 4 requests)
-            const int bm = (L % 128 == 0 && ncb * (a.M / 128) >= 256) ? 128 : ((L % 64 == 0 && ncb * (a.M / 64) >= 256) ? 64 : 0);
-            if (bm && omin >= 0 && H <= 64) {
-                const dim3 gt(ncb, a.M / bm);
-                const size_t lds = (size_t)(2 * (bm + H) + 2 * 32 * wnb) * 80;
-                if (bm == 128 && wnb == 4) hipLaunchKernelGGL((k_conv_taps<4, 4>), gt, dim3(256), lds, st, a, H);
-                else if (bm == 128) hipLaunchKernelGGL((k_conv_taps<4, 3>), gt, dim3(256), lds, st, a, H);
-                else if (wnb == 4) hipLaunchKernelGGL((k_conv_taps<2, 4>), gt, dim3(256), lds, st, a, H);
-                else hipLaunchKernelGGL((k_conv_taps<2, 3>), gt, dim3(256), lds, st, a, H);
-                return VOX_OK;
-            }
-        }
         if (wnb && ((w.n + 32 * wnb - 1) / (32 * wnb)) * ((a.M + 127) / 128) >= 256) {
             const dim3 gb((w.n + 32 * wnb - 1) / (32 * wnb), (a.M + 127) / 128);
             if (wnb == 4) hipLaunchKernelGGL((k_conv_gemm<32, 4, 4>), gb, dim3(256), 0, st, a);
@@ -1408,6 +1666,96 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
     return vox_fail(VOX_ERR_INVALID, "codec gemm: no tile variant");
 }
 
+static void state_update(hipStream_t st, float* state, const int* slots, const float* x, int n, int L, int P, int C) {
+    hipLaunchKernelGGL(k_state_update, dim3((C + 255) / 256, n), dim3(256), 0, st, state, slots, x, L, P, C);
+}
+
+// ---- convolutions over S2 rows (k_conv_dma) ----
+template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI>
+static int conv_dma_launch(hipStream_t st, ConvDmaArgs& a) {
+    constexpr int lds = S * (NP * BM + BN) * BK * 2, threads = 64 * WM * WN * WK;
+    static_assert(lds + BM * 4 <= 160 * 1024, "LDS of a CU");
+    const auto kern = k_conv_dma<BM, BN, WM, WN, WK, BK, S, NP, EPI>;
+    if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    a.tm = (a.M + BM - 1) / BM;
+    a.tn = ((EPI == CONV_GLU ? 2 * a.N : a.N) + BN - 1) / BN;
+    a.tiles8 = (a.tm * a.tn + 7) & ~7;
+    a.mfast = (size_t)a.n_taps * a.N > (size_t)a.M * 2;      // weights larger than rows: each XCD reads its own columns of them
+    const int jobs = a.job.state ? a.job.n * ((a.job.C + threads - 1) / threads) : 0;
+    hipLaunchKernelGGL(kern, dim3(a.tiles8 + jobs), dim3(threads), lds, st, a);
+    return VOX_OK;
+}
+// The smallest tile that leaves no CU a second round (the waves of a block share K): a call of few rows is a chain of dependent steps,
+// and more blocks, fewer columns and more waves per step each shorten it.  Past one 64 x 64 tile per CU the waves take outputs, not K;
+// past two the tile grows (fewer bytes through LDS per product).  us, against the staged kernels, two-term rows (M rows, N x taps x Cin):
+//   M = 10: 3072 x 512 7.1 -> 4.4, 512 x 1024 10.4 -> 4.9 | 40: 1024 x 4096 33 -> 7.8, 1536 x 7 x 1024 58 -> 14, 6144 x 2 x 1536 31 -> 14
+//   M = 320: 768 x 7 x 768 48 -> 16, 1920 x 2 x 768 22 -> 12 | 1600: 384 x 7 x 384 36 -> 18 | 6400: 192 x 7 x 192 30 -> 18.5
+//   M = 1280: 1536 x 7 x 1024 157 -> 72, 6144 x 2 x 1536 157 -> 84 | 10240: 768 x 7 x 768 194 -> 134, 1920 x 2 x 768 168 -> 131
+//   M = 51200: 384 x 7 x 384 250 -> 193 (rounds of 256 tiles decide: 128 x 256 leaves a quarter of its columns empty there, > 245)
+template <int NP, int EPI>
+static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
+    const int n2 = EPI == CONV_GLU ? 2 * a.N : a.N;
+    const auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n2 + bn - 1) / bn); };
+    const bool k64 = a.Cin % 64 == 0, k128 = a.Cin % 128 == 0;      // (other Cin: 32-channel steps, waves take outputs)
+    if (k128) {
+        if constexpr (EPI != CONV_GLU)
+            if (tiles(16, 16) <= 256) return conv_dma_launch<16, 16, 1, 1, 4, 128, 8, NP, EPI>(st, a);
+        if (tiles(16, 32) <= 256) {
+            if (a.Cin % 256 == 0) return conv_dma_launch<16, 32, 1, 1, 8, 256, 4, NP, EPI>(st, a);
+            return conv_dma_launch<16, 32, 1, 1, 4, 128, 6, NP, EPI>(st, a);
+        }
+        if (tiles(16, 64) <= 256) return conv_dma_launch<16, 64, 1, 2, 4, 128, 5, NP, EPI>(st, a);
+        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 4, 128, 4, NP, EPI>(st, a);
+        if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 2, 2, 4, 128, 3, NP, EPI>(st, a);
+    }
+    if (k64) {
+        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 2, 64, 6, NP, EPI>(st, a);
+        if (tiles(64, 64) <= 512) return conv_dma_launch<64, 64, 2, 2, 1, 64, 3, NP, EPI>(st, a);
+    }
+    if constexpr (EPI == 0) {
+        // what the busiest CU multiplies, weighted by how well each tile does it
+        const auto cost = [&](int bm, int bn, double w) { return (double)((tiles(bm, bn) + 255) / 256) * bm * bn * w; };
+        const double c[6] = {cost(128, 256, 1.0), cost(256, 192, 1.0), cost(128, 192, 1.08), cost(128, 128, 1.07), cost(64, 128, 1.17), cost(64, 96, 1.25)};
+        int best = 0;
+        for (int i = 1; i < 6; ++i) best = c[i] < c[best] ? i : best;
+        switch (best) {
+            case 0: return conv_dma_launch<128, 256, 4, 4, 1, 32, 3, NP, EPI>(st, a);
+            case 1: return conv_dma_launch<256, 192, 8, 2, 1, 32, 3, NP, EPI>(st, a);
+            case 2: return conv_dma_launch<128, 192, 4, 2, 1, 32, 2, NP, EPI>(st, a);
+            case 3: return conv_dma_launch<128, 128, 4, 2, 1, 32, 3, NP, EPI>(st, a);
+            case 4:
+                if (k64) return conv_dma_launch<64, 128, 2, 2, 1, 64, 2, NP, EPI>(st, a);
+                return conv_dma_launch<64, 128, 2, 2, 1, 32, 4, NP, EPI>(st, a);
+            default: return conv_dma_launch<64, 96, 4, 1, 1, 32, 4, NP, EPI>(st, a);
+        }
+    }
+    if (k64) return conv_dma_launch<64, 128, 2, 2, 1, 64, 2, NP, EPI>(st, a);
+    return conv_dma_launch<64, 64, 2, 2, 1, 32, 6, NP, EPI>(st, a);
+}
+// The operands and the shape of a conv over S2 rows; the caller adds the epilogue (out / out2 / ...) and hands it to conv_s2.
+static ConvDmaArgs conv_s2_args(const vox_conv_w& w, const float* x, const float* state, const int* slots, int n, int L, int P, const int* offs) {
+    ConvDmaArgs a{};
+    a.x = x; a.state = state; a.slots = slots; a.w = (const bf16_t*)w.w; a.bias = w.bias;
+    a.M = n * L; a.N = w.n; a.Cin = w.cin; a.L = L; a.P = P; a.n_taps = w.n_taps;
+    a.bias_mod = w.bias_mod > 0 ? w.bias_mod : w.n;
+    a.sn_mod = w.n;
+    for (int k = 0; k < w.n_taps && k < CG_MAXTAPS; ++k) a.off[k] = offs ? offs[k] : 0;
+    return a;
+}
+static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
+    if (a.Cin % CG_BK) return vox_fail(VOX_ERR_INVALID, "codec conv: Cin %d %% %d != 0", a.Cin, CG_BK);
+    if (a.n_taps > CG_MAXTAPS) return vox_fail(VOX_ERR_INVALID, "codec conv: too many taps");
+    if (a.N % 16 || a.sn_mod % 8 || a.bias_mod % 8) return vox_fail(VOX_ERR_INVALID, "codec conv: %d channels (groups of %d)", a.N, a.sn_mod);
+    a.planes = g_conv_planes;
+    if (epi == CONV_GLU) {
+        a.N /= 2;
+        a.sn_mod = a.N;
+        return a.planes == 2 ? conv_dma_pick<2, CONV_GLU>(st, a) : conv_dma_pick<1, CONV_GLU>(st, a);
+    }
+    if (epi == CONV_GELU) return a.planes == 2 ? conv_dma_pick<2, CONV_GELU>(st, a) : conv_dma_pick<1, CONV_GELU>(st, a);
+    return a.planes == 2 ? conv_dma_pick<2, 0>(st, a) : conv_dma_pick<1, 0>(st, a);
+}
+
 // A residual unit as ONE launch (k_res_unit) where the tile can cover all channels and the stage has enough rows to fill the chip;
 // *fused = 0 and nothing launched otherwise (the caller then runs the two convs).  x: the S2 activated input rows; h: the fp32
 // residual stream, updated in place; out2: the NEXT consumer's activation of the new h — must not alias x.
@@ -1422,10 +1770,11 @@ static bool res_unit_192() {
     return on;
 }
 static int conv_unit(hipStream_t st, const vox_conv_w& w1, const vox_conv_w& w2, const float* x, const float* state, const int* slots, int n, int L,
-                     int P, const int* offs, const vox_snake_w& act2, float* h, float* out2, const vox_snake_w* nx, int out2_s2, int* fused) {
+                     int P, const int* offs, const vox_snake_w& act2, const float* h, float* ho, float* out2, const vox_snake_w* nx, int out2_s2,
+                     int* fused) {
     *fused = 0;
     const int C = w1.n;
-    if (!res_unit_on() || !conv_taps_on() || g_conv_planes != 2 || w1.n_taps < 2 || w1.n_taps > CG_MAXTAPS || w2.n_taps != 1 || w1.cin != C ||
+    if (!res_unit_on() || g_conv_planes != 2 || w1.n_taps < 2 || w1.n_taps > CG_MAXTAPS || w2.n_taps != 1 || w1.cin != C ||
         w2.cin != C || w2.n != C || (C != 96 && !(C == 192 && res_unit_192())) || out2 == x || !nx)
         return VOX_OK;
     int H = 0, omin = 0;
@@ -1437,7 +1786,7 @@ static int conv_unit(hipStream_t st, const vox_conv_w& w1, const vox_conv_w& w2,
     a1.n_taps = w1.n_taps; a1.planes = 2; a1.x_s2 = 1; a1.bias_mod = w1.bias_mod > 0 ? w1.bias_mod : C;
     a1.sn_alpha = act2.alpha; a1.sn_invb = act2.inv_beta; a1.sn_mod = C;
     for (int k = 0; k < w1.n_taps; ++k) a1.off[k] = offs[k];
-    a2.w = (const bf16_t*)w2.w; a2.bias = w2.bias; a2.res = h; a2.out = h; a2.M = M; a2.N = C; a2.Cin = C; a2.L = L; a2.n_taps = 1; a2.planes = 2;
+    a2.w = (const bf16_t*)w2.w; a2.bias = w2.bias; a2.res = h; a2.out = ho; a2.M = M; a2.N = C; a2.Cin = C; a2.L = L; a2.n_taps = 1; a2.planes = 2;
     a2.x_s2 = 1; a2.bias_mod = w2.bias_mod > 0 ? w2.bias_mod : C; a2.out2 = out2; a2.sn_alpha = nx->alpha; a2.sn_invb = nx->inv_beta; a2.sn_mod = C;
     a2.out2_s2 = out2_s2;
     const size_t p1 = (size_t)(2 * (bm + H) + 2 * C) * 80, p3 = (size_t)2 * bm * (C + 8) * 2 + (size_t)2 * C * 80;
@@ -1464,9 +1813,6 @@ static void snake(hipStream_t st, const float* x, const vox_snake_w& s, float* y
     int grid = (int)((total + 255) / 256);
     if (grid > 4096) grid = 4096;
     hipLaunchKernelGGL(k_snake, dim3(grid), dim3(256), 0, st, x, s.alpha, s.inv_beta, y, total, C);
-}
-static void state_update(hipStream_t st, float* state, const int* slots, const float* x, int n, int L, int P, int C) {
-    hipLaunchKernelGGL(k_state_update, dim3((C + 255) / 256, n), dim3(256), 0, st, state, slots, x, L, P, C);
 }
 
 extern "C" {
@@ -1563,22 +1909,50 @@ int vox_codec_reset_slot(vox_codec* m, void* stream, int slot) {
 }
 
 // codes: int32 [n, T, code_stride] (first num_quantizers columns used); slots: int32 [n]; out: fp32 [n, T*hop]
-int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int code_stride, const int32_t* slots, int n,
-                           int T, float* out) {
-    if (!m || !codes || !slots || !out) return vox_fail(VOX_ERR_INVALID, "codec_decode_chunk: NULL");
-    if (n < 1 || n > m->max_batch || T < 1 || T > m->T) return vox_fail(VOX_ERR_INVALID, "codec_decode_chunk: n=%d T=%d out of range", n, T);
-    m->decoded = true;
-    hipStream_t st = (hipStream_t)stream;
-    struct PlanesGuard { int saved; explicit PlanesGuard(int p) : saved(g_conv_planes) { g_conv_planes = p; } ~PlanesGuard() { g_conv_planes = saved; } } pg(m->planes);
+}  // extern "C"
+
+// RoPE, the ring's new rows and the attention of layer l: qkv fp32 [nL, 3 HD] -> out [nL, HD] (fp32 or S2 rows)
+static void codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* slots, int n, int L, float* qkv, float* out, int s2) {
+    const vox_codec_config& c = m->cfg;
+    const int HD = c.num_heads * c.head_dim;
+    bf16_t* ring = m->ring + (size_t)l * m->max_slots * c.window * 2 * HD;
+    // (VOX_CODEC_ATTN2=0: RoPE / ring write and the attention as two launches — A/B timing; bit-identical)
+    static const bool attn2 = [] { const char* e = getenv("VOX_CODEC_ATTN2"); return !(e && e[0] == '0'); }();
+    const size_t lds2 = (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + L * c.window) * 4;
+    if (attn2 && c.head_dim == 64 && L <= c.window && lds2 <= 64 * 1024) {
+        hipLaunchKernelGGL(k_codec_attn2<64>, dim3(c.num_heads, n), dim3(256), lds2, st, qkv, ring, slots, m->pos, out, L, c.num_heads, c.window,
+                           m->w.inv_freq, s2);
+    } else {
+        hipLaunchKernelGGL(k_codec_rope_kv, dim3(n * L), dim3(256), 0, st, qkv, ring, slots, m->pos, L, c.num_heads, c.head_dim, c.window,
+                           m->w.inv_freq);
+        hipLaunchKernelGGL(k_codec_attn, dim3(c.num_heads, n), dim3(256),
+                           (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + 4 * c.window) * 4, st, qkv, ring, slots, m->pos, out, L,
+                           c.num_heads, c.head_dim, c.window, s2);
+    }
+}
+// the final conv over x (fp32 rows, activated), its history and the slots' positions (T codec frames on)
+static void codec_final(vox_codec* m, hipStream_t st, const float* x, const int32_t* slots, int n, int T, int L, float* out) {
+    const vox_codec_weights& w = m->w;
+    const int cl = m->cfg.decoder_dim >> 4;
+    if (L >= 512 && cl % 4 == 0 && (size_t)(134 * (cl + 1) + 7 * cl) * 4 <= 60 * 1024)
+        hipLaunchKernelGGL(k_final_conv_rows, dim3((L + 127) / 128, n), dim3(128), (size_t)(134 * (cl + 1) + 7 * cl) * 4, st, x, m->st_final, slots,
+                           w.final_w, w.final_b, out, L, cl);
+    else
+        hipLaunchKernelGGL(k_final_conv, dim3((L + 3) / 4, n), dim3(256), 0, st, x, m->st_final, slots, w.final_w, w.final_b, out, L, cl);
+    state_update(st, m->st_final, slots, x, n, L, 6, cl);
+    hipLaunchKernelGGL(k_pos_advance, dim3((n + 255) / 256), dim3(256), 0, st, m->pos, slots, n, T);
+}
+// One chunk with fp32 activations, split three ways inside each conv (planes == 3).
+static int codec_chunk_f32(vox_codec* m, hipStream_t st, const int32_t* codes, int code_stride, const int32_t* slots, int n, int T, float* out) {
     const vox_codec_config& c = m->cfg;
     const vox_codec_weights& w = m->w;
-    const int HD = c.num_heads * c.head_dim, H = c.hidden, LD = c.latent_dim;
+    const int H = c.hidden, LD = c.latent_dim;
     float *A = m->buf[0], *B = m->buf[1], *C = m->buf[2], *D = m->buf[3];
     const int off0[1] = {0};
     int L = T;
 
     hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.num_quantizers, c.codebook_size,
-                       c.vq_dim, m->q0, m->qr);
+                       c.vq_dim, m->q0, m->qr, 0);
     VOX_TRY(conv_gemm(st, w.rvq_first_out, m->q0, nullptr, slots, n, L, 0, off0, A, nullptr, nullptr, 0));
     VOX_TRY(conv_gemm(st, w.rvq_rest_out, m->qr, nullptr, slots, n, L, 0, off0, B, A, nullptr, 0));      // B = A + rest
     const int off3[3] = {2, 1, 0};
@@ -1588,22 +1962,9 @@ int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int
     VOX_TRY(conv_gemm(st, w.in_proj, A, nullptr, slots, n, L, 0, off0, B, nullptr, nullptr, 0));          // h = B [nL,H]
     for (int l = 0; l < c.num_layers; ++l) {
         const vox_codec_layer_w& lw = w.layers[l];
-        bf16_t* ring = m->ring + (size_t)l * m->max_slots * c.window * 2 * HD;
         hipLaunchKernelGGL(k_rmsnorm_f32, dim3(n * L), dim3(256), 0, st, B, lw.ln1, C, H, c.rms_eps);
         VOX_TRY(conv_gemm(st, lw.qkv, C, nullptr, slots, n, L, 0, off0, D, nullptr, nullptr, 0));        // D [nL,3HD]
-        // (VOX_CODEC_ATTN2=0: RoPE / ring write and the attention as two launches — A/B timing; bit-identical)
-        static const bool attn2 = [] { const char* e = getenv("VOX_CODEC_ATTN2"); return !(e && e[0] == '0'); }();
-        const size_t lds2 = (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + L * c.window) * 4;
-        if (attn2 && c.head_dim == 64 && L <= c.window && lds2 <= 64 * 1024) {
-            hipLaunchKernelGGL(k_codec_attn2<64>, dim3(c.num_heads, n), dim3(256), lds2,
-                               st, D, ring, slots, m->pos, C, L, c.num_heads, c.window, w.inv_freq);       // C [nL,HD]
-        } else {
-            hipLaunchKernelGGL(k_codec_rope_kv, dim3(n * L), dim3(256), 0, st, D, ring, slots, m->pos, L, c.num_heads,
-                               c.head_dim, c.window, w.inv_freq);
-            hipLaunchKernelGGL(k_codec_attn, dim3(c.num_heads, n), dim3(256),
-                               (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + 4 * c.window) * 4,
-                               st, D, ring, slots, m->pos, C, L, c.num_heads, c.head_dim, c.window);         // C [nL,HD]
-        }
+        codec_attention(m, st, l, slots, n, L, D, C, 0);                                                 // C [nL,HD]
         VOX_TRY(conv_gemm(st, lw.o, C, nullptr, slots, n, L, 0, off0, B, B, lw.scale1, 0));              // h += s1*o(attn)
         hipLaunchKernelGGL(k_rmsnorm_f32, dim3(n * L), dim3(256), 0, st, B, lw.ln2, C, H, c.rms_eps);
         VOX_TRY(conv_gemm(st, lw.gate_up, C, nullptr, slots, n, L, 0, off0, D, nullptr, nullptr, 0));    // D [nL,2I]
@@ -1611,7 +1972,6 @@ int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int
                            (size_t)n * L, c.intermediate);
         VOX_TRY(conv_gemm(st, lw.down, C, nullptr, slots, n, L, 0, off0, B, B, lw.scale2, 0));           // h += s2*down
     }
-    hipLaunchKernelGGL(k_pos_advance, dim3((n + 255) / 256), dim3(256), 0, st, m->pos, slots, n, L);
     hipLaunchKernelGGL(k_rmsnorm_f32, dim3(n * L), dim3(256), 0, st, B, w.final_norm, C, H, c.rms_eps);
     VOX_TRY(conv_gemm(st, w.out_proj, C, nullptr, slots, n, L, 0, off0, A, nullptr, nullptr, 0));         // A [nL,latent]
     // ---- upsample x2 x2 with ConvNeXt ----
@@ -1620,7 +1980,7 @@ int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int
         VOX_TRY(conv_gemm(st, uw.tconv, A, nullptr, slots, n, L, 0, off0, B, nullptr, nullptr, 0));      // B [n*2L, latent]
         L *= 2;
         hipLaunchKernelGGL(k_dwconv_ln, dim3(n * L), dim3(256), (size_t)LD * 4, st, B, m->st_dw[u], slots, uw.dw_w, uw.dw_b,
-                           uw.ln_w, uw.ln_b, C, L, LD, 1e-6f);
+                           uw.ln_w, uw.ln_b, C, L, LD, 1e-6f, 0);
         state_update(st, m->st_dw[u], slots, B, n, L, 6, LD);
         VOX_TRY(conv_gemm(st, uw.pw1, C, nullptr, slots, n, L, 0, off0, D, nullptr, nullptr, 1));        // GELU
         VOX_TRY(conv_gemm(st, uw.pw2, D, nullptr, slots, n, L, 0, off0, A, B, uw.gamma, 0));             // A = B + gamma*pw2
@@ -1632,10 +1992,6 @@ int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int
     // SnakeBeta is fused into the epilogue of the conv that produces its input: a conv whose output is only ever consumed
     // through a snake (conv1 of a residual unit) writes just the activated tensor, the others write both (the plain tensor
     // is the residual branch).  t1 always holds the activated input of the next conv.
-    // Two-term mode (planes == 2, the default): the activated tensors t1 / t3 — only ever read as GEMM operands — are kept as S2
-    // rows (ConvGemmArgs), split once where they are produced; the residual stream h stays fp32.  Their history rows (st_tc /
-    // st_ru) are byte copies of those rows, i.e. in the same format: change the mode only on freshly reset slots.
-    const int s2 = m->planes == 2;
     float* h = B;      // current activations
     float* t1 = A;
     float* t2 = C;
@@ -1646,8 +2002,7 @@ int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int
         const int cin = c.decoder_dim >> b, cout = c.decoder_dim >> (b + 1), r = c.rates[b];
         const int offt[2] = {0, 1};
         // t2 [n*L*r, cout] = tconv(t1); t3 = act1 of unit 0 applied to it (t1 is still being read by other blocks)
-        VOX_TRY(conv_gemm(st, bw.tconv, t1, m->st_tc[b], slots, n, L, 1, offt, t2, nullptr, nullptr, 0, t3, &bw.res[0].act1, cout,
-                          nullptr, nullptr, nullptr, 0.0f, s2 && b > 0, s2));
+        VOX_TRY(conv_gemm(st, bw.tconv, t1, m->st_tc[b], slots, n, L, 1, offt, t2, nullptr, nullptr, 0, t3, &bw.res[0].act1, cout));
         state_update(st, m->st_tc[b], slots, t1, n, L, 1, cin);
         L *= r;
         { float* x = h; h = t2; t2 = x; }
@@ -1657,35 +2012,148 @@ int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int
             const int d = u == 0 ? 1 : (u == 1 ? 3 : 9);
             const int offd[7] = {6 * d, 5 * d, 4 * d, 3 * d, 2 * d, d, 0};
             const vox_snake_w* nx = u < 2 ? &bw.res[u + 1].act1 : (b < 3 ? &w.blocks[b + 1].snake0 : &w.final_snake);
-            if (s2) {
-                // the whole unit in one launch where the tile covers all channels (k_res_unit): the activated intermediate stays on chip;
-                // the next activation goes to t3 (neighbouring tiles still read their halo rows of t1), then the two swap
-                int fused = 0;
-                VOX_TRY(conv_unit(st, rw.conv1, rw.conv2, t1, m->st_ru[b][u], slots, n, L, 6 * d, offd, rw.act2, h, t3, nx, !(b == 3 && u == 2), &fused));
-                if (fused) {
-                    state_update(st, m->st_ru[b][u], slots, t1, n, L, 6 * d, cout);
-                    { float* x = t1; t1 = t3; t3 = x; }
-                    continue;
-                }
-            }
             // t3 = act2(conv1(t1))   (the plain conv1 output has no other consumer)
-            VOX_TRY(conv_gemm(st, rw.conv1, t1, m->st_ru[b][u], slots, n, L, 6 * d, offd, nullptr, nullptr, nullptr, 0, t3, &rw.act2, cout,
-                              nullptr, nullptr, nullptr, 0.0f, s2, s2));
+            VOX_TRY(conv_gemm(st, rw.conv1, t1, m->st_ru[b][u], slots, n, L, 6 * d, offd, nullptr, nullptr, nullptr, 0, t3, &rw.act2, cout));
             state_update(st, m->st_ru[b][u], slots, t1, n, L, 6 * d, cout);
             // h += conv2(t3); t1 = the next consumer's activation of the new h
-            VOX_TRY(conv_gemm(st, rw.conv2, t3, nullptr, slots, n, L, 0, off0, h, h, nullptr, 0, t1, nx, cout,
-                              nullptr, nullptr, nullptr, 0.0f, s2, s2 && !(b == 3 && u == 2)));      // (the final conv reads fp32 rows)
+            VOX_TRY(conv_gemm(st, rw.conv2, t3, nullptr, slots, n, L, 0, off0, h, h, nullptr, 0, t1, nx, cout));
         }
     }
-    const int cl = c.decoder_dim >> 4;
-    if (L >= 512 && cl % 4 == 0 && (size_t)(134 * (cl + 1) + 7 * cl) * 4 <= 60 * 1024)
-        hipLaunchKernelGGL(k_final_conv_rows, dim3((L + 127) / 128, n), dim3(128), (size_t)(134 * (cl + 1) + 7 * cl) * 4, st, t1, m->st_final,
-                           slots, w.final_w, w.final_b, out, L, cl);
-    else
-        hipLaunchKernelGGL(k_final_conv, dim3((L + 3) / 4, n), dim3(256), 0, st, t1, m->st_final, slots, w.final_w, w.final_b, out,
-                           L, cl);
-    state_update(st, m->st_final, slots, t1, n, L, 6, cl);
+    codec_final(m, st, t1, slots, n, T, L, out);
     return VOX_OK;
+}
+
+// One chunk with S2 activations (planes 1 and 2): every tensor that only convs read is written as S2 rows by whatever produces it, and what
+// stood between two convs (RMSNorm, SiLU, SnakeBeta) is in the epilogue of the first: 86 launches of 134.  RMSNorm: the producer writes h * w
+// beside h, the consumer scales its sums by the rows' 1 / rms.
+static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, int code_stride, const int32_t* slots, int n, int T, float* out) {
+    const vox_codec_config& c = m->cfg;
+    const vox_codec_weights& w = m->w;
+    const int LD = c.latent_dim;
+    float *A = m->buf[0], *B = m->buf[1], *C = m->buf[2], *D = m->buf[3];
+    const int off3[3] = {2, 1, 0}, off7[7] = {6, 5, 4, 3, 2, 1, 0};
+    int L = T;
+    // A conv's history is rewritten after the conv has read it: by extra blocks of the next launch (its output must not be the history's
+    // source), or by a launch of its own where the next one is no k_conv_dma.
+    ConvJob job{};
+    auto later = [&](float* state, const float* x, int P, int ch) { job = ConvJob{state, x, L, P, ch, n}; };
+    auto flush = [&] {
+        if (job.state) state_update(st, job.state, slots, job.x, n, job.L, job.P, job.C);
+        job = ConvJob{};
+    };
+    auto conv = [&](const vox_conv_w& cw, const float* x, const float* state, int P, const int* offs) { return conv_s2_args(cw, x, state, slots, n, L, P, offs); };
+    auto run = [&](ConvDmaArgs& a, int epi = 0) {
+        a.job = job;
+        job = ConvJob{};
+        return conv_s2(st, a, epi);
+    };
+    auto s2_out = [](ConvDmaArgs& a, float* y, const float* nw = nullptr) { a.out2 = y; a.out2_s2 = 1; a.nw = nw; };
+    auto act_out = [](ConvDmaArgs& a, float* y, const vox_snake_w& sn, int ch, int s2 = 1) {
+        a.out2 = y; a.out2_s2 = s2; a.sn_alpha = sn.alpha; a.sn_invb = sn.inv_beta; a.sn_mod = ch;
+    };
+    auto rms_in = [&](ConvDmaArgs& a, const float* h) { a.rms_x = h; a.rms_eps = c.rms_eps; };
+
+    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.num_quantizers, c.codebook_size, c.vq_dim, m->q0, m->qr, 1);
+    { ConvDmaArgs a = conv(w.rvq_first_out, m->q0, nullptr, 0, nullptr); a.out = A; VOX_TRY(run(a)); }
+    { ConvDmaArgs a = conv(w.rvq_rest_out, m->qr, nullptr, 0, nullptr); a.res = A; s2_out(a, B); VOX_TRY(run(a)); }
+    { ConvDmaArgs a = conv(w.pre_conv, B, m->st_pre, 2, off3); s2_out(a, A); VOX_TRY(run(a)); }             // A [nL, latent]
+    later(m->st_pre, B, 2, c.codebook_dim);
+    // ---- transformer: h = C (fp32), D = S2 of h * the next norm's weight ----
+    { ConvDmaArgs a = conv(w.in_proj, A, nullptr, 0, nullptr); a.out = C; s2_out(a, D, c.num_layers ? w.layers[0].ln1 : w.final_norm); VOX_TRY(run(a)); }
+    for (int l = 0; l < c.num_layers; ++l) {
+        const vox_codec_layer_w& lw = w.layers[l];
+        { ConvDmaArgs a = conv(lw.qkv, D, nullptr, 0, nullptr); rms_in(a, C); a.out = A; VOX_TRY(run(a)); }
+        codec_attention(m, st, l, slots, n, L, A, B, 1);
+        { ConvDmaArgs a = conv(lw.o, B, nullptr, 0, nullptr); a.res = C; a.scale = lw.scale1; a.out = C; s2_out(a, D, lw.ln2); VOX_TRY(run(a)); }
+        { ConvDmaArgs a = conv(lw.gate_up, D, nullptr, 0, nullptr); rms_in(a, C); s2_out(a, A); VOX_TRY(run(a, CONV_GLU)); }
+        { ConvDmaArgs a = conv(lw.down, A, nullptr, 0, nullptr); a.res = C; a.scale = lw.scale2; a.out = C;
+          s2_out(a, D, l + 1 < c.num_layers ? w.layers[l + 1].ln1 : w.final_norm); VOX_TRY(run(a)); }
+    }
+    { ConvDmaArgs a = conv(w.out_proj, D, nullptr, 0, nullptr); rms_in(a, C); s2_out(a, A); VOX_TRY(run(a)); }      // A [nL, latent]
+    // ---- upsample x2 x2 with ConvNeXt ----
+    for (int u = 0; u < 2; ++u) {
+        const vox_codec_up_w& uw = w.up[u];
+        { ConvDmaArgs a = conv(uw.tconv, A, nullptr, 0, nullptr); a.out = B; VOX_TRY(run(a)); }                     // B [n*2L, latent]
+        L *= 2;
+        hipLaunchKernelGGL(k_dwconv_ln, dim3(n * L), dim3(256), (size_t)LD * 4, st, B, m->st_dw[u], slots, uw.dw_w, uw.dw_b, uw.ln_w, uw.ln_b, C, L, LD,
+                           1e-6f, 1);
+        later(m->st_dw[u], B, 6, LD);
+        { ConvDmaArgs a = conv(uw.pw1, C, nullptr, 0, nullptr); s2_out(a, D); VOX_TRY(run(a, CONV_GELU)); }
+        { ConvDmaArgs a = conv(uw.pw2, D, nullptr, 0, nullptr); a.res = B; a.scale = uw.gamma; s2_out(a, A); VOX_TRY(run(a)); }
+    }
+    // ---- decoder.  SnakeBeta is in the epilogue of the conv that produces its input; h stays fp32 and is written only where a residual
+    // branch reads it.  free: the two buffers that hold neither h nor x (job.x may still be one of them). ----
+    { ConvDmaArgs a = conv(w.dec0, A, m->st_dec0, 6, off7); act_out(a, C, w.blocks[0].snake0, c.decoder_dim); VOX_TRY(run(a)); }
+    later(m->st_dec0, A, 6, LD);
+    float *h = B, *x = C, *free_[2] = {A, D};
+    auto take = [&](float* avoid) {          // a free buffer other than `avoid`; its place is left empty (NULL)
+        float** f = free_[0] && free_[0] != avoid ? &free_[0] : &free_[1];
+        float* p = *f;
+        *f = nullptr;
+        return p;
+    };
+    auto put = [&](float* p) { (free_[0] ? free_[1] : free_[0]) = p; };
+    for (int b = 0; b < 4; ++b) {
+        const vox_codec_block_w& bw = w.blocks[b];
+        const int cin = c.decoder_dim >> b, cout = c.decoder_dim >> (b + 1);
+        const int offt[2] = {0, 1};
+        {   // h' [n*L*r, cout] = tconv(x), x' = act1 of unit 0 applied to it.  The old h is dead: three buffers to choose from
+            float *old_x = x, *xn = take(const_cast<float*>(job.x)), *hn = h;
+            ConvDmaArgs a = conv(bw.tconv, x, m->st_tc[b], 1, offt);
+            a.out = hn;
+            act_out(a, xn, bw.res[0].act1, cout);
+            VOX_TRY(run(a));
+            later(m->st_tc[b], old_x, 1, cin);
+            x = xn;
+            put(old_x);
+        }
+        L *= c.rates[b];
+        for (int u = 0; u < 3; ++u) {
+            const vox_codec_res_w& rw = bw.res[u];
+            const int d = u == 0 ? 1 : (u == 1 ? 3 : 9), last = b == 3 && u == 2;
+            const int offd[7] = {6 * d, 5 * d, 4 * d, 3 * d, 2 * d, d, 0};
+            const vox_snake_w* nx = u < 2 ? &bw.res[u + 1].act1 : (b < 3 ? &w.blocks[b + 1].snake0 : &w.final_snake);
+            float *y = take(const_cast<float*>(job.x)), *ho = u < 2 ? h : nullptr;      // (after unit 2 only the activation of h goes on)
+            // the whole unit in one launch where the tile covers all channels (k_res_unit): the activated intermediate stays on chip
+            int fused = 0;
+            VOX_TRY(conv_unit(st, rw.conv1, rw.conv2, x, m->st_ru[b][u], slots, n, L, 6 * d, offd, rw.act2, h, ho, y, nx, !last, &fused));
+            if (fused) {
+                flush();
+                later(m->st_ru[b][u], x, 6 * d, cout);
+                put(x);
+                x = y;
+                continue;
+            }
+            ConvDmaArgs a1 = conv(rw.conv1, x, m->st_ru[b][u], 6 * d, offd);      // y = act2(conv1(x))
+            act_out(a1, y, rw.act2, cout);
+            VOX_TRY(run(a1));
+            later(m->st_ru[b][u], x, 6 * d, cout);
+            float* z = take(nullptr);                                              // h += conv2(y); z = the next consumer's activation of it
+            ConvDmaArgs a2 = conv(rw.conv2, y, nullptr, 0, nullptr);
+            a2.res = h;
+            a2.out = ho;
+            act_out(a2, z, *nx, cout, !last);                                      // (the final conv reads fp32 rows)
+            VOX_TRY(run(a2));
+            put(x);
+            put(y);
+            x = z;
+        }
+    }
+    flush();
+    codec_final(m, st, x, slots, n, T, L, out);
+    return VOX_OK;
+}
+
+extern "C" {
+
+int vox_codec_decode_chunk(vox_codec* m, void* stream, const int32_t* codes, int code_stride, const int32_t* slots, int n,
+                           int T, float* out) {
+    if (!m || !codes || !slots || !out) return vox_fail(VOX_ERR_INVALID, "codec_decode_chunk: NULL");
+    if (n < 1 || n > m->max_batch || T < 1 || T > m->T) return vox_fail(VOX_ERR_INVALID, "codec_decode_chunk: n=%d T=%d out of range", n, T);
+    m->decoded = true;
+    hipStream_t st = (hipStream_t)stream;
+    struct PlanesGuard { int saved; explicit PlanesGuard(int p) : saved(g_conv_planes) { g_conv_planes = p; } ~PlanesGuard() { g_conv_planes = saved; } } pg(m->planes);
+    return m->planes <= 2 ? codec_chunk_s2(m, st, codes, code_stride, slots, n, T, out) : codec_chunk_f32(m, st, codes, code_stride, slots, n, T, out);
 }
 
 }  // extern "C"
@@ -1950,7 +2418,7 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
     float *A = m->buf[0], *B = m->buf[1], *Cb = m->buf[2], *Db = m->buf[3];
     const int off0[1] = {0};
     int L = T;
-    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.n_q, c.bins, c.vq_dim, m->q0, m->qr);
+    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.n_q, c.bins, c.vq_dim, m->q0, m->qr, 0);
     VOX_TRY(conv_gemm(st, w.rvq_first_out, m->q0, nullptr, sl, n, L, 0, off0, A, nullptr, nullptr, 0));
     VOX_TRY(conv_gemm(st, w.rvq_rest_out, m->qr, nullptr, sl, n, L, 0, off0, B, A, nullptr, 0));            // B [nL, dim]
     {
