@@ -1,4 +1,4 @@
-"""The LDS-DMA convolutions of the Qwen3 codec (k_conv_dma) at the shapes where their tiles can go wrong, against the CPU oracle in fp32.
+"""The LDS-DMA convolutions of the Qwen3 codec (k_conv_dma, k_conv_unit) at the shapes where their tiles can go wrong, against the CPU oracle in fp32.
 
 Channel counts that are multiples of 32, 64, 128 and 256 only (the k-steps of the tiles), fewer rows than one tile and rows that do not
 fill the last one, intermediate sizes that end inside a gate / up pair, chunks shorter than a conv's look-back (the history shifts in
@@ -30,6 +30,7 @@ CASES = [
     ((128, 64, 64, 96, 4, 16, 512, [4, 2, 2, 2]), 5, 3),       # 64-channel steps, 15 rows of a 16-row tile
     ((256, 128, 128, 128, 2, 64, 512, [2, 3, 2, 2]), 17, 1),   # 128-channel steps, 17 rows: one into a second tile; head dim 64
     ((512, 384, 384, 640, 6, 64, 1024, [2, 2, 2, 3]), 2, 4),   # 128-channel steps only
+    ((64, 96, 96, 96, 2, 16, 1536, [2, 2, 2, 2]), 3, 1),       # whole residual units of 64 rows whose look-back (54) is nearly all history
     ((512, 256, 512, 768, 8, 64, 512, [8, 5, 4, 3]), 4, 2),    # 256-channel steps, the last block's 32 channels over many rows
 ]
 

@@ -73,9 +73,9 @@ struct ConvGemmArgs {
     float ln_eps;
     // "S2" rows: an activation row of Cin values stored as its two leading bf16 terms, [Cin x bf16 h][Cin x bf16 m] (x ~ h + m, 16
     // significand bits; the same 4 * Cin bytes as the fp32 row, so buffers, history state and k_state_update are format-agnostic).
-    // The producing GEMM's epilogue splits each value ONCE (out2_s2); the consuming GEMM (x_s2, planes = 2) stages plain bf16 — the
-    // per-tap three-way split of fp32 rows made the many-row decoder convs VALU-bound (MFMA 16 % busy; round-3 planes probe).
-    int x_s2, out2_s2;
+    // The producing epilogue splits each value ONCE (out2_s2); the consumers (k_conv_dma, k_conv_unit) read plain bf16 — the per-tap
+    // split of fp32 rows made the many-row decoder convs VALU-bound (MFMA 16 % busy).
+    int out2_s2;
     int dev;               // development builds (-DVOX_DEV_KNOBS, VOX_CODEC_DEV): 1 skip the K loop, 2 no out2 stores, 4 no out stores, 8 no residual loads
 };
 #ifdef VOX_DEV_KNOBS
@@ -145,20 +145,7 @@ __device__ __forceinline__ void conv_epilogue(const ConvGemmArgs& a, f32x4 (&acc
                 if (a.out && ok && !CG_DEV(a, 4)) a.out[o] = v;
                 if (a.out2 && !CG_DEV(a, 2)) {
                     const float sv2 = snake_f(v, ca[j], ci[j]);
-                    if (a.out2_s2) {
-                        // S2 row of the consumer: [sn_mod x h][sn_mod x m]; a lane pair (columns c, c + 1) stores one 32-bit word per
-                        // term (the even lane the h pair, the odd lane the m pair) instead of two 16-bit stores each
-                        bf16_t hb, mbf;
-                        split2(sv2, hb, mbf);
-                        const unsigned hp = __shfl_xor((unsigned)hb, 1, 64), mp = __shfl_xor((unsigned)mbf, 1, 64);
-                        bf16_t* r16 = reinterpret_cast<bf16_t*>(a.out2 + (size_t)m * a.N) + (size_t)cj[j] * 2 * a.sn_mod;
-                        if (ok) {
-                            if (!(l15 & 1)) *reinterpret_cast<unsigned*>(r16 + cc[j]) = (unsigned)hb | (hp << 16);
-                            else *reinterpret_cast<unsigned*>(r16 + a.sn_mod + cc[j] - 1) = mp | ((unsigned)mbf << 16);
-                        }
-                    } else if (ok) {
-                        a.out2[o] = sv2;
-                    }
+                    if (ok) a.out2[o] = sv2;
                 }
             }
     }
@@ -282,203 +269,6 @@ __global__ __launch_bounds__(256, (WM * WN > 12 ? 3 : 4)) void k_conv_gemm(ConvG
     conv_epilogue<WM, WN>(a, acc, m0, n0, wm, wn, lane);
 }
 
-// Multi-tap convolution over S2 rows, activation tile staged ONCE per 32-channel chunk for all taps: the BM + H rows (H = the largest
-// look-back) a tile's taps read go to LDS together and every tap's MFMAs read them at its own row shift, so the activation staging
-// (global loads, LDS writes, barriers) is paid once per chunk instead of once per tap (7 x for the residual units' dilated convs, whose
-// time was that staging: 365 us for 7 taps against 233 us for the whole 1-tap conv2 at 614 k rows).  Weights: one tap's BN x 32 slice at
-// a time, double-buffered, one barrier per tap.  Accumulation order: chunk-major, taps inside, the m term before the h term.
-// Requires: all offsets in [0, H], L % BM == 0 (a tile lies inside one request).  Dynamic LDS: (2 (BM + H) + 2 BN) x 80 bytes.
-template <int WM, int WN>
-__device__ __forceinline__ void conv_taps_kloop(const ConvGemmArgs& a, int H, unsigned char* smem_raw, f32x4 (&acc)[WM][WN], int m0, int n0) {
-    constexpr int BM = 32 * WM, BN = 32 * WN, LD = 40, NBR = (BN * 4 + 255) / 256;
-    const int R = BM + H;
-    bf16_t* As = reinterpret_cast<bf16_t*>(smem_raw);          // [2][R][LD]
-    bf16_t* Bs = As + (size_t)2 * R * LD;                       // [2][BN][LD]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = (wave >> 1) * 16 * WM, wn = (wave & 1) * 16 * WN;
-    const int rb = m0 / a.L, t0 = m0 - rb * a.L;
-    const int fr = lane & 15, fk = (lane >> 4) * 8;
-#pragma unroll
-    for (int i = 0; i < WM; ++i)
-#pragma unroll
-        for (int j = 0; j < WN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
-    const bf16_t* xrows = reinterpret_cast<const bf16_t*>(a.x) + (size_t)rb * a.L * 2 * a.Cin;
-    const bf16_t* srows = a.state ? reinterpret_cast<const bf16_t*>(a.state) + (size_t)a.slots[rb] * a.P * 2 * a.Cin : nullptr;
-    // Weights: the (chunk, tap) pairs form ONE stream s = chunk * n_taps + tap; the slice of step s + 2 is requested before the MFMAs of
-    // step s and goes to LDS behind the MFMAs of step s + 1 (two register sets, chosen by the parity of s: the stream loop is unrolled by
-    // two so that the choice is static).  One step ahead — the round-3 form — a slice had one tap's MFMAs (24 of them, ~0.16 us) to come
-    // back from L2 (~0.6 us): every tap waited for its weights, the matrix cores were 27 % busy.  LDS buffers: parity of s, as before.
-    uint4 wv0[NBR], wv1[NBR];
-    auto fetchB = [&](uint4 (&wv)[NBR], int tap, int c0) {
-#pragma unroll
-        for (int i = 0; i < NBR; ++i) {
-            const int idx = tid + 256 * i, bn = n0 + (idx >> 2);
-            wv[i] = make_uint4(0, 0, 0, 0);
-            if (idx < BN * 4 && bn < a.N) wv[i] = *reinterpret_cast<const uint4*>(a.w + ((size_t)tap * a.N + bn) * a.Cin + c0 + (idx & 3) * 8);
-        }
-    };
-    auto storeB = [&](const uint4 (&wv)[NBR], int q) {
-#pragma unroll
-        for (int i = 0; i < NBR; ++i) {
-            const int idx = tid + 256 * i;
-            if (idx < BN * 4) *reinterpret_cast<uint4*>(Bs + ((size_t)q * BN + (idx >> 2)) * LD + (idx & 3) * 8) = wv[i];
-        }
-    };
-    // the tile's rows of the NEXT chunk travel in registers while this chunk's taps run (all requests issued together, nothing waits
-    // on them until the chunk boundary)
-    constexpr int NAR = ((BM + 64) * 8 + 255) / 256;
-    uint4 av[NAR];
-    auto fetchA = [&](int c0) {
-#pragma unroll
-        for (int i = 0; i < NAR; ++i) {
-            const int e = tid + 256 * i, j = e >> 3, p = (e >> 2) & 1, seg = e & 3, st = t0 - H + j;
-            av[i] = make_uint4(0, 0, 0, 0);
-            const bf16_t* row = nullptr;
-            if (e < R * 8) {
-                if (st >= 0) row = xrows + (size_t)st * 2 * a.Cin;
-                else if (srows && a.P + st >= 0) row = srows + (size_t)(a.P + st) * 2 * a.Cin;
-            }
-            if (row) av[i] = *reinterpret_cast<const uint4*>(row + p * a.Cin + c0 + seg * 8);
-        }
-    };
-    auto storeA = [&]() {
-#pragma unroll
-        for (int i = 0; i < NAR; ++i) {
-            const int e = tid + 256 * i, j = e >> 3, p = (e >> 2) & 1, seg = e & 3;
-            if (e < R * 8) *reinterpret_cast<uint4*>(As + ((size_t)p * R + j) * LD + seg * 8) = av[i];
-        }
-    };
-    const int nck = CG_DEV(a, 1) ? 0 : a.Cin >> 5;
-    const int nt = a.n_taps, total = nck * nt;
-    if (total == 0) return;
-    // (tap, chunk offset) of stream index s
-    int f_tap = 0, f_c0 = 0;                       // of the next slice to REQUEST
-    auto advance_f = [&]() { if (++f_tap == nt) { f_tap = 0; f_c0 += 32; } };
-    fetchA(0);
-    fetchB(wv0, 0, 0); advance_f();
-    if (total > 1) { fetchB(wv1, f_tap, f_c0); advance_f(); }
-    __syncthreads();              // (the caller may have used the LDS before)
-    storeB(wv0, 0);
-    int tap = 0, ck = 0;                            // of the step being computed
-    // one step: F = the register set that is free (its slice, step s, is in LDS), S = the set holding step s + 1
-    auto step = [&](int s_, uint4 (&F)[NBR], const uint4 (&S)[NBR]) {
-        if (tap == 0) {           // chunk boundary: the previous step's closing barrier says nobody reads the old tile any more
-            storeA();
-            __syncthreads();
-            if (ck + 1 < nck) fetchA((ck + 1) * 32);
-        }
-        if (s_ + 2 < total) { fetchB(F, f_tap, f_c0); advance_f(); }
-        const int sh = H - a.off[tap];
-        const bf16_t* Bq = Bs + (size_t)(s_ & 1) * BN * LD;
-        uint4 bfr[WN];
-#pragma unroll
-        for (int j = 0; j < WN; ++j) bfr[j] = *reinterpret_cast<const uint4*>(Bq + (wn + j * 16 + fr) * LD + fk);
-#pragma unroll
-        for (int p = 1; p >= 0; --p) {      // smaller term first
-#pragma unroll
-            for (int i = 0; i < WM; ++i) {
-                const uint4 afr = *reinterpret_cast<const uint4*>(As + ((size_t)p * R + wm + i * 16 + fr + sh) * LD + fk);
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(afr), as_cbf8(bfr[j]), acc[i][j], 0, 0, 0);
-            }
-        }
-        if (s_ + 1 < total) storeB(S, (s_ + 1) & 1);
-        __syncthreads();          // the next step's weights are visible; this step's buffer may be overwritten by the step after next
-        if (++tap == nt) { tap = 0; ++ck; }
-    };
-    for (int s_ = 0; s_ < total; s_ += 2) {
-        step(s_, wv0, wv1);
-        if (s_ + 1 < total) step(s_ + 1, wv1, wv0);
-    }
-}
-
-// A whole residual unit of the decoder in ONE kernel:  h += conv2(act2(conv1(x)))  and  out2 = act_next(h)  — conv1 = the dilated 7-tap
-// conv over S2 rows (conv_taps_kloop), conv2 = the 1-tap C -> C conv.  The block's tile covers ALL C output channels of conv1, so the
-// activated intermediate (the whole K of conv2) is on chip: it goes from the accumulators through Snake + the two-term split into LDS
-// as the A operand of the second GEMM instead of to HBM and back (per unit at 614 k rows x 96 channels: 236 MB written + 236 MB read).
-// Accumulation orders are those of the two kernels it replaces (conv2: 32-channel chunks in order, the m term before the h term), so the
-// results are bit-identical.  a2.out2 must not alias a1.x: a neighbouring tile still reads its halo rows of x.
-// Dynamic LDS: max((2 (BM + H) + 2 BN) x 80, 2 BM (C + 8) x 2 + 2 BN x 80) bytes.
-template <int WM, int WN>
-__global__ __launch_bounds__(256, (WM * WN >= 12 ? 2 : 3)) void k_res_unit(ConvGemmArgs a1, ConvGemmArgs a2, int H) {
-    constexpr int BM = 32 * WM, BN = 32 * WN, LD = 40, NBR = (BN * 4 + 255) / 256;
-    extern __shared__ __attribute__((aligned(16))) unsigned char smem_raw[];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int m0 = blockIdx.y * BM;
-    const int wm = (wave >> 1) * 16 * WM, wn = (wave & 1) * 16 * WN;
-    const int fr = lane & 15, fk = (lane >> 4) * 8;
-    f32x4 acc[WM][WN];
-    conv_taps_kloop<WM, WN>(a1, H, smem_raw, acc, m0, 0);
-    // ---- the activated intermediate as the second GEMM's A operand: [2 terms][BM][C + 8] bf16
-    const int C = a1.N, LD2 = C + 8;
-    bf16_t* A2 = reinterpret_cast<bf16_t*>(smem_raw);
-    bf16_t* B2 = A2 + (size_t)2 * BM * LD2;                     // [2][BN][LD]
-    uint4 wv[NBR];
-    auto fetchB = [&](int c0) {
-#pragma unroll
-        for (int i = 0; i < NBR; ++i) {
-            const int idx = tid + 256 * i, bn = idx >> 2;
-            wv[i] = make_uint4(0, 0, 0, 0);
-            if (idx < BN * 4 && bn < a2.N) wv[i] = *reinterpret_cast<const uint4*>(a2.w + (size_t)bn * a2.Cin + c0 + (idx & 3) * 8);
-        }
-    };
-    auto storeB = [&](int q) {
-#pragma unroll
-        for (int i = 0; i < NBR; ++i) {
-            const int idx = tid + 256 * i;
-            if (idx < BN * 4) *reinterpret_cast<uint4*>(B2 + ((size_t)q * BN + (idx >> 2)) * LD + (idx & 3) * 8) = wv[i];
-        }
-    };
-    fetchB(0);
-    __syncthreads();                                            // every wave is done with the first GEMM's tiles
-    {
-        const int l15 = lane & 15, rg = (lane >> 4) * 4;
-#pragma unroll
-        for (int j = 0; j < WN; ++j) {
-            const int n = wn + j * 16 + l15;
-            const float cb = a1.bias ? a1.bias[n % a1.bias_mod] : 0.0f;
-            const int cc = n % a1.sn_mod;
-            const float ca = a1.sn_alpha[cc], ci = a1.sn_invb[cc];
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float sv = snake_f(acc[i][j][r] + cb, ca, ci);
-                    bf16_t hb, mb;
-                    split2(sv, hb, mb);
-                    const int row = wm + i * 16 + rg + r;
-                    A2[(size_t)row * LD2 + n] = hb;
-                    A2[((size_t)BM + row) * LD2 + n] = mb;
-                    acc[i][j][r] = 0.0f;
-                }
-        }
-    }
-    storeB(0);
-    __syncthreads();
-    const int nck = C >> 5;
-    for (int ck = 0; ck < nck; ++ck) {
-        if (ck + 1 < nck) fetchB((ck + 1) * 32);
-        const bf16_t* Bq = B2 + (size_t)(ck & 1) * BN * LD;
-        uint4 bfr[WN];
-#pragma unroll
-        for (int j = 0; j < WN; ++j) bfr[j] = *reinterpret_cast<const uint4*>(Bq + (wn + j * 16 + fr) * LD + fk);
-#pragma unroll
-        for (int p = 1; p >= 0; --p) {          // smaller term first
-#pragma unroll
-            for (int i = 0; i < WM; ++i) {
-                const uint4 afr = *reinterpret_cast<const uint4*>(A2 + ((size_t)p * BM + wm + i * 16 + fr) * LD2 + ck * 32 + fk);
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(afr), as_cbf8(bfr[j]), acc[i][j], 0, 0, 0);
-            }
-        }
-        if (ck + 1 < nck) storeB((ck + 1) & 1);
-        __syncthreads();
-    }
-    conv_epilogue<WM, WN>(a2, acc, m0, 0, wm, wn, lane);
-}
-
 // LayerNorm row statistics by the 16 lanes l16 = 0..15 of a row group (two passes over float4 chunks, butterfly inside the group).
 // Shared by the GEMM with the fused LayerNorm and by k_flow_ln, so a row normalises to the same bits on either path (a request's output
 // must not depend on how many requests share its batch).
@@ -521,6 +311,19 @@ struct ConvJob {           // history rows <- the last P rows of [history ++ x],
     const float* x;
     int L, P, C, n;
 };
+// new history = last P rows of [history ++ x]; one thread per (request, channel), rows ascending (in place)
+__device__ __forceinline__ void conv_job(const ConvJob& j, const int* slots, int block, int threads) {
+    const int per = (j.C + threads - 1) / threads, b = block / per, c = block % per * threads + (int)threadIdx.x;
+    if (c >= j.C) return;
+    float* s = j.state + (size_t)slots[b] * j.P * j.C + c;
+    const float* x = j.x + (size_t)b * j.L * j.C + c;
+#pragma unroll 6
+    for (int i = 0; i < j.P; ++i) {
+        const int e = j.L + i;
+        s[(size_t)i * j.C] = e < j.P ? s[(size_t)e * j.C] : x[(size_t)(e - j.P) * j.C];
+    }
+}
+static int conv_job_blocks(const ConvJob& j, int threads) { return j.state ? j.n * ((j.C + threads - 1) / threads) : 0; }
 struct ConvDmaArgs : ConvGemmArgs {
     int tm, tn, tiles8, mfast;      // tiles along M and N; their number rounded up to 8; 1: the blocks of an XCD walk the rows first
     const float* rms_x;    // fp32 rows [M, Cin] whose 1 / rms scales the sums of row m (the rows' RMSNorm, its weight already in x), or NULL
@@ -554,7 +357,8 @@ __device__ __forceinline__ void conv_put_s2(bf16_t* row, int width, int c, const
 // The epilogue of W neighbouring channels (n ..) of MT rows (m, m + 16, ..) that one lane holds: constants once, every row's residual
 // requested ahead of the first store, 16-byte accesses throughout.
 template <bool GELU, int W, int MT>
-__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n) {
+__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n,
+                                             const f32x4* res_ready = nullptr) {
     if (n >= a.N) return;          // (N and the group width are multiples of W)
     float b[W], s[W], al[W], ib[W], nw[W], rs[MT][W];
     const auto fetch = [](float (&d)[W], const float* p) {
@@ -570,7 +374,12 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
     if (a.scale) fetch(s, a.scale + n);
     if (a.sn_alpha) { fetch(al, a.sn_alpha + cc); fetch(ib, a.sn_invb + cc); }
     if (a.nw) fetch(nw, a.nw + n);
-    if (a.res)
+    if (res_ready) {
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int e = 0; e < W; ++e) rs[i][e] = res_ready[i * (W / 4) + e / 4][e % 4];
+    } else if (a.res)
 #pragma unroll
         for (int i = 0; i < MT; ++i)
             if (m + 16 * i < a.M) fetch(rs[i], a.res + (size_t)(m + 16 * i) * a.N + n);
@@ -631,17 +440,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     __shared__ float rms_s[BM];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     if ((int)blockIdx.x >= a.tiles8) {
-        // new history = last P rows of [history ++ x]; one thread per (request, channel), rows ascending (in place)
-        const ConvJob& j = a.job;
-        const int per = (j.C + 64 * NWV - 1) / (64 * NWV), e0 = (int)blockIdx.x - a.tiles8, b = e0 / per, c = (e0 % per) * 64 * NWV + tid;
-        if (c >= j.C) return;
-        float* s = j.state + (size_t)a.slots[b] * j.P * j.C + c;
-        const float* x = j.x + (size_t)b * j.L * j.C + c;
-#pragma unroll 6
-        for (int i = 0; i < j.P; ++i) {
-            const int e = j.L + i;
-            s[(size_t)i * j.C] = e < j.P ? s[(size_t)e * j.C] : x[(size_t)(e - j.P) * j.C];
-        }
+        conv_job(a.job, a.slots, (int)blockIdx.x - a.tiles8, 64 * NWV);
         return;
     }
     const int t = ((int)blockIdx.x & 7) * (a.tiles8 >> 3) + ((int)blockIdx.x >> 3);
@@ -807,6 +606,188 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     }
 }
 
+// A whole residual unit of the decoder:  h += conv2(act2(conv1(x)))  and  out2 = act_next(h);  conv1: 7 taps, dilated, conv2: one tap, C -> C.
+// A block takes 16 MT NW rows of one request and ALL C channels of them; a wave takes 16 MT rows.  conv1 walks K in 32-channel chunks: a
+// chunk's rows with their look-back (up to 64) are staged once for the seven taps (two buffers, the next chunk's requests spread over the
+// taps of this one), the weights are a stream of C x 32 slices through S stages.  What the lanes then hold, eight neighbouring channels
+// of a row, is after SnakeBeta and the two-term split the activation operand of conv2 as it stands: conv2 is C / 32 further slices of the
+// same stream, and the intermediate never leaves the registers.  x, the history and the weights arrive by LDS DMA as in k_conv_dma.
+// Bound: memory (x, h read, h, out2 written: 944 MB at 614 400 rows x 96) beside the matrix cores and the activations' VALU work: 309 us there,
+// 3.1 TB/s (326 with the residual asked for in the epilogue; four stages or 64-row blocks 311 - 332); the staged form of this kernel, with
+// the intermediate through LDS, took 461 - 498.
+template <int C, int NW, int MT, int S>
+__global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaArgs a1, ConvDmaArgs a2, int H) {
+    constexpr int BM = 16 * MT * NW, R = BM + 64, NT = C / 16, NP = NT / 2, NCK = C / 32, TAPS = 7;
+    constexpr int SA = 2 * R * 64, SW = C * 64, CA = SA / 1024, CW = SW / 1024, NA = (CA + NW - 1) / NW, NB = (CW + NW - 1) / NW;
+    constexpr int AT = (NA + TAPS - S + 1) / (TAPS - S + 2), AN = (NA + AT - 1) / AT;      // requests for rows per tap, taps that make them
+    static_assert(AN <= TAPS - S + 2, "a chunk's rows are asked for by the taps that the next chunk's first wait covers");
+    extern __shared__ __attribute__((aligned(1024))) char conv_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    if ((int)blockIdx.x >= a1.tiles8) {
+        conv_job(a1.job, a1.slots, (int)blockIdx.x - a1.tiles8, 64 * NW);
+        return;
+    }
+    const int t = ((int)blockIdx.x & 7) * (a1.tiles8 >> 3) + ((int)blockIdx.x >> 3);
+    if (t >= a1.tm) return;
+    const int m0 = t * BM, fr = lane & 15, fk = lane >> 4;
+    const int b = m0 / a1.L, t0 = m0 - b * a1.L;
+    constexpr int rb = C * 4;
+    // rows t0 - H .. t0 + BM - 1 at LDS rows 0 .. (the buffer's last rows repeat the tile's last one: no tap reads them)
+    const char* xp[NA];
+    int step[NA];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int q = (i * NW + wv) % CA * 64 + lane, pl = q / (R * 4), r = q / 4 % R, pc = (q & 3) ^ ((r >> 1) & 3);
+        int e = t0 - H + r;
+        e = e < t0 + BM ? e : t0 + BM - 1;
+        const bool hist = e < 0 && a1.state && a1.P + e >= 0;
+        const char* p = e >= 0 ? reinterpret_cast<const char*>(a1.x) + ((size_t)b * a1.L + e) * rb
+                               : reinterpret_cast<const char*>(a1.state) + ((size_t)a1.slots[b] * a1.P + a1.P + e) * rb;
+        xp[i] = e >= 0 || hist ? p + pl * C * 2 + pc * 16 : reinterpret_cast<const char*>(g_conv_zero_row);
+        step[i] = e >= 0 || hist ? 64 : 0;
+    }
+    const auto wswz = [](int r) { return ((r >> 1) & 1) | ((r >> 2) & 2); };      // (rows are read as in k_conv_dma's PAIR order)
+    unsigned wo[NB];
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        const int q = (i * NW + wv) % CW * 64 + lane, r = q / 4;
+        wo[i] = (unsigned)(r * C + ((q & 3) ^ wswz(r)) * 8) * 2;
+    }
+    // the residual rows: asked for first where registers allow (their wait is the first rows' own)
+    constexpr bool EARLY = C == 96 && MT == 1;
+    f32x4 res[EARLY ? NP : 1][2];
+    if (EARLY) {
+#pragma unroll
+        for (int p = 0; p < NP; ++p)
+#pragma unroll
+            for (int q = 0; q < 2; ++q)
+                res[p][q] = *reinterpret_cast<const f32x4*>(a2.res + (size_t)(m0 + wv * 16 + fr) * C + p * 32 + fk * 8 + 4 * q);
+    }
+    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)conv_lds;
+    auto rows = [&](int i, int buf) {
+        conv_dma16(xp[i], __builtin_amdgcn_readfirstlane(sbase + buf * SA + (i * NW + wv) % CA * 1024));
+        xp[i] += step[i];
+    };
+    int rt = 0, rc = 0, rs = 0;      // tap, chunk and stage of the next slice; past conv1's chunks: conv2's
+    auto slice = [&]() {
+        const bool second = rc >= NCK;
+        const int kc = second ? (rt < NCK ? rt : NCK - 1) : rc;      // (past the last slice it is asked for again)
+        const size_t at = reinterpret_cast<size_t>(second ? a2.w : a1.w) + ((second ? 0 : rt * C * C) + kc * 32) * 2;
+        const char* base = reinterpret_cast<const char*>((size_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 |
+                                                         (unsigned)__builtin_amdgcn_readfirstlane((int)at));
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const unsigned ld = __builtin_amdgcn_readfirstlane(sbase + 2 * SA + rs * SW + (i * NW + wv) % CW * 1024);
+            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(wo[i]), "s"(base), "s"(ld) : "memory");
+        }
+        rs = rs == S - 1 ? 0 : rs + 1;
+        if (++rt == TAPS && !second) {
+            rt = 0;
+            ++rc;
+        }
+    };
+    f32x4 acc[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < NA; ++i) rows(i, 0);
+#pragma unroll
+    for (int i = 0; i < S - 1; ++i) slice();
+    const int wfr = (fr >> 2) * 8 + (fr & 3), wpiece = (fk ^ wswz(wfr)) * 16;
+    int ws = 0;      // stage of the slice being multiplied
+    auto weights = [&](cbf16x8 (&wf)[NT]) {
+        const char* p = conv_lds + 2 * SA + ws * SW + wfr * 64 + wpiece;
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wf[j] = *reinterpret_cast<const cbf16x8*>(p + ((j >> 1) * 32 + (j & 1) * 4) * 64);
+        ws = ws == S - 1 ? 0 : ws + 1;
+    };
+    auto chunk = [&](int ck, auto last_tag) {
+        constexpr bool LAST = decltype(last_tag)::value;
+        const char* As = conv_lds + (ck & 1) * SA;
+        auto tap = [&](auto tap_tag) {
+            constexpr int T = decltype(tap_tag)::value;
+            // requests younger than this tap's slice: S - 2 slices and what the taps since then asked of the next chunk's rows
+            constexpr int lo = T - S + 2 > 0 ? (T - S + 2) * AT : 0, hi = T * AT < NA ? T * AT : NA, young = (S - 2) * NB + (!LAST && hi > lo ? hi - lo : 0);
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(young) : "memory");
+#pragma unroll
+            for (int q = T * AT; q < (T + 1) * AT; ++q)
+                if (!LAST && q < NA) rows(q, (ck + 1) & 1);
+            slice();
+            const int r0 = wv * MT * 16 + fr + H - a1.off[T];
+            cbf16x8 wf[NT];
+            weights(wf);
+#pragma unroll
+            for (int p = 1; p >= 0; --p)
+#pragma unroll
+                for (int i = 0; i < MT; ++i) {
+                    const int r = r0 + i * 16;
+                    const cbf16x8 af = *reinterpret_cast<const cbf16x8*>(As + (p * R + r) * 64 + (fk ^ ((r >> 1) & 3)) * 16);
+#pragma unroll
+                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af, acc[i][j], 0, 0, 0);
+                }
+        };
+        tap(std::integral_constant<int, 0>{}); tap(std::integral_constant<int, 1>{}); tap(std::integral_constant<int, 2>{});
+        tap(std::integral_constant<int, 3>{}); tap(std::integral_constant<int, 4>{}); tap(std::integral_constant<int, 5>{});
+        tap(std::integral_constant<int, 6>{});
+    };
+    for (int ck = 0; ck + 1 < NCK; ++ck) chunk(ck, std::false_type{});
+    chunk(NCK - 1, std::true_type{});
+    // act2 of the sums, split: the operand of conv2 (channels 32 p + 8 fk + 0..7 of the lane's row)
+    cbf16x8 y[MT][NP][2];
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        const int c = p * 32 + fk * 8;
+        float bi[8], al[8], ib[8];
+#pragma unroll
+        for (int q = 0; q < 2; ++q) {
+            const f32x4 tb = a1.bias ? *reinterpret_cast<const f32x4_a4*>(a1.bias + c + 4 * q) : (f32x4){0.f, 0.f, 0.f, 0.f};
+            const f32x4 ta = *reinterpret_cast<const f32x4_a4*>(a1.sn_alpha + c + 4 * q), ti = *reinterpret_cast<const f32x4_a4*>(a1.sn_invb + c + 4 * q);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) { bi[4 * q + e] = tb[e]; al[4 * q + e] = ta[e]; ib[4 * q + e] = ti[e]; }
+        }
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            unsigned h[4], m[4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float v0 = snake_f(acc[i][2 * p + e / 2][e % 2 * 2] + bi[2 * e], al[2 * e], ib[2 * e]);
+                const float v1 = snake_f(acc[i][2 * p + e / 2][e % 2 * 2 + 1] + bi[2 * e + 1], al[2 * e + 1], ib[2 * e + 1]);
+                h[e] = pack_bf2(v0, v1);
+                m[e] = pack_bf2(v0 - bflo(h[e]), v1 - bfhi(h[e]));
+            }
+            y[i][p][0] = as_cbf8(make_uint4(h[0], h[1], h[2], h[3]));
+            y[i][p][1] = as_cbf8(make_uint4(m[0], m[1], m[2], m[3]));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int k = 0; k < NP; ++k) {
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * NB) : "memory");
+        slice();
+        cbf16x8 wf[NT];
+        weights(wf);
+#pragma unroll
+        for (int p = 1; p >= 0; --p)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], y[i][k][p], acc[i][j], 0, 0, 0);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (the repeated last slices: nothing may land after the block has ended)
+#pragma unroll
+    for (int p = 0; p < NP; ++p) {
+        f32x4 v[MT][2];
+#pragma unroll
+        for (int i = 0; i < MT; ++i) { v[i][0] = acc[i][2 * p]; v[i][1] = acc[i][2 * p + 1]; }
+        conv_dma_out<false, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
+    }
+}
+
 // Few-row variant (M <= 48: the transformer and the first upsampling stages of a single request's chunk): tile
 // 16(M) x 64(N), one n-tile per wave, K walked in BK-wide chunks (128 where Cin allows) with the same one-step
 // register prefetch.  These stages run a handful of blocks: time = number of dependent K steps, so the steps are wide.
@@ -925,13 +906,7 @@ __global__ __launch_bounds__(256) void k_conv_gemm_skinny(ConvGemmArgs a) {
         if (a.out) a.out[o] = v;
         if (a.out2) {
             const float sv2 = snake_f(v, a.sn_alpha[n % a.sn_mod], a.sn_invb[n % a.sn_mod]);
-            if (a.out2_s2) {
-                const int cw = a.sn_mod, j = n / cw, c = n - j * cw;
-                bf16_t* r16 = reinterpret_cast<bf16_t*>(a.out2 + (size_t)m * a.N) + (size_t)j * 2 * cw;
-                split2(sv2, r16[c], r16[cw + c]);
-            } else {
-                a.out2[o] = sv2;
-            }
+            a.out2[o] = sv2;
         }
     }
 }
@@ -1681,8 +1656,7 @@ static int conv_dma_launch(hipStream_t st, ConvDmaArgs& a) {
     a.tn = ((EPI == CONV_GLU ? 2 * a.N : a.N) + BN - 1) / BN;
     a.tiles8 = (a.tm * a.tn + 7) & ~7;
     a.mfast = (size_t)a.n_taps * a.N > (size_t)a.M * 2;      // weights larger than rows: each XCD reads its own columns of them
-    const int jobs = a.job.state ? a.job.n * ((a.job.C + threads - 1) / threads) : 0;
-    hipLaunchKernelGGL(kern, dim3(a.tiles8 + jobs), dim3(threads), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3(a.tiles8 + conv_job_blocks(a.job, threads)), dim3(threads), lds, st, a);
     return VOX_OK;
 }
 // The smallest tile that leaves no CU a second round (the waves of a block share K): a call of few rows is a chain of dependent steps,
@@ -1756,56 +1730,35 @@ static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
     return a.planes == 2 ? conv_dma_pick<2, 0>(st, a) : conv_dma_pick<1, 0>(st, a);
 }
 
-// A residual unit as ONE launch (k_res_unit) where the tile can cover all channels and the stage has enough rows to fill the chip;
-// *fused = 0 and nothing launched otherwise (the caller then runs the two convs).  x: the S2 activated input rows; h: the fp32
-// residual stream, updated in place; out2: the NEXT consumer's activation of the new h — must not alias x.
-static bool res_unit_on() {
-    static const bool on = [] { const char* e = getenv("VOX_RES_UNIT"); return !(e && e[0] == '0'); }();
-    return on;
+// A residual unit as ONE launch (k_conv_unit) where its tile can cover all channels and the rows fill the chip; *fused = 0 and nothing
+// launched otherwise (the caller then runs the two convs).  a1: conv1 with act2 (sn_*), a2: conv2 with res, out and the NEXT consumer's
+// activation, whose rows must not be a1's: a neighbouring tile still reads its look-back there.  (a1.job is done by extra blocks.)
+template <int C, int NW, int MT, int S>
+static int conv_unit_launch(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int H) {
+    constexpr int BM = 16 * MT * NW, lds = 2 * 2 * (BM + 64) * 64 + S * C * 64;
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    const auto kern = k_conv_unit<C, NW, MT, S>;
+    if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    a1.tm = a1.M / BM;
+    a1.tiles8 = (a1.tm + 7) & ~7;
+    hipLaunchKernelGGL(kern, dim3(a1.tiles8 + conv_job_blocks(a1.job, 64 * NW)), dim3(64 * NW), lds, st, a1, a2, H);
+    return VOX_OK;
 }
-// (measured at 614 k / 205 k rows, B = 32: the 96-channel unit 544 -> 390-430 us fused; the 192-channel unit with the 64 x 192 tile it
-// needs 482 -> 500 us — its two launches stay.  VOX_RES_UNIT_192=1 fuses it all the same, for timing.)
-static bool res_unit_192() {
-    static const bool on = [] { const char* e = getenv("VOX_RES_UNIT_192"); return e && e[0] == '1'; }();
-    return on;
-}
-static int conv_unit(hipStream_t st, const vox_conv_w& w1, const vox_conv_w& w2, const float* x, const float* state, const int* slots, int n, int L,
-                     int P, const int* offs, const vox_snake_w& act2, const float* h, float* ho, float* out2, const vox_snake_w* nx, int out2_s2,
-                     int* fused) {
+static int conv_unit(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int* fused) {
     *fused = 0;
-    const int C = w1.n;
-    if (!res_unit_on() || g_conv_planes != 2 || w1.n_taps < 2 || w1.n_taps > CG_MAXTAPS || w2.n_taps != 1 || w1.cin != C ||
-        w2.cin != C || w2.n != C || (C != 96 && !(C == 192 && res_unit_192())) || out2 == x || !nx)
+    const int C = a1.N;
+    if (g_conv_planes != 2 || a1.n_taps != 7 || a2.n_taps != 1 || a1.Cin != C || a2.Cin != C || a2.N != C || (C != 96 && C != 192) ||
+        a2.out2 == a1.x || a1.bias_mod != C || a2.bias_mod != C || !a1.sn_alpha)
         return VOX_OK;
     int H = 0, omin = 0;
-    for (int k = 0; k < w1.n_taps; ++k) { H = offs[k] > H ? offs[k] : H; omin = offs[k] < omin ? offs[k] : omin; }
-    const int M = n * L, bm = C == 96 ? 128 : 64;
-    if (omin < 0 || H > 64 || L % bm || M / bm < 256) return VOX_OK;
-    ConvGemmArgs a1{}, a2{};
-    a1.x = x; a1.state = state; a1.slots = slots; a1.w = (const bf16_t*)w1.w; a1.bias = w1.bias; a1.M = M; a1.N = C; a1.Cin = C; a1.L = L; a1.P = P;
-    a1.n_taps = w1.n_taps; a1.planes = 2; a1.x_s2 = 1; a1.bias_mod = w1.bias_mod > 0 ? w1.bias_mod : C;
-    a1.sn_alpha = act2.alpha; a1.sn_invb = act2.inv_beta; a1.sn_mod = C;
-    for (int k = 0; k < w1.n_taps; ++k) a1.off[k] = offs[k];
-    a2.w = (const bf16_t*)w2.w; a2.bias = w2.bias; a2.res = h; a2.out = ho; a2.M = M; a2.N = C; a2.Cin = C; a2.L = L; a2.n_taps = 1; a2.planes = 2;
-    a2.x_s2 = 1; a2.bias_mod = w2.bias_mod > 0 ? w2.bias_mod : C; a2.out2 = out2; a2.sn_alpha = nx->alpha; a2.sn_invb = nx->inv_beta; a2.sn_mod = C;
-    a2.out2_s2 = out2_s2;
-    const size_t p1 = (size_t)(2 * (bm + H) + 2 * C) * 80, p3 = (size_t)2 * bm * (C + 8) * 2 + (size_t)2 * C * 80;
-    const size_t lds = p1 > p3 ? p1 : p3;
-    const dim3 g(1, M / bm);
-    // (the > 64 KB dynamic-LDS opt-in is a per-device function attribute: the detokenizer may live on a second GPU)
-    static bool attr_done[2][16] = {};
-    int dev_id = 0;
-    (void)hipGetDevice(&dev_id);
-    bool& done = attr_done[C == 96 ? 0 : 1][dev_id & 15];
-    if (C == 96) {
-        if (!done && lds > 64 * 1024) { VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_res_unit<4, 3>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); done = true; }
-        hipLaunchKernelGGL((k_res_unit<4, 3>), g, dim3(256), lds, st, a1, a2, H);
-    } else {
-        if (!done && lds > 64 * 1024) { VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_res_unit<2, 6>), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024)); done = true; }
-        hipLaunchKernelGGL((k_res_unit<2, 6>), g, dim3(256), lds, st, a1, a2, H);
-    }
+    for (int k = 0; k < a1.n_taps; ++k) { H = a1.off[k] > H ? a1.off[k] : H; omin = a1.off[k] < omin ? a1.off[k] : omin; }
+    // 96 channels: always (one request, 19 200 rows: 27 -> 18 us; 614 400 rows: 600 -> 309).  192 channels: from a tile per CU on (204 800
+    // rows: 424 -> 325; 6 400 rows, 100 tiles: 28 -> 30, there the two launches stay)
+    if (omin < 0 || H > 64 || a1.L % 64 || !a2.res || (C == 192 && a1.M / 64 < 256)) return VOX_OK;
     *fused = 1;
-    return VOX_OK;
+    if (C == 192) return conv_unit_launch<192, 4, 1, 3>(st, a1, a2, H);
+    if (a1.L % 128 == 0 && a1.M / 128 >= 256) return conv_unit_launch<96, 8, 1, 3>(st, a1, a2, H);
+    return conv_unit_launch<96, 4, 1, 3>(st, a1, a2, H);
 }
 
 static void snake(hipStream_t st, const float* x, const vox_snake_w& s, float* y, size_t rows, int C) {
@@ -2114,25 +2067,25 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
             const int offd[7] = {6 * d, 5 * d, 4 * d, 3 * d, 2 * d, d, 0};
             const vox_snake_w* nx = u < 2 ? &bw.res[u + 1].act1 : (b < 3 ? &w.blocks[b + 1].snake0 : &w.final_snake);
             float *y = take(const_cast<float*>(job.x)), *ho = u < 2 ? h : nullptr;      // (after unit 2 only the activation of h goes on)
-            // the whole unit in one launch where the tile covers all channels (k_res_unit): the activated intermediate stays on chip
+            ConvDmaArgs a1 = conv(rw.conv1, x, m->st_ru[b][u], 6 * d, offd);      // y = act2(conv1(x))
+            act_out(a1, y, rw.act2, cout);
+            ConvDmaArgs a2 = conv(rw.conv2, y, nullptr, 0, nullptr);               // h += conv2(y), and the next consumer's activation of it
+            a2.res = h;
+            a2.out = ho;
+            act_out(a2, y, *nx, cout, !last);                                      // (the final conv reads fp32 rows)
             int fused = 0;
-            VOX_TRY(conv_unit(st, rw.conv1, rw.conv2, x, m->st_ru[b][u], slots, n, L, 6 * d, offd, rw.act2, h, ho, y, nx, !last, &fused));
+            a1.job = job;
+            VOX_TRY(conv_unit(st, a1, a2, &fused));
             if (fused) {
-                flush();
                 later(m->st_ru[b][u], x, 6 * d, cout);
                 put(x);
                 x = y;
                 continue;
             }
-            ConvDmaArgs a1 = conv(rw.conv1, x, m->st_ru[b][u], 6 * d, offd);      // y = act2(conv1(x))
-            act_out(a1, y, rw.act2, cout);
             VOX_TRY(run(a1));
             later(m->st_ru[b][u], x, 6 * d, cout);
-            float* z = take(nullptr);                                              // h += conv2(y); z = the next consumer's activation of it
-            ConvDmaArgs a2 = conv(rw.conv2, y, nullptr, 0, nullptr);
-            a2.res = h;
-            a2.out = ho;
-            act_out(a2, z, *nx, cout, !last);                                      // (the final conv reads fp32 rows)
+            float* z = take(nullptr);
+            a2.out2 = z;
             VOX_TRY(run(a2));
             put(x);
             put(y);
