@@ -75,6 +75,7 @@ struct ConvGemmArgs {
     // significand bits; the same 4 * Cin bytes as the fp32 row, so buffers, history state and k_state_update are format-agnostic).
     // The producing epilogue splits each value ONCE (out2_s2); the consumers (k_conv_dma, k_conv_unit) read plain bf16 — the per-tap
     // split of fp32 rows made the many-row decoder convs VALU-bound (MFMA 16 % busy).
+    // NP = 3: "S3" rows, [h][m][l], 6 * Cin bytes, the value itself.
     int out2_s2;
     int dev;               // development builds (-DVOX_DEV_KNOBS, VOX_CODEC_DEV): 1 skip the K loop, 2 no out2 stores, 4 no out stores, 8 no residual loads
 };
@@ -328,7 +329,8 @@ struct ConvDmaArgs : ConvGemmArgs {
     int tm, tn, tiles8, mfast;      // tiles along M and N; their number rounded up to 8; 1: the blocks of an XCD walk the rows first
     const float* rms_x;    // fp32 rows [M, Cin] whose 1 / rms scales the sums of row m (the rows' RMSNorm, its weight already in x), or NULL
     float rms_eps;
-    const float* nw;       // out2 <- S2 of v * nw[n] (no activation), or NULL
+    const float* nw;       // out2 <- terms of v * nw[n] (no activation), or NULL
+    int elu;               // out2 <- ELU of v
     ConvJob job;
 };
 __device__ uint4 g_conv_zero_row[1];        // what a tap reads outside the chunk and its history
@@ -337,26 +339,28 @@ __device__ __forceinline__ void conv_dma16(const char* p, unsigned lds) {
     asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
 }
 typedef f32x4 f32x4_a4 __attribute__((aligned(4)));       // (per-channel constants are where the caller's tensors have them)
-// W neighbouring channels of a row as its two terms
-template <int W>
-__device__ __forceinline__ void conv_put_s2(bf16_t* row, int width, int c, const float (&v)[W]) {
-    unsigned h[W / 2], m[W / 2];
+// W neighbouring channels of a row as its T terms
+template <int T, int W>
+__device__ __forceinline__ void conv_put_terms(bf16_t* row, int width, int c, const float (&v)[W]) {
+    float r[W];
 #pragma unroll
-    for (int e = 0; e < W / 2; ++e) {
-        h[e] = pack_bf2(v[2 * e], v[2 * e + 1]);
-        m[e] = pack_bf2(v[2 * e] - bflo(h[e]), v[2 * e + 1] - bfhi(h[e]));
-    }
-    if constexpr (W == 8) {
-        *reinterpret_cast<uint4*>(row + c) = make_uint4(h[0], h[1], h[2], h[3]);
-        *reinterpret_cast<uint4*>(row + width + c) = make_uint4(m[0], m[1], m[2], m[3]);
-    } else {
-        *reinterpret_cast<uint2*>(row + c) = make_uint2(h[0], h[1]);
-        *reinterpret_cast<uint2*>(row + width + c) = make_uint2(m[0], m[1]);
+    for (int e = 0; e < W; ++e) r[e] = v[e];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+        unsigned h[W / 2];
+#pragma unroll
+        for (int e = 0; e < W / 2; ++e) {
+            h[e] = pack_bf2(r[2 * e], r[2 * e + 1]);
+            r[2 * e] -= bflo(h[e]);
+            r[2 * e + 1] -= bfhi(h[e]);
+        }
+        if constexpr (W == 8) *reinterpret_cast<uint4*>(row + (size_t)t * width + c) = make_uint4(h[0], h[1], h[2], h[3]);
+        else *reinterpret_cast<uint2*>(row + (size_t)t * width + c) = make_uint2(h[0], h[1]);
     }
 }
 // The epilogue of W neighbouring channels (n ..) of MT rows (m, m + 16, ..) that one lane holds: constants once, every row's residual
 // requested ahead of the first store, 16-byte accesses throughout.
-template <bool GELU, int W, int MT>
+template <int T, bool GELU, int W, int MT>
 __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n,
                                              const f32x4* res_ready = nullptr) {
     if (n >= a.N) return;          // (N and the group width are multiples of W)
@@ -405,10 +409,11 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
 #pragma unroll
         for (int e = 0; e < W; ++e) {
             if (a.sn_alpha) v[e] = snake_f(v[e], al[e], ib[e]);
+            else if (a.elu) v[e] = v[e] > 0.0f ? v[e] : expm1f(v[e]);
             else if (a.nw) v[e] *= nw[e];
         }
         if (a.out2_s2) {
-            conv_put_s2<W>(reinterpret_cast<bf16_t*>(a.out2 + (size_t)(m + 16 * i) * a.N) + (size_t)cj * 2 * a.sn_mod, a.sn_mod, cc, v);
+            conv_put_terms<T>(reinterpret_cast<bf16_t*>(a.out2) + ((size_t)(m + 16 * i) * a.N + (size_t)cj * a.sn_mod) * T, a.sn_mod, cc, v);
         } else {
 #pragma unroll
             for (int q = 0; q < W / 4; ++q) *reinterpret_cast<float4*>(a.out2 + o + 4 * q) = make_float4(v[4 * q], v[4 * q + 1], v[4 * q + 2], v[4 * q + 3]);
@@ -423,7 +428,7 @@ __device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x
         const float gv = g[e] * rms, uv = u[e] * rms;
         v[e] = (gv / (1.0f + expf(-gv))) * uv;
     }
-    conv_put_s2<4>(reinterpret_cast<bf16_t*>(a.out2 + (size_t)m * a.N), a.N, n, v);
+    conv_put_terms<2>(reinterpret_cast<bf16_t*>(a.out2) + (size_t)m * a.N * 2, a.N, n, v);
 }
 #define CONV_GELU 1
 #define CONV_GLU 2
@@ -447,7 +452,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     if (t >= a.tm * a.tn) return;
     const int m0 = (a.mfast ? t % a.tm : t / a.tn) * BM, n0 = (a.mfast ? t / a.tm : t % a.tn) * BN;      // (glu: n0 counts gate and up columns)
     const int wk = wv % WK, wmn = wv / WK, wm = wmn / WN, wn = wmn % WN, fr = lane & 15, fk = lane >> 4;
-    const int rb = a.Cin * 4;
+    const int rb = a.Cin * (NP == 3 ? 6 : 4);
     // The weights are the first operand of the MFMA: a lane's four sums are neighbouring channels of one row.  PAIR: tiles j and j + 1 take the
     // weight rows 8 q + 0..3 and 8 q + 4..7 (q = 0..3), so that they hold eight neighbouring channels together.
     const auto wswz = [](int r) {
@@ -591,7 +596,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
                     for (int q = 0; q < P; ++q) v[i][q] = acc[i][j + q];
-                conv_dma_out<EPI == CONV_GELU, 4 * P, MT>(a, v, rms, m0 + rl, n);
+                conv_dma_out<NP == 3 ? 3 : 2, EPI == CONV_GELU, 4 * P, MT>(a, v, rms, m0 + rl, n);
             } else {
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
@@ -599,7 +604,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                         f32x4 v[1][P];
 #pragma unroll
                         for (int q = 0; q < P; ++q) v[0][q] = sum(i * NT + j + q);
-                        conv_dma_out<EPI == CONV_GELU, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
+                        conv_dma_out<NP == 3 ? 3 : 2, EPI == CONV_GELU, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
                     }
             }
         }
@@ -784,7 +789,7 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
         f32x4 v[MT][2];
 #pragma unroll
         for (int i = 0; i < MT; ++i) { v[i][0] = acc[i][2 * p]; v[i][1] = acc[i][2 * p + 1]; }
-        conv_dma_out<false, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
+        conv_dma_out<2, false, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
     }
 }
 
@@ -1102,31 +1107,35 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
 // ================================================================================================
 // small kernels
 // ================================================================================================
-// element c of row `row` of a C-wide activation: fp32, or the two terms of an S2 row
-__device__ __forceinline__ void put_row(float* y, size_t row, int C, int c, float v, int s2) {
-    if (s2) {
-        bf16_t* r16 = reinterpret_cast<bf16_t*>(y + row * C);
-        split2(v, r16[c], r16[C + c]);
-    } else {
+// element c of row `row` of a C-wide activation: fp32 (terms == 0), or the two / three terms of an S2 / S3 row
+__device__ __forceinline__ void put_row(float* y, size_t row, int C, int c, float v, int terms) {
+    if (terms == 0) {
         y[row * C + c] = v;
+        return;
+    }
+    bf16_t* r16 = reinterpret_cast<bf16_t*>(y) + row * C * terms + c;
+    for (int t = 0; t < terms; ++t) {
+        const bf16_t h = f2bf(v);
+        r16[(size_t)t * C] = h;
+        v -= bf2f(h);
     }
 }
 // RVQ decode: q0 = emb[0][code0], qr = sum_{k>=1} emb[k][code_k] (sequential in k)      qwen3_codec.py:1204-1210
 __global__ __launch_bounds__(256) void k_rvq(const int* codes, int code_stride, const float* emb, int Q, int bins, int vq,
-                                             float* q0, float* qr, int s2) {
+                                             float* q0, float* qr, int terms) {
     const int row = blockIdx.x;
     const int* cr = codes + (size_t)row * code_stride;
     for (int d = threadIdx.x; d < vq; d += 256) {
         int c0 = cr[0];
         c0 = c0 < 0 ? 0 : (c0 >= bins ? bins - 1 : c0);          // postprocess clamps to [0, bins-1] (qwen3_tts.py:2027)
-        put_row(q0, row, vq, d, emb[((size_t)c0) * vq + d], s2);
+        put_row(q0, row, vq, d, emb[((size_t)c0) * vq + d], terms);
         float s = 0.0f;
         for (int k = 1; k < Q; ++k) {
             int c = cr[k];
             c = c < 0 ? 0 : (c >= bins ? bins - 1 : c);
             s = s + emb[((size_t)k * bins + c) * vq + d];
         }
-        put_row(qr, row, vq, d, s, s2);
+        put_row(qr, row, vq, d, s, terms);
     }
 }
 
@@ -1204,7 +1213,7 @@ __global__ __launch_bounds__(256) void k_codec_rope_kv(float* qkv, bf16_t* ring,
 // One block per (head, request): K/V ring tile in LDS (row stride D+1: conflict-free both for "lane = key" in the
 // scores and "lane = dim" in PV), the T queries of the chunk spread over the four waves.
 __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16_t* ring, const int* slots, const long* pos,
-                                                    float* out, int T, int H, int D, int Wn, int s2) {
+                                                    float* out, int T, int H, int D, int Wn, int terms) {
     extern __shared__ float sm[];   // K [Wn][D+1], V [Wn][D+1], Q [T][D], P [4][Wn]
     const int LD = D + 1;
     float* Ks = sm;
@@ -1259,7 +1268,7 @@ __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16
         for (int d = lane; d < D; d += 64) {
             float o = 0.0f;
             for (int j = 0; j < nvis; ++j) o = fmaf(P[j], Vs[j * LD + d], o);
-            put_row(out, (size_t)(b * T + i), HD, h * D + d, o / ls, s2);
+            put_row(out, (size_t)(b * T + i), HD, h * D + d, o / ls, terms);
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
@@ -1276,7 +1285,7 @@ __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16
 // (profiles/round4_codec_attn_ab.txt).
 template <int D>
 __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* ring, const int* slots, const long* pos, float* out, int T,
-                                                     int H, int Wn, const float* inv_freq, int s2) {
+                                                     int H, int Wn, const float* inv_freq, int terms) {
     extern __shared__ float sm[];   // K [Wn][D+1], V [Wn][D+1], Q [T][D], P [T][Wn]
     constexpr int LD = D + 1, half = D / 2, CH = D / 8;
     float* Ks = sm;
@@ -1374,7 +1383,7 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
                 for (int u = 0; u < 8; ++u) o = fmaf(pv[u], vv[u], o);
             }
             for (; j < nvis; ++j) o = fmaf(P[j], Vs[j * LD + d], o);
-            put_row(out, (size_t)(b * T + i), HD, h * D + d, o / ls, s2);
+            put_row(out, (size_t)(b * T + i), HD, h * D + d, o / ls, terms);
         }
     }
 }
@@ -1398,7 +1407,7 @@ __global__ __launch_bounds__(256) void k_silu_mul_f32(const float* gu, float* h,
 // ConvNeXt front: causal depthwise conv k=7 (+bias) then LayerNorm over channels.   qwen3_codec.py:447-450
 __global__ __launch_bounds__(256) void k_dwconv_ln(const float* x, const float* state, const int* slots, const float* w,
                                                    const float* wb, const float* lnw, const float* lnb, float* y, int L,
-                                                   int C, float eps, int s2) {
+                                                   int C, float eps, int terms) {
     __shared__ float red[4];
     extern __shared__ float ybuf[];   // [C]
     const int row = blockIdx.x, b = row / L, t = row % L;
@@ -1422,7 +1431,7 @@ __global__ __launch_bounds__(256) void k_dwconv_ln(const float* x, const float* 
         sq += d * d;
     }
     const float rstd = rsqrtf(block_sum(sq, red) / (float)C + eps);
-    for (int c = threadIdx.x; c < C; c += 256) put_row(y, (size_t)row, C, c, (ybuf[c] - mean) * rstd * lnw[c] + lnb[c], s2);
+    for (int c = threadIdx.x; c < C; c += 256) put_row(y, (size_t)row, C, c, (ybuf[c] - mean) * rstd * lnw[c] + lnb[c], terms);
 }
 
 // final causal conv k=7, C -> 1, + clamp(-1,1).  One wave per output sample group.
@@ -1443,53 +1452,87 @@ __global__ __launch_bounds__(256) void k_final_conv(const float* x, const float*
     if (lane == 0) out[(size_t)b * L + t] = fminf(1.0f, fmaxf(-1.0f, acc + bias));
 }
 
-// The same conv for many rows: 128 consecutive outputs of one request per block (2 waves, one output per lane).  The 134 input rows the
-// block needs are staged in LDS once (coalesced 16-byte loads; row stride C + 1 words, so the 64 lanes of a wave — 64 consecutive rows,
-// same channel — hit 64 different banks), the weights beside them (read as broadcasts).  The one-wave-per-output form above re-reads
-// every input row 7 times through 4-byte strided loads with an integer division per element: 518 us for 614 k outputs (236 MB of input).
-// Per output: four partial sums over the channel residues mod 4, taps outermost, added ((s0 + s1) + (s2 + s3)) + bias.
-__global__ __launch_bounds__(128) void k_final_conv_rows(const float* x, const float* state, const int* slots, const float* w,
-                                                         float bias, float* out, int L, int C) {
-    extern __shared__ __attribute__((aligned(16))) float fsm[];      // [134][C + 1] rows, then [7][C] weights (tap-major)
-    const int b = blockIdx.y, t0 = blockIdx.x * 128, LD = C + 1;
-    float* ws = fsm + 134 * LD;
-    const float* st = state + (size_t)slots[b] * 6 * C;
+// The last conv of a decoder (K taps, C = 32 V channels -> 1), every row read once: out[t] = bias + sum_k (w_k . x[t - (K-1) + k]).  Eight lanes
+// hold a row in V 16-byte pieces each and make its K products together (the weights stay in their registers); the K sums of a row go to
+// LDS, an output adds K of them.  32 IT rows per block, the first K - 1 of them only for their products.  Rows before the chunk come from
+// the history (NULL: zero).  Memory bound: 614 400 rows of 96 channels 155 -> 72 us, 307 200 of 64 (K = 3) 88 -> 24 (one output per lane
+// out of LDS rows, and one wave per output, before).
+template <int K, int V, int IT, bool CLAMP>
+__global__ __launch_bounds__(256) void k_final_taps(const float* x, const float* state, const int* slots, const float* w, float bias, float* out, int L) {
+    constexpr int C = 32 * V, ROWS = 32 * IT, OUT = ROWS - (K - 1);
+    __shared__ __attribute__((aligned(16))) float ws[K * C];
+    __shared__ float part[ROWS * K];
+    const int b = blockIdx.y, t0 = blockIdx.x * OUT, tid = threadIdx.x, l8 = tid & 7, rg = tid >> 3;
     const float* xb = x + (size_t)b * L * C;
-    const int c4n = C >> 2, total = 134 * c4n;
-    for (int e0 = 0; e0 < total; e0 += 128 * 8) {      // eight requests per thread in flight, then their LDS stores
-        float4 v[8];
+    const float* sb = state ? state + (size_t)slots[b] * (K - 1) * C : nullptr;
+    for (int e = tid; e < K * C; e += 256) ws[e % K * C + e / K] = w[e];
+    float4 v[IT < 4 ? IT : 4][V];
+    const auto fetch = [&](int it0) {
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = e0 + i * 128 + threadIdx.x, j = e / c4n, c4 = e - j * c4n, r = t0 + j;      // r indexes [state(6) ++ x]
-            v[i] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (e < total) {
-                if (r < 6) v[i] = *reinterpret_cast<const float4*>(st + (size_t)r * C + c4 * 4);
-                else if (r - 6 < L) v[i] = *reinterpret_cast<const float4*>(xb + (size_t)(r - 6) * C + c4 * 4);
-            }
-        }
+        for (int i = 0; i < (IT < 4 ? IT : 4); ++i) {
+            const int r = t0 - (K - 1) + (it0 + i) * 32 + rg;
+            const float* p = r >= 0 ? (r < L ? xb + (size_t)r * C : nullptr) : (sb ? sb + (size_t)(K - 1 + r) * C : nullptr);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int e = e0 + i * 128 + threadIdx.x, j = e / c4n, c4 = e - j * c4n;
-            if (e < total) {
-                float* d = fsm + j * LD + c4 * 4;
-                d[0] = v[i].x; d[1] = v[i].y; d[2] = v[i].z; d[3] = v[i].w;
-            }
+            for (int q = 0; q < V; ++q) v[i][q] = p ? *reinterpret_cast<const float4*>(p + (q * 8 + l8) * 4) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
-    }
-    for (int e = threadIdx.x; e < 7 * C; e += 128) { const int k = e / C, c = e - k * C; ws[e] = w[c * 7 + k]; }
+    };
+    fetch(0);
     __syncthreads();
-    const int t = t0 + threadIdx.x;
-    if (t >= L) return;
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    for (int k = 0; k < 7; ++k) {
-        const float* xr = fsm + (threadIdx.x + k) * LD;
-        const float* wk = ws + k * C;
-        for (int c = 0; c < C; c += 4) {
-            s0 = __fmaf_rn(wk[c], xr[c], s0); s1 = __fmaf_rn(wk[c + 1], xr[c + 1], s1);
-            s2 = __fmaf_rn(wk[c + 2], xr[c + 2], s2); s3 = __fmaf_rn(wk[c + 3], xr[c + 3], s3);
+    float4 wr[K][V];
+#pragma unroll
+    for (int k = 0; k < K; ++k)
+#pragma unroll
+        for (int q = 0; q < V; ++q) wr[k][q] = *reinterpret_cast<const float4*>(ws + k * C + (q * 8 + l8) * 4);
+#pragma unroll
+    for (int it0 = 0; it0 < IT; it0 += 4) {
+        if (it0) fetch(it0);
+#pragma unroll
+        for (int i = 0; i < (IT < 4 ? IT : 4); ++i) {
+            float s[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                s[k] = 0.0f;
+                if (k < K) {
+#pragma unroll
+                    for (int q = 0; q < V; ++q) {
+                        s[k] = __fmaf_rn(wr[k][q].x, v[i][q].x, s[k]); s[k] = __fmaf_rn(wr[k][q].y, v[i][q].y, s[k]);
+                        s[k] = __fmaf_rn(wr[k][q].z, v[i][q].z, s[k]); s[k] = __fmaf_rn(wr[k][q].w, v[i][q].w, s[k]);
+                    }
+                }
+            }
+            // the eight lanes' sums: halves are exchanged, so that lane k ends with tap k
+#pragma unroll
+            for (int o = 4; o >= 1; o >>= 1)
+#pragma unroll
+                for (int k = 0; k < o; ++k) {
+                    const bool up = l8 & o;
+                    const float keep = up ? s[k + o] : s[k], give = up ? s[k] : s[k + o];
+                    s[k] = keep + __shfl_xor(give, o, 64);
+                }
+            if (l8 < K) part[((it0 + i) * 32 + rg) * K + l8] = s[0];
         }
     }
-    out[(size_t)b * L + t] = fminf(1.0f, fmaxf(-1.0f, ((s0 + s1) + (s2 + s3)) + bias));
+    __syncthreads();
+    const int t = t0 + tid;
+    if (tid >= OUT || t >= L) return;
+    float o = 0.0f;
+#pragma unroll
+    for (int k = 0; k < K; ++k) o += part[(tid + k) * K + k];
+    o += bias;
+    out[(size_t)b * L + t] = CLAMP ? fminf(1.0f, fmaxf(-1.0f, o)) : o;
+}
+// few outputs: 64-row blocks, so that one request still fills the chip
+template <int K, bool CLAMP>
+static bool final_taps(hipStream_t st, const float* x, const float* state, const int* slots, const float* w, float bias, float* out, int n, int L, int C) {
+    const bool few = (long)n * ((L + 255) / 256) < 512;
+#define VOX_FT(V_) \
+    case V_: \
+        if (few) hipLaunchKernelGGL((k_final_taps<K, V_, 2, CLAMP>), dim3((L + 64 - K) / (65 - K), n), dim3(256), 0, st, x, state, slots, w, bias, out, L); \
+        else hipLaunchKernelGGL((k_final_taps<K, V_, 8, CLAMP>), dim3((L + 256 - K) / (257 - K), n), dim3(256), 0, st, x, state, slots, w, bias, out, L); \
+        return true;
+    if (C % 32 == 0) switch (C / 32) { VOX_FT(1) VOX_FT(2) VOX_FT(3) VOX_FT(4) }
+#undef VOX_FT
+    return false;
 }
 
 // ================================================================================================
@@ -1665,6 +1708,7 @@ static int conv_dma_launch(hipStream_t st, ConvDmaArgs& a) {
 //   M = 10: 3072 x 512 7.1 -> 4.4, 512 x 1024 10.4 -> 4.9 | 40: 1024 x 4096 33 -> 7.8, 1536 x 7 x 1024 58 -> 14, 6144 x 2 x 1536 31 -> 14
 //   M = 320: 768 x 7 x 768 48 -> 16, 1920 x 2 x 768 22 -> 12 | 1600: 384 x 7 x 384 36 -> 18 | 6400: 192 x 7 x 192 30 -> 18.5
 //   M = 1280: 1536 x 7 x 1024 157 -> 72, 6144 x 2 x 1536 157 -> 84 | 10240: 768 x 7 x 768 194 -> 134, 1920 x 2 x 768 168 -> 131
+//   three-term rows: M = 320: 4096 x 2 x 1024 45 -> 30 (64 x 128; 64 x 64), 76 800: 256 x 2 x 128 67 (128 x 128), 307 200: 32 x 3 x 64 53
 //   M = 51200: 384 x 7 x 384 250 -> 193 (rounds of 256 tiles decide: 128 x 256 leaves a quarter of its columns empty there, > 245)
 template <int NP, int EPI>
 static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
@@ -1675,24 +1719,43 @@ static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
         if constexpr (EPI != CONV_GLU)
             if (tiles(16, 16) <= 256) return conv_dma_launch<16, 16, 1, 1, 4, 128, 8, NP, EPI>(st, a);
         if (tiles(16, 32) <= 256) {
-            if (a.Cin % 256 == 0) return conv_dma_launch<16, 32, 1, 1, 8, 256, 4, NP, EPI>(st, a);
+            if (a.Cin % 256 == 0) return conv_dma_launch<16, 32, 1, 1, 8, 256, NP == 3 ? 3 : 4, NP, EPI>(st, a);
             return conv_dma_launch<16, 32, 1, 1, 4, 128, 6, NP, EPI>(st, a);
         }
         if (tiles(16, 64) <= 256) return conv_dma_launch<16, 64, 1, 2, 4, 128, 5, NP, EPI>(st, a);
-        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 4, 128, 4, NP, EPI>(st, a);
-        if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 2, 2, 4, 128, 3, NP, EPI>(st, a);
+        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 4, 128, NP == 3 ? 3 : 4, NP, EPI>(st, a);
+        if constexpr (NP != 3)
+            if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 2, 2, 4, 128, 3, NP, EPI>(st, a);
     }
     if (k64) {
         if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 2, 64, 6, NP, EPI>(st, a);
-        if (tiles(64, 64) <= 512) return conv_dma_launch<64, 64, 2, 2, 1, 64, 3, NP, EPI>(st, a);
+        if constexpr (NP == 3) {
+            if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 2, 2, 2, 64, 4, NP, EPI>(st, a);
+            if (tiles(64, 128) <= 256) return conv_dma_launch<64, 128, 2, 4, 2, 64, 2, NP, EPI>(st, a);
+        } else if (tiles(64, 64) <= 512) {
+            return conv_dma_launch<64, 64, 2, 2, 1, 64, 3, NP, EPI>(st, a);
+        }
     }
-    if constexpr (EPI == 0) {
-        // what the busiest CU multiplies, weighted by how well each tile does it
-        const auto cost = [&](int bm, int bn, double w) { return (double)((tiles(bm, bn) + 255) / 256) * bm * bn * w; };
-        const double c[6] = {cost(128, 256, 1.0), cost(256, 192, 1.0), cost(128, 192, 1.08), cost(128, 128, 1.07), cost(64, 128, 1.17), cost(64, 96, 1.25)};
+    // what the busiest CU multiplies, weighted by how well each tile does it
+    const auto cost = [&](int bm, int bn, double w) { return (double)((tiles(bm, bn) + 255) / 256) * bm * bn * w; };
+    const auto least = [](const double* c, int n) {
         int best = 0;
-        for (int i = 1; i < 6; ++i) best = c[i] < c[best] ? i : best;
-        switch (best) {
+        for (int i = 1; i < n; ++i) best = c[i] < c[best] ? i : best;
+        return best;
+    };
+    if constexpr (NP == 3 && EPI == 0) {
+        const double c[6] = {cost(128, 192, 1.0), cost(128, 128, 1.1), cost(64, 128, 1.25), cost(64, 96, 1.35), cost(64, 64, 1.45), cost(128, 32, 1.7)};
+        switch (least(c, 6)) {
+            case 0: return conv_dma_launch<128, 192, 4, 2, 1, 32, 2, NP, EPI>(st, a);
+            case 1: return conv_dma_launch<128, 128, 4, 2, 1, 32, 2, NP, EPI>(st, a);
+            case 2: return conv_dma_launch<64, 128, 4, 2, 1, 32, 3, NP, EPI>(st, a);
+            case 3: return conv_dma_launch<64, 96, 4, 1, 1, 32, 4, NP, EPI>(st, a);
+            case 4: return conv_dma_launch<64, 64, 2, 2, 1, 32, 4, NP, EPI>(st, a);
+            default: return conv_dma_launch<128, 32, 8, 1, 1, 32, 3, NP, EPI>(st, a);
+        }
+    } else if constexpr (EPI == 0) {
+        const double c[6] = {cost(128, 256, 1.0), cost(256, 192, 1.0), cost(128, 192, 1.08), cost(128, 128, 1.07), cost(64, 128, 1.17), cost(64, 96, 1.25)};
+        switch (least(c, 6)) {
             case 0: return conv_dma_launch<128, 256, 4, 4, 1, 32, 3, NP, EPI>(st, a);
             case 1: return conv_dma_launch<256, 192, 8, 2, 1, 32, 3, NP, EPI>(st, a);
             case 2: return conv_dma_launch<128, 192, 4, 2, 1, 32, 2, NP, EPI>(st, a);
@@ -1702,9 +1765,12 @@ static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
                 return conv_dma_launch<64, 128, 2, 2, 1, 32, 4, NP, EPI>(st, a);
             default: return conv_dma_launch<64, 96, 4, 1, 1, 32, 4, NP, EPI>(st, a);
         }
+    } else if constexpr (NP == 3) {
+        return conv_dma_launch<64, 128, 4, 2, 1, 32, 3, NP, EPI>(st, a);
+    } else {
+        if (k64) return conv_dma_launch<64, 128, 2, 2, 1, 64, 2, NP, EPI>(st, a);
+        return conv_dma_launch<64, 64, 2, 2, 1, 32, 6, NP, EPI>(st, a);
     }
-    if (k64) return conv_dma_launch<64, 128, 2, 2, 1, 64, 2, NP, EPI>(st, a);
-    return conv_dma_launch<64, 64, 2, 2, 1, 32, 6, NP, EPI>(st, a);
 }
 // The operands and the shape of a conv over S2 rows; the caller adds the epilogue (out / out2 / ...) and hands it to conv_s2.
 static ConvDmaArgs conv_s2_args(const vox_conv_w& w, const float* x, const float* state, const int* slots, int n, int L, int P, const int* offs) {
@@ -1726,8 +1792,9 @@ static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
         a.sn_mod = a.N;
         return a.planes == 2 ? conv_dma_pick<2, CONV_GLU>(st, a) : conv_dma_pick<1, CONV_GLU>(st, a);
     }
-    if (epi == CONV_GELU) return a.planes == 2 ? conv_dma_pick<2, CONV_GELU>(st, a) : conv_dma_pick<1, CONV_GELU>(st, a);
-    return a.planes == 2 ? conv_dma_pick<2, 0>(st, a) : conv_dma_pick<1, 0>(st, a);
+    if (epi == CONV_GELU)
+        return a.planes == 3 ? conv_dma_pick<3, CONV_GELU>(st, a) : a.planes == 2 ? conv_dma_pick<2, CONV_GELU>(st, a) : conv_dma_pick<1, CONV_GELU>(st, a);
+    return a.planes == 3 ? conv_dma_pick<3, 0>(st, a) : a.planes == 2 ? conv_dma_pick<2, 0>(st, a) : conv_dma_pick<1, 0>(st, a);
 }
 
 // A residual unit as ONE launch (k_conv_unit) where its tile can cover all channels and the rows fill the chip; *fused = 0 and nothing
@@ -1865,7 +1932,7 @@ int vox_codec_reset_slot(vox_codec* m, void* stream, int slot) {
 }  // extern "C"
 
 // RoPE, the ring's new rows and the attention of layer l: qkv fp32 [nL, 3 HD] -> out [nL, HD] (fp32 or S2 rows)
-static void codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* slots, int n, int L, float* qkv, float* out, int s2) {
+static void codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* slots, int n, int L, float* qkv, float* out, int terms) {
     const vox_codec_config& c = m->cfg;
     const int HD = c.num_heads * c.head_dim;
     bf16_t* ring = m->ring + (size_t)l * m->max_slots * c.window * 2 * HD;
@@ -1874,23 +1941,20 @@ static void codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* 
     const size_t lds2 = (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + L * c.window) * 4;
     if (attn2 && c.head_dim == 64 && L <= c.window && lds2 <= 64 * 1024) {
         hipLaunchKernelGGL(k_codec_attn2<64>, dim3(c.num_heads, n), dim3(256), lds2, st, qkv, ring, slots, m->pos, out, L, c.num_heads, c.window,
-                           m->w.inv_freq, s2);
+                           m->w.inv_freq, terms);
     } else {
         hipLaunchKernelGGL(k_codec_rope_kv, dim3(n * L), dim3(256), 0, st, qkv, ring, slots, m->pos, L, c.num_heads, c.head_dim, c.window,
                            m->w.inv_freq);
         hipLaunchKernelGGL(k_codec_attn, dim3(c.num_heads, n), dim3(256),
                            (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + 4 * c.window) * 4, st, qkv, ring, slots, m->pos, out, L,
-                           c.num_heads, c.head_dim, c.window, s2);
+                           c.num_heads, c.head_dim, c.window, terms);
     }
 }
 // the final conv over x (fp32 rows, activated), its history and the slots' positions (T codec frames on)
 static void codec_final(vox_codec* m, hipStream_t st, const float* x, const int32_t* slots, int n, int T, int L, float* out) {
     const vox_codec_weights& w = m->w;
     const int cl = m->cfg.decoder_dim >> 4;
-    if (L >= 512 && cl % 4 == 0 && (size_t)(134 * (cl + 1) + 7 * cl) * 4 <= 60 * 1024)
-        hipLaunchKernelGGL(k_final_conv_rows, dim3((L + 127) / 128, n), dim3(128), (size_t)(134 * (cl + 1) + 7 * cl) * 4, st, x, m->st_final, slots,
-                           w.final_w, w.final_b, out, L, cl);
-    else
+    if (!final_taps<7, true>(st, x, m->st_final, slots, w.final_w, w.final_b, out, n, L, cl))
         hipLaunchKernelGGL(k_final_conv, dim3((L + 3) / 4, n), dim3(256), 0, st, x, m->st_final, slots, w.final_w, w.final_b, out, L, cl);
     state_update(st, m->st_final, slots, x, n, L, 6, cl);
     hipLaunchKernelGGL(k_pos_advance, dim3((n + 255) / 256), dim3(256), 0, st, m->pos, slots, n, T);
@@ -2006,7 +2070,7 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
     };
     auto rms_in = [&](ConvDmaArgs& a, const float* h) { a.rms_x = h; a.rms_eps = c.rms_eps; };
 
-    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.num_quantizers, c.codebook_size, c.vq_dim, m->q0, m->qr, 1);
+    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.num_quantizers, c.codebook_size, c.vq_dim, m->q0, m->qr, 2);
     { ConvDmaArgs a = conv(w.rvq_first_out, m->q0, nullptr, 0, nullptr); a.out = A; VOX_TRY(run(a)); }
     { ConvDmaArgs a = conv(w.rvq_rest_out, m->qr, nullptr, 0, nullptr); a.res = A; s2_out(a, B); VOX_TRY(run(a)); }
     { ConvDmaArgs a = conv(w.pre_conv, B, m->st_pre, 2, off3); s2_out(a, A); VOX_TRY(run(a)); }             // A [nL, latent]
@@ -2016,7 +2080,7 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
     for (int l = 0; l < c.num_layers; ++l) {
         const vox_codec_layer_w& lw = w.layers[l];
         { ConvDmaArgs a = conv(lw.qkv, D, nullptr, 0, nullptr); rms_in(a, C); a.out = A; VOX_TRY(run(a)); }
-        codec_attention(m, st, l, slots, n, L, A, B, 1);
+        codec_attention(m, st, l, slots, n, L, A, B, 2);
         { ConvDmaArgs a = conv(lw.o, B, nullptr, 0, nullptr); a.res = C; a.scale = lw.scale1; a.out = C; s2_out(a, D, lw.ln2); VOX_TRY(run(a)); }
         { ConvDmaArgs a = conv(lw.gate_up, D, nullptr, 0, nullptr); rms_in(a, C); s2_out(a, A); VOX_TRY(run(a, CONV_GLU)); }
         { ConvDmaArgs a = conv(lw.down, A, nullptr, 0, nullptr); a.res = C; a.scale = lw.scale2; a.out = C;
@@ -2029,7 +2093,7 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
         { ConvDmaArgs a = conv(uw.tconv, A, nullptr, 0, nullptr); a.out = B; VOX_TRY(run(a)); }                     // B [n*2L, latent]
         L *= 2;
         hipLaunchKernelGGL(k_dwconv_ln, dim3(n * L), dim3(256), (size_t)LD * 4, st, B, m->st_dw[u], slots, uw.dw_w, uw.dw_b, uw.ln_w, uw.ln_b, C, L, LD,
-                           1e-6f, 1);
+                           1e-6f, 2);
         later(m->st_dw[u], B, 6, LD);
         { ConvDmaArgs a = conv(uw.pw1, C, nullptr, 0, nullptr); s2_out(a, D); VOX_TRY(run(a, CONV_GELU)); }
         { ConvDmaArgs a = conv(uw.pw2, D, nullptr, 0, nullptr); a.res = B; a.scale = uw.gamma; s2_out(a, A); VOX_TRY(run(a)); }
@@ -2131,7 +2195,7 @@ __global__ __launch_bounds__(256) void k_mimi_upsample(const float* x, const flo
         y[i] = cur * w[c * 4 + j] + prev * w[c * 4 + j + 2];
     }
 }
-__global__ __launch_bounds__(256) void k_layernorm_f32(const float* x, const float* w, const float* b, float* y, int C, float eps) {
+__global__ __launch_bounds__(256) void k_layernorm_f32(const float* x, const float* w, const float* b, float* y, int C, float eps, int terms = 0) {
     __shared__ float red[8];
     const float* xr = x + (size_t)blockIdx.x * C;
     float s = 0.0f;
@@ -2146,7 +2210,7 @@ __global__ __launch_bounds__(256) void k_layernorm_f32(const float* x, const flo
     if ((threadIdx.x & 63) == 0) red[4 + (threadIdx.x >> 6)] = v;
     __syncthreads();
     const float rstd = rsqrtf((red[4] + red[5] + red[6] + red[7]) / (float)C + eps);
-    for (int i = threadIdx.x; i < C; i += 256) y[(size_t)blockIdx.x * C + i] = (xr[i] - mean) * rstd * w[i] + b[i];
+    for (int i = threadIdx.x; i < C; i += 256) put_row(y, blockIdx.x, C, i, (xr[i] - mean) * rstd * w[i] + b[i], terms);
 }
 __global__ __launch_bounds__(256) void k_elu(const float* x, float* y, size_t total) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
@@ -2203,7 +2267,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn(const float* qkv, float* out,
         for (int d = lane; d < D; d += 64) {
             float o = 0.0f;
             for (int jj = 0; jj <= i; ++jj) o = fmaf(P[jj], Vs[jj * LD + d], o);
-            out[((size_t)(b * L + i)) * HD + (size_t)h * D + d] = o / ls;
+            put_row(out, (size_t)(b * L + i), HD, h * D + d, o / ls, 3);
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
@@ -2279,7 +2343,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn_stream(const float* qkv, floa
         for (int d = lane; d < D; d += 64) {
             float o = 0.0f;
             for (int jj = jlo; jj <= jhi; ++jj) o = fmaf(P[jj], vr[(size_t)((lo + jj) % RC) * HD + d], o);
-            out[((size_t)(b * L + i)) * HD + (size_t)h * D + d] = o / ls;
+            put_row(out, (size_t)(b * L + i), HD, h * D + d, o / ls, 3);
         }
         __builtin_amdgcn_wave_barrier();
         __threadfence_block();
@@ -2317,6 +2381,10 @@ struct vox_mimi {
     long* pos = nullptr;
 };
 
+// fp32 rows as S3 rows
+__global__ __launch_bounds__(256) void k_terms3(const float* x, float* y, int C) {
+    for (int c = threadIdx.x; c < C; c += 256) put_row(y, blockIdx.x, C, c, x[(size_t)blockIdx.x * C + c], 3);
+}
 static void elu(hipStream_t st, const float* x, float* y, size_t total) {
     int grid = (int)((total + 255) / 256);
     if (grid > 4096) grid = 4096;
@@ -2342,10 +2410,11 @@ int vox_mimi_create(vox_ctx* ctx, const vox_mimi_config* cfg, const vox_mimi_wei
     }
     const size_t tr = (size_t)2 * max_frames * (3 * cfg->dim > cfg->ffn ? 3 * cfg->dim : cfg->ffn);
     maxf = (maxf > tr ? maxf : tr) * max_batch;
-    bool ok = hipMalloc((void**)&m->q0, (size_t)max_batch * max_frames * cfg->vq_dim * 4) == hipSuccess &&
-              hipMalloc((void**)&m->qr, (size_t)max_batch * max_frames * cfg->vq_dim * 4) == hipSuccess &&
+    // (6 bytes an element: a buffer holds fp32 or S3 rows)
+    bool ok = hipMalloc((void**)&m->q0, (size_t)max_batch * max_frames * cfg->vq_dim * 6) == hipSuccess &&
+              hipMalloc((void**)&m->qr, (size_t)max_batch * max_frames * cfg->vq_dim * 6) == hipSuccess &&
               hipMalloc((void**)&m->zero_slots, (size_t)max_batch * 4) == hipSuccess;
-    for (int i = 0; i < 4; ++i) ok = ok && hipMalloc((void**)&m->buf[i], maxf * 4) == hipSuccess;
+    for (int i = 0; i < 4; ++i) ok = ok && hipMalloc((void**)&m->buf[i], maxf * 6) == hipSuccess;
     if (!ok) return vox_fail(VOX_ERR_NOMEM, "mimi_create: hipMalloc failed");
     VOX_HIP(hipMemset(m->zero_slots, 0, (size_t)max_batch * 4));
     *out = m;
@@ -2361,19 +2430,35 @@ void vox_mimi_destroy(vox_mimi* m) {
 }
 }  // extern "C"
 
-// slots == NULL: stateless chunk (fresh state: the reference's MimiDecoder.decode); else streaming on the given state slots
+// slots == NULL: stateless chunk (fresh state: the reference's MimiDecoder.decode); else streaming on the given state slots.
+// Activations that only convs read are S3 rows (three bf16 terms: the fp32 value), written by whatever produces them; ELU is in the
+// epilogue of the conv in front of it, a conv's history in extra blocks of the next launch (as in codec_chunk_s2).
 static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_stride, const int32_t* slots, int n, int T, float* out) {
     const vox_mimi_config& c = m->cfg;
     const vox_mimi_weights& w = m->w;
     const int C = c.dim, H = c.num_heads, D = c.dim / c.num_heads;
     const bool S = slots != nullptr;
     const int* sl = S ? slots : m->zero_slots;
+    struct PlanesGuard { int saved; PlanesGuard() : saved(g_conv_planes) { g_conv_planes = 3; } ~PlanesGuard() { g_conv_planes = saved; } } pg;
     float *A = m->buf[0], *B = m->buf[1], *Cb = m->buf[2], *Db = m->buf[3];
-    const int off0[1] = {0};
     int L = T;
-    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.n_q, c.bins, c.vq_dim, m->q0, m->qr, 0);
-    VOX_TRY(conv_gemm(st, w.rvq_first_out, m->q0, nullptr, sl, n, L, 0, off0, A, nullptr, nullptr, 0));
-    VOX_TRY(conv_gemm(st, w.rvq_rest_out, m->qr, nullptr, sl, n, L, 0, off0, B, A, nullptr, 0));            // B [nL, dim]
+    ConvJob job{};
+    auto later = [&](float* state, const float* x, int P, int ch) {
+        if (S) job = ConvJob{state, x, L, P, ch / 2 * 3, n};
+    };
+    auto conv = [&](const vox_conv_w& cw, const float* x, const float* state, int P, const int* offs) {
+        return conv_s2_args(cw, x, S ? state : nullptr, sl, n, L, S ? P : 0, offs);
+    };
+    auto run = [&](ConvDmaArgs& a, int epi = 0) {
+        a.job = job;
+        job = ConvJob{};
+        return conv_s2(st, a, epi);
+    };
+    auto terms = [](ConvDmaArgs& a, float* y) { a.out2 = y; a.out2_s2 = 1; };
+    auto elu_out = [](ConvDmaArgs& a, float* y, int ch, int t = 1) { a.out2 = y; a.out2_s2 = t; a.elu = 1; a.sn_mod = ch; };
+    hipLaunchKernelGGL(k_rvq, dim3(n * L), dim3(256), 0, st, codes, code_stride, w.emb, c.n_q, c.bins, c.vq_dim, m->q0, m->qr, 3);
+    { ConvDmaArgs a = conv(w.rvq_first_out, m->q0, nullptr, 0, nullptr); a.out = A; VOX_TRY(run(a)); }
+    { ConvDmaArgs a = conv(w.rvq_rest_out, m->qr, nullptr, 0, nullptr); a.res = A; a.out = B; VOX_TRY(run(a)); }            // B [nL, dim]
     {
         const size_t total = (size_t)n * 2 * L * C;
         int grid = (int)((total + 255) / 256);
@@ -2384,8 +2469,8 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
     L *= 2;
     for (int l = 0; l < c.num_layers; ++l) {                                                                 // h = A
         const vox_mimi_layer_w& lw = w.layers[l];
-        hipLaunchKernelGGL(k_layernorm_f32, dim3(n * L), dim3(256), 0, st, A, lw.ln1_w, lw.ln1_b, Cb, C, c.ln_eps);
-        VOX_TRY(conv_gemm(st, lw.qkv, Cb, nullptr, sl, n, L, 0, off0, Db, nullptr, nullptr, 0));             // Db [nL, 3*dim]
+        hipLaunchKernelGGL(k_layernorm_f32, dim3(n * L), dim3(256), 0, st, A, lw.ln1_w, lw.ln1_b, Cb, C, c.ln_eps, 3);
+        { ConvDmaArgs a = conv(lw.qkv, Cb, nullptr, 0, nullptr); a.out = Db; VOX_TRY(run(a)); }              // Db [nL, 3*dim]
         if (S) {
             const size_t ring = (size_t)m->max_slots * m->ring_cap * C;
             const size_t smem = ((size_t)L * D + (size_t)(c.context + L) * (D + 1) + 4 * (size_t)(c.context + L)) * 4;
@@ -2395,41 +2480,40 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
             hipLaunchKernelGGL(k_mimi_attn, dim3(H, n), dim3(256), (size_t)(L * D + 2 * L * (D + 1) + 4 * L) * 4, st, Db, Cb, L, H, D,
                                c.context, c.max_period);
         }
-        VOX_TRY(conv_gemm(st, lw.o, Cb, nullptr, sl, n, L, 0, off0, A, A, lw.scale1, 0));                    // h += s1 * o(attn)
-        hipLaunchKernelGGL(k_layernorm_f32, dim3(n * L), dim3(256), 0, st, A, lw.ln2_w, lw.ln2_b, Cb, C, c.ln_eps);
-        VOX_TRY(conv_gemm(st, lw.fc1, Cb, nullptr, sl, n, L, 0, off0, Db, nullptr, nullptr, 1));             // GELU
-        VOX_TRY(conv_gemm(st, lw.fc2, Db, nullptr, sl, n, L, 0, off0, A, A, lw.scale2, 0));                  // h += s2 * mlp
+        { ConvDmaArgs a = conv(lw.o, Cb, nullptr, 0, nullptr); a.res = a.out = A; a.scale = lw.scale1; VOX_TRY(run(a)); }   // h += s1 * o(attn)
+        hipLaunchKernelGGL(k_layernorm_f32, dim3(n * L), dim3(256), 0, st, A, lw.ln2_w, lw.ln2_b, Cb, C, c.ln_eps, 3);
+        { ConvDmaArgs a = conv(lw.fc1, Cb, nullptr, 0, nullptr); terms(a, Db); VOX_TRY(run(a, CONV_GELU)); }
+        { ConvDmaArgs a = conv(lw.fc2, Db, nullptr, 0, nullptr); a.res = a.out = A; a.scale = lw.scale2;                    // h += s2 * mlp
+          if (l == c.num_layers - 1) terms(a, Cb);
+          VOX_TRY(run(a)); }
     }
     if (S) hipLaunchKernelGGL(k_pos_advance, dim3((n + 255) / 256), dim3(256), 0, st, m->pos, sl, n, L);
-    // ---- SEANet decoder ----
+    if (!c.num_layers) hipLaunchKernelGGL(k_terms3, dim3(n * L), dim3(256), 0, st, A, Cb, C);
+    // ---- SEANet decoder: x = the activated rows of the next conv; h only where a residual reads it ----
     int offk[CG_MAXTAPS];
-    for (int k = 0; k < c.kernel_size; ++k) offk[k] = c.kernel_size - 1 - k;
+    for (int k = 0; k < c.kernel_size && k < CG_MAXTAPS; ++k) offk[k] = c.kernel_size - 1 - k;
     const int Pk = c.kernel_size - 1;
-    VOX_TRY(conv_gemm(st, w.dec0, A, S ? m->st_dec0 : nullptr, sl, n, L, S ? Pk : 0, offk, B, nullptr, nullptr, 0));   // B [nL, 16 nf]
-    if (S) state_update(st, m->st_dec0, sl, A, n, L, Pk, C);
-    float *h = B, *t1 = A, *t2 = Cb, *t3 = Db;
     int ch = 16 * c.n_filters;
+    { ConvDmaArgs a = conv(w.dec0, Cb, m->st_dec0, Pk, offk); elu_out(a, B, ch); VOX_TRY(run(a)); }           // B [nL, 16 nf]
+    later(m->st_dec0, Cb, Pk, C);
+    float *x = B, *h = A, *f0 = Db, *f1 = Cb;      // (f1 may be the pending history's source: the next launch must not write it)
     for (int b = 0; b < 4; ++b) {
         const vox_mimi_block_w& bw = w.blocks[b];
-        const int r = c.ratios[b];
-        elu(st, h, t1, (size_t)n * L * ch);
-        const int offt[2] = {0, 1};
-        VOX_TRY(conv_gemm(st, bw.tconv, t1, S ? m->st_tc[b] : nullptr, sl, n, L, S ? 1 : 0, offt, t2, nullptr, nullptr, 0));   // t2 [n*L*r, ch/2]
-        if (S) state_update(st, m->st_tc[b], sl, t1, n, L, 1, ch);
-        L *= r;
+        const int offt[2] = {0, 1}, off3[3] = {2, 1, 0};
+        { ConvDmaArgs a = conv(bw.tconv, x, m->st_tc[b], 1, offt); a.out = h; elu_out(a, f0, ch / 2); VOX_TRY(run(a)); }     // h [n*L*r, ch/2]
+        later(m->st_tc[b], x, 1, ch);
+        { float* o = x; x = f0; f0 = f1; f1 = o; }
+        L *= c.ratios[b];
         ch /= 2;
-        { float* x = h; h = t2; t2 = x; }
-        elu(st, h, t1, (size_t)n * L * ch);
-        const int off3[3] = {2, 1, 0};
-        VOX_TRY(conv_gemm(st, bw.conv1, t1, S ? m->st_c1[b] : nullptr, sl, n, L, S ? 2 : 0, off3, t3, nullptr, nullptr, 0));   // t3 [nL, ch/2]
-        if (S) state_update(st, m->st_c1[b], sl, t1, n, L, 2, ch);
-        elu(st, t3, t1, (size_t)n * L * (ch / 2));
-        VOX_TRY(conv_gemm(st, bw.conv2, t1, nullptr, sl, n, L, 0, off0, h, h, nullptr, 0));                  // h += conv2(...)
+        { ConvDmaArgs a = conv(bw.conv1, x, m->st_c1[b], 2, off3); elu_out(a, f0, ch / 2); VOX_TRY(run(a)); }                // f0 [nL, ch/2]
+        later(m->st_c1[b], x, 2, ch);
+        { ConvDmaArgs a = conv(bw.conv2, f0, nullptr, 0, nullptr); a.res = h; elu_out(a, f1, ch, b < 3); VOX_TRY(run(a)); }   // (the final conv reads fp32 rows)
+        { float* o = x; x = f1; f1 = o; }                                                                                     // h += conv2(...), activated
     }
-    elu(st, h, t1, (size_t)n * L * ch);
-    hipLaunchKernelGGL(k_mimi_final, dim3((L + 3) / 4, n), dim3(256), 0, st, t1, w.final_w, w.final_b, out, L, ch, c.last_kernel_size,
-                       S ? m->st_final : nullptr, sl);
-    if (S) state_update(st, m->st_final, sl, t1, n, L, c.last_kernel_size - 1, ch);
+    if (c.last_kernel_size != 3 || !final_taps<3, false>(st, x, S ? m->st_final : nullptr, sl, w.final_w, w.final_b, out, n, L, ch))
+        hipLaunchKernelGGL(k_mimi_final, dim3((L + 3) / 4, n), dim3(256), 0, st, x, w.final_w, w.final_b, out, L, ch, c.last_kernel_size,
+                           S ? m->st_final : nullptr, sl);
+    if (S) state_update(st, m->st_final, sl, x, n, L, c.last_kernel_size - 1, ch);
     return VOX_OK;
 }
 
@@ -2447,13 +2531,13 @@ int vox_mimi_stream_enable(vox_mimi* m, int max_slots) {
     if (c.kernel_size - 1 > 8 || c.last_kernel_size < 2) return vox_fail(VOX_ERR_INVALID, "mimi_stream_enable: unsupported kernel sizes");
     const size_t S = max_slots, C = c.dim;
     m->ring_cap = c.context + 2 * m->max_frames;           // >= context + L - 1
-    bool ok = hipMalloc((void**)&m->st_up, S * C * 4) == hipSuccess && hipMalloc((void**)&m->st_dec0, S * (c.kernel_size - 1) * C * 4) == hipSuccess &&
+    bool ok = hipMalloc((void**)&m->st_up, S * C * 4) == hipSuccess && hipMalloc((void**)&m->st_dec0, S * (c.kernel_size - 1) * C * 6) == hipSuccess &&
               hipMalloc((void**)&m->kring, (size_t)c.num_layers * S * m->ring_cap * C * 4) == hipSuccess &&
               hipMalloc((void**)&m->vring, (size_t)c.num_layers * S * m->ring_cap * C * 4) == hipSuccess &&
               hipMalloc((void**)&m->pos, S * sizeof(long)) == hipSuccess;
     size_t ch = (size_t)16 * c.n_filters;
     for (int b = 0; ok && b < 4; ++b) {
-        ok = hipMalloc((void**)&m->st_tc[b], S * ch * 4) == hipSuccess && hipMalloc((void**)&m->st_c1[b], S * 2 * (ch / 2) * 4) == hipSuccess;
+        ok = hipMalloc((void**)&m->st_tc[b], S * ch * 6) == hipSuccess && hipMalloc((void**)&m->st_c1[b], S * 2 * (ch / 2) * 6) == hipSuccess;
         ch /= 2;
     }
     ok = ok && hipMalloc((void**)&m->st_final, S * (c.last_kernel_size - 1) * ch * 4) == hipSuccess;
@@ -2470,11 +2554,12 @@ int vox_mimi_reset_slot(vox_mimi* m, void* stream, int slot) {
     const vox_mimi_config& c = m->cfg;
     const size_t C = c.dim;
     VOX_HIP(hipMemsetAsync(m->st_up + (size_t)slot * C, 0, C * 4, st));
-    VOX_HIP(hipMemsetAsync(m->st_dec0 + (size_t)slot * (c.kernel_size - 1) * C, 0, (c.kernel_size - 1) * C * 4, st));
+    const auto zero6 = [&](float* p, size_t elems) { return hipMemsetAsync(reinterpret_cast<char*>(p) + (size_t)slot * elems * 6, 0, elems * 6, st); };      // (S3 rows)
+    VOX_HIP(zero6(m->st_dec0, (c.kernel_size - 1) * C));
     size_t ch = (size_t)16 * c.n_filters;
     for (int b = 0; b < 4; ++b) {
-        VOX_HIP(hipMemsetAsync(m->st_tc[b] + (size_t)slot * ch, 0, ch * 4, st));
-        VOX_HIP(hipMemsetAsync(m->st_c1[b] + (size_t)slot * 2 * (ch / 2), 0, 2 * (ch / 2) * 4, st));
+        VOX_HIP(zero6(m->st_tc[b], ch));
+        VOX_HIP(zero6(m->st_c1[b], 2 * (ch / 2)));
         ch /= 2;
     }
     VOX_HIP(hipMemsetAsync(m->st_final + (size_t)slot * (c.last_kernel_size - 1) * ch, 0, (c.last_kernel_size - 1) * ch * 4, st));
