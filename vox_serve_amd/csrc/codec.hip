@@ -1284,7 +1284,7 @@ __global__ __launch_bounds__(256) void k_codec_attn(const float* qkv, const bf16
 // chain of the two kernels above: bit-identical (waveform digests equal).  Chunk of 1 / 8 / 32 requests: 1.95 -> 1.76, 3.53 -> 3.34, 7.70 -> 7.47 ms
 // (profiles/round4_codec_attn_ab.txt).
 template <int D>
-__global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* ring, const int* slots, const long* pos, float* out, int T,
+__global__ __launch_bounds__(1024) void k_codec_attn2(const float* qkv, bf16_t* ring, const int* slots, const long* pos, float* out, int T,
                                                      int H, int Wn, const float* inv_freq, int terms) {
     extern __shared__ float sm[];   // K [Wn][D+1], V [Wn][D+1], Q [T][D], P [T][Wn]
     constexpr int LD = D + 1, half = D / 2, CH = D / 8;
@@ -1292,14 +1292,14 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
     float* Vs = Ks + (size_t)Wn * LD;
     float* Qs = Vs + (size_t)Wn * LD;
     float* Ps = Qs + (size_t)T * D;
-    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = blockDim.x;
     const int HD = H * D;
     const int slot = slots[b];
     const long p0 = pos[slot];
     const long lo = p0 + T - Wn;   // absolute position of logical slot 0
     bf16_t* rbase = ring + (size_t)slot * Wn * 2 * HD + (size_t)h * D;
     // history rows: logical slots 0 .. Wn - T - 1 (absolute positions lo .. p0 - 1; negative = the never-written zero rows)
-    for (int c = tid; c < (Wn - T) * CH; c += 256) {
+    for (int c = tid; c < (Wn - T) * CH; c += nt) {
         const int j = c / CH, d0 = (c % CH) * 8;
         const long ap = lo + j;
         uint4 kq = make_uint4(0, 0, 0, 0), vq = kq;
@@ -1316,7 +1316,7 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
         vd[4] = bf2f((bf16_t)(vq.z & 0xffff)); vd[5] = bf2f((bf16_t)(vq.z >> 16)); vd[6] = bf2f((bf16_t)(vq.w & 0xffff)); vd[7] = bf2f((bf16_t)(vq.w >> 16));
     }
     // the chunk's T new rows: RoPE (NeoX halves) on q and k, k / v rounded to bf16 for the ring — and for this launch's own tile
-    for (int e = tid; e < T * half; e += 256) {
+    for (int e = tid; e < T * half; e += nt) {
         const int t = e / half, i = e % half, j = Wn - T + t;
         const long p = p0 + t;
         const float ang = (float)p * inv_freq[i];
@@ -1333,7 +1333,7 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
         Ks[j * LD + i] = bf2f(k0);
         Ks[j * LD + i + half] = bf2f(k1);
     }
-    for (int e = tid; e < T * D; e += 256) {
+    for (int e = tid; e < T * D; e += nt) {
         const int t = e / D, d = e % D, j = Wn - T + t;
         const long p = p0 + t;
         const bf16_t v16 = f2bf(qkv[((size_t)(b * T + t)) * 3 * HD + 2 * HD + (size_t)h * D + d]);
@@ -1342,7 +1342,7 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
     }
     __syncthreads();
     const float scale = rsqrtf((float)D);
-    for (int pr = tid; pr < T * Wn; pr += 256) {
+    for (int pr = tid; pr < T * Wn; pr += nt) {
         const int i = pr / Wn, j = pr % Wn;
         const int nvis = Wn - T + i + 1;
         float sc = -INFINITY;
@@ -1357,7 +1357,7 @@ __global__ __launch_bounds__(256) void k_codec_attn2(const float* qkv, bf16_t* r
         Ps[pr] = sc;
     }
     __syncthreads();
-    for (int i = wave; i < T; i += 4) {
+    for (int i = wave; i < T; i += nt >> 6) {
         float* P = Ps + (size_t)i * Wn;
         const int nvis = Wn - T + i + 1;
         float mx = -INFINITY;
@@ -1684,6 +1684,8 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
     return vox_fail(VOX_ERR_INVALID, "codec gemm: no tile variant");
 }
 
+// a wave per query of a (head, request): the rounds of a wave are a serial chain of a few thousand clocks each
+static int attn_threads(int L) { return 64 * (L < 4 ? 4 : L > 16 ? 16 : L); }
 static void state_update(hipStream_t st, float* state, const int* slots, const float* x, int n, int L, int P, int C) {
     hipLaunchKernelGGL(k_state_update, dim3((C + 255) / 256, n), dim3(256), 0, st, state, slots, x, L, P, C);
 }
@@ -1940,7 +1942,7 @@ static void codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* 
     static const bool attn2 = [] { const char* e = getenv("VOX_CODEC_ATTN2"); return !(e && e[0] == '0'); }();
     const size_t lds2 = (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + L * c.window) * 4;
     if (attn2 && c.head_dim == 64 && L <= c.window && lds2 <= 64 * 1024) {
-        hipLaunchKernelGGL(k_codec_attn2<64>, dim3(c.num_heads, n), dim3(256), lds2, st, qkv, ring, slots, m->pos, out, L, c.num_heads, c.window,
+        hipLaunchKernelGGL(k_codec_attn2<64>, dim3(c.num_heads, n), dim3(attn_threads(L)), lds2, st, qkv, ring, slots, m->pos, out, L, c.num_heads, c.window,
                            m->w.inv_freq, terms);
     } else {
         hipLaunchKernelGGL(k_codec_rope_kv, dim3(n * L), dim3(256), 0, st, qkv, ring, slots, m->pos, L, c.num_heads, c.head_dim, c.window,
@@ -2220,16 +2222,16 @@ __global__ __launch_bounds__(256) void k_elu(const float* x, float* y, size_t to
 }
 // causal attention inside one chunk of L <= 64 tokens with RoPE on interleaved pairs at positions 0..L-1
 // (apply_rope mimi.py:874-931; offset 0: stateless).  qkv rows [3][H][D]; one block per (head, request).
-__global__ __launch_bounds__(256) void k_mimi_attn(const float* qkv, float* out, int L, int H, int D, int context, float max_period) {
-    extern __shared__ float sm[];   // Q [L][D], K [L][D+1], V [L][D+1], P [4][L]
+__global__ __launch_bounds__(1024) void k_mimi_attn(const float* qkv, float* out, int L, int H, int D, int context, float max_period) {
+    extern __shared__ float sm[];   // Q [L][D], K [L][D+1], V [L][D+1], P [waves][L]
     const int LD = D + 1;
     float* Qs = sm;
     float* Ks = Qs + (size_t)L * D;
     float* Vs = Ks + (size_t)L * LD;
     float* Ps = Vs + (size_t)L * LD;
-    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int h = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nt = blockDim.x;
     const int HD = H * D;
-    for (int e = tid; e < L * (D / 2); e += 256) {
+    for (int e = tid; e < L * (D / 2); e += nt) {
         const int t = e / (D / 2), i = e % (D / 2);
         const float* r = qkv + ((size_t)(b * L + t)) * 3 * HD + (size_t)h * D + 2 * i;
         const float freq = expf((float)i * (-logf(max_period) * 2.0f / (float)D));
@@ -2246,7 +2248,7 @@ __global__ __launch_bounds__(256) void k_mimi_attn(const float* qkv, float* out,
     __syncthreads();
     const float scale = rsqrtf((float)D);
     float* P = Ps + (size_t)wave * L;
-    for (int i = wave; i < L; i += 4) {
+    for (int i = wave; i < L; i += nt >> 6) {
         const float* q = Qs + (size_t)i * D;
         const int j = lane;
         const bool vis = j < L && j <= i && (i - j) < context;
@@ -2477,7 +2479,7 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
             hipLaunchKernelGGL(k_mimi_attn_stream, dim3(H, n), dim3(256), smem, st, Db, Cb, m->kring + l * ring, m->vring + l * ring,
                                m->pos, sl, L, H, D, c.context, m->ring_cap, c.max_period);
         } else {
-            hipLaunchKernelGGL(k_mimi_attn, dim3(H, n), dim3(256), (size_t)(L * D + 2 * L * (D + 1) + 4 * L) * 4, st, Db, Cb, L, H, D,
+            hipLaunchKernelGGL(k_mimi_attn, dim3(H, n), dim3(attn_threads(L)), (size_t)(L * D + 2 * L * (D + 1) + attn_threads(L) / 64 * L) * 4, st, Db, Cb, L, H, D,
                                c.context, c.max_period);
         }
         { ConvDmaArgs a = conv(lw.o, Cb, nullptr, 0, nullptr); a.res = a.out = A; a.scale = lw.scale1; VOX_TRY(run(a)); }   // h += s1 * o(attn)
