@@ -299,6 +299,7 @@ __device__ __forceinline__ void ln_row_stats(const float* row, int C, int l16, f
 // pieces lie swizzled by row (in the address that each lane reads), so the fragment reads of 16 rows do not meet in a bank.
 // WK > 1: the waves share the 32-channel slices of a step and add their sums through LDS at the end — a call of a few rows then has
 // every wave of a CU at work on one small tile.
+// WP = 2: every tap has two weight planes (n_taps * N rows apart; fp32 weights as two terms) that share the tap's rows.
 // EPI: 0, CONV_GELU, or CONV_GLU: columns come in pairs (n, N + n) of w, out2 <- S2 of silu(v[n]) * v[N + n], N columns.
 // The weights are the MFMA's first operand, so a lane ends with 4 (8) neighbouring channels of one row: the residual, the constants and both
 // outputs move in 16-byte accesses without a lane exchange.  With a lane per column the same epilogue cost more than the products of the
@@ -432,10 +433,10 @@ __device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x
 }
 #define CONV_GELU 1
 #define CONV_GLU 2
-template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI>
+template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI, int WP = 1>
 __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8;
-    constexpr int SA = NP * BM * BK * 2, SB = BN * BK * 2, ST = SA + SB, CA = SA / 1024, CB = SB / 1024;
+    constexpr int SA = NP * BM * BK * 2, SB = WP * BN * BK * 2, ST = SA + SB, CA = SA / 1024, CB = SB / 1024;
     constexpr bool PAIR = EPI != CONV_GLU && NT % 2 == 0;
     constexpr int NA = (CA + NWV - 1) / NWV, NB = (CB + NWV - 1) / NWV;      // (where the waves do not divide them some chunks are asked for twice)
     static_assert(SA % 1024 == 0 && SB % 1024 == 0 && KS % WK == 0 && (BM * PPR) % 64 == 0, "whole wave instructions");
@@ -474,7 +475,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-        const int q = (i * NWV + wv) % CB * 64 + lane, r = q / PPR, pc = (q % PPR) ^ wswz(r);
+        const int q = (i * NWV + wv) % CB * 64 + lane, r = q / PPR % BN, pl = q / (BN * PPR), pc = (q % PPR) ^ wswz(r);
         int n = n0 + r;
         if (EPI == CONV_GLU) {
             n = (n0 >> 1) + (r >> 5) * 16 + (r & 15);
@@ -482,7 +483,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         } else {
             n = n < a.N ? n : a.N - 1;
         }
-        wp[i] = reinterpret_cast<const char*>(a.w) + ((size_t)n * a.Cin + pc * 8) * 2;
+        wp[i] = reinterpret_cast<const char*>(a.w) + (((size_t)pl * a.n_taps * a.N + n) * a.Cin + pc * 8) * 2;
     }
     const int nck = a.Cin / BK, nit = a.n_taps * nck;
     const size_t wtap = (size_t)(EPI == CONV_GLU ? 2 * a.N : a.N) * a.Cin * 2 - (size_t)a.Cin * 2;      // from the end of one tap's row to the next tap's
@@ -547,18 +548,23 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         for (int k = 0; k < KS / WK; ++k) {
             const int piece = (((wk * (KS / WK) + k) * 4 + fk) ^ (BK == 32 ? (fr >> 1) & 3 : fr & 7)) * 16;
             const int wpiece = (((wk * (KS / WK) + k) * 4 + fk) ^ wswz(wfr)) * 16;
-            cbf16x8 bf[NT];
+            cbf16x8 bf[WP][NT];
 #pragma unroll
-            for (int j = 0; j < NT; ++j) bf[j] = *reinterpret_cast<const cbf16x8*>(bs + (PAIR ? (j >> 1) * 32 + (j & 1) * 4 : j * 16) * BK * 2 + wpiece);
+            for (int w = 0; w < WP; ++w)
+#pragma unroll
+                for (int j = 0; j < NT; ++j)
+                    bf[w][j] = *reinterpret_cast<const cbf16x8*>(bs + (w * BN + (PAIR ? (j >> 1) * 32 + (j & 1) * 4 : j * 16)) * BK * 2 + wpiece);
 #pragma unroll
             for (int p = NP - 1; p >= 0; --p) {
                 cbf16x8 af[MT];
 #pragma unroll
                 for (int i = 0; i < MT; ++i) af[i] = *reinterpret_cast<const cbf16x8*>(as + (p * BM + i * 16) * BK * 2 + piece);
 #pragma unroll
-                for (int i = 0; i < MT; ++i)
+                for (int w = WP - 1; w >= 0; --w)
 #pragma unroll
-                    for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[j], af[i], acc[i][j], 0, 0, 0);
+                    for (int i = 0; i < MT; ++i)
+#pragma unroll
+                        for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[w][j], af[i], acc[i][j], 0, 0, 0);
             }
         }
         stage = stage == S - 1 ? 0 : stage + 1;
@@ -1153,12 +1159,12 @@ __global__ __launch_bounds__(256) void k_state_update(float* state, const int* s
 
 // SnakeBeta: y = x + inv_beta[c] * sin(x * alpha[c])^2          qwen3_codec.py:1004-1018 (alpha/beta pre-exponentiated)
 __global__ __launch_bounds__(256) void k_snake(const float* x, const float* alpha, const float* inv_beta, float* y,
-                                               size_t total, int C) {
+                                               size_t total, int C, int terms) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
         const int c = (int)(i % C);
         const float v = x[i];
         const float s = sinf(v * alpha[c]);
-        y[i] = v + inv_beta[c] * (s * s);
+        put_row(y, i / C, C, (int)(i % C), v + inv_beta[c] * (s * s), terms);
     }
 }
 
@@ -1691,11 +1697,11 @@ static void state_update(hipStream_t st, float* state, const int* slots, const f
 }
 
 // ---- convolutions over S2 rows (k_conv_dma) ----
-template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI>
+template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI, int WP = 1>
 static int conv_dma_launch(hipStream_t st, ConvDmaArgs& a) {
-    constexpr int lds = S * (NP * BM + BN) * BK * 2, threads = 64 * WM * WN * WK;
+    constexpr int lds = S * (NP * BM + WP * BN) * BK * 2, threads = 64 * WM * WN * WK;
     static_assert(lds + BM * 4 <= 160 * 1024, "LDS of a CU");
-    const auto kern = k_conv_dma<BM, BN, WM, WN, WK, BK, S, NP, EPI>;
+    const auto kern = k_conv_dma<BM, BN, WM, WN, WK, BK, S, NP, EPI, WP>;
     if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     a.tm = (a.M + BM - 1) / BM;
     a.tn = ((EPI == CONV_GLU ? 2 * a.N : a.N) + BN - 1) / BN;
@@ -1830,11 +1836,11 @@ static int conv_unit(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int* fuse
     return conv_unit_launch<96, 4, 1, 3>(st, a1, a2, H);
 }
 
-static void snake(hipStream_t st, const float* x, const vox_snake_w& s, float* y, size_t rows, int C) {
+static void snake(hipStream_t st, const float* x, const vox_snake_w& s, float* y, size_t rows, int C, int terms = 0) {
     const size_t total = rows * C;
     int grid = (int)((total + 255) / 256);
     if (grid > 4096) grid = 4096;
-    hipLaunchKernelGGL(k_snake, dim3(grid), dim3(256), 0, st, x, s.alpha, s.inv_beta, y, total, C);
+    hipLaunchKernelGGL(k_snake, dim3(grid), dim3(256), 0, st, x, s.alpha, s.inv_beta, y, total, C, terms);
 }
 
 extern "C" {
@@ -3089,20 +3095,20 @@ __global__ __launch_bounds__(256) void k_hift_add_snake3(const float* y, const f
         const float v = y[((size_t)b * Ly + ty) * C + c] + si[i];
         x[i] = v;
         float s_;
-        s_ = sinf(v * al0[c]); a0[i] = v + ib0[c] * (s_ * s_);
-        if (a1) { s_ = sinf(v * al1[c]); a1[i] = v + ib1[c] * (s_ * s_); }
-        if (a2) { s_ = sinf(v * al2[c]); a2[i] = v + ib2[c] * (s_ * s_); }
+        s_ = sinf(v * al0[c]); put_row(a0, row, C, c, v + ib0[c] * (s_ * s_), 3);
+        if (a1) { s_ = sinf(v * al1[c]); put_row(a1, row, C, c, v + ib1[c] * (s_ * s_), 3); }
+        if (a2) { s_ = sinf(v * al2[c]); put_row(a2, row, C, c, v + ib2[c] * (s_ * s_), 3); }
     }
 }
 // x = leaky_relu(((r0 + r1) + r2) / nk, slope)   (hifigan.py:613-621; r1 / r2 NULL when fewer kernels)
 __global__ __launch_bounds__(256) void k_hift_avg_lrelu(const float* r0, const float* r1, const float* r2, float* x, size_t total, float nk,
-                                                         float slope) {
+                                                         float slope, int C, int terms) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (size_t)gridDim.x * 256) {
         float v = r0[i];
         if (r1) v = v + r1[i];
         if (r2) v = v + r2[i];
         if (nk != 1.0f) v = v / nk;
-        x[i] = v > 0.0f ? v : v * slope;
+        put_row(x, i / C, C, (int)(i % C), v > 0.0f ? v : v * slope, terms);
     }
 }
 // magnitude / phase heads -> irfft per frame -> window -> overlap-add / window^2 -> trim n_fft/2 -> clamp  (hifigan.py:554-594, 623-628)
@@ -3203,7 +3209,7 @@ int vox_hift_create(vox_ctx* ctx, const vox_hift_config* cfg, const vox_hift_wei
     m->buf_floats = worst * max_batch;
     const size_t L = (size_t)max_T * m->scale, F = rows + 1;
     bool ok = true;
-    for (int i = 0; i < 9; ++i) ok = ok && hipMalloc((void**)&m->buf[i], m->buf_floats * 4) == hipSuccess;
+    for (int i = 0; i < 9; ++i) ok = ok && hipMalloc((void**)&m->buf[i], m->buf_floats * 6) == hipSuccess;      // (fp32 or S3 rows)
     ok = ok && hipMalloc((void**)&m->f0, (size_t)max_batch * max_T * 4) == hipSuccess &&
          hipMalloc((void**)&m->ph, (size_t)max_batch * max_T * (cfg->nb_harmonics + 1) * 4) == hipSuccess &&
          hipMalloc((void**)&m->src, (size_t)max_batch * L * 4) == hipSuccess &&
@@ -3227,6 +3233,24 @@ int vox_hift_create(vox_ctx* ctx, const vox_hift_config* cfg, const vox_hift_wei
     return VOX_OK;
 }
 
+// A conv with two weight planes over S3 rows.  A request's samples must not depend on how many others are decoded with it, so all tiles add
+// in one order (64 channels at a time, two waves a half each): rows decide only which of them it is.  us, staged kernels before:
+// 3584 rows x 256 channels, 7 taps 77 -> 22.5; 17 920 x 128 56 -> 36; 53 768 x 64 37 -> 27; one request: 448 x 256 36 -> 12, 6721 x 64 15 -> 9
+static int hift_conv(hipStream_t st, ConvDmaArgs& a) {
+    if (a.Cin % CG_BK || a.N % 16 || a.n_taps % 2 || a.n_taps > CG_MAXTAPS || a.bias_mod % 8)
+        return vox_fail(VOX_ERR_INVALID, "hift conv: %d -> %d channels, %d taps", a.Cin, a.N, a.n_taps);
+    a.n_taps /= 2;
+    a.planes = 3;
+    const auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+    if (a.Cin % 64) return conv_dma_launch<64, 64, 2, 2, 1, 32, 3, 3, 0, 2>(st, a);
+    if (tiles(16, 32) <= 256) return conv_dma_launch<16, 32, 1, 1, 2, 64, 5, 3, 0, 2>(st, a);
+    if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 2, 64, 4, 3, 0, 2>(st, a);
+    if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 4, 2, 2, 64, 2, 3, 0, 2>(st, a);
+    // many rows: rounds of a CU's tiles (17 920 x 128: 1120 of 32 x 64 in five small rounds; 53 768 x 64: 421 of 128 x 64 in two)
+    if ((tiles(128, 64) + 255) / 256 * 4 <= (tiles(32, 64) + 255) / 256 * 1.3) return conv_dma_launch<128, 64, 4, 2, 2, 64, 2, 3, 0, 2>(st, a);
+    return conv_dma_launch<32, 64, 1, 2, 2, 64, 2, 3, 0, 2>(st, a);
+}
+
 // one ResBlock (hifigan.py:134-141) on rows L per request: a = snake1_0(x) is given; result in `r` (x itself is left untouched);
 // t1 scratch.  The next iteration's first Snake and this iteration's second Snake are fused into the producing conv's epilogue.
 static int hift_resblock(hipStream_t st, const vox_hift_resblock_w& rb, const vox_hift_config& c, int k, const float* x, float* a, float* t1,
@@ -3235,9 +3259,13 @@ static int hift_resblock(hipStream_t st, const vox_hift_resblock_w& rb, const vo
     hift_conv_offsets(k, 1, off2);
     for (int j = 0; j < 3; ++j) {
         hift_conv_offsets(k, c.dilations[j], off1);
-        VOX_TRY(conv_gemm(st, rb.c1[j], a, nullptr, nullptr, n, L, 0, off1, nullptr, nullptr, nullptr, 0, t1, &rb.a2[j]));
-        VOX_TRY(conv_gemm(st, rb.c2[j], t1, nullptr, nullptr, n, L, 0, off2, r, j == 0 ? x : r, nullptr, 0, j < 2 ? a : nullptr,
-                          j < 2 ? &rb.a1[j + 1] : nullptr));
+        ConvDmaArgs a1 = conv_s2_args(rb.c1[j], a, nullptr, nullptr, n, L, 0, off1), a2 = conv_s2_args(rb.c2[j], t1, nullptr, nullptr, n, L, 0, off2);
+        a1.out2 = t1; a1.out2_s2 = 1; a1.sn_alpha = rb.a2[j].alpha; a1.sn_invb = rb.a2[j].inv_beta;
+        a2.res = j == 0 ? x : r;
+        a2.out = r;
+        if (j < 2) { a2.out2 = a; a2.out2_s2 = 1; a2.sn_alpha = rb.a1[j + 1].alpha; a2.sn_invb = rb.a1[j + 1].inv_beta; }
+        VOX_TRY(hift_conv(st, a1));
+        VOX_TRY(hift_conv(st, a2));
     }
     return VOX_OK;
 }
@@ -3286,9 +3314,9 @@ int vox_hift_decode(vox_hift* m, void* stream, const float* mel, int n, int T, c
     // ---- conv_pre ----
     hift_conv_offsets(7, 1, off);
     VOX_TRY(conv_gemm(st, w.conv_pre, B[0], nullptr, nullptr, n, T, 0, off, B[1], nullptr, nullptr, 0));
-    hipLaunchKernelGGL(k_hift_avg_lrelu, dim3(ew_grid((size_t)n * T * c.base_channels)), dim3(256), 0, st, B[1], nullptr, nullptr, B[1],
-                       (size_t)n * T * c.base_channels, 1.0f, c.lrelu_slope);
-    float* cur = B[1];                     // leaky_relu'ed stage input
+    hipLaunchKernelGGL(k_hift_avg_lrelu, dim3(ew_grid((size_t)n * T * c.base_channels)), dim3(256), 0, st, B[1], nullptr, nullptr, B[2],
+                       (size_t)n * T * c.base_channels, 1.0f, c.lrelu_slope, c.base_channels, 3);
+    float* cur = B[2];                     // leaky_relu'ed stage input (S3 rows; fp32 behind the last stage)
     int Lc = T, ch = c.base_channels;
     // strides of source_downs: cumulative products of the LATER stages' rates (hifigan.py:497-500)
     for (int i = 0; i < c.n_stages; ++i) {
@@ -3301,7 +3329,7 @@ int vox_hift_decode(vox_hift* m, void* stream, const float* mel, int n, int T, c
         for (int q = 0; q < 9; ++q) if (B[q] != cur) pool[np++] = B[q];
         float *Y = pool[0], *S = pool[1], *A = pool[2], *T1 = pool[3], *X = pool[4], *A1 = pool[5], *A2 = pool[6], *R2 = pool[7];
         hift_tconv_offsets(k, u, off);
-        VOX_TRY(conv_gemm(st, w.ups[i], cur, nullptr, nullptr, n, Lc, 0, off, Y, nullptr, nullptr, 0));
+        { ConvDmaArgs a = conv_s2_args(w.ups[i], cur, nullptr, nullptr, n, Lc, 0, off); a.out = Y; VOX_TRY(hift_conv(st, a)); }
         int sstride = 1;
         for (int q = i + 1; q < c.n_stages; ++q) sstride *= c.upsample_rates[q];
         const int sk = sstride == 1 ? 1 : 2 * sstride, spad = sstride == 1 ? 0 : sstride / 2;
@@ -3309,7 +3337,7 @@ int vox_hift_decode(vox_hift* m, void* stream, const float* mel, int n, int T, c
         hipLaunchKernelGGL(k_hift_sd, dim3(ew_grid((size_t)n * Lx * cout)), dim3(256), 0, st, m->stft, m->sd_wt[i], w.sd_b[i], S, n, F, nb2, Lx, cout,
                            sk, sstride, spad);
         // source resblock: S <- resblock(S)
-        snake(st, S, w.src_rb[i].a1[0], A, (size_t)n * Lx, cout);
+        snake(st, S, w.src_rb[i].a1[0], A, (size_t)n * Lx, cout, 3);
         VOX_TRY(hift_resblock(st, w.src_rb[i], c, c.source_resblock_kernels[i], S, A, T1, X, n, Lx));       // result in X (scratch here)
         // x = pad(Y) + si, first Snakes of the stage's resblocks
         const vox_hift_resblock_w* rb = &w.rb[i * c.n_kernels];
@@ -3324,7 +3352,7 @@ int vox_hift_decode(vox_hift* m, void* stream, const float* mel, int n, int T, c
         for (int r = 0; r < c.n_kernels; ++r) VOX_TRY(hift_resblock(st, rb[r], c, c.resblock_kernels[r], Xs, As[r], T1, Rs[r], n, Lx));
         // average + the next stage's leaky_relu (slope 0.01 before conv_post: F.leaky_relu's default)
         hipLaunchKernelGGL(k_hift_avg_lrelu, dim3(ew_grid((size_t)n * Lx * cout)), dim3(256), 0, st, Rs[0], c.n_kernels > 1 ? Rs[1] : nullptr,
-                           c.n_kernels > 2 ? Rs[2] : nullptr, Xs, (size_t)n * Lx * cout, (float)c.n_kernels, last ? 0.01f : c.lrelu_slope);
+                           c.n_kernels > 2 ? Rs[2] : nullptr, Xs, (size_t)n * Lx * cout, (float)c.n_kernels, last ? 0.01f : c.lrelu_slope, cout, last ? 0 : 3);
         cur = Xs; Lc = Lx; ch = cout;
     }
     if (Lc != F) return vox_fail(VOX_ERR_INVALID, "hift_decode: frame count mismatch");
