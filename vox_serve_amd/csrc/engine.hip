@@ -371,7 +371,7 @@ int vox_stack_create(vox_ctx* ctx, const vox_stack_config* cfg, const vox_layer_
     }
     if (hipMalloc(&s->qkv, R * (nq + 2 * nkv) * 2) != hipSuccess || hipMalloc(&s->q, R * nq * 2) != hipSuccess ||
         hipMalloc(&s->h, R * cfg->ffn * 2) != hipSuccess || hipMalloc(&s->attn_out, R * nq * 2) != hipSuccess ||
-        hipMalloc(&s->xn, R * cfg->hidden * 2) != hipSuccess || hipMalloc(&s->skws, s->skws_bytes) != hipSuccess ||
+        hipMalloc(&s->xn, (R + 15) / 16 * 16 * cfg->hidden * 2) != hipSuccess || hipMalloc(&s->skws, s->skws_bytes) != hipSuccess ||
         hipMalloc((void**)&s->attn_ws, s->attn_ws_floats * 4) != hipSuccess) {
         delete s;
         return vox_fail(VOX_ERR_NOMEM, "stack_create: hipMalloc failed");

@@ -1513,6 +1513,172 @@ __global__ __launch_bounds__(512) void k_gemm_fullk(LinArgs a) {
     VOX_TR_END(1, (MT << 24) | (KSTEPS << 16) | (PRO << 12) | (EPI << 8) | (ROWSPLIT ? 16 : 0) | CT)
 }
 
+// ================================================================================================
+// linear for 33..128 rows with K >= 2048 (prefills): the arithmetic of k_gemm_fullk (eight contiguous K ranges, a wave each, MFMA k-steps
+// ascending, partial sums added in wave order: the same bits), the operands through LDS.  k_gemm_fullk runs its 32-row form once per row
+// tile: every block waits out the latency of its weights, and the row tiles of a column fetch them again.  Here a block has NT column
+// tiles (gate and up beside each other) and up to 80 rows; a wave's k-step (weights and rows, 1 KB per 16 x 32 tile) comes by
+// global_load_lds into its own S-stage ring.  Nothing is shared before the final sum, so there is no barrier in the loop: a wave waits for
+// its own requests, takes the step into registers, asks for the step S further on and multiplies.  Rows come normalised (k_norm_rows).
+// Bound by the L2 -> LDS path: a block moves its rows once more per NT column tiles.  75 rows, us, k_gemm_fullk before: gate / up
+// 6144 x 2048 42 -> 18, down 2048 x 6144 18.5 -> 14, q | k | v 4096 x 2048 20.6 -> 11, o 2048 x 2048 8.4 -> 6.2 (beside the first and the
+// third a norm launch of 4.5).  More than two stages give nothing (14.0 / 14.5 / 14.8 with 2 / 3 / 5); fragment-major rows are worth a
+// sixth (1 KB requests: gate / up 20.7 -> 17.7), which is why the norm writes them so.
+// ================================================================================================
+// (m0 holds the LDS address of the instruction; nothing else in this kernel uses it)
+__device__ __forceinline__ void rows_dma16(const char* p, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
+}
+template <int MT, int NT, int EPI, int S>
+__global__ __launch_bounds__(512) void k_gemm_rows(LinArgs a) {
+    constexpr bool SM = (EPI == EPI_SILU_MUL);
+    constexpr int NB = SM ? 2 : 1, NW = NB * NT, STAGE = (NW + MT) * 1024;
+    extern __shared__ __attribute__((aligned(1024))) char rows_lds[];
+    static_assert(NB * MT * 8 * 1024 <= 8 * S * STAGE, "partial sums of one column tile");
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15;
+    const int ctile = (blockIdx.x / (8 * a.row_tiles)) * 8 + (blockIdx.x & 7), r0 = ((blockIdx.x >> 3) % a.row_tiles) * a.rt_rows;
+    const int bt = a.B - r0 < a.rt_rows ? a.B - r0 : a.rt_rows;
+    const int ks_n = a.K >> 8, k0 = wave * ks_n;        // this wave's k-steps: k0 .. k0 + ks_n - 1 of 32
+    // row-major operands: four lanes take the 64 bytes of a row, the piece swizzled by the row; fragment-major ones: a tile is 1 KB as it stands
+    const int lr = lane >> 2, pc = (lane & 3) ^ ((lr >> 1) & 3);
+    const bool wf = a.W_frag != nullptr, xf = a.x_frag != nullptr;
+    const char *wp[NW], *xp[MT];
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int nb = i / NT, t = ctile * NT + i % NT;
+        wp[i] = wf ? reinterpret_cast<const char*>(nb ? a.W2_frag : a.W_frag) + ((size_t)t * (a.K >> 5) + k0) * 1024 + lane * 16
+                   : reinterpret_cast<const char*>(nb ? a.W2 : a.W) + ((size_t)(t * 16 + lr) * a.K + k0 * 32) * 2 + pc * 16;
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        if (xf) {
+            const int t = (r0 >> 4) + m, last = (a.B - 1) >> 4;
+            xp[m] = reinterpret_cast<const char*>(a.x_frag) + ((size_t)(t < last ? t : last) * (a.K >> 5) + k0) * 1024 + lane * 16;
+        } else {
+            const int row = m * 16 + lr;
+            xp[m] = reinterpret_cast<const char*>(x_row_ptr(a, r0 + (row < bt ? row : bt - 1))) + k0 * 64 + pc * 16;
+        }
+    }
+    const int wstep = wf ? 1024 : 64, xstep = xf ? 1024 : 64;
+    const unsigned sbase = __builtin_amdgcn_readfirstlane((unsigned)(size_t)(__attribute__((address_space(3))) char*)rows_lds + wave * (S * STAGE));
+    int rq = 0;
+    auto request = [&](int stage) {
+        const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * STAGE);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) rows_dma16(wp[i], ls + i * 1024);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) rows_dma16(xp[m], ls + (NW + m) * 1024);
+        if (++rq >= ks_n) return;      // (past the last step the same one is asked for again: the count in flight stays the same)
+#pragma unroll
+        for (int i = 0; i < NW; ++i) wp[i] += wstep;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) xp[m] += xstep;
+    };
+    u32 res_raw[NT][4], bias_raw[NT];
+    if (!SM && wave < MT) {       // (the residual of the outputs this thread will finish: asked for first)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) {
+            const int n = (ctile * NT + j) * 16 + fr;
+            if (a.residual)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int b = wave * 16 + (lane >> 4) * 4 + r;
+                    res_raw[j][r] = a.residual[(size_t)(r0 + (b < bt ? b : bt - 1)) * a.N + n];
+                }
+            if (a.bias) bias_raw[j] = a.bias[n];
+        }
+    }
+#pragma unroll
+    for (int s = 0; s < S; ++s) request(s);
+    f32x4_t acc[NW][MT];
+#pragma unroll
+    for (int i = 0; i < NW; ++i)
+#pragma unroll
+        for (int m = 0; m < MT; ++m) acc[i][m] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    const int off_rm = fr * 64 + ((lane >> 4) ^ ((fr >> 1) & 3)) * 16, woff = wf ? lane * 16 : off_rm, xoff = xf ? lane * 16 : off_rm;
+    const char* mine = rows_lds + wave * (S * STAGE);
+    int stage = 0;
+    for (int k = 0; k < ks_n; ++k) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 1) * (NW + MT)) : "memory");
+        uint4 wv[NW], xv[MT];
+#pragma unroll
+        for (int i = 0; i < NW; ++i) wv[i] = *reinterpret_cast<const uint4*>(mine + stage * STAGE + i * 1024 + woff);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) xv[m] = *reinterpret_cast<const uint4*>(mine + stage * STAGE + (NW + m) * 1024 + xoff);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (the step is in registers: its stage may be written again)
+        request(stage);
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+#pragma unroll
+            for (int i = 0; i < NW; ++i) acc[i][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(xv[m]), as_bf8(wv[i]), acc[i][m], 0, 0, 0);
+        stage = stage == S - 1 ? 0 : stage + 1;
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");            // (the repeated last steps: nothing may land any more)
+    f32x4_t* red = reinterpret_cast<f32x4_t*>(rows_lds);        // [wave][nb][m][lane]
+#pragma unroll
+    for (int j = 0; j < NT; ++j) {
+        __syncthreads();
+#pragma unroll
+        for (int nb = 0; nb < NB; ++nb)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) red[((wave * NB + nb) * MT + m) * 64 + lane] = acc[nb * NT + j][m];
+        __syncthreads();
+        if (wave >= MT) continue;
+        const int m = wave;               // thread (m, lane) finishes D fragment m: its column, rows m * 16 + (lane >> 4) * 4 + r
+        f32x4_t v = red[m * 64 + lane], u = SM ? red[((NB - 1) * MT + m) * 64 + lane] : v;
+#pragma unroll
+        for (int w = 1; w < 8; ++w) {
+            v += red[(w * NB * MT + m) * 64 + lane];
+            if (SM) u += red[((w * NB + NB - 1) * MT + m) * 64 + lane];
+        }
+        const int n = (ctile * NT + j) * 16 + fr;
+        const float bv = !SM && a.bias ? bf2f((bf16_t)bias_raw[j]) : 0.0f;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const int b = m * 16 + (lane >> 4) * 4 + r;
+            if (b >= bt) continue;
+            const size_t oi = (size_t)(r0 + b) * a.N + n;
+            bf16_t o;
+            if (SM) {
+                o = f2bf(bfround(silu_c(bfround(v[r]))) * bfround(u[r]));
+            } else {
+                float f = v[r];
+                if (a.bias) f = f + bv;
+                o = f2bf(f);
+                if (a.residual) o = f2bf(bf2f((bf16_t)res_raw[j][r]) + bf2f(o));
+            }
+            if (a.y_rowmajor) a.y[oi] = o;
+            if (a.y_frag) a.y_frag[frag_off(r0 + b, n, a.N)] = o;
+        }
+    }
+}
+// RMSNorm of rows with k_gemm_fullk's sums: a row's eight K ranges, four interleaved 16-byte sequences each.  32 lanes per row, one per
+// (range, sequence), which keep their KS chunks for the product.  y: fragment-major (rows rounded up to 16).
+template <int KS>
+__global__ __launch_bounds__(256) void k_norm_rows(LinArgs a, bf16_t* y) {
+    const int lane = threadIdx.x & 31, row = blockIdx.x * 8 + (threadIdx.x >> 5);
+    const int r = row < a.B ? row : a.B - 1;
+    const uint4 *x = x_row_ptr(a, r) + (lane >> 2) * (KS * 4) + (lane & 3), *w = reinterpret_cast<const uint4*>(a.nw) + (lane >> 2) * (KS * 4) + (lane & 3);
+    uint4 xv[KS], gv[KS];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) xv[s] = x[s * 4];
+#pragma unroll
+    for (int s = 0; s < KS; ++s) gv[s] = w[s * 4];
+    float ss = 0.0f;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) ss = sq8(xv[s], ss);
+    ss += __shfl_xor(ss, 1);
+    ss += __shfl_xor(ss, 2);
+    float t = 0.0f;
+#pragma unroll
+    for (int g = 0; g < 8; ++g) t += __shfl(ss, (threadIdx.x & 32) + g * 4);
+    const float rinv = 1.0f / sqrtf(t / (float)a.K + a.eps);
+    if (row >= a.B) return;
+    uint4* o = reinterpret_cast<uint4*>(y) + ((size_t)(row >> 4) * (KS * 8) + (lane >> 2) * KS) * 64 + (row & 15) + 16 * (lane & 3);      // (frag_off)
+#pragma unroll
+    for (int s = 0; s < KS; ++s) o[s * 64] = norm_chunk(xv[s], gv[s], rinv);
+}
+
 // row-major [rows][K] -> fragment-major (one thread per 16-byte chunk)
 __global__ __launch_bounds__(256) void k_swizzle_frag(const uint4* src, uint4* dst, int rows, int K) {
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;       // destination chunk index
@@ -1610,6 +1776,51 @@ static int launch_gemm_fullk_t(hipStream_t st, const LinArgs& a0) {
     hipLaunchKernelGGL((k_gemm_fullk<MT, KSTEPS, PRO, EPI, false>), dim3((a.N + 15) / 16), dim3(512), 0, st, a);
     return VOX_OK;
 }
+template <int MT, int NT, int EPI, int S>
+static int launch_gemm_rows_t(hipStream_t st, const LinArgs& a) {
+    constexpr int lds = 8 * S * ((EPI == EPI_SILU_MUL ? 2 : 1) * NT + MT) * 1024;
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    const auto kern = k_gemm_rows<MT, NT, EPI, S>;
+    if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL(kern, dim3(a.N / (16 * NT) * a.row_tiles), dim3(512), lds, st, a);
+    return VOX_OK;
+}
+// Rows of a block: all of them (up to 80) where the columns alone give a block per CU, halves of them for the narrow outputs.
+template <int EPI>
+static int launch_gemm_rows(hipStream_t st, const LinArgs& a0) {
+    LinArgs a = a0;
+    const int t16 = (a.B + 15) / 16;
+    a.row_tiles = EPI != EPI_SILU_MUL && a.N / 16 < 256 ? 2 : t16 > 5 ? 2 : 1;
+    const int mt = (t16 + a.row_tiles - 1) / a.row_tiles;
+    a.rt_rows = 16 * mt;
+    if constexpr (EPI == EPI_SILU_MUL) {
+        if (a.N % 256 == 0) {
+            switch (mt) {
+                case 3: return launch_gemm_rows_t<3, 2, EPI, 2>(st, a);
+                case 4: return launch_gemm_rows_t<4, 2, EPI, 2>(st, a);
+                default: return launch_gemm_rows_t<5, 2, EPI, 2>(st, a);
+            }
+        }
+        switch (mt) {
+            case 3: return launch_gemm_rows_t<3, 1, EPI, 2>(st, a);
+            case 4: return launch_gemm_rows_t<4, 1, EPI, 2>(st, a);
+            default: return launch_gemm_rows_t<5, 1, EPI, 2>(st, a);
+        }
+    } else {
+        switch (mt) {
+            case 2: return launch_gemm_rows_t<2, 1, EPI, 2>(st, a);
+            case 3: return launch_gemm_rows_t<3, 1, EPI, 2>(st, a);
+            case 4: return launch_gemm_rows_t<4, 1, EPI, 2>(st, a);
+            default: return launch_gemm_rows_t<5, 1, EPI, 2>(st, a);
+        }
+    }
+}
+// 33..128 rows (N % 128 by fullk_shape_ok).  K = 1024 (depth blocks) stays with k_gemm_fullk: a norm launch costs what the tiles save there.
+// Operands that do not lie on 16 bytes stay there too.
+static bool gemm_rows_ok(const LinearCall& c) {
+    const size_t at = (size_t)c.W | (size_t)c.W2 | (size_t)c.x | (size_t)(c.x_stride * 2);
+    return c.B > 32 && c.K >= 2048 && (at & 15) == 0 && (c.pro == PRO_COPY || (c.norm_scratch && (c.K == 2048 || c.K == 4096)));      // (4096: normalised by k_rmsnorm before)
+}
 template <int PRO, int EPI>
 static int launch_gemm_fullk(hipStream_t st, const LinArgs& a) {
     const int ks = a.K / 256;
@@ -1692,8 +1903,16 @@ int vox_launch_linear(vox_ctx* ctx, hipStream_t st, const LinearCall& call) {
 #endif
         hipLaunchKernelGGL(k_rmsnorm, dim3((c.B + 3) / 4), dim3(256), 0, st, a.x, a.nw, (bf16_t*)c.norm_scratch, c.B, c.K, c.eps);
         a.x = (const bf16_t*)c.norm_scratch; a.x_stride = c.K; a.x_frag = nullptr;
+        if (c.B > 32 && gemm_rows_ok(c)) return epi == EPI_SILU_MUL ? launch_gemm_rows<EPI_SILU_MUL>(st, a) : launch_gemm_rows<EPI_STORE>(st, a);
         if (epi == EPI_SILU_MUL) return launch_gemm_fullk<PRO_COPY, EPI_SILU_MUL>(st, a);
         return launch_gemm_fullk<PRO_COPY, EPI_STORE>(st, a);
+    }
+    if (linear_is_fullk(c) && gemm_rows_ok(c) && (epi == EPI_STORE || (epi == EPI_SILU_MUL && pro == PRO_RMSNORM))) {
+        if (pro == PRO_RMSNORM) {
+            hipLaunchKernelGGL(k_norm_rows<8>, dim3((c.B + 7) / 8), dim3(256), 0, st, a, (bf16_t*)c.norm_scratch);
+            a.x_frag = (const bf16_t*)c.norm_scratch;
+        }
+        return epi == EPI_STORE ? launch_gemm_rows<EPI_STORE>(st, a) : launch_gemm_rows<EPI_SILU_MUL>(st, a);
     }
     if (linear_is_fullk(c)) {
         if (pro == PRO_RMSNORM && epi == EPI_STORE) return launch_gemm_fullk<PRO_RMSNORM, EPI_STORE>(st, a);

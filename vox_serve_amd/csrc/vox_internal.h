@@ -56,7 +56,7 @@ struct LinearCall {
     const void* post_norm_w = nullptr;
     void* post_norm_out = nullptr;
     const void* x_prenormed = nullptr;
-    void* norm_scratch = nullptr;   // [B,K] bf16: lets > 32-row calls with a norm prologue normalise once up front
+    void* norm_scratch = nullptr;   // [B rounded up to 16, K] bf16: lets > 32-row calls with a norm prologue normalise once up front
     int keep_weights = 0;   // weights are re-read within the frame (depth loop): do not stream them past the caches
     // 9..32 rows path (full-K MFMA GEMM) only — "fragment-major" operands: tile (t, k-step ks) of a [rows or cols][K] matrix
     // is the 1 KiB block [64 lanes][8 bf16] an MFMA 16x16x32 operand register holds (lane = (row % 16) + 16 * ((k % 32) / 8)),
