@@ -313,19 +313,43 @@ struct ConvJob {           // history rows <- the last P rows of [history ++ x],
     const float* x;
     int L, P, C, n;
 };
-// new history = last P rows of [history ++ x]; one thread per (request, channel), rows ascending (in place)
+// new history = last P rows of [history ++ x].  A chunk of at least P rows replaces it: 16 bytes a thread and turn, four turns (the 54 rows
+// of a dilated conv, row by row in one thread, outlasted the launch they rode on: 15 us against 9).  A shorter one shifts it: one thread per
+// (request, channel), rows ascending (in place).
+__host__ __device__ __forceinline__ bool conv_job_whole(const ConvJob& j) { return j.L >= j.P && j.C % 4 == 0; }
+__host__ __device__ __forceinline__ int conv_job_per(const ConvJob& j, int threads) {      // blocks of a request
+    return conv_job_whole(j) ? (j.P * (j.C / 4) + 4 * threads - 1) / (4 * threads) : (j.C + threads - 1) / threads;
+}
 __device__ __forceinline__ void conv_job(const ConvJob& j, const int* slots, int block, int threads) {
-    const int per = (j.C + threads - 1) / threads, b = block / per, c = block % per * threads + (int)threadIdx.x;
+    const int per = conv_job_per(j, threads), b = block / per, e0 = block % per;
+    float* s = j.state + (size_t)slots[b] * j.P * j.C;
+    const float* x = j.x + (size_t)b * j.L * j.C;
+    if (conv_job_whole(j)) {
+        const float4* src = reinterpret_cast<const float4*>(x + (size_t)(j.L - j.P) * j.C);
+        const int n4 = j.P * (j.C / 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int e = (e0 * 4 + i) * threads + (int)threadIdx.x;
+            if (e < n4) reinterpret_cast<float4*>(s)[e] = src[e];
+        }
+        return;
+    }
+    const int c = e0 * threads + (int)threadIdx.x;
     if (c >= j.C) return;
-    float* s = j.state + (size_t)slots[b] * j.P * j.C + c;
-    const float* x = j.x + (size_t)b * j.L * j.C + c;
-#pragma unroll 6
     for (int i = 0; i < j.P; ++i) {
         const int e = j.L + i;
-        s[(size_t)i * j.C] = e < j.P ? s[(size_t)e * j.C] : x[(size_t)(e - j.P) * j.C];
+        s[(size_t)i * j.C + c] = e < j.P ? s[(size_t)e * j.C + c] : x[(size_t)(e - j.P) * j.C + c];
     }
 }
-static int conv_job_blocks(const ConvJob& j, int threads) { return j.state ? j.n * ((j.C + threads - 1) / threads) : 0; }
+static int conv_job_blocks(const ConvJob& j, int threads) { return j.state ? j.n * conv_job_per(j, threads) : 0; }
+// what is left at the end of a chunk: two histories (state NULL: none) and the slots' positions
+__global__ __launch_bounds__(256) void k_conv_jobs(ConvJob a, ConvJob b, int na, int nb, const int* slots, long* pos, int n, int T) {
+    const int i = (int)blockIdx.x;
+    if (i < na) conv_job(a, slots, i, 256);
+    else if (i < na + nb) conv_job(b, slots, i - na, 256);
+    else
+        for (int k = threadIdx.x; k < n; k += 256) pos[slots[k]] += T;
+}
 struct ConvDmaArgs : ConvGemmArgs {
     int tm, tn, tiles8, mfast;      // tiles along M and N; their number rounded up to 8; 1: the blocks of an XCD walk the rows first
     const float* rms_x;    // fp32 rows [M, Cin] whose 1 / rms scales the sums of row m (the rows' RMSNorm, its weight already in x), or NULL
@@ -1762,8 +1786,11 @@ static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
             default: return conv_dma_launch<128, 32, 8, 1, 1, 32, 3, NP, EPI>(st, a);
         }
     } else if constexpr (EPI == 0) {
-        const double c[6] = {cost(128, 256, 1.0), cost(256, 192, 1.0), cost(128, 192, 1.08), cost(128, 128, 1.07), cost(64, 128, 1.17), cost(64, 96, 1.25)};
-        switch (least(c, 6)) {
+        // (128 x 128: two blocks a CU in step, so past 512 tiles it is pairs of rounds that count: 51 200 x 384 206 us for 193 of 256 x 192)
+        const double two = tiles(128, 128) > 512 && (tiles(128, 128) + 255) / 256 % 2 ? 16384 * 1.07 : 0.0;
+        const double c[7] = {cost(128, 256, 1.0), cost(256, 192, 1.0),  cost(128, 192, 1.08), cost(128, 128, 1.07) + two,
+                             cost(64, 128, 1.25), cost(64, 96, 1.4), cost(128, 96, 1.3)};
+        switch (least(c, 7)) {
             case 0: return conv_dma_launch<128, 256, 4, 4, 1, 32, 3, NP, EPI>(st, a);
             case 1: return conv_dma_launch<256, 192, 8, 2, 1, 32, 3, NP, EPI>(st, a);
             case 2: return conv_dma_launch<128, 192, 4, 2, 1, 32, 2, NP, EPI>(st, a);
@@ -1771,7 +1798,8 @@ static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
             case 4:
                 if (k64) return conv_dma_launch<64, 128, 2, 2, 1, 64, 2, NP, EPI>(st, a);
                 return conv_dma_launch<64, 128, 2, 2, 1, 32, 4, NP, EPI>(st, a);
-            default: return conv_dma_launch<64, 96, 4, 1, 1, 32, 4, NP, EPI>(st, a);
+            case 5: return conv_dma_launch<64, 96, 4, 1, 1, 32, 4, NP, EPI>(st, a);
+            default: return conv_dma_launch<128, 96, 4, 1, 1, 32, 2, NP, EPI>(st, a);
         }
     } else if constexpr (NP == 3) {
         return conv_dma_launch<64, 128, 4, 2, 1, 32, 3, NP, EPI>(st, a);
@@ -1958,14 +1986,15 @@ static void codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* 
                            c.num_heads, c.head_dim, c.window, terms);
     }
 }
-// the final conv over x (fp32 rows, activated), its history and the slots' positions (T codec frames on)
-static void codec_final(vox_codec* m, hipStream_t st, const float* x, const int32_t* slots, int n, int T, int L, float* out) {
+// the final conv over x (fp32 rows, activated), its history, a history still due and the slots' positions (T codec frames on)
+static void codec_final(vox_codec* m, hipStream_t st, const float* x, const int32_t* slots, int n, int T, int L, float* out, const ConvJob& pending = ConvJob{}) {
     const vox_codec_weights& w = m->w;
     const int cl = m->cfg.decoder_dim >> 4;
     if (!final_taps<7, true>(st, x, m->st_final, slots, w.final_w, w.final_b, out, n, L, cl))
         hipLaunchKernelGGL(k_final_conv, dim3((L + 3) / 4, n), dim3(256), 0, st, x, m->st_final, slots, w.final_w, w.final_b, out, L, cl);
-    state_update(st, m->st_final, slots, x, n, L, 6, cl);
-    hipLaunchKernelGGL(k_pos_advance, dim3((n + 255) / 256), dim3(256), 0, st, m->pos, slots, n, T);
+    const ConvJob last{m->st_final, x, L, 6, cl, n};
+    const int na = conv_job_blocks(pending, 256), nb = conv_job_blocks(last, 256);
+    hipLaunchKernelGGL(k_conv_jobs, dim3(na + nb + 1), dim3(256), 0, st, pending, last, na, nb, slots, m->pos, n, T);
 }
 // One chunk with fp32 activations, split three ways inside each conv (planes == 3).
 static int codec_chunk_f32(vox_codec* m, hipStream_t st, const int32_t* codes, int code_stride, const int32_t* slots, int n, int T, float* out) {
@@ -2059,13 +2088,9 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
     const int off3[3] = {2, 1, 0}, off7[7] = {6, 5, 4, 3, 2, 1, 0};
     int L = T;
     // A conv's history is rewritten after the conv has read it: by extra blocks of the next launch (its output must not be the history's
-    // source), or by a launch of its own where the next one is no k_conv_dma.
+    // source); the last one's with the final conv's.
     ConvJob job{};
     auto later = [&](float* state, const float* x, int P, int ch) { job = ConvJob{state, x, L, P, ch, n}; };
-    auto flush = [&] {
-        if (job.state) state_update(st, job.state, slots, job.x, n, job.L, job.P, job.C);
-        job = ConvJob{};
-    };
     auto conv = [&](const vox_conv_w& cw, const float* x, const float* state, int P, const int* offs) { return conv_s2_args(cw, x, state, slots, n, L, P, offs); };
     auto run = [&](ConvDmaArgs& a, int epi = 0) {
         a.job = job;
@@ -2164,8 +2189,7 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
             x = z;
         }
     }
-    flush();
-    codec_final(m, st, x, slots, n, T, L, out);
+    codec_final(m, st, x, slots, n, T, L, out, job);
     return VOX_OK;
 }
 
