@@ -1,4 +1,4 @@
-"""The LDS-DMA convolutions of the Qwen3 codec (k_conv_dma, k_conv_unit) at the shapes where their tiles can go wrong, against the CPU oracle in fp32.
+"""The LDS-DMA convolutions of the Qwen3 codec and of Mimi (k_conv_dma, k_conv_unit) at the shapes where their tiles can go wrong, against the CPU oracle in fp32.
 
 Channel counts that are multiples of 32, 64, 128 and 256 only (the k-steps of the tiles), fewer rows than one tile and rows that do not
 fill the last one, intermediate sizes that end inside a gate / up pair, chunks shorter than a conv's look-back (the history shifts in
@@ -50,4 +50,26 @@ def test_conv_tiles_against_fp32(dev, shape, n, chunk, precision):  # noqa: F811
     got = torch.cat([dec.decode_chunk(codes[:, :, t:t + chunk], cache)[0].cpu().clone() for t in range(0, 3 * chunk, chunk)], -1).numpy()
     assert got.shape == ref.shape and rms(ref) > 1e-3
     assert rms(got - ref) < (1e-4 if precision == "fp32" else 2 ** 8 * 1e-4), (rms(got - ref), rms(ref))
+    dec.close()
+
+
+@pytest.mark.parametrize("n,T", [(18, 2), (5, 3), (2, 1)])
+def test_mimi_units_do_not_depend_on_rows(dev, n, T):  # noqa: F811
+    """Mimi at its real widths: whole units of 128 and of 64 rows, and (odd frame counts) the two launches in their place, against a request
+    alone.  Products are exact and the sums fp32: another order moves a sample by some 2^-24 of the signal per stage, far below 1e-5."""
+    from oracle import mimi_ref as MR
+    from vox_serve_amd.tokenizer.mimi import MimiConfig, MimiDecoder
+    cfg = MR.MimiCfg()
+    W = MR.random_mimi_weights(cfg, seed=2)
+    pc = MimiConfig(**{k: getattr(cfg, k) for k in MimiConfig.__dataclass_fields__ if hasattr(cfg, k)})
+    dec = MimiDecoder(W, pc, device=dev, max_batch=n, max_frames=T)
+    codes = torch.randint(0, cfg.bins, (n, cfg.n_q, T), generator=torch.Generator().manual_seed(n))
+    both = dec.decode(codes).cpu().numpy()
+    assert rms(both) > 1e-4
+    for i in (0, n - 1):
+        one = dec.decode(codes[i:i + 1]).cpu().numpy()
+        assert rms(one - both[i:i + 1]) < 1e-5 * rms(both)
+    if n == 2:
+        ref = MR.MimiRef(cfg, W).decode(codes).numpy()
+        assert rms(both - ref) < 1e-5 * max(1.0, rms(ref))
     dec.close()

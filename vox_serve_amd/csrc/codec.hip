@@ -641,19 +641,21 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     }
 }
 
-// A whole residual unit of the decoder:  h += conv2(act2(conv1(x)))  and  out2 = act_next(h);  conv1: 7 taps, dilated, conv2: one tap, C -> C.
+// A whole residual unit of a decoder:  h += conv2(act2(conv1(x)))  and  out2 = act_next(h);  conv1: TAPS taps C -> CH, conv2: one tap CH -> C;
+// T = 2: SnakeBeta over two-term rows (Qwen3 codec: 7 taps, dilated, CH = C), T = 3: ELU over three-term rows (Mimi: 3 taps, CH = C / 2).
 // A block takes 16 MT NW rows of one request and ALL C channels of them; a wave takes 16 MT rows.  conv1 walks K in 32-channel chunks: a
-// chunk's rows with their look-back (up to 64) are staged once for the seven taps (two buffers, the next chunk's requests spread over the
+// chunk's rows with their look-back (up to HP) are staged once for all taps (two buffers, the next chunk's requests spread over the
 // taps of this one), the weights are a stream of C x 32 slices through S stages.  What the lanes then hold, eight neighbouring channels
 // of a row, is after SnakeBeta and the two-term split the activation operand of conv2 as it stands: conv2 is C / 32 further slices of the
 // same stream, and the intermediate never leaves the registers.  x, the history and the weights arrive by LDS DMA as in k_conv_dma.
 // Bound: memory (x, h read, h, out2 written: 944 MB at 614 400 rows x 96) beside the matrix cores and the activations' VALU work: 309 us there,
 // 3.1 TB/s (326 with the residual asked for in the epilogue; four stages or 64-row blocks 311 - 332); the staged form of this kernel, with
 // the intermediate through LDS, took 461 - 498.
-template <int C, int NW, int MT, int S>
-__global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaArgs a1, ConvDmaArgs a2, int H) {
-    constexpr int BM = 16 * MT * NW, R = BM + 64, NT = C / 16, NP = NT / 2, NCK = C / 32, TAPS = 7;
-    constexpr int SA = 2 * R * 64, SW = C * 64, CA = SA / 1024, CW = SW / 1024, NA = (CA + NW - 1) / NW, NB = (CW + NW - 1) / NW;
+template <int C, int CH, int TAPS, int T, int HP, int NW, int MT, int S>
+__global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_conv_unit(ConvDmaArgs a1, ConvDmaArgs a2, int H) {
+    constexpr int BM = 16 * MT * NW, R = BM + HP, NT = CH / 16, NP = CH / 32, NT2 = C / 16, NCK = C / 32;
+    constexpr int SA = T * R * 64, CA = SA / 1024, NA = (CA + NW - 1) / NW, CW1 = CH / 16, CW2 = C / 16, SW = (C > CH ? C : CH) * 64;
+    constexpr int NB = ((C > CH ? CW2 : CW1) + NW - 1) / NW;       // requests of a wave per slice (the smaller kind repeats some)
     constexpr int AT = (NA + TAPS - S + 1) / (TAPS - S + 2), AN = (NA + AT - 1) / AT;      // requests for rows per tap, taps that make them
     static_assert(AN <= TAPS - S + 2, "a chunk's rows are asked for by the taps that the next chunk's first wait covers");
     extern __shared__ __attribute__((aligned(1024))) char conv_lds[];
@@ -666,7 +668,7 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
     if (t >= a1.tm) return;
     const int m0 = t * BM, fr = lane & 15, fk = lane >> 4;
     const int b = m0 / a1.L, t0 = m0 - b * a1.L;
-    constexpr int rb = C * 4;
+    constexpr int rb = C * (T == 3 ? 6 : 4);
     // rows t0 - H .. t0 + BM - 1 at LDS rows 0 .. (the buffer's last rows repeat the tile's last one: no tap reads them)
     const char* xp[NA];
     int step[NA];
@@ -682,18 +684,19 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
         step[i] = e >= 0 || hist ? 64 : 0;
     }
     const auto wswz = [](int r) { return ((r >> 1) & 1) | ((r >> 2) & 2); };      // (rows are read as in k_conv_dma's PAIR order)
-    unsigned wo[NB];
+    unsigned wo1[NB], wo2[NB];
 #pragma unroll
     for (int i = 0; i < NB; ++i) {
-        const int q = (i * NW + wv) % CW * 64 + lane, r = q / 4;
-        wo[i] = (unsigned)(r * C + ((q & 3) ^ wswz(r)) * 8) * 2;
+        const int c1 = (i * NW + wv) % CW1 * 16 + (lane >> 2), c2 = (i * NW + wv) % CW2 * 16 + (lane >> 2);
+        wo1[i] = (unsigned)(c1 * C + ((lane & 3) ^ wswz(c1)) * 8) * 2;
+        wo2[i] = (unsigned)(c2 * CH + ((lane & 3) ^ wswz(c2)) * 8) * 2;
     }
     // the residual rows: asked for first where registers allow (their wait is the first rows' own)
-    constexpr bool EARLY = C == 96 && MT == 1;
-    f32x4 res[EARLY ? NP : 1][2];
+    constexpr bool EARLY = C <= 128 && MT == 1;
+    f32x4 res[EARLY ? NT2 / 2 : 1][2];
     if (EARLY) {
 #pragma unroll
-        for (int p = 0; p < NP; ++p)
+        for (int p = 0; p < NT2 / 2; ++p)
 #pragma unroll
             for (int q = 0; q < 2; ++q)
                 res[p][q] = *reinterpret_cast<const f32x4*>(a2.res + (size_t)(m0 + wv * 16 + fr) * C + p * 32 + fk * 8 + 4 * q);
@@ -706,14 +709,16 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
     int rt = 0, rc = 0, rs = 0;      // tap, chunk and stage of the next slice; past conv1's chunks: conv2's
     auto slice = [&]() {
         const bool second = rc >= NCK;
-        const int kc = second ? (rt < NCK ? rt : NCK - 1) : rc;      // (past the last slice it is asked for again)
-        const size_t at = reinterpret_cast<size_t>(second ? a2.w : a1.w) + ((second ? 0 : rt * C * C) + kc * 32) * 2;
+        const int kc = second ? (rt < NP ? rt : NP - 1) : rc;      // (past the last slice it is asked for again)
+        const size_t at = reinterpret_cast<size_t>(second ? a2.w : a1.w) + ((second ? 0 : rt * C * CH) + kc * 32) * 2;
         const char* base = reinterpret_cast<const char*>((size_t)__builtin_amdgcn_readfirstlane((int)(at >> 32)) << 32 |
                                                          (unsigned)__builtin_amdgcn_readfirstlane((int)at));
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const unsigned ld = __builtin_amdgcn_readfirstlane(sbase + 2 * SA + rs * SW + (i * NW + wv) % CW * 1024);
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(wo[i]), "s"(base), "s"(ld) : "memory");
+            const int c = i * NW + wv;
+            const unsigned ld = __builtin_amdgcn_readfirstlane(sbase + 2 * SA + rs * SW + (second ? c % CW2 : c % CW1) * 1024);
+            const unsigned off = second ? wo2[i] : wo1[i];
+            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(ld) : "memory");
         }
         rs = rs == S - 1 ? 0 : rs + 1;
         if (++rt == TAPS && !second) {
@@ -732,29 +737,29 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
     for (int i = 0; i < S - 1; ++i) slice();
     const int wfr = (fr >> 2) * 8 + (fr & 3), wpiece = (fk ^ wswz(wfr)) * 16;
     int ws = 0;      // stage of the slice being multiplied
-    auto weights = [&](cbf16x8 (&wf)[NT]) {
+    auto weights = [&](auto& wf) {
         const char* p = conv_lds + 2 * SA + ws * SW + wfr * 64 + wpiece;
 #pragma unroll
-        for (int j = 0; j < NT; ++j) wf[j] = *reinterpret_cast<const cbf16x8*>(p + ((j >> 1) * 32 + (j & 1) * 4) * 64);
+        for (int j = 0; j < (int)(sizeof(wf) / sizeof(wf[0])); ++j) wf[j] = *reinterpret_cast<const cbf16x8*>(p + ((j >> 1) * 32 + (j & 1) * 4) * 64);
         ws = ws == S - 1 ? 0 : ws + 1;
     };
     auto chunk = [&](int ck, auto last_tag) {
         constexpr bool LAST = decltype(last_tag)::value;
         const char* As = conv_lds + (ck & 1) * SA;
         auto tap = [&](auto tap_tag) {
-            constexpr int T = decltype(tap_tag)::value;
+            constexpr int TP = decltype(tap_tag)::value;
             // requests younger than this tap's slice: S - 2 slices and what the taps since then asked of the next chunk's rows
-            constexpr int lo = T - S + 2 > 0 ? (T - S + 2) * AT : 0, hi = T * AT < NA ? T * AT : NA, young = (S - 2) * NB + (!LAST && hi > lo ? hi - lo : 0);
+            constexpr int lo = TP - S + 2 > 0 ? (TP - S + 2) * AT : 0, hi = TP * AT < NA ? TP * AT : NA, young = (S - 2) * NB + (!LAST && hi > lo ? hi - lo : 0);
             asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(young) : "memory");
 #pragma unroll
-            for (int q = T * AT; q < (T + 1) * AT; ++q)
+            for (int q = TP * AT; q < (TP + 1) * AT; ++q)
                 if (!LAST && q < NA) rows(q, (ck + 1) & 1);
             slice();
-            const int r0 = wv * MT * 16 + fr + H - a1.off[T];
+            const int r0 = wv * MT * 16 + fr + H - a1.off[TP];
             cbf16x8 wf[NT];
             weights(wf);
 #pragma unroll
-            for (int p = 1; p >= 0; --p)
+            for (int p = T - 1; p >= 0; --p)
 #pragma unroll
                 for (int i = 0; i < MT; ++i) {
                     const int r = r0 + i * 16;
@@ -764,13 +769,16 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
                 }
         };
         tap(std::integral_constant<int, 0>{}); tap(std::integral_constant<int, 1>{}); tap(std::integral_constant<int, 2>{});
-        tap(std::integral_constant<int, 3>{}); tap(std::integral_constant<int, 4>{}); tap(std::integral_constant<int, 5>{});
-        tap(std::integral_constant<int, 6>{});
+        if constexpr (TAPS == 7) {
+            tap(std::integral_constant<int, 3>{}); tap(std::integral_constant<int, 4>{}); tap(std::integral_constant<int, 5>{});
+            tap(std::integral_constant<int, 6>{});
+        }
     };
+    static_assert(TAPS == 3 || TAPS == 7, "tap list");
     for (int ck = 0; ck + 1 < NCK; ++ck) chunk(ck, std::false_type{});
     chunk(NCK - 1, std::true_type{});
     // act2 of the sums, split: the operand of conv2 (channels 32 p + 8 fk + 0..7 of the lane's row)
-    cbf16x8 y[MT][NP][2];
+    cbf16x8 y[MT][NP][T];
 #pragma unroll
     for (int p = 0; p < NP; ++p) {
         const int c = p * 32 + fk * 8;
@@ -778,48 +786,61 @@ __global__ __launch_bounds__(64 * NW, C == 96 ? 4 : 2) void k_conv_unit(ConvDmaA
 #pragma unroll
         for (int q = 0; q < 2; ++q) {
             const f32x4 tb = a1.bias ? *reinterpret_cast<const f32x4_a4*>(a1.bias + c + 4 * q) : (f32x4){0.f, 0.f, 0.f, 0.f};
-            const f32x4 ta = *reinterpret_cast<const f32x4_a4*>(a1.sn_alpha + c + 4 * q), ti = *reinterpret_cast<const f32x4_a4*>(a1.sn_invb + c + 4 * q);
+            f32x4 ta = tb, ti = tb;
+            if constexpr (T == 2) {
+                ta = *reinterpret_cast<const f32x4_a4*>(a1.sn_alpha + c + 4 * q);
+                ti = *reinterpret_cast<const f32x4_a4*>(a1.sn_invb + c + 4 * q);
+            }
 #pragma unroll
             for (int e = 0; e < 4; ++e) { bi[4 * q + e] = tb[e]; al[4 * q + e] = ta[e]; ib[4 * q + e] = ti[e]; }
         }
 #pragma unroll
         for (int i = 0; i < MT; ++i) {
-            unsigned h[4], m[4];
+            float v[8];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const float v0 = snake_f(acc[i][2 * p + e / 2][e % 2 * 2] + bi[2 * e], al[2 * e], ib[2 * e]);
-                const float v1 = snake_f(acc[i][2 * p + e / 2][e % 2 * 2 + 1] + bi[2 * e + 1], al[2 * e + 1], ib[2 * e + 1]);
-                h[e] = pack_bf2(v0, v1);
-                m[e] = pack_bf2(v0 - bflo(h[e]), v1 - bfhi(h[e]));
+            for (int e = 0; e < 8; ++e) {
+                v[e] = acc[i][2 * p + e / 4][e % 4] + bi[e];
+                if constexpr (T == 2) v[e] = snake_f(v[e], al[e], ib[e]);
+                else v[e] = v[e] > 0.0f ? v[e] : expm1f(v[e]);
             }
-            y[i][p][0] = as_cbf8(make_uint4(h[0], h[1], h[2], h[3]));
-            y[i][p][1] = as_cbf8(make_uint4(m[0], m[1], m[2], m[3]));
+#pragma unroll
+            for (int t3 = 0; t3 < T; ++t3) {
+                unsigned h[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    h[e] = pack_bf2(v[2 * e], v[2 * e + 1]);
+                    v[2 * e] -= bflo(h[e]);
+                    v[2 * e + 1] -= bfhi(h[e]);
+                }
+                y[i][p][t3] = as_cbf8(make_uint4(h[0], h[1], h[2], h[3]));
+            }
         }
     }
+    f32x4 out[MT][NT2];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NT2; ++j) out[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int k = 0; k < NP; ++k) {
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * NB) : "memory");
         slice();
-        cbf16x8 wf[NT];
+        cbf16x8 wf[NT2];
         weights(wf);
 #pragma unroll
-        for (int p = 1; p >= 0; --p)
+        for (int p = T - 1; p >= 0; --p)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], y[i][k][p], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < NT2; ++j) out[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], y[i][k][p], out[i][j], 0, 0, 0);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (the repeated last slices: nothing may land after the block has ended)
 #pragma unroll
-    for (int p = 0; p < NP; ++p) {
+    for (int p = 0; p < NT2 / 2; ++p) {
         f32x4 v[MT][2];
 #pragma unroll
-        for (int i = 0; i < MT; ++i) { v[i][0] = acc[i][2 * p]; v[i][1] = acc[i][2 * p + 1]; }
-        conv_dma_out<2, false, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
+        for (int i = 0; i < MT; ++i) { v[i][0] = out[i][2 * p]; v[i][1] = out[i][2 * p + 1]; }
+        conv_dma_out<T, false, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
     }
 }
 
@@ -1836,11 +1857,11 @@ static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
 // A residual unit as ONE launch (k_conv_unit) where its tile can cover all channels and the rows fill the chip; *fused = 0 and nothing
 // launched otherwise (the caller then runs the two convs).  a1: conv1 with act2 (sn_*), a2: conv2 with res, out and the NEXT consumer's
 // activation, whose rows must not be a1's: a neighbouring tile still reads its look-back there.  (a1.job is done by extra blocks.)
-template <int C, int NW, int MT, int S>
+template <int C, int CH, int TAPS, int T, int HP, int NW, int MT, int S>
 static int conv_unit_launch(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int H) {
-    constexpr int BM = 16 * MT * NW, lds = 2 * 2 * (BM + 64) * 64 + S * C * 64;
+    constexpr int BM = 16 * MT * NW, lds = 2 * T * (BM + HP) * 64 + S * (C > CH ? C : CH) * 64;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
-    const auto kern = k_conv_unit<C, NW, MT, S>;
+    const auto kern = k_conv_unit<C, CH, TAPS, T, HP, NW, MT, S>;
     if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     a1.tm = a1.M / BM;
     a1.tiles8 = (a1.tm + 7) & ~7;
@@ -1859,9 +1880,28 @@ static int conv_unit(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int* fuse
     // rows: 424 -> 325; 6 400 rows, 100 tiles: 28 -> 30, there the two launches stay)
     if (omin < 0 || H > 64 || a1.L % 64 || !a2.res || (C == 192 && a1.M / 64 < 256)) return VOX_OK;
     *fused = 1;
-    if (C == 192) return conv_unit_launch<192, 4, 1, 3>(st, a1, a2, H);
-    if (a1.L % 128 == 0 && a1.M / 128 >= 256) return conv_unit_launch<96, 8, 1, 3>(st, a1, a2, H);
-    return conv_unit_launch<96, 4, 1, 3>(st, a1, a2, H);
+    if (C == 192) return conv_unit_launch<192, 192, 7, 2, 64, 4, 1, 3>(st, a1, a2, H);
+    if (a1.L % 128 == 0 && a1.M / 128 >= 256) return conv_unit_launch<96, 96, 7, 2, 64, 8, 1, 3>(st, a1, a2, H);
+    return conv_unit_launch<96, 96, 7, 2, 64, 4, 1, 3>(st, a1, a2, H);
+}
+
+// The same for Mimi's units (3 taps C -> C / 2, ELU, one tap back to C, three-term rows): the last two stages.  307 200 rows x 64: 145 us
+// in two launches -> 86 (276 MB: 3.2 TB/s), 76 800 x 128: 78 -> 65.
+static int conv_unit_elu(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int* fused) {
+    *fused = 0;
+    const int C = a2.N;
+    if (a1.n_taps != 3 || a2.n_taps != 1 || a1.Cin != C || a1.N * 2 != C || a2.Cin * 2 != C || (C != 64 && C != 128) || a1.bias_mod != a1.N ||
+        a2.bias_mod != C || a2.out2 == a1.x || !a2.res || !a1.elu)
+        return VOX_OK;
+    int H = 0, omin = 0;
+    for (int k = 0; k < 3; ++k) { H = a1.off[k] > H ? a1.off[k] : H; omin = a1.off[k] < omin ? a1.off[k] : omin; }
+    if (omin < 0 || H > 16 || a1.L % 64) return VOX_OK;
+    *fused = 1;
+    if (C == 64) {
+        if (a1.L % 128 == 0 && a1.M / 128 >= 256) return conv_unit_launch<64, 32, 3, 3, 16, 8, 1, 3>(st, a1, a2, H);
+        return conv_unit_launch<64, 32, 3, 3, 16, 4, 1, 3>(st, a1, a2, H);
+    }
+    return conv_unit_launch<128, 64, 3, 3, 16, 4, 1, 3>(st, a1, a2, H);
 }
 
 static void snake(hipStream_t st, const float* x, const vox_snake_w& s, float* y, size_t rows, int C, int terms = 0) {
@@ -2537,15 +2577,32 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
         { float* o = x; x = f0; f0 = f1; f1 = o; }
         L *= c.ratios[b];
         ch /= 2;
-        { ConvDmaArgs a = conv(bw.conv1, x, m->st_c1[b], 2, off3); elu_out(a, f0, ch / 2); VOX_TRY(run(a)); }                // f0 [nL, ch/2]
+        ConvDmaArgs a1 = conv(bw.conv1, x, m->st_c1[b], 2, off3), a2 = conv(bw.conv2, f0, nullptr, 0, nullptr);
+        elu_out(a1, f0, ch / 2);                                  // f0 [nL, ch/2]
+        a2.res = h;
+        elu_out(a2, f0, ch, b < 3);                               // h + conv2(f0), activated (the final conv reads fp32 rows)
+        int fused = 0;
+        a1.job = job;
+        VOX_TRY(conv_unit_elu(st, a1, a2, &fused));
+        if (fused) {
+            job = ConvJob{};
+            later(m->st_c1[b], x, 2, ch);
+            { float* o = x; x = f0; f0 = f1; f1 = o; }
+            continue;
+        }
+        VOX_TRY(run(a1));
         later(m->st_c1[b], x, 2, ch);
-        { ConvDmaArgs a = conv(bw.conv2, f0, nullptr, 0, nullptr); a.res = h; elu_out(a, f1, ch, b < 3); VOX_TRY(run(a)); }   // (the final conv reads fp32 rows)
-        { float* o = x; x = f1; f1 = o; }                                                                                     // h += conv2(...), activated
+        a2.out2 = f1;
+        VOX_TRY(run(a2));
+        { float* o = x; x = f1; f1 = o; }
     }
     if (c.last_kernel_size != 3 || !final_taps<3, false>(st, x, S ? m->st_final : nullptr, sl, w.final_w, w.final_b, out, n, L, ch))
         hipLaunchKernelGGL(k_mimi_final, dim3((L + 3) / 4, n), dim3(256), 0, st, x, w.final_w, w.final_b, out, L, ch, c.last_kernel_size,
                            S ? m->st_final : nullptr, sl);
-    if (S) state_update(st, m->st_final, sl, x, n, L, c.last_kernel_size - 1, ch);
+    if (S) {
+        if (job.state) state_update(st, job.state, sl, job.x, n, job.L, job.P, job.C);
+        state_update(st, m->st_final, sl, x, n, L, c.last_kernel_size - 1, ch);
+    }
     return VOX_OK;
 }
 
