@@ -62,3 +62,18 @@ def test_activation_behind_both_products(rows, mlp):
     # (a routed layer: a choice that bf16 rounding flips moves a whole row, so the bar holds for nine rows of ten)
     err = U.rel_err(got, KR.forward(cfg, S, toks), None if mlp["kind"] == "dense" else 0.9)
     assert err < BF16_BAR, err
+
+
+# K of the second product = the layer's inner width: one step into the second round of requests, two whole rounds, one step into the third,
+# three whole rounds and one step into a fourth (taken in turn)
+@pytest.mark.parametrize("rows,inner", [(2, 2080), (16, 4096), (7, 4128), (8, 6144), (16, 6176)])
+def test_rounds_of_a_few_row_product(rows, inner):
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.dense(inner))], width=64, vocab=50)
+    S = P.random_checkpoint(cfg, seed=5)
+    toks = torch.randint(0, 50, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
+    d = U.Driver(cfg, S, dtype=torch.bfloat16, page_size=16, pages=20, max_rows=rows)
+    try:
+        got = d.run_cut("r", toks, [rows])
+    finally:
+        d.close()
+    assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR

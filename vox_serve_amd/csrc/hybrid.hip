@@ -1146,7 +1146,10 @@ static void hb_settle(hipStream_t st, hb_pending& pd, int n, int W) {
 // 2..16 rows, bf16: one MFMA row tile; a block owns 16 output columns and its eight waves take the 32-wide k-steps w, w + 8, ...
 // with both fragments straight from memory (the weight fragment is one 16-byte request per lane, the activation fragment two,
 // converted to bf16 in registers); the eight partial tiles are added in wave order.  Needs K % 32 == 0.
-template <int EPI>
+// A wave asks for eight of its steps at once.  NIT = 2, 3: K has that many such rounds and the next round's requests go out before this
+// one's products (two register sets, straight-line code: a conditional request would make every wait a full one); one after the other each
+// round waited out the trip to memory (8 rows, 2048 x 5632: 17.1 us, now 14.9).  NIT = 0: any number of rounds, in turn.
+template <int EPI, int NIT>
 __global__ __launch_bounds__(512) void k_hb_gemm_rows16(const float* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
                                                         int N, int K, hb_rowmap rm) {
     __shared__ float red[8][16][17];
@@ -1167,26 +1170,41 @@ __global__ __launch_bounds__(512) void k_hb_gemm_rows16(const float* A, long lda
     hb_join_in jin;
     if (EPI == HB_EPI_JOIN && mine) jin = hb_join_load(rm.join, C + (size_t)orow * ldc, orow, n0 + ocol);
     constexpr int U = 8;
-    for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
-        uint4 wf[U];
-        float4 a0[U], a1[U];
+    uint4 wf[NIT ? 2 : 1][U];
+    float4 a0[NIT ? 2 : 1][U], a1[NIT ? 2 : 1][U];
+    auto fetch = [&](int set, int s0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int sidx = s0 + 8 * u;
-            const bool valid = sidx < nsteps;
-            const int k = (valid ? sidx : s0) << 5;
-            wf[u] = *(const uint4*)(wrow + k);
-            a0[u] = *(const float4*)(arow + k);
-            a1[u] = *(const float4*)(arow + k + 4);
-            if (!valid || !rowok) { a0[u] = make_float4(0.f, 0.f, 0.f, 0.f); a1[u] = a0[u]; }
+            const int sidx = s0 + 8 * u, k = (sidx < nsteps ? sidx : wv < nsteps ? wv : 0) << 5;
+            wf[set][u] = *(const uint4*)(wrow + k);
+            a0[set][u] = *(const float4*)(arow + k);
+            a1[set][u] = *(const float4*)(arow + k + 4);
         }
+    };
+    auto multiply = [&](int set, int s0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             union { uint4 q; hb_bf16x8 b; } af, bfv;
-            af.q.x = pack_bf2(a0[u].x, a0[u].y); af.q.y = pack_bf2(a0[u].z, a0[u].w);
-            af.q.z = pack_bf2(a1[u].x, a1[u].y); af.q.w = pack_bf2(a1[u].z, a1[u].w);
-            bfv.q = wf[u];
+            const bool ok = s0 + 8 * u < nsteps && rowok;
+            float4 x0 = a0[set][u], x1 = a1[set][u];
+            if (!ok) { x0 = make_float4(0.f, 0.f, 0.f, 0.f); x1 = x0; }
+            af.q.x = pack_bf2(x0.x, x0.y); af.q.y = pack_bf2(x0.z, x0.w);
+            af.q.z = pack_bf2(x1.x, x1.y); af.q.w = pack_bf2(x1.z, x1.w);
+            bfv.q = wf[set][u];
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af.b, bfv.b, acc, 0, 0, 0);
+        }
+    };
+    if constexpr (NIT > 0) {
+        fetch(0, wv);
+#pragma unroll
+        for (int i = 0; i < NIT; ++i) {
+            if (i + 1 < NIT) fetch((i + 1) & 1, wv + 8 * U * (i + 1));
+            multiply(i & 1, wv + 8 * U * i);
+        }
+    } else {
+        for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
+            fetch(0, s0);
+            multiply(0, s0);
         }
     }
 #pragma unroll
@@ -1208,7 +1226,11 @@ template <int EPI>
 bool hb_try_rows16(hipStream_t st, const float* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
                    const hb_rowmap& rm, int nz) {
     if (M < 2 || M > 16 || (K & 31) || (lda & 3) || ((size_t)A & 15) || ((size_t)W & 15) || !hb_batch_aligned(rm, nz, 2)) return false;
-    hipLaunchKernelGGL((k_hb_gemm_rows16<EPI>), dim3((N + 15) / 16, nz), dim3(512), 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
+    const int nit = ((K >> 5) + 63) / 64;
+    const dim3 grid((N + 15) / 16, nz), block(512);
+    if (nit == 2) hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, 2>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
+    else if (nit == 3) hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, 3>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
+    else hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, 0>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
     return true;
 }
 template <int EPI>
