@@ -292,7 +292,7 @@ __device__ __forceinline__ void ln_row_stats(const float* row, int C, int l16, f
 }
 
 // ================================================================================================
-// Convolutions over S2 rows through LDS DMA.  BM x BN outputs per block of WM x WN x WK waves; K is walked tap by tap in steps of BK
+// Convolutions over S2 (NP = 1: their first terms; 2) and S3 (NP = 3) rows through LDS DMA.  BM x BN outputs per block of WM x WN x WK waves; K is walked tap by tap in steps of BK
 // channels.  A step's NP x BM activation rows (a row may lie in the chunk, in the history or in neither) and BN weight rows go from memory
 // straight into one of S LDS stages (global_load_lds, 1 KB per wave instruction); S - 1 steps are in flight and no register holds them.
 // One wait + barrier per step: every wave's part of the step has landed, and nobody reads the stage of the step before any more.  16-byte
