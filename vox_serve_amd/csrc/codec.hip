@@ -359,10 +359,6 @@ struct ConvDmaArgs : ConvGemmArgs {
     ConvJob job;
 };
 __device__ uint4 g_conv_zero_row[1];        // what a tap reads outside the chunk and its history
-// (m0 holds the LDS address of the instruction; nothing else in the kernels that use it does)
-__device__ __forceinline__ void conv_dma16(const char* p, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
-}
 typedef f32x4 f32x4_a4 __attribute__((aligned(4)));       // (per-channel constants are where the caller's tensors have them)
 // W neighbouring channels of a row as its T terms
 template <int T, int W>
@@ -527,9 +523,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     auto request = [&](int stage) {
         const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * ST);
 #pragma unroll
-        for (int i = 0; i < NA; ++i) conv_dma16(cur[i], ls + (i * NWV + wv) % CA * 1024);
+        for (int i = 0; i < NA; ++i) lds_dma16(cur[i], ls + (i * NWV + wv) % CA * 1024);
 #pragma unroll
-        for (int i = 0; i < NB; ++i) conv_dma16(wp[i], ls + SA + (i * NWV + wv) % CB * 1024);
+        for (int i = 0; i < NB; ++i) lds_dma16(wp[i], ls + SA + (i * NWV + wv) % CB * 1024);
         if (++rq >= nit) return;     // (past the last step the same one is asked for again: the count in flight stays the same)
 #pragma unroll
         for (int i = 0; i < NA; ++i) cur[i] += step[i];
@@ -703,7 +699,7 @@ __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_co
     }
     const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)conv_lds;
     auto rows = [&](int i, int buf) {
-        conv_dma16(xp[i], __builtin_amdgcn_readfirstlane(sbase + buf * SA + (i * NW + wv) % CA * 1024));
+        lds_dma16(xp[i], __builtin_amdgcn_readfirstlane(sbase + buf * SA + (i * NW + wv) % CA * 1024));
         xp[i] += step[i];
     };
     int rt = 0, rc = 0, rs = 0;      // tap, chunk and stage of the next slice; past conv1's chunks: conv2's
@@ -718,7 +714,7 @@ __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_co
             const int c = i * NW + wv;
             const unsigned ld = __builtin_amdgcn_readfirstlane(sbase + 2 * SA + rs * SW + (second ? c % CW2 : c % CW1) * 1024);
             const unsigned off = second ? wo2[i] : wo1[i];
-            asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(ld) : "memory");
+            lds_dma16(base, off, ld);
         }
         rs = rs == S - 1 ? 0 : rs + 1;
         if (++rt == TAPS && !second) {

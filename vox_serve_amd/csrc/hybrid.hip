@@ -639,10 +639,6 @@ struct hb_glu_args {
     float limit, alpha, up_offset;
     int gelu;
 };
-// (m0 holds the LDS address of the instruction; nothing else in this kernel uses it)
-__device__ __forceinline__ void hb_dma16(const void* base, unsigned off, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory");
-}
 template <int BM, int BN, int WM, int WN, int S, int EPI, bool GLU, bool LIST>
 __global__ __launch_bounds__(WM * WN * 64) void k_hb_gemm_dma(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
                                                               int N, int K, hb_rowmap rm, hb_glu_args glu) {
@@ -687,9 +683,9 @@ __global__ __launch_bounds__(WM * WN * 64) void k_hb_gemm_dma(const bf16_t* A, l
     auto request = [&](int stage, int k0) {
         const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * (STAGE * 2));
 #pragma unroll
-        for (int i = 0; i < NA; ++i) hb_dma16(A, ao[i] + k0 * 2, ls + i * NWV * 1024);
+        for (int i = 0; i < NA; ++i) lds_dma16(A, ao[i] + k0 * 2, ls + i * NWV * 1024);
 #pragma unroll
-        for (int i = 0; i < NW; ++i) hb_dma16(Wt, wo[i] + k0 * 2, ls + BM * 128 + i * NWV * 1024);
+        for (int i = 0; i < NW; ++i) lds_dma16(Wt, wo[i] + k0 * 2, ls + BM * 128 + i * NWV * 1024);
     };
     hb_f32x4 acc[MT][NT];
 #pragma unroll

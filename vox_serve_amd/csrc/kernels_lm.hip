@@ -1525,10 +1525,6 @@ __global__ __launch_bounds__(512) void k_gemm_fullk(LinArgs a) {
 // third a norm launch of 4.5).  More than two stages give nothing (14.0 / 14.5 / 14.8 with 2 / 3 / 5); fragment-major rows are worth a
 // sixth (1 KB requests: gate / up 20.7 -> 17.7), which is why the norm writes them so.
 // ================================================================================================
-// (m0 holds the LDS address of the instruction; nothing else in this kernel uses it)
-__device__ __forceinline__ void rows_dma16(const char* p, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory");
-}
 template <int MT, int NT, int EPI, int S>
 __global__ __launch_bounds__(512) void k_gemm_rows(LinArgs a) {
     constexpr bool SM = (EPI == EPI_SILU_MUL);
@@ -1565,9 +1561,9 @@ __global__ __launch_bounds__(512) void k_gemm_rows(LinArgs a) {
     auto request = [&](int stage) {
         const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * STAGE);
 #pragma unroll
-        for (int i = 0; i < NW; ++i) rows_dma16(wp[i], ls + i * 1024);
+        for (int i = 0; i < NW; ++i) lds_dma16(wp[i], ls + i * 1024);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) rows_dma16(xp[m], ls + (NW + m) * 1024);
+        for (int m = 0; m < MT; ++m) lds_dma16(xp[m], ls + (NW + m) * 1024);
         if (++rq >= ks_n) return;      // (past the last step the same one is asked for again: the count in flight stays the same)
 #pragma unroll
         for (int i = 0; i < NW; ++i) wp[i] += wstep;
