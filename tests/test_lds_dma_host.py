@@ -37,3 +37,12 @@ def test_m0_is_settled_when_the_dma_reads_it(text, source):
     wrote = next(i for i, t in enumerate(text) if re.match(r"s_\w+ m0,", t))
     assert wrote < load and wait_states(text[wrote + 1:load]) >= 1
     assert '"m0"' in source
+
+
+@pytest.mark.parametrize("text,source", BLOCKS)
+def test_a_scalar_base_is_settled_when_the_dma_reads_it(text, source):
+    """The base comes from outside the block, where v_readfirstlane or v_readlane may have written it last: five wait states between a vector
+    write of a scalar register and the memory instruction that addresses with it."""
+    load = next(i for i, t in enumerate(text) if "load_lds" in t)
+    if not text[load].endswith("off"):
+        assert wait_states(text[:load]) >= 5

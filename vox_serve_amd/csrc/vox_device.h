@@ -41,13 +41,15 @@ __device__ __forceinline__ const T* assume_global(const T* p) {
     return (const T*)(const __attribute__((address_space(1))) T*)p;
 }
 // Memory -> LDS without a register on the way (one wave instruction: 64 lanes x 16 bytes to lds, lds + 16, ...): from p, or from a scalar
-// base + a 32-bit offset per lane.  The waits of such a kernel are its own (vmcnt).  m0 holds the LDS address; the wait state that a
-// scalar write of m0 needs before the instruction reads it stands here, because the compiler inserts none inside an asm.
+// base + a 32-bit offset per lane.  The waits of such a kernel are its own (vmcnt).  m0 holds the LDS address.  The compiler inserts no wait
+// states inside an asm, so they stand here: one between a scalar write of m0 and the instruction that reads it; five between a vector
+// write of a scalar register (v_readfirstlane, or v_readlane of a spilled one, may be the last thing in front) and the memory instruction
+// that takes its base from it (s_mov is the first of them).
 __device__ __forceinline__ void lds_dma16(const void* p, unsigned lds) {
     asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(p), "s"(lds) : "memory", "m0");
 }
 __device__ __forceinline__ void lds_dma16(const void* base, unsigned off, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
+    asm volatile("s_mov_b32 m0, %2\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds) : "memory", "m0");
 }
 __device__ __forceinline__ float dot8(uint4 w, uint4 x, float a) {
     a = __fmaf_rn(bflo(w.x), bflo(x.x), a);
