@@ -297,9 +297,13 @@ __device__ __forceinline__ void ln_row_stats(const float* row, int C, int l16, f
 // straight into one of S LDS stages (global_load_lds, 1 KB per wave instruction); S - 1 steps are in flight and no register holds them.
 // One wait + barrier per step: every wave's part of the step has landed, and nobody reads the stage of the step before any more.  16-byte
 // pieces lie swizzled by row (in the address that each lane reads), so the fragment reads of 16 rows do not meet in a bank.
-// WK > 1: the waves share the 32-channel slices of a step and add their sums through LDS at the end — a call of a few rows then has
-// every wave of a CU at work on one small tile.
-// WP = 2: every tap has two weight planes (n_taps * N rows apart; fp32 weights as two terms) that share the tap's rows.
+// WP = 1: every output adds its products tap by tap, 32 channels at a time in ascending order, the lowest term first, in whatever tile the
+// rows pick, so a request's samples do not depend on its batch.  WK > 1: WM * WN * (WK - 1) further waves only load.  In a small tile the
+// few waves that multiply are a serial chain (barrier, LDS reads, dependent MFMAs), and their share of the requests stood in it (10 rows, 20
+// and 40 rows, us, 4 or 8 waves that share K / one such wave with loads / with loaders: 3072 x 512 6.5 / 6.9 / 5.5, 1024 x 4096 8.7 / 11.3 / 9.6,
+// 1536 x 7 x 1024 14.4 / 18.1 / 14.5, 6144 x 2 x 1536 14.7 / 16.9 / 13.1).
+// WP = 2: every tap has two weight planes (n_taps * N rows apart; fp32 weights as two terms) that share the tap's rows; WK waves share the
+// 32-channel slices of a step and add their sums through LDS at the end (hift_conv keeps one such order for all its tiles).
 // EPI: 0, CONV_GELU, or CONV_GLU: columns come in pairs (n, N + n) of w, out2 <- S2 of silu(v[n]) * v[N + n], N columns.
 // The weights are the MFMA's first operand, so a lane ends with 4 (8) neighbouring channels of one row: the residual, the constants and both
 // outputs move in 16-byte accesses without a lane exchange.  With a lane per column the same epilogue cost more than the products of the
@@ -356,6 +360,7 @@ struct ConvDmaArgs : ConvGemmArgs {
     float rms_eps;
     const float* nw;       // out2 <- terms of v * nw[n] (no activation), or NULL
     int elu;               // out2 <- ELU of v
+    int parts;             // three-term rows: sums start anew every 256 channels (conv_long_sums)
     ConvJob job;
 };
 __device__ uint4 g_conv_zero_row[1];        // what a tap reads outside the chunk and its history
@@ -455,12 +460,13 @@ __device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x
 #define CONV_GLU 2
 template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI, int WP = 1>
 __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
-    constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8;
+    constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8, KW = WP == 2 ? WK : 1;
     constexpr int SA = NP * BM * BK * 2, SB = WP * BN * BK * 2, ST = SA + SB, CA = SA / 1024, CB = SB / 1024;
     constexpr bool PAIR = EPI != CONV_GLU && NT % 2 == 0;
-    constexpr int NA = (CA + NWV - 1) / NWV, NB = (CB + NWV - 1) / NWV;      // (where the waves do not divide them some chunks are asked for twice)
-    static_assert(SA % 1024 == 0 && SB % 1024 == 0 && KS % WK == 0 && (BM * PPR) % 64 == 0, "whole wave instructions");
-    static_assert(WK == 1 || NWV * MT * NT * 1024 <= S * ST, "partial sums");
+    constexpr int NC = WM * WN, NLD = KW == 1 && WK > 1 ? NWV - NC : NWV;      // waves that multiply one part of K; waves that load
+    constexpr int NA = (CA + NLD - 1) / NLD, NB = (CB + NLD - 1) / NLD;      // (where the waves do not divide them some chunks are asked for twice)
+    static_assert(SA % 1024 == 0 && SB % 1024 == 0 && KS % KW == 0 && (BM * PPR) % 64 == 0, "whole wave instructions");
+    static_assert(KW == 1 || NWV * MT * NT * 1024 <= S * ST, "partial sums");
     static_assert((BK & (BK - 1)) == 0 && (EPI != CONV_GLU || NT % 2 == 0), "swizzle; gate and up columns in one lane");
     extern __shared__ __attribute__((aligned(1024))) char conv_lds[];
     __shared__ float rms_s[BM];
@@ -472,7 +478,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     const int t = ((int)blockIdx.x & 7) * (a.tiles8 >> 3) + ((int)blockIdx.x >> 3);
     if (t >= a.tm * a.tn) return;
     const int m0 = (a.mfast ? t % a.tm : t / a.tn) * BM, n0 = (a.mfast ? t / a.tm : t % a.tn) * BN;      // (glu: n0 counts gate and up columns)
-    const int wk = wv % WK, wmn = wv / WK, wm = wmn / WN, wn = wmn % WN, fr = lane & 15, fk = lane >> 4;
+    const int wk = wv / NC, wmn = wv % NC, wm = wmn / WN, wn = wmn % WN, fr = lane & 15, fk = lane >> 4, lw = NLD < NWV ? wv - NC : wv;
+    const bool loads = NLD == NWV || lw >= 0, multiplies = NLD == NWV || lw < 0;
     const int rb = a.Cin * (NP == 3 ? 6 : 4);
     // The weights are the first operand of the MFMA: a lane's four sums are neighbouring channels of one row.  PAIR: tiles j and j + 1 take the
     // weight rows 8 q + 0..3 and 8 q + 4..7 (q = 0..3), so that they hold eight neighbouring channels together.
@@ -483,27 +490,29 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     // per DMA instruction of the wave: the lane's row of the chunk (its time), that row in x and the row that time 0 would have in the history
     const char *xp[NA], *sp[NA], *cur[NA], *wp[NB];
     int ts[NA], step[NA];
+    if (loads) {
 #pragma unroll
-    for (int i = 0; i < NA; ++i) {
-        const int q = (i * NWV + wv) % CA * 64 + lane, pl = q / (BM * PPR), r = q / PPR % BM, pc = (q % PPR) ^ (BK == 32 ? (r >> 1) & 3 : r & 7);
-        int m = m0 + r;
-        m = m < a.M ? m : a.M - 1;                  // (rows past the end repeat the last one: nothing of them is stored)
-        const int b = m / a.L;
-        ts[i] = m - b * a.L;
-        xp[i] = reinterpret_cast<const char*>(a.x) + (size_t)m * rb + pl * a.Cin * 2 + pc * 16;
-        sp[i] = a.state ? reinterpret_cast<const char*>(a.state) + ((size_t)a.slots[b] * a.P + a.P + ts[i]) * rb + pl * a.Cin * 2 + pc * 16 : nullptr;
-    }
-#pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        const int q = (i * NWV + wv) % CB * 64 + lane, r = q / PPR % BN, pl = q / (BN * PPR), pc = (q % PPR) ^ wswz(r);
-        int n = n0 + r;
-        if (EPI == CONV_GLU) {
-            n = (n0 >> 1) + (r >> 5) * 16 + (r & 15);
-            n = (n < a.N ? n : a.N - 1) + ((r >> 4) & 1) * a.N;
-        } else {
-            n = n < a.N ? n : a.N - 1;
+        for (int i = 0; i < NA; ++i) {
+            const int q = (i * NLD + lw) % CA * 64 + lane, pl = q / (BM * PPR), r = q / PPR % BM, pc = (q % PPR) ^ (BK == 32 ? (r >> 1) & 3 : r & 7);
+            int m = m0 + r;
+            m = m < a.M ? m : a.M - 1;                  // (rows past the end repeat the last one: nothing of them is stored)
+            const int b = m / a.L;
+            ts[i] = m - b * a.L;
+            xp[i] = reinterpret_cast<const char*>(a.x) + (size_t)m * rb + pl * a.Cin * 2 + pc * 16;
+            sp[i] = a.state ? reinterpret_cast<const char*>(a.state) + ((size_t)a.slots[b] * a.P + a.P + ts[i]) * rb + pl * a.Cin * 2 + pc * 16 : nullptr;
         }
-        wp[i] = reinterpret_cast<const char*>(a.w) + (((size_t)pl * a.n_taps * a.N + n) * a.Cin + pc * 8) * 2;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) {
+            const int q = (i * NLD + lw) % CB * 64 + lane, r = q / PPR % BN, pl = q / (BN * PPR), pc = (q % PPR) ^ wswz(r);
+            int n = n0 + r;
+            if (EPI == CONV_GLU) {
+                n = (n0 >> 1) + (r >> 5) * 16 + (r & 15);
+                n = (n < a.N ? n : a.N - 1) + ((r >> 4) & 1) * a.N;
+            } else {
+                n = n < a.N ? n : a.N - 1;
+            }
+            wp[i] = reinterpret_cast<const char*>(a.w) + (((size_t)pl * a.n_taps * a.N + n) * a.Cin + pc * 8) * 2;
+        }
     }
     const int nck = a.Cin / BK, nit = a.n_taps * nck;
     const size_t wtap = (size_t)(EPI == CONV_GLU ? 2 * a.N : a.N) * a.Cin * 2 - (size_t)a.Cin * 2;      // from the end of one tap's row to the next tap's
@@ -519,13 +528,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         }
     };
     int rt = 0, rc = 0, rq = 0;      // tap, chunk and number of the next request
-    tap_rows(0);
     auto request = [&](int stage) {
         const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * ST);
 #pragma unroll
-        for (int i = 0; i < NA; ++i) lds_dma16(cur[i], ls + (i * NWV + wv) % CA * 1024);
+        for (int i = 0; i < NA; ++i) lds_dma16(cur[i], ls + (i * NLD + lw) % CA * 1024);
 #pragma unroll
-        for (int i = 0; i < NB; ++i) lds_dma16(wp[i], ls + SA + (i * NWV + wv) % CB * 1024);
+        for (int i = 0; i < NB; ++i) lds_dma16(wp[i], ls + SA + (i * NLD + lw) % CB * 1024);
         if (++rq >= nit) return;     // (past the last step the same one is asked for again: the count in flight stays the same)
 #pragma unroll
         for (int i = 0; i < NA; ++i) cur[i] += step[i];
@@ -538,8 +546,11 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
             for (int i = 0; i < NB; ++i) wp[i] += wtap;
         }
     };
+    if (loads) {
+        tap_rows(0);
 #pragma unroll
-    for (int s = 0; s < S - 1; ++s) request(s);
+        for (int s = 0; s < S - 1; ++s) request(s);
+    }
     if (a.rms_x) {
         for (int r = wv; r < BM; r += NWV) {
             const int m = m0 + r < a.M ? m0 + r : a.M - 1;
@@ -553,21 +564,50 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
             if (lane == 0) rms_s[r] = rsqrtf(s / (float)a.Cin + a.rms_eps);
         }
     }
-    f32x4 acc[MT][NT];
+    int stage = 0;
+    auto landed = [&]() { asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NB)) : "memory"); };
+    if (!multiplies) {
+        for (int it = 0; it < nit; ++it) {
+            landed();
+            request(stage == 0 ? S - 1 : stage - 1);
+            stage = stage == S - 1 ? 0 : stage + 1;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+    constexpr bool PARTS = NP == 3 && WP == 1 && BK >= 64;      // tiles that know ConvDmaArgs::parts
+    f32x4 acc[MT][NT], done[PARTS ? MT : 1][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NT; ++j) {
+            acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            if (PARTS) done[i][j] = acc[i][j];
+        }
+    auto part_done = [&]() {
+        if constexpr (PARTS)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int j = 0; j < NT; ++j) {
+                    done[i][j] += acc[i][j];
+                    acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+                }
+    };
     const int wfr = PAIR ? (fr >> 2) * 8 + (fr & 3) : fr;
-    int stage = 0;
     for (int it = 0; it < nit; ++it) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NB)) : "memory");
-        request(stage == 0 ? S - 1 : stage - 1);
+        if (loads) {
+            landed();
+            request(stage == 0 ? S - 1 : stage - 1);
+        } else {
+            asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        }
+        if (PARTS && a.parts && it % (256 / BK) == 0) part_done();
         const char *as = conv_lds + stage * ST + (wm * MT * 16 + fr) * BK * 2, *bs = conv_lds + stage * ST + SA + (wn * NT * 16 + wfr) * BK * 2;
 #pragma unroll
-        for (int k = 0; k < KS / WK; ++k) {
-            const int piece = (((wk * (KS / WK) + k) * 4 + fk) ^ (BK == 32 ? (fr >> 1) & 3 : fr & 7)) * 16;
-            const int wpiece = (((wk * (KS / WK) + k) * 4 + fk) ^ wswz(wfr)) * 16;
+        for (int k = 0; k < KS / KW; ++k) {
+            const int piece = (((wk * (KS / KW) + k) * 4 + fk) ^ (BK == 32 ? (fr >> 1) & 3 : fr & 7)) * 16;
+            const int wpiece = (((wk * (KS / KW) + k) * 4 + fk) ^ wswz(wfr)) * 16;
             cbf16x8 bf[WP][NT];
 #pragma unroll
             for (int w = 0; w < WP; ++w)
@@ -589,26 +629,32 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         }
         stage = stage == S - 1 ? 0 : stage + 1;
     }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");        // (the repeated last steps: nothing may land any more)
+    if (KW > 1) asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");        // (the repeated last steps: nothing may land any more)
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (PARTS)
+#pragma unroll
+        for (int i = 0; i < MT; ++i)
+#pragma unroll
+            for (int j = 0; j < NT; ++j) acc[i][j] = done[i][j] + acc[i][j];
     constexpr int FR = MT * NT;
-    f32x4* part = reinterpret_cast<f32x4*>(conv_lds) + (size_t)wmn * WK * FR * 64 + lane;
-    if (WK > 1) {
+    f32x4* part = reinterpret_cast<f32x4*>(conv_lds) + (size_t)wmn * KW * FR * 64 + lane;
+    if (KW > 1) {
 #pragma unroll
         for (int f = 0; f < FR; ++f) part[(wk * FR + f) * 64] = acc[f / NT][f % NT];
         __syncthreads();
     }
     auto sum = [&](int f) {
-        if (WK == 1) return acc[f / NT][f % NT];
+        if (KW == 1) return acc[f / NT][f % NT];
         f32x4 v = part[f * 64];
 #pragma unroll
-        for (int k = 1; k < WK; ++k) v += part[(k * FR + f) * 64];
+        for (int k = 1; k < KW; ++k) v += part[(k * FR + f) * 64];
         return v;
     };
     const int rl = wm * MT * 16 + fr, nl = n0 + wn * NT * 16;
     if constexpr (EPI == CONV_GLU) {
 #pragma unroll
         for (int f = 0; f < FR; f += 2)
-            if (WK == 1 || (f / 2) % WK == wk)
+            if (KW == 1 || (f / 2) % KW == wk)
                 conv_dma_glu(a, sum(f), sum(f + 1), rms_s[rl + f / NT * 16], m0 + rl + f / NT * 16, (nl >> 1) + f % NT * 8 + fk * 4);
     } else {
         constexpr int P = PAIR ? 2 : 1;
@@ -616,7 +662,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
 #pragma unroll
         for (int j = 0; j < NT; j += P) {
             const int n = nl + j * 16 + fk * 4 * P;
-            if constexpr (WK == 1) {
+            if constexpr (KW == 1) {
                 f32x4 v[MT][P];
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
@@ -626,7 +672,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
             } else {
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
-                    if ((i * (NT / P) + j / P) % WK == wk) {
+                    if ((i * (NT / P) + j / P) % KW == wk) {
                         f32x4 v[1][P];
 #pragma unroll
                         for (int q = 0; q < P; ++q) v[0][q] = sum(i * NT + j + q);
@@ -1610,7 +1656,7 @@ static thread_local int g_conv_planes = 3;
 // time is the number of dependent K steps, not MFMA issue
 static thread_local int g_conv_skinny_rows = 48;
 // k_rows_gemm for eligible shapes: the flows only (their row bound is unbounded, so one kernel serves a shape at every batch size; the
-// codecs' and HiFT's few-row stages become many-row stages as the batch grows and must keep the staged kernels' summation order)
+// codecs' and HiFT's few-row stages become many-row stages as the batch grows and must keep one summation order)
 static thread_local bool g_conv_rows_gemm = false;
 // few-row GEMMs walk K in 256-wide steps where Cin allows (half the dependent steps of the 128-wide walk; same accumulation order, so
 // the results are bit-identical).  VOX_SKINNY_BK256=0 keeps the 128-wide walk (A/B timing).
@@ -1751,36 +1797,47 @@ static int conv_dma_launch(hipStream_t st, ConvDmaArgs& a) {
     hipLaunchKernelGGL(kern, dim3(a.tiles8 + conv_job_blocks(a.job, threads)), dim3(threads), lds, st, a);
     return VOX_OK;
 }
-// The smallest tile that leaves no CU a second round (the waves of a block share K): a call of few rows is a chain of dependent steps,
-// and more blocks, fewer columns and more waves per step each shorten it.  Past one 64 x 64 tile per CU the waves take outputs, not K;
-// past two the tile grows (fewer bytes through LDS per product).  us, against the staged kernels, two-term rows (M rows, N x taps x Cin):
-//   M = 10: 3072 x 512 7.1 -> 4.4, 512 x 1024 10.4 -> 4.9 | 40: 1024 x 4096 33 -> 7.8, 1536 x 7 x 1024 58 -> 14, 6144 x 2 x 1536 31 -> 14
-//   M = 320: 768 x 7 x 768 48 -> 16, 1920 x 2 x 768 22 -> 12 | 1600: 384 x 7 x 384 36 -> 18 | 6400: 192 x 7 x 192 30 -> 18.5
+// The smallest tile that leaves no CU a second round: a call of few rows is a chain of dependent steps, and more blocks, fewer columns and
+// deeper steps each shorten it.  Past one 64 x 64 tile per CU the waves all load and multiply; past two the tile grows (fewer bytes through
+// LDS per product).  us, against the staged kernels, two-term rows (M rows, N x taps x Cin):
+//   M = 10: 3072 x 512 7.1 -> 5.4, 512 x 1024 10.4 -> 5.7 | 20: 4096 x 1024 5.7, 1024 x 4096 9.6 | 40: 1536 x 7 x 1024 58 -> 14.5, 6144 x 2 x 1536 31 -> 13.1
+//   M = 320: 768 x 7 x 768 48 -> 15.2, 1920 x 2 x 768 22 -> 11.3 | 1600: 384 x 7 x 384 36 -> 16.4 | 6400: 192 x 7 x 192 30 -> 19
 //   M = 1280: 1536 x 7 x 1024 157 -> 72, 6144 x 2 x 1536 157 -> 84 | 10240: 768 x 7 x 768 194 -> 134, 1920 x 2 x 768 168 -> 131
-//   three-term rows: M = 320: 4096 x 2 x 1024 45 -> 30 (64 x 128; 64 x 64), 76 800: 256 x 2 x 128 67 (128 x 128), 307 200: 32 x 3 x 64 53
+//   three-term rows: M = 320: 1024 x 7 x 512 18.8, 4096 x 2 x 1024 45 -> 28 | 2560: 256 x 3 x 512 14.4 | 76 800: 256 x 2 x 128 67 (128 x 128)
 //   M = 51200: 384 x 7 x 384 250 -> 193 (rounds of 256 tiles decide: 128 x 256 leaves a quarter of its columns empty there, > 245)
+// Two multiplying waves and eight that load beat one of either kind in 16 x 32 tiles (10 rows, 3072 x 512: 5.4; four loaders 5.9; 16 x 16 with
+// one and four: 5.8).
+// Three-term rows carry the fp32 values, so the order of a long sum is what is left of the error: from 768 products on an output adds parts of
+// 256 channels (a property of the layer, as the order has to be).  Mimi against 64 bits, 16 requests of 10 frames: 1.26e-6 in one run, 6.6e-7 so.
+// Their many-row tile is 64 x 128; 128 x 128 has no registers for the parts (15 360 rows, 640 x 2 x 256: 46 us, with parts 57).
+static bool conv_long_sums(int taps, int cin) { return cin % 64 == 0 && taps * cin >= 768; }
 template <int NP, int EPI>
 static int conv_dma_pick(hipStream_t st, ConvDmaArgs& a) {
     const int n2 = EPI == CONV_GLU ? 2 * a.N : a.N;
     const auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((n2 + bn - 1) / bn); };
-    const bool k64 = a.Cin % 64 == 0, k128 = a.Cin % 128 == 0;      // (other Cin: 32-channel steps, waves take outputs)
+    const bool k64 = a.Cin % 64 == 0, k128 = a.Cin % 128 == 0;      // (other Cin: 32-channel steps)
+    a.parts = NP == 3 && conv_long_sums(a.n_taps, a.Cin);
     if (k128) {
-        if constexpr (EPI != CONV_GLU)
-            if (tiles(16, 16) <= 256) return conv_dma_launch<16, 16, 1, 1, 4, 128, 8, NP, EPI>(st, a);
-        if (tiles(16, 32) <= 256) {
-            if (a.Cin % 256 == 0) return conv_dma_launch<16, 32, 1, 1, 8, 256, NP == 3 ? 3 : 4, NP, EPI>(st, a);
-            return conv_dma_launch<16, 32, 1, 1, 4, 128, 6, NP, EPI>(st, a);
+        if constexpr (EPI == CONV_GLU) {      // (gate and up columns in one wave; 10 rows, 2048 x 512: 16 x 32 5.9, 16 x 64 6.4)
+            if (a.Cin % 256 == 0 && tiles(16, 32) <= 256) return conv_dma_launch<16, 32, 1, 1, 9, 256, 4, NP, EPI>(st, a);
+            if (tiles(16, 64) <= 256) return conv_dma_launch<16, 64, 1, 2, 5, 128, 5, NP, EPI>(st, a);
+        } else {
+            if (tiles(16, 32) <= 256) {
+                if (a.Cin % 256 == 0) return conv_dma_launch<16, 32, 1, 2, 5, 256, 3, NP, EPI>(st, a);
+                return conv_dma_launch<16, 32, 1, 2, 5, 128, 6, NP, EPI>(st, a);
+            }
+            if (tiles(16, 64) <= 256) return conv_dma_launch<16, 64, 1, 4, 2, 128, 3, NP, EPI>(st, a);
         }
-        if (tiles(16, 64) <= 256) return conv_dma_launch<16, 64, 1, 2, 4, 128, 5, NP, EPI>(st, a);
-        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 4, 128, NP == 3 ? 3 : 4, NP, EPI>(st, a);
-        if constexpr (NP != 3)
-            if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 2, 2, 4, 128, 3, NP, EPI>(st, a);
+        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 2, 2, 3, 128, 3, NP, EPI>(st, a);
     }
     if (k64) {
-        if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 1, 2, 2, 64, 6, NP, EPI>(st, a);
+        if (tiles(32, 64) <= 256) {
+            if constexpr (EPI == CONV_GLU) return conv_dma_launch<32, 64, 2, 2, 2, 64, 6, NP, EPI>(st, a);
+            else return conv_dma_launch<32, 64, 2, 4, 1, 64, 6, NP, EPI>(st, a);
+        }
+        if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 4, 2, 2, 64, 4, NP, EPI>(st, a);
         if constexpr (NP == 3) {
-            if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 2, 2, 2, 64, 4, NP, EPI>(st, a);
-            if (tiles(64, 128) <= 256) return conv_dma_launch<64, 128, 2, 4, 2, 64, 2, NP, EPI>(st, a);
+            if (tiles(64, 128) <= 256 || a.parts) return conv_dma_launch<64, 128, 2, 4, 2, 64, 2, NP, EPI>(st, a);
         } else if (tiles(64, 64) <= 512) {
             return conv_dma_launch<64, 64, 2, 2, 1, 64, 3, NP, EPI>(st, a);
         }
