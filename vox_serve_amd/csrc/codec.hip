@@ -304,7 +304,7 @@ __device__ __forceinline__ void ln_row_stats(const float* row, int C, int l16, f
 // 1536 x 7 x 1024 14.4 / 18.1 / 14.5, 6144 x 2 x 1536 14.7 / 16.9 / 13.1).
 // WP = 2: every tap has two weight planes (n_taps * N rows apart; fp32 weights as two terms) that share the tap's rows; WK waves share the
 // 32-channel slices of a step and add their sums through LDS at the end (hift_conv keeps one such order for all its tiles).
-// EPI: 0, CONV_GELU, or CONV_GLU: columns come in pairs (n, N + n) of w, out2 <- S2 of silu(v[n]) * v[N + n], N columns.
+// EPI: 0, CONV_GELU, CONV_GLU: columns come in pairs (n, N + n) of w, out2 <- S2 of silu(v[n]) * v[N + n], N columns; or CONV_CHUNKS.
 // The weights are the MFMA's first operand, so a lane ends with 4 (8) neighbouring channels of one row: the residual, the constants and both
 // outputs move in 16-byte accesses without a lane exchange.  With a lane per column the same epilogue cost more than the products of the
 // one-tap convs (us, rows x channels, residual + h + activation: 51 200 x 384 134 -> 67, 204 800 x 192 240 -> 175 = 3.6 TB/s).
@@ -458,6 +458,7 @@ __device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x
 }
 #define CONV_GELU 1
 #define CONV_GLU 2
+#define CONV_CHUNKS 3      // 0, with K in k_conv_unit's order: 32 channels at a time, all taps of them (a step of 64: two such slices)
 template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI, int WP = 1>
 __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8, KW = WP == 2 ? WK : 1;
@@ -488,12 +489,16 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         return BK == 32 ? (r >> 1) & 3 : r & 7;
     };
     // per DMA instruction of the wave: the lane's row of the chunk (its time), that row in x and the row that time 0 would have in the history
-    const char *xp[NA], *sp[NA], *cur[NA], *wp[NB];
+    const char *xp[NA], *sp[NA], *cur[NA], *wp[NB], *wbase[EPI == CONV_CHUNKS ? NB : 1];
     int ts[NA], step[NA];
+    bool half_a = false, half_b[EPI == CONV_CHUNKS ? NB : 1];      // (the lane's piece is of the step's second slice)
+    static_assert(EPI != CONV_CHUNKS || BK == 64, "two slices a step");
     if (loads) {
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
-            const int q = (i * NLD + lw) % CA * 64 + lane, pl = q / (BM * PPR), r = q / PPR % BM, pc = (q % PPR) ^ (BK == 32 ? (r >> 1) & 3 : r & 7);
+            const int q = (i * NLD + lw) % CA * 64 + lane, pl = q / (BM * PPR), r = q / PPR % BM, pc8 = (q % PPR) ^ (BK == 32 ? (r >> 1) & 3 : r & 7);
+            const int pc = EPI == CONV_CHUNKS ? pc8 & 3 : pc8;
+            if (EPI == CONV_CHUNKS) half_a = pc8 > 3;      // (the same for every i: whole rows of eight pieces apart)
             int m = m0 + r;
             m = m < a.M ? m : a.M - 1;                  // (rows past the end repeat the last one: nothing of them is stored)
             const int b = m / a.L;
@@ -503,7 +508,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
-            const int q = (i * NLD + lw) % CB * 64 + lane, r = q / PPR % BN, pl = q / (BN * PPR), pc = (q % PPR) ^ wswz(r);
+            const int q = (i * NLD + lw) % CB * 64 + lane, r = q / PPR % BN, pl = q / (BN * PPR), pc8 = (q % PPR) ^ wswz(r);
+            const int pc = EPI == CONV_CHUNKS ? pc8 & 3 : pc8;
             int n = n0 + r;
             if (EPI == CONV_GLU) {
                 n = (n0 >> 1) + (r >> 5) * 16 + (r & 15);
@@ -512,22 +518,43 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                 n = n < a.N ? n : a.N - 1;
             }
             wp[i] = reinterpret_cast<const char*>(a.w) + (((size_t)pl * a.n_taps * a.N + n) * a.Cin + pc * 8) * 2;
+            if constexpr (EPI == CONV_CHUNKS) {
+                wbase[i] = wp[i];
+                half_b[i] = pc8 > 3;
+            }
         }
     }
     const int nck = a.Cin / BK, nit = a.n_taps * nck;
     const size_t wtap = (size_t)(EPI == CONV_GLU ? 2 * a.N : a.N) * a.Cin * 2 - (size_t)a.Cin * 2;      // from the end of one tap's row to the next tap's
     const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)conv_lds;
+    auto row_of = [&](int i, int off) {
+        const int e = ts[i] - off;
+        const bool in = e >= 0 && e < a.L, hist = e < 0 && a.state && a.P + e >= 0;
+        cur[i] = in ? xp[i] - (ptrdiff_t)off * rb : hist ? sp[i] - (ptrdiff_t)off * rb : reinterpret_cast<const char*>(g_conv_zero_row);
+        step[i] = in || hist ? BK * 2 : 0;
+    };
     auto tap_rows = [&](int tap) {
         const int off = a.off[tap];
 #pragma unroll
-        for (int i = 0; i < NA; ++i) {
-            const int e = ts[i] - off;
-            const bool in = e >= 0 && e < a.L, hist = e < 0 && a.state && a.P + e >= 0;
-            cur[i] = in ? xp[i] - (ptrdiff_t)off * rb : hist ? sp[i] - (ptrdiff_t)off * rb : reinterpret_cast<const char*>(g_conv_zero_row);
-            step[i] = in || hist ? BK * 2 : 0;
-        }
+        for (int i = 0; i < NA; ++i) row_of(i, off);
     };
     int rt = 0, rc = 0, rq = 0;      // tap, chunk and number of the next request
+    int t0 = 0, c0 = 0, t1 = 1, c1 = 0;      // CONV_CHUNKS: tap and chunk of the step's two slices; a lane holds a piece of one of them
+    const int off0 = a.off[0], dil = EPI == CONV_CHUNKS ? off0 - a.off[1] : 0;
+    auto slices = [&]() {
+        const int o0 = off0 - t0 * dil, o1 = off0 - t1 * dil;
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            row_of(i, half_a ? o1 : o0);
+            cur[i] += step[i] ? (half_a ? c1 : c0) * 64 : 0;
+        }
+        const ptrdiff_t w0 = ((ptrdiff_t)t0 * a.N * a.Cin + c0 * 32) * 2, w1 = ((ptrdiff_t)t1 * a.N * a.Cin + c1 * 32) * 2;
+#pragma unroll
+        for (int i = 0; i < NB; ++i) wp[i] = wbase[i] + (half_b[i] ? w1 : w0);
+        t0 += 2; t1 += 2;
+        if (t0 >= a.n_taps) { t0 -= a.n_taps; ++c0; }
+        if (t1 >= a.n_taps) { t1 -= a.n_taps; ++c1; }
+    };
     auto request = [&](int stage) {
         const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * ST);
 #pragma unroll
@@ -535,6 +562,10 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
 #pragma unroll
         for (int i = 0; i < NB; ++i) lds_dma16(wp[i], ls + SA + (i * NLD + lw) % CB * 1024);
         if (++rq >= nit) return;     // (past the last step the same one is asked for again: the count in flight stays the same)
+        if (EPI == CONV_CHUNKS) {
+            slices();
+            return;
+        }
 #pragma unroll
         for (int i = 0; i < NA; ++i) cur[i] += step[i];
 #pragma unroll
@@ -547,7 +578,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         }
     };
     if (loads) {
-        tap_rows(0);
+        if (EPI == CONV_CHUNKS) slices();
+        else tap_rows(0);
 #pragma unroll
         for (int s = 0; s < S - 1; ++s) request(s);
     }
@@ -1892,6 +1924,15 @@ static ConvDmaArgs conv_s2_args(const vox_conv_w& w, const float* x, const float
     for (int k = 0; k < w.n_taps && k < CG_MAXTAPS; ++k) a.off[k] = offs ? offs[k] : 0;
     return a;
 }
+// The first conv of a 192-channel unit of few rows (conv_unit).  us beside the tap-major walk: 640 rows 10.5 / 9.7, 1 280 10.7 / 9.9, 2 560 12.2 / 10.1,
+// 5 120 15.8 / 11.8, 6 400 18.8 / 18.9 — a step's two slices are of two taps, so every lane has its addresses worked out anew each step.
+static int conv_dma_chunks(hipStream_t st, ConvDmaArgs& a) {
+    const auto tiles = [&](int bm, int bn) { return (long)((a.M + bm - 1) / bm) * ((a.N + bn - 1) / bn); };
+    if (tiles(16, 64) <= 256) return conv_dma_launch<16, 64, 1, 4, 2, 64, 6, 2, CONV_CHUNKS>(st, a);
+    if (tiles(32, 64) <= 256) return conv_dma_launch<32, 64, 2, 4, 2, 64, 6, 2, CONV_CHUNKS>(st, a);
+    if (tiles(64, 64) <= 256) return conv_dma_launch<64, 64, 4, 2, 2, 64, 4, 2, CONV_CHUNKS>(st, a);
+    return conv_dma_launch<64, 96, 4, 2, 2, 64, 3, 2, CONV_CHUNKS>(st, a);
+}
 static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
     if (a.Cin % CG_BK) return vox_fail(VOX_ERR_INVALID, "codec conv: Cin %d %% %d != 0", a.Cin, CG_BK);
     if (a.n_taps > CG_MAXTAPS) return vox_fail(VOX_ERR_INVALID, "codec conv: too many taps");
@@ -1902,13 +1943,14 @@ static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
         a.sn_mod = a.N;
         return a.planes == 2 ? conv_dma_pick<2, CONV_GLU>(st, a) : conv_dma_pick<1, CONV_GLU>(st, a);
     }
+    if (epi == CONV_CHUNKS) return conv_dma_chunks(st, a);
     if (epi == CONV_GELU)
         return a.planes == 3 ? conv_dma_pick<3, CONV_GELU>(st, a) : a.planes == 2 ? conv_dma_pick<2, CONV_GELU>(st, a) : conv_dma_pick<1, CONV_GELU>(st, a);
     return a.planes == 3 ? conv_dma_pick<3, 0>(st, a) : a.planes == 2 ? conv_dma_pick<2, 0>(st, a) : conv_dma_pick<1, 0>(st, a);
 }
 
-// A residual unit as ONE launch (k_conv_unit) where its tile can cover all channels and the rows fill the chip; *fused = 0 and nothing
-// launched otherwise (the caller then runs the two convs).  a1: conv1 with act2 (sn_*), a2: conv2 with res, out and the NEXT consumer's
+// A residual unit as ONE launch (k_conv_unit) where its tile can cover all channels and the rows fill the chip (*fused = 1); otherwise nothing
+// is launched and the caller runs the two convs, the first in k_conv_unit's order when *fused = CONV_CHUNKS.  a1: conv1 with act2 (sn_*), a2: conv2 with res, out and the NEXT consumer's
 // activation, whose rows must not be a1's: a neighbouring tile still reads its look-back there.  (a1.job is done by extra blocks.)
 template <int C, int CH, int TAPS, int T, int HP, int NW, int MT, int S>
 static int conv_unit_launch(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int H) {
@@ -1929,9 +1971,15 @@ static int conv_unit(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int* fuse
         return VOX_OK;
     int H = 0, omin = 0;
     for (int k = 0; k < a1.n_taps; ++k) { H = a1.off[k] > H ? a1.off[k] : H; omin = a1.off[k] < omin ? a1.off[k] : omin; }
-    // 96 channels: always (one request, 19 200 rows: 27 -> 18 us; 614 400 rows: 600 -> 309).  192 channels: from a tile per CU on (204 800
-    // rows: 424 -> 325; 6 400 rows, 100 tiles: 28 -> 30, there the two launches stay)
-    if (omin < 0 || H > 64 || a1.L % 64 || !a2.res || (C == 192 && a1.M / 64 < 256)) return VOX_OK;
+    for (int k = 2; k < a1.n_taps; ++k)
+        if (a1.off[k - 1] - a1.off[k] != a1.off[0] - a1.off[1]) return VOX_OK;
+    // 96 channels: always (one request, 19 200 rows: 27 -> 18 us; 614 400 rows: 600 -> 309).  192 channels: from 8192 rows on (12 800 rows two
+    // launches 48 us, one 32; 204 800: 412 and 327); below, two launches that add in the same order (6 400 rows 27 and 30, 1 280: 16 and 29)
+    if (omin < 0 || H > 64 || a1.L % 64 || !a2.res) return VOX_OK;
+    if (C == 192 && a1.M <= 8192) {
+        *fused = CONV_CHUNKS;
+        return VOX_OK;
+    }
     *fused = 1;
     if (C == 192) return conv_unit_launch<192, 192, 7, 2, 64, 4, 1, 3>(st, a1, a2, H);
     if (a1.L % 128 == 0 && a1.M / 128 >= 256) return conv_unit_launch<96, 96, 7, 2, 64, 8, 1, 3>(st, a1, a2, H);
@@ -2266,13 +2314,13 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
             int fused = 0;
             a1.job = job;
             VOX_TRY(conv_unit(st, a1, a2, &fused));
-            if (fused) {
+            if (fused == 1) {
                 later(m->st_ru[b][u], x, 6 * d, cout);
                 put(x);
                 x = y;
                 continue;
             }
-            VOX_TRY(run(a1));
+            VOX_TRY(run(a1, fused));
             later(m->st_ru[b][u], x, 6 * d, cout);
             float* z = take(nullptr);
             a2.out2 = z;
