@@ -93,3 +93,25 @@ def test_mimi_does_not_depend_on_its_batch(dev, n, T):  # noqa: F811
         ref = MR.MimiRef(cfg, W).decode(codes).numpy()
         assert rms(both.numpy() - ref) < 1e-5 * max(1.0, rms(ref))
     dec.close()
+
+
+def test_sine_behind_the_first_conv_is_exact_at_large_arguments(dev):  # noqa: F811
+    """The SnakeBeta between the decoder's first conv and its first transposed conv takes libm's accuracy: with alpha = e^9 a sine that
+    reduces its argument in fp32 is off by some 8000 * 2^-24 = 5e-4.  The conv's weights are zero, so what the sine reads is exact (its bias).
+    Bar: two-term operands through some 30 convs in sequence, sqrt(30) * 2^-17 = 4e-5 of the signal, times four."""
+    from vox_serve_amd.tokenizer.qwen3_codec import Qwen3CodecConfig, Qwen3TTSDecoder
+    cfg = cfg_of(64, 96, 32, 160, 2, 16, 512, [3, 2, 2, 2])
+    W = CR.random_codec_weights(cfg, seed=7)
+    g = torch.Generator().manual_seed(3)
+    W["decoder.0.conv.weight"].zero_()
+    W["decoder.0.conv.bias"] = 2 * torch.rand(cfg.decoder_dim, generator=g) - 1
+    W["decoder.1.block.0.alpha"].fill_(9.0)
+    codes = torch.randint(0, cfg.codebook_size, (2, cfg.num_quantizers, 4), generator=g)
+    ref = oracle_exact(cfg, W, codes, 2)
+    pc = Qwen3CodecConfig(**{k: getattr(cfg, k) for k in Qwen3CodecConfig.__dataclass_fields__})
+    dec = Qwen3TTSDecoder(W, pc, device=dev, max_batch=2, max_slots=2, detokenize_interval=2)
+    cache = dec.init_cache(2)
+    got = torch.cat([dec.decode_chunk(codes[:, :, t:t + 2], cache)[0].cpu().clone() for t in (0, 2)], -1).numpy()
+    off, size = rms(got - ref), rms(ref)
+    assert size > 1e-2 and off < 1.6e-4 * size
+    dec.close()

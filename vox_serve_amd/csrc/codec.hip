@@ -98,6 +98,24 @@ __device__ __forceinline__ float snake_f(float v, float alpha, float invb) {
     return v + invb * (s_ * s_);
 }
 
+// The same with the sine right to fp32, for one conv's epilogue (no room for libm's table there): revolutions, the nearest half turn and its
+// Taylor series in fp64, remainder below (pi / 2)^17 / 17! = 6e-12.
+__device__ __forceinline__ float snake_exact(float v, float alpha, float invb) {
+    const double r = (double)(v * alpha) * 0.15915494309189533577;
+    double q = r - rint(r);
+    if (fabs(q) > 0.25) q = copysign(0.5, q) - q;
+    const double t = q * 6.28318530717958647693, t2 = t * t;
+    double s = -1.0 / 1307674368000.0;
+    s = fma(s, t2, 1.0 / 6227020800.0);
+    s = fma(s, t2, -1.0 / 39916800.0);
+    s = fma(s, t2, 1.0 / 362880.0);
+    s = fma(s, t2, -1.0 / 5040.0);
+    s = fma(s, t2, 1.0 / 120.0);
+    s = fma(s, t2, -1.0 / 6.0);
+    const float s_ = (float)fma(t * t2, s, t);
+    return v + invb * (s_ * s_);
+}
+
 // Epilogue of the tiled conv GEMMs (2 x 2 waves, WM x WN 16x16 tiles per wave)
 template <int WM, int WN>
 __device__ __forceinline__ void conv_epilogue(const ConvGemmArgs& a, f32x4 (&acc)[WM][WN], int m0, int n0, int wm, int wn, int lane) {
@@ -384,9 +402,13 @@ __device__ __forceinline__ void conv_put_terms(bf16_t* row, int width, int c, co
         else *reinterpret_cast<uint2*>(row + (size_t)t * width + c) = make_uint2(h[0], h[1]);
     }
 }
+#define CONV_GELU 1
+#define CONV_GLU 2
+#define CONV_CHUNKS 3      // 0, with K in k_conv_unit's order: 32 channels at a time, all taps of them (a step of 64: two such slices)
+#define CONV_SINE 4        // 0, with snake_exact for SnakeBeta
 // The epilogue of W neighbouring channels (n ..) of MT rows (m, m + 16, ..) that one lane holds: constants once, every row's residual
 // requested ahead of the first store, 16-byte accesses throughout.
-template <int T, bool GELU, int W, int MT>
+template <int T, int EPI, int W, int MT>
 __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n,
                                              const f32x4* res_ready = nullptr) {
     if (n >= a.N) return;          // (N and the group width are multiples of W)
@@ -424,7 +446,7 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
             v[e] = acc[i][e / 4][e % 4];
             if (rms) v[e] *= rr;
             if (a.bias) v[e] += b[e];
-            if (GELU) v[e] = 0.5f * v[e] * (1.0f + erff(v[e] * 0.70710678118654752440f));
+            if (EPI == CONV_GELU) v[e] = 0.5f * v[e] * (1.0f + erff(v[e] * 0.70710678118654752440f));
             if (a.scale) v[e] = s[e] * v[e];
             if (a.res) v[e] = rs[i][e] + v[e];
         }
@@ -434,7 +456,7 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
         if (!a.out2) continue;
 #pragma unroll
         for (int e = 0; e < W; ++e) {
-            if (a.sn_alpha) v[e] = snake_f(v[e], al[e], ib[e]);
+            if (a.sn_alpha) v[e] = EPI == CONV_SINE ? snake_exact(v[e], al[e], ib[e]) : snake_f(v[e], al[e], ib[e]);
             else if (a.elu) v[e] = v[e] > 0.0f ? v[e] : expm1f(v[e]);
             else if (a.nw) v[e] *= nw[e];
         }
@@ -456,9 +478,6 @@ __device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x
     }
     conv_put_terms<2>(reinterpret_cast<bf16_t*>(a.out2) + (size_t)m * a.N * 2, a.N, n, v);
 }
-#define CONV_GELU 1
-#define CONV_GLU 2
-#define CONV_CHUNKS 3      // 0, with K in k_conv_unit's order: 32 channels at a time, all taps of them (a step of 64: two such slices)
 template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI, int WP = 1>
 __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8, KW = WP == 2 ? WK : 1;
@@ -700,7 +719,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
                     for (int q = 0; q < P; ++q) v[i][q] = acc[i][j + q];
-                conv_dma_out<NP == 3 ? 3 : 2, EPI == CONV_GELU, 4 * P, MT>(a, v, rms, m0 + rl, n);
+                conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, MT>(a, v, rms, m0 + rl, n);
             } else {
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
@@ -708,7 +727,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                         f32x4 v[1][P];
 #pragma unroll
                         for (int q = 0; q < P; ++q) v[0][q] = sum(i * NT + j + q);
-                        conv_dma_out<NP == 3 ? 3 : 2, EPI == CONV_GELU, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
+                        conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
                     }
             }
         }
@@ -914,7 +933,7 @@ __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_co
         f32x4 v[MT][2];
 #pragma unroll
         for (int i = 0; i < MT; ++i) { v[i][0] = out[i][2 * p]; v[i][1] = out[i][2 * p + 1]; }
-        conv_dma_out<T, false, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
+        conv_dma_out<T, 0, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
     }
 }
 
@@ -1944,6 +1963,7 @@ static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
         return a.planes == 2 ? conv_dma_pick<2, CONV_GLU>(st, a) : conv_dma_pick<1, CONV_GLU>(st, a);
     }
     if (epi == CONV_CHUNKS) return conv_dma_chunks(st, a);
+    if (epi == CONV_SINE) return a.planes == 2 ? conv_dma_pick<2, CONV_SINE>(st, a) : conv_dma_pick<1, CONV_SINE>(st, a);
     if (epi == CONV_GELU)
         return a.planes == 3 ? conv_dma_pick<3, CONV_GELU>(st, a) : a.planes == 2 ? conv_dma_pick<2, CONV_GELU>(st, a) : conv_dma_pick<1, CONV_GELU>(st, a);
     return a.planes == 3 ? conv_dma_pick<3, 0>(st, a) : a.planes == 2 ? conv_dma_pick<2, 0>(st, a) : conv_dma_pick<1, 0>(st, a);
@@ -2219,7 +2239,8 @@ static int codec_chunk_f32(vox_codec* m, hipStream_t st, const int32_t* codes, i
 }
 
 // One chunk with S2 activations (planes 1 and 2): every tensor that only convs read is written as S2 rows by whatever produces it, and what
-// stood between two convs (RMSNorm, SiLU, SnakeBeta) is in the epilogue of the first: 86 launches of 134.  RMSNorm: the producer writes h * w
+// stood between two convs (RMSNorm, SiLU, SnakeBeta) is in the epilogue of the first: 86 launches of 134.  The SnakeBeta behind dec0 is the one
+// that planes == 3 takes on its own (libm's sine): snake_exact.  RMSNorm: the producer writes h * w
 // beside h, the consumer scales its sums by the rows' 1 / rms.
 static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, int code_stride, const int32_t* slots, int n, int T, float* out) {
     const vox_codec_config& c = m->cfg;
@@ -2274,7 +2295,7 @@ static int codec_chunk_s2(vox_codec* m, hipStream_t st, const int32_t* codes, in
     }
     // ---- decoder.  SnakeBeta is in the epilogue of the conv that produces its input; h stays fp32 and is written only where a residual
     // branch reads it.  free: the two buffers that hold neither h nor x (job.x may still be one of them). ----
-    { ConvDmaArgs a = conv(w.dec0, A, m->st_dec0, 6, off7); act_out(a, C, w.blocks[0].snake0, c.decoder_dim); VOX_TRY(run(a)); }
+    { ConvDmaArgs a = conv(w.dec0, A, m->st_dec0, 6, off7); act_out(a, C, w.blocks[0].snake0, c.decoder_dim); VOX_TRY(run(a, CONV_SINE)); }
     later(m->st_dec0, A, 6, LD);
     float *h = B, *x = C, *free_[2] = {A, D};
     auto take = [&](float* avoid) {          // a free buffer other than `avoid`; its place is left empty (NULL)
