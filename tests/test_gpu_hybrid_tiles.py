@@ -65,7 +65,7 @@ def test_activation_behind_both_products(rows, mlp):
 
 
 # K of the second product = the layer's inner width: one step into the second round of requests, two whole rounds, one step into the third,
-# three whole rounds and one step into a fourth (taken in turn)
+# three whole rounds and one step into a fourth; both forms of the kernel (up to eight rows and more)
 @pytest.mark.parametrize("rows,inner", [(2, 2080), (16, 4096), (7, 4128), (8, 6144), (16, 6176)])
 def test_rounds_of_a_few_row_product(rows, inner):
     cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.dense(inner))], width=64, vocab=50)

@@ -1142,10 +1142,10 @@ static void hb_settle(hipStream_t st, hb_pending& pd, int n, int W) {
 // 2..16 rows, bf16: one MFMA row tile; a block owns 16 output columns and its eight waves take the 32-wide k-steps w, w + 8, ...
 // with both fragments straight from memory (the weight fragment is one 16-byte request per lane, the activation fragment two,
 // converted to bf16 in registers); the eight partial tiles are added in wave order.  Needs K % 32 == 0.
-// A wave asks for eight of its steps at once.  NIT = 2, 3: K has that many such rounds and the next round's requests go out before this
-// one's products (two register sets, straight-line code: a conditional request would make every wait a full one); one after the other each
-// round waited out the trip to memory (8 rows, 2048 x 5632: 17.1 us, now 14.9).  NIT = 0: any number of rounds, in turn.
-template <int EPI, int NIT>
+// A wave asks for eight of its steps at once.  Rows and steps past the end are zeroed where they are multiplied (LATE) or where they arrive: the
+// rule is hb_rows16_late's.  Asking for the next eight before these are multiplied (two register sets) gained nothing over LATE where K is
+// 4096 or 6144, left one block per CU (8 rows, 16384 x 4096 36.4 us, so 40.6) and did whole rounds for a single step (16384 x 2080 20.8, 33.5).
+template <int EPI, bool LATE>
 __global__ __launch_bounds__(512) void k_hb_gemm_rows16(const float* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
                                                         int N, int K, hb_rowmap rm) {
     __shared__ float red[8][16][17];
@@ -1166,41 +1166,28 @@ __global__ __launch_bounds__(512) void k_hb_gemm_rows16(const float* A, long lda
     hb_join_in jin;
     if (EPI == HB_EPI_JOIN && mine) jin = hb_join_load(rm.join, C + (size_t)orow * ldc, orow, n0 + ocol);
     constexpr int U = 8;
-    uint4 wf[NIT ? 2 : 1][U];
-    float4 a0[NIT ? 2 : 1][U], a1[NIT ? 2 : 1][U];
-    auto fetch = [&](int set, int s0) {
+    for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
+        uint4 wf[U];
+        float4 a0[U], a1[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int sidx = s0 + 8 * u, k = (sidx < nsteps ? sidx : wv < nsteps ? wv : 0) << 5;
-            wf[set][u] = *(const uint4*)(wrow + k);
-            a0[set][u] = *(const float4*)(arow + k);
-            a1[set][u] = *(const float4*)(arow + k + 4);
+            const int sidx = s0 + 8 * u;
+            const bool valid = sidx < nsteps;
+            const int k = (valid ? sidx : LATE ? wv : s0) << 5;
+            wf[u] = *(const uint4*)(wrow + k);
+            a0[u] = *(const float4*)(arow + k);
+            a1[u] = *(const float4*)(arow + k + 4);
+            if (!LATE && (!valid || !rowok)) { a0[u] = make_float4(0.f, 0.f, 0.f, 0.f); a1[u] = a0[u]; }
         }
-    };
-    auto multiply = [&](int set, int s0) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             union { uint4 q; hb_bf16x8 b; } af, bfv;
-            const bool ok = s0 + 8 * u < nsteps && rowok;
-            float4 x0 = a0[set][u], x1 = a1[set][u];
-            if (!ok) { x0 = make_float4(0.f, 0.f, 0.f, 0.f); x1 = x0; }
+            float4 x0 = a0[u], x1 = a1[u];
+            if (LATE && !(s0 + 8 * u < nsteps && rowok)) { x0 = make_float4(0.f, 0.f, 0.f, 0.f); x1 = x0; }
             af.q.x = pack_bf2(x0.x, x0.y); af.q.y = pack_bf2(x0.z, x0.w);
             af.q.z = pack_bf2(x1.x, x1.y); af.q.w = pack_bf2(x1.z, x1.w);
-            bfv.q = wf[set][u];
+            bfv.q = wf[u];
             acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af.b, bfv.b, acc, 0, 0, 0);
-        }
-    };
-    if constexpr (NIT > 0) {
-        fetch(0, wv);
-#pragma unroll
-        for (int i = 0; i < NIT; ++i) {
-            if (i + 1 < NIT) fetch((i + 1) & 1, wv + 8 * U * (i + 1));
-            multiply(i & 1, wv + 8 * U * i);
-        }
-    } else {
-        for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
-            fetch(0, s0);
-            multiply(0, s0);
         }
     }
 #pragma unroll
@@ -1218,15 +1205,18 @@ __global__ __launch_bounds__(512) void k_hb_gemm_rows16(const float* A, long lda
 static inline bool hb_batch_aligned(const hb_rowmap& rm, int nz, size_t wsize) {
     return nz == 1 || ((rm.w_stride * wsize) % 16 == 0 && (rm.a_stride * 4) % 16 == 0);
 }
+// Up to eight rows: late zeroing while the blocks are one to a CU and K fills a round of requests (us, early and late: 8 rows, 2048 x 2048 7.1, 6.6;
+// 2048 x 5632 16.5, 15.0; 2048 x 11264 32.0, 27.6; 2 rows, 4096 x 2048 7.3, 6.2), and in one round of many blocks (8 rows, 11264 x 2048
+// 16.6, 15.1; 32000 x 2048 39.1, 36.2).  Early elsewhere: several rounds of many blocks (6144 x 5632 26.1, 27.8; 8192 x 4096 18.5, 20.1),
+// 257 to 511 blocks (6144 x 2048 10.5, 10.9), short K (4096 x 512 6.2, 6.6), more rows (16 rows, 2048 x 2048 7.6, 7.9).
+static bool hb_rows16_late(int M, unsigned blocks, int K) { return M <= 8 && (blocks <= 256 ? K >= 2048 : blocks >= 512 && K <= 2048); }
 template <int EPI>
 bool hb_try_rows16(hipStream_t st, const float* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
                    const hb_rowmap& rm, int nz) {
     if (M < 2 || M > 16 || (K & 31) || (lda & 3) || ((size_t)A & 15) || ((size_t)W & 15) || !hb_batch_aligned(rm, nz, 2)) return false;
-    const int nit = ((K >> 5) + 63) / 64;
     const dim3 grid((N + 15) / 16, nz), block(512);
-    if (nit == 2) hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, 2>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
-    else if (nit == 3) hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, 3>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
-    else hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, 0>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
+    if (hb_rows16_late(M, grid.x * nz, K)) hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, true>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
+    else hipLaunchKernelGGL((k_hb_gemm_rows16<EPI, false>), grid, block, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm);
     return true;
 }
 template <int EPI>
