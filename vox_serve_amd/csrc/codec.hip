@@ -4192,12 +4192,16 @@ __global__ void k_flow_slots(int* slots, int N, int B) {
 // activation rows): a lane then holds four neighbouring columns of one row, which is what it stores, normalises and splits.
 //   k_tb_qkv   rows = residual + feed-forward parts of the block before, LayerNorm, q | k | v: grid (row tiles, 256-column groups)
 //   k_tb_ff    attention out + residual, LayerNorm, GELU feed-forward: grid (row tiles, 4); block y owns a quarter of the hidden columns from
-//              ff1 to its part of ff2 (parts [4] + the residual rows are added by whoever reads them, in a fixed order); the out product is
-//              done by all four
+//              ff1 to its two eighths of ff2's sums (they and the residual rows are added by whoever reads them); the out product is done by
+//              all four
+// Sums, LayerNorm statistics and the order of every addition are those of the general launches (k_rows_gemm: K in four runs of 64, or in eight
+// from 512 on, added in ascending order), so the two forms give the same bits: the phase of the vocoder's source multiplies what a mel
+// differs by some hundred times.
 // What one of these leaves for another (parts, the residual rows) lies in the order of the lanes, [row tile][wave][tile][lane] x 4 floats:
 // whole lines per request (as [row][256] every request touched 16 lines: k_tb_qkv 12.8 us against 8.3 with plain rows to read).
-// Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 8.2 /
-// 10.3 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 12.7; a window of 8 requests 45.9 -> 31.6 ms.  A row's result depends on that row only.
+// Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 8.3 /
+// 10.7 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 13.2 (with each product as one sum, four parts and other LayerNorm
+// sums: 8.3 / 10.3 and 12.7).  A row's result depends on that row only.
 #define TB_C 256
 #define TB_IN 512
 #define TB_FF 1024
@@ -4232,46 +4236,69 @@ __device__ __forceinline__ void tb_put(uint4* pl, int kb_n, int wave, int t, int
 #pragma unroll
     for (int p = 0; p < 3; ++p) d[p * kb_n * 128] = s.t[p];
 }
-// LayerNorm of the rows whose columns lie 8 to a lane (two tiles of four) over the block's eight waves; red: [2][8][16]
-__device__ __forceinline__ void tb_layernorm(float4 (&v)[2], const float4 (&w)[2], const float4 (&b)[2], float* red, int wave, int lane) {
+// A row's sum over its 256 columns from the sums s[t] of four neighbouring ones (two per lane): eight neighbouring columns, then the two
+// 32-column blocks of a run of 64, then its four groups of eight, then the runs.  red: [8][16] x 4 floats, one for each call of a block
+__device__ __forceinline__ float tb_row_sum(float s0, float s1, float4* red, int wave, int lane) {
     const int fr = lane & 15;
-    float s = ((v[0].x + v[0].y) + (v[0].z + v[0].w)) + ((v[1].x + v[1].y) + (v[1].z + v[1].w));
-    s += __shfl_xor(s, 16, 64); s += __shfl_xor(s, 32, 64);
-    if (lane < 16) red[wave * 16 + fr] = s;
+    s0 += __shfl_xor(s0, 16, 64);
+    s1 += __shfl_xor(s1, 16, 64);
+    if (!(lane & 16)) {
+        float* d = reinterpret_cast<float*>(red + wave * 16 + fr) + (lane >> 5);
+        d[0] = s0;
+        d[2] = s1;
+    }
     __syncthreads();
-    float tot = red[fr];
+    float tot = 0.0f;
 #pragma unroll
-    for (int i = 1; i < 8; ++i) tot += red[i * 16 + fr];
-    const float mean = tot / (float)TB_C;
-    float q = 0.0f;
+    for (int i = 0; i < 4; ++i) {
+        const float4 a = red[2 * i * 16 + fr], b = red[(2 * i + 1) * 16 + fr];
+        const float run = ((a.x + b.x) + (a.y + b.y)) + ((a.z + b.z) + (a.w + b.w));
+        tot = i == 0 ? run : tot + run;
+    }
+    return tot;
+}
+// LayerNorm of the rows whose columns lie 8 to a lane (two tiles of four) over the block's eight waves; red: [2][8][16] x 4 floats
+__device__ __forceinline__ void tb_layernorm(float4 (&v)[2], const float4 (&w)[2], const float4 (&b)[2], float4* red, int wave, int lane) {
+    const float mean = tb_row_sum((v[0].x + v[0].y) + (v[0].z + v[0].w), (v[1].x + v[1].y) + (v[1].z + v[1].w), red, wave, lane) / (float)TB_C;
+    float q[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         v[t] = make_float4(v[t].x - mean, v[t].y - mean, v[t].z - mean, v[t].w - mean);
-        q += (v[t].x * v[t].x + v[t].y * v[t].y) + (v[t].z * v[t].z + v[t].w * v[t].w);
+        q[t] = (v[t].x * v[t].x + v[t].y * v[t].y) + (v[t].z * v[t].z + v[t].w * v[t].w);
     }
-    q += __shfl_xor(q, 16, 64); q += __shfl_xor(q, 32, 64);
-    if (lane < 16) red[128 + wave * 16 + fr] = q;
-    __syncthreads();
-    float var = red[128 + fr];
-#pragma unroll
-    for (int i = 1; i < 8; ++i) var += red[128 + i * 16 + fr];
+    const float var = tb_row_sum(q[0], q[1], red + 128, wave, lane);
     const float rstd = rsqrtf(var / (float)TB_C + 1e-5f);
 #pragma unroll
     for (int t = 0; t < 2; ++t)
         v[t] = make_float4(v[t].x * rstd * w[t].x + b[t].x, v[t].y * rstd * w[t].y + b[t].y, v[t].z * rstd * w[t].z + b[t].z, v[t].w * rstd * w[t].w + b[t].w);
 }
-// two column tiles against the rows in pl (KB k-blocks, three terms, low terms first)
+// two column tiles against the rows in pl (KB k-blocks, three terms, low terms first) as the sums of runs of RUN k-blocks
+template <int KB, int RUN>
+__device__ __forceinline__ void tb_runs(const uint4 (&wf)[2][KB], const uint4* pl, int lane, f32x4 (&acc)[KB / RUN][2]) {
+#pragma unroll
+    for (int i = 0; i < KB / RUN; ++i) {
+        acc[i][0] = acc[i][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = i * RUN; kb < (i + 1) * RUN; ++kb)
+#pragma unroll
+            for (int p = 2; p >= 0; --p) {
+                const uint4 x = pl[(p * KB + kb) * 64 + lane];
+#pragma unroll
+                for (int t = 0; t < 2; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[i][t], 0, 0, 0);
+            }
+    }
+}
+// the whole product: runs of two k-blocks, added in ascending order
 template <int KB>
 __device__ __forceinline__ void tb_product(const uint4 (&wf)[2][KB], const uint4* pl, int lane, f32x4 (&acc)[2]) {
-    acc[0] = acc[1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    f32x4 r[KB / 2][2];
+    tb_runs<KB, 2>(wf, pl, lane, r);
 #pragma unroll
-    for (int kb = 0; kb < KB; ++kb)
+    for (int t = 0; t < 2; ++t) {
+        acc[t] = r[0][t];
 #pragma unroll
-        for (int p = 2; p >= 0; --p) {
-            const uint4 x = pl[(p * KB + kb) * 64 + lane];
-#pragma unroll
-            for (int t = 0; t < 2; ++t) acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[t], 0, 0, 0);
-        }
+        for (int i = 1; i < KB / 2; ++i) acc[t] += r[i][t];
+    }
 }
 template <int KB>
 __device__ __forceinline__ void tb_weights(uint4 (&wf)[2][KB], const bf16_t* w, int tile, int kb_all, int kb0, int lane) {
@@ -4282,18 +4309,24 @@ __device__ __forceinline__ void tb_weights(uint4 (&wf)[2][KB], const bf16_t* w, 
 }
 // floats of column tile 2 wave + t of row tile `rt` in lane order
 __device__ __forceinline__ size_t tb_at(int rt, int wave, int t, int lane) { return ((((size_t)rt * 8 + wave) * 2 + t) * 64 + lane) * 4; }
-// rows [.][256] = parts[4] + (((parts[0] + parts[1]) + parts[2]) + parts[3]), ps floats apart
-__device__ __forceinline__ float4 tb_sum(const float* p, size_t ps) {
-    float4 v[5];
+// Planes of a block's scratch, ps floats apart: ff2's sums (the first two eighths, then an eighth each), the residual rows behind the out product,
+// and those in front of it (the sum of the planes that the block before has left)
+#define TB_PARTS 7
+#define TB_PLANES 9
+// rows [.][256] = residual + ((parts[0] + ... + parts[6]) + b2)
+__device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
+    float4 v[TB_PARTS + 1];
 #pragma unroll
-    for (int i = 0; i < 5; ++i) v[i] = *reinterpret_cast<const float4*>(p + i * ps);
-    return tb_add(v[4], tb_add(tb_add(tb_add(v[0], v[1]), v[2]), v[3]));
+    for (int i = 0; i <= TB_PARTS; ++i) v[i] = *reinterpret_cast<const float4*>(p + i * ps);
+#pragma unroll
+    for (int i = 1; i < TB_PARTS; ++i) v[0] = tb_add(v[0], v[i]);
+    return tb_add(v[TB_PARTS], tb_add(v[0], b2));
 }
 template <bool PARTS>
-__global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* parts, size_t ps, const bf16_t* w, const float* lnw, const float* lnb,
+__global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* parts, const float* b2, size_t ps, const bf16_t* w, const float* lnw, const float* lnb,
                                                 float* qkv, float* h_out, int M, int N) {
     __shared__ uint4 pl[3 * 8 * 64];
-    __shared__ float red[256];
+    __shared__ float4 red[256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4;
     const int m = blockIdx.x * 16 + fr, row = m < M ? m : M - 1, tile = (blockIdx.y * 8 + wave) * 2;
     float4 v[2], lw[2], lb[2];
@@ -4301,7 +4334,8 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int c = (wave * 2 + t) * 16 + kq * 4;
-        v[t] = PARTS ? tb_sum(parts + tb_at(blockIdx.x, wave, t, lane), ps) : *reinterpret_cast<const float4*>(h + (size_t)row * TB_C + c);
+        v[t] = PARTS ? tb_sum(parts + tb_at(blockIdx.x, wave, t, lane), ps, *reinterpret_cast<const float4*>(b2 + c))
+                     : *reinterpret_cast<const float4*>(h + (size_t)row * TB_C + c);
         lw[t] = *reinterpret_cast<const float4*>(lnw + c);
         lb[t] = *reinterpret_cast<const float4*>(lnb + c);
     }
@@ -4322,12 +4356,12 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
 }
 // lane_h: h lies in lane order
 __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h, int lane_h, FlowPacked w, const float* b_out, const float* lnw, const float* lnb,
-                                               const float* b1, const float* b2, float* parts, size_t ps, int M) {
+                                               const float* b1, float* parts, size_t ps, int M) {
     __shared__ uint4 pl[3 * 16 * 64];
-    __shared__ float red[256];
+    __shared__ float4 red[256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4, q = blockIdx.y;
     const int m0 = blockIdx.x * 16, m = m0 + fr, row = m < M ? m : M - 1;
-    float4 a[2][2], res[2], bo[2], lw[2], lb[2], bh[2], by[2];
+    float4 a[2][2], res[2], bo[2], lw[2], lb[2], bh[2];
 #pragma unroll
     for (int i = 0; i < 2; ++i) {      // the attention rows: thread = (row, 8 columns)
         const float* s = att + (size_t)(m0 + (tid & 15) < M ? m0 + (tid & 15) : M - 1) * TB_IN + ((tid >> 4) + 32 * i) * 8;
@@ -4344,7 +4378,6 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
         lw[t] = *reinterpret_cast<const float4*>(lnw + c);
         lb[t] = *reinterpret_cast<const float4*>(lnb + c);
         bh[t] = *reinterpret_cast<const float4*>(b1 + q * 256 + c);
-        by[t] = *reinterpret_cast<const float4*>(b2 + c);
     }
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
@@ -4380,21 +4413,23 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
         tb_put(hid, 8, wave, t, lane, make_float4(g[0], g[1], g[2], g[3]));
     }
     __syncthreads();
-    tb_product<8>(w2, hid, lane, acc);
+    f32x4 y[2][2];
+    tb_runs<8, 4>(w2, hid, lane, y);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        float4 y = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
         const size_t o = tb_at(blockIdx.x, wave, t, lane);
         if (q == 0) {
-            y = tb_add(y, by[t]);
-            *reinterpret_cast<float4*>(parts + 4 * ps + o) = x[t];
+            y[1][t] = y[0][t] + y[1][t];
+            *reinterpret_cast<float4*>(parts + TB_PARTS * ps + o) = x[t];
+        } else {
+            *reinterpret_cast<f32x4*>(parts + (size_t)(2 * q - 1) * ps + o) = y[0][t];
         }
-        *reinterpret_cast<float4*>(parts + (size_t)q * ps + o) = y;
+        *reinterpret_cast<f32x4*>(parts + (size_t)(2 * q) * ps + o) = y[1][t];
     }
 }
-__global__ __launch_bounds__(256) void k_tb_join(const float* parts, size_t ps, float* h, int M) {
+__global__ __launch_bounds__(256) void k_tb_join(const float* parts, const float* b2, size_t ps, float* h, int M) {
     const int i = blockIdx.x * 256 + threadIdx.x, lane = i & 63, col = (i >> 6 & 15) * 16 + (lane >> 4) * 4, m = (i >> 10) * 16 + (lane & 15);
-    if (m < M) *reinterpret_cast<float4*>(h + (size_t)m * TB_C + col) = tb_sum(parts + (size_t)i * 4, ps);
+    if (m < M) *reinterpret_cast<float4*>(h + (size_t)m * TB_C + col) = tb_sum(parts + (size_t)i * 4, ps, *reinterpret_cast<const float4*>(b2 + col));
 }
 // fragment-major copies of every transformer block's weights, or an empty list where a block has other sizes (then the general launches run)
 static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, std::vector<FlowPacked>& out, void** mem) {
@@ -4424,20 +4459,19 @@ static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, 
     }
     return hipGetLastError() == hipSuccess;
 }
-// floats of scratch for M rows: four parts, the residual rows of the block before and of this one
-static size_t tb_room(int M) { return (size_t)((M + 15) / 16) * 16 * TB_C * 6; }
-// q | k | v of the rows into qkv (first: of h itself; else of what the block before has left in ws)
-static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* h, float* ws, bool first, float* qkv, int M) {
+static size_t tb_plane(size_t M) { return (M + 15) / 16 * 16 * TB_C; }      // floats of a plane of M rows
+// q | k | v of the rows into qkv (before: the block before, which has left them in ws; NULL: of h itself)
+static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* h, float* ws, const vox_flow_tblock_w* before, float* qkv, int M) {
     const dim3 g((M + 15) / 16, 3 * TB_IN / 256);
-    const size_t ps = tb_room(M) / 6;
-    if (first) hipLaunchKernelGGL(k_tb_qkv<false>, g, dim3(512), 0, st, h, ws, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN);
-    else hipLaunchKernelGGL(k_tb_qkv<true>, g, dim3(512), 0, st, h, ws, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws + 5 * ps, M, 3 * TB_IN);
+    const size_t ps = tb_plane(M);
+    if (!before) hipLaunchKernelGGL(k_tb_qkv<false>, g, dim3(512), 0, st, h, ws, nullptr, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN);
+    else hipLaunchKernelGGL(k_tb_qkv<true>, g, dim3(512), 0, st, h, ws, before->ff2.bias, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws + (TB_PLANES - 1) * ps, M, 3 * TB_IN);
 }
 static void tb_ff(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* att, float* h, float* ws, bool first, bool last, int M) {
-    const size_t ps = tb_room(M) / 6;
-    hipLaunchKernelGGL(k_tb_ff, dim3((M + 15) / 16, 4), dim3(512), 0, st, att, first ? h : ws + 5 * ps, first ? 0 : 1, f, w.out.bias, w.ln3_w, w.ln3_b,
-                       w.ff1.bias, w.ff2.bias, ws, ps, M);
-    if (last) hipLaunchKernelGGL(k_tb_join, dim3((unsigned)((M + 15) / 16 * 4)), dim3(256), 0, st, ws, ps, h, M);
+    const size_t ps = tb_plane(M);
+    hipLaunchKernelGGL(k_tb_ff, dim3((M + 15) / 16, 4), dim3(512), 0, st, att, first ? h : ws + (TB_PLANES - 1) * ps, first ? 0 : 1, f, w.out.bias, w.ln3_w,
+                       w.ln3_b, w.ff1.bias, ws, ps, M);
+    if (last) hipLaunchKernelGGL(k_tb_join, dim3((unsigned)((M + 15) / 16 * 4)), dim3(256), 0, st, ws, w.ff2.bias, ps, h, M);
 }
 
 struct vox_flow {
@@ -4449,6 +4483,7 @@ struct vox_flow {
     std::vector<vox_flow_tblock_w> tblocks;
     std::vector<FlowPacked> packed;         // per transformer block, or empty
     void* packed_mem = nullptr;
+    float* tb_ws = nullptr;                 // their scratch: TB_PLANES planes of the most rows
     int max_batch, max_T, max_prompt_T, n_res, n_att;
     std::vector<float> dt;                  // host: Euler step sizes
     float* tb = nullptr;                    // [n_steps][n_res][C]: mlp_r(Mish(time_mlp(emb_s)))
@@ -4485,7 +4520,7 @@ void vox_flow_destroy(vox_flow* m) {
     (void)hipFree(m->s_enc); (void)hipFree(m->s_up); (void)hipFree(m->s_att); (void)hipFree(m->s_cnn1); (void)hipFree(m->s_cnn2);
     (void)hipFree(m->s_eidx); (void)hipFree(m->s_cidx);
     for (void* p : m->conv1x_mem) (void)hipFree(p);
-    (void)hipFree(m->packed_mem);
+    (void)hipFree(m->packed_mem); (void)hipFree(m->tb_ws);
     delete m;
 }
 
@@ -4642,8 +4677,8 @@ static int flow_run(vox_flow* m, hipStream_t st, const int32_t* tokens, int B, i
             for (int j = 0; j < c.est_blocks; ++j, ++li) {
                 const vox_flow_tblock_w& tw = m->tblocks[li];
                 float* kv = (evolve ? m->s_att : m->att_kv) + ((size_t)s * m->n_att + li) * att_layer;
-                const FlowPacked* pk = m->packed.empty() || tb_room(N * T2) > m->buf_floats ? nullptr : &m->packed[li];
-                if (pk) tb_qkv(st, *pk, tw, h, a1, j == 0, a2, N * T2);
+                const FlowPacked* pk = m->packed.empty() ? nullptr : &m->packed[li];
+                if (pk) tb_qkv(st, *pk, tw, h, m->tb_ws, j ? &m->tblocks[li - 1] : nullptr, a2, N * T2);
                 else VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, T2, a2, 0));
                 FlowAttn a{a2, init ? nullptr : kv, nullptr, nullptr, nullptr, a3, T2, HE, hd, Tc, capA, B, att_half, 1.0f / sqrtf((float)hd)};
                 if (evolve) { a.cidx = m->s_cidx; a.prefix = c.prefix; a.ring_head = evolve->att_head; }
@@ -4654,7 +4689,7 @@ static int flow_run(vox_flow* m, hipStream_t st, const int32_t* tokens, int B, i
                 if (init)
                     hipLaunchKernelGGL(k_flow_cache_store, dim3(ew_grid((size_t)N * HE * capA * 2 * hd)), dim3(256), 0, st, a2, kv, T2, HE, hd, capA,
                                        c.prefix, att_half, N);
-                if (pk) { tb_ff(st, *pk, tw, a3, h, a1, j == 0, j + 1 == c.est_blocks, N * T2); continue; }
+                if (pk) { tb_ff(st, *pk, tw, a3, h, m->tb_ws, j == 0, j + 1 == c.est_blocks, N * T2); continue; }
                 VOX_TRY(conv_gemm(st, tw.out, a3, nullptr, nullptr, N, T2, 0, FLOW_OFF0, h, h, nullptr, 0));
                 VOX_TRY(ln_gemm(st, tw.ff1, h, tw.ln3_w, tw.ln3_b, 1e-5f, a1, N, T2, a2, 1));
                 VOX_TRY(conv_gemm(st, tw.ff2, a2, nullptr, nullptr, N, T2, 0, FLOW_OFF0, h, h, nullptr, 0));
@@ -4736,6 +4771,7 @@ int vox_flow_create(vox_ctx* ctx, const vox_flow_config* cfg, const vox_flow_wei
         m->conv1x.push_back(cx);
     }
     ok = ok && tb_pack(m->tblocks, C, inner, m->packed, &m->packed_mem);
+    if (!m->packed.empty()) alloc(&m->tb_ws, TB_PLANES * tb_plane(rows));
     if (!ok) { vox_flow_destroy(m); return vox_fail(VOX_ERR_NOMEM, "flow_create: hipMalloc failed"); }
     // time projections of every Euler step and resnet, once: tb[s][r] = mlp_r(Mish(linear_2(SiLU(linear_1(emb_s)))))
     hipStream_t st = nullptr;
@@ -5078,6 +5114,7 @@ struct vox_glmflow {
     std::vector<vox_flow_tblock_w> tblocks;
     std::vector<FlowPacked> packed;         // per transformer block, or empty
     void* packed_mem = nullptr;
+    float* tb_ws = nullptr;                 // their scratch: TB_PLANES planes of the most rows
     int max_batch, max_T, max_mel, n_res, n_att;
     std::vector<float> dt;
     float* tb = nullptr;
@@ -5093,7 +5130,7 @@ extern "C" {
 void vox_glmflow_destroy(vox_glmflow* m) {
     if (!m) return;
     for (int i = 0; i < 10; ++i) (void)hipFree(m->buf[i]);
-    (void)hipFree(m->tb); (void)hipFree(m->spk); (void)hipFree(m->pe); (void)hipFree(m->pp); (void)hipFree(m->packed_mem);
+    (void)hipFree(m->tb); (void)hipFree(m->spk); (void)hipFree(m->pe); (void)hipFree(m->pp); (void)hipFree(m->packed_mem); (void)hipFree(m->tb_ws);
     delete m;
 }
 
@@ -5127,6 +5164,7 @@ int vox_glmflow_create(vox_ctx* ctx, const vox_glmflow_config* cfg, const vox_gl
     alloc(&m->pe, (size_t)2 * FLOW_MAXKEYS * D);
     alloc(&m->pp, (size_t)2 * FLOW_MAXKEYS * D);
     ok = ok && tb_pack(m->tblocks, C, inner, m->packed, &m->packed_mem);
+    if (!m->packed.empty()) alloc(&m->tb_ws, TB_PLANES * tb_plane(rows));
     if (!ok) { vox_glmflow_destroy(m); return vox_fail(VOX_ERR_NOMEM, "glmflow_create: hipMalloc failed"); }
     hipStream_t st = nullptr;
     g_conv_planes = 3;
@@ -5200,12 +5238,12 @@ int vox_glmflow_decode(vox_glmflow* m, void* stream, const int32_t* tokens, int 
     auto tblocks = [&](float* h, int rows_T, int& li, float* a1, float* a2, float* a3) -> int {
         for (int j = 0; j < c.est_blocks; ++j, ++li) {
             const vox_flow_tblock_w& tw = m->tblocks[li];
-            const FlowPacked* pk = m->packed.empty() || tb_room(N * rows_T) > m->buf_floats ? nullptr : &m->packed[li];
-            if (pk) tb_qkv(st, *pk, tw, h, a1, j == 0, a2, N * rows_T);
+            const FlowPacked* pk = m->packed.empty() ? nullptr : &m->packed[li];
+            if (pk) tb_qkv(st, *pk, tw, h, m->tb_ws, j ? &m->tblocks[li - 1] : nullptr, a2, N * rows_T);
             else VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, rows_T, a2, 0));
             FlowAttn a{a2, nullptr, nullptr, nullptr, nullptr, a3, rows_T, HE, hd, 0, 0, 0, 0, 1.0f / sqrtf((float)hd), 0};
             launch_flow_attn(st, a, rows_T, HE, N);
-            if (pk) { tb_ff(st, *pk, tw, a3, h, a1, j == 0, j + 1 == c.est_blocks, N * rows_T); continue; }
+            if (pk) { tb_ff(st, *pk, tw, a3, h, m->tb_ws, j == 0, j + 1 == c.est_blocks, N * rows_T); continue; }
             VOX_TRY(conv_gemm(st, tw.out, a3, nullptr, nullptr, N, rows_T, 0, FLOW_OFF0, h, h, nullptr, 0));
             VOX_TRY(ln_gemm(st, tw.ff1, h, tw.ln3_w, tw.ln3_b, 1e-5f, a1, N, rows_T, a2, 1));
             VOX_TRY(conv_gemm(st, tw.ff2, a2, nullptr, nullptr, N, rows_T, 0, FLOW_OFF0, h, h, nullptr, 0));
