@@ -84,11 +84,6 @@ struct ConvGemmArgs {
 #else
 #define CG_DEV(a, bit) 0
 #endif
-// the two leading bf16 terms of v
-__device__ __forceinline__ void split2(float v, bf16_t& h, bf16_t& m) {
-    h = f2bf(v);
-    m = f2bf(v - bf2f(h));
-}
 // sin for the fused epilogues: explicit reduction to revolutions + the hardware v_sin_f32 (absolute error ~1e-6 on [-1, 1]:
 // far inside the 1e-4 waveform bar, and sin^2 enters scaled by 1/beta ~ 1).  The libm sinf (argument-reduction table,
 // private array) cannot be inlined into a GEMM epilogue without spilling the accumulators to scratch.
@@ -1197,12 +1192,12 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
             for (int r = 0; r < 4; ++r) red[wave][mt * NT + t][r * 64 + lane] = acc[mt][t][r];
     __syncthreads();
     // work item e = (tile, accumulator component r): row m0 + 16 mt + 4 (lane / 16) + r, column n0 + 16 t + lane % 16; wave w takes
-    // the items w, w + WV, ...  Two passes: every operand of every item of this wave (bias, scale, row scale, residual, Snake constants)
+    // the items w, w + WV, ...  Two passes: every operand of every item of this wave (bias, scale, row scale, residual)
     // is requested first, branch-free (clamped indices), THEN the arithmetic and the stores — item by item the loads of item i + 1 could not
     // move above the stores of item i (the residual may alias the output), and an item cost up to three dependent round trips: the
     // epilogue was most of this kernel's time.  Per element the operations and their order are unchanged.
     constexpr int NE = (MT * NT * 4 + WV - 1) / WV;
-    float e_b[NE], e_s[NE], e_rs[NE], e_res[NE], e_a[NE], e_i[NE];
+    float e_b[NE], e_s[NE], e_rs[NE], e_res[NE];
     const int Mc = a.M - 1, Nc = a.N - 1;
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
@@ -1213,8 +1208,6 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
         e_s[i] = a.scale ? a.scale[n] : 1.0f;
         e_rs[i] = a.rscale ? a.rscale[m] : 1.0f;
         e_res[i] = a.res ? a.res[(size_t)m * a.N + n] : 0.0f;
-        e_a[i] = a.out2 ? a.sn_alpha[n % a.sn_mod] : 0.0f;
-        e_i[i] = a.out2 ? a.sn_invb[n % a.sn_mod] : 0.0f;
     }
 #pragma unroll
     for (int i = 0; i < NE; ++i) {
@@ -1234,17 +1227,7 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
         const size_t o = (size_t)m * a.N + n;
         if (a.res) v = e_res[i] + sv * v;
         else if (a.scale) v = sv * v;
-        if (a.out) a.out[o] = v;
-        if (a.out2) {
-            const float sv2 = snake_f(v, e_a[i], e_i[i]);
-            if (a.out2_s2) {
-                const int cw = a.sn_mod, jj = n / cw, c = n - jj * cw;
-                bf16_t* r16 = reinterpret_cast<bf16_t*>(a.out2 + (size_t)m * a.N) + (size_t)jj * 2 * cw;
-                split2(sv2, r16[c], r16[cw + c]);
-            } else {
-                a.out2[o] = sv2;
-            }
-        }
+        a.out[o] = v;
     }
 }
 
@@ -1752,7 +1735,7 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
     a.bias_mod = w.bias_mod > 0 ? w.bias_mod : w.n; a.gelu = gelu;
     if (out2 && sn) { a.out2 = out2; a.sn_alpha = sn->alpha; a.sn_invb = sn->inv_beta; a.sn_mod = sn_mod > 0 ? sn_mod : w.n; }
     for (int k = 0; k < w.n_taps; ++k) a.off[k] = offs ? offs[k] : 0;
-    if (g_conv_rows_gemm && rows_gemm_on() && a.M <= g_conv_skinny_rows && w.cin % 32 == 0 && (w.n_taps * w.cin) % 128 == 0 && (!ln_w || (w.n_taps == 1 && a.off[0] == 0))) {
+    if (g_conv_rows_gemm && rows_gemm_on() && out && !out2 && a.M <= g_conv_skinny_rows && w.cin % 32 == 0 && (w.n_taps * w.cin) % 128 == 0 && (!ln_w || (w.n_taps == 1 && a.off[0] == 0))) {
         // every operand requested up front, K split over the block's waves (k_rows_gemm): 8 waves from K = 512 on
         const int K = w.n_taps * w.cin, wv = (K >= 512 && K % 256 == 0 && rows_wv8_on()) ? 8 : 4, kb = K / (32 * wv);
         const int tiles = ((w.n + 15) / 16) * ((a.M + 15) / 16);
