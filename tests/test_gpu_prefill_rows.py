@@ -15,7 +15,7 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("B,N_,K", [(33, 128, 2048), (48, 256, 2048), (49, 128, 3072), (64, 4096, 2048), (65, 128, 6144), (80, 128, 2048),
-                                    (81, 4096, 2048), (97, 128, 4096), (128, 384, 2048)])
+                                    (81, 4096, 2048), (97, 128, 4096), (128, 384, 2048), (35, 4224, 2048), (64, 6144, 2048), (79, 5120, 3072), (50, 8192, 2048)])
 def test_linear_rows_bit_exact(dev, B, N_, K):  # noqa: F811
     from vox_serve_amd import _native as N
     rng = np.random.default_rng(B + N_ + K)

@@ -1520,10 +1520,12 @@ __global__ __launch_bounds__(512) void k_gemm_fullk(LinArgs a) {
 // tiles (gate and up beside each other) and up to 80 rows; a wave's k-step (weights and rows, 1 KB per 16 x 32 tile) comes by
 // global_load_lds into its own S-stage ring.  Nothing is shared before the final sum, so there is no barrier in the loop: a wave waits for
 // its own requests, takes the step into registers, asks for the step S further on and multiplies.  Rows come normalised (k_norm_rows).
-// Bound by the L2 -> LDS path: a block moves its rows once more per NT column tiles.  75 rows, us, k_gemm_fullk before: gate / up
-// 6144 x 2048 42 -> 18, down 2048 x 6144 18.5 -> 14, q | k | v 4096 x 2048 20.6 -> 11, o 2048 x 2048 8.4 -> 6.2 (beside the first and the
-// third a norm launch of 4.5).  More than two stages give nothing (14.0 / 14.5 / 14.8 with 2 / 3 / 5); fragment-major rows are worth a
-// sixth (1 KB requests: gate / up 20.7 -> 17.7), which is why the norm writes them so.
+// Bound by the L2 -> LDS path: a block moves its rows once more per NT column tiles.  75 rows, us inside a prefill, k_gemm_fullk before:
+// gate / up 6144 x 2048 42 -> 18, down 2048 x 6144 18.5 -> 14.4, q | k | v 4096 x 2048 20.6 -> 10.3, o 2048 x 2048 8.4 -> 7.7 (beside the first
+// and the third a norm launch of 4.8); 48 rows 15.5 / 12.1 / 8.3 / 6.5, 128 rows 27.7 / 19 / 14 / 9.  Qwen3 talker prefill with its first
+// frame, us, before and now: 33 rows 3145 / 3061, 48 3175 / 3076, 64 3201 / 3186, 65 3980 / 3313, 80 4041 / 3335, 96 4190 / 3739, 128 4814 /
+// 4168.  More than two stages give nothing (14.0 / 14.5 / 14.8 with 2 / 3 / 5); fragment-major rows are worth a sixth (1 KB requests: gate /
+// up 20.7 -> 17.7), which is why the norm writes them so.
 // ================================================================================================
 template <int MT, int NT, int EPI, int S>
 __global__ __launch_bounds__(512) void k_gemm_rows(LinArgs a) {
@@ -1781,12 +1783,14 @@ static int launch_gemm_rows_t(hipStream_t st, const LinArgs& a) {
     hipLaunchKernelGGL(kern, dim3(a.N / (16 * NT) * a.row_tiles), dim3(512), lds, st, a);
     return VOX_OK;
 }
-// Rows of a block: all of them (up to 80) where the columns alone give a block per CU, halves of them for the narrow outputs.
+// Rows of a block: all of them (up to 80) where the columns alone give whole rounds of a block per CU, halves of them for narrower outputs and
+// between one round and two.  Bare linears, us, k_gemm_fullk / whole / halves: 4096 x 4096, 64 rows 26 / 15.5 / 16.3; 8192 x 6144 78 / 55 / 63;
+// 6144 x 2048 19.8 / 20.9 / 19.1 with weights from memory, 19.7 / 16.9 / 14.7 from cache; 5120 x 4096 38 / 25 / 22; 6144 x 8192, 80 rows 112 / 73 / 65.
 template <int EPI>
 static int launch_gemm_rows(hipStream_t st, const LinArgs& a0) {
     LinArgs a = a0;
     const int t16 = (a.B + 15) / 16;
-    a.row_tiles = EPI != EPI_SILU_MUL && a.N / 16 < 256 ? 2 : t16 > 5 ? 2 : 1;
+    a.row_tiles = EPI != EPI_SILU_MUL && a.N / 16 < 512 && a.N / 16 != 256 ? 2 : t16 > 5 ? 2 : 1;
     const int mt = (t16 + a.row_tiles - 1) / a.row_tiles;
     a.rt_rows = 16 * mt;
     if constexpr (EPI == EPI_SILU_MUL) {
