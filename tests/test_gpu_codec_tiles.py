@@ -5,8 +5,9 @@ fill the last one, intermediate sizes that end inside a gate / up pair, chunks s
 place) and a batch whose requests end inside a tile.
 
 Tolerance: the waveform bar of the decoder, RMS <= 1e-4 against fp32 (two bf16 terms keep 16 significand bits of every operand: relative
-2^-17 per product, and the sums are fp32).  In the bf16 operand mode one term keeps 8 bits, 2^-9 per operand.  That mode rounds where the
-staged kernels rounded, so it is held to the same multiple of its own rounding: 2^8 times the bar."""
+2^-17 per product, and the sums are fp32).  In the bf16 operand mode one term keeps 8 bits, 2^-9 per operand, through some 30 convs in
+sequence: sqrt(30) * 2^-9 of the signal, times four = 4.3e-2 (a waveform of the mode is off by 1.4e-2 to 2.3e-2; 32 channels of one tap lost
+anywhere move it by 8e-2 to 1.8e-1 at the median of all weights)."""
 import numpy as np
 import pytest
 import torch
@@ -32,7 +33,9 @@ CASES = [
     ((512, 384, 384, 640, 6, 64, 1024, [2, 2, 2, 3]), 2, 4),   # 128-channel steps only
     ((64, 96, 96, 96, 2, 16, 1536, [2, 2, 2, 2]), 3, 1),       # whole residual units of 64 rows whose look-back (54) is nearly all history
     ((512, 256, 512, 768, 8, 64, 512, [8, 5, 4, 3]), 4, 2),    # 256-channel steps, the last block's 32 channels over many rows
+    ((64, 96, 32, 160, 2, 16, 1536, [8, 5, 4, 3]), 18, 1),     # whole units of 192 channels (11 520 rows) and, in eight waves, of 96 (34 560)
 ]
+BF16_BAR = 4 * 30 ** 0.5 * 2 ** -9      # of the signal
 
 
 @pytest.mark.parametrize("shape,n,chunk", CASES)
@@ -49,7 +52,7 @@ def test_conv_tiles_against_fp32(dev, shape, n, chunk, precision):  # noqa: F811
     cache = dec.init_cache(n)
     got = torch.cat([dec.decode_chunk(codes[:, :, t:t + chunk], cache)[0].cpu().clone() for t in range(0, 3 * chunk, chunk)], -1).numpy()
     assert got.shape == ref.shape and rms(ref) > 1e-3
-    assert rms(got - ref) < (1e-4 if precision == "fp32" else 2 ** 8 * 1e-4), (rms(got - ref), rms(ref))
+    assert rms(got - ref) < (1e-4 if precision == "fp32" else BF16_BAR * rms(ref)), (rms(got - ref), rms(ref))
     dec.close()
 
 

@@ -736,9 +736,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
 // taps of this one), the weights are a stream of C x 32 slices through S stages.  What the lanes then hold, eight neighbouring channels
 // of a row, is after SnakeBeta and the two-term split the activation operand of conv2 as it stands: conv2 is C / 32 further slices of the
 // same stream, and the intermediate never leaves the registers.  x, the history and the weights arrive by LDS DMA as in k_conv_dma.
-// Bound: memory (x, h read, h, out2 written: 944 MB at 614 400 rows x 96) beside the matrix cores and the activations' VALU work: 309 us there,
-// 3.1 TB/s (326 with the residual asked for in the epilogue; four stages or 64-row blocks 311 - 332); the staged form of this kernel, with
-// the intermediate through LDS, took 461 - 498.
+// Bound: memory (x, h read, h, out2 written: 944 MB at 614 400 rows x 96) beside the matrix cores and the activations' VALU work: 335 us on
+// average there within a chunk, 2.8 TB/s; the staged form of this kernel, with the intermediate through LDS, took 461 - 498.  (Against 309 when
+// timed alone: 326 with the residual asked for in the epilogue, 311 - 332 with four stages or 64-row blocks.)
 template <int C, int CH, int TAPS, int T, int HP, int NW, int MT, int S>
 __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_conv_unit(ConvDmaArgs a1, ConvDmaArgs a2, int H) {
     constexpr int BM = 16 * MT * NW, R = BM + HP, NT = CH / 16, NP = CH / 32, NT2 = C / 16, NCK = C / 32;
@@ -1675,6 +1675,7 @@ struct vox_codec {
     int planes = 2;     // operand planes of the conv GEMMs (vox_codec_set_operand_planes)
     bool decoded = false;   // a chunk has run: the slots' streaming history is stored in the format `planes` implies
     // state (per slot)
+    // (one or two operand planes: all but st_dw and st_final hold the two bf16 terms that the conv which reads them would make of a row, 4 bytes a value)
     float *st_pre, *st_dw[2], *st_dec0, *st_tc[4], *st_ru[4][3], *st_final;
     bf16_t* ring;   // [layers][slots][Wn][2][HD]
     long* pos;      // [slots]
@@ -1976,8 +1977,9 @@ static int conv_unit(hipStream_t st, ConvDmaArgs& a1, ConvDmaArgs& a2, int* fuse
     for (int k = 0; k < a1.n_taps; ++k) { H = a1.off[k] > H ? a1.off[k] : H; omin = a1.off[k] < omin ? a1.off[k] : omin; }
     for (int k = 2; k < a1.n_taps; ++k)
         if (a1.off[k - 1] - a1.off[k] != a1.off[0] - a1.off[1]) return VOX_OK;
-    // 96 channels: always (one request, 19 200 rows: 27 -> 18 us; 614 400 rows: 600 -> 309).  192 channels: from 8192 rows on (12 800 rows two
-    // launches 48 us, one 32; 204 800: 412 and 327); below, two launches that add in the same order (6 400 rows 27 and 30, 1 280: 16 and 29)
+    // 96 channels: always (within a chunk: one request, 19 200 rows 27 -> 20 us, 614 400 rows 600 -> 335).  192 channels: from 8192 rows on (12 800
+    // rows two launches 48 us, one 32; 204 800: 412 and 327 timed alone, 424 and 382 within a chunk); below, two launches that add in the same
+    // order (6 400 rows 27 and 30, 1 280: 16 and 29)
     if (omin < 0 || H > 64 || a1.L % 64 || !a2.res) return VOX_OK;
     if (C == 192 && a1.M <= 8192) {
         *fused = CONV_CHUNKS;

@@ -1243,7 +1243,9 @@ static inline bool hb_dma_ok(const bf16_t* W, size_t a_rows, size_t N, int K, co
 // than M).  2048 rows, N x K = 2560 x 2048: 128 x 128 / four waves, two blocks per CU 38.1 us, eight waves, four stages, one block 44.8; at
 // exactly one tile per CU (2048 x 2048) 32.3 and 25.1.  Below 224 tiles of 128: 64 x 64 (1024 rows, 2048 x 2048: 17.1 against 24.0), with
 // four stages while there are at most two blocks per CU (512 rows, 2048 x 5632: 25.6 against 42.0 with two stages; 200 rows, 11264 x 2048,
-// 704 tiles: 27.0 against 20.6).
+// 704 tiles: 27.0 against 20.6).  All forms, against the staged kernel (whole prompt steps of four layers of width 2048; us, 17 / 100 / 512 / 2048
+// rows): Kazozen 899 / 1046 / 1462 / 3212 -> 498 / 594 / 879 / 1823, Gaparax (HB_EPI_JOIN, whose epilogue keeps 272 bytes of scratch a lane) 1165 /
+// 1395 / 2007 / 4891 -> 669 / 863 / 1304 / 3416; at width 512 no row count is slower either.
 template <int EPI, bool GLU, bool LIST>
 void hb_launch_dma(hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
                    const hb_rowmap& rm, int groups, int rows, hb_glu_args glu = hb_glu_args{}) {
