@@ -16,18 +16,17 @@ pytestmark = pytest.mark.gpu
 class _GeneralBlocks:
     """The native library with a create call that gives every transformer block's q | k | v a zero bias."""
 
-    def __init__(self, lib, zeros):
-        self._lib, self._zeros = lib, zeros
+    def __init__(self, lib, zeros, blocks):
+        self._lib, self._zeros, self._blocks = lib, zeros, blocks
 
     def __getattr__(self, name):
         f = getattr(self._lib, name)
-        if name != "vox_flow_create":
+        if name not in ("vox_flow_create", "vox_glmflow_create"):
             return f
 
         def create(ctx, cfg, fw, *rest):
-            c, w = cfg._obj, fw._obj
-            for i in range((2 + c.est_mid) * c.est_blocks):
-                w.tblocks[i].qkv.bias = self._zeros.data_ptr()
+            for i in range(self._blocks):
+                fw._obj.tblocks[i].qkv.bias = self._zeros.data_ptr()
             return f(ctx, cfg, fw, *rest)
         return create
 
@@ -55,6 +54,35 @@ def test_fused_blocks_add_as_the_general_launches(monkeypatch, B, T, blocks):
     zeros = torch.zeros(3 * fc.est_heads * fc.est_head_dim, device="cuda:0")
     lib = CF.N.lib()
     with monkeypatch.context() as mp:
-        mp.setattr(CF.N, "lib", lambda: _GeneralBlocks(lib, zeros))
+        mp.setattr(CF.N, "lib", lambda: _GeneralBlocks(lib, zeros, fc.n_att))
         prompt_general, general = mels()
     assert rms(got) > 0.5 and np.array_equal(prompt, prompt_general) and np.array_equal(got, general)
+
+
+# GLM-4-Voice's flow: two row counts a step (all mel frames and every second), an odd number of frames among them
+@pytest.mark.parametrize("B,T,blocks", [(1, 3, 1), (3, 8, 2), (2, 25, 4)])
+def test_glm_blocks_add_as_the_general_launches(monkeypatch, B, T, blocks):
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    from oracle import glm_dec_ref as GR
+    from tests.test_gpu_glm_decoder import glm_flow_plugin_cfg
+    from vox_serve_amd.tokenizer import glm as GM
+    fc = GR.GlmFlowCfg(vocab=113, enc_layers=1, est_mid=1, est_blocks=blocks)
+    W = GR.random_glm_flow_weights(fc, seed=T)
+    tok = torch.randint(0, 113, (B, T), generator=torch.Generator().manual_seed(B))
+    z = GR.glm_cfm_noise(1, 0, B, fc.mel, fc.mel_len(T))
+
+    def mels():
+        flow = GM.GLMFlow(W, glm_flow_plugin_cfg(fc), device="cuda:0", max_batch=B, max_T=T, seed=1)
+        try:
+            return flow.inference(tok, noise=z).cpu().numpy()
+        finally:
+            flow.close()
+
+    got = mels()
+    zeros = torch.zeros(3 * fc.est_heads * fc.est_head_dim, device="cuda:0")
+    lib = GM.N.lib()
+    with monkeypatch.context() as mp:
+        mp.setattr(GM.N, "lib", lambda: _GeneralBlocks(lib, zeros, (4 + fc.est_mid) * blocks))
+        general = mels()
+    assert rms(got) > 0.3 and np.array_equal(got, general)
