@@ -77,3 +77,17 @@ def test_rounds_of_a_few_row_product(rows, inner):
     finally:
         d.close()
     assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR
+
+
+# every tile: 32 x 32, 64 x 32, 128 x 64, 128 x 128, 192 x 128, 256 x 128, 256 x 192, 256 x 160 (whose columns do not divide among the waves), rows
+# and columns with remainders; fewer k-tiles than stages
+@pytest.mark.parametrize("rows,vocab,width", [(33, 515, 192), (63, 6145, 512), (65, 8193, 64), (65, 16769, 256), (129, 24001, 64), (255, 28673, 128),
+                                              (257, 16769, 192), (257, 16769, 512)])
+def test_a_row_has_the_same_logits_in_every_tile(rows, vocab, width):
+    test_a_row_has_the_same_logits_in_every_tile_form(rows, vocab, width)
+
+
+# gate and up products in 64 x 64, 192 x 128 and 256 x 192, columns that are no multiple of a block's
+@pytest.mark.parametrize("rows,mlp", [(300, P.dense(1088)), (129, P.dense(8384)), (300, P.dense(11328)), (257, P.dense(16448)), (131, P.moe(4, 4, 5632, 0, 0))])
+def test_activation_behind_both_products_in_every_tile(rows, mlp):
+    test_activation_behind_both_products(rows, mlp)

@@ -624,15 +624,22 @@ __global__ __launch_bounds__(256) void k_hb_gemm_bf16(const float* A, long lda, 
 }
 
 // More than 16 rows, both operands bf16 in memory, K a multiple of 64: BM x BN outputs per block, WM x WN waves.  k-tiles of 64 go from memory
-// straight into LDS (global_load_lds, 1 KB per wave instruction = eight 128-byte rows) and S stages of them are kept in flight: a tile's
-// requests are S - 1 tiles old when it is multiplied, and no register holds them.  One wait + barrier per k-tile: it says that every wave's
-// part of tile t has landed and that nobody reads the stage of tile t - 1 any more, which is then requested anew.  The 16-byte pieces of a
-// row lie at piece ^ (row & 7) (the swizzle is in the address each lane reads), so the fragment reads of 16 rows do not meet in a bank.
-// Per output the products are added as in k_hb_gemm_bf16 (k ascending in steps of 32): the same bits.
-// The blocks of one XCD (block id modulo 8) take neighbouring tiles, 512 rows deep, so that its L2 holds what they share.
-// Bound by the L2 -> LDS path (one k-tile of 128 x 128 moves 32 KB for 515 matrix clocks) and, for wide outputs, by their stores.
-// Measured against k_hb_gemm_bf16<64> (2048 rows; us): 2048 x 2048 64.7 -> 25.1, 2048 x 5632 (N x K) 160 -> 51, 11264 x 2048 305 -> 118;
-// 200 rows: 2048 x 2048 31.4 -> 11.6; 64 rows: 31.0 -> 11.2.  Staged through registers instead the same tiles took 34.7 / 74.6 / 151.
+// straight into LDS (global_load_lds, 1 KB per wave instruction = eight 128-byte rows) and S stages of them are kept in flight: no register
+// holds them.  The 16-byte pieces of a row lie at piece ^ (row & 7) (the swizzle is in the address each lane reads), so the fragment reads of
+// 16 rows do not meet in a bank.
+// A wave's fragments are read half a k-tile (32 columns of K) before they are multiplied, a read between every few products: all waves of a
+// block pass its barrier together, so without that the LDS reads and the matrix cores take turns.  One wait + barrier per k-tile, in its middle:
+// it says that every wave's part of tile t + 1 has landed and that every wave holds the second half of tile t in registers, so tile t's stage
+// is requested anew (tile t + S).  (MT * NT products hide MT + NT reads; at least two waves per SIMD are asked of the compiler, which otherwise
+// keeps the sums in accumulation registers and copies them around on every pass.)
+// Per output the products are added as in k_hb_gemm_bf16 (k ascending in steps of 32): the same bits, whatever the tile.
+// The blocks of one XCD (block id modulo 8) take neighbouring tiles, 1024 rows deep, so that its L2 holds what they share.
+// The weights are the first operand: a lane then holds four neighbouring columns of a row, one 16-byte store (HB_EPI_JOIN, whose update goes
+// through every stream of a column, has them second).
+// Bound by LDS (operand reads and the tiles that land, 128 bytes a clock: 1.2 - 1.5 times that was measured) and, over tiles of 256 rows, by what
+// each CU gets from L2 (75 KB/us).  2048 rows; N x K; us, reading the fragments where they are multiplied and now: 2048 x 2048 27.9 -> 22.4,
+// 5120 x 2048 82 -> 40.2 (256 x 160: one tile per CU), 4096 x 2048 45 -> 34.5, 2048 x 5632 55.4 -> 51.5, 11264 x 2048 with hb_glu 121 -> 88.  With
+// k-tiles of 32 and up to eight stages each: 48 / 42 / 66 / 98 for the last four; sixteen waves (64 x 64 each): 55 for the second.
 // GLU: the block's columns are BN / 2 gate rows and the BN / 2 up rows beside them, interleaved so that a lane owns both; what is stored is
 // hb_glu of the two, rounded to bf16 as the product behind it reads it (C: bf16 [.][ff], N = ff): neither product is written to memory.
 struct hb_glu_args {
@@ -640,11 +647,12 @@ struct hb_glu_args {
     int gelu;
 };
 template <int BM, int BN, int WM, int WN, int S, int EPI, bool GLU, bool LIST>
-__global__ __launch_bounds__(WM * WN * 64) void k_hb_gemm_dma(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
-                                                              int N, int K, hb_rowmap rm, hb_glu_args glu) {
-    constexpr int BK = 64, NWV = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16, CN = GLU ? BN / 2 : BN, NA = BM / 8 / NWV, NW = BN / 8 / NWV;
+__global__ __launch_bounds__(WM * WN * 64, 2) void k_hb_gemm_dma(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M,
+                                                                 int N, int K, hb_rowmap rm, hb_glu_args glu) {
+    constexpr int BK = 64, NWV = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16, CN = GLU ? BN / 2 : BN, NA = BM / 8 / NWV, NW = (BN / 8 + NWV - 1) / NWV;
     constexpr int STAGE = (BM + BN) * BK, U = NT * 8;       // U: gate (up) columns of a wave
-    static_assert(BM % (8 * NWV) == 0 && BN % (8 * NWV) == 0 && (!GLU || NT % 2 == 0), "whole wave instructions");
+    constexpr bool TR = EPI != HB_EPI_JOIN;                 // the weights are the first operand
+    static_assert(BM % (8 * NWV) == 0 && BN % 8 == 0 && BN / 8 >= NWV && (!GLU || NT % 2 == 0) && S > 2 - (BM >= 256) && (S - 1) * (NA + NW) < 64, "whole wave instructions");
     extern __shared__ __attribute__((aligned(1024))) bf16_t smem[];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int* lst = nullptr;
@@ -657,13 +665,15 @@ __global__ __launch_bounds__(WM * WN * 64) void k_hb_gemm_dma(const bf16_t* A, l
     const int tm = (M + BM - 1) / BM, tn = (N + CN - 1) / CN, total = tm * tn, per = (total + 7) >> 3;
     const int in_xcd = (int)blockIdx.x >> 3, t = ((int)blockIdx.x & 7) * per + in_xcd;
     if (in_xcd >= per || t >= total) return;
-    constexpr int GM = 512 / BM;
+    constexpr int GM = 1024 / BM;
     const int g0 = t / (GM * tn) * GM, gh = tm - g0 < GM ? tm - g0 : GM, tg = t - g0 * tn;
     const int m0 = (g0 + tg % gh) * BM, n0 = tg / gh * CN;
     const int wm = wv / WN, wn = wv % WN, fr = lane & 15, fk = lane >> 4;
-    // byte offsets of this lane's 16 bytes of each of its rows (rows past the end repeat the last one: nothing of them is stored)
+    // byte offsets of this lane's 16 bytes of each of its rows (rows past the end repeat the last one: nothing of them is stored; a wave
+    // that has no eight rows of W left in the last round repeats those of the round before)
     const unsigned pc = ((lane & 7) ^ (lane >> 3)) * 16;
     unsigned ao[NA], wo[NW];
+    int cw[NW];
 #pragma unroll
     for (int i = 0; i < NA; ++i) {
         int gm = m0 + (wv + i * NWV) * 8 + (lane >> 3);
@@ -673,66 +683,125 @@ __global__ __launch_bounds__(WM * WN * 64) void k_hb_gemm_dma(const bf16_t* A, l
     }
 #pragma unroll
     for (int i = 0; i < NW; ++i) {
-        const int r = (wv + i * NWV) * 8 + (lane >> 3);
+        cw[i] = wv + i * NWV < BN / 8 ? wv + i * NWV : wv + i * NWV - NWV;
+        const int r = cw[i] * 8 + (lane >> 3);
         int gn = GLU ? n0 + r / (2 * U) * U + r % U : n0 + r;
         gn = gn < N ? gn : N - 1;
         if (GLU && r % (2 * U) >= U) gn += N;
         wo[i] = (unsigned)gn * (unsigned)(K * 2) + pc;
     }
-    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)smem + wv * 1024;
+    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)smem;
     auto request = [&](int stage, int k0) {
         const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * (STAGE * 2));
+        const bf16_t *ak = A + k0, *wk = Wt + k0;
 #pragma unroll
-        for (int i = 0; i < NA; ++i) lds_dma16(A, ao[i] + k0 * 2, ls + i * NWV * 1024);
+        for (int i = 0; i < NA; ++i) lds_dma16(ak, ao[i], ls + (wv + i * NWV) * 1024);
 #pragma unroll
-        for (int i = 0; i < NW; ++i) lds_dma16(Wt, wo[i] + k0 * 2, ls + BM * 128 + i * NWV * 1024);
+        for (int i = 0; i < NW; ++i) lds_dma16(wk, wo[i], ls + BM * 128 + cw[i] * 1024);
     };
     hb_f32x4 acc[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
         for (int j = 0; j < NT; ++j) acc[i][j] = hb_f32x4{0.f, 0.f, 0.f, 0.f};
-    const int nt = K / BK, klast = K - BK;
+    hb_bf16x8 a0[MT], w0[NT], a1[MT], w1[NT];
+    const int p0 = (fk ^ (fr & 7)) << 3, p1 = ((4 + fk) ^ (fr & 7)) << 3;
+    const int arow = (wm * MT * 16 + fr) * BK, wrow = BM * BK + (wn * NT * 16 + fr) * BK;
+    auto read = [&](const bf16_t* sp, int piece, hb_bf16x8 (&af)[MT], hb_bf16x8 (&wf)[NT]) {
 #pragma unroll
-    for (int s = 0; s < S - 1; ++s) request(s, s * BK < klast ? s * BK : klast);
-    int stage = 0;
-    for (int kt = 0; kt < nt; ++kt) {
-        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
-        const int kn = (kt + S - 1) * BK;
-        request(stage == 0 ? S - 1 : stage - 1, kn < klast ? kn : klast);
-        const bf16_t *as = smem + stage * STAGE + (wm * MT * 16 + fr) * BK, *ws = smem + stage * STAGE + BM * BK + (wn * NT * 16 + fr) * BK;
+        for (int j = 0; j < NT; ++j) wf[j] = *(const hb_bf16x8*)(sp + wrow + j * 16 * BK + piece);
 #pragma unroll
-        for (int ks = 0; ks < 2; ++ks) {
-            const int piece = ((ks * 4 + fk) ^ (fr & 7)) << 3;
-            hb_bf16x8 af[MT], wf[NT];
+        for (int i = 0; i < MT; ++i) af[i] = *(const hb_bf16x8*)(sp + arow + i * 16 * BK + piece);
+    };
+    // the products of one half tile, the reads of the next one (issued in front) spread between them
+    auto multiply = [&](const hb_bf16x8 (&af)[MT], const hb_bf16x8 (&wf)[NT]) {
 #pragma unroll
-            for (int i = 0; i < MT; ++i) af[i] = *(const hb_bf16x8*)(as + i * 16 * BK + piece);
-#pragma unroll
-            for (int j = 0; j < NT; ++j) wf[j] = *(const hb_bf16x8*)(ws + j * 16 * BK + piece);
+        for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
+                acc[i][j] = TR ? __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0)
+                               : __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], wf[j], acc[i][j], 0, 0, 0);
+        constexpr int G = MT * NT / (MT + NT);
+        if constexpr (G > 0) {
 #pragma unroll
-                for (int j = 0; j < NT; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i], wf[j], acc[i][j], 0, 0, 0);
+            for (int g = 0; g < MT + NT; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x8, G, 0);        // G products,
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // one LDS read
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, MT * NT - G * (MT + NT), 0);
         }
+    };
+    const int nt = K / BK, klast = K - BK;
+#pragma unroll
+    for (int s = 0; s < S; ++s) request(s, s * BK < klast ? s * BK : klast);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * (NA + NW)) : "memory");
+    read(smem, p0, a0, w0);
+    int stage = 0;
+    for (int kt = 0; kt < nt; ++kt) {
+        __builtin_amdgcn_sched_barrier(0);
+        read(smem + stage * STAGE, p1, a1, w1);
+        multiply(a0, w0);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
+        const int kn = (kt + S) * BK;
+        request(stage, kn < klast ? kn : klast);
         stage = stage == S - 1 ? 0 : stage + 1;
+        __builtin_amdgcn_sched_barrier(0);
+        read(smem + stage * STAGE, p0, a0, w0);
+        multiply(a1, w1);
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (the repeated last tiles: nothing may land after the block has ended)
+    // acc[i][j][r]: weight row (column of C) fk * 4 + r of tile j, row fr of tile i (without TR the other way round)
     if constexpr (GLU) {
+        const bool vec = (N & 3) == 0 && (ldc & 3) == 0 && ((size_t)C & 7) == 0;
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
+        for (int i = 0; i < MT; ++i) {
+            const int gm = m0 + (wm * MT + i) * 16 + fr;
+            if (gm >= M) continue;
+            bf16_t* row = (bf16_t*)C + (size_t)(LIST ? lst[gm] : gm) * ldc;
 #pragma unroll
             for (int j = 0; j < NT / 2; ++j) {
-                const int gn = n0 + wn * U + j * 16 + fr;
+                const int gn = n0 + wn * U + j * 16 + fk * 4;
                 if (gn >= N) continue;
-                const float bg = bias ? bias[gn] : 0.f, bu = bias ? bias[N + gn] : 0.f;
+                float y[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int gm = m0 + (wm * MT + i) * 16 + fk * 4 + r;
-                    if (gm < M)
-                        ((bf16_t*)C)[(size_t)(LIST ? lst[gm] : gm) * ldc + gn] =
-                            f2bf(hb_glu(acc[i][j][r] + bg, acc[i][j + NT / 2][r] + bu, glu.limit, glu.alpha, glu.up_offset, glu.gelu));
+                    const int c = gn + r < N ? gn + r : N - 1;
+                    y[r] = hb_glu(acc[i][j][r] + (bias ? bias[c] : 0.f), acc[i][j + NT / 2][r] + (bias ? bias[N + c] : 0.f), glu.limit, glu.alpha,
+                                  glu.up_offset, glu.gelu);
+                }
+                if (vec) *(uint2*)(row + gn) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
+                else
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (gn + r < N) row[gn + r] = f2bf(y[r]);
+            }
+        }
+    } else if constexpr (TR) {
+        const bool vec = (N & 3) == 0 && (ldc & 3) == 0 && ((size_t)C & 15) == 0;
+#pragma unroll
+        for (int i = 0; i < MT; ++i) {
+            const int gm = m0 + (wm * MT + i) * 16 + fr;
+            if (gm >= M) continue;
+            float* row = C + (size_t)(LIST ? lst[gm] : gm) * ldc;
+#pragma unroll
+            for (int j = 0; j < NT; ++j) {
+                const int gn = n0 + (wn * NT + j) * 16 + fk * 4;
+                if (gn >= N) continue;
+                if (vec) {
+                    float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+                    if constexpr (EPI == HB_EPI_RESID || EPI == HB_EPI_RESID_SCALED) v = *(const float4*)(row + gn);
+                    float y[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) hb_epilogue<EPI>(y + r, acc[i][j][r], bias ? bias[gn + r] : 0.f, hb_epi_arg<EPI>(rm, gn + r));
+                    *(float4*)(row + gn) = make_float4(y[0], y[1], y[2], y[3]);
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (gn + r < N) hb_epilogue<EPI>(row + gn + r, acc[i][j][r], bias ? bias[gn + r] : 0.f, hb_epi_arg<EPI>(rm, gn + r));
                 }
             }
+        }
     } else {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
@@ -1239,18 +1308,33 @@ __global__ __launch_bounds__(256) void k_hb_to_bf16(const float* A, long lda, bf
 static inline bool hb_dma_ok(const bf16_t* W, size_t a_rows, size_t N, int K, const hb_rowmap& rm) {
     return K > 0 && K % 64 == 0 && ((size_t)W & 15) == 0 && (rm.w_stride & 7) == 0 && a_rows * K < (1ull << 31) && N * K < (1ull << 31);
 }
-// Tiles by how many blocks they leave for 256 compute units (`rows`: rows of a product as far as the host knows; a gathered one has fewer
-// than M).  2048 rows, N x K = 2560 x 2048: 128 x 128 / four waves, two blocks per CU 38.1 us, eight waves, four stages, one block 44.8; at
-// exactly one tile per CU (2048 x 2048) 32.3 and 25.1.  Below 224 tiles of 128: 64 x 64 (1024 rows, 2048 x 2048: 17.1 against 24.0), with
-// four stages while there are at most two blocks per CU (512 rows, 2048 x 5632: 25.6 against 42.0 with two stages; 200 rows, 11264 x 2048,
-// 704 tiles: 27.0 against 20.6).  All forms, against the staged kernel (whole prompt steps of four layers of width 2048; us, 17 / 100 / 512 / 2048
-// rows): Kazozen 899 / 1046 / 1462 / 3212 -> 498 / 594 / 879 / 1823, Gaparax (HB_EPI_JOIN, whose epilogue keeps 272 bytes of scratch a lane) 1165 /
-// 1395 / 2007 / 4891 -> 669 / 863 / 1304 / 3416; at width 512 no row count is slower either.
+// A tile form: its size, what a block of it takes in ns (K / 64 steps of `step` beside `fixed`), and what share of that another round of blocks adds
+// (less than one where two blocks fit a CU).  Measured at K = 512, 2048 and 5632, N = 512 to 11264, 20 to 2048 rows.
+struct hb_tile {
+    int bm, bn;
+    float step, fixed, next;
+};
+static inline float hb_tile_ns(const hb_tile& t, int rows, int N, int K, int groups, int cols) {
+    const int blocks = hb_tile_count(rows, N, t.bm, t.bn / cols) * groups, rounds = (blocks + 255) / 256;
+    return (K / 64 * t.step + t.fixed) * (1.0f + (rounds - 1) * t.next);
+}
+// The tile whose blocks are through first by that measure, `rows` being the rows of a product as far as the host knows (a gathered one has fewer
+// than M): a wide tile moves fewer bytes per product, but a last round that is nearly empty costs as much as a full one.  Rows, N x K: tile
+// chosen, us, against the four forms of 64 and 128 that stood here before: 20, 2048 x 2048: 32 x 32, 7.4 (64 x 64 9.8); 200, 2048 x 5632: 64 x 32, 20 (25);
+// 300, 4096 x 2048: 128 x 64, 16 (21); 1024, 5120 x 2048: 192 x 128, 27 (44); 2048 rows: with the kernel.
 template <int EPI, bool GLU, bool LIST>
 void hb_launch_dma(hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
                    const hb_rowmap& rm, int groups, int rows, hb_glu_args glu = hb_glu_args{}) {
     constexpr int G = GLU ? 2 : 1;
-    const int t128 = hb_tile_count(rows, N, 128, 128 / G) * groups, t64 = hb_tile_count(rows, N, 64, 64 / G) * groups;
+    static const hb_tile T[] = {{32, GLU ? 64 : 32, GLU ? 190.f : 160.f, 2600.f, GLU ? 0.7f : 0.6f}, {64, 32, 195.f, 2900.f, 0.65f}, {64, 64, 290.f, 2300.f, 0.72f},
+                                {128, 64, 420.f, 2400.f, 0.84f}, {128, 128, 527.f, 5300.f, 1.f}, {192, 128, 625.f, 5800.f, 1.f},
+                                {256, 128, 710.f, 7500.f, 1.f}, {256, 192, 1120.f, 7000.f, 1.f}, {256, 160, 780.f, 9500.f, 1.f}};
+    int best = 0;
+    float ns = 0.f;
+    for (int i = 0; i < (GLU ? 8 : 9); ++i) {
+        const float v = hb_tile_ns(T[i], rows, N, K, groups, G);
+        if (i == 0 || v < ns) { best = i; ns = v; }
+    }
 #define HB_DMA(BM_, BN_, WM_, WN_, S_) \
     do { \
         constexpr int lds = S_ * (BM_ + BN_) * 128; \
@@ -1259,10 +1343,21 @@ void hb_launch_dma(hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, c
         hipLaunchKernelGGL(kern, dim3((hb_tile_count(M, N, BM_, BN_ / G) + 7) & ~7, groups), dim3(WM_ * WN_ * 64), lds, st, A, lda, W, bias, C, ldc, M, N, K, \
                            rm, glu); \
     } while (0)
-    if (t128 > 256) HB_DMA(128, 128, 2, 2, 2);
-    else if (t128 >= 224) HB_DMA(128, 128, 4, 2, 4);
-    else if (t64 <= 512) HB_DMA(64, 64, 2, 2, 4);
-    else HB_DMA(64, 64, 2, 2, 2);
+    switch (best) {
+    case 0:
+        if constexpr (GLU) HB_DMA(32, 64, 2, 2, 6);
+        else HB_DMA(32, 32, 2, 2, 8);
+        break;
+    case 1: HB_DMA(64, 32, 4, 1, 6); break;
+    case 2: HB_DMA(64, 64, 2, 2, 4); break;
+    case 3: HB_DMA(128, 64, 2, 2, 3); break;
+    case 4: HB_DMA(128, 128, 4, 2, 4); break;
+    case 5: HB_DMA(192, 128, 4, 2, 3); break;
+    case 6: HB_DMA(256, 128, 4, 2, 3); break;
+    case 7: HB_DMA(256, 192, 4, 2, 2); break;
+    default:
+        if constexpr (!GLU) HB_DMA(256, 160, 4, 2, 3);
+    }
 #undef HB_DMA
 }
 // the rows of A as bf16: rm.a16 when the kernel before has left them so, else rounded into the workspace (NULL: neither is possible)
