@@ -91,3 +91,20 @@ def test_a_row_has_the_same_logits_in_every_tile(rows, vocab, width):
 @pytest.mark.parametrize("rows,mlp", [(300, P.dense(1088)), (129, P.dense(8384)), (300, P.dense(11328)), (257, P.dense(16448)), (131, P.moe(4, 4, 5632, 0, 0))])
 def test_activation_behind_both_products_in_every_tile(rows, mlp):
     test_activation_behind_both_products(rows, mlp)
+
+
+# Window attention of 64 and 128 dims, steps of more rows than the few-row form takes: 1, 2, 8, 16 and 32 query heads to a key head (a block's 64
+# columns are 64 to 2 rows), pages that are no power of two, kept tokens before the window, portions that start inside and behind it
+@pytest.mark.parametrize("heads,kv,dim,page,window,keep,cuts", [(2, 2, 64, 16, 70, 3, [65, 66, 70]), (4, 2, 128, 24, 40, 5, [130, 67]), (8, 1, 64, 8, 300, 0, [129, 90]),
+                                                                (16, 1, 128, 32, 64, 70, [200, 65]), (32, 1, 64, 40, 33, 1, [67, 66]), (3, 1, 64, 16, 50, 2, [70, 66])])
+def test_window_attention_heads_of_a_key_head_together(heads, kv, dim, page, window, keep, cuts):
+    cfg = P.config([P.attention(heads=heads, kv_heads=kv, dim=dim, vdim=dim, size=window, keep=keep, mlp=P.dense(64))], width=64, vocab=50)
+    S = P.random_checkpoint(cfg, seed=heads, gain=1.3)
+    n = sum(cuts)
+    toks = torch.randint(0, 50, (n,), generator=torch.Generator().manual_seed(dim + n)).tolist()
+    d = U.Driver(cfg, S, dtype=torch.bfloat16, page_size=page, pages=(n + page - 1) // page + 1, max_rows=max(cuts))
+    try:
+        got = d.run_cut("r", toks, cuts)
+    finally:
+        d.close()
+    assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR

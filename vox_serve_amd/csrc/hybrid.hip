@@ -24,6 +24,7 @@ namespace {
 
 typedef __bf16 hb_bf16x8 __attribute__((ext_vector_type(8)));
 typedef float hb_f32x4 __attribute__((ext_vector_type(4)));
+typedef short hb_i16x4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ float hb_wave_sum(float v) {
 #pragma unroll
@@ -1369,6 +1370,11 @@ static const bf16_t* hb_rows16(hipStream_t st, hb_ws16 ws, const hb_rowmap& rm, 
     lda = K;
     return ws.p;
 }
+// hb_gemm reads A as bf16 anyway (and the workspace has room for its rows)
+static inline bool hb_takes16(const bf16_t* W, hb_ws16 ws, int M, int N, int K) {
+    return M > 16 && hb_dma_ok(W, M, N, K, hb_plain()) && (size_t)M * K <= ws.n;
+}
+static inline bool hb_takes16(const float*, hb_ws16, int, int, int) { return false; }
 // rm.count != NULL: `groups` gathered GEMMs of at most M rows each (about `rows`) in one launch (see hb_rowmap), their rows among the first
 // a_rows of A
 template <int EPI>
@@ -3309,12 +3315,9 @@ template <typename T> static int hb_lat_dp(int D) {
 // Tile t of the launch (blocks in descending order) is found by walking the requests' row counts (ceil(rows / 4) tiles each); blocks beyond the last tile leave.
 #define HB_LM_VLD 72      // keys per row of the transposed value tile (64 + 8: rows 16 bytes apart in banks)
 __device__ __forceinline__ void hb_split_bf16x8(const float* v, uint4& hi, uint4& lo) {
-    float h[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) h[i] = bfround(v[i]);
-    hi = make_uint4(pack_bf2(h[0], h[1]), pack_bf2(h[2], h[3]), pack_bf2(h[4], h[5]), pack_bf2(h[6], h[7]));
-    lo = make_uint4(pack_bf2(v[0] - h[0], v[1] - h[1]), pack_bf2(v[2] - h[2], v[3] - h[3]), pack_bf2(v[4] - h[4], v[5] - h[5]),
-                    pack_bf2(v[6] - h[6], v[7] - h[7]));
+    hi = make_uint4(pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7]));
+    lo = make_uint4(pack_bf2(v[0] - bflo(hi.x), v[1] - bfhi(hi.x)), pack_bf2(v[2] - bflo(hi.y), v[3] - bfhi(hi.y)),
+                    pack_bf2(v[4] - bflo(hi.z), v[5] - bfhi(hi.z)), pack_bf2(v[6] - bflo(hi.w), v[7] - bfhi(hi.w)));
 }
 __device__ __forceinline__ hb_f32x4 hb_mfma_bf16(uint4 a, uint4 b, hb_f32x4 c) {
     union { uint4 u; hb_bf16x8 v; } x, y;
@@ -4332,6 +4335,231 @@ __global__ __launch_bounds__(256) void k_hb_win_attn_mfma(const float* q, long l
             }
 }
 
+// The same for keys and values of D = 64 or 128 dims: a block's 64 query columns are all HPG = 1 << hsh heads of a key head beside each other (64 / HPG
+// consecutive rows of one request; column c of the block: row c / HPG, head c % HPG; 16 columns per wave), so a tile of keys is loaded once for
+// every head that reads it.  Tiles of 64 keys and values go straight into LDS, the next tile's while one is multiplied (two stages, one barrier a tile,
+// no register, no vector work); the values stay [key][dim] and are transposed on the way to the operand (ds_read_b64_tr_b16: 16 lanes, 4 keys x 16
+// dims).  Pieces of a row are swizzled through the address a lane loads from, so neither operand's reads meet in a bank.  Products, weights and
+// their order are those of the form above, and so are the tiles (the kept tokens and the window's start of the 64 rows around the block's): the
+// same bits.
+// Bound by the vector work of the softmax, the products (query and weights in two terms: 64 a wave and tile) and the operand reads, about 1000 clocks
+// each per wave and tile, and by the imbalance of the first rows (up to 34 tiles a CU, 26.5 on average).  2048 rows, 16 heads of 128 over 4, window
+// 1024 + 4: 100 us staged through registers per head, 55 here (63 with page arithmetic by division and 64-bit addresses).
+// the larger of a column's four lanes (l ^ 16, l ^ 32)
+__device__ __forceinline__ float hb_col_max(float v) {
+    const vox_u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r.x), __uint_as_float(r.y));
+    const vox_u2 s = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(s.x), __uint_as_float(s.y));
+}
+// NEAR: the page size is a power of two and a byte of the cache's halves is addressed in 32 bits
+template <int D, bool NEAR>
+__global__ __launch_bounds__(256, 2) void k_hb_win_attn_dma(const float* q, long ldq, const bf16_t* cache, float* out, bf16_t* out16, long ldo, const int* pos,
+                                                            const int* req_rows, int n_req, const int* ptab, int pts, int G, int hsh, int ps, long v_base,
+                                                            hb_win w, float scale, hb_sink sink, const float* gate, long ldg, float out_scale, int fold) {
+    constexpr int KS = D / 32, CT = D / 16, PP = D / 8, RB = D * 2, RPI = 1024 / RB, NI = 16 / RPI, TILE = 64 * RB;      // PP: 16-byte pieces of a row
+    constexpr float LOG2E = 1.44269504088896340736f, LOWEST = -1e30f;
+    extern __shared__ __attribute__((aligned(1024))) char smem_w[];      // [stage][keys | values][64][RB]
+    const int tid = threadIdx.x, wv = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, col = lane & 15, g4 = lane >> 4;
+    const int hpg = 1 << hsh, BR = 64 >> hsh;
+    const int nt_all = gridDim.y, half = (nt_all + 1) >> 1;
+    int t = nt_all - 1 - (int)blockIdx.y, rq = -1, rs = 0, re = 0, r64 = 0;
+    if (fold && (int)blockIdx.y >= half) t = (int)blockIdx.y - half;
+    for (int r = 0; r < n_req; ++r) {
+        const int a = req_rows[r], b = req_rows[r + 1], nt = (b - a + BR - 1) >> (6 - hsh);
+        if (t < nt) { rq = r; rs = a + BR * t; re = b; r64 = a + (BR * t & ~63); break; }
+        t -= nt;
+    }
+    if (rq < 0) return;
+    const int g = blockIdx.x;
+    const int nrows = re - rs < BR ? re - rs : BR;
+    const int w_first = (wv * 16) >> hsh, w_end = (wv * 16 + 15) >> hsh, w_last = w_end < nrows ? w_end : nrows - 1;      // the wave's rows of the tile
+    const bool active = w_first < nrows;
+    const int p0 = pos[r64], pl = pos[rs + nrows - 1];
+    const int wp_first = active ? pos[rs + w_first] : 0, wp_hi = active ? pos[rs + w_last] : -1;
+    const int lo_t = hb_win_start(w, p0), kept = w.keep < lo_t ? w.keep : lo_t, nkt = (kept + 63) >> 6;
+    const int ntiles = nkt + ((pl - lo_t + 64) >> 6);
+    const int wlo_first = hb_win_start(w, wp_first), wlo_hi = active ? hb_win_start(w, wp_hi) : 0;
+    const int* pt = ptab + (size_t)rq * pts;
+    const float zmul = scale * LOG2E;
+    const int r_in = (wv * 16 + col) >> hsh, h = g * hpg + ((wv * 16 + col) & (hpg - 1));
+    const bool rowok = r_in < nrows;
+    const int row = rs + (rowok ? r_in : nrows - 1);      // (a column without a row follows the last one)
+    const int p = pos[row], lo_r = hb_win_start(w, p);
+    // tiles: this lane's rows of a tile are wv * 16 + i * RPI + lane / PP, its piece lane % PP of each holds another one of the row
+    const int psh = __builtin_ctz(ps), kr = lane / PP, slot = lane % PP;
+    const unsigned ld = (unsigned)G * RB;                  // bytes from a token's row to the next one's
+    const char *kb = (const char*)cache + (size_t)g * RB, *vb = (const char*)(cache + v_base) + (size_t)g * RB;
+    unsigned kpc[NI], vpc[NI];
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+        const int key = wv * 16 + i * RPI + kr;
+        kpc[i] = 16u * (slot ^ (D == 128 ? key & 15 : (key >> 1) & 7));
+        vpc[i] = 16u * (((slot >> 1) ^ (D == 128 ? key & 7 : (key >> 1) & 3)) * 2 + (slot & 1));
+    }
+    const int key0 = wv * 16 + kr;
+    int page[NI], off[NI];
+    auto locate = [&](int c) {                             // where the lane's rows of tile c lie (rows past its end repeat the last one: weight 0)
+        const int base = c < nkt ? c * 64 : lo_t + (c - nkt) * 64, end = c < nkt ? kept : pl + 1;
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            int tk = base + i * RPI + key0;
+            tk = tk < end ? tk : end - 1;
+            const int pg = NEAR ? tk >> psh : tk / ps;
+            off[i] = NEAR ? tk & (ps - 1) : tk - pg * ps;
+            page[i] = pt[pg];
+        }
+    };
+    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem_w + wv * 16 * RB;
+    auto request = [&](int stage) {
+        const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * 2 * TILE);
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+            if constexpr (NEAR) {
+                const unsigned r = (unsigned)(page[i] << psh | off[i]) * ld;
+                lds_dma16(kb, r + kpc[i], ls + i * 1024);
+                lds_dma16(vb, r + vpc[i], ls + TILE + i * 1024);
+            } else {
+                const size_t r = ((size_t)page[i] * ps + off[i]) * ld;
+                lds_dma16(kb + r + kpc[i], ls + i * 1024);
+                lds_dma16(vb + r + vpc[i], ls + TILE + i * 1024);
+            }
+        }
+    };
+    locate(0);
+    uint4 qh[KS], ql[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) {
+        const float* src = q + (size_t)row * ldq + (size_t)h * D + ks * 32 + g4 * 8;
+        const float4 a = *(const float4*)src, b = *(const float4*)(src + 4);
+        const float v[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+        hb_split_bf16x8(v, qh[ks], ql[ks]);
+    }
+    request(0);
+    if (ntiles > 1) locate(1);
+    hb_f32x4 oacc[CT];
+    float m = LOWEST, l = 0.f;         // running maximum of the column (log2 units), the lane's share of its sum
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) oacc[ct] = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int c = 0; c < ntiles; ++c) {
+        const bool early = c < nkt;                  // a tile of kept tokens: every row sees those below `kept`
+        const int base = early ? c * 64 : lo_t + (c - nkt) * 64;
+        // tile c has landed for every wave, and nobody reads the other stage any more
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (c + 1 < ntiles) {
+            request((c + 1) & 1);
+            if (c + 2 < ntiles) locate(c + 2);
+        }
+        // (a wave whose rows see no key of the tile)
+        if (!active || (!early && (base > wp_hi || (base + 63 < wlo_first && base >= w.keep)))) continue;
+        const char *kt_s = smem_w + (c & 1) * 2 * TILE, *vt_s = kt_s + TILE;
+        hb_f32x4 st[4];
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt) st[kt] = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+            uint4 a[4];
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+                a[kt] = *(const uint4*)(kt_s + (kt * 16 + col) * RB + 16 * ((ks * 4 + g4) ^ (D == 128 ? col : col >> 1)));
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) st[kt] = hb_mfma_bf16(a[kt], qh[ks], st[kt]);
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) st[kt] = hb_mfma_bf16(a[kt], ql[ks], st[kt]);
+        }
+        // lane (col, g4) holds the scores of column `col` against keys base + kt*16 + g4*4 + i
+        const bool full = early ? base + 63 < kept : (base + 63 <= wp_first && base >= wlo_hi);     // every row of the wave sees the whole tile
+        float z[4][4], top = LOWEST;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float s = st[kt][i] * zmul;
+                if (!full) {
+                    const int key = base + kt * 16 + g4 * 4 + i;
+                    const bool see = early ? key < kept : key <= p && (key >= lo_r || key < w.keep);
+                    s = see ? s : -INFINITY;
+                }
+                z[kt][i] = s;
+                top = fmaxf(top, s);
+            }
+        top = hb_col_max(top);
+        if (__ballot(top > m)) {
+            const float mn = fmaxf(m, top), alpha = __builtin_amdgcn_exp2f(m - mn);
+            m = mn;
+            l *= alpha;
+#pragma unroll
+            for (int ct = 0; ct < CT; ++ct)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) oacc[ct][i] *= alpha;
+        }
+        float sum = 0.f;
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                z[kt][i] = __builtin_amdgcn_exp2f(z[kt][i] - m);
+                sum += z[kt][i];
+            }
+        l += sum;
+        uint4 ph[2], plo[2];
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const float v[8] = {z[2 * kk][0], z[2 * kk][1], z[2 * kk][2], z[2 * kk][3], z[2 * kk + 1][0], z[2 * kk + 1][1], z[2 * kk + 1][2],
+                                z[2 * kk + 1][3]};
+            hb_split_bf16x8(v, ph[kk], plo[kk]);
+        }
+        // O^T[dim][column] += V^T[dim][key] P[key][column]: keys kk*32 + g4*4 + 0..3 and 16 above, in the order in which a lane holds its weights
+#pragma unroll
+        for (int kk = 0; kk < 2; ++kk) {
+            const int key = kk * 32 + g4 * 4 + (col >> 2);
+            const char* vr = vt_s + key * RB + (col & 3) * 8;
+            const int sw0 = D == 128 ? key & 7 : (key >> 1) & 3;      // (the same for key + 16)
+#pragma unroll
+            for (int half_ct = 0; half_ct < CT; half_ct += 4) {
+                uint4 a[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const char* v0 = vr + 32 * ((half_ct + e) ^ sw0);
+                    union { hb_i16x4 v[2]; uint4 u; } x;
+                    x.v[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) hb_i16x4*)v0);
+                    x.v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) hb_i16x4*)(v0 + 16 * RB));
+                    a[e] = x.u;
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) oacc[half_ct + e] = hb_mfma_bf16(a[e], ph[kk], oacc[half_ct + e]);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) oacc[half_ct + e] = hb_mfma_bf16(a[e], plo[kk], oacc[half_ct + e]);
+            }
+        }
+    }
+    float den = l, f = out_scale;
+    den += __shfl_xor(den, 16, 64);
+    den += __shfl_xor(den, 32, 64);
+    if (!rowok) return;
+    if (sink.on) {
+        const float sk = hb_sink_of(sink, h) * LOG2E, mm = fmaxf(m, sk), a = __builtin_amdgcn_exp2f(m - mm);
+        den = fmaf(den, a, __builtin_amdgcn_exp2f(sk - mm));
+        f *= a;
+    }
+    f /= den;
+    const size_t o = (size_t)row * ldo + (size_t)h * D;
+    const float* gr = gate ? gate + (size_t)row * ldg + (size_t)h * D : nullptr;
+#pragma unroll
+    for (int ct = 0; ct < CT; ++ct) {
+        const int cc = ct * 16 + g4 * 4;
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) y[i] = oacc[ct][i] * f;
+        if (gr) {
+            const float4 gv = *(const float4*)(gr + cc);
+            y[0] *= hb_sigmoid(gv.x); y[1] *= hb_sigmoid(gv.y); y[2] *= hb_sigmoid(gv.z); y[3] *= hb_sigmoid(gv.w);
+        }
+        if (out16) *(uint2*)(out16 + o + cc) = make_uint2(pack_bf2(y[0], y[1]), pack_bf2(y[2], y[3]));
+        else *(float4*)(out + o + cc) = make_float4(y[0], y[1], y[2], y[3]);
+    }
+}
+
 // ---- routed feed-forward --------------------------------------------------------------------------------------------------
 // One block per row: router logits z_j = router[j] . h in fp32 (lane-strided sums over four waves and a butterfly: an order fixed by
 // the width, the same for every step shape), then one wave: s = softmax(z) over all nE router outputs, choice = s + correction, the `top` largest choices (first
@@ -4967,9 +5195,23 @@ static int hb_sig_attention(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* 
 
 // The matrix-core window attention for steps of many rows over a bf16 cache.  false: the sizes do not fit it (head dims that are no
 // multiple of 8, or above 256).
+// o16 != NULL: the rows may be left as bf16 there instead of in out; says so in *as16
 static bool hb_try_win_mfma(hipStream_t st, const vox_hybrid_io* io, const vox_hybrid_layer& L, const bf16_t* cache, const float* q, long ldp,
-                            float* out, long ldo, const hb_sink& sink, const float* gate, long v_base, int n, int n_req, int ps) {
+                            float* out, long ldo, const hb_sink& sink, const float* gate, long v_base, int n, int n_req, int ps, bf16_t* o16, bool* as16) {
     if ((L.dim & 7) || (L.vdim & 7) || L.dim > 256 || L.vdim > 256 || (ldp & 3) || ((size_t)q & 15) || ((size_t)cache & 15)) return false;
+    const int hpg = L.heads / L.kv_heads;
+    // a lane's whole row pieces, heads that fill a block's columns: the form that loads a tile for all of them
+    if (L.dim == L.vdim && (L.dim == 64 || L.dim == 128) && (hpg & (hpg - 1)) == 0 && hpg <= 64 && (ldo & 3) == 0 && ((size_t)out & 15) == 0 && ((size_t)gate & 15) == 0) {
+        const int hsh = __builtin_ctz(hpg), br = 64 >> hsh, lds = 2 * 2 * 64 * L.dim * 2;
+        const dim3 g2(L.kv_heads, (n + (br - 1) * n_req) / br);       // (at least the sum of the requests' tiles)
+        const bool near = (ps & (ps - 1)) == 0 && (size_t)v_base * 2 < (1ull << 32);      // (v_base: what the keys take, and the values)
+        auto kern = L.dim == 128 ? (near ? k_hb_win_attn_dma<128, true> : k_hb_win_attn_dma<128, false>) :
+                                   (near ? k_hb_win_attn_dma<64, true> : k_hb_win_attn_dma<64, false>);
+        *as16 = o16 != nullptr;
+        hipLaunchKernelGGL(kern, g2, dim3(256), lds, st, q, ldp, cache, out, o16, ldo, io->pos, io->req_rows, n_req, io->page_table, io->pt_stride,
+                           L.kv_heads, hsh, ps, v_base, hb_win{L.window, L.keep_first}, L.scale, sink, gate, ldp, L.out_scale, g2.x * g2.y <= 2 * 256 ? 1 : 0);
+        return true;
+    }
     const int ks_n = (L.dim + 31) / 32, ct_n = (L.vdim + 15) / 16;
     const size_t lds = (size_t)64 * (ks_n * 32 + 8) * 2 + (size_t)ct_n * 16 * HB_SIG_VLD * 2;
     const dim3 grid(L.heads, (n + 63 * n_req) / 64), block(256);      // (at least the sum of the requests' tiles)
@@ -4987,19 +5229,19 @@ static bool hb_try_win_mfma(hipStream_t st, const vox_hybrid_io* io, const vox_h
     return true;
 }
 static bool hb_try_win_mfma(hipStream_t, const vox_hybrid_io*, const vox_hybrid_layer&, const float*, const float*, long, float*, long, const hb_sink&,
-                            const float*, long, int, int, int) { return false; }
+                            const float*, long, int, int, int, bf16_t*, bool*) { return false; }
 // keys a position can see at most
 static int hb_win_keys(const vox_hybrid_layer& L, int max_kvlen) {
     return L.window > 0 && L.window < max_kvlen - L.keep_first ? L.window + L.keep_first : max_kvlen;
 }
 template <typename T>
 static int hb_win_attention(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const vox_hybrid_layer& L, const T* cache, long ldp, int n, int n_req,
-                            int max_kvlen, long v_base) {
+                            int max_kvlen, long v_base, bf16_t* o16, bool* as16) {
     const int H = L.heads, G = L.kv_heads, ps = m->cfg.page_size, n_mix = H * L.vdim;
     const hb_sink sink{L.sinks ? 1 : 0, L.sinks};
     const float* gate = L.out_gate ? m->proj + H * L.dim + (L.kv_shared ? 0 : G * (L.dim + L.vdim)) : nullptr;
     const bool few = n <= HB_ATTN_SEG_ROWS;
-    if (!few && hb_try_win_mfma(st, io, L, cache, m->proj, ldp, m->mix, (long)n_mix, sink, gate, v_base, n, n_req, ps)) return VOX_OK;
+    if (!few && hb_try_win_mfma(st, io, L, cache, m->proj, ldp, m->mix, (long)n_mix, sink, gate, v_base, n, n_req, ps, o16, as16)) return VOX_OK;
     const int hpb = hb_sig_heads(L);
     const int nchunks = (hb_win_keys(L, max_kvlen) + 63) / 64;
     const int want = few ? (nchunks < HB_SIG_MAX_SEG ? nchunks : HB_SIG_MAX_SEG) : 1, cpb = (nchunks + want - 1) / want, nseg = (nchunks + cpb - 1) / cpb;
@@ -5041,6 +5283,9 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
     const vox_hybrid_config& c = m->cfg;
     const int W = c.width, ps = c.page_size;
     const int n_in = hb_layer_in(L), n_proj = hb_layer_proj(L), n_mix = L.heads * L.vdim;
+    // a mixer may leave its rows rounded to bf16 here for the closing product, when that one would round them itself
+    bf16_t* const mix16 = hb_takes16((const T*)L.w_out, m->ws16, n, W, n_mix) ? m->ws16.p : nullptr;
+    bool mix_as16 = false;
     jn.scale = L.ls1;
     if (L.res_gate) { jn.gate = m->proj + n_in - L.res_gate; jn.ldg = n_proj; }
     if (L.kind == VOX_MIXER_SHIFT_DECAY) {
@@ -5286,7 +5531,7 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
         const long v_base = (long)c.max_pages * ps * G * L.dim;
         hipLaunchKernelGGL((k_hb_win_prep<T>), dim3(n, L.kv_shared ? 1 : 3), dim3(256), 0, st, m->proj, (long)n_proj, (T*)cache, L.q_norm, L.k_norm,
                            L.inv_freq, L.rot_mag != 0.f ? L.rot_mag : 1.0f, io->pos, io->page, io->slot, H, G, L.dim, L.vdim, L.rot_dims, ps, v_base, c.eps);
-        VOX_TRY(hb_win_attention<T>(m, st, io, L, (const T*)cache, (long)n_proj, n, n_req, max_kvlen, v_base));
+        VOX_TRY(hb_win_attention<T>(m, st, io, L, (const T*)cache, (long)n_proj, n, n_req, max_kvlen, v_base, mix16, &mix_as16));
     } else if (L.kind == VOX_MIXER_SIGMOID_ATTN) {
         const int H = L.heads, G = L.kv_heads;
         const long v_base = (long)c.max_pages * ps * G * L.dim;
@@ -5346,7 +5591,7 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
             hipLaunchKernelGGL(hb_merge_kernel(L.vdim), dim3(n, H), dim3(64), 0, st, m->attn_ws, nseg, m->mix, (long)n_mix, io->pos, H, L.vdim, window, P,
                                HB_ATTN_SEG, gate, (long)n_proj, L.out_scale, 64, sink, 0, 0);
     }
-    return hb_gemm_resid<T>(m->ws16, st, m->mix, n_mix, (const T*)L.w_out, nullptr, cur, ldx, n, W, n_mix, jn);
+    return hb_gemm_resid<T>(m->ws16, st, m->mix, n_mix, (const T*)L.w_out, nullptr, cur, ldx, n, W, n_mix, jn, mix_as16 ? mix16 : nullptr);
 }
 
 // Routed feed-forward of the rows h2 (first completed by `post` when it names a sublayer's output), added to cur.  Few rows: one GEMV pair per routed entry; more: the entries are
