@@ -108,3 +108,51 @@ def test_window_attention_heads_of_a_key_head_together(heads, kv, dim, page, win
     finally:
         d.close()
     assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR
+
+
+# 2 to 16 rows: units of a dense layer in one launch each (the halves of the inner width: one round of requests, one step into the second; nine rows
+# and an inner width that is no multiple of 64 go on in the general product), routed layers with all experts in one tile, a last tile with one expert,
+# more experts than are summed at a time, all rows on every expert
+@pytest.mark.parametrize("rows,mlp", [(2, P.dense(64)), (8, P.dense(4096)), (7, P.dense(4224)), (9, P.dense(4224)), (5, P.dense(104)), (16, P.dense(2080)),
+                                      (2, P.moe(2, 2, 64, 0, 0)), (8, P.moe(3, 1, 2048, 0, 0)), (7, P.moe(5, 5, 2112, 0, 0)), (8, P.moe(48, 6, 128, 4, 2)),
+                                      (3, P.moe(48, 16, 64, 0, 0)), (6, P.moe(8, 2, 96, 0, 0))])
+def test_few_row_units(rows, mlp):
+    test_activation_behind_both_products(rows, mlp)
+
+
+# ... beside a layer whose choices include outputs without an expert, and one whose weights multiply an expert's input
+@pytest.mark.parametrize("rows", [2, 8])
+@pytest.mark.parametrize("over", [dict(identity=5), dict(scale_input=True)])
+def test_few_row_routed_forms(rows, over):
+    import dataclasses
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.moe(6, 3, 64, 0, 0))], width=64, vocab=50)
+    base = kazozen.config_from_dict(cfg)
+    layer = base.layers[-1]
+    d = dataclasses.replace(base, layers=[*base.layers[:-1], dataclasses.replace(layer, moe=dataclasses.replace(layer.moe, **over))])
+    W = kazozen.pack_weights(P.random_checkpoint(cfg, seed=3), base)
+    n_out = layer.moe.experts + d.layers[-1].moe.identity
+    g = torch.Generator().manual_seed(1)
+    for k in list(W):
+        if "router" in k and W[k].dim() == 2:
+            W[k] = torch.randn(n_out, W[k].shape[1], generator=g)
+        elif "correction" in k:
+            W[k] = torch.zeros(n_out)
+    toks = torch.randint(0, 50, (9,), generator=g, dtype=torch.int32)
+
+    def logits(cuts):
+        eng = HybridEngine(d, W, dtype=torch.bfloat16, max_batch=1, page_size=16, max_pages=2, max_seq_len=32, max_prefill_rows=16, max_out=16)
+        out, at = [], 0
+        try:
+            for n in cuts:
+                eng.row_ids[:n, 0] = toks[at: at + n].cuda()
+                eng.upload_plan(pos=range(at, at + n), kvlen=range(at + 1, at + n + 1), page=[0] * n, slot=range(at, at + n), q_req=[0] * n, last_rows=list(range(n)),
+                                indptr=[0, 1], indices=[0], req_rows=[0, n], state=[0])
+                eng.step(n, 1, n, sample=False, max_kvlen=at + n)
+                out.append(eng.out_logits[:n].float().cpu().clone())
+                at += n
+        finally:
+            eng.close()
+        return torch.cat(out)
+    # one row at a time takes each entry's vectors apart; the bar is that of the other bf16 comparisons
+    err = U.rel_err(logits([rows]), logits([1] * rows))
+    assert err < BF16_BAR, err

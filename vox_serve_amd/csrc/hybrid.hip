@@ -4897,6 +4897,233 @@ __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, cons
     }
 }
 
+// ---- 2 to 16 rows, bf16: gate and up rows with their activation; down rows of up to 8 rows, dense or routed ----------------------------
+// The routed entries of a step: entry row*top + k uses expert sel[.]; at most 64 entries, one a lane.
+struct hb_entries {
+    const int* sel;
+    const float* wgt;
+    int top, experts, scale_input;
+};
+// y = hb_glu(A . Wg^T + b, A . Wu^T + b): k_hb_gemm_rows16's product and sums on a tile of eight gate and the same eight up columns, so the
+// activation is in its epilogue.  ROUTED: block (columns, entry); the first entry of an expert takes all of that expert's (each weight is read once a
+// step), the blocks of the others end at once.  out: rows (entries) of ldo elements, bf16 where out16.
+// Bound by the weights' way from memory.  8 rows, 2048 wide, us: dense 11264 x 2048 (46 MB) 15.4 + 4.8 for the activation's own launch -> 16.0; routed, 16
+// choices among 8 experts of 2048 (up to 134 MB of distinct rows, 268 with each entry reading its own) 38.7 -> 27.8.  Rows without an entry
+// read row 0 (loads that only some lanes make: 36 instead of 28).  Column tiles walked by one block, with the next tile's weights asked for
+// ahead and the rows kept: 32 - 57, the registers leave too few blocks.
+template <bool ROUTED>
+__global__ __launch_bounds__(512) void k_hb_glu_rows(const float* A, long lda, const bf16_t* Wt, const float* bias, void* out, long ldo, int out16, int M, int ff,
+                                                     int K, hb_glu_args glu, hb_entries en) {
+    __shared__ float red[8][16][17];
+    __shared__ int ent[16];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
+    unsigned long long left = 0;
+    int cnt = M;
+    if (ROUTED) {
+        const int ne = M * en.top, e = en.sel[blockIdx.y];
+        if (e >= en.experts) return;
+        left = __ballot(lane < ne && en.sel[lane < ne ? lane : 0] == e);
+        if (__builtin_ctzll(left) != (int)blockIdx.y) return;
+        cnt = __popcll(left);
+        Wt += (size_t)e * 2 * ff * K;
+    }
+    const int n0 = blockIdx.x * 8, n = n0 + (col & 7), nsteps = K >> 5;
+    const bf16_t* wrow = Wt + ((size_t)(col >> 3) * ff + (n < ff ? n : ff - 1)) * K + kb * 8;
+    const int orow = threadIdx.x >> 3, oc = threadIdx.x & 7;
+    for (int done = 0; done < cnt; done += 16) {      // (an expert has an entry of a row once; more than 16 only where scores are no numbers)
+        const bool rowok = col < cnt - done;
+        int entry = rowok ? col : 0;
+        if (ROUTED) {
+            entry = 0;
+            for (int i = 0; i < 16 && left; ++i, left &= left - 1)
+                if (i == col) entry = __builtin_ctzll(left);
+        }
+        if (threadIdx.x < 16) ent[col] = entry;
+        const int arow_i = ROUTED ? entry / en.top : entry;
+        const float* arow = A + (size_t)arow_i * lda + kb * 8;
+        const float xs = ROUTED && en.scale_input ? en.wgt[entry] : 1.0f;
+        hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+        constexpr int U = 8;
+        for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
+            uint4 wf[U];
+            float4 a0[U], a1[U];
+#pragma unroll
+            for (int u = 0; u < U; ++u) wf[u] = *(const uint4*)(wrow + ((s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5));
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const int k = (s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5;
+                a0[u] = *(const float4*)(arow + k);
+                a1[u] = *(const float4*)(arow + k + 4);
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (s0 + 8 * u >= nsteps) break;
+                union { uint4 q; hb_bf16x8 b; } af, bfv;      // (tile rows without an entry are never read)
+                af.q.x = pack_bf2(a0[u].x * xs, a0[u].y * xs); af.q.y = pack_bf2(a0[u].z * xs, a0[u].w * xs);
+                af.q.z = pack_bf2(a1[u].x * xs, a1[u].y * xs); af.q.w = pack_bf2(a1[u].z * xs, a1[u].w * xs);
+                bfv.q = wf[u];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af.b, bfv.b, acc, 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[wv][kb * 4 + r][col] = acc[r];
+        __syncthreads();
+        if (threadIdx.x < 128 && orow < cnt - done && n0 + oc < ff) {
+            float g = red[0][orow][oc], u = red[0][orow][8 + oc];
+#pragma unroll
+            for (int w = 1; w < 8; ++w) { g += red[w][orow][oc]; u += red[w][orow][8 + oc]; }
+            const float y = hb_glu(g + (bias ? bias[n0 + oc] : 0.f), u + (bias ? bias[ff + n0 + oc] : 0.f), glu.limit, glu.alpha, glu.up_offset, glu.gelu);
+            const size_t o = (size_t)ent[orow] * ldo + n0 + oc;
+            if (out16) ((bf16_t*)out)[o] = f2bf(y);
+            else ((float*)out)[o] = y;
+        }
+        if (ROUTED) __syncthreads();
+    }
+}
+// The product behind it for up to 8 rows: x joins sum_k wgt_k * (identity ? h : down_{e_k} . act_k) (ROUTED, k ascending) or down . act + b.  A block owns
+// eight output columns; an MFMA tile is two segments of eight rows and those columns, of which the two squares on its diagonal are read: two of
+// the step's distinct experts, or (dense) the two halves of K.  The eight waves take a segment's k-steps w, w + 8, ..., with the next
+// eight asked for before these are multiplied; a wave walks all segments without a barrier, the partial sums wait in LDS (SEGS segments at a time).
+// Sixteen columns a block would leave every second CU without one at 2048 columns, and with an expert to a block the sum over k takes a
+// further launch.  8 rows, us: 2048 x 5632 (23 MB) 15.0 -> 11.5; 2048 x 2048, 16 choices among 8 experts (67 MB) 22.0 -> 15.9.
+template <bool ROUTED>
+__global__ __launch_bounds__(512) void k_hb_down_rows8(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, const float* h, long ldh, float* C, long ldc,
+                                                       int M, int N, int K, hb_join join, hb_entries en) {
+    constexpr int SEGS = ROUTED ? 16 : 2, U = 8;
+    __shared__ float red[SEGS / 2][8][128];
+    __shared__ float eo[ROUTED ? 64 : 2][64];            // segment, [row][column]
+    __shared__ int s_expert[64], s_sel[64], s_seg[64], s_entry[ROUTED ? 64 * 8 : 1];
+    __shared__ float s_wgt[64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, kb = lane >> 4, half = col >> 3, c8 = col & 7;
+    const int n0 = blockIdx.x * 8, n = n0 + c8 < N ? n0 + c8 : N - 1, ne = ROUTED ? M * en.top : 0;
+    int nd = 2;
+    if (ROUTED) {
+        const int s = lane < ne ? en.sel[lane] : en.experts;
+        if (wv == 0) { s_sel[lane] = s; s_wgt[lane] = lane < ne ? en.wgt[lane] : 0.f; }
+        unsigned long long todo = __ballot(s < en.experts);
+        for (nd = 0; todo; ++nd) {      // distinct experts in the order of their first entry
+            const int e = __builtin_amdgcn_readlane(s, __builtin_ctzll(todo));
+            if (tid == 0) s_expert[nd] = e;
+            if (wv == 0 && s == e) s_seg[lane] = nd;
+            todo &= ~__ballot(s == e);
+        }
+        __syncthreads();
+        // the entry of row i % 8 for segment i / 8; a row without one reads any of them (its sums are never used: loads that only some lanes make cost
+        // more than they save)
+        for (int i = tid; i < nd * 8; i += 512) {
+            int at = 0;
+            if ((i & 7) < M)
+                for (int k = en.top - 1; k >= 0; --k)
+                    if (s_sel[(i & 7) * en.top + k] == s_expert[i >> 3]) at = (i & 7) * en.top + k;
+            s_entry[i] = at;
+        }
+        __syncthreads();
+    }
+    const int ks = ROUTED ? K : K >> 1, nsteps = ks >> 5, chunks = (nsteps + 8 * U - 1) / (8 * U);
+    const int orow = tid >> 3, oc = tid & 7;
+    const bool mine = tid < 64 && orow < M && n0 + oc < N;
+    hb_join_in jin;
+    if (mine) jin = hb_join_load(join, C + (size_t)orow * ldc, orow, n0 + oc);
+    for (int d0 = 0; d0 < nd; d0 += SEGS) {
+        const int pairs = ((nd - d0 < SEGS ? nd - d0 : SEGS) + 1) >> 1, total = pairs * chunks;
+        const bf16_t *wrow = nullptr, *arow = nullptr;
+        // eight steps of the chunk i = pair * chunks + chunk
+        auto load = [&](int i, uint4 (&wf)[U], uint4 (&af)[U]) {
+            const int pr = i / chunks, s0 = (i - pr * chunks) * 8 * U + wv;
+            if (i == pr * chunks) {
+                const int d = d0 + 2 * pr + half < nd ? d0 + 2 * pr + half : nd - 1;
+                const int row = ROUTED ? s_entry[d * 8 + c8] : c8 < M ? c8 : 0;
+                wrow = Wt + (ROUTED ? ((size_t)s_expert[d] * N + n) * K : (size_t)n * K + (size_t)half * ks) + kb * 8;
+                arow = A + (size_t)row * lda + (ROUTED ? 0 : (size_t)half * ks) + kb * 8;
+            }
+#pragma unroll
+            for (int u = 0; u < U; ++u) wf[u] = *(const uint4*)(wrow + ((s0 + 8 * u < nsteps ? s0 + 8 * u : 0) << 5));
+#pragma unroll
+            for (int u = 0; u < U; ++u) af[u] = *(const uint4*)(arow + ((s0 + 8 * u < nsteps ? s0 + 8 * u : 0) << 5));
+        };
+        hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+        auto multiply = [&](int i, const uint4 (&wf)[U], const uint4 (&af)[U]) {
+            const int pr = i / chunks, s0 = (i - pr * chunks) * 8 * U + wv;
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                if (s0 + 8 * u >= nsteps) break;
+                union { uint4 q; hb_bf16x8 b; } a, w;
+                a.q = af[u];
+                w.q = wf[u];
+                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, w.b, acc, 0, 0, 0);
+            }
+            if (i - pr * chunks == chunks - 1) {
+                if ((kb >> 1) == half)
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) red[pr][wv][(kb * 4 + r) * 8 + c8] = acc[r];
+                acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        };
+        uint4 w0[U], a0[U], w1[U], a1[U];
+        load(0, w0, a0);
+        for (int i = 0; i < total; i += 2) {
+            if (i + 1 < total) load(i + 1, w1, a1);
+            multiply(i, w0, a0);
+            if (i + 2 < total) load(i + 2, w0, a0);
+            if (i + 1 < total) multiply(i + 1, w1, a1);
+        }
+        __syncthreads();
+        for (int i = tid; i < pairs * 128; i += 512) {
+            const int pr = i >> 7, d = d0 + 2 * pr + (i >> 6 & 1);
+            float v = red[pr][0][i & 127];
+#pragma unroll
+            for (int w = 1; w < 8; ++w) v += red[pr][w][i & 127];
+            if (d < nd) eo[d][i & 63] = v;
+        }
+        __syncthreads();
+    }
+    if (!mine) return;
+    float v = 0.f;
+    if (ROUTED)
+        for (int k = 0; k < en.top; ++k) {
+            const int i = orow * en.top + k;
+            if (s_sel[i] >= en.experts) v = fmaf(s_wgt[i], h[(size_t)orow * ldh + n0 + oc], v);
+            else v = fmaf(en.scale_input ? 1.0f : s_wgt[i], eo[s_seg[i]][tid], v);
+        }
+    else v = eo[0][tid] + eo[1][tid] + (bias ? bias[n0 + oc] : 0.f);
+    hb_join_apply(join, jin, C + (size_t)orow * ldc, orow, n0 + oc, v);
+}
+static bool hb_glu_rows_ok(const float* A, long lda, const bf16_t* W, int M, int K) {
+    return M >= 2 && M <= 16 && !(K & 31) && !(lda & 3) && !((size_t)A & 15) && !((size_t)W & 15);
+}
+static bool hb_down_rows_ok(const bf16_t* W, int M, int ff) { return M <= 8 && !(ff & 63) && !((size_t)W & 15); }
+// Columns up to which a dense down product takes eight a block: a block to each CU.  8 rows, us, k_hb_gemm_rows16 and this: 2048 x 5632 15.0,
+// 11.5; 2560 x 6912 18.9, 20.3; 3072 x 8192 19.4, 21.3; 4096 x 11008 34.1, 34.8.
+#define HB_DOWN8_COLS 2048
+// Dense unit of a few rows; false: its shape is the general launches'.  *done: the down product is in it too.
+static bool hb_try_ff_rows(hipStream_t st, const float* A, long lda, const bf16_t* w_up, const float* b_up, const bf16_t* w_down, const float* b_down, float* act,
+                           float* C, long ldc, int M, int W, int ff, hb_glu_args glu, const hb_join& join, bool* done) {
+    if (!hb_glu_rows_ok(A, lda, w_up, M, W)) return false;
+    *done = W <= HB_DOWN8_COLS && hb_down_rows_ok(w_down, M, ff);
+    hipLaunchKernelGGL(k_hb_glu_rows<false>, dim3((ff + 7) / 8), dim3(512), 0, st, A, lda, w_up, b_up, (void*)act, (long)ff, *done ? 1 : 0, M, ff, W, glu,
+                       hb_entries{});
+    if (*done)
+        hipLaunchKernelGGL(k_hb_down_rows8<false>, dim3((W + 7) / 8), dim3(512), 0, st, (const bf16_t*)act, (long)ff, w_down, b_down, (const float*)nullptr, 0L, C, ldc, M,
+                           W, ff, join, hb_entries{});
+    return true;
+}
+static bool hb_try_ff_rows(hipStream_t, const float*, long, const float*, const float*, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args,
+                           const hb_join&, bool*) { return false; }
+// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.  Both products, us,
+// entry by entry and this, 8 rows with 16 choices among 8 experts: 2048 wide 60.7, 43.7; 2560 86, 63.6; 3072 125, 79; 4096 231, 103.
+static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16_t* w_gate_up, const bf16_t* w_down, float* act, float* C, long ldc, int M, int W,
+                            int ff, hb_glu_args glu, const hb_join& join, hb_entries en) {
+    if (M * en.top > 64 || en.experts < 1 || !hb_glu_rows_ok(h, ldh, w_gate_up, M, W) || !hb_down_rows_ok(w_down, M, ff)) return false;
+    hipLaunchKernelGGL(k_hb_glu_rows<true>, dim3((ff + 7) / 8, M * en.top), dim3(512), 0, st, h, ldh, w_gate_up, (const float*)nullptr, (void*)act, (long)ff, 1, M, ff, W,
+                       glu, en);
+    hipLaunchKernelGGL(k_hb_down_rows8<true>, dim3((W + 7) / 8), dim3(512), 0, st, (const bf16_t*)act, (long)ff, w_down, (const float*)nullptr, h, ldh, C, ldc, M, W, ff,
+                       join, en);
+    return true;
+}
+static bool hb_try_moe_rows(hipStream_t, const float*, long, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args, const hb_join&, hb_entries) {
+    return false;
+}
+
 __global__ void k_hb_copy_rows(const float* src, long lds_, float* dst, long ldd, int W) {
     const int row = blockIdx.x;
     for (int i = threadIdx.x; i < W; i += blockDim.x) dst[(size_t)row * ldd + i] = src[(size_t)row * lds_ + i];
@@ -5608,6 +5835,10 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
     hipLaunchKernelGGL(router, dim3(n), dim3(256), (size_t)(6 * nE + top + (E.groups > 1 ? E.groups : 0)) * 4, st, h2, ldh, E.router, E.correction, W, nE, top,
                        m->moe_sel, m->moe_wgt, E.score_kind == VOX_ROUTER_SIGMOID ? 1 : 0, E.renorm, E.router_bias, E.groups, E.keep,
                        E.weight_scale != 0.f ? E.weight_scale : 1.0f, E.group_best_two, post, post.y ? const_cast<float*>(h2) : (float*)nullptr);
+    if (n <= HB_MOE_GEMV_ROWS && !up_down && !L.res_gate && E.shared_ff == 0 &&
+        hb_try_moe_rows(st, h2, ldh, (const T*)E.w_gate_up, (const T*)E.w_down, m->moe_act, cur, ldx, n, W, ff, hb_glu_args{E.limit, E.act_alpha, E.up_offset, 0}, jn,
+                        hb_entries{m->moe_sel, m->moe_wgt, top, E.experts, E.scale_input}))
+        return VOX_OK;
     if (n <= HB_MOE_GEMV_ROWS) {
         const int per = top + (E.shared_ff > 0 ? 1 : 0), maxf = ff > E.shared_ff ? ff : E.shared_ff;
         const hb_moe_small q{m->moe_sel, m->moe_wgt, top, E.experts, ff, E.shared_ff, m->max_eff, E.limit, E.shared_limit, E.act_alpha, E.up_offset,
@@ -5729,6 +5960,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             const float* hd = parallel ? hf : m->h2;
             const float limit = L.ff_limit > 0.f ? L.ff_limit : INFINITY, alpha = L.ff_alpha != 0.f ? L.ff_alpha : 1.0f;
             const bf16_t* act16 = nullptr;      // the activations as bf16, when the products behind them left them so
+            bool whole = false;                 // the down product is done too
             if (post && n == 1 && hb_try_post_gemv<T>(st, pd, true, (const T*)L.w_up, L.b_up, m->ff_act, L.ff, W, limit, alpha, L.ff_up_offset,
                                                       L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0)) {
                 // (one row of a post-normed layer: norm, both products and the activation in one launch)
@@ -5744,7 +5976,9 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             } else {
                 if (post) hd = pd.x;
                 const int gelu = L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0;
-                if (hb_try_glu(m->ws16, st, hd, ldf, n, (const T*)L.w_up, L.b_up, m->ff_act, n, L.ff, W, (const T*)L.w_down, W, hb_plain(), 1, n, (size_t)n,
+                if (hb_try_ff_rows(st, hd, ldf, (const T*)L.w_up, L.b_up, (const T*)L.w_down, L.b_down, m->ff_act, dst, ldd, n, W, L.ff,
+                                   hb_glu_args{limit, alpha, L.ff_up_offset, gelu}, j2, &whole)) {
+                } else if (hb_try_glu(m->ws16, st, hd, ldf, n, (const T*)L.w_up, L.b_up, m->ff_act, n, L.ff, W, (const T*)L.w_down, W, hb_plain(), 1, n, (size_t)n,
                                hb_glu_args{limit, alpha, L.ff_up_offset, gelu}))
                     act16 = (const bf16_t*)m->ff_act;
                 else {
@@ -5753,7 +5987,8 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
                                        (const int*)nullptr, 0, L.ff_up_offset, gelu, 0, 0);
                 }
             }
-            VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->ff_act, L.ff, (const T*)L.w_down, L.b_down, dst, ldd, n, W, L.ff, j2, act16));
+            if (!whole)
+                VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->ff_act, L.ff, (const T*)L.w_down, L.b_down, dst, ldd, n, W, L.ff, j2, act16));
         } else if (L.ff > 0) {
             // up rows with their activation, then (a residual gate) its rows, as one product
             const int nf = L.ff + L.res_gate, epi = L.ff_act == VOX_ACT_RELU2 ? HB_EPI_RELU2 : HB_EPI_GELU;
