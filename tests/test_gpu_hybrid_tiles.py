@@ -156,3 +156,11 @@ def test_few_row_routed_forms(rows, over):
     # one row at a time takes each entry's vectors apart; the bar is that of the other bf16 comparisons
     err = U.rel_err(logits([rows]), logits([1] * rows))
     assert err < BF16_BAR, err
+
+
+# Steps of up to 32 rows, four heads of a key head at 128 dims: one and three of 16-key groups, a chunk's last key, kept tokens before the window, two
+# key heads, groups of eight heads, and (4170 keys) two chunks to a block
+@pytest.mark.parametrize("heads,kv,page,window,keep,cuts", [(4, 1, 16, 300, 0, [17, 31, 16, 1, 2]), (8, 2, 24, 70, 5, [130, 3, 32]), (8, 1, 40, 64, 70, [140, 1, 5]),
+                                                            (4, 1, 128, 5000, 0, [2080, 2080, 10])])
+def test_window_attention_of_few_rows(heads, kv, page, window, keep, cuts):
+    test_window_attention_heads_of_a_key_head_together(heads, kv, 128, page, window, keep, cuts)
