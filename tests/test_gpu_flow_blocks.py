@@ -33,3 +33,9 @@ def test_rows_around_a_tile(B, T, blocks):
         flow.close()
     assert rms(want) > 0.5 and rms(pm - pm_o.numpy()) < 1e-4 and rms(got - want.numpy()) < 1e-4
     assert np.array_equal(got[-1:], alone)          # a request's mels do not depend on its batch
+
+
+# more row tiles than six blocks each fit the chip: three column tiles a wave, with a remainder of 12 rows and with none
+@pytest.mark.parametrize("B,T,blocks", [(7, 25, 2), (8, 28, 1)])
+def test_rows_of_many_tiles(B, T, blocks):
+    test_rows_around_a_tile(B, T, blocks)

@@ -4184,8 +4184,8 @@ __global__ void k_flow_slots(int* slots, int N, int B) {
 // differs by some hundred times.
 // What one of these leaves for another (parts, the residual rows) lies in the order of the lanes, [row tile][wave][tile][lane] x 4 floats:
 // whole lines per request (as [row][256] every request touched 16 lines: k_tb_qkv 12.8 us against 8.3 with plain rows to read).
-// Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 8.3 /
-// 10.7 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 13.2 (with each product as one sum, four parts and other LayerNorm
+// Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 7.4 /
+// 9.1 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 13.2 (with each product as one sum, four parts and other LayerNorm
 // sums: 8.3 / 10.3 and 12.7).  A row's result depends on that row only.
 #define TB_C 256
 #define TB_IN 512
@@ -4257,38 +4257,39 @@ __device__ __forceinline__ void tb_layernorm(float4 (&v)[2], const float4 (&w)[2
     for (int t = 0; t < 2; ++t)
         v[t] = make_float4(v[t].x * rstd * w[t].x + b[t].x, v[t].y * rstd * w[t].y + b[t].y, v[t].z * rstd * w[t].z + b[t].z, v[t].w * rstd * w[t].w + b[t].w);
 }
-// two column tiles against the rows in pl (KB k-blocks, three terms, low terms first) as the sums of runs of RUN k-blocks
-template <int KB, int RUN>
-__device__ __forceinline__ void tb_runs(const uint4 (&wf)[2][KB], const uint4* pl, int lane, f32x4 (&acc)[KB / RUN][2]) {
+// NT column tiles against the rows in pl (KB k-blocks, three terms, low terms first) as the sums of runs of RUN k-blocks
+template <int KB, int RUN, int NT>
+__device__ __forceinline__ void tb_runs(const uint4 (&wf)[NT][KB], const uint4* pl, int lane, f32x4 (&acc)[KB / RUN][NT]) {
 #pragma unroll
     for (int i = 0; i < KB / RUN; ++i) {
-        acc[i][0] = acc[i][1] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int kb = i * RUN; kb < (i + 1) * RUN; ++kb)
 #pragma unroll
             for (int p = 2; p >= 0; --p) {
                 const uint4 x = pl[(p * KB + kb) * 64 + lane];
 #pragma unroll
-                for (int t = 0; t < 2; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[i][t], 0, 0, 0);
+                for (int t = 0; t < NT; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[i][t], 0, 0, 0);
             }
     }
 }
 // the whole product: runs of two k-blocks, added in ascending order
-template <int KB>
-__device__ __forceinline__ void tb_product(const uint4 (&wf)[2][KB], const uint4* pl, int lane, f32x4 (&acc)[2]) {
-    f32x4 r[KB / 2][2];
-    tb_runs<KB, 2>(wf, pl, lane, r);
+template <int KB, int NT>
+__device__ __forceinline__ void tb_product(const uint4 (&wf)[NT][KB], const uint4* pl, int lane, f32x4 (&acc)[NT]) {
+    f32x4 r[KB / 2][NT];
+    tb_runs<KB, 2, NT>(wf, pl, lane, r);
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int t = 0; t < NT; ++t) {
         acc[t] = r[0][t];
 #pragma unroll
         for (int i = 1; i < KB / 2; ++i) acc[t] += r[i][t];
     }
 }
-template <int KB>
-__device__ __forceinline__ void tb_weights(uint4 (&wf)[2][KB], const bf16_t* w, int tile, int kb_all, int kb0, int lane) {
+template <int KB, int NT>
+__device__ __forceinline__ void tb_weights(uint4 (&wf)[NT][KB], const bf16_t* w, int tile, int kb_all, int kb0, int lane) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
+    for (int t = 0; t < NT; ++t)
 #pragma unroll
         for (int kb = 0; kb < KB; ++kb) wf[t][kb] = *reinterpret_cast<const uint4*>(w + ((size_t)(tile + t) * kb_all + kb0 + kb) * 512 + lane * 8);
 }
@@ -4307,15 +4308,16 @@ __device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
     for (int i = 1; i < TB_PARTS; ++i) v[0] = tb_add(v[0], v[i]);
     return tb_add(v[TB_PARTS], tb_add(v[0], b2));
 }
-template <bool PARTS>
+// NT column tiles a wave, 128 NT columns a block.
+template <bool PARTS, int NT>
 __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* parts, const float* b2, size_t ps, const bf16_t* w, const float* lnw, const float* lnb,
                                                 float* qkv, float* h_out, int M, int N) {
     __shared__ uint4 pl[3 * 8 * 64];
     __shared__ float4 red[256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4;
-    const int m = blockIdx.x * 16 + fr, row = m < M ? m : M - 1, tile = (blockIdx.y * 8 + wave) * 2;
+    const int m = blockIdx.x * 16 + fr, row = m < M ? m : M - 1, tile = (blockIdx.y * 8 + wave) * NT;
     float4 v[2], lw[2], lb[2];
-    uint4 wf[2][8];
+    uint4 wf[NT][8];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int c = (wave * 2 + t) * 16 + kq * 4;
@@ -4324,7 +4326,7 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
         lw[t] = *reinterpret_cast<const float4*>(lnw + c);
         lb[t] = *reinterpret_cast<const float4*>(lnb + c);
     }
-    tb_weights<8>(wf, w, tile, 8, 0, lane);
+    tb_weights<8, NT>(wf, w, tile, 8, 0, lane);
     if (PARTS && blockIdx.y == 0)
 #pragma unroll
         for (int t = 0; t < 2; ++t) *reinterpret_cast<float4*>(h_out + tb_at(blockIdx.x, wave, t, lane)) = v[t];
@@ -4332,11 +4334,11 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
 #pragma unroll
     for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, v[t]);
     __syncthreads();
-    f32x4 acc[2];
-    tb_product<8>(wf, pl, lane, acc);
+    f32x4 acc[NT];
+    tb_product<8, NT>(wf, pl, lane, acc);
     if (m < M)
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int t = 0; t < NT; ++t)
             *reinterpret_cast<float4*>(qkv + (size_t)m * N + (tile + t) * 16 + kq * 4) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
 }
 // lane_h: h lies in lane order
@@ -4354,7 +4356,7 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
         a[i][1] = *reinterpret_cast<const float4*>(s + 4);
     }
     uint4 wo[2][16];
-    tb_weights<16>(wo, w.out, wave * 2, 16, 0, lane);
+    tb_weights<16, 2>(wo, w.out, wave * 2, 16, 0, lane);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int c = (wave * 2 + t) * 16 + kq * 4;
@@ -4373,9 +4375,9 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
     }
     __syncthreads();
     f32x4 acc[2];
-    tb_product<16>(wo, pl, lane, acc);
+    tb_product<16, 2>(wo, pl, lane, acc);
     uint4 w1[2][8], w2[2][8];
-    tb_weights<8>(w1, w.ff1, q * 16 + wave * 2, 8, 0, lane);
+    tb_weights<8, 2>(w1, w.ff1, q * 16 + wave * 2, 8, 0, lane);
     float4 x[2], n[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) n[t] = x[t] = tb_add(res[t], tb_add(make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]), bo[t]));
@@ -4383,8 +4385,8 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
 #pragma unroll
     for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, n[t]);
     __syncthreads();
-    tb_product<8>(w1, pl, lane, acc);
-    tb_weights<8>(w2, w.ff2, wave * 2, 32, q * 8, lane);
+    tb_product<8, 2>(w1, pl, lane, acc);
+    tb_weights<8, 2>(w2, w.ff2, wave * 2, 32, q * 8, lane);
     uint4* const hid = pl + 3 * 8 * 64;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -4399,7 +4401,7 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
     }
     __syncthreads();
     f32x4 y[2][2];
-    tb_runs<8, 4>(w2, hid, lane, y);
+    tb_runs<8, 4, 2>(w2, hid, lane, y);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const size_t o = tb_at(blockIdx.x, wave, t, lane);
@@ -4447,10 +4449,20 @@ static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, 
 static size_t tb_plane(size_t M) { return (M + 15) / 16 * 16 * TB_C; }      // floats of a plane of M rows
 // q | k | v of the rows into qkv (before: the block before, which has left them in ws; NULL: of h itself)
 static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* h, float* ws, const vox_flow_tblock_w* before, float* qkv, int M) {
-    const dim3 g((M + 15) / 16, 3 * TB_IN / 256);
+    const int tiles = (M + 15) / 16;
     const size_t ps = tb_plane(M);
-    if (!before) hipLaunchKernelGGL(k_tb_qkv<false>, g, dim3(512), 0, st, h, ws, nullptr, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN);
-    else hipLaunchKernelGGL(k_tb_qkv<true>, g, dim3(512), 0, st, h, ws, before->ff2.bias, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws + (TB_PLANES - 1) * ps, M, 3 * TB_IN);
+#define TB_QKV(NT_) \
+    do { \
+        const dim3 g(tiles, 3 * TB_IN / (128 * NT_)); \
+        if (!before) hipLaunchKernelGGL((k_tb_qkv<false, NT_>), g, dim3(512), 0, st, h, ws, nullptr, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN); \
+        else hipLaunchKernelGGL((k_tb_qkv<true, NT_>), g, dim3(512), 0, st, h, ws, before->ff2.bias, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws + (TB_PLANES - 1) * ps, M, \
+                                3 * TB_IN); \
+    } while (0)
+    // A block adds up its rows' planes (128 KB) whatever it multiplies them by (64 KB a tile of a wave): where two tiles a wave make more blocks than
+    // CUs, three move less.  896 rows, us (first / later blocks of a level), two, three, four tiles: 8.4 / 10.6, 7.4 / 9.1, 8.4 / 10.3.
+    if (tiles * (3 * TB_IN / 256) <= 256) TB_QKV(2);
+    else TB_QKV(3);
+#undef TB_QKV
 }
 static void tb_ff(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* att, float* h, float* ws, bool first, bool last, int M) {
     const size_t ps = tb_plane(M);
