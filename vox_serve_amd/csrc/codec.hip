@@ -3665,6 +3665,11 @@ struct FlowAttn {
     // cached keys beyond the first `prefix` rows sit in a ring that starts at ring_head (logical row j -> physical row below)
     const int* cidx;
     int prefix, ring_head;
+    // k_flow_attn_mfma<.., true>: the out projection's packed weights and the planes (one a head, ps floats apart, rows of 256) that take its sums over
+    // that head's 64 columns, in the place of `out`
+    const bf16_t* wo;
+    float* parts;
+    size_t ps;
 };
 __device__ __forceinline__ int flow_cache_row(int j, int prefix, int head, int cap) {
     return (head == 0 || j < prefix) ? j : prefix + (head + j - prefix) % (cap - prefix);
@@ -3875,6 +3880,139 @@ __global__ __launch_bounds__(256) void k_flow_attn_tile(FlowAttn a, int QG) {
         __builtin_amdgcn_wave_barrier();      // ps / qs are rewritten by the wave's next query
     }
 }
+// Parts of the estimator's fused transformer blocks (below) that their attention uses too
+#define TB_C 256
+#define TB_IN 512
+#define TB_FF 1024
+struct FlowPacked {
+    const bf16_t *qkv = nullptr, *out = nullptr, *ff1 = nullptr, *ff2 = nullptr;
+};
+// w [N][K] bf16 -> tiles of 16 rows x 32 columns (row tile major), each as the 64 lanes of an MFMA operand hold it
+__global__ __launch_bounds__(256) void k_pack_frag(const bf16_t* w, bf16_t* out, int K, size_t chunks) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i >= chunks) return;
+    const int kb_n = K >> 5, lane = (int)(i & 63);
+    const size_t tile = i >> 6, kb = tile % kb_n, rt = tile / kb_n;
+    *reinterpret_cast<uint4*>(out + i * 8) = *reinterpret_cast<const uint4*>(w + (rt * 16 + (lane & 15)) * K + kb * 32 + (lane >> 4) * 8);
+}
+struct tb_split {
+    uint2 t[3];      // four values' leading, second and third bf16 terms
+};
+__device__ __forceinline__ tb_split tb_split3(float4 v) {
+    tb_split s;
+    s.t[0] = make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
+    const float4 r = make_float4(v.x - bflo(s.t[0].x), v.y - bfhi(s.t[0].x), v.z - bflo(s.t[0].y), v.w - bfhi(s.t[0].y));
+    s.t[1] = make_uint2(pack_bf2(r.x, r.y), pack_bf2(r.z, r.w));
+    s.t[2] = make_uint2(pack_bf2(r.x - bflo(s.t[1].x), r.y - bfhi(s.t[1].x)), pack_bf2(r.z - bflo(s.t[1].y), r.w - bfhi(s.t[1].y)));
+    return s;
+}
+__device__ __forceinline__ float4 tb_add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
+// Column tile 2 wave + t of 256 columns as an operand of the next product: k-block `wave`, k group 2 t + kq / 2
+__device__ __forceinline__ void tb_put(uint4* pl, int kb_n, int wave, int t, int lane, float4 v) {
+    const tb_split s = tb_split3(v);
+    const int fr = lane & 15, kq = lane >> 4;
+    uint2* d = reinterpret_cast<uint2*>(pl + wave * 64 + (2 * t + (kq >> 1)) * 16 + fr) + (kq & 1);
+#pragma unroll
+    for (int p = 0; p < 3; ++p) d[p * kb_n * 128] = s.t[p];
+}
+// A row's sum over its 256 columns from the sums s[t] of four neighbouring ones (two per lane): eight neighbouring columns, then the two
+// 32-column blocks of a run of 64, then its four groups of eight, then the runs.  red: [8][16] x 4 floats, one for each call of a block
+__device__ __forceinline__ float tb_row_sum(float s0, float s1, float4* red, int wave, int lane) {
+    const int fr = lane & 15;
+    s0 += __shfl_xor(s0, 16, 64);
+    s1 += __shfl_xor(s1, 16, 64);
+    if (!(lane & 16)) {
+        float* d = reinterpret_cast<float*>(red + wave * 16 + fr) + (lane >> 5);
+        d[0] = s0;
+        d[2] = s1;
+    }
+    __syncthreads();
+    float tot = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const float4 a = red[2 * i * 16 + fr], b = red[(2 * i + 1) * 16 + fr];
+        const float run = ((a.x + b.x) + (a.y + b.y)) + ((a.z + b.z) + (a.w + b.w));
+        tot = i == 0 ? run : tot + run;
+    }
+    return tot;
+}
+// The same sum of a row that lies in one wave, four columns to a lane
+__device__ __forceinline__ float tb_row_sum64(float s) {
+    s += __shfl_xor(s, 1, 64);      // eight neighbouring columns
+    s += __shfl_xor(s, 8, 64);      // the two 32-column blocks of a run of 64
+    s += __shfl_xor(s, 2, 64);
+    s += __shfl_xor(s, 4, 64);
+    return ((__shfl(s, 0, 64) + __shfl(s, 16, 64)) + __shfl(s, 32, 64)) + __shfl(s, 48, 64);
+}
+// LayerNorm of the rows whose columns lie 8 to a lane (two tiles of four) over the block's eight waves; red: [2][8][16] x 4 floats
+__device__ __forceinline__ void tb_layernorm(float4 (&v)[2], const float4 (&w)[2], const float4 (&b)[2], float4* red, int wave, int lane) {
+    const float mean = tb_row_sum((v[0].x + v[0].y) + (v[0].z + v[0].w), (v[1].x + v[1].y) + (v[1].z + v[1].w), red, wave, lane) / (float)TB_C;
+    float q[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        v[t] = make_float4(v[t].x - mean, v[t].y - mean, v[t].z - mean, v[t].w - mean);
+        q[t] = (v[t].x * v[t].x + v[t].y * v[t].y) + (v[t].z * v[t].z + v[t].w * v[t].w);
+    }
+    const float var = tb_row_sum(q[0], q[1], red + 128, wave, lane);
+    const float rstd = rsqrtf(var / (float)TB_C + 1e-5f);
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+        v[t] = make_float4(v[t].x * rstd * w[t].x + b[t].x, v[t].y * rstd * w[t].y + b[t].y, v[t].z * rstd * w[t].z + b[t].z, v[t].w * rstd * w[t].w + b[t].w);
+}
+// NT column tiles against the rows in pl (KB k-blocks, three terms, low terms first) as the sums of runs of RUN k-blocks
+// (TURN: a row's place among the 16 of a k group is turned by the group, tb_turn)
+__device__ __forceinline__ int tb_turn(int kb, int g, int row) { return row ^ ((g + 4 * kb) & 15); }
+template <int KB, int RUN, int NT, bool TURN = false>
+__device__ __forceinline__ void tb_runs(const uint4 (&wf)[NT][KB], const uint4* pl, int lane, f32x4 (&acc)[KB / RUN][NT]) {
+#pragma unroll
+    for (int i = 0; i < KB / RUN; ++i) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kb = i * RUN; kb < (i + 1) * RUN; ++kb)
+#pragma unroll
+            for (int p = 2; p >= 0; --p) {
+                const uint4 x = pl[(p * KB + kb) * 64 + (TURN ? (lane & 48) + tb_turn(kb, lane >> 4, lane & 15) : lane)];
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[i][t], 0, 0, 0);
+            }
+    }
+}
+// the whole product: runs of two k-blocks, added in ascending order
+template <int KB, int NT, bool TURN = false>
+__device__ __forceinline__ void tb_product(const uint4 (&wf)[NT][KB], const uint4* pl, int lane, f32x4 (&acc)[NT]) {
+    f32x4 r[KB / 2][NT];
+    tb_runs<KB, 2, NT, TURN>(wf, pl, lane, r);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        acc[t] = r[0][t];
+#pragma unroll
+        for (int i = 1; i < KB / 2; ++i) acc[t] += r[i][t];
+    }
+}
+template <int KB, int NT>
+__device__ __forceinline__ void tb_weights(uint4 (&wf)[NT][KB], const bf16_t* w, int tile, int kb_all, int kb0, int lane) {
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb) wf[t][kb] = *reinterpret_cast<const uint4*>(w + ((size_t)(tile + t) * kb_all + kb0 + kb) * 512 + lane * 8);
+}
+// floats of column tile 2 wave + t of row tile `rt` in lane order
+__device__ __forceinline__ size_t tb_at(int rt, int wave, int t, int lane) { return ((((size_t)rt * 8 + wave) * 2 + t) * 64 + lane) * 4; }
+// Planes of a block's scratch, ps floats apart: ff2's sums (the first two eighths, then an eighth each), the residual rows behind the out product,
+// and those in front of it (the sum of the planes that the block before has left)
+#define TB_PARTS 7
+#define TB_PLANES 9
+#define TB_HEADS 8      // planes of the heads' sums of the out product behind them, rows of 256
+// rows [.][256] = residual + ((parts[0] + ... + parts[6]) + b2)
+__device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
+    float4 v[TB_PARTS + 1];
+#pragma unroll
+    for (int i = 0; i <= TB_PARTS; ++i) v[i] = *reinterpret_cast<const float4*>(p + i * ps);
+#pragma unroll
+    for (int i = 1; i < TB_PARTS; ++i) v[0] = tb_add(v[0], v[i]);
+    return tb_add(v[TB_PARTS], tb_add(v[0], b2));
+}
 // The estimators' attention on the matrix cores (no relative-position term, dk = 64, at most 256 keys: every CosyVoice2 / GLM estimator
 // call).  A block owns 16 consecutive queries of one (request, head); its WV (8) waves take the 16-key tiles w, w + WV for
 // BOTH products, so nothing but the row maxima, the row sums and the 16 x 64 partial outputs crosses a wave:
@@ -3886,13 +4024,18 @@ __global__ __launch_bounds__(256) void k_flow_attn_tile(FlowAttn a, int QG) {
 //                     are the four 16-dim output tiles (dim = 4 (l % 16) + tile), so a lane's four accumulators are one float4 of the row
 // and the partial outputs of the WV waves are summed in the fixed order w0 + w1 + ... and scaled by 1 / sum.  A (request, head, query)'s
 // result depends on that request's rows only.
-template <int DK, int WV>
+// OUT (fused transformer blocks: 8 heads, 256 channels): the block multiplies its 16 x 64 outputs by the head's 64 columns of the out projection too (32 KB of
+// weights), one of that product's eight runs of K: the feed-forward launch adds the heads' planes in order and has the product's bits without
+// its 256 KB of weights a block.  896 rows: 12.0 -> 13.8 us here, 13.1 -> 10.8 there and 9.1 -> 8.5 in the next q | k | v.  (Two query
+// tiles a block, which read each key once for both: 15.2.)
+template <int DK, int WV, bool OUT>
 __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
     static_assert(DK == 64, "operand layout below is written for 64-dim heads");
     constexpr int KT = 16 / WV, PS = KT * 16 + 4, OS = DK + 4;      // WV waves x KT key tiles of 16: at most 256 keys
     __shared__ float red_mx[WV][16], red_sum[WV][16];
     __shared__ __attribute__((aligned(16))) float Ps[WV][16][PS];
     __shared__ __attribute__((aligned(16))) float Os[WV][16][OS];
+    __shared__ uint4 pl[OUT ? 3 * 2 * 64 : 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fr = lane & 15, kq = lane >> 4;
     const int i0 = blockIdx.x * 16, h = blockIdx.y, n = blockIdx.z;
     const int HD = a.H * DK, ld = 3 * HD, S = a.Tc + a.T, nt = (S + 15) >> 4;
@@ -3951,6 +4094,8 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
             mx[r] = fmaxf(mx[r], s);
         }
     }
+    uint4 wf[OUT ? 2 : 1][2];      // (in flight while the outputs are formed)
+    if constexpr (OUT) tb_weights<2, 2>(wf, a.wo, wave * 2, 16, h * 2, lane);
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
 #pragma unroll
@@ -3999,7 +4144,7 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
         *reinterpret_cast<float4*>(&Os[wave][4 * kq + r][4 * fr]) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
     __syncthreads();
     const int qi = tid >> 4, c4 = (tid & 15) * 4;
-    if (tid < 256 && i0 + qi < a.T) {
+    if (tid < 256 && (OUT || i0 + qi < a.T)) {
         float l = red_sum[0][qi];
         float4 o4 = *reinterpret_cast<const float4*>(&Os[0][qi][c4]);
 #pragma unroll
@@ -4009,7 +4154,23 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
             o4.x += pw.x; o4.y += pw.y; o4.z += pw.z; o4.w += pw.w;
         }
         const float inv = 1.0f / l;
-        *reinterpret_cast<float4*>(a.out + ((size_t)n * a.T + i0 + qi) * HD + h * DK + c4) = make_float4(o4.x * inv, o4.y * inv, o4.z * inv, o4.w * inv);
+        o4 = make_float4(o4.x * inv, o4.y * inv, o4.z * inv, o4.w * inv);
+        if constexpr (OUT) {      // (wave = rows 4 wave .. + 3, columns 4 (lane % 16) ..)
+            const tb_split s = tb_split3(o4);
+            const int g = (tid & 15) >> 1;
+            uint2* d = reinterpret_cast<uint2*>(pl + (g >> 2) * 64 + (g & 3) * 16 + tb_turn(g >> 2, g & 3, qi)) + (tid & 1);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) d[p * 2 * 128] = s.t[p];
+        } else *reinterpret_cast<float4*>(a.out + ((size_t)n * a.T + i0 + qi) * HD + h * DK + c4) = o4;
+    }
+    if constexpr (OUT) {
+        __syncthreads();
+        f32x4 y[1][2];
+        tb_runs<2, 2, 2, true>(wf, pl, lane, y);
+        if (i0 + fr < a.T)
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+                *reinterpret_cast<f32x4*>(a.parts + h * a.ps + ((size_t)n * a.T + i0 + fr) * TB_C + (wave * 2 + t) * 16 + kq * 4) = y[0][t];
     }
 }
 // VOX_FLOW_ATTN_MFMA=0: the VALU attention kernels for every call (A/B timing)
@@ -4022,13 +4183,15 @@ static bool flow_attn_tile_on() {
     static const bool on = [] { const char* e = getenv("VOX_FLOW_ATTN_TILE"); return !(e && e[0] == '0'); }();
     return on;
 }
+static bool flow_attn_mfma_takes(const FlowAttn& a, int T) { return !a.P && !a.bu && a.dk == 64 && a.Tc + T <= 256 && flow_attn_mfma_on(); }
 static void launch_flow_attn(hipStream_t st, const FlowAttn& a, int T, int H, int N) {
     const int S = a.Tc + T;
     const size_t lds = ((size_t)S * (2 * a.dk + 4) + 4 * ((S + 3) & ~3) + 4 * a.dk) * sizeof(float);
-    if (!a.P && !a.bu && a.dk == 64 && S <= 256 && flow_attn_mfma_on()) {
+    if (flow_attn_mfma_takes(a, T)) {
         static const bool wv4 = [] { const char* e = getenv("VOX_FLOW_ATTN_WV"); return e && atoi(e) == 4; }();      // A/B: four waves x four key tiles
-        if (wv4) hipLaunchKernelGGL((k_flow_attn_mfma<64, 4>), dim3((T + 15) / 16, H, N), dim3(256), 0, st, a);
-        else hipLaunchKernelGGL((k_flow_attn_mfma<64, 8>), dim3((T + 15) / 16, H, N), dim3(512), 0, st, a);
+        if (a.parts) hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, true>), dim3((T + 15) / 16, H, N), dim3(512), 0, st, a);
+        else if (wv4) hipLaunchKernelGGL((k_flow_attn_mfma<64, 4, false>), dim3((T + 15) / 16, H, N), dim3(256), 0, st, a);
+        else hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, false>), dim3((T + 15) / 16, H, N), dim3(512), 0, st, a);
         return;
     }
     if (!a.P && a.dk == 64 && lds <= 150 * 1024 && flow_attn_tile_on()) {
@@ -4176,138 +4339,18 @@ __global__ void k_flow_slots(int* slots, int N, int B) {
 // fragment-major copy (1 KB per wave request, whole lines) straight into registers.  Products are taken transposed (weight rows x
 // activation rows): a lane then holds four neighbouring columns of one row, which is what it stores, normalises and splits.
 //   k_tb_qkv   rows = residual + feed-forward parts of the block before, LayerNorm, q | k | v: grid (row tiles, 256-column groups)
-//   k_tb_ff    attention out + residual, LayerNorm, GELU feed-forward: grid (row tiles, 4); block y owns a quarter of the hidden columns from
-//              ff1 to its two eighths of ff2's sums (they and the residual rows are added by whoever reads them); the out product is done by
-//              all four
+//   k_tb_ff    heads' sums of the out product + residual, LayerNorm, GELU feed-forward: grid (row tiles, 4); block y owns a quarter of the hidden
+//              columns from ff1 to its two eighths of ff2's sums (they and the residual rows are added by whoever reads them).  Where the attention has
+//              left its rows instead (more than 256 keys), the out product is done by all four
 // Sums, LayerNorm statistics and the order of every addition are those of the general launches (k_rows_gemm: K in four runs of 64, or in eight
 // from 512 on, added in ascending order), so the two forms give the same bits: the phase of the vocoder's source multiplies what a mel
 // differs by some hundred times.
 // What one of these leaves for another (parts, the residual rows) lies in the order of the lanes, [row tile][wave][tile][lane] x 4 floats:
 // whole lines per request (as [row][256] every request touched 16 lines: k_tb_qkv 12.8 us against 8.3 with plain rows to read).
 // Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 7.4 /
-// 9.1 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 13.2 (with each product as one sum, four parts and other LayerNorm
+// 9.1 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 10.8, with 1.8 for the out product in
+// the attention (13.1 with it here, in all four blocks of a row tile; with each product as one sum, four parts and other LayerNorm
 // sums: 8.3 / 10.3 and 12.7).  A row's result depends on that row only.
-#define TB_C 256
-#define TB_IN 512
-#define TB_FF 1024
-struct FlowPacked {
-    const bf16_t *qkv = nullptr, *out = nullptr, *ff1 = nullptr, *ff2 = nullptr;
-};
-// w [N][K] bf16 -> tiles of 16 rows x 32 columns (row tile major), each as the 64 lanes of an MFMA operand hold it
-__global__ __launch_bounds__(256) void k_pack_frag(const bf16_t* w, bf16_t* out, int K, size_t chunks) {
-    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-    if (i >= chunks) return;
-    const int kb_n = K >> 5, lane = (int)(i & 63);
-    const size_t tile = i >> 6, kb = tile % kb_n, rt = tile / kb_n;
-    *reinterpret_cast<uint4*>(out + i * 8) = *reinterpret_cast<const uint4*>(w + (rt * 16 + (lane & 15)) * K + kb * 32 + (lane >> 4) * 8);
-}
-struct tb_split {
-    uint2 t[3];      // four values' leading, second and third bf16 terms
-};
-__device__ __forceinline__ tb_split tb_split3(float4 v) {
-    tb_split s;
-    s.t[0] = make_uint2(pack_bf2(v.x, v.y), pack_bf2(v.z, v.w));
-    const float4 r = make_float4(v.x - bflo(s.t[0].x), v.y - bfhi(s.t[0].x), v.z - bflo(s.t[0].y), v.w - bfhi(s.t[0].y));
-    s.t[1] = make_uint2(pack_bf2(r.x, r.y), pack_bf2(r.z, r.w));
-    s.t[2] = make_uint2(pack_bf2(r.x - bflo(s.t[1].x), r.y - bfhi(s.t[1].x)), pack_bf2(r.z - bflo(s.t[1].y), r.w - bfhi(s.t[1].y)));
-    return s;
-}
-__device__ __forceinline__ float4 tb_add(float4 a, float4 b) { return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w); }
-// Column tile 2 wave + t of 256 columns as an operand of the next product: k-block `wave`, k group 2 t + kq / 2
-__device__ __forceinline__ void tb_put(uint4* pl, int kb_n, int wave, int t, int lane, float4 v) {
-    const tb_split s = tb_split3(v);
-    const int fr = lane & 15, kq = lane >> 4;
-    uint2* d = reinterpret_cast<uint2*>(pl + wave * 64 + (2 * t + (kq >> 1)) * 16 + fr) + (kq & 1);
-#pragma unroll
-    for (int p = 0; p < 3; ++p) d[p * kb_n * 128] = s.t[p];
-}
-// A row's sum over its 256 columns from the sums s[t] of four neighbouring ones (two per lane): eight neighbouring columns, then the two
-// 32-column blocks of a run of 64, then its four groups of eight, then the runs.  red: [8][16] x 4 floats, one for each call of a block
-__device__ __forceinline__ float tb_row_sum(float s0, float s1, float4* red, int wave, int lane) {
-    const int fr = lane & 15;
-    s0 += __shfl_xor(s0, 16, 64);
-    s1 += __shfl_xor(s1, 16, 64);
-    if (!(lane & 16)) {
-        float* d = reinterpret_cast<float*>(red + wave * 16 + fr) + (lane >> 5);
-        d[0] = s0;
-        d[2] = s1;
-    }
-    __syncthreads();
-    float tot = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const float4 a = red[2 * i * 16 + fr], b = red[(2 * i + 1) * 16 + fr];
-        const float run = ((a.x + b.x) + (a.y + b.y)) + ((a.z + b.z) + (a.w + b.w));
-        tot = i == 0 ? run : tot + run;
-    }
-    return tot;
-}
-// LayerNorm of the rows whose columns lie 8 to a lane (two tiles of four) over the block's eight waves; red: [2][8][16] x 4 floats
-__device__ __forceinline__ void tb_layernorm(float4 (&v)[2], const float4 (&w)[2], const float4 (&b)[2], float4* red, int wave, int lane) {
-    const float mean = tb_row_sum((v[0].x + v[0].y) + (v[0].z + v[0].w), (v[1].x + v[1].y) + (v[1].z + v[1].w), red, wave, lane) / (float)TB_C;
-    float q[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        v[t] = make_float4(v[t].x - mean, v[t].y - mean, v[t].z - mean, v[t].w - mean);
-        q[t] = (v[t].x * v[t].x + v[t].y * v[t].y) + (v[t].z * v[t].z + v[t].w * v[t].w);
-    }
-    const float var = tb_row_sum(q[0], q[1], red + 128, wave, lane);
-    const float rstd = rsqrtf(var / (float)TB_C + 1e-5f);
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-        v[t] = make_float4(v[t].x * rstd * w[t].x + b[t].x, v[t].y * rstd * w[t].y + b[t].y, v[t].z * rstd * w[t].z + b[t].z, v[t].w * rstd * w[t].w + b[t].w);
-}
-// NT column tiles against the rows in pl (KB k-blocks, three terms, low terms first) as the sums of runs of RUN k-blocks
-template <int KB, int RUN, int NT>
-__device__ __forceinline__ void tb_runs(const uint4 (&wf)[NT][KB], const uint4* pl, int lane, f32x4 (&acc)[KB / RUN][NT]) {
-#pragma unroll
-    for (int i = 0; i < KB / RUN; ++i) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) acc[i][t] = (f32x4){0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int kb = i * RUN; kb < (i + 1) * RUN; ++kb)
-#pragma unroll
-            for (int p = 2; p >= 0; --p) {
-                const uint4 x = pl[(p * KB + kb) * 64 + lane];
-#pragma unroll
-                for (int t = 0; t < NT; ++t) acc[i][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(wf[t][kb]), as_cbf8(x), acc[i][t], 0, 0, 0);
-            }
-    }
-}
-// the whole product: runs of two k-blocks, added in ascending order
-template <int KB, int NT>
-__device__ __forceinline__ void tb_product(const uint4 (&wf)[NT][KB], const uint4* pl, int lane, f32x4 (&acc)[NT]) {
-    f32x4 r[KB / 2][NT];
-    tb_runs<KB, 2, NT>(wf, pl, lane, r);
-#pragma unroll
-    for (int t = 0; t < NT; ++t) {
-        acc[t] = r[0][t];
-#pragma unroll
-        for (int i = 1; i < KB / 2; ++i) acc[t] += r[i][t];
-    }
-}
-template <int KB, int NT>
-__device__ __forceinline__ void tb_weights(uint4 (&wf)[NT][KB], const bf16_t* w, int tile, int kb_all, int kb0, int lane) {
-#pragma unroll
-    for (int t = 0; t < NT; ++t)
-#pragma unroll
-        for (int kb = 0; kb < KB; ++kb) wf[t][kb] = *reinterpret_cast<const uint4*>(w + ((size_t)(tile + t) * kb_all + kb0 + kb) * 512 + lane * 8);
-}
-// floats of column tile 2 wave + t of row tile `rt` in lane order
-__device__ __forceinline__ size_t tb_at(int rt, int wave, int t, int lane) { return ((((size_t)rt * 8 + wave) * 2 + t) * 64 + lane) * 4; }
-// Planes of a block's scratch, ps floats apart: ff2's sums (the first two eighths, then an eighth each), the residual rows behind the out product,
-// and those in front of it (the sum of the planes that the block before has left)
-#define TB_PARTS 7
-#define TB_PLANES 9
-// rows [.][256] = residual + ((parts[0] + ... + parts[6]) + b2)
-__device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
-    float4 v[TB_PARTS + 1];
-#pragma unroll
-    for (int i = 0; i <= TB_PARTS; ++i) v[i] = *reinterpret_cast<const float4*>(p + i * ps);
-#pragma unroll
-    for (int i = 1; i < TB_PARTS; ++i) v[0] = tb_add(v[0], v[i]);
-    return tb_add(v[TB_PARTS], tb_add(v[0], b2));
-}
 // NT column tiles a wave, 128 NT columns a block.
 template <bool PARTS, int NT>
 __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* parts, const float* b2, size_t ps, const bf16_t* w, const float* lnw, const float* lnb,
@@ -4329,7 +4372,7 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
     tb_weights<8, NT>(wf, w, tile, 8, 0, lane);
     if (PARTS && blockIdx.y == 0)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) *reinterpret_cast<float4*>(h_out + tb_at(blockIdx.x, wave, t, lane)) = v[t];
+        for (int t = 0; t < 2; ++t) *reinterpret_cast<float4*>(h_out + (size_t)(blockIdx.x * 16 + fr) * TB_C + (wave * 2 + t) * 16 + kq * 4) = v[t];
     tb_layernorm(v, lw, lb, red, wave, lane);
 #pragma unroll
     for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, v[t]);
@@ -4341,52 +4384,91 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
         for (int t = 0; t < NT; ++t)
             *reinterpret_cast<float4*>(qkv + (size_t)m * N + (tile + t) * 16 + kq * 4) = make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]);
 }
-// lane_h: h lies in lane order
-__global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h, int lane_h, FlowPacked w, const float* b_out, const float* lnw, const float* lnb,
+// OUT: att = the heads' planes of the out product (os floats apart, rows of 256).  A wave takes two whole rows, which it adds up, normalises and splits by
+// itself: a request is a row's 1 KB, and no LayerNorm sum waits for the other waves.  Else att = the attention rows, and the product is done here.
+template <bool OUT>
+__global__ __launch_bounds__(512) void k_tb_ff(const float* att, size_t os, const float* h, FlowPacked w, const float* b_out, const float* lnw, const float* lnb,
                                                const float* b1, float* parts, size_t ps, int M) {
     __shared__ uint4 pl[3 * 16 * 64];
-    __shared__ float4 red[256];
+    __shared__ float4 red[OUT ? 1 : 256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4, q = blockIdx.y;
     const int m0 = blockIdx.x * 16, m = m0 + fr, row = m < M ? m : M - 1;
-    float4 a[2][2], res[2], bo[2], lw[2], lb[2], bh[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {      // the attention rows: thread = (row, 8 columns)
-        const float* s = att + (size_t)(m0 + (tid & 15) < M ? m0 + (tid & 15) : M - 1) * TB_IN + ((tid >> 4) + 32 * i) * 8;
-        a[i][0] = *reinterpret_cast<const float4*>(s);
-        a[i][1] = *reinterpret_cast<const float4*>(s + 4);
-    }
-    uint4 wo[2][16];
-    tb_weights<16, 2>(wo, w.out, wave * 2, 16, 0, lane);
-#pragma unroll
-    for (int t = 0; t < 2; ++t) {
-        const int c = (wave * 2 + t) * 16 + kq * 4;
-        res[t] = *reinterpret_cast<const float4*>(h + (lane_h ? tb_at(blockIdx.x, wave, t, lane) : (size_t)row * TB_C + c));
-        bo[t] = *reinterpret_cast<const float4*>(b_out + c);
-        lw[t] = *reinterpret_cast<const float4*>(lnw + c);
-        lb[t] = *reinterpret_cast<const float4*>(lnb + c);
-        bh[t] = *reinterpret_cast<const float4*>(b1 + q * 256 + c);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const tb_split s0 = tb_split3(a[i][0]), s1 = tb_split3(a[i][1]);
-        const int k8 = (tid >> 4) + 32 * i;
-#pragma unroll
-        for (int p = 0; p < 3; ++p) pl[(p * 16 + (k8 >> 2)) * 64 + (k8 & 3) * 16 + (tid & 15)] = make_uint4(s0.t[p].x, s0.t[p].y, s1.t[p].x, s1.t[p].y);
-    }
-    __syncthreads();
-    f32x4 acc[2];
-    tb_product<16, 2>(wo, pl, lane, acc);
     uint4 w1[2][8], w2[2][8];
-    tb_weights<8, 2>(w1, w.ff1, q * 16 + wave * 2, 8, 0, lane);
-    float4 x[2], n[2];
+    float4 bh[2];
+    f32x4 acc[2];
+    if constexpr (OUT) {
+        float4 v[2][8], res[2];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) n[t] = x[t] = tb_add(res[t], tb_add(make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]), bo[t]));
-    tb_layernorm(n, lw, lb, red, wave, lane);      // (its barriers: every wave has read the attention rows)
+        for (int i = 0; i < 2; ++i) {
+            const size_t r = m0 + 2 * wave + i < M ? m0 + 2 * wave + i : M - 1;
 #pragma unroll
-    for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, n[t]);
+            for (int p = 0; p < 8; ++p) v[i][p] = *reinterpret_cast<const float4*>(att + p * os + r * TB_C + lane * 4);
+            res[i] = *reinterpret_cast<const float4*>(h + r * TB_C + lane * 4);
+        }
+        const float4 bo = *reinterpret_cast<const float4*>(b_out + lane * 4), lw = *reinterpret_cast<const float4*>(lnw + lane * 4),
+                     lb = *reinterpret_cast<const float4*>(lnb + lane * 4);
+        tb_weights<8, 2>(w1, w.ff1, q * 16 + wave * 2, 8, 0, lane);
+        const int kb = lane >> 3, g = (lane >> 1) & 3;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const int r = 2 * wave + i;
+#pragma unroll
+            for (int p = 1; p < 8; ++p) v[i][0] = tb_add(v[i][0], v[i][p]);
+            float4 x = tb_add(res[i], tb_add(v[i][0], bo));
+            if (q == 0) *reinterpret_cast<float4*>(parts + TB_PARTS * ps + tb_at(blockIdx.x, kb, (lane >> 2) & 1, (lane & 3) * 16 + r)) = x;
+            const float mean = tb_row_sum64((x.x + x.y) + (x.z + x.w)) / (float)TB_C;
+            x = make_float4(x.x - mean, x.y - mean, x.z - mean, x.w - mean);
+            const float var = tb_row_sum64((x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w));
+            const float rstd = rsqrtf(var / (float)TB_C + 1e-5f);
+            const tb_split s = tb_split3(make_float4(x.x * rstd * lw.x + lb.x, x.y * rstd * lw.y + lb.y, x.z * rstd * lw.z + lb.z, x.w * rstd * lw.w + lb.w));
+            uint2* d = reinterpret_cast<uint2*>(pl + kb * 64 + g * 16 + tb_turn(kb, g, r)) + (lane & 1);
+#pragma unroll
+            for (int p = 0; p < 3; ++p) d[p * 8 * 128] = s.t[p];
+        }
+    } else {
+        float4 a[2][2], res[2], bo[2], lw[2], lb[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {      // the attention rows: thread = (row, 8 columns)
+            const float* s = att + (size_t)(m0 + (tid & 15) < M ? m0 + (tid & 15) : M - 1) * TB_IN + ((tid >> 4) + 32 * i) * 8;
+            a[i][0] = *reinterpret_cast<const float4*>(s);
+            a[i][1] = *reinterpret_cast<const float4*>(s + 4);
+        }
+        uint4 wo[2][16];
+        tb_weights<16, 2>(wo, w.out, wave * 2, 16, 0, lane);
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const int c = (wave * 2 + t) * 16 + kq * 4;
+            res[t] = *reinterpret_cast<const float4*>(h + (size_t)row * TB_C + c);
+            bo[t] = *reinterpret_cast<const float4*>(b_out + c);
+            lw[t] = *reinterpret_cast<const float4*>(lnw + c);
+            lb[t] = *reinterpret_cast<const float4*>(lnb + c);
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const tb_split s0 = tb_split3(a[i][0]), s1 = tb_split3(a[i][1]);
+            const int k8 = (tid >> 4) + 32 * i;
+#pragma unroll
+            for (int p = 0; p < 3; ++p) pl[(p * 16 + (k8 >> 2)) * 64 + (k8 & 3) * 16 + (tid & 15)] = make_uint4(s0.t[p].x, s0.t[p].y, s1.t[p].x, s1.t[p].y);
+        }
+        __syncthreads();
+        tb_product<16, 2>(wo, pl, lane, acc);
+        tb_weights<8, 2>(w1, w.ff1, q * 16 + wave * 2, 8, 0, lane);
+        float4 n[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            n[t] = tb_add(res[t], tb_add(make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]), bo[t]));
+            if (q == 0) *reinterpret_cast<float4*>(parts + TB_PARTS * ps + tb_at(blockIdx.x, wave, t, lane)) = n[t];
+        }
+        tb_layernorm(n, lw, lb, red, wave, lane);      // (its barriers: every wave has read the attention rows)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, n[t]);
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t) bh[t] = *reinterpret_cast<const float4*>(b1 + q * 256 + (wave * 2 + t) * 16 + kq * 4);
+    if (OUT) tb_weights<8, 2>(w2, w.ff2, wave * 2, 32, q * 8, lane);
     __syncthreads();
-    tb_product<8, 2>(w1, pl, lane, acc);
-    tb_weights<8, 2>(w2, w.ff2, wave * 2, 32, q * 8, lane);
+    tb_product<8, 2, OUT>(w1, pl, lane, acc);
+    if (!OUT) tb_weights<8, 2>(w2, w.ff2, wave * 2, 32, q * 8, lane);
     uint4* const hid = pl + 3 * 8 * 64;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -4407,7 +4489,6 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, const float* h,
         const size_t o = tb_at(blockIdx.x, wave, t, lane);
         if (q == 0) {
             y[1][t] = y[0][t] + y[1][t];
-            *reinterpret_cast<float4*>(parts + TB_PARTS * ps + o) = x[t];
         } else {
             *reinterpret_cast<f32x4*>(parts + (size_t)(2 * q - 1) * ps + o) = y[0][t];
         }
@@ -4447,6 +4528,14 @@ static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, 
     return hipGetLastError() == hipSuccess;
 }
 static size_t tb_plane(size_t M) { return (M + 15) / 16 * 16 * TB_C; }      // floats of a plane of M rows
+static float* tb_heads(float* ws, int M) { return ws + TB_PLANES * tb_plane(M); }
+// the attention of a fused block: leaves the out product's planes where its matrix-core form runs (true), else the attention rows
+static bool tb_attn(hipStream_t st, FlowAttn a, const FlowPacked* pk, float* ws, int T, int H, int N) {
+    const bool parts = pk && H == TB_HEADS && flow_attn_mfma_takes(a, T);
+    if (parts) { a.wo = pk->out; a.parts = tb_heads(ws, N * T); a.ps = tb_plane(N * T); }
+    launch_flow_attn(st, a, T, H, N);
+    return parts;
+}
 // q | k | v of the rows into qkv (before: the block before, which has left them in ws; NULL: of h itself)
 static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* h, float* ws, const vox_flow_tblock_w* before, float* qkv, int M) {
     const int tiles = (M + 15) / 16;
@@ -4464,10 +4553,14 @@ static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w&
     else TB_QKV(3);
 #undef TB_QKV
 }
-static void tb_ff(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* att, float* h, float* ws, bool first, bool last, int M) {
+// att: the attention rows, or (from_parts) the heads' planes of the out product, which the attention has left behind the block's own planes
+static void tb_ff(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& w, const float* att, float* h, float* ws, bool first, bool last, int M,
+                  bool from_parts) {
     const size_t ps = tb_plane(M);
-    hipLaunchKernelGGL(k_tb_ff, dim3((M + 15) / 16, 4), dim3(512), 0, st, att, first ? h : ws + (TB_PLANES - 1) * ps, first ? 0 : 1, f, w.out.bias, w.ln3_w,
-                       w.ln3_b, w.ff1.bias, ws, ps, M);
+    const float* in = first ? h : ws + (TB_PLANES - 1) * ps;
+    const dim3 g((M + 15) / 16, 4);
+    if (from_parts) hipLaunchKernelGGL(k_tb_ff<true>, g, dim3(512), 0, st, tb_heads(ws, M), ps, in, f, w.out.bias, w.ln3_w, w.ln3_b, w.ff1.bias, ws, ps, M);
+    else hipLaunchKernelGGL(k_tb_ff<false>, g, dim3(512), 0, st, att, 0, in, f, w.out.bias, w.ln3_w, w.ln3_b, w.ff1.bias, ws, ps, M);
     if (last) hipLaunchKernelGGL(k_tb_join, dim3((unsigned)((M + 15) / 16 * 4)), dim3(256), 0, st, ws, w.ff2.bias, ps, h, M);
 }
 
@@ -4480,7 +4573,7 @@ struct vox_flow {
     std::vector<vox_flow_tblock_w> tblocks;
     std::vector<FlowPacked> packed;         // per transformer block, or empty
     void* packed_mem = nullptr;
-    float* tb_ws = nullptr;                 // their scratch: TB_PLANES planes of the most rows
+    float* tb_ws = nullptr;                 // their scratch: TB_PLANES + TB_HEADS planes of the most rows
     int max_batch, max_T, max_prompt_T, n_res, n_att;
     std::vector<float> dt;                  // host: Euler step sizes
     float* tb = nullptr;                    // [n_steps][n_res][C]: mlp_r(Mish(time_mlp(emb_s)))
@@ -4679,14 +4772,14 @@ static int flow_run(vox_flow* m, hipStream_t st, const int32_t* tokens, int B, i
                 else VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, T2, a2, 0));
                 FlowAttn a{a2, init ? nullptr : kv, nullptr, nullptr, nullptr, a3, T2, HE, hd, Tc, capA, B, att_half, 1.0f / sqrtf((float)hd)};
                 if (evolve) { a.cidx = m->s_cidx; a.prefix = c.prefix; a.ring_head = evolve->att_head; }
-                launch_flow_attn(st, a, T2, HE, N);
+                const bool parts = tb_attn(st, a, pk, m->tb_ws, T2, HE, N);
                 if (evolve)
                     hipLaunchKernelGGL(k_flow_cache_append, dim3(ew_grid((size_t)N * HE * T2 * 2 * hd)), dim3(256), 0, st, a2, kv, m->s_cidx, att_half,
                                        T2, HE, hd, capA, c.prefix, Tc, evolve->att_head, N);
                 if (init)
                     hipLaunchKernelGGL(k_flow_cache_store, dim3(ew_grid((size_t)N * HE * capA * 2 * hd)), dim3(256), 0, st, a2, kv, T2, HE, hd, capA,
                                        c.prefix, att_half, N);
-                if (pk) { tb_ff(st, *pk, tw, a3, h, m->tb_ws, j == 0, j + 1 == c.est_blocks, N * T2); continue; }
+                if (pk) { tb_ff(st, *pk, tw, a3, h, m->tb_ws, j == 0, j + 1 == c.est_blocks, N * T2, parts); continue; }
                 VOX_TRY(conv_gemm(st, tw.out, a3, nullptr, nullptr, N, T2, 0, FLOW_OFF0, h, h, nullptr, 0));
                 VOX_TRY(ln_gemm(st, tw.ff1, h, tw.ln3_w, tw.ln3_b, 1e-5f, a1, N, T2, a2, 1));
                 VOX_TRY(conv_gemm(st, tw.ff2, a2, nullptr, nullptr, N, T2, 0, FLOW_OFF0, h, h, nullptr, 0));
@@ -4768,7 +4861,7 @@ int vox_flow_create(vox_ctx* ctx, const vox_flow_config* cfg, const vox_flow_wei
         m->conv1x.push_back(cx);
     }
     ok = ok && tb_pack(m->tblocks, C, inner, m->packed, &m->packed_mem);
-    if (!m->packed.empty()) alloc(&m->tb_ws, TB_PLANES * tb_plane(rows));
+    if (!m->packed.empty()) alloc(&m->tb_ws, (TB_PLANES + TB_HEADS) * tb_plane(rows));
     if (!ok) { vox_flow_destroy(m); return vox_fail(VOX_ERR_NOMEM, "flow_create: hipMalloc failed"); }
     // time projections of every Euler step and resnet, once: tb[s][r] = mlp_r(Mish(linear_2(SiLU(linear_1(emb_s)))))
     hipStream_t st = nullptr;
@@ -5111,7 +5204,7 @@ struct vox_glmflow {
     std::vector<vox_flow_tblock_w> tblocks;
     std::vector<FlowPacked> packed;         // per transformer block, or empty
     void* packed_mem = nullptr;
-    float* tb_ws = nullptr;                 // their scratch: TB_PLANES planes of the most rows
+    float* tb_ws = nullptr;                 // their scratch: TB_PLANES + TB_HEADS planes of the most rows
     int max_batch, max_T, max_mel, n_res, n_att;
     std::vector<float> dt;
     float* tb = nullptr;
@@ -5161,7 +5254,7 @@ int vox_glmflow_create(vox_ctx* ctx, const vox_glmflow_config* cfg, const vox_gl
     alloc(&m->pe, (size_t)2 * FLOW_MAXKEYS * D);
     alloc(&m->pp, (size_t)2 * FLOW_MAXKEYS * D);
     ok = ok && tb_pack(m->tblocks, C, inner, m->packed, &m->packed_mem);
-    if (!m->packed.empty()) alloc(&m->tb_ws, TB_PLANES * tb_plane(rows));
+    if (!m->packed.empty()) alloc(&m->tb_ws, (TB_PLANES + TB_HEADS) * tb_plane(rows));
     if (!ok) { vox_glmflow_destroy(m); return vox_fail(VOX_ERR_NOMEM, "glmflow_create: hipMalloc failed"); }
     hipStream_t st = nullptr;
     g_conv_planes = 3;
@@ -5239,8 +5332,8 @@ int vox_glmflow_decode(vox_glmflow* m, void* stream, const int32_t* tokens, int 
             if (pk) tb_qkv(st, *pk, tw, h, m->tb_ws, j ? &m->tblocks[li - 1] : nullptr, a2, N * rows_T);
             else VOX_TRY(ln_gemm(st, tw.qkv, h, tw.ln1_w, tw.ln1_b, 1e-5f, a1, N, rows_T, a2, 0));
             FlowAttn a{a2, nullptr, nullptr, nullptr, nullptr, a3, rows_T, HE, hd, 0, 0, 0, 0, 1.0f / sqrtf((float)hd), 0};
-            launch_flow_attn(st, a, rows_T, HE, N);
-            if (pk) { tb_ff(st, *pk, tw, a3, h, m->tb_ws, j == 0, j + 1 == c.est_blocks, N * rows_T); continue; }
+            const bool parts = tb_attn(st, a, pk, m->tb_ws, rows_T, HE, N);
+            if (pk) { tb_ff(st, *pk, tw, a3, h, m->tb_ws, j == 0, j + 1 == c.est_blocks, N * rows_T, parts); continue; }
             VOX_TRY(conv_gemm(st, tw.out, a3, nullptr, nullptr, N, rows_T, 0, FLOW_OFF0, h, h, nullptr, 0));
             VOX_TRY(ln_gemm(st, tw.ff1, h, tw.ln3_w, tw.ln3_b, 1e-5f, a1, N, rows_T, a2, 1));
             VOX_TRY(conv_gemm(st, tw.ff2, a2, nullptr, nullptr, N, rows_T, 0, FLOW_OFF0, h, h, nullptr, 0));
