@@ -110,9 +110,9 @@ def test_window_attention_heads_of_a_key_head_together(heads, kv, dim, page, win
     assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR
 
 
-# 2 to 16 rows: units of a dense layer in one launch each (the halves of the inner width: one round of requests, one step into the second; nine rows
-# and an inner width that is no multiple of 64 go on in the general product), routed layers with all experts in one tile, a last tile with one expert,
-# more experts than are summed at a time, all rows on every expert
+# 2 to 16 rows: units of a dense layer in one launch each (an inner width of one round of requests, of one step into the second; nine rows
+# and an inner width that is no multiple of 32 go on in the general product), routed layers whose experts have one entry, several and all rows, rows of
+# one piece and of several
 @pytest.mark.parametrize("rows,mlp", [(2, P.dense(64)), (8, P.dense(4096)), (7, P.dense(4224)), (9, P.dense(4224)), (5, P.dense(104)), (16, P.dense(2080)),
                                       (2, P.moe(2, 2, 64, 0, 0)), (8, P.moe(3, 1, 2048, 0, 0)), (7, P.moe(5, 5, 2112, 0, 0)), (8, P.moe(48, 6, 128, 4, 2)),
                                       (3, P.moe(48, 16, 64, 0, 0)), (6, P.moe(8, 2, 96, 0, 0))])

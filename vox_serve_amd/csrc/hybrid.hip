@@ -4123,73 +4123,57 @@ __global__ __launch_bounds__(256) void k_hb_win_attn_rows(const float* q, long l
         out[(size_t)row * ldo + (size_t)h * vdim + j] = a;
     }
 }
-// The same for four heads of a key head at 128 key and value dims in a bf16 cache.  16 lanes hold a token's row, so a request is four whole rows, each read
-// once a block (above, every wave reads all keys, 16 bytes of 64 rows a request).  A lane's sums over its eight dims, one for each of its four keys and
-// heads, are as many as the lanes of a row and add up in one halving exchange; the weighted sums of a lane's eight columns do so over the four
-// keys of a request.
-// Bound by the chain of page id, rows, scores and weights.  8 rows of 1024 keys, 16 heads over 4 (17 MB): 13.8 -> 8.8 us, of which a launch is 4.5.
+// The same sums for four heads of a key head at 128 key and value dims in a bf16 cache, with the keys of a chunk read once: a request is four whole rows
+// (above, every wave reads all keys, 16 bytes of 64 rows a request), which go through LDS to the lanes that score them.  Equal bits.
+// Bound by the chain of page id, rows, scores and weights.  8 rows of 1024 keys, 16 heads over 4 (17 MB): 13.8 -> 9.5 us, of which a launch is 4.5.
 __global__ __launch_bounds__(256) void k_hb_win_attn_rows4(const float* q, long ldq, const bf16_t* cache, float* out, long ldo, const int* pos, const int* row_req,
                                                            const int* ptab, int pts, int H, int G, int ps, long v_base, hb_win w, float scale, hb_sink sink, int cpb,
                                                            float* part, const float* gate, long ldg, float out_scale) {
     constexpr int D = 128, HPB = 4;
-    __shared__ float dots[HPB][64];
-    __shared__ __attribute__((aligned(16))) float pw[64][HPB];
-    __shared__ float ml[HPB][3];                     // what the sums so far are multiplied by, maximum, sum
-    __shared__ __attribute__((aligned(16))) float red[4][HPB * D];
+    __shared__ __attribute__((aligned(16))) uint4 ks[64 * 16];      // key k: its sixteen pieces, piece j at j ^ (k & 15)
+    __shared__ __attribute__((aligned(16))) float qs[HPB][D], pw[64][HPB];
+    __shared__ float ml[HPB][3];                                    // what the sums so far are multiplied by, maximum, sum
+    __shared__ float red[4][HPB * D];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), l16 = lane & 15, kg = lane >> 4;
     const int row = blockIdx.x, h0 = blockIdx.y * HPB, g = h0 / (H / G), p = pos[row];
     const int* pt = ptab + (size_t)row_req[row] * pts;
     const int lo = hb_win_start(w, p), kept = w.keep < lo ? w.keep : lo, total = kept + p - lo + 1, nchunks = (total + 63) >> 6;
     const int c0 = blockIdx.z * cpb, c1 = c0 + cpb < nchunks ? c0 + cpb : nchunks;
     if (c0 >= nchunks) return;
-    float qf[HPB][8];
-#pragma unroll
-    for (int h = 0; h < HPB; ++h) {
-        const float* s = q + (size_t)row * ldq + (size_t)(h0 + h) * D + l16 * 8;
-        const float4 x = *(const float4*)s, y = *(const float4*)(s + 4);
-        qf[h][0] = x.x; qf[h][1] = x.y; qf[h][2] = x.z; qf[h][3] = x.w;
-        qf[h][4] = y.x; qf[h][5] = y.y; qf[h][6] = y.z; qf[h][7] = y.w;
-    }
+    const float2 q2 = *(const float2*)(q + (size_t)row * ldq + (size_t)h0 * D + tid * 2);
     const size_t ld = (size_t)G * D;
-    float m = -INFINITY, l = 0.f, acc[HPB][8];
+    float m = -INFINITY, l = 0.f, acc[HPB][2];
 #pragma unroll
-    for (int h = 0; h < HPB; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
+    for (int h = 0; h < HPB; ++h) acc[h][0] = acc[h][1] = 0.f;
     for (int c = c0; c < c1; ++c) {
         const int base = c * 64, cnt = total - base < 64 ? total - base : 64;
-        uint4 kq[4], vq[4];
+        uint4 kq[4];
+        u32 v0[16];
+        const int u0 = base + (lane < cnt ? lane : cnt - 1), t = u0 < kept ? u0 : lo + (u0 - kept);
+        const int tok = pt[t / ps] * ps + t % ps;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {      // request r: keys 16 wv + 4 r .. + 3 of the chunk
-            const int k = wv * 16 + r * 4 + kg, u = base + (k < cnt ? k : cnt - 1), t = u < kept ? u : lo + (u - kept);
-            const size_t at = (size_t)(pt[t / ps] * ps + t % ps) * ld + (size_t)g * D + l16 * 8;
-            kq[r] = *(const uint4*)(cache + at);
-            vq[r] = *(const uint4*)(cache + v_base + at);
-        }
-        float a16[16];      // key r, head h
+        for (int r = 0; r < 4; ++r)      // request r: keys 16 wv + 4 r .. + 3 of the chunk
+            kq[r] = *(const uint4*)(cache + (size_t)__shfl(tok, wv * 16 + r * 4 + kg, 64) * ld + (size_t)g * D + l16 * 8);
+        const bf16_t* vb = cache + v_base + (size_t)g * D + 2 * lane;
+#pragma unroll
+        for (int x = 0; x < 16; ++x) v0[x] = *(const u32*)(vb + (size_t)__builtin_amdgcn_readlane(tok, wv * 16 + x) * ld);
+        if (c == c0) *(float2*)&qs[0][tid * 2] = q2;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-            const float kf[8] = {bflo(kq[r].x), bfhi(kq[r].x), bflo(kq[r].y), bfhi(kq[r].y), bflo(kq[r].z), bfhi(kq[r].z), bflo(kq[r].w), bfhi(kq[r].w)};
-#pragma unroll
-            for (int h = 0; h < HPB; ++h) {
-                float d = 0.f;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) d = fmaf(qf[h][e], kf[e], d);
-                a16[r * HPB + h] = d;
-            }
+            const int k = wv * 16 + r * 4 + kg;
+            ks[k * 16 + (l16 ^ (k & 15))] = kq[r];
         }
-        float a8[8], a4[4], a2[2];
-        const bool u8 = lane & 8, u4 = lane & 4, u2 = lane & 2, u1 = lane & 1;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) a8[i] = (u8 ? a16[i + 8] : a16[i]) + __shfl_xor(u8 ? a16[i] : a16[i + 8], 8, 64);
-#pragma unroll
-        for (int i = 0; i < 4; ++i) a4[i] = (u4 ? a8[i + 4] : a8[i]) + __shfl_xor(u4 ? a8[i] : a8[i + 4], 4, 64);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) a2[i] = (u2 ? a4[i + 2] : a4[i]) + __shfl_xor(u2 ? a4[i] : a4[i + 2], 2, 64);
-        dots[l16 & 3][wv * 16 + (l16 >> 2) * 4 + kg] = (u1 ? a2[1] : a2[0]) + __shfl_xor(u1 ? a2[0] : a2[1], 1, 64);
         __syncthreads();
-        {      // wave = head
-            const float z = lane < cnt ? dots[wv][lane] * scale : -INFINITY;
+        {      // wave = head, lane = key
+            float dot = 0.f;
+#pragma unroll
+            for (int j = 0; j < 16; ++j) {
+                const uint4 u = ks[lane * 16 + (j ^ (lane & 15))];
+                const float4 qa = *(const float4*)&qs[wv][j * 8], qb = *(const float4*)&qs[wv][j * 8 + 4];
+                dot = fmaf(qa.x, bflo(u.x), dot); dot = fmaf(qa.y, bfhi(u.x), dot); dot = fmaf(qa.z, bflo(u.y), dot); dot = fmaf(qa.w, bfhi(u.y), dot);
+                dot = fmaf(qb.x, bflo(u.z), dot); dot = fmaf(qb.y, bfhi(u.z), dot); dot = fmaf(qb.z, bflo(u.w), dot); dot = fmaf(qb.w, bfhi(u.w), dot);
+            }
+            const float z = lane < cnt ? dot * scale : -INFINITY;
             const float mn = fmaxf(m, hb_wave_max(z)), e = lane < cnt ? expf(z - mn) : 0.f, alpha = expf(m - mn);
             l = fmaf(l, alpha, hb_wave_sum(e));
             m = mn;
@@ -4201,36 +4185,23 @@ __global__ __launch_bounds__(256) void k_hb_win_attn_rows4(const float* q, long 
 #pragma unroll
             for (int h = 0; h < HPB; ++h) {
                 const float alpha = ml[h][0];
-#pragma unroll
-                for (int e = 0; e < 8; ++e) acc[h][e] *= alpha;
+                acc[h][0] *= alpha;
+                acc[h][1] *= alpha;
             }
         }
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {      // (weights behind the last key are zero)
-            const float4 pk = *(const float4*)pw[wv * 16 + r * 4 + kg];
-            const float vf[8] = {bflo(vq[r].x), bfhi(vq[r].x), bflo(vq[r].y), bfhi(vq[r].y), bflo(vq[r].z), bfhi(vq[r].z), bflo(vq[r].w), bfhi(vq[r].w)};
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                acc[0][e] = fmaf(pk.x, vf[e], acc[0][e]);
-                acc[1][e] = fmaf(pk.y, vf[e], acc[1][e]);
-                acc[2][e] = fmaf(pk.z, vf[e], acc[2][e]);
-                acc[3][e] = fmaf(pk.w, vf[e], acc[3][e]);
-            }
+        for (int x = 0; x < 16; ++x) {      // (weights behind the last key are zero)
+            const float4 pk = *(const float4*)pw[wv * 16 + x];
+            const float a = bflo(v0[x]), b = bfhi(v0[x]);
+            acc[0][0] = fmaf(pk.x, a, acc[0][0]); acc[0][1] = fmaf(pk.x, b, acc[0][1]);
+            acc[1][0] = fmaf(pk.y, a, acc[1][0]); acc[1][1] = fmaf(pk.y, b, acc[1][1]);
+            acc[2][0] = fmaf(pk.z, a, acc[2][0]); acc[2][1] = fmaf(pk.z, b, acc[2][1]);
+            acc[3][0] = fmaf(pk.w, a, acc[3][0]); acc[3][1] = fmaf(pk.w, b, acc[3][1]);
         }
         if (c + 1 < c1) __syncthreads();
     }
-    // the four keys of a request: lane group kg is left with head kg
-    float s2[2][8], s1[8];
-    const bool u32_ = lane & 32, u16_ = lane & 16;
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
-#pragma unroll
-        for (int e = 0; e < 8; ++e) s2[h][e] = (u32_ ? acc[h + 2][e] : acc[h][e]) + __shfl_xor(u32_ ? acc[h][e] : acc[h + 2][e], 32, 64);
-#pragma unroll
-    for (int e = 0; e < 8; ++e) s1[e] = (u16_ ? s2[1][e] : s2[0][e]) + __shfl_xor(u16_ ? s2[0][e] : s2[1][e], 16, 64);
-    float4* mine = (float4*)(red[wv] + kg * D + l16 * 8);
-    mine[0] = make_float4(s1[0], s1[1], s1[2], s1[3]);
-    mine[1] = make_float4(s1[4], s1[5], s1[6], s1[7]);
+    for (int h = 0; h < HPB; ++h) *(float2*)&red[wv][h * D + 2 * lane] = make_float2(acc[h][0], acc[h][1]);
     __syncthreads();
     for (int i = tid; i < HPB * D; i += 256) {
         float a = ((red[0][i] + red[1][i]) + red[2][i]) + red[3][i];
@@ -5027,227 +4998,290 @@ __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, cons
     }
 }
 
-// ---- 2 to 16 rows, bf16: gate and up rows with their activation; down rows of up to 8 rows, dense or routed ----------------------------
+// ---- 2 to 16 rows, bf16: units of a dense layer; 2 to 8 rows: routed layers --------------------------------------------------------------
+// All of these add as the launches in whose place they stand (k_hb_gemm_rows16; k_hb_moe_gate_up and k_hb_moe_down_combine) and give the same bits: a
+// choice of experts turns on the last of them.
+//
+// y = hb_glu(A . Wg^T + b, A . Wu^T + b): k_hb_gemm_rows16's product and sums on a tile of eight gate and the same eight up columns, so the
+// activation is in its epilogue.  out: rows of ldo elements, bf16 where out16.
+// Bound by the weights' way from memory.  8 rows, 11264 x 2048 (46 MB): 15.4 us + 4.8 for the activation's own launch -> 16.0.  Column tiles walked by one
+// block, with the next tile's weights asked for ahead and the rows kept: 22 - 28, the registers leave too few blocks.
+__global__ __launch_bounds__(512) void k_hb_glu_rows(const float* A, long lda, const bf16_t* Wt, const float* bias, void* out, long ldo, int out16, int M, int ff,
+                                                     int K, hb_glu_args glu) {
+    __shared__ float red[8][16][17];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
+    const int n0 = blockIdx.x * 8, n = n0 + (col & 7), nsteps = K >> 5;
+    const bf16_t* wrow = Wt + ((size_t)(col >> 3) * ff + (n < ff ? n : ff - 1)) * K + kb * 8;
+    const float* arow = A + (size_t)(col < M ? col : 0) * lda + kb * 8;      // (tile rows past the end are never read)
+    hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int U = 8;
+    for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
+        uint4 wf[U];
+        float4 a0[U], a1[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = (s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5;
+            wf[u] = *(const uint4*)(wrow + k);
+            a0[u] = *(const float4*)(arow + k);
+            a1[u] = *(const float4*)(arow + k + 4);
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            if (s0 + 8 * u >= nsteps) break;
+            union { uint4 q; hb_bf16x8 b; } af, bfv;
+            af.q.x = pack_bf2(a0[u].x, a0[u].y); af.q.y = pack_bf2(a0[u].z, a0[u].w);
+            af.q.z = pack_bf2(a1[u].x, a1[u].y); af.q.w = pack_bf2(a1[u].z, a1[u].w);
+            bfv.q = wf[u];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af.b, bfv.b, acc, 0, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[wv][kb * 4 + r][col] = acc[r];
+    __syncthreads();
+    const int orow = threadIdx.x >> 3, oc = threadIdx.x & 7;
+    if (threadIdx.x >= 128 || orow >= M || n0 + oc >= ff) return;
+    float g = red[0][orow][oc], u = red[0][orow][8 + oc];
+#pragma unroll
+    for (int w = 1; w < 8; ++w) { g += red[w][orow][oc]; u += red[w][orow][8 + oc]; }
+    const float y = hb_glu(g + (bias ? bias[n0 + oc] : 0.f), u + (bias ? bias[ff + n0 + oc] : 0.f), glu.limit, glu.alpha, glu.up_offset, glu.gelu);
+    const size_t o = (size_t)orow * ldo + n0 + oc;
+    if (out16) ((bf16_t*)out)[o] = f2bf(y);
+    else ((float*)out)[o] = y;
+}
+// The product behind it, x joins A . W^T + b, for up to 8 rows: k_hb_gemm_rows16's sums with eight output columns to a block, so that 2048 columns are a block to
+// each CU.  The eight rows and columns leave three quarters of a tile: its halves are the k-steps of two of that kernel's eight waves, w and
+// w + 4, of which the squares on the diagonal are read.  Eight steps of both are asked for before the eight in front of them are multiplied.
+// 8 rows, 2048 x 5632 (23 MB): 15.0 -> 9.7 us.
+__global__ __launch_bounds__(256) void k_hb_down_rows8(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M, int N, int K,
+                                                       hb_join join) {
+    constexpr int U = 8;
+    __shared__ float red[8][64];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, kb = lane >> 4, half = col >> 3, c8 = col & 7;
+    const int n0 = blockIdx.x * 8, n = n0 + c8 < N ? n0 + c8 : N - 1, nsteps = K >> 5, mine0 = wv + 4 * half;
+    const int orow = tid >> 3, oc = tid & 7;
+    const bool mine = tid < 64 && orow < M && n0 + oc < N;
+    hb_join_in jin;
+    if (mine) jin = hb_join_load(join, C + (size_t)orow * ldc, orow, n0 + oc);
+    const bf16_t *wrow = Wt + (size_t)n * K + kb * 8, *arow = A + (size_t)(c8 < M ? c8 : 0) * lda + kb * 8;
+    auto load = [&](int s0, uint4 (&wf)[U], uint4 (&af)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int s = mine0 + s0 + 8 * u, k = (s < nsteps ? s : 0) << 5;
+            wf[u] = *(const uint4*)(wrow + k);
+            af[u] = *(const uint4*)(arow + k);
+        }
+    };
+    hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+    auto multiply = [&](int s0, const uint4 (&wf)[U], const uint4 (&af)[U]) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            union { uint4 q; hb_bf16x8 b; } a, w;
+            a.q = mine0 + s0 + 8 * u < nsteps ? af[u] : make_uint4(0, 0, 0, 0);
+            w.q = wf[u];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, w.b, acc, 0, 0, 0);
+        }
+    };
+    uint4 w0[U], a0[U], w1[U], a1[U];
+    load(0, w0, a0);
+    for (int s0 = 0; s0 < nsteps; s0 += 16 * U) {
+        if (s0 + 8 * U < nsteps) load(s0 + 8 * U, w1, a1);
+        multiply(s0, w0, a0);
+        if (s0 + 16 * U < nsteps) load(s0 + 16 * U, w0, a0);
+        if (s0 + 8 * U < nsteps) multiply(s0 + 8 * U, w1, a1);
+    }
+    if ((kb >> 1) == half)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[mine0][((kb & 1) * 4 + r) * 8 + c8] = acc[r];
+    __syncthreads();
+    if (!mine) return;
+    const float sum = ((((((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid]) + red[4][tid]) + red[5][tid]) + red[6][tid]) + red[7][tid];
+    hb_join_apply(join, jin, C + (size_t)orow * ldc, orow, n0 + oc, sum + (bias ? bias[n0 + oc] : 0.f));
+}
 // The routed entries of a step: entry row*top + k uses expert sel[.]; at most 64 entries, one a lane.
 struct hb_entries {
     const int* sel;
     const float* wgt;
     int top, experts, scale_input;
 };
-// y = hb_glu(A . Wg^T + b, A . Wu^T + b): k_hb_gemm_rows16's product and sums on a tile of eight gate and the same eight up columns, so the
-// activation is in its epilogue.  ROUTED: block (columns, entry); the first entry of an expert takes all of that expert's (each weight is read once a
-// step), the blocks of the others end at once.  out: rows (entries) of ldo elements, bf16 where out16.
-// Bound by the weights' way from memory.  8 rows, 2048 wide, us: dense 11264 x 2048 (46 MB) 15.4 + 4.8 for the activation's own launch -> 16.0; routed, 16
-// choices among 8 experts of 2048 (up to 134 MB of distinct rows, 268 with each entry reading its own) 38.7 -> 27.8.  Rows without an entry
-// read row 0 (loads that only some lanes make: 36 instead of 28).  Column tiles walked by one block, with the next tile's weights asked for
-// ahead and the rows kept: 32 - 57, the registers leave too few blocks.
-template <bool ROUTED>
-__global__ __launch_bounds__(512) void k_hb_glu_rows(const float* A, long lda, const bf16_t* Wt, const float* bias, void* out, long ldo, int out16, int M, int ff,
-                                                     int K, hb_glu_args glu, hb_entries en) {
-    __shared__ float red[8][16][17];
-    __shared__ int ent[16];
-    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
-    unsigned long long left = 0;
-    int cnt = M;
-    if (ROUTED) {
-        const int ne = M * en.top, e = en.sel[blockIdx.y];
-        if (e >= en.experts) return;
-        left = __ballot(lane < ne && en.sel[lane < ne ? lane : 0] == e);
-        if (__builtin_ctzll(left) != (int)blockIdx.y) return;
-        cnt = __popcll(left);
-        Wt += (size_t)e * 2 * ff * K;
+// acc + the products of eight bf16 pairs, in order
+__device__ __forceinline__ float hb_dot8(uint4 u, uint4 v, float a) {
+    a = fmaf(bflo(u.x), bflo(v.x), a); a = fmaf(bfhi(u.x), bfhi(v.x), a); a = fmaf(bflo(u.y), bflo(v.y), a); a = fmaf(bfhi(u.y), bfhi(v.y), a);
+    a = fmaf(bflo(u.z), bflo(v.z), a); a = fmaf(bfhi(u.z), bfhi(v.z), a); a = fmaf(bflo(u.w), bflo(v.w), a); return fmaf(bfhi(u.w), bfhi(v.w), a);
+}
+// Gate and up rows of the routed entries with their activation, k_hb_moe_gate_up's sums (hb_dot_wave).  Block (columns, entry): the first entry of an expert
+// takes all of that expert's, the blocks of the others end at once, so a weight is read and widened once a step, not once an entry.  The
+// entries' rows lie in LDS as the bf16 that the products see; a wave has two gate and two up rows and multiplies a piece of them by all entries.
+// Bound by the weights' way from memory and the products on the vector units, which keep the order of the sums (on the matrix cores 27.8).  8 rows, 16
+// choices among 8 experts of 2048 x 2048 (up to 134 MB of distinct rows, 268 with each entry reading
+// its own): 38.7 -> 31.8 us.
+#define HB_MOE_UP_ROWS 8
+__global__ __launch_bounds__(256) void k_hb_moe_up_rows(const float* h, long ldh, const bf16_t* w_gate_up, bf16_t* act, int W, int ff, int M, hb_glu_args glu,
+                                                        hb_entries en) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t rows[];      // [HB_MOE_UP_ROWS][W]
+    constexpr int NC = 4, NE = HB_MOE_UP_ROWS;
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ne = M * en.top, e = en.sel[blockIdx.y];
+    if (e >= en.experts) return;
+    unsigned long long left = __ballot(lane < ne && en.sel[lane < ne ? lane : 0] == e);
+    if (__builtin_ctzll(left) != (int)blockIdx.y) return;
+    const int n0 = blockIdx.x * 8 + wv * 2;
+    const bf16_t* w[4];      // gate, gate, up, up
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const int n = n0 + (r & 1) < ff ? n0 + (r & 1) : ff - 1;
+        w[r] = w_gate_up + ((size_t)e * 2 * ff + (size_t)(r >> 1) * ff + n) * W + lane * 8;
     }
-    const int n0 = blockIdx.x * 8, n = n0 + (col & 7), nsteps = K >> 5;
-    const bf16_t* wrow = Wt + ((size_t)(col >> 3) * ff + (n < ff ? n : ff - 1)) * K + kb * 8;
-    const int orow = threadIdx.x >> 3, oc = threadIdx.x & 7;
-    for (int done = 0; done < cnt; done += 16) {      // (an expert has an entry of a row once; more than 16 only where scores are no numbers)
-        const bool rowok = col < cnt - done;
-        int entry = rowok ? col : 0;
-        if (ROUTED) {
-            entry = 0;
-            for (int i = 0; i < 16 && left; ++i, left &= left - 1)
-                if (i == col) entry = __builtin_ctzll(left);
+    uint4 wr[NC][4];
+    auto load = [&](int c0) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+            const int k = lane * 8 + 512 * (c0 + c), o = k < W ? 512 * (c0 + c) : 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) wr[c][r] = *(const uint4*)(w[r] + (k < W || lane * 8 < W ? o : -lane * 8));
         }
-        if (threadIdx.x < 16) ent[col] = entry;
-        const int arow_i = ROUTED ? entry / en.top : entry;
-        const float* arow = A + (size_t)arow_i * lda + kb * 8;
-        const float xs = ROUTED && en.scale_input ? en.wgt[entry] : 1.0f;
-        hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
-        constexpr int U = 8;
-        for (int s0 = wv; s0 < nsteps; s0 += 8 * U) {
-            uint4 wf[U];
-            float4 a0[U], a1[U];
+    };
+    while (left) {      // (an expert has an entry of a row once; more than 8 only where scores are no numbers)
+        int nb = 0, ent[NE];
 #pragma unroll
-            for (int u = 0; u < U; ++u) wf[u] = *(const uint4*)(wrow + ((s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5));
+        for (int j = 0; j < NE; ++j) {
+            ent[j] = left ? __builtin_ctzll(left) : 0;
+            nb += left ? 1 : 0;
+            left &= left - 1;
+        }
+        load(0);
 #pragma unroll
-            for (int u = 0; u < U; ++u) {
-                const int k = (s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5;
-                a0[u] = *(const float4*)(arow + k);
-                a1[u] = *(const float4*)(arow + k + 4);
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (s0 + 8 * u >= nsteps) break;
-                union { uint4 q; hb_bf16x8 b; } af, bfv;      // (tile rows without an entry are never read)
-                af.q.x = pack_bf2(a0[u].x * xs, a0[u].y * xs); af.q.y = pack_bf2(a0[u].z * xs, a0[u].w * xs);
-                af.q.z = pack_bf2(a1[u].x * xs, a1[u].y * xs); af.q.w = pack_bf2(a1[u].z * xs, a1[u].w * xs);
-                bfv.q = wf[u];
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af.b, bfv.b, acc, 0, 0, 0);
+        for (int j = 0; j < NE; ++j) {
+            if (j >= nb) break;
+            const float* x = h + (size_t)(ent[j] / en.top) * ldh;
+            const float xs = en.scale_input ? en.wgt[ent[j]] : 1.0f;
+            for (int k = tid * 4; k < W; k += 1024) {
+                const float4 v = *(const float4*)(x + k);
+                *(uint2*)(rows + (size_t)j * W + k) = make_uint2(pack_bf2(v.x * xs, v.y * xs), pack_bf2(v.z * xs, v.w * xs));
             }
         }
-#pragma unroll
-        for (int r = 0; r < 4; ++r) red[wv][kb * 4 + r][col] = acc[r];
         __syncthreads();
-        if (threadIdx.x < 128 && orow < cnt - done && n0 + oc < ff) {
-            float g = red[0][orow][oc], u = red[0][orow][8 + oc];
+        float acc[NE][4];
 #pragma unroll
-            for (int w = 1; w < 8; ++w) { g += red[w][orow][oc]; u += red[w][orow][8 + oc]; }
-            const float y = hb_glu(g + (bias ? bias[n0 + oc] : 0.f), u + (bias ? bias[ff + n0 + oc] : 0.f), glu.limit, glu.alpha, glu.up_offset, glu.gelu);
-            const size_t o = (size_t)ent[orow] * ldo + n0 + oc;
-            if (out16) ((bf16_t*)out)[o] = f2bf(y);
-            else ((float*)out)[o] = y;
+        for (int j = 0; j < NE; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[j][r] = 0.f;
+        for (int c0 = 0; c0 * 512 < W; c0 += NC) {
+            if (c0 > 0) load(c0);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int k = lane * 8 + 512 * (c0 + c);
+                if (k >= W) break;
+                float wf[4][8];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const uint4 u = wr[c][r];
+                    wf[r][0] = bflo(u.x); wf[r][1] = bfhi(u.x); wf[r][2] = bflo(u.y); wf[r][3] = bfhi(u.y);
+                    wf[r][4] = bflo(u.z); wf[r][5] = bfhi(u.z); wf[r][6] = bflo(u.w); wf[r][7] = bfhi(u.w);
+                }
+#pragma unroll
+                for (int j = 0; j < NE; ++j) {
+                    if (j >= nb) break;
+                    const uint4 u = *(const uint4*)(rows + (size_t)j * W + k);
+                    const float xf[8] = {bflo(u.x), bfhi(u.x), bflo(u.y), bfhi(u.y), bflo(u.z), bfhi(u.z), bflo(u.w), bfhi(u.w)};
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(wf[r][i], xf[i], acc[j][r]);
+                }
+            }
         }
-        if (ROUTED) __syncthreads();
+        // hb_wave_sum's tree, with the values spread over the lanes at its first two steps: lanes 0, 16, 32, 48 are left with row 0, 1, 2, 3
+        const bool b5 = lane & 32, b4 = lane & 16;
+#pragma unroll
+        for (int j = 0; j < NE; ++j) {
+            if (j >= nb) break;
+            const float v0 = (b5 ? acc[j][2] : acc[j][0]) + __shfl_xor(b5 ? acc[j][0] : acc[j][2], 32, 64);
+            const float v1 = (b5 ? acc[j][3] : acc[j][1]) + __shfl_xor(b5 ? acc[j][1] : acc[j][3], 32, 64);
+            float v = (b4 ? v1 : v0) + __shfl_xor(b4 ? v0 : v1, 16, 64);
+#pragma unroll
+            for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+            const float up = __shfl_xor(v, 32, 64);
+            const int n = n0 + (lane >> 4);
+            if (lane < 32 && (lane & 15) == 0 && n < ff)
+                act[(size_t)ent[j] * ff + n] = f2bf(hb_glu(v, up, glu.limit, glu.alpha, glu.up_offset, glu.gelu));
+        }
+        if (left) __syncthreads();
     }
 }
-// The product behind it for up to 8 rows: x joins sum_k wgt_k * (identity ? h : down_{e_k} . act_k) (ROUTED, k ascending) or down . act + b.  A block owns
-// eight output columns; an MFMA tile is two segments of eight rows and those columns, of which the two squares on its diagonal are read: two of
-// the step's distinct experts, or (dense) the two halves of K.  The eight waves take a segment's k-steps w, w + 8, ..., with the next
-// eight asked for before these are multiplied; a wave walks all segments without a barrier, the partial sums wait in LDS (SEGS segments at a time).
-// Sixteen columns a block would leave every second CU without one at 2048 columns, and with an expert to a block the sum over k takes a
-// further launch.  8 rows, us: 2048 x 5632 (23 MB) 15.0 -> 11.5; 2048 x 2048, 16 choices among 8 experts (67 MB) 22.0 -> 15.9.
-template <bool ROUTED>
-__global__ __launch_bounds__(512) void k_hb_down_rows8(const bf16_t* A, long lda, const bf16_t* Wt, const float* bias, const float* h, long ldh, float* C, long ldc,
-                                                       int M, int N, int K, hb_join join, hb_entries en) {
-    constexpr int SEGS = ROUTED ? 16 : 2, U = 8;
-    __shared__ float red[SEGS / 2][8][128];
-    __shared__ float eo[ROUTED ? 64 : 2][64];            // segment, [row][column]
-    __shared__ int s_expert[64], s_sel[64], s_seg[64], s_entry[ROUTED ? 64 * 8 : 1];
-    __shared__ float s_wgt[64];
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), col = lane & 15, kb = lane >> 4, half = col >> 3, c8 = col & 7;
-    const int n0 = blockIdx.x * 8, n = n0 + c8 < N ? n0 + c8 : N - 1, ne = ROUTED ? M * en.top : 0;
-    int nd = 2;
-    if (ROUTED) {
-        const int s = lane < ne ? en.sel[lane] : en.experts;
-        if (wv == 0) { s_sel[lane] = s; s_wgt[lane] = lane < ne ? en.wgt[lane] : 0.f; }
-        unsigned long long todo = __ballot(s < en.experts);
-        for (nd = 0; todo; ++nd) {      // distinct experts in the order of their first entry
-            const int e = __builtin_amdgcn_readlane(s, __builtin_ctzll(todo));
-            if (tid == 0) s_expert[nd] = e;
-            if (wv == 0 && s == e) s_seg[lane] = nd;
-            todo &= ~__ballot(s == e);
+// x joins sum_k wgt_k * (identity ? h : down_{e_k} . act_k), k ascending: k_hb_moe_down_combine's sums, a wave per (row, column) like there, of activations that
+// are bf16 already (rounding them was most of that kernel's arithmetic).  The rows' blocks of four columns follow each other on one XCD, so an
+// expert's rows come from memory once and from that L2 for its other entries; a wave asks for two entries' rows at a time.
+// 8 rows, 2048 x 2048, 16 choices among 8 experts (67 MB of distinct rows): 22.0 -> 20.4 us.  Taken once per block, for all entries from LDS: 23.3 with one
+// column a wave, 25.1 with two; that leaves too few waves for the sums, whose order keeps them off the matrix cores.
+__global__ __launch_bounds__(256) void k_hb_moe_down_rows(const bf16_t* act, const bf16_t* w_down, const float* h, long ldh, float* C, long ldc, int M, int N, int K,
+                                                          hb_join join, hb_entries en) {
+    constexpr int NC = 4;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), in_xcd = (int)blockIdx.x >> 3;
+    const int row = in_xcd % M, c = (in_xcd / M * 8 + ((int)blockIdx.x & 7)) * 4 + wv;
+    if (c >= N) return;
+    const hb_join_in jin = hb_join_load(join, C + (size_t)row * ldc, row, c);
+    const bool b5 = lane & 32;
+    float acc = 0.f;
+    for (int k0 = 0; k0 < en.top; k0 += 2) {
+        const int i0 = row * en.top + k0, i1 = k0 + 1 < en.top ? i0 + 1 : i0, e0 = en.sel[i0], e1 = en.sel[i1];
+        const float w0 = en.wgt[i0], w1 = en.wgt[i1];
+        const bf16_t *p0 = w_down + ((size_t)(e0 < en.experts ? e0 : 0) * N + c) * K, *p1 = w_down + ((size_t)(e1 < en.experts ? e1 : 0) * N + c) * K;
+        const bf16_t *x0 = act + (size_t)i0 * K, *x1 = act + (size_t)i1 * K;
+        float a0 = 0.f, a1 = 0.f;
+        for (int b = lane * 8; b < K; b += 512 * NC) {
+            uint4 u0[NC], u1[NC], v0[NC], v1[NC];
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int k = b + 512 * i < K ? b + 512 * i : b;
+                u0[i] = *(const uint4*)(p0 + k);
+                v0[i] = *(const uint4*)(x0 + k);
+                u1[i] = *(const uint4*)(p1 + k);
+                v1[i] = *(const uint4*)(x1 + k);
+            }
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                if (b + 512 * i >= K) break;
+                a0 = hb_dot8(u0[i], v0[i], a0);
+                a1 = hb_dot8(u1[i], v1[i], a1);
+            }
         }
-        __syncthreads();
-        // the entry of row i % 8 for segment i / 8; a row without one reads any of them (its sums are never used: loads that only some lanes make cost
-        // more than they save)
-        for (int i = tid; i < nd * 8; i += 512) {
-            int at = 0;
-            if ((i & 7) < M)
-                for (int k = en.top - 1; k >= 0; --k)
-                    if (s_sel[(i & 7) * en.top + k] == s_expert[i >> 3]) at = (i & 7) * en.top + k;
-            s_entry[i] = at;
-        }
-        __syncthreads();
+        float v = (b5 ? a1 : a0) + __shfl_xor(b5 ? a0 : a1, 32, 64);      // (hb_wave_sum's tree: its first step leaves an entry to each half of the wave)
+#pragma unroll
+        for (int o = 16; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
+        const float d1 = __shfl(v, 32, 64);
+        if (e0 >= en.experts) acc = fmaf(w0, h[(size_t)row * ldh + c], acc);
+        else acc = fmaf(en.scale_input ? 1.0f : w0, v, acc);
+        if (k0 + 1 >= en.top) break;
+        if (e1 >= en.experts) acc = fmaf(w1, h[(size_t)row * ldh + c], acc);
+        else acc = fmaf(en.scale_input ? 1.0f : w1, d1, acc);
     }
-    const int ks = ROUTED ? K : K >> 1, nsteps = ks >> 5, chunks = (nsteps + 8 * U - 1) / (8 * U);
-    const int orow = tid >> 3, oc = tid & 7;
-    const bool mine = tid < 64 && orow < M && n0 + oc < N;
-    hb_join_in jin;
-    if (mine) jin = hb_join_load(join, C + (size_t)orow * ldc, orow, n0 + oc);
-    for (int d0 = 0; d0 < nd; d0 += SEGS) {
-        const int pairs = ((nd - d0 < SEGS ? nd - d0 : SEGS) + 1) >> 1, total = pairs * chunks;
-        const bf16_t *wrow = nullptr, *arow = nullptr;
-        // eight steps of the chunk i = pair * chunks + chunk
-        auto load = [&](int i, uint4 (&wf)[U], uint4 (&af)[U]) {
-            const int pr = i / chunks, s0 = (i - pr * chunks) * 8 * U + wv;
-            if (i == pr * chunks) {
-                const int d = d0 + 2 * pr + half < nd ? d0 + 2 * pr + half : nd - 1;
-                const int row = ROUTED ? s_entry[d * 8 + c8] : c8 < M ? c8 : 0;
-                wrow = Wt + (ROUTED ? ((size_t)s_expert[d] * N + n) * K : (size_t)n * K + (size_t)half * ks) + kb * 8;
-                arow = A + (size_t)row * lda + (ROUTED ? 0 : (size_t)half * ks) + kb * 8;
-            }
-#pragma unroll
-            for (int u = 0; u < U; ++u) wf[u] = *(const uint4*)(wrow + ((s0 + 8 * u < nsteps ? s0 + 8 * u : 0) << 5));
-#pragma unroll
-            for (int u = 0; u < U; ++u) af[u] = *(const uint4*)(arow + ((s0 + 8 * u < nsteps ? s0 + 8 * u : 0) << 5));
-        };
-        hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
-        auto multiply = [&](int i, const uint4 (&wf)[U], const uint4 (&af)[U]) {
-            const int pr = i / chunks, s0 = (i - pr * chunks) * 8 * U + wv;
-#pragma unroll
-            for (int u = 0; u < U; ++u) {
-                if (s0 + 8 * u >= nsteps) break;
-                union { uint4 q; hb_bf16x8 b; } a, w;
-                a.q = af[u];
-                w.q = wf[u];
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, w.b, acc, 0, 0, 0);
-            }
-            if (i - pr * chunks == chunks - 1) {
-                if ((kb >> 1) == half)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) red[pr][wv][(kb * 4 + r) * 8 + c8] = acc[r];
-                acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
-            }
-        };
-        uint4 w0[U], a0[U], w1[U], a1[U];
-        load(0, w0, a0);
-        for (int i = 0; i < total; i += 2) {
-            if (i + 1 < total) load(i + 1, w1, a1);
-            multiply(i, w0, a0);
-            if (i + 2 < total) load(i + 2, w0, a0);
-            if (i + 1 < total) multiply(i + 1, w1, a1);
-        }
-        __syncthreads();
-        for (int i = tid; i < pairs * 128; i += 512) {
-            const int pr = i >> 7, d = d0 + 2 * pr + (i >> 6 & 1);
-            float v = red[pr][0][i & 127];
-#pragma unroll
-            for (int w = 1; w < 8; ++w) v += red[pr][w][i & 127];
-            if (d < nd) eo[d][i & 63] = v;
-        }
-        __syncthreads();
-    }
-    if (!mine) return;
-    float v = 0.f;
-    if (ROUTED)
-        for (int k = 0; k < en.top; ++k) {
-            const int i = orow * en.top + k;
-            if (s_sel[i] >= en.experts) v = fmaf(s_wgt[i], h[(size_t)orow * ldh + n0 + oc], v);
-            else v = fmaf(en.scale_input ? 1.0f : s_wgt[i], eo[s_seg[i]][tid], v);
-        }
-    else v = eo[0][tid] + eo[1][tid] + (bias ? bias[n0 + oc] : 0.f);
-    hb_join_apply(join, jin, C + (size_t)orow * ldc, orow, n0 + oc, v);
+    if (lane == 0) hb_join_apply(join, jin, C + (size_t)row * ldc, row, c, acc);
 }
 static bool hb_glu_rows_ok(const float* A, long lda, const bf16_t* W, int M, int K) {
     return M >= 2 && M <= 16 && !(K & 31) && !(lda & 3) && !((size_t)A & 15) && !((size_t)W & 15);
 }
-static bool hb_down_rows_ok(const bf16_t* W, int M, int ff) { return M <= 8 && !(ff & 63) && !((size_t)W & 15); }
-// Columns up to which a dense down product takes eight a block: a block to each CU.  8 rows, us, k_hb_gemm_rows16 and this: 2048 x 5632 15.0,
-// 11.5; 2560 x 6912 18.9, 20.3; 3072 x 8192 19.4, 21.3; 4096 x 11008 34.1, 34.8.
+// Columns up to which a dense down product takes eight a block: a block to each CU (with the halves of K in the halves of a tile, k_hb_gemm_rows16 and
+// this, us: 2560 x 6912 18.9, 20.3; 3072 x 8192 19.4, 21.3; 4096 x 11008 34.1, 34.8).
 #define HB_DOWN8_COLS 2048
 // Dense unit of a few rows; false: its shape is the general launches'.  *done: the down product is in it too.
 static bool hb_try_ff_rows(hipStream_t st, const float* A, long lda, const bf16_t* w_up, const float* b_up, const bf16_t* w_down, const float* b_down, float* act,
                            float* C, long ldc, int M, int W, int ff, hb_glu_args glu, const hb_join& join, bool* done) {
     if (!hb_glu_rows_ok(A, lda, w_up, M, W)) return false;
-    *done = W <= HB_DOWN8_COLS && hb_down_rows_ok(w_down, M, ff);
-    hipLaunchKernelGGL(k_hb_glu_rows<false>, dim3((ff + 7) / 8), dim3(512), 0, st, A, lda, w_up, b_up, (void*)act, (long)ff, *done ? 1 : 0, M, ff, W, glu,
-                       hb_entries{});
+    *done = M <= 8 && W <= HB_DOWN8_COLS && !(ff & 31) && !((size_t)w_down & 15);
+    hipLaunchKernelGGL(k_hb_glu_rows, dim3((ff + 7) / 8), dim3(512), 0, st, A, lda, w_up, b_up, (void*)act, (long)ff, *done ? 1 : 0, M, ff, W, glu);
     if (*done)
-        hipLaunchKernelGGL(k_hb_down_rows8<false>, dim3((W + 7) / 8), dim3(512), 0, st, (const bf16_t*)act, (long)ff, w_down, b_down, (const float*)nullptr, 0L, C, ldc, M,
-                           W, ff, join, hb_entries{});
+        hipLaunchKernelGGL(k_hb_down_rows8, dim3((W + 7) / 8), dim3(256), 0, st, (const bf16_t*)act, (long)ff, w_down, b_down, C, ldc, M, W, ff, join);
     return true;
 }
 static bool hb_try_ff_rows(hipStream_t, const float*, long, const float*, const float*, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args,
                            const hb_join&, bool*) { return false; }
-// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.  Both products, us,
-// entry by entry and this, 8 rows with 16 choices among 8 experts: 2048 wide 60.7, 43.7; 2560 86, 63.6; 3072 125, 79; 4096 231, 103.
+// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.
 static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16_t* w_gate_up, const bf16_t* w_down, float* act, float* C, long ldc, int M, int W,
                             int ff, hb_glu_args glu, const hb_join& join, hb_entries en) {
-    if (M * en.top > 64 || en.experts < 1 || !hb_glu_rows_ok(h, ldh, w_gate_up, M, W) || !hb_down_rows_ok(w_down, M, ff)) return false;
-    hipLaunchKernelGGL(k_hb_glu_rows<true>, dim3((ff + 7) / 8, M * en.top), dim3(512), 0, st, h, ldh, w_gate_up, (const float*)nullptr, (void*)act, (long)ff, 1, M, ff, W,
-                       glu, en);
-    hipLaunchKernelGGL(k_hb_down_rows8<true>, dim3((W + 7) / 8), dim3(512), 0, st, (const bf16_t*)act, (long)ff, w_down, (const float*)nullptr, h, ldh, C, ldc, M, W, ff,
-                       join, en);
+    const size_t lds = (size_t)HB_MOE_UP_ROWS * W * 2;
+    if (M < 2 || M * en.top > 64 || en.experts < 1 || (W & 7) || (ldh & 3) || ((size_t)h & 15) || ((size_t)w_gate_up & 15) || (ff & 7) || ((size_t)w_down & 15) ||
+        lds > 64 * 1024) return false;
+    hipLaunchKernelGGL(k_hb_moe_up_rows, dim3((ff + 7) / 8, M * en.top), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
+    hipLaunchKernelGGL(k_hb_moe_down_rows, dim3((W + 31) / 32 * 8 * M), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
     return true;
 }
 static bool hb_try_moe_rows(hipStream_t, const float*, long, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args, const hb_join&, hb_entries) {
