@@ -164,3 +164,21 @@ def test_few_row_routed_forms(rows, over):
                                                             (4, 1, 128, 5000, 0, [2080, 2080, 10])])
 def test_window_attention_of_few_rows(heads, kv, page, window, keep, cuts):
     test_window_attention_heads_of_a_key_head_together(heads, kv, 128, page, window, keep, cuts)
+
+
+# Stacks of post-normed layers, more than 16 rows: the rows that every product reads are left as bf16 by the norm before it (rows of one, two and four
+# pieces of 1024 columns, and of a width that it takes element by element); entries of an expert listed in one round and in several
+@pytest.mark.parametrize("rows,width", [(17, 64), (40, 1088), (33, 2112), (20, 70), (700, 128)])
+def test_stack_of_post_normed_layers(rows, width):
+    a = dict(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2)
+    cfg = P.config([P.attention(mlp=P.dense(128), **a), P.attention(mlp=P.moe(4, 2, 64, 0, 0), kv_from=0, **a), P.attention(mlp=P.moe(9, 3, 64, 3, 2), **a)], width=width,
+                   vocab=50)
+    S = P.random_checkpoint(cfg, seed=width)
+    toks = torch.randint(0, 50, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
+    d = U.Driver(cfg, S, dtype=torch.bfloat16, page_size=16, pages=(rows + 15) // 16, max_rows=rows)
+    try:
+        got = d.run_cut("r", toks, [rows])
+    finally:
+        d.close()
+    err = U.rel_err(got, KR.forward(cfg, S, toks), 0.8)      # (a choice that bf16 rounding flips moves a whole row, in each of two layers)
+    assert err < BF16_BAR, err

@@ -322,10 +322,11 @@ struct hb_post {
     const float *w, *b;
     float eps;
     int rms;
+    bf16_t* x16;            // the new rows as bf16 too, at the stride of x (register form), or NULL
 };
 // NC > 0: rows of at most 1024 * NC columns whose operands lie on 16-byte boundaries; thread t owns the columns 4t .. 4t+3 of every 1024,
 // everything is requested at the start and the new row stays in its registers (out) as well as in xo (NULL: not written)
-template <int NC> __device__ __forceinline__ void hb_post_row(const hb_post& p, int row, const float* xr, float* xo, int W, float (*red)[4], float4 (&out)[NC]) {
+template <int NC> __device__ __forceinline__ void hb_post_row(const hb_post& p, int row, const float* xr, float* xo, long ldx, int W, float (*red)[4], float4 (&out)[NC]) {
     const float* yr = p.y + (size_t)row * p.ldy;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     float4 y[NC], g[NC], b[NC];
@@ -366,7 +367,10 @@ template <int NC> __device__ __forceinline__ void hb_post_row(const hb_post& p, 
         out[i].y += y[i].y * inv * g[i].y + b[i].y;
         out[i].z += y[i].z * inv * g[i].z + b[i].z;
         out[i].w += y[i].w * inv * g[i].w + b[i].w;
-        if (xo && k < W) *(float4*)(xo + k) = out[i];
+        if (xo && k < W) {
+            *(float4*)(xo + k) = out[i];
+            if (p.x16) *(uint2*)(p.x16 + (size_t)row * ldx + k) = make_uint2(pack_bf2(out[i].x, out[i].y), pack_bf2(out[i].z, out[i].w));
+        }
     }
 }
 // any width and alignment, in place
@@ -401,7 +405,7 @@ template <int NC> __global__ __launch_bounds__(256) void k_hb_post_norm(hb_post 
     float* xr = x + (size_t)blockIdx.x * ldx;
     if constexpr (NC > 0) {
         float4 out[NC];
-        hb_post_row<NC>(p, blockIdx.x, xr, xr, W, red, out);
+        hb_post_row<NC>(p, blockIdx.x, xr, xr, ldx, W, red, out);
     } else hb_post_row_any(p, blockIdx.x, xr, W, red);
 }
 static void hb_post_norm(hipStream_t st, int n, const hb_post& p, float* x, long ldx, int W) {
@@ -1138,7 +1142,7 @@ __global__ __launch_bounds__(256) void k_hb_post_gemv(hb_post p, const float* x,
         wr1[i] = *(const uint4*)(w1 + kc);
     }
     float4 out[NC];
-    hb_post_row<NC>(p, 0, x, blockIdx.x == 0 ? x_out : nullptr, K, red, out);
+    hb_post_row<NC>(p, 0, x, blockIdx.x == 0 ? x_out : nullptr, 0, K, red, out);
 #pragma unroll
     for (int i = 0; i < NC; ++i)
         *(float4*)(xs + threadIdx.x * 4 + 1024 * i) = make_float4(hb_operand<T>(out[i].x), hb_operand<T>(out[i].y), hb_operand<T>(out[i].z), hb_operand<T>(out[i].w));
@@ -1187,6 +1191,8 @@ struct hb_pending {
     hb_post p;          // p.y NULL: nothing pending
     float *x, *x_next;
     long ldx;
+    bf16_t* buf16;      // room for the rows of x as bf16 at its stride, when the products that read x would round all of them, else NULL
+    const bf16_t* x16;  // what is there, or NULL.  2048 rows: the products' own launches for it, 21 x 5.4 us of a Kazozen prompt, against 0.4 each
 };
 // true: the product was launched with the pending norm in front of it; x and x_next have changed places
 template <typename T>
@@ -1205,7 +1211,10 @@ static bool hb_try_post_gemv(hipStream_t st, hb_pending& pd, bool glu, const T* 
     return true;
 }
 static void hb_settle(hipStream_t st, hb_pending& pd, int n, int W) {
-    if (pd.p.y) hb_post_norm(st, n, pd.p, pd.x, pd.ldx, W);
+    if (!pd.p.y) return;
+    pd.p.x16 = hb_post_pieces(pd.p, pd.x, pd.ldx, W) ? pd.buf16 : nullptr;
+    hb_post_norm(st, n, pd.p, pd.x, pd.ldx, W);
+    pd.x16 = pd.p.x16;
     pd.p.y = nullptr;
 }
 
@@ -4697,7 +4706,7 @@ __global__ __launch_bounds__(256) void k_hb_moe_router(const float* h, long ldh,
     if constexpr (NC > 0) {
         router_rows(0);
         float* xr = x_out + (size_t)row * ldh;
-        hb_post_row<NC>(post, row, xr, xr, W, red, mine4);
+        hb_post_row<NC>(post, row, xr, xr, ldh, W, red, mine4);
     } else if (post.y) {
         hb_post_row_any(post, row, x_out + (size_t)row * ldh, W, red);
         __syncthreads();
@@ -5365,6 +5374,7 @@ struct vox_hybrid {
     float *moe_wgt = nullptr, *moe_act = nullptr, *moe_out = nullptr;
     int *moe_sel = nullptr, *moe_list = nullptr, *moe_count = nullptr;
     bf16_t* logits16 = nullptr;
+    bf16_t* x16 = nullptr;                  // [max_rows][2 width]: the rows of a post-normed stream rounded to bf16, at its stride
     hb_ws16 ws16{nullptr, 0};               // [max_rows][widest operand]: rows of a product rounded to bf16
     float* attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
@@ -5749,7 +5759,11 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
         hn = m->h;
         ldh = W;
     }
-    if (hn) VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, hn, ldh, (const T*)L.w_in, L.b_in, m->proj, n_proj, n, n_in, W));
+    if (hn) {
+        hb_rowmap rm = hb_plain();
+        if (pd) rm.a16 = pd->x16;
+        VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, hn, ldh, (const T*)L.w_in, L.b_in, m->proj, n_proj, n, n_in, W, rm));
+    }
     const int vt = (L.vdim + 63) / 64;
     // dims per wave of the scans: the smallest of 16 / 32 / 64 that covers dim with at most 16 waves
     const int dpw = L.dim <= 16 * HB_SCAN_MAX_WAVES ? 16 : (L.dim <= 32 * HB_SCAN_MAX_WAVES ? 32 : 64);
@@ -5991,13 +6005,14 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
 // Routed feed-forward of the rows h2 (first completed by `post` when it names a sublayer's output), added to cur.  Few rows: one GEMV pair per routed entry; more: the entries are
 // listed per expert and every expert multiplies its own rows in one tile launch.
 template <typename T>
-static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, const float* h2, long ldh, const hb_post& post, float* cur, long ldx, int n, hb_join jn) {
+static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, const float* h2, long ldh, hb_post post, float* cur, long ldx, int n, hb_join jn) {
     const vox_hybrid_moe& E = *L.moe;
     jn.scale = L.ls2;
     if (L.res_gate) { jn.gate = m->rgate; jn.ldg = m->cfg.width; }
     const int W = m->cfg.width, nE = E.experts + E.identity, top = E.top, ne = n * top, ff = E.ff;
     const int up_down = E.expert_form == VOX_EXPERT_UP_DOWN ? 1 : 0, relu2 = E.expert_act == VOX_ACT_RELU2 ? 1 : 0, nf = up_down ? 1 : 2;
     const int nc = post.y && ((size_t)E.router & 15) == 0 ? hb_post_pieces(post, h2, ldh, W) : 0;
+    if (nc == 0 || E.scale_input) post.x16 = nullptr;
     auto router = nc == 1 ? k_hb_moe_router<1> : nc == 2 ? k_hb_moe_router<2> : nc == 4 ? k_hb_moe_router<4> : k_hb_moe_router<0>;
     hipLaunchKernelGGL(router, dim3(n), dim3(256), (size_t)(6 * nE + top + (E.groups > 1 ? E.groups : 0)) * 4, st, h2, ldh, E.router, E.correction, W, nE, top,
                        m->moe_sel, m->moe_wgt, E.score_kind == VOX_ROUTER_SIGMOID ? 1 : 0, E.renorm, E.router_bias, E.groups, E.keep,
@@ -6023,7 +6038,8 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
         const int cap = m->cfg.max_rows;
         hipLaunchKernelGGL(k_hb_moe_group, dim3(E.experts), dim3(256), 0, st, m->moe_sel, ne, cap, m->moe_list, m->moe_count);
         const int rows = (int)(((size_t)ne + E.experts - 1) / E.experts);        // of an expert, were they all alike
-        const hb_rowmap up{m->moe_count, m->moe_list, cap, top, (long)nf * ff * W, 0, 0, 0, E.scale_input ? m->moe_wgt : (const float*)nullptr, 0.f};
+        hb_rowmap up{m->moe_count, m->moe_list, cap, top, (long)nf * ff * W, 0, 0, 0, E.scale_input ? m->moe_wgt : (const float*)nullptr, 0.f};
+        up.a16 = post.x16;
         hb_rowmap down{m->moe_count, m->moe_list, cap, 1, (long)W * ff, 0, 0, 0};
         if (!up_down && !E.scale_input && hb_try_glu(m->ws16, st, h2, ldh, n, (const T*)E.w_gate_up, nullptr, m->moe_act, n, ff, W, (const T*)E.w_down, W, up,
                                                      E.experts, rows, (size_t)ne, hb_glu_args{E.limit, E.act_alpha, E.up_offset, 0}))
@@ -6067,6 +6083,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
     float *cur = m->xa, *other = m->xb;
     hb_pending pd{};
     pd.ldx = ldx;
+    pd.buf16 = n > 16 ? m->x16 : nullptr;
     for (int ri = 0; ri < c.n_runs; ++ri) {
         const vox_hybrid_run& run = m->runs[ri];
         const vox_hybrid_layer& L = m->layers[run.layer];
@@ -6074,6 +6091,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             hb_settle(st, pd, n, W);
             VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, cur, ldx, (const T*)m->w.loop_in, nullptr, other, ldx, n, W, 2 * W));
             float* t = cur; cur = other; other = t;
+            pd.x16 = nullptr;
         }
         const bool has_ff = L.ff > 0 || L.moe;
         // what a sublayer reads (src), and how its result joins the stream(s): with several streams each sublayer leaves what the next
@@ -6099,7 +6117,10 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             j1.store = j2.store = 1;
             pd.x = cur;
             pd.x_next = other;
-        } else hb_settle(st, pd, n, W);
+        } else {
+            hb_settle(st, pd, n, W);
+            pd.x16 = nullptr;
+        }
         // a parallel layer norms x once for both branches before anything is added; a mixer with a sibling needs the normed rows twice
         const float* hn = nullptr;
         if (parallel || L.sibling >= 0) {
@@ -6113,12 +6134,14 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             pd.p = post1;
             if (L.ff > 0 && !L.moe && !(n == 1 && L.ff_kind == VOX_FF_GATED)) hb_settle(st, pd, n, W);
         }
+        if (L.sibling >= 0) pd.x16 = nullptr;
         if (L.sibling >= 0)
             VOX_TRY(hb_mixer<T>(m, st, io, m->layers[L.sibling], run.side_cache, run.side_pool, run.side_state, hn, W, src, lds_x, cur, ldx, n, n_req,
                                 max_kvlen, j1));
         if (L.moe) {
             if (!parallel && !post) hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h2, nullptr, nullptr, (long)W, L.norm2_b);
-            const hb_post p1 = pd.p;
+            hb_post p1 = pd.p;
+            if (p1.y) { p1.x16 = pd.buf16; pd.x16 = nullptr; }
             pd.p.y = nullptr;
             VOX_TRY(hb_moe<T>(m, st, L, post ? pd.x : hf, ldf, post ? p1 : none, dst, ldd, n, j2));
         } else if (L.ff > 0 && L.ff_kind == VOX_FF_GATED) {
@@ -6143,13 +6166,15 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             } else {
                 if (post) hd = pd.x;
                 const int gelu = L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0;
+                hb_rowmap rm = hb_plain();
+                if (post) rm.a16 = pd.x16;
                 if (hb_try_ff_rows(st, hd, ldf, (const T*)L.w_up, L.b_up, (const T*)L.w_down, L.b_down, m->ff_act, dst, ldd, n, W, L.ff,
                                    hb_glu_args{limit, alpha, L.ff_up_offset, gelu}, j2, &whole)) {
-                } else if (hb_try_glu(m->ws16, st, hd, ldf, n, (const T*)L.w_up, L.b_up, m->ff_act, n, L.ff, W, (const T*)L.w_down, W, hb_plain(), 1, n, (size_t)n,
+                } else if (hb_try_glu(m->ws16, st, hd, ldf, n, (const T*)L.w_up, L.b_up, m->ff_act, n, L.ff, W, (const T*)L.w_down, W, rm, 1, n, (size_t)n,
                                hb_glu_args{limit, alpha, L.ff_up_offset, gelu}))
                     act16 = (const bf16_t*)m->ff_act;
                 else {
-                    VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, hd, ldf, (const T*)L.w_up, L.b_up, m->ff, 2 * L.ff, n, 2 * L.ff, W));
+                    VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, hd, ldf, (const T*)L.w_up, L.b_up, m->ff, 2 * L.ff, n, 2 * L.ff, W, rm));
                     hipLaunchKernelGGL(k_hb_glu_clamp, dim3(n, (L.ff + 1023) / 1024), dim3(256), 0, st, m->ff, m->ff_act, L.ff, limit, alpha,
                                        (const int*)nullptr, 0, L.ff_up_offset, gelu, 0, 0);
                 }
@@ -6378,6 +6403,7 @@ int vox_hybrid_create(vox_ctx* ctx, const vox_hybrid_config* cfg, const vox_hybr
     }
     if (ok && m->any_rgate) ok = hipMalloc((void**)&m->rgate, R * W * 4) == hipSuccess;
     if (ok && m->any_post) ok = hipMalloc((void**)&m->y, R * W * 4) == hipSuccess;
+    if (ok && m->any_post && m->ws16.n && cfg->streams <= 0 && R * 2 * W < (1ull << 31)) ok = hipMalloc((void**)&m->x16, R * 2 * W * 2) == hipSuccess;      // (a tile's offsets are 32 bits)
     if (ok && m->any_shift) ok = hipMalloc((void**)&m->shift, 5 * R * W * 4) == hipSuccess;
     if (ok && m->max_gated) ok = hipMalloc((void**)&m->ff_act, R * (size_t)m->max_gated * 4) == hipSuccess;
     if (ok && m->scan_ws_floats && cfg->max_rows > HB_SCAN_CHUNK) ok = hipMalloc((void**)&m->scan_ws, m->scan_ws_floats * 4) == hipSuccess;
@@ -6419,7 +6445,7 @@ int vox_hybrid_create(vox_ctx* ctx, const vox_hybrid_config* cfg, const vox_hybr
 void vox_hybrid_destroy(vox_hybrid* m) {
     if (!m) return;
     (void)hipFree(m->xa); (void)hipFree(m->xb); (void)hipFree(m->h); (void)hipFree(m->h2); (void)hipFree(m->proj); (void)hipFree(m->mix);
-    (void)hipFree(m->ff); (void)hipFree(m->ff_act); (void)hipFree(m->u); (void)hipFree(m->y); (void)hipFree(m->ones); (void)hipFree(m->rgate); (void)hipFree(m->hout); (void)hipFree(m->logits16); (void)hipFree(m->ws16.p); (void)hipFree(m->attn_ws); (void)hipFree(m->shift); (void)hipFree(m->scan_ws);
+    (void)hipFree(m->ff); (void)hipFree(m->ff_act); (void)hipFree(m->u); (void)hipFree(m->y); (void)hipFree(m->x16); (void)hipFree(m->ones); (void)hipFree(m->rgate); (void)hipFree(m->hout); (void)hipFree(m->logits16); (void)hipFree(m->ws16.p); (void)hipFree(m->attn_ws); (void)hipFree(m->shift); (void)hipFree(m->scan_ws);
     (void)hipFree(m->moe_wgt); (void)hipFree(m->moe_sel); (void)hipFree(m->moe_act); (void)hipFree(m->moe_out);
     (void)hipFree(m->moe_list); (void)hipFree(m->moe_count);
     delete m;
