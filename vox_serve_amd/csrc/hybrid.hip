@@ -4861,26 +4861,30 @@ __global__ __launch_bounds__(256) void k_hb_moe_router(const float* h, long ldh,
         wgt[(size_t)row * top + k] = (renorm ? sc[pick[k]] / den : sc[pick[k]]) * wscale;
     }
 }
-// Block e lists the entries (row*top + k) routed to expert e, ascending: list[e*cap + 0 .. count[e]).
-__global__ __launch_bounds__(256) void k_hb_moe_group(const int* sel, int n_entries, int cap, int* list, int* count) {
-    __shared__ int wsum[4];
-    __shared__ int base;
+// Block e lists the entries (row*top + k) routed to expert e, ascending: list[e*cap + 0 .. count[e]).  A round of 1024 entries costs two barriers and a
+// trip to memory: 4096 entries, 256 threads 11.2 us, this 5.2.
+__global__ __launch_bounds__(1024) void k_hb_moe_group(const int* sel, int n_entries, int cap, int* list, int* count) {
+    __shared__ int wsum[2][16];
     const int e = blockIdx.x, lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    if (threadIdx.x == 0) base = 0;
-    __syncthreads();
-    for (int i0 = 0; i0 < n_entries; i0 += 256) {
-        const int i = i0 + threadIdx.x;
-        const bool hit = i < n_entries && sel[i] == e;
+    int base = 0, flip = 0;
+    int s = (int)threadIdx.x < n_entries ? sel[threadIdx.x] : -1;
+    for (int i0 = 0; i0 < n_entries; i0 += 1024, flip ^= 1) {
+        const int i = i0 + threadIdx.x, nxt = i + 1024 < n_entries ? sel[i + 1024] : -1;
+        const bool hit = s == e;
         const unsigned long long bal = __ballot(hit);
         const int before = __popcll(bal & ((1ull << lane) - 1ull));
-        if (lane == 0) wsum[wv] = __popcll(bal);
-        __syncthreads();
-        int off = base;
-        for (int w = 0; w < wv; ++w) off += wsum[w];
-        if (hit) list[(size_t)e * cap + off + before] = i;
-        __syncthreads();
-        if (threadIdx.x == 0) base += wsum[0] + wsum[1] + wsum[2] + wsum[3];
-        __syncthreads();
+        if (lane == 0) wsum[flip][wv] = __popcll(bal);
+        __syncthreads();      // (the round after writes the other half, and its barrier comes before this half is written again)
+        int off = 0, all = 0;
+#pragma unroll
+        for (int w = 0; w < 16; ++w) {
+            const int c = wsum[flip][w];
+            if (w < wv) off += c;
+            all += c;
+        }
+        if (hit) list[(size_t)e * cap + base + off + before] = i;
+        base += all;
+        s = nxt;
     }
     if (threadIdx.x == 0) count[e] = base;
 }
@@ -4993,9 +4997,31 @@ __global__ __launch_bounds__(256) void k_hb_moe_down_combine(const float* h, lon
 }
 // x[row] += sum_k wgt[row*top + k] * (identity output ? h[row] : expert_out[row*top + k]), k ascending
 // (scale_input: an expert's output enters with weight 1, its input was scaled instead)
+// An entry's place does not depend on its choice, so its row is asked for beside it; four columns a thread where everything lies on 16 bytes (vec).
+// 2048 rows of 2048, top 2: 22.3 -> 11.8 us.
 __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, const float* h, long ldh, const float* eo, const int* sel,
-                                                        const float* wgt, int top, int experts, int W, int scale_input, hb_join join) {
+                                                        const float* wgt, int top, int experts, int W, int scale_input, hb_join join, int vec) {
     const int row = blockIdx.x;
+    if (vec) {
+        for (int i = threadIdx.x * 4; i < W; i += 1024) {
+            float a[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 2
+            for (int k = 0; k < top; ++k) {
+                const size_t en = (size_t)row * top + k;
+                float4 v = *(const float4*)(eo + en * W + i);
+                const bool ident = sel[en] >= experts;
+                if (ident) v = *(const float4*)(h + (size_t)row * ldh + i);
+                const float w = scale_input && !ident ? 1.0f : wgt[en];
+                a[0] = fmaf(w, v.x, a[0]); a[1] = fmaf(w, v.y, a[1]); a[2] = fmaf(w, v.z, a[2]); a[3] = fmaf(w, v.w, a[3]);
+            }
+            if (join.store && !join.gate && !join.scale && join.streams == 0)
+                *(float4*)(x + (size_t)row * ldx + i) = make_float4(0.f + a[0], 0.f + a[1], 0.f + a[2], 0.f + a[3]);
+            else
+#pragma unroll
+                for (int c = 0; c < 4; ++c) hb_join_add(join, x + (size_t)row * ldx, row, i + c, a[c]);
+        }
+        return;
+    }
     for (int i = threadIdx.x; i < W; i += 256) {
         float acc = 0.f;
         for (int k = 0; k < top; ++k) {
@@ -6036,7 +6062,7 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
     if (L.res_gate) VOX_TRY(hb_gemm<T>(m->ws16, st, HB_EPI_STORE, h2, ldh, (const T*)L.w_gate_ff, L.b_gate_ff, m->rgate, W, n, W, W));
     if (E.experts > 0) {
         const int cap = m->cfg.max_rows;
-        hipLaunchKernelGGL(k_hb_moe_group, dim3(E.experts), dim3(256), 0, st, m->moe_sel, ne, cap, m->moe_list, m->moe_count);
+        hipLaunchKernelGGL(k_hb_moe_group, dim3(E.experts), dim3(1024), 0, st, m->moe_sel, ne, cap, m->moe_list, m->moe_count);
         const int rows = (int)(((size_t)ne + E.experts - 1) / E.experts);        // of an expert, were they all alike
         hb_rowmap up{m->moe_count, m->moe_list, cap, top, (long)nf * ff * W, 0, 0, 0, E.scale_input ? m->moe_wgt : (const float*)nullptr, 0.f};
         up.a16 = post.x16;
@@ -6051,8 +6077,9 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
         }
         VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(m->ws16, st, m->moe_act, (long)ff, (const T*)E.w_down, nullptr, m->moe_out, (long)W, n, W, ff, down, E.experts, rows, ne));
     }
+    const int vec = !(W & 3) && !(ldx & 3) && !(ldh & 3) && !(((size_t)cur | (size_t)h2 | (size_t)m->moe_out) & 15) ? 1 : 0;
     hipLaunchKernelGGL(k_hb_moe_combine, dim3(n), dim3(256), 0, st, cur, ldx, h2, ldh, m->moe_out, m->moe_sel, m->moe_wgt, top, E.experts, W,
-                       E.scale_input, jn);
+                       E.scale_input, jn, vec);
     if (E.shared_ff > 0) {
         const int sf = E.shared_ff;
         const bool fused = !up_down && hb_try_glu(m->ws16, st, h2, ldh, n, (const T*)E.shared_gate_up, nullptr, m->moe_act, n, sf, W, (const T*)E.shared_down, W,
