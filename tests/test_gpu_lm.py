@@ -5,6 +5,8 @@ Bar: <= 8 rows per call -> BIT-EXACT logits, sampled ids, repetition caches and 
 greedy, seeded top-k, seeded top-p-only (the full-vocabulary sampler) and repetition penalty with a persisted
 cache.  Longer prefills run the bf16-MFMA linears: statistical bf16 bar, then the oracle adopts the GPU state.
 """
+import dataclasses
+
 import numpy as np
 import pytest
 import torch
@@ -167,6 +169,13 @@ def test_cosyvoice2_tiny_repetition_window(dev):
     S = LR.random_cosyvoice2_state_dict(cfg, seed=4, std=0.08)
     run_parity(dev, "cosy", cfg, S, [8, 6], 16, penalty=2.0, window=2)
     run_parity(dev, "cosy", cfg, S, [8, 6], 16, penalty=2.0, window=-1, sampler_kw=dict(top_k=0, top_p=0.9, temperature=0.7))
+
+
+def test_glm_tiny_large_vocabulary(dev):
+    """Rows that several blocks prepare and count (32768 entries and more; odd rows do not lie on 16 bytes), with a repetition penalty."""
+    cfg = dataclasses.replace(LR.tiny_glm_cfg(), vocab_in=40003, vocab_out=40003)
+    S = LR.random_glm_state_dict(cfg, seed=3, std=0.08)
+    run_parity(dev, "glm", cfg, S, [8, 6], 6, penalty=2.0, window=-1, sampler_kw=dict(top_k=0, top_p=0.9, temperature=0.7))
 
 
 def test_against_reference_goldens(dev, golden):

@@ -282,6 +282,8 @@ def test_stochastic_sampler_bit_exact(dev, B, V, k, p, mp, T_):
                                           (3, 3072, 0, 1.0, 0.1, 1.0),        # Zonos min-p (zonos.py:591-599)
                                           (2, 65536, 0, 0.9, 0.05, 0.7), (2, 4096, 0, 0.0, 0.0, 1.0),
                                           (2, 2048, 0, 1.0, 0.0, 1.0),        # full multinomial
+                                          (3, 32768, 0, 0.8, 0.0, 0.9), (3, 32771, 0, 1.0, 0.05, 1.0), (1, 262144, 0, 0.95, 0.0, 1.0),      # a row's parts: first size, remainders, largest
+                                          (2, 32767, 0, 0.8, 0.0, 0.9),
                                           (2, 168960, 50, 1.0, 0.0, 0.9), (2, 156940, 25, 0.8, 0.0, 1.0)])
 def test_full_vocab_sampler_bit_exact(dev, B, V, k, p, mp, T_):
     """top-p-only / min-p-only ("bucket" contract) and top-k over vocabularies too large for LDS."""

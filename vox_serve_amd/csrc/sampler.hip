@@ -25,6 +25,8 @@ struct SampArgs {
     float top_p, min_p, temperature, penalty;
     int V, n_suppress, W, C, greedy, top_k, out_stride, out_col, emb_vocab, H, feat_init;
     u32* ws_hist;        // [rows][65536], all-zero between launches (bucket mode)
+    u32* ws_max;         // [rows][SAMP_WS_PARTS] largest keys of a row's parts (bucket mode, large vocabularies)
+    float* ws_coarse;    // [rows][256] coarse masses (likewise)
     uint16_t* ws_keys;   // [rows][SAMP_WS_VMAX] (bucket mode; top-k mode when V > 32768)
 };
 
@@ -69,13 +71,17 @@ __device__ __forceinline__ void emit_pick(const SampArgs& a, int b, int picked, 
 }
 
 // suppress mask + repetition penalty, in place on the row (sampling.py:101-127, qwen3_tts.py:1894-1895)
-__device__ __forceinline__ void preprocess_row(const SampArgs& a, bf16_t* lg, int b, int tid, int nthr) {
+// Entries lo .. hi - 1 of row b: suppressed ones, then the repetition penalty.  (A barrier of the caller's block is behind each step.)
+__device__ __forceinline__ void preprocess_part(const SampArgs& a, bf16_t* lg, int b, int lo, int hi, int tid, int nthr) {
     if (a.n_suppress > 0) {
-        for (int j = tid; j < a.n_suppress; j += nthr) lg[a.suppress_ids[j]] = 0xFF7F;
+        for (int j = tid; j < a.n_suppress; j += nthr) {
+            const int id = a.suppress_ids[j];
+            if (id >= lo && id < hi) lg[id] = 0xFF7F;
+        }
         __syncthreads();
     }
     if (a.rep_cache && a.penalty != 1.0f) {
-        for (int v = tid; v < a.V; v += nthr) {
+        for (int v = lo + tid; v < hi; v += nthr) {
             int m = 0;
             for (int w = 0; w < a.W; ++w) m |= a.rep_cache[(((size_t)b * a.W + w) * a.C) * a.V + v];
             if (m) {
@@ -86,6 +92,7 @@ __device__ __forceinline__ void preprocess_row(const SampArgs& a, bf16_t* lg, in
         __syncthreads();
     }
 }
+__device__ __forceinline__ void preprocess_row(const SampArgs& a, bf16_t* lg, int b, int tid, int nthr) { preprocess_part(a, lg, b, 0, a.V, tid, nthr); }
 
 __global__ __launch_bounds__(256) void k_sample(SampArgs a) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -393,7 +400,7 @@ __global__ __launch_bounds__(256) void k_sample_topk(SampArgs a) {
 }
 
 // ---- full-vocabulary ("bucket") mode: top-p-only / min-p-only over any V -------------------------
-// Contract: oracle/voxref.c::sample_bucket / bk_find.  One 1024-thread block per row.  The 65536-bin key
+// Contract: oracle/voxref.c::sample_bucket / bk_find.  One 1024-thread block per row (from 32768 entries on: behind two launches of many).  The 65536-bin key
 // histogram lives in a per-context global scratch (L2-resident, 256 KiB per row) that is all-zero between
 // launches; the sortable keys are kept beside it so later passes do not redo the temperature division.
 struct BK {
@@ -425,30 +432,49 @@ struct BKShared {
     float acc, tot;
 };
 
-// all threads of the block call this; result in S.kp / S.j / S.tot
+// 256 values, entry 64 i + lane in r[i]: 0 + value 255 + value 254 + ..., in that order
+__device__ __forceinline__ float bk_sum_desc(const float (&r)[4]) {
+    float t = 0.0f;
+#pragma unroll
+    for (int i = 3; i >= 0; --i) {
+        if (!__ballot(!(r[i] == 0.0f))) continue;      // (the sum is not negative: zeros change nothing)
+#pragma unroll
+        for (int l = 63; l >= 0; --l) t = t + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[i]), l));
+    }
+    return t;
+}
+// all threads of the block call this; result in S.kp / S.j / S.tot.  The first wave walks the bins with the values in its registers (from LDS by one thread
+// a step was a trip to LDS; zeros are passed over, they change no sum)
 __device__ void bk_find_blk(const BK& c, float thr, int strict, BKShared& S, int tid) {
-    if (tid == 0) {
-        float acc = 0.0f;
+    const int lane = tid & 63;
+    if (tid < 64) {
+        float acc = 0.0f, r[4];
         int hf = -1, last_h = -1;
-        for (int h = 255; h >= 0; --h) {
-            const float ch = S.Cc[h];
-            if (ch > 0.0f) {
-                last_h = h;
-                if (bk_cmp(acc + ch, thr, strict)) {
-                    hf = h;
-                    break;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = S.Cc[64 * i + lane];
+#pragma unroll
+        for (int i = 3; i >= 0; --i) {
+            unsigned long long todo = hf < 0 ? __ballot(!(r[i] == 0.0f)) : 0ull;
+            while (todo) {
+                const int l = 63 - __builtin_clzll(todo);
+                todo ^= 1ull << l;
+                const float ch = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[i]), l));
+                if (ch > 0.0f) {
+                    last_h = 64 * i + l;
+                    if (bk_cmp(acc + ch, thr, strict)) {
+                        hf = last_h;
+                        break;
+                    }
                 }
+                acc = acc + ch;
             }
-            acc = acc + ch;
         }
-        S.whole = 0;
-        if (hf < 0) {
-            hf = last_h;
-            S.whole = 1;
-            acc = 0.0f;
+        const bool none = hf < 0;
+        if (lane == 0) {
+            S.whole = none ? 1 : 0;
+            S.hf = none ? last_h : hf;
+            S.acc = none ? 0.0f : acc;
         }
-        S.hf = hf;
-        S.acc = acc;
     }
     __syncthreads();
     const int hf = S.hf;
@@ -459,22 +485,29 @@ __device__ void bk_find_blk(const BK& c, float thr, int strict, BKShared& S, int
         S.fm[tid] = bk_mass(c, key, n);
     }
     __syncthreads();
-    if (tid == 0) {
-        float acc2 = S.acc;
+    if (tid < 64) {
+        float acc2 = S.acc, r[4];
         int kp = -1, last_k = -1;
         const int whole = S.whole;
-        for (int f = 255; f >= 0; --f) {
-            const float mk = S.fm[f];
-            if (mk > 0.0f) {
-                last_k = hf << 8 | f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = S.fm[64 * i + lane];
+#pragma unroll
+        for (int i = 3; i >= 0; --i) {
+            unsigned long long todo = kp < 0 ? __ballot(r[i] > 0.0f) : 0ull;
+            while (todo) {
+                const int l = 63 - __builtin_clzll(todo);
+                todo ^= 1ull << l;
+                const float mk = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[i]), l));
+                last_k = hf << 8 | (64 * i + l);
                 if (!whole && bk_cmp(acc2 + mk, thr, strict)) {
-                    kp = hf << 8 | f;
+                    kp = last_k;
                     break;
                 }
                 acc2 = acc2 + mk;
             }
         }
-        if (kp < 0) {
+        if (lane != 0) {}
+        else if (kp < 0) {
             S.kp = last_k;
             S.j = S.fcnt[last_k & 255];
             S.tot = acc2;
@@ -495,10 +528,94 @@ __device__ void bk_find_blk(const BK& c, float thr, int strict, BKShared& S, int
     __syncthreads();
 }
 
+// Rows of 32768 entries and more, first launch: SAMP_WS_PARTS blocks a row prepare its logits, leave their keys and the largest one, and add their
+// histograms (built in LDS, 16 bits a bin, so that a bin costs one global addition a block) to the row's.  By one block a row this was half of
+// the sampler's time; 8 rows of 168960, the whole sampler: 217 -> 64 us (13, 5 and 46).
+__global__ __launch_bounds__(1024) void k_bucket_keys(SampArgs a) {
+    __shared__ __attribute__((aligned(16))) u32 lhist[32768];      // bins 2 i and 2 i + 1 in the halves of word i
+    __shared__ u32 wred[16];
+    const int part = blockIdx.x, b = blockIdx.y, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int per = ((a.V + SAMP_WS_PARTS - 1) / SAMP_WS_PARTS + 7) & ~7, lo = min(a.V, part * per), hi = min(a.V, lo + per);
+    bf16_t* lg = a.logits + (size_t)b * a.V;
+    uint16_t* keys = a.ws_keys + (size_t)b * SAMP_WS_VMAX;
+    u32* hist = a.ws_hist + (size_t)b * 65536;
+    for (int i = tid; i < 8192; i += 1024) reinterpret_cast<uint4*>(lhist)[i] = make_uint4(0, 0, 0, 0);
+    preprocess_part(a, lg, b, lo, hi, tid, 1024);
+    __syncthreads();
+    u32 kmx = 0;
+    auto take = [&](bf16_t x) {
+        const u32 ky = key_of(f2bf(bf2f(x) / a.temperature));
+        kmx = ky > kmx ? ky : kmx;
+        atomicAdd(&lhist[ky >> 1], 1u << ((ky & 1) * 16));
+        return ky;
+    };
+    if ((reinterpret_cast<uintptr_t>(lg) & 15u) == 0) {      // (lo and the keys' rows lie on 16 bytes)
+        for (int v = lo + 8 * tid; v + 8 <= hi; v += 8192) {
+            const uint4 q = *reinterpret_cast<const uint4*>(lg + v);
+            uint4 o;
+            o.x = take((bf16_t)(q.x & 0xffff)); o.x |= take((bf16_t)(q.x >> 16)) << 16;
+            o.y = take((bf16_t)(q.y & 0xffff)); o.y |= take((bf16_t)(q.y >> 16)) << 16;
+            o.z = take((bf16_t)(q.z & 0xffff)); o.z |= take((bf16_t)(q.z >> 16)) << 16;
+            o.w = take((bf16_t)(q.w & 0xffff)); o.w |= take((bf16_t)(q.w >> 16)) << 16;
+            *reinterpret_cast<uint4*>(keys + v) = o;
+        }
+        for (int v = lo + ((hi - lo) & ~7) + tid; v < hi; v += 1024) keys[v] = (uint16_t)take(lg[v]);
+    } else {
+        for (int v = lo + tid; v < hi; v += 1024) keys[v] = (uint16_t)take(lg[v]);
+    }
+#pragma unroll
+    for (int off = 32; off >= 1; off >>= 1) {
+        const u32 o = __shfl_xor(kmx, off, VOX_WAVE);
+        kmx = o > kmx ? o : kmx;
+    }
+    if (lane == 0) wred[wave] = kmx;
+    __syncthreads();
+    if (tid == 0) {
+        for (int w = 1; w < 16; ++w) kmx = wred[w] > kmx ? wred[w] : kmx;
+        a.ws_max[b * SAMP_WS_PARTS + part] = kmx;
+    }
+    for (int i = tid; i < 8192; i += 1024) {
+        const uint4 q = reinterpret_cast<const uint4*>(lhist)[i];
+        const u32 n[4] = {q.x, q.y, q.z, q.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (n[e] & 0xffffu) atomicAdd(hist + 8 * i + 2 * e, n[e] & 0xffffu);
+            if (n[e] >> 16) atomicAdd(hist + 8 * i + 2 * e + 1, n[e] >> 16);
+        }
+    }
+}
+__device__ __forceinline__ u32 bk_row_max(const SampArgs& a, int b) {
+    u32 kmx = 0;
+    for (int i = 0; i < SAMP_WS_PARTS; ++i) {
+        const u32 o = a.ws_max[b * SAMP_WS_PARTS + i];
+        kmx = o > kmx ? o : kmx;
+    }
+    return kmx;
+}
+__device__ __forceinline__ BK bk_of(const SampArgs& a, const u32* hist, u32 kmx) {
+    BK c;
+    c.hist = hist; c.m = bf2f(bits_of(kmx)); c.min_cut = a.min_p > 0.0f ? a.min_p * 1.0f : 0.0f;
+    c.lim_key = -1; c.lim_cnt = 0;
+    return c;
+}
+// ... second launch: a wave a coarse bin, its 256 bins' masses in registers, added in descending order
+__global__ __launch_bounds__(512) void k_bucket_coarse(SampArgs a) {
+    const int b = blockIdx.y, lane = threadIdx.x & 63, h = blockIdx.x * 8 + (threadIdx.x >> 6);
+    const u32* hist = a.ws_hist + (size_t)b * 65536;
+    u32 n[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) n[i] = ld_l2(hist + (h << 8) + 64 * i + lane);
+    const BK c = bk_of(a, hist, bk_row_max(a, b));
+    float r[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = bk_mass(c, (u32)(h << 8 | (64 * i + lane)), n[i]);
+    const float t = bk_sum_desc(r);
+    if (lane == 0) a.ws_coarse[b * 256 + h] = t;
+}
+// PARTS: keys, histogram and coarse masses have been left by the two launches above
+template <bool PARTS>
 __global__ __launch_bounds__(1024) void k_sample_bucket(SampArgs a) {
-    // pass 1's histogram of one sign's 32768 keys (128 KiB); the coarse pass's staging tile reuses its head afterwards
-    __shared__ __attribute__((aligned(16))) u32 lhist[32768];
-    u32 (*tile)[33] = reinterpret_cast<u32 (*)[33]>(lhist);
+    __shared__ u32 tile[PARTS ? 1 : 256][33];      // the coarse pass's staging tile
     __shared__ BKShared S;
     __shared__ u32 wred[16];
     __shared__ int sh_pick;
@@ -507,108 +624,54 @@ __global__ __launch_bounds__(1024) void k_sample_bucket(SampArgs a) {
     bf16_t* lg = a.logits + (size_t)b * V;
     u32* hist = a.ws_hist + (size_t)b * 65536;
     uint16_t* keys = a.ws_keys + (size_t)b * SAMP_WS_VMAX;
-
-    preprocess_row(a, lg, b, tid, 1024);
-
-    // pass 1: keys, histogram, largest key.  Large vocabularies: the histogram is built in LDS, one sign of the values at a time (32768 keys
-    // each), and written to the global 65536-bin table with plain stores of the non-zero bins — as 168960 global atomics per row it was 160
-    // of the kernel's 300 us (a row of logits falls into a few thousand bins, and same-address atomics serialise in L2); the second half
-    // is counted from the keys the first one stored (no second division).  300 -> 207 us per call at 168960 entries.  Small vocabularies
-    // keep the global atomics (the two 128 KiB LDS sweeps per half would cost more than they save).
-    // (Measured and rejected: the coarse masses summed straight from the LDS histogram — 64-way bank conflicts on 2 of 16 waves: +30 us.)
     u32 kmx = 0;
-    if (V >= 32768) {
-        for (int half = 1; half >= 0; --half) {
-            for (int i = tid; i < 8192; i += 1024) reinterpret_cast<uint4*>(lhist)[i] = make_uint4(0, 0, 0, 0);
-            __syncthreads();
-            if (half) {
-                // (the row in 16-byte chunks, two in flight per thread)
-                auto take = [&](bf16_t x, int v) {
-                    const u32 ky = key_of(f2bf(bf2f(x) / a.temperature));
-                    keys[v] = (uint16_t)ky;
-                    kmx = ky > kmx ? ky : kmx;
-                    if (ky >> 15) atomicAdd(&lhist[ky & 0x7FFFu], 1u);
-                };
-                auto take8 = [&](const uint4 q, int v0) {
-                    take((bf16_t)(q.x & 0xffff), v0); take((bf16_t)(q.x >> 16), v0 + 1); take((bf16_t)(q.y & 0xffff), v0 + 2); take((bf16_t)(q.y >> 16), v0 + 3);
-                    take((bf16_t)(q.z & 0xffff), v0 + 4); take((bf16_t)(q.z >> 16), v0 + 5); take((bf16_t)(q.w & 0xffff), v0 + 6); take((bf16_t)(q.w >> 16), v0 + 7);
-                };
-                int head = (int)(((16u - (unsigned)(reinterpret_cast<uintptr_t>(lg) & 15u)) & 15u) >> 1);
-                head = head < V ? head : V;
-                for (int v = tid; v < head; v += 1024) take(lg[v], v);
-                const int nvec = (V - head) >> 3;
-                const uint4* lv = reinterpret_cast<const uint4*>(lg + head);
-                int i = tid;
-                for (; i + 1024 < nvec; i += 2048) {
-                    const uint4 q0 = lv[i], q1 = lv[i + 1024];
-                    take8(q0, head + 8 * i);
-                    take8(q1, head + 8 * (i + 1024));
-                }
-                if (i < nvec) take8(lv[i], head + 8 * i);
-                for (int v = head + 8 * nvec + tid; v < V; v += 1024) take(lg[v], v);
-            } else {
-                const int nk = V >> 3;
-                const uint4* kv = reinterpret_cast<const uint4*>(keys);
-                auto cnt = [&](u32 ky) { if (!(ky >> 15)) atomicAdd(&lhist[ky], 1u); };
-                for (int i = tid; i < nk; i += 1024) {
-                    const uint4 q = kv[i];
-                    cnt(q.x & 0xffff); cnt(q.x >> 16); cnt(q.y & 0xffff); cnt(q.y >> 16); cnt(q.z & 0xffff); cnt(q.z >> 16); cnt(q.w & 0xffff); cnt(q.w >> 16);
-                }
-                for (int v = 8 * nk + tid; v < V; v += 1024) cnt(keys[v]);
-            }
-            __syncthreads();
-            for (int i = tid; i < 32768; i += 1024) {
-                const u32 n = lhist[i];
-                if (n) hist[(half << 15) | i] = n;
-            }
-            __syncthreads();
-        }
-    } else {
+    if constexpr (!PARTS) {
+        preprocess_row(a, lg, b, tid, 1024);
+        // pass 1: keys, histogram, largest key
         for (int v = tid; v < V; v += 1024) {
             const u32 ky = key_of(f2bf(bf2f(lg[v]) / a.temperature));
             keys[v] = (uint16_t)ky;
             atomicAdd(hist + ky, 1u);
             kmx = ky > kmx ? ky : kmx;
         }
-    }
 #pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-        const u32 o = __shfl_xor(kmx, off, VOX_WAVE);
-        kmx = o > kmx ? o : kmx;
-    }
-    if (lane == 0) wred[wave] = kmx;
-    __threadfence();
-    __syncthreads();
-    kmx = wred[0];
-    for (int w = 1; w < 16; ++w) kmx = wred[w] > kmx ? wred[w] : kmx;
-
-    BK c;
-    c.hist = hist; c.m = bf2f(bits_of(kmx)); c.min_cut = a.min_p > 0.0f ? a.min_p * 1.0f : 0.0f;
-    c.lim_key = -1; c.lim_cnt = 0;
-
-    // pass 2: coarse masses, thread h sums its 256 keys in descending order; tiles staged coalesced
-    float csum = 0.0f;
-    for (int t = 7; t >= 0; --t) {
-        __syncthreads();
-        for (int e = tid; e < 8192; e += 1024) {
-            const int h = e >> 5, f = e & 31;
-            tile[h][f] = ld_l2(hist + (h << 8) + (t << 5) + f);
+        for (int off = 32; off >= 1; off >>= 1) {
+            const u32 o = __shfl_xor(kmx, off, VOX_WAVE);
+            kmx = o > kmx ? o : kmx;
         }
+        if (lane == 0) wred[wave] = kmx;
+        __threadfence();
         __syncthreads();
-        if (tid < 256)
-            for (int f = 31; f >= 0; --f) csum = csum + bk_mass(c, (u32)(tid << 8 | t << 5 | f), tile[tid][f]);
-    }
-    if (tid < 256) S.Cc[tid] = csum;
+        kmx = wred[0];
+        for (int w = 1; w < 16; ++w) kmx = wred[w] > kmx ? wred[w] : kmx;
+    } else kmx = bk_row_max(a, b);
+    BK c = bk_of(a, hist, kmx);
+    if constexpr (!PARTS) {
+        // pass 2: coarse masses, thread h sums its 256 keys in descending order; tiles staged coalesced
+        float csum = 0.0f;
+        for (int t = 7; t >= 0; --t) {
+            __syncthreads();
+            for (int e = tid; e < 8192; e += 1024) {
+                const int h = e >> 5, f = e & 31;
+                tile[h][f] = ld_l2(hist + (h << 8) + (t << 5) + f);
+            }
+            __syncthreads();
+            if (tid < 256)
+                for (int f = 31; f >= 0; --f) csum = csum + bk_mass(c, (u32)(tid << 8 | t << 5 | f), tile[tid][f]);
+        }
+        if (tid < 256) S.Cc[tid] = csum;
+    } else if (tid < 256) S.Cc[tid] = a.ws_coarse[b * 256 + tid];
     __syncthreads();
 
-    float tot;
-    if (tid == 0) {
-        float t0 = 0.0f;
-        for (int h = 255; h >= 0; --h) t0 = t0 + S.Cc[h];
-        S.tot = t0;
+    if (tid < 64) {
+        float r[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) r[i] = S.Cc[64 * i + lane];
+        const float t0 = bk_sum_desc(r);
+        if (lane == 0) S.tot = t0;
     }
     __syncthreads();
-    tot = S.tot;
+    float tot = S.tot;
     if (a.top_p < 1.0f) {
         bk_find_blk(c, a.top_p * tot, 0, S, tid);
         c.lim_key = S.kp;
@@ -623,10 +686,12 @@ __global__ __launch_bounds__(1024) void k_sample_bucket(SampArgs a) {
             if (tid < lh) S.Cc[tid] = 0.0f;
         }
         __syncthreads();
-        if (tid == 0) {
-            float s2 = 0.0f;
-            for (int f = 255; f >= 0; --f) s2 = s2 + S.fm[f];
-            S.Cc[lh] = s2;
+        if (tid < 64) {
+            float r[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) r[i] = S.fm[64 * i + lane];
+            const float s2 = bk_sum_desc(r);
+            if (lane == 0) S.Cc[lh] = s2;
         }
         __syncthreads();
     }
@@ -634,18 +699,28 @@ __global__ __launch_bounds__(1024) void k_sample_bucket(SampArgs a) {
     const float u = (float)(philox_u32(a.seed, off, (u32)b) >> 8) * (1.0f / 16777216.0f);
     bk_find_blk(c, u * tot, 1, S, tid);
     const u32 kp = (u32)S.kp, j = S.j;
-#if defined(BK_STOP) && BK_STOP == 3
-    if (kmx != 0x12345u) return;
-#endif
 
-    // pass 3: the j-th element (ascending index) whose key is kp; wave w owns a contiguous index range
+    // pass 3: the j-th element (ascending index) whose key is kp; wave w owns a contiguous index range, a lane eight neighbours of each 512
     const int chunk = ((V + 15) / 16 + 63) & ~63;
-    const int lo = wave * chunk, hi = min(V, lo + chunk);
+    const int lo = min(V, wave * chunk), hi = min(V, lo + chunk);
+    auto matches = [&](int base) -> u32 {      // bit i: entry base + 8 lane + i has the key
+        const int v = base + 8 * lane;
+        if (v >= hi) return 0;
+        u32 m = 0;
+        if (v + 8 <= hi) {
+            const uint4 q = *reinterpret_cast<const uint4*>(keys + v);
+            m = ((q.x & 0xffff) == kp ? 1u : 0) | ((q.x >> 16) == kp ? 2u : 0) | ((q.y & 0xffff) == kp ? 4u : 0) | ((q.y >> 16) == kp ? 8u : 0) |
+                ((q.z & 0xffff) == kp ? 16u : 0) | ((q.z >> 16) == kp ? 32u : 0) | ((q.w & 0xffff) == kp ? 64u : 0) | ((q.w >> 16) == kp ? 128u : 0);
+        } else {
+            for (int i = 0; v + i < hi; ++i) m |= keys[v + i] == kp ? 1u << i : 0;
+        }
+        return m;
+    };
     u32 cnt = 0;
-    for (int base = lo; base < hi; base += 64) {
-        const int v = base + lane;
-        cnt += __popcll(__ballot(v < hi && keys[v] == kp));
-    }
+#pragma unroll 4
+    for (int base = lo; base < hi; base += 512) cnt += __popc(matches(base));
+#pragma unroll
+    for (int o = 32; o >= 1; o >>= 1) cnt += __shfl_xor(cnt, o, VOX_WAVE);
     if (lane == 0) wred[wave] = cnt;
     if (tid == 0) sh_pick = -1;
     __syncthreads();
@@ -653,13 +728,21 @@ __global__ __launch_bounds__(1024) void k_sample_bucket(SampArgs a) {
     for (int w = 0; w < wave; ++w) before += wred[w];
     if (before < j && j <= before + cnt) {
         u32 run = before;
-        for (int base = lo; base < hi; base += 64) {
-            const int v = base + lane;
-            const bool mt = v < hi && keys[v] == kp;
-            const unsigned long long bal = __ballot(mt);
-            const u32 mine = run + __popcll(bal & ((1ull << lane) - 1ull)) + 1;
-            if (mt && mine == j) sh_pick = v;
-            run += __popcll(bal);
+        for (int base = lo; base < hi; base += 512) {
+            const u32 m = matches(base), n = __popc(m);
+            u32 upto = n;      // matches of the lanes up to this one
+#pragma unroll
+            for (int o = 1; o < 64; o <<= 1) {
+                const u32 g = __shfl_up(upto, o, VOX_WAVE);
+                if (lane >= o) upto += g;
+            }
+            const u32 first = run + upto - n;
+            if (first < j && j <= first + n) {
+                u32 left = m;
+                for (u32 i = j - first; i > 1; --i) left &= left - 1;
+                sh_pick = base + 8 * lane + __ffs(left) - 1;
+            }
+            run += __shfl(upto, 63, VOX_WAVE);
             if (run >= j) break;
         }
     }
@@ -687,6 +770,8 @@ int vox_launch_sample(hipStream_t st, const SampleCall& c) {
     if (c.emb2_table && ((c.H2 % 8) || !c.emb2_dst || c.emb_vocab <= 0)) return vox_fail(VOX_ERR_INVALID, "sample: bad second gather");
     a.ws_hist = (u32*)c.ws;
     a.ws_keys = c.ws ? reinterpret_cast<uint16_t*>((char*)c.ws + (size_t)SAMP_WS_ROWS * 65536 * 4) : nullptr;
+    a.ws_max = c.ws ? reinterpret_cast<u32*>((char*)c.ws + (size_t)SAMP_WS_ROWS * (65536 * 4 + SAMP_WS_VMAX * 2)) : nullptr;
+    a.ws_coarse = reinterpret_cast<float*>(a.ws_max ? a.ws_max + SAMP_WS_ROWS * SAMP_WS_PARTS : nullptr);
     if (c.emb_table && (c.H % 8)) return vox_fail(VOX_ERR_INVALID, "sample: H%8!=0");
     size_t smem = 0;
     if (!greedy) {
@@ -698,7 +783,12 @@ int vox_launch_sample(hipStream_t st, const SampleCall& c) {
                 return vox_fail(VOX_ERR_INVALID, "sample: B %d > %d or V %d > %d", c.B, SAMP_WS_ROWS, c.V, SAMP_WS_VMAX);
         }
         if (bucket) {
-            hipLaunchKernelGGL(k_sample_bucket, dim3(c.B), dim3(1024), 0, st, a);
+            // from 32768 entries on a histogram per block in LDS costs less than its two 128 KB sweeps
+            if (c.V >= 32768) {
+                hipLaunchKernelGGL(k_bucket_keys, dim3(SAMP_WS_PARTS, c.B), dim3(1024), 0, st, a);
+                hipLaunchKernelGGL(k_bucket_coarse, dim3(32, c.B), dim3(512), 0, st, a);
+                hipLaunchKernelGGL(k_sample_bucket<true>, dim3(c.B), dim3(1024), 0, st, a);
+            } else hipLaunchKernelGGL(k_sample_bucket<false>, dim3(c.B), dim3(1024), 0, st, a);
             return VOX_OK;
         }
         if (c.cfg.top_k > SAMP_KMAX)

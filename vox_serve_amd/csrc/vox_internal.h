@@ -26,13 +26,14 @@ struct vox_ctx {
     int device;
     int n_cu;
     int64_t lds_bytes, hbm_bytes;
-    void* samp_ws;   // sampler scratch: SAMP_WS_ROWS x (65536 u32 histogram, all-zero between launches) + keys
+    void* samp_ws;   // sampler scratch: SAMP_WS_ROWS x (65536 u32 histogram, all-zero between launches) + keys, largest keys of a row's parts, coarse masses
     int exact_rows = 2;   // linears with at most this many rows use the wave64 VALU kernels, more rows the matrix cores (vox_ctx_set_exact_rows)
 };
 // sampler scratch geometry (sampler.hip): one LM stream per context uses it at a time
 #define SAMP_WS_ROWS 64
 #define SAMP_WS_VMAX 262144
-#define SAMP_WS_BYTES ((size_t)SAMP_WS_ROWS * (65536 * 4 + SAMP_WS_VMAX * 2))
+#define SAMP_WS_PARTS 16       // blocks that share a row of a large vocabulary
+#define SAMP_WS_BYTES ((size_t)SAMP_WS_ROWS * (65536 * 4 + SAMP_WS_VMAX * 2 + (SAMP_WS_PARTS + 256) * 4))
 
 struct vox_graph {
     hipGraph_t graph;
