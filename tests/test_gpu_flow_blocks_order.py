@@ -59,8 +59,9 @@ def test_fused_blocks_add_as_the_general_launches(monkeypatch, B, T, blocks):
     assert rms(got) > 0.5 and np.array_equal(prompt, prompt_general) and np.array_equal(got, general)
 
 
-# GLM-4-Voice's flow: two row counts a step (all mel frames and every second), an odd number of frames among them
-@pytest.mark.parametrize("B,T,blocks", [(1, 3, 1), (3, 8, 2), (2, 25, 4)])
+# GLM-4-Voice's flow: two row counts a step (all mel frames and every second), an odd number of frames among them;
+# 1032 and 1376 rows: four and two column tiles a wave, the out product in the feed-forward again
+@pytest.mark.parametrize("B,T,blocks", [(1, 3, 1), (3, 8, 2), (2, 25, 4), (6, 25, 2), (8, 25, 2)])
 def test_glm_blocks_add_as_the_general_launches(monkeypatch, B, T, blocks):
     if not torch.cuda.is_available():
         pytest.skip("no GPU")

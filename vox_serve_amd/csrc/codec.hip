@@ -4341,7 +4341,7 @@ __global__ void k_flow_slots(int* slots, int N, int B) {
 //   k_tb_qkv   rows = residual + feed-forward parts of the block before, LayerNorm, q | k | v: grid (row tiles, 256-column groups)
 //   k_tb_ff    heads' sums of the out product + residual, LayerNorm, GELU feed-forward: grid (row tiles, 4); block y owns a quarter of the hidden
 //              columns from ff1 to its two eighths of ff2's sums (they and the residual rows are added by whoever reads them).  Where the attention has
-//              left its rows instead (more than 256 keys), the out product is done by all four
+//              left its rows instead (tb_attn), the out product is done by all four
 // Sums, LayerNorm statistics and the order of every addition are those of the general launches (k_rows_gemm: K in four runs of 64, or in eight
 // from 512 on, added in ascending order), so the two forms give the same bits: the phase of the vocoder's source multiplies what a mel
 // differs by some hundred times.
@@ -4529,9 +4529,11 @@ static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, 
 }
 static size_t tb_plane(size_t M) { return (M + 15) / 16 * 16 * TB_C; }      // floats of a plane of M rows
 static float* tb_heads(float* ws, int M) { return ws + TB_PLANES * tb_plane(M); }
-// the attention of a fused block: leaves the out product's planes where its matrix-core form runs (true), else the attention rows
+// the attention of a fused block: leaves the out product's planes where its matrix-core form runs (true), else the attention rows.  While the feed-forward's
+// blocks have a CU each: with more, its shorter blocks gain less than the attention's longer ones lose (1032 rows, us, rows and planes: 15.0 + 22.7, 17.5
+// + 20.7; 1376 rows 15.5 + 23.2, 17.9 + 21.7; 2064 rows 25.9 + 33.3, 30.0 + 32.3).
 static bool tb_attn(hipStream_t st, FlowAttn a, const FlowPacked* pk, float* ws, int T, int H, int N) {
-    const bool parts = pk && H == TB_HEADS && flow_attn_mfma_takes(a, T);
+    const bool parts = pk && H == TB_HEADS && (N * T + 15) / 16 * 4 <= 256 && flow_attn_mfma_takes(a, T);
     if (parts) { a.wo = pk->out; a.parts = tb_heads(ws, N * T); a.ps = tb_plane(N * T); }
     launch_flow_attn(st, a, T, H, N);
     return parts;
@@ -4548,9 +4550,11 @@ static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w&
                                 3 * TB_IN); \
     } while (0)
     // A block adds up its rows' planes (128 KB) whatever it multiplies them by (64 KB a tile of a wave): where two tiles a wave make more blocks than
-    // CUs, three move less.  896 rows, us (first / later blocks of a level), two, three, four tiles: 8.4 / 10.6, 7.4 / 9.1, 8.4 / 10.3.
-    if (tiles * (3 * TB_IN / 256) <= 256) TB_QKV(2);
-    else TB_QKV(3);
+    // CUs, three or four move less as long as theirs fit.  896 rows, us (first / later blocks of a level), two, three, four tiles: 8.4 / 10.6, 7.4 /
+    // 9.1, 8.4 / 10.3; later blocks of 1032 rows, two, three, four: 14.2, 16.1, 11.4.
+    if (tiles * 6 <= 256 || tiles * 3 > 256) TB_QKV(2);
+    else if (tiles * 4 <= 256) TB_QKV(3);
+    else TB_QKV(4);
 #undef TB_QKV
 }
 // att: the attention rows, or (from_parts) the heads' planes of the out product, which the attention has left behind the block's own planes
