@@ -1717,7 +1717,7 @@ static int rows_mt2_blocks() {
 // 16 x 16 output tiles above which a k_rows_gemm block takes 2 / 4 column tiles (VOX_ROWS_NT2 / VOX_ROWS_NT4)
 static int rows_nt_tiles(int which) {
     static const int v2 = [] { const char* e = getenv("VOX_ROWS_NT2"); return e ? atoi(e) : 256; }();
-    static const int v4 = [] { const char* e = getenv("VOX_ROWS_NT4"); return e ? atoi(e) : 2048; }();
+    static const int v4 = [] { const char* e = getenv("VOX_ROWS_NT4"); return e ? atoi(e) : 512; }();
     return which ? v4 : v2;
 }
 static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const float* state, const int* slots, int n,
@@ -1742,8 +1742,11 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
         const int tiles = ((w.n + 15) / 16) * ((a.M + 15) / 16);
         // column tiles per block: one while the call is a handful of row tiles (latency: more blocks in flight), two from 256 tiles on
         // once there are >= 16 row tiles (every block re-loads and re-splits its A rows: at 448+ rows that traffic and VALU work
-        // outweigh the extra blocks — CosyVoice2 chunk 49.7 -> 46.6 ms at B=8, 36.6 -> 35.2 at B=4, unchanged at B=1), four above 2048
-        int nt = tiles > rows_nt_tiles(1) ? 4 : tiles > (a.M >= 256 ? rows_nt_tiles(0) : 1024) ? 2 : 1;
+        // outweigh the extra blocks — CosyVoice2 chunk 49.7 -> 46.6 ms at B=8, 36.6 -> 35.2 at B=4, unchanged at B=1), four above 512
+        // (above 2048, and this: 8 requests of 28 tokens, 896 rows, 28.61 and 28.16 ms; 4 of 20 22.60, 22.54; 1 of 28 20.58 both), but above
+        // 2048 below those 16 row tiles and from 1025 rows on (GLM-4-Voice's flow with 512 there too, 1032 rows 53.7 and 54.2 ms, 1376 rows 57.3, 57.8)
+        const int four = a.M >= 256 && a.M <= 1024 ? rows_nt_tiles(1) : 2048;
+        int nt = tiles > four ? 4 : tiles > (a.M >= 256 ? rows_nt_tiles(0) : 1024) ? 2 : 1;
         while (nt > 1 && nt * kb > 16) nt >>= 1;
         const int mt = (tiles / nt >= rows_mt2_blocks() && kb <= 4 && (wv == 4 || nt <= 2)) ? 2 : 1;      // (the 8-wave sum buffer: MT NT <= 4)
         if (ln_w) { a.ln_w = ln_w; a.ln_b = ln_b; a.ln_eps = ln_eps; }
