@@ -5309,7 +5309,8 @@ static bool hb_try_ff_rows(hipStream_t st, const float* A, long lda, const bf16_
 }
 static bool hb_try_ff_rows(hipStream_t, const float*, long, const float*, const float*, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args,
                            const hb_join&, bool*) { return false; }
-// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.
+// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.  Both products, us,
+// entry by entry and this: 8 rows of 1024 18.6, 18.2; of 2048 60.7, 52.2; of 4096 231, 137; 4 rows of 2048 32.6, 29.1; 2 rows of 2048 24.2, 22.2, of 4096 67.4, 55.4.
 static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16_t* w_gate_up, const bf16_t* w_down, float* act, float* C, long ldc, int M, int W,
                             int ff, hb_glu_args glu, const hb_join& join, hb_entries en) {
     const size_t lds = (size_t)HB_MOE_UP_ROWS * W * 2;
