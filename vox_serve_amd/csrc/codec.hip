@@ -3673,6 +3673,10 @@ struct FlowAttn {
     const bf16_t* wo;
     float* parts;
     size_t ps;
+    // and its items (request, head, query tile) as tb_item gives them: items of an XCD, XCDs with one more, the inverses (tb_inverse) of a request's items
+    // and of its query tiles
+    int per, rest;
+    unsigned inv_n, inv_h;
 };
 __device__ __forceinline__ int flow_cache_row(int j, int prefix, int head, int cap) {
     return (head == 0 || j < prefix) ? j : prefix + (head + j - prefix) % (cap - prefix);
@@ -3883,7 +3887,25 @@ __global__ __launch_bounds__(256) void k_flow_attn_tile(FlowAttn a, int QG) {
         __builtin_amdgcn_wave_barrier();      // ps / qs are rewritten by the wave's next query
     }
 }
-// Parts of the estimator's fused transformer blocks (below) that their attention uses too
+// Parts of the estimator's fused transformer blocks (below) that their attention uses too.
+//
+// Which of a launch's items a block takes: the blocks of one XCD (block id modulo 8) take neighbouring ones, every XCD as many as the next, so that what
+// blocks beside each other read, and what the launch before left for them, is in that XCD's L2.  All of a block's launches have their items in the
+// order of the rows.  With the row tile or the query tile as the grid's fast index that was so only where eight divides it: a feed-forward of 42 row
+// tiles 12.2 us, one of 48 11.3, now 10.6 and 10.6; q | k | v of later blocks of a level 8.8 (40 tiles 8.0), now 7.3.  (Padded to eight row tiles instead,
+// 42 leave two XCDs more q | k | v blocks than CUs: 10.8.  Only q | k | v and feed-forward in this order: 8.1 and 10.6.)  The shares are counted on
+// the host: counted in the kernels, a launch of few blocks took 0.1 longer.
+struct tb_share {
+    int per, rest;      // items of an XCD, of which the first `rest` have one more
+};
+static tb_share tb_shares(int items) { return tb_share{items >> 3, items & 7}; }
+__device__ __forceinline__ int tb_item(tb_share s) {
+    const int xcd = (int)blockIdx.x & 7;
+    return xcd * s.per + (xcd < s.rest ? xcd : s.rest) + ((int)blockIdx.x >> 3);
+}
+// x / d as tb_quotient(x, tb_inverse(d)): exact while x * d < 2^24 and x / d < 256
+static unsigned tb_inverse(int d) { return ((1u << 24) + (unsigned)d - 1) / (unsigned)d; }
+__device__ __forceinline__ int tb_quotient(int x, unsigned inverse) { return (int)((unsigned)x * inverse >> 24); }
 #define TB_C 256
 #define TB_IN 512
 #define TB_FF 1024
@@ -4029,7 +4051,7 @@ __device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
 // result depends on that request's rows only.
 // OUT (fused transformer blocks: 8 heads, 256 channels): the block multiplies its 16 x 64 outputs by the head's 64 columns of the out projection too (32 KB of
 // weights), one of that product's eight runs of K: the feed-forward launch adds the heads' planes in order and has the product's bits without
-// its 256 KB of weights a block.  896 rows: 12.0 -> 13.8 us here, 13.1 -> 10.8 there and 9.1 -> 8.5 in the next q | k | v.  (Two query
+// its 256 KB of weights a block.  896 rows: 11.4 -> 13.0 us here, 13.0 -> 10.8 there and 9.1 -> 8.3 in the next q | k | v.  (Two query
 // tiles a block, which read each key once for both: 15.2.)
 template <int DK, int WV, bool OUT>
 __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
@@ -4040,7 +4062,14 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
     __shared__ __attribute__((aligned(16))) float Os[WV][16][OS];
     __shared__ uint4 pl[OUT ? 3 * 2 * 64 : 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fr = lane & 15, kq = lane >> 4;
-    const int i0 = blockIdx.x * 16, h = blockIdx.y, n = blockIdx.z;
+    int i0 = blockIdx.x * 16, h = blockIdx.y, n = blockIdx.z;
+    if constexpr (OUT) {
+        const int qt = (a.T + 15) >> 4, item = tb_item(tb_share{a.per, a.rest});
+        n = tb_quotient(item, a.inv_n);
+        const int nh = item - n * qt * a.H;
+        h = tb_quotient(nh, a.inv_h);
+        i0 = (nh - h * qt) * 16;
+    }
     const int HD = a.H * DK, ld = 3 * HD, S = a.Tc + a.T, nt = (S + 15) >> 4;
     const float* cache = a.cache ? a.cache + (a.cidx ? (size_t)a.cidx[n] * a.cache_half_stride : a.B > 0 ? (size_t)(n / a.B) * a.cache_half_stride : 0) +
                                        (size_t)h * a.Tcap * 2 * DK : nullptr;
@@ -4186,13 +4215,24 @@ static bool flow_attn_tile_on() {
     static const bool on = [] { const char* e = getenv("VOX_FLOW_ATTN_TILE"); return !(e && e[0] == '0'); }();
     return on;
 }
+// the fused blocks' order of items; false: their numbers are beyond the divisions'
+static bool flow_attn_near(FlowAttn& a, int T, int H, int N) {
+    const long per_n = (long)((T + 15) / 16) * H;
+    if (N >= 256 || H >= 256 || N * per_n * per_n >= 1l << 24) return false;
+    const tb_share s = tb_shares((int)(N * per_n));
+    a.per = s.per;
+    a.rest = s.rest;
+    a.inv_n = tb_inverse((int)per_n);
+    a.inv_h = tb_inverse((T + 15) / 16);
+    return true;
+}
 static bool flow_attn_mfma_takes(const FlowAttn& a, int T) { return !a.P && !a.bu && a.dk == 64 && a.Tc + T <= 256 && flow_attn_mfma_on(); }
 static void launch_flow_attn(hipStream_t st, const FlowAttn& a, int T, int H, int N) {
     const int S = a.Tc + T;
     const size_t lds = ((size_t)S * (2 * a.dk + 4) + 4 * ((S + 3) & ~3) + 4 * a.dk) * sizeof(float);
     if (flow_attn_mfma_takes(a, T)) {
         static const bool wv4 = [] { const char* e = getenv("VOX_FLOW_ATTN_WV"); return e && atoi(e) == 4; }();      // A/B: four waves x four key tiles
-        if (a.parts) hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, true>), dim3((T + 15) / 16, H, N), dim3(512), 0, st, a);
+        if (a.parts) hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, true>), dim3((T + 15) / 16 * H * N), dim3(512), 0, st, a);
         else if (wv4) hipLaunchKernelGGL((k_flow_attn_mfma<64, 4, false>), dim3((T + 15) / 16, H, N), dim3(256), 0, st, a);
         else hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, false>), dim3((T + 15) / 16, H, N), dim3(512), 0, st, a);
         return;
@@ -4351,31 +4391,33 @@ __global__ void k_flow_slots(int* slots, int N, int B) {
 // What one of these leaves for another (parts, the residual rows) lies in the order of the lanes, [row tile][wave][tile][lane] x 4 floats:
 // whole lines per request (as [row][256] every request touched 16 lines: k_tb_qkv 12.8 us against 8.3 with plain rows to read).
 // Bound by the dependent chain of a block (row loads, three products, two LayerNorm exchanges) and the launch; 896 rows: 16.3 us (qkv) -> 7.4 /
-// 9.1 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 10.8, with 1.8 for the out product in
+// 8.3 (first / later blocks), 32 us (out, ff1, ff2 as three launches) -> 10.8, with 1.6 for the out product in
 // the attention (13.1 with it here, in all four blocks of a row tile; with each product as one sum, four parts and other LayerNorm
 // sums: 8.3 / 10.3 and 12.7).  A row's result depends on that row only.
 // NT column tiles a wave, 128 NT columns a block.
+// Grid: the blocks of a row tile beside each other, in tb_item's order, here and in the attention between them.
 template <bool PARTS, int NT>
 __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* parts, const float* b2, size_t ps, const bf16_t* w, const float* lnw, const float* lnb,
-                                                float* qkv, float* h_out, int M, int N) {
+                                                float* qkv, float* h_out, int M, int N, tb_share share) {
     __shared__ uint4 pl[3 * 8 * 64];
     __shared__ float4 red[256];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4;
-    const int m = blockIdx.x * 16 + fr, row = m < M ? m : M - 1, tile = (blockIdx.y * 8 + wave) * NT;
+    const int item = tb_item(share), rt = item / (12 / NT), part = item % (12 / NT);
+    const int m = rt * 16 + fr, row = m < M ? m : M - 1, tile = (part * 8 + wave) * NT;
     float4 v[2], lw[2], lb[2];
     uint4 wf[NT][8];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
         const int c = (wave * 2 + t) * 16 + kq * 4;
-        v[t] = PARTS ? tb_sum(parts + tb_at(blockIdx.x, wave, t, lane), ps, *reinterpret_cast<const float4*>(b2 + c))
+        v[t] = PARTS ? tb_sum(parts + tb_at(rt, wave, t, lane), ps, *reinterpret_cast<const float4*>(b2 + c))
                      : *reinterpret_cast<const float4*>(h + (size_t)row * TB_C + c);
         lw[t] = *reinterpret_cast<const float4*>(lnw + c);
         lb[t] = *reinterpret_cast<const float4*>(lnb + c);
     }
     tb_weights<8, NT>(wf, w, tile, 8, 0, lane);
-    if (PARTS && blockIdx.y == 0)
+    if (PARTS && part == 0)
 #pragma unroll
-        for (int t = 0; t < 2; ++t) *reinterpret_cast<float4*>(h_out + (size_t)(blockIdx.x * 16 + fr) * TB_C + (wave * 2 + t) * 16 + kq * 4) = v[t];
+        for (int t = 0; t < 2; ++t) *reinterpret_cast<float4*>(h_out + (size_t)(rt * 16 + fr) * TB_C + (wave * 2 + t) * 16 + kq * 4) = v[t];
     tb_layernorm(v, lw, lb, red, wave, lane);
 #pragma unroll
     for (int t = 0; t < 2; ++t) tb_put(pl, 8, wave, t, lane, v[t]);
@@ -4391,11 +4433,11 @@ __global__ __launch_bounds__(512) void k_tb_qkv(const float* h, const float* par
 // itself: a request is a row's 1 KB, and no LayerNorm sum waits for the other waves.  Else att = the attention rows, and the product is done here.
 template <bool OUT>
 __global__ __launch_bounds__(512) void k_tb_ff(const float* att, size_t os, const float* h, FlowPacked w, const float* b_out, const float* lnw, const float* lnb,
-                                               const float* b1, float* parts, size_t ps, int M) {
+                                               const float* b1, float* parts, size_t ps, int M, tb_share share) {
     __shared__ uint4 pl[3 * 16 * 64];
     __shared__ float4 red[OUT ? 1 : 256];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4, q = blockIdx.y;
-    const int m0 = blockIdx.x * 16, m = m0 + fr, row = m < M ? m : M - 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, fr = lane & 15, kq = lane >> 4;
+    const int item = tb_item(share), rt = item >> 2, q = item & 3, m0 = rt * 16, m = m0 + fr, row = m < M ? m : M - 1;
     uint4 w1[2][8], w2[2][8];
     float4 bh[2];
     f32x4 acc[2];
@@ -4418,7 +4460,7 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, size_t os, cons
 #pragma unroll
             for (int p = 1; p < 8; ++p) v[i][0] = tb_add(v[i][0], v[i][p]);
             float4 x = tb_add(res[i], tb_add(v[i][0], bo));
-            if (q == 0) *reinterpret_cast<float4*>(parts + TB_PARTS * ps + tb_at(blockIdx.x, kb, (lane >> 2) & 1, (lane & 3) * 16 + r)) = x;
+            if (q == 0) *reinterpret_cast<float4*>(parts + TB_PARTS * ps + tb_at(rt, kb, (lane >> 2) & 1, (lane & 3) * 16 + r)) = x;
             const float mean = tb_row_sum64((x.x + x.y) + (x.z + x.w)) / (float)TB_C;
             x = make_float4(x.x - mean, x.y - mean, x.z - mean, x.w - mean);
             const float var = tb_row_sum64((x.x * x.x + x.y * x.y) + (x.z * x.z + x.w * x.w));
@@ -4460,7 +4502,7 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, size_t os, cons
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
             n[t] = tb_add(res[t], tb_add(make_float4(acc[t][0], acc[t][1], acc[t][2], acc[t][3]), bo[t]));
-            if (q == 0) *reinterpret_cast<float4*>(parts + TB_PARTS * ps + tb_at(blockIdx.x, wave, t, lane)) = n[t];
+            if (q == 0) *reinterpret_cast<float4*>(parts + TB_PARTS * ps + tb_at(rt, wave, t, lane)) = n[t];
         }
         tb_layernorm(n, lw, lb, red, wave, lane);      // (its barriers: every wave has read the attention rows)
 #pragma unroll
@@ -4489,7 +4531,7 @@ __global__ __launch_bounds__(512) void k_tb_ff(const float* att, size_t os, cons
     tb_runs<8, 4, 2>(w2, hid, lane, y);
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
-        const size_t o = tb_at(blockIdx.x, wave, t, lane);
+        const size_t o = tb_at(rt, wave, t, lane);
         if (q == 0) {
             y[1][t] = y[0][t] + y[1][t];
         } else {
@@ -4532,11 +4574,10 @@ static bool tb_pack(const std::vector<vox_flow_tblock_w>& tb, int C, int inner, 
 }
 static size_t tb_plane(size_t M) { return (M + 15) / 16 * 16 * TB_C; }      // floats of a plane of M rows
 static float* tb_heads(float* ws, int M) { return ws + TB_PLANES * tb_plane(M); }
-// the attention of a fused block: leaves the out product's planes where its matrix-core form runs (true), else the attention rows.  While the feed-forward's
-// blocks have a CU each: with more, its shorter blocks gain less than the attention's longer ones lose (1032 rows, us, rows and planes: 15.0 + 22.7, 17.5
-// + 20.7; 1376 rows 15.5 + 23.2, 17.9 + 21.7; 2064 rows 25.9 + 33.3, 30.0 + 32.3).
+// the attention of a fused block: leaves the out product's planes where its matrix-core form runs (true), else the attention rows (ms, rows and planes:
+// CosyVoice2 1 request of 10 tokens 19.9, 19.1; 8 of 28 28.2, 28.0; 16 48.6, 47.0; 32 83.4, 81.3; GLM-4-Voice 6 of 25 49.3, 48.4; 32 148.0, 144.7)
 static bool tb_attn(hipStream_t st, FlowAttn a, const FlowPacked* pk, float* ws, int T, int H, int N) {
-    const bool parts = pk && H == TB_HEADS && (N * T + 15) / 16 * 4 <= 256 && flow_attn_mfma_takes(a, T);
+    const bool parts = pk && H == TB_HEADS && flow_attn_mfma_takes(a, T) && flow_attn_near(a, T, H, N);
     if (parts) { a.wo = pk->out; a.parts = tb_heads(ws, N * T); a.ps = tb_plane(N * T); }
     launch_flow_attn(st, a, T, H, N);
     return parts;
@@ -4547,14 +4588,15 @@ static void tb_qkv(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w&
     const size_t ps = tb_plane(M);
 #define TB_QKV(NT_) \
     do { \
-        const dim3 g(tiles, 3 * TB_IN / (128 * NT_)); \
-        if (!before) hipLaunchKernelGGL((k_tb_qkv<false, NT_>), g, dim3(512), 0, st, h, ws, nullptr, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN); \
+        const dim3 g(tiles * (12 / NT_)); \
+        const tb_share share = tb_shares(tiles * (12 / NT_)); \
+        if (!before) hipLaunchKernelGGL((k_tb_qkv<false, NT_>), g, dim3(512), 0, st, h, ws, nullptr, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws, M, 3 * TB_IN, share); \
         else hipLaunchKernelGGL((k_tb_qkv<true, NT_>), g, dim3(512), 0, st, h, ws, before->ff2.bias, ps, f.qkv, w.ln1_w, w.ln1_b, qkv, ws + (TB_PLANES - 1) * ps, M, \
-                                3 * TB_IN); \
+                                3 * TB_IN, share); \
     } while (0)
     // A block adds up its rows' planes (128 KB) whatever it multiplies them by (64 KB a tile of a wave): where two tiles a wave make more blocks than
-    // CUs, three or four move less as long as theirs fit.  896 rows, us (first / later blocks of a level), two, three, four tiles: 8.4 / 10.6, 7.4 /
-    // 9.1, 8.4 / 10.3; later blocks of 1032 rows, two, three, four: 14.2, 16.1, 11.4.
+    // CUs, three or four move less as long as theirs fit.  Detokenizers, ms, two, three and four tiles a wave: CosyVoice2 6 requests of 28 tokens
+    // (672 rows) 26.3, 26.9, 27.5; 7 (784) 28.3, 27.4, 28.1; 8 (896) 28.8, 28.1, 28.7; GLM-4-Voice 5 (860) 37.6, 36.7, 37.5; 6 (1032) 49.6, 51.8, 49.4.
     if (tiles * 6 <= 256 || tiles * 3 > 256) TB_QKV(2);
     else if (tiles * 4 <= 256) TB_QKV(3);
     else TB_QKV(4);
@@ -4565,9 +4607,10 @@ static void tb_ff(hipStream_t st, const FlowPacked& f, const vox_flow_tblock_w& 
                   bool from_parts) {
     const size_t ps = tb_plane(M);
     const float* in = first ? h : ws + (TB_PLANES - 1) * ps;
-    const dim3 g((M + 15) / 16, 4);
-    if (from_parts) hipLaunchKernelGGL(k_tb_ff<true>, g, dim3(512), 0, st, tb_heads(ws, M), ps, in, f, w.out.bias, w.ln3_w, w.ln3_b, w.ff1.bias, ws, ps, M);
-    else hipLaunchKernelGGL(k_tb_ff<false>, g, dim3(512), 0, st, att, 0, in, f, w.out.bias, w.ln3_w, w.ln3_b, w.ff1.bias, ws, ps, M);
+    const dim3 g((M + 15) / 16 * 4);
+    const tb_share share = tb_shares((M + 15) / 16 * 4);
+    if (from_parts) hipLaunchKernelGGL(k_tb_ff<true>, g, dim3(512), 0, st, tb_heads(ws, M), ps, in, f, w.out.bias, w.ln3_w, w.ln3_b, w.ff1.bias, ws, ps, M, share);
+    else hipLaunchKernelGGL(k_tb_ff<false>, g, dim3(512), 0, st, att, 0, in, f, w.out.bias, w.ln3_w, w.ln3_b, w.ff1.bias, ws, ps, M, share);
     if (last) hipLaunchKernelGGL(k_tb_join, dim3((unsigned)((M + 15) / 16 * 4)), dim3(256), 0, st, ws, w.ff2.bias, ps, h, M);
 }
 
