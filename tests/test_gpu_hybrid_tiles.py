@@ -132,11 +132,7 @@ def test_few_row_routed_forms(rows, over):
     W = kazozen.pack_weights(P.random_checkpoint(cfg, seed=3), base)
     n_out = layer.moe.experts + d.layers[-1].moe.identity
     g = torch.Generator().manual_seed(1)
-    for k in list(W):
-        if "router" in k and W[k].dim() == 2:
-            W[k] = torch.randn(n_out, W[k].shape[1], generator=g)
-        elif "correction" in k:
-            W[k] = torch.zeros(n_out)
+    W["layers"][-1]["moe"].update(router=torch.randn(n_out, d.width, generator=g), correction=torch.zeros(n_out))
     toks = torch.randint(0, 50, (9,), generator=g, dtype=torch.int32)
 
     def logits(cuts):

@@ -235,3 +235,17 @@ def test_oracle_routing_groups():
     assert pick(groups={"count": 2, "keep": 1}, top=3) == [(5, 0.38), (3, 0.21), (4, 0.06)]
     Q["correction"] = torch.tensor([-2.0, -2.0, -2.0, -3.0, -3.0, -3.0], dtype=torch.float64)
     assert pick(groups={"count": 2, "keep": 1}, top=2) == [(0, 0.3), (2, 0.22)]
+
+
+@pytest.mark.parametrize("over", [dict(identity=5), dict(experts=7), dict(ff=16)])
+def test_routed_weights_of_another_size_are_refused(over):
+    """A router with fewer rows than the layer has outputs would be read past its end."""
+    import dataclasses
+    from vox_serve_amd.engine_hybrid import check_routed
+    from vox_serve_amd.model.kazozen import config_from_dict, pack_weights
+    cfg = small()
+    c = config_from_dict(cfg)
+    e, w = c.layers[1].moe, pack_weights(P.random_checkpoint(cfg, seed=1), c)["layers"][1]["moe"]
+    check_routed(1, e, w, c.width)
+    with pytest.raises(ValueError, match="layer 1"):
+        check_routed(1, dataclasses.replace(e, **over), w, c.width)

@@ -300,6 +300,17 @@ def reduced_bigram(bigram) -> tuple:
     return (n, a % n, b % n)
 
 
+def check_routed(layer, e, w, width):
+    """The tensors of a routed feed-forward have the sizes that its kernels read: router rows for every output, those without an expert among them."""
+    n, units = e.experts + e.identity, 1 if e.expert_form == "up_down" else 2
+    sizes = {"router": n * width, "correction": n, "router_bias": n, "w_gate_up": e.experts * units * e.ff * width, "w_down": e.experts * e.ff * width,
+             "shared_gate_up": units * e.shared_ff * width, "shared_down": e.shared_ff * width}
+    for name, size in sizes.items():
+        t = w.get(name)
+        if t is not None and t.numel() != size:
+            raise ValueError(f"layer {layer}: {name} {tuple(t.shape)}, {e.experts} experts, {e.identity} outputs without one, inner width {e.ff}, width {width}")
+
+
 class HybridEngine(Qwen3Engine):
     """`weights`: {"embedding", "head", "final_norm", "loop_in" (or None), "layers": [per layer dict with norm1, norm2, w_in,
     b_in, w_out, lower, head_norm, w_up, w_down, b_up, b_down; per mixer kind also q_norm, k_norm | conv_w, conv_b, w_gates, b_gates,
@@ -411,6 +422,7 @@ class HybridEngine(Qwen3Engine):
                 c.decay = vec(torch.tensor([float(a) for a in m.decay], dtype=torch.float32))
             if m.moe is not None:
                 e, ew = m.moe, lw["moe"]
+                check_routed(i, e, ew, W)
                 mc = HybridMoEC(e.experts, e.identity, e.top, e.ff, e.shared_ff, e.limit, e.shared_limit, e.act_alpha,
                                 vec(ew["router"]), vec(ew.get("correction")), mat(ew.get("w_gate_up")), mat(ew.get("w_down")),
                                 mat(ew.get("shared_gate_up")), mat(ew.get("shared_down")), ROUTER_SCORES[e.score], int(e.renorm),
