@@ -574,6 +574,13 @@ typedef struct {
 } vox_hybrid_io;
 int vox_hybrid_create(vox_ctx* ctx, const vox_hybrid_config* cfg, const vox_hybrid_weights* w, vox_hybrid** out);
 void vox_hybrid_destroy(vox_hybrid* m);
+/* on: steps take the launches that serve any size in the place of those for some sizes (units and routed layers of few rows, window attention of whole
+ * key heads, activations behind gate and up products, rows left as bf16 by the launch before, every product tile but the smallest).  Both give the
+ * same bits: what a check of one against the other sets. */
+void vox_hybrid_set_general(vox_hybrid* m, int on);
+/* the tile that a bf16 product of more than 16 rows takes: rows << 16 | columns.  kind: 0 = plain, 1 = gate and up columns with their activation (n: columns
+ * behind it), 2 = a sum that joins gated or several residual streams; groups: products in the launch (routed experts), `rows` of each. */
+int vox_hybrid_tile(int kind, int rows, int n, int k, int groups);
 /* ids: [n_rows] token ids of the rows.  max_kvlen: a bound on (position + 1) of every row (grid bound of the attention; 0 = the
  * engine's max_seq_len).  sampling NULL: logits only; else one pick per request from output rows 0..n_req-1. */
 int vox_hybrid_step(vox_hybrid* m, void* stream, const vox_hybrid_io* io, const int32_t* ids, int n_rows, int n_req, int n_out,

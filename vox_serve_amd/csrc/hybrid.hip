@@ -812,14 +812,19 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_hb_gemm_dma(const bf16_t* A
         for (int i = 0; i < MT; ++i)
 #pragma unroll
             for (int j = 0; j < NT; ++j) {
-                const int gn = n0 + (wn * NT + j) * 16 + fr;
-                if (gn >= N) continue;
+                // (HB_EPI_JOIN: what four rows read is asked for before the first of them is written)
+                const int gn = n0 + (wn * NT + j) * 16 + fr, gm = m0 + (wm * MT + i) * 16 + fk * 4;
+                if (gn >= N || gm >= M) continue;
                 const float b = bias ? bias[gn] : 0.f;
+                hb_join_in in[4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const int gm = m0 + (wm * MT + i) * 16 + fk * 4 + r;
-                    if (gm < M) hb_finish<EPI>(rm, C, ldc, LIST ? lst[gm] : gm, gn, acc[i][j][r], b);
+                    const int row = gm + r < M ? gm + r : M - 1;
+                    in[r] = hb_join_load(rm.join, C + (size_t)row * ldc, row, gn);
                 }
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (gm + r < M) hb_join_apply(rm.join, in[r], C + (size_t)(gm + r) * ldc, gm + r, gn, acc[i][j][r] + b);
             }
     }
 }
@@ -1302,10 +1307,11 @@ template <int EPI>
 bool hb_try_rows16(hipStream_t, const float*, long, const float*, const float*, float*, long, int, int, int, const hb_rowmap&, int) { return false; }
 
 static inline int hb_tile_count(int M, int N, int bm, int bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); }
-// room for the rows of a product rounded to bf16
+// room for the rows of a product rounded to bf16; general: vox_hybrid_set_general
 struct hb_ws16 {
     bf16_t* p;
     size_t n;
+    bool general;
 };
 __global__ __launch_bounds__(256) void k_hb_to_bf16(const float* A, long lda, bf16_t* out, int K8, size_t n8) {
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < n8; i += (size_t)gridDim.x * 256) {
@@ -1322,29 +1328,42 @@ static inline bool hb_dma_ok(const bf16_t* W, size_t a_rows, size_t N, int K, co
 // (less than one where two blocks fit a CU).  Measured at K = 512, 2048 and 5632, N = 512 to 11264, 20 to 2048 rows.
 struct hb_tile {
     int bm, bn;
-    float step, fixed, next;
+    float step, fixed, next;      // step 0: not a form of this kind of product
 };
-static inline float hb_tile_ns(const hb_tile& t, int rows, int N, int K, int groups, int cols) {
-    const int blocks = hb_tile_count(rows, N, t.bm, t.bn / cols) * groups, rounds = (blocks + 255) / 256;
-    return (K / 64 * t.step + t.fixed) * (1.0f + (rounds - 1) * t.next);
-}
+enum { HB_TILE_PLAIN = 0, HB_TILE_GLU = 1, HB_TILE_JOIN = 2 };
+static const hb_tile HB_TILES[3][9] = {
+    {{32, 32, 160.f, 2600.f, 0.6f}, {64, 32, 195.f, 2900.f, 0.65f}, {64, 64, 290.f, 2300.f, 0.72f}, {128, 64, 420.f, 2400.f, 0.84f}, {128, 128, 527.f, 5300.f, 1.f},
+     {192, 128, 625.f, 5800.f, 1.f}, {256, 128, 710.f, 7500.f, 1.f}, {256, 192, 1120.f, 7000.f, 1.f}, {256, 160, 780.f, 9500.f, 1.f}},
+    {{32, 64, 190.f, 2600.f, 0.7f}, {64, 32, 0.f, 0.f, 0.f}, {64, 64, 290.f, 2300.f, 0.72f}, {128, 64, 420.f, 2400.f, 0.84f}, {128, 128, 527.f, 5300.f, 1.f},
+     {192, 128, 625.f, 5800.f, 1.f}, {256, 128, 710.f, 7500.f, 1.f}, {256, 192, 1120.f, 7000.f, 1.f}, {256, 160, 0.f, 0.f, 0.f}},
+    // HB_EPI_JOIN: its epilogue, which waits for what it reads, is most of a block's time (costs fitted to whole steps); over 128 x 128 it would keep 208 to
+    // 400 bytes of scratch a lane.  Prompt steps of four Gaparax layers, us, all sums that join in 32 x 32, 64 x 32, 64 x 64, 128 x 64, 128 x 128: width 1024,
+    // 200 rows 464, 493, 537, 635, 662; 1024 rows 1031, 995, 1016, 1136, 1156; 2048 rows 1788, 1721, 1672, 1764, 1773; width 2048, 700 rows 1536, 1506, 1472,
+    // 1543, 1575; 2048 rows 3604, 3361, 3204, 3131, 3110.
+    {{32, 32, 160.f, 6400.f, 0.52f}, {64, 32, 195.f, 11900.f, 0.46f}, {64, 64, 290.f, 17300.f, 0.36f}, {128, 64, 0.f, 0.f, 0.f}, {128, 128, 527.f, 28700.f, 0.7f},
+     {192, 128, 0.f, 0.f, 0.f}, {256, 128, 0.f, 0.f, 0.f}, {256, 192, 0.f, 0.f, 0.f}, {256, 160, 0.f, 0.f, 0.f}}};
 // The tile whose blocks are through first by that measure, `rows` being the rows of a product as far as the host knows (a gathered one has fewer
 // than M): a wide tile moves fewer bytes per product, but a last round that is nearly empty costs as much as a full one.  Rows, N x K: tile
 // chosen, us, against the four forms of 64 and 128 that stood here before: 20, 2048 x 2048: 32 x 32, 7.4 (64 x 64 9.8); 200, 2048 x 5632: 64 x 32, 20 (25);
 // 300, 4096 x 2048: 128 x 64, 16 (21); 1024, 5120 x 2048: 192 x 128, 27 (44); 2048 rows: with the kernel.
-template <int EPI, bool GLU, bool LIST>
-void hb_launch_dma(hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
-                   const hb_rowmap& rm, int groups, int rows, hb_glu_args glu = hb_glu_args{}) {
-    constexpr int G = GLU ? 2 : 1;
-    static const hb_tile T[] = {{32, GLU ? 64 : 32, GLU ? 190.f : 160.f, 2600.f, GLU ? 0.7f : 0.6f}, {64, 32, 195.f, 2900.f, 0.65f}, {64, 64, 290.f, 2300.f, 0.72f},
-                                {128, 64, 420.f, 2400.f, 0.84f}, {128, 128, 527.f, 5300.f, 1.f}, {192, 128, 625.f, 5800.f, 1.f},
-                                {256, 128, 710.f, 7500.f, 1.f}, {256, 192, 1120.f, 7000.f, 1.f}, {256, 160, 780.f, 9500.f, 1.f}};
+static int hb_pick_tile(int kind, int rows, int N, int K, int groups) {
     int best = 0;
     float ns = 0.f;
-    for (int i = 0; i < (GLU ? 8 : 9); ++i) {
-        const float v = hb_tile_ns(T[i], rows, N, K, groups, G);
+    for (int i = 0; i < 9; ++i) {
+        const hb_tile& t = HB_TILES[kind][i];
+        if (t.step == 0.f) continue;
+        const int blocks = hb_tile_count(rows, N, t.bm, kind == HB_TILE_GLU ? t.bn / 2 : t.bn) * groups, rounds = (blocks + 255) / 256;
+        const float v = (K / 64 * t.step + t.fixed) * (1.0f + (rounds - 1) * t.next);
         if (i == 0 || v < ns) { best = i; ns = v; }
     }
+    return best;
+}
+template <int EPI, bool GLU, bool LIST>
+void hb_launch_dma(hb_ws16 ws, hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K,
+                   const hb_rowmap& rm, int groups, int rows, hb_glu_args glu = hb_glu_args{}) {
+    constexpr int G = GLU ? 2 : 1;
+    constexpr bool JOIN = EPI == HB_EPI_JOIN;
+    const int best = ws.general ? 0 : hb_pick_tile(GLU ? HB_TILE_GLU : JOIN ? HB_TILE_JOIN : HB_TILE_PLAIN, rows, N, K, groups);
 #define HB_DMA(BM_, BN_, WM_, WN_, S_) \
     do { \
         constexpr int lds = S_ * (BM_ + BN_) * 128; \
@@ -1358,15 +1377,19 @@ void hb_launch_dma(hipStream_t st, const bf16_t* A, long lda, const bf16_t* W, c
         if constexpr (GLU) HB_DMA(32, 64, 2, 2, 6);
         else HB_DMA(32, 32, 2, 2, 8);
         break;
-    case 1: HB_DMA(64, 32, 4, 1, 6); break;
+    case 1:
+        if constexpr (!GLU) HB_DMA(64, 32, 4, 1, 6);
+        break;
     case 2: HB_DMA(64, 64, 2, 2, 4); break;
-    case 3: HB_DMA(128, 64, 2, 2, 3); break;
     case 4: HB_DMA(128, 128, 4, 2, 4); break;
-    case 5: HB_DMA(192, 128, 4, 2, 3); break;
-    case 6: HB_DMA(256, 128, 4, 2, 3); break;
-    case 7: HB_DMA(256, 192, 4, 2, 2); break;
     default:
-        if constexpr (!GLU) HB_DMA(256, 160, 4, 2, 3);
+        if constexpr (!JOIN) {
+            if (best == 3) HB_DMA(128, 64, 2, 2, 3);
+            else if (best == 5) HB_DMA(192, 128, 4, 2, 3);
+            else if (best == 6) HB_DMA(256, 128, 4, 2, 3);
+            else if (best == 7) HB_DMA(256, 192, 4, 2, 2);
+            else if constexpr (!GLU) HB_DMA(256, 160, 4, 2, 3);
+        }
     }
 #undef HB_DMA
 }
@@ -1381,7 +1404,7 @@ static const bf16_t* hb_rows16(hipStream_t st, hb_ws16 ws, const hb_rowmap& rm, 
 }
 // hb_gemm reads A as bf16 anyway (and the workspace has room for its rows)
 static inline bool hb_takes16(const bf16_t* W, hb_ws16 ws, int M, int N, int K) {
-    return M > 16 && hb_dma_ok(W, M, N, K, hb_plain()) && (size_t)M * K <= ws.n;
+    return M > 16 && !ws.general && hb_dma_ok(W, M, N, K, hb_plain()) && (size_t)M * K <= ws.n;
 }
 static inline bool hb_takes16(const float*, hb_ws16, int, int, int) { return false; }
 // rm.count != NULL: `groups` gathered GEMMs of at most M rows each (about `rows`) in one launch (see hb_rowmap), their rows among the first
@@ -1394,8 +1417,8 @@ int hb_gemm_tiles(hb_ws16 ws, hipStream_t st, const float* A, long lda, const bf
     if (M > 16 && (groups == 1 || (rm.count && EPI == HB_EPI_STORE)) && hb_dma_ok(W, a_rows, N, K, rm)) {
         long ld16 = lda;
         if (const bf16_t* a16 = hb_rows16(st, ws, rm, A, ld16, a_rows, K)) {
-            if (!rm.count) hb_launch_dma<EPI, false, false>(st, a16, ld16, W, bias, C, ldc, M, N, K, rm, 1, rows);
-            else if constexpr (EPI == HB_EPI_STORE) hb_launch_dma<EPI, false, true>(st, a16, ld16, W, bias, C, ldc, M, N, K, rm, groups, rows);
+            if (!rm.count) hb_launch_dma<EPI, false, false>(ws, st, a16, ld16, W, bias, C, ldc, M, N, K, rm, 1, rows);
+            else if constexpr (EPI == HB_EPI_STORE) hb_launch_dma<EPI, false, true>(ws, st, a16, ld16, W, bias, C, ldc, M, N, K, rm, groups, rows);
             return VOX_OK;
         }
     }
@@ -1414,11 +1437,11 @@ int hb_gemm_tiles(hb_ws16, hipStream_t st, const float* A, long lda, const float
 // of W, Wu = the next.  false: these operands do not allow it (the two steps are the caller's).  K_next: columns of the product that reads y.
 static bool hb_try_glu(hb_ws16 ws, hipStream_t st, const float* A, long lda, int a_rows, const bf16_t* W, const float* bias, void* y, int M, int ff, int K,
                        const bf16_t* w_next, int n_next, const hb_rowmap& rm, int groups, int rows, size_t y_rows, hb_glu_args glu) {
-    if (M <= 16 || !hb_dma_ok(W, a_rows, 2 * (size_t)ff, K, rm) || !hb_dma_ok(w_next, y_rows, n_next, ff, rm)) return false;
+    if (M <= 16 || ws.general || !hb_dma_ok(W, a_rows, 2 * (size_t)ff, K, rm) || !hb_dma_ok(w_next, y_rows, n_next, ff, rm)) return false;
     const bf16_t* a16 = hb_rows16(st, ws, rm, A, lda, a_rows, K);
     if (!a16) return false;
-    if (rm.count) hb_launch_dma<HB_EPI_STORE, true, true>(st, a16, lda, W, bias, (float*)y, ff, M, ff, K, rm, groups, rows, glu);
-    else hb_launch_dma<HB_EPI_STORE, true, false>(st, a16, lda, W, bias, (float*)y, ff, M, ff, K, rm, 1, rows, glu);
+    if (rm.count) hb_launch_dma<HB_EPI_STORE, true, true>(ws, st, a16, lda, W, bias, (float*)y, ff, M, ff, K, rm, groups, rows, glu);
+    else hb_launch_dma<HB_EPI_STORE, true, false>(ws, st, a16, lda, W, bias, (float*)y, ff, M, ff, K, rm, 1, rows, glu);
     return true;
 }
 static bool hb_try_glu(hb_ws16, hipStream_t, const float*, long, int, const float*, const float*, void*, int, int, int, const float*, int, const hb_rowmap&, int,
@@ -4861,7 +4884,7 @@ __global__ __launch_bounds__(256) void k_hb_moe_router(const float* h, long ldh,
         wgt[(size_t)row * top + k] = (renorm ? sc[pick[k]] / den : sc[pick[k]]) * wscale;
     }
 }
-// Block e lists the entries (row*top + k) routed to expert e, ascending: list[e*cap + 0 .. count[e]).  A round of 1024 entries costs two barriers and a
+// Block e lists the entries (row*top + k) routed to expert e, ascending: list[e*cap + 0 .. count[e]).  A round of 1024 entries costs a barrier and a
 // trip to memory: 4096 entries, 256 threads 11.2 us, this 5.2.
 __global__ __launch_bounds__(1024) void k_hb_moe_group(const int* sel, int n_entries, int cap, int* list, int* count) {
     __shared__ int wsum[2][16];
@@ -4998,7 +5021,8 @@ __global__ __launch_bounds__(256) void k_hb_moe_down_combine(const float* h, lon
 // x[row] += sum_k wgt[row*top + k] * (identity output ? h[row] : expert_out[row*top + k]), k ascending
 // (scale_input: an expert's output enters with weight 1, its input was scaled instead)
 // An entry's place does not depend on its choice, so its row is asked for beside it; four columns a thread where everything lies on 16 bytes (vec).
-// 2048 rows of 2048, top 2: 22.3 -> 11.8 us.
+// What four columns join is read before the first of them is written: 2048 rows, top 2, us: of 2048 22.3 -> 11.8; into two gated streams, of 2048 55.5 ->
+// 42.4, of 1024 21.7 -> 22.0 (28.7 with each column's reads behind the writes of the one before).
 __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, const float* h, long ldh, const float* eo, const int* sel,
                                                         const float* wgt, int top, int experts, int W, int scale_input, hb_join join, int vec) {
     const int row = blockIdx.x;
@@ -5016,9 +5040,13 @@ __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, cons
             }
             if (join.store && !join.gate && !join.scale && join.streams == 0)
                 *(float4*)(x + (size_t)row * ldx + i) = make_float4(0.f + a[0], 0.f + a[1], 0.f + a[2], 0.f + a[3]);
-            else
+            else {
+                hb_join_in in[4];
 #pragma unroll
-                for (int c = 0; c < 4; ++c) hb_join_add(join, x + (size_t)row * ldx, row, i + c, a[c]);
+                for (int c = 0; c < 4; ++c) in[c] = hb_join_load(join, x + (size_t)row * ldx, row, i + c);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) hb_join_apply(join, in[c], x + (size_t)row * ldx, row, i + c, a[c]);
+            }
         }
         return;
     }
@@ -5408,7 +5436,7 @@ struct vox_hybrid {
     int *moe_sel = nullptr, *moe_list = nullptr, *moe_count = nullptr;
     bf16_t* logits16 = nullptr;
     bf16_t* x16 = nullptr;                  // [max_rows][2 width]: the rows of a post-normed stream rounded to bf16, at its stride
-    hb_ws16 ws16{nullptr, 0};               // [max_rows][widest operand]: rows of a product rounded to bf16
+    hb_ws16 ws16{nullptr, 0, false};             // [max_rows][widest operand]: rows of a product rounded to bf16
     float* attn_ws = nullptr;
     size_t attn_ws_bytes = 0;
     int max_in = 0, max_mix = 0, max_ff = 0;
@@ -5631,11 +5659,11 @@ static int hb_sig_attention(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* 
 // multiple of 8, or above 256).
 // o16 != NULL: the rows may be left as bf16 there instead of in out; says so in *as16
 static bool hb_try_win_mfma(hipStream_t st, const vox_hybrid_io* io, const vox_hybrid_layer& L, const bf16_t* cache, const float* q, long ldp,
-                            float* out, long ldo, const hb_sink& sink, const float* gate, long v_base, int n, int n_req, int ps, bf16_t* o16, bool* as16) {
+                            float* out, long ldo, const hb_sink& sink, const float* gate, long v_base, int n, int n_req, int ps, bf16_t* o16, bool* as16, bool general) {
     if ((L.dim & 7) || (L.vdim & 7) || L.dim > 256 || L.vdim > 256 || (ldp & 3) || ((size_t)q & 15) || ((size_t)cache & 15)) return false;
     const int hpg = L.heads / L.kv_heads;
     // a lane's whole row pieces, heads that fill a block's columns: the form that loads a tile for all of them
-    if (L.dim == L.vdim && (L.dim == 64 || L.dim == 128) && (hpg & (hpg - 1)) == 0 && hpg <= 64 && (ldo & 3) == 0 && ((size_t)out & 15) == 0 && ((size_t)gate & 15) == 0) {
+    if (!general && L.dim == L.vdim && (L.dim == 64 || L.dim == 128) && (hpg & (hpg - 1)) == 0 && hpg <= 64 && (ldo & 3) == 0 && ((size_t)out & 15) == 0 && ((size_t)gate & 15) == 0) {
         const int hsh = __builtin_ctz(hpg), br = 64 >> hsh, lds = 2 * 2 * 64 * L.dim * 2;
         const dim3 g2(L.kv_heads, (n + (br - 1) * n_req) / br);       // (at least the sum of the requests' tiles)
         const bool near = (ps & (ps - 1)) == 0 && (size_t)v_base * 2 < (1ull << 32);      // (v_base: what the keys take, and the values)
@@ -5663,7 +5691,7 @@ static bool hb_try_win_mfma(hipStream_t st, const vox_hybrid_io* io, const vox_h
     return true;
 }
 static bool hb_try_win_mfma(hipStream_t, const vox_hybrid_io*, const vox_hybrid_layer&, const float*, const float*, long, float*, long, const hb_sink&,
-                            const float*, long, int, int, int, bf16_t*, bool*) { return false; }
+                            const float*, long, int, int, int, bf16_t*, bool*, bool) { return false; }
 // keys a position can see at most
 static int hb_win_keys(const vox_hybrid_layer& L, int max_kvlen) {
     return L.window > 0 && L.window < max_kvlen - L.keep_first ? L.window + L.keep_first : max_kvlen;
@@ -5675,7 +5703,7 @@ static int hb_win_attention(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* 
     const hb_sink sink{L.sinks ? 1 : 0, L.sinks};
     const float* gate = L.out_gate ? m->proj + H * L.dim + (L.kv_shared ? 0 : G * (L.dim + L.vdim)) : nullptr;
     const bool few = n <= HB_ATTN_SEG_ROWS;
-    if (!few && hb_try_win_mfma(st, io, L, cache, m->proj, ldp, m->mix, (long)n_mix, sink, gate, v_base, n, n_req, ps, o16, as16)) return VOX_OK;
+    if (!few && hb_try_win_mfma(st, io, L, cache, m->proj, ldp, m->mix, (long)n_mix, sink, gate, v_base, n, n_req, ps, o16, as16, m->ws16.general)) return VOX_OK;
     const int hpb = hb_sig_heads(L);
     const int nchunks = (hb_win_keys(L, max_kvlen) + 63) / 64;
     const int want = few ? (nchunks < HB_SIG_MAX_SEG ? nchunks : HB_SIG_MAX_SEG) : 1, cpb = (nchunks + want - 1) / want, nseg = (nchunks + cpb - 1) / cpb;
@@ -5686,7 +5714,7 @@ static int hb_win_attention(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* 
     hipLaunchKernelGGL((k_hb_win_attn_rows<T, HPB_>), dim3(n, H / HPB_, nseg), dim3(256), lds, st, m->proj, ldp, cache, m->mix, (long)n_mix, io->pos, \
                        io->row_req, io->page_table, io->pt_stride, H, G, L.dim, L.vdim, ps, v_base, hb_win{L.window, L.keep_first}, L.scale, sink, cpb, \
                        part, gate, ldp, L.out_scale)
-    if (sizeof(T) == 2 && hpb == 4 && L.dim == 128 && L.vdim == 128 && !((size_t)cache & 15) && !((size_t)m->proj & 15) && !(ldp & 3))
+    if (sizeof(T) == 2 && !m->ws16.general && hpb == 4 && L.dim == 128 && L.vdim == 128 && !((size_t)cache & 15) && !((size_t)m->proj & 15) && !(ldp & 3))
         hipLaunchKernelGGL(k_hb_win_attn_rows4, dim3(n, H / 4, nseg), dim3(256), 0, st, m->proj, ldp, (const bf16_t*)cache, m->mix, (long)n_mix, io->pos, io->row_req,
                            io->page_table, io->pt_stride, H, G, ps, v_base, hb_win{L.window, L.keep_first}, L.scale, sink, cpb, part, gate, ldp, L.out_scale);
     else if (hpb == 4) HB_WR(4);
@@ -6050,7 +6078,7 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
     hipLaunchKernelGGL(router, dim3(n), dim3(256), (size_t)(6 * nE + top + (E.groups > 1 ? E.groups : 0)) * 4, st, h2, ldh, E.router, E.correction, W, nE, top,
                        m->moe_sel, m->moe_wgt, E.score_kind == VOX_ROUTER_SIGMOID ? 1 : 0, E.renorm, E.router_bias, E.groups, E.keep,
                        E.weight_scale != 0.f ? E.weight_scale : 1.0f, E.group_best_two, post, post.y ? const_cast<float*>(h2) : (float*)nullptr);
-    if (n <= HB_MOE_GEMV_ROWS && !up_down && !L.res_gate && E.shared_ff == 0 &&
+    if (n <= HB_MOE_GEMV_ROWS && !m->ws16.general && !up_down && !L.res_gate && E.shared_ff == 0 &&
         hb_try_moe_rows(st, h2, ldh, (const T*)E.w_gate_up, (const T*)E.w_down, m->moe_act, cur, ldx, n, W, ff, hb_glu_args{E.limit, E.act_alpha, E.up_offset, 0}, jn,
                         hb_entries{m->moe_sel, m->moe_wgt, top, E.experts, E.scale_input}))
         return VOX_OK;
@@ -6084,7 +6112,7 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
         }
         VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(m->ws16, st, m->moe_act, (long)ff, (const T*)E.w_down, nullptr, m->moe_out, (long)W, n, W, ff, down, E.experts, rows, ne));
     }
-    const int vec = !(W & 3) && !(ldx & 3) && !(ldh & 3) && !(((size_t)cur | (size_t)h2 | (size_t)m->moe_out) & 15) ? 1 : 0;
+    const int vec = !m->ws16.general && !(W & 3) && !(ldx & 3) && !(ldh & 3) && !(((size_t)cur | (size_t)h2 | (size_t)m->moe_out) & 15) ? 1 : 0;
     hipLaunchKernelGGL(k_hb_moe_combine, dim3(n), dim3(256), 0, st, cur, ldx, h2, ldh, m->moe_out, m->moe_sel, m->moe_wgt, top, E.experts, W,
                        E.scale_input, jn, vec);
     if (E.shared_ff > 0) {
@@ -6117,7 +6145,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
     float *cur = m->xa, *other = m->xb;
     hb_pending pd{};
     pd.ldx = ldx;
-    pd.buf16 = n > 16 ? m->x16 : nullptr;
+    pd.buf16 = n > 16 && !m->ws16.general ? m->x16 : nullptr;
     for (int ri = 0; ri < c.n_runs; ++ri) {
         const vox_hybrid_run& run = m->runs[ri];
         const vox_hybrid_layer& L = m->layers[run.layer];
@@ -6202,7 +6230,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
                 const int gelu = L.ff_act == VOX_ACT_GELU_TANH ? 1 : 0;
                 hb_rowmap rm = hb_plain();
                 if (post) rm.a16 = pd.x16;
-                if (hb_try_ff_rows(st, hd, ldf, (const T*)L.w_up, L.b_up, (const T*)L.w_down, L.b_down, m->ff_act, dst, ldd, n, W, L.ff,
+                if (!m->ws16.general && hb_try_ff_rows(st, hd, ldf, (const T*)L.w_up, L.b_up, (const T*)L.w_down, L.b_down, m->ff_act, dst, ldd, n, W, L.ff,
                                    hb_glu_args{limit, alpha, L.ff_up_offset, gelu}, j2, &whole)) {
                 } else if (hb_try_glu(m->ws16, st, hd, ldf, n, (const T*)L.w_up, L.b_up, m->ff_act, n, L.ff, W, (const T*)L.w_down, W, rm, 1, n, (size_t)n,
                                hb_glu_args{limit, alpha, L.ff_up_offset, gelu}))
@@ -6483,6 +6511,15 @@ void vox_hybrid_destroy(vox_hybrid* m) {
     (void)hipFree(m->moe_wgt); (void)hipFree(m->moe_sel); (void)hipFree(m->moe_act); (void)hipFree(m->moe_out);
     (void)hipFree(m->moe_list); (void)hipFree(m->moe_count);
     delete m;
+}
+
+void vox_hybrid_set_general(vox_hybrid* m, int on) {
+    if (m) m->ws16.general = on != 0;
+}
+int vox_hybrid_tile(int kind, int rows, int n, int k, int groups) {
+    if (kind < HB_TILE_PLAIN || kind > HB_TILE_JOIN || rows < 1 || n < 1 || k < 1 || groups < 1) return 0;
+    const hb_tile& t = HB_TILES[kind][hb_pick_tile(kind, rows, n, k, groups)];
+    return t.bm << 16 | t.bn;
 }
 
 int vox_hybrid_step(vox_hybrid* m, void* stream, const vox_hybrid_io* io, const int32_t* ids, int n_rows, int n_req, int n_out,

@@ -336,6 +336,8 @@ class HybridEngine(Qwen3Engine):
         L, vp, ci = self.L, ctypes.c_void_p, ctypes.c_int
         L.vox_hybrid_create.restype, L.vox_hybrid_create.argtypes = ci, [vp, ctypes.POINTER(HybridConfigC), ctypes.POINTER(HybridWeightsC), ctypes.POINTER(vp)]
         L.vox_hybrid_destroy.restype, L.vox_hybrid_destroy.argtypes = None, [vp]
+        L.vox_hybrid_set_general.restype, L.vox_hybrid_set_general.argtypes = None, [vp, ci]
+        L.vox_hybrid_tile.restype, L.vox_hybrid_tile.argtypes = ci, [ci] * 5
         L.vox_hybrid_step.restype, L.vox_hybrid_step.argtypes = ci, [vp, vp, ctypes.POINTER(HybridIO), vp, ci, ci, ci, ci, ctypes.POINTER(N.SamplingCfg), ctypes.c_uint64, ci]
         dev = self.device
         self._keep = []
