@@ -2,6 +2,9 @@
 
 A zero bias on q | k | v, which the fused blocks do not take, sends a block to the general launches and changes no sum."""
 import ctypes
+import os
+import subprocess
+import sys
 
 import numpy as np
 import pytest
@@ -88,3 +91,29 @@ def test_glm_blocks_add_as_the_general_launches(monkeypatch, B, T, blocks):
         mp.setattr(GM.N, "lib", lambda: _GeneralBlocks(lib, zeros, (4 + fc.est_mid) * blocks))
         general = mels()
     assert rms(got) > 0.3 and np.array_equal(got, general)
+
+
+def _mels(path):
+    from vox_serve_amd.tokenizer import cosyvoice_flow as CF
+    fc = FR.FlowCfg(vocab=200, enc_layers=1, up_layers=1, est_mid=1, est_blocks=2)
+    g = torch.Generator().manual_seed(3)
+    flow = CF.CosyVoice2Flow(FR.random_flow_weights(fc, seed=3), flow_plugin_cfg(fc), device="cuda:0", max_batch=2, max_T=40, max_prompt_T=48, seed=1)
+    try:
+        flow.set_prompt(torch.randint(0, 200, (1, 5), generator=g), 0.7 * torch.randn(1, 10, fc.mel, generator=g), torch.randn(1, fc.spk_dim, generator=g),
+                        noise=FR.cfm_noise(1, 0, fc.mel, 16))
+        np.save(path, flow.forward_chunk(torch.randint(0, 200, (2, 40), generator=g), noise=FR.cfm_noise(1, 1, fc.mel, 80)).cpu().numpy())
+    finally:
+        flow.close()
+
+
+def test_attention_of_four_waves_reaches_the_fused_blocks(tmp_path):
+    """VOX_FLOW_ATTN_WV=4 adds a query's keys in four parts instead of eight: other bits beyond 64 keys, the same mels.  (A process of its own: the switch is read once.)"""
+    if not torch.cuda.is_available():
+        pytest.skip("no GPU")
+    out = []
+    for waves in ("8", "4"):
+        path = tmp_path / f"{waves}.npy"
+        subprocess.run([sys.executable, "-c", f"from tests.test_gpu_flow_blocks_order import _mels; _mels({str(path)!r})"], check=True, timeout=100,
+                       cwd=os.path.dirname(os.path.dirname(os.path.abspath(__file__))), env=dict(os.environ, VOX_FLOW_ATTN_WV=waves))
+        out.append(np.load(path))
+    assert rms(out[0]) > 0.5 and not np.array_equal(*out) and rms(out[0] - out[1]) < 1e-4

@@ -1714,10 +1714,11 @@ static int rows_mt2_blocks() {
     static const int v = [] { const char* e = getenv("VOX_ROWS_MT2"); const int x = e ? atoi(e) : 1024; return x > 0 ? x : (1 << 30); }();
     return v;
 }
-// 16 x 16 output tiles above which a k_rows_gemm block takes 2 / 4 column tiles (VOX_ROWS_NT2 / VOX_ROWS_NT4)
+// 16 x 16 output tiles above which a k_rows_gemm block takes 2 / 4 column tiles where a call has 256 rows and more (VOX_ROWS_NT2; VOX_ROWS_NT4: at every row
+// count; 0: by the rule in conv_gemm)
 static int rows_nt_tiles(int which) {
     static const int v2 = [] { const char* e = getenv("VOX_ROWS_NT2"); return e ? atoi(e) : 256; }();
-    static const int v4 = [] { const char* e = getenv("VOX_ROWS_NT4"); return e ? atoi(e) : 512; }();
+    static const int v4 = [] { const char* e = getenv("VOX_ROWS_NT4"); return e ? atoi(e) : 0; }();
     return which ? v4 : v2;
 }
 static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const float* state, const int* slots, int n,
@@ -1745,7 +1746,7 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
         // outweigh the extra blocks — CosyVoice2 chunk 49.7 -> 46.6 ms at B=8, 36.6 -> 35.2 at B=4, unchanged at B=1), four above 512
         // (above 2048, and this: 8 requests of 28 tokens, 896 rows, 28.61 and 28.16 ms; 4 of 20 22.60, 22.54; 1 of 28 20.58 both), but above
         // 2048 below those 16 row tiles and from 1025 rows on (GLM-4-Voice's flow with 512 there too, 1032 rows 53.7 and 54.2 ms, 1376 rows 57.3, 57.8)
-        const int four = a.M >= 256 && a.M <= 1024 ? rows_nt_tiles(1) : 2048;
+        const int four = rows_nt_tiles(1) ? rows_nt_tiles(1) : a.M >= 256 && a.M <= 1024 ? 512 : 2048;
         int nt = tiles > four ? 4 : tiles > (a.M >= 256 ? rows_nt_tiles(0) : 1024) ? 2 : 1;
         while (nt > 1 && nt * kb > 16) nt >>= 1;
         const int mt = (tiles / nt >= rows_mt2_blocks() && kb <= 4 && (wv == 4 || nt <= 2)) ? 2 : 1;      // (the 8-wave sum buffer: MT NT <= 4)
@@ -4226,14 +4227,18 @@ static bool flow_attn_near(FlowAttn& a, int T, int H, int N) {
     a.inv_h = tb_inverse((T + 15) / 16);
     return true;
 }
+// VOX_FLOW_ATTN_WV=4: four waves x four key tiles, which leave their rows for the out product (A/B timing)
+static bool flow_attn_wv4() {
+    static const bool on = [] { const char* e = getenv("VOX_FLOW_ATTN_WV"); return e && atoi(e) == 4; }();
+    return on;
+}
 static bool flow_attn_mfma_takes(const FlowAttn& a, int T) { return !a.P && !a.bu && a.dk == 64 && a.Tc + T <= 256 && flow_attn_mfma_on(); }
 static void launch_flow_attn(hipStream_t st, const FlowAttn& a, int T, int H, int N) {
     const int S = a.Tc + T;
     const size_t lds = ((size_t)S * (2 * a.dk + 4) + 4 * ((S + 3) & ~3) + 4 * a.dk) * sizeof(float);
     if (flow_attn_mfma_takes(a, T)) {
-        static const bool wv4 = [] { const char* e = getenv("VOX_FLOW_ATTN_WV"); return e && atoi(e) == 4; }();      // A/B: four waves x four key tiles
         if (a.parts) hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, true>), dim3((T + 15) / 16 * H * N), dim3(512), 0, st, a);
-        else if (wv4) hipLaunchKernelGGL((k_flow_attn_mfma<64, 4, false>), dim3((T + 15) / 16, H, N), dim3(256), 0, st, a);
+        else if (flow_attn_wv4()) hipLaunchKernelGGL((k_flow_attn_mfma<64, 4, false>), dim3((T + 15) / 16, H, N), dim3(256), 0, st, a);
         else hipLaunchKernelGGL((k_flow_attn_mfma<64, 8, false>), dim3((T + 15) / 16, H, N), dim3(512), 0, st, a);
         return;
     }
@@ -4577,7 +4582,7 @@ static float* tb_heads(float* ws, int M) { return ws + TB_PLANES * tb_plane(M); 
 // the attention of a fused block: leaves the out product's planes where its matrix-core form runs (true), else the attention rows (ms, rows and planes:
 // CosyVoice2 1 request of 10 tokens 19.9, 19.1; 8 of 28 28.2, 28.0; 16 48.6, 47.0; 32 83.4, 81.3; GLM-4-Voice 6 of 25 49.3, 48.4; 32 148.0, 144.7)
 static bool tb_attn(hipStream_t st, FlowAttn a, const FlowPacked* pk, float* ws, int T, int H, int N) {
-    const bool parts = pk && H == TB_HEADS && flow_attn_mfma_takes(a, T) && flow_attn_near(a, T, H, N);
+    const bool parts = pk && H == TB_HEADS && !flow_attn_wv4() && flow_attn_mfma_takes(a, T) && flow_attn_near(a, T, H, N);
     if (parts) { a.wo = pk->out; a.parts = tb_heads(ws, N * T); a.ps = tb_plane(N * T); }
     launch_flow_attn(st, a, T, H, N);
     return parts;
