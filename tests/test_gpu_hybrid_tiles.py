@@ -23,7 +23,7 @@ def _gpu():
         pytest.skip("no GPU")
 
 
-# (rows, vocabulary): 128 x 128 on four waves (with remainders of 2 rows and 1 column), on eight waves, 64 x 64 with two stages, and one k-tile
+# (rows, vocabulary): 192 x 128 (remainders of 2 rows and 1 column), 128 x 64 twice, 192 x 128 of one k-tile, against the 64 x 64 that 17 rows take
 @pytest.mark.parametrize("rows,vocab,width", [(130, 16769, 128), (255, 14400, 192), (65, 19201, 128), (129, 28673, 64)])
 def test_a_row_has_the_same_logits_in_every_tile_form(rows, vocab, width):
     cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2)], width=width, vocab=vocab, bigram=None)
@@ -65,7 +65,7 @@ def test_activation_behind_both_products(rows, mlp):
 
 
 # K of the second product = the layer's inner width: one step into the second round of requests, two whole rounds, one step into the third,
-# three whole rounds and one step into a fourth; both forms of the kernel (up to eight rows and more)
+# three whole rounds and one step into a fourth; up to eight rows the unit's own launch, more the general one, which zeroes early
 @pytest.mark.parametrize("rows,inner", [(2, 2080), (16, 4096), (7, 4128), (8, 6144), (16, 6176)])
 def test_rounds_of_a_few_row_product(rows, inner):
     cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.dense(inner))], width=64, vocab=50)
@@ -79,15 +79,44 @@ def test_rounds_of_a_few_row_product(rows, inner):
     assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR
 
 
-# every tile: 32 x 32, 64 x 32, 128 x 64, 128 x 128, 192 x 128, 256 x 128, 256 x 192, 256 x 160 (whose columns do not divide among the waves), rows
-# and columns with remainders; fewer k-tiles than stages
+# The general few-row product where it zeroes late: up to eight rows of few columns, K = heads x 32 (a whole round of requests, a step into the second, two
+# whole rounds, a step into the fourth) ...
+@pytest.mark.parametrize("rows,heads", [(2, 64), (8, 65), (7, 128), (8, 193)])
+def test_rounds_of_a_few_row_product_of_few_columns(rows, heads):
+    cfg = P.config([P.attention(heads=heads, kv_heads=1, dim=8, vdim=32, size=50, keep=2)], width=64, vocab=50)
+    S = P.random_checkpoint(cfg, seed=heads)
+    toks = torch.randint(0, 50, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
+    d = U.Driver(cfg, S, dtype=torch.bfloat16, page_size=16, pages=20, max_rows=rows)
+    try:
+        got = d.run_cut("r", toks, [rows])
+    finally:
+        d.close()
+    assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR
+
+
+# ... and of many columns, K = width: a few steps, a whole round
+@pytest.mark.parametrize("rows,width", [(2, 96), (7, 2048)])
+def test_few_row_product_of_many_columns(rows, width):
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2)], width=width, vocab=8200)
+    S = P.random_checkpoint(cfg, seed=width)
+    toks = torch.randint(0, 8200, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
+    d = U.Driver(cfg, S, dtype=torch.bfloat16, page_size=16, pages=20, max_rows=rows)
+    try:
+        got = d.run_cut("r", toks, [rows])
+    finally:
+        d.close()
+    assert U.rel_err(got, KR.forward(cfg, S, toks)) < BF16_BAR
+
+
+# the other tiles: 32 x 32, 64 x 32, 128 x 64, 128 x 128, 192 x 128, 256 x 128, 256 x 192, 256 x 160 (whose columns do not divide among the waves), rows
+# and columns with remainders; most with fewer k-tiles than stages (a stage that is filled again: test_gpu_hybrid_order.py)
 @pytest.mark.parametrize("rows,vocab,width", [(33, 515, 192), (63, 6145, 512), (65, 8193, 64), (65, 16769, 256), (129, 24001, 64), (255, 28673, 128),
                                               (257, 16769, 192), (257, 16769, 512)])
 def test_a_row_has_the_same_logits_in_every_tile(rows, vocab, width):
     test_a_row_has_the_same_logits_in_every_tile_form(rows, vocab, width)
 
 
-# gate and up products in 64 x 64, 192 x 128 and 256 x 192, columns that are no multiple of a block's
+# gate and up products in 64 x 64, 192 x 128 and 256 x 192, columns that are no multiple of a block's, one k-tile
 @pytest.mark.parametrize("rows,mlp", [(300, P.dense(1088)), (129, P.dense(8384)), (300, P.dense(11328)), (257, P.dense(16448)), (131, P.moe(4, 4, 5632, 0, 0))])
 def test_activation_behind_both_products_in_every_tile(rows, mlp):
     test_activation_behind_both_products(rows, mlp)
@@ -163,11 +192,12 @@ def test_window_attention_of_few_rows(heads, kv, page, window, keep, cuts):
 
 
 # Stacks of post-normed layers, more than 16 rows: the rows that every product reads are left as bf16 by the norm before it (rows of one, two and four
-# pieces of 1024 columns, and of a width that it takes element by element); entries of an expert listed in one round and in several
+# pieces of 1024 columns, and of a width that it takes element by element); up to 6300 entries, listed in one round of 1024 and in several.  (All experts
+# are chosen: no choice that bf16 rounding could flip, so every row counts.)
 @pytest.mark.parametrize("rows,width", [(17, 64), (40, 1088), (33, 2112), (20, 70), (700, 128)])
 def test_stack_of_post_normed_layers(rows, width):
     a = dict(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2)
-    cfg = P.config([P.attention(mlp=P.dense(128), **a), P.attention(mlp=P.moe(4, 2, 64, 0, 0), kv_from=0, **a), P.attention(mlp=P.moe(9, 3, 64, 3, 2), **a)], width=width,
+    cfg = P.config([P.attention(mlp=P.dense(128), **a), P.attention(mlp=P.moe(4, 4, 64, 0, 0), kv_from=0, **a), P.attention(mlp=P.moe(9, 9, 64, 3, 3), **a)], width=width,
                    vocab=50)
     S = P.random_checkpoint(cfg, seed=width)
     toks = torch.randint(0, 50, (rows,), generator=torch.Generator().manual_seed(rows)).tolist()
@@ -176,5 +206,5 @@ def test_stack_of_post_normed_layers(rows, width):
         got = d.run_cut("r", toks, [rows])
     finally:
         d.close()
-    err = U.rel_err(got, KR.forward(cfg, S, toks), 0.8)      # (a choice that bf16 rounding flips moves a whole row, in each of two layers)
+    err = U.rel_err(got, KR.forward(cfg, S, toks))
     assert err < BF16_BAR, err
