@@ -116,11 +116,12 @@ def test_dense_units_of_few_rows(width, ff, cuts):
     check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)
 
 
-# 2 to 8 rows, routed layers: rows of one piece, of a few columns into the next, of two whole rounds; one, two and up to 64 entries; more
-# choices than experts' halves; inner widths of one and several rounds
-@pytest.mark.parametrize("width,moe,cuts", [(64, (2, 2, 64, 0, 0), [2, 8, 3]), (512, (3, 1, 2048, 0, 0), [8, 7]), (2048, (8, 2, 2048, 4, 2), [8, 2, 5]),
-                                            (2056, (4, 2, 64, 0, 0), [8, 3]), (4096, (5, 5, 72, 0, 0), [7, 8, 2]), (3080, (4, 3, 520, 0, 0), [4, 6]),
-                                            (256, (48, 6, 128, 4, 2), [8, 6]), (64, (48, 16, 64, 0, 0), [3, 4]), (128, (16, 8, 40, 0, 0), [8, 8])])
+# 2 to 8 rows, routed layers of wide experts (inner widths of 2048 and more, or many weights in all): rows of one piece, of a few columns into the next, of
+# two whole rounds; one to 64 entries, an odd one at the end; inner widths of one round, a few columns into the next, two rounds, and less than one piece
+@pytest.mark.parametrize("width,moe,cuts", [(64, (2, 2, 2048, 0, 0), [2, 8, 3]), (512, (3, 1, 4096, 0, 0), [8, 7]), (2048, (8, 2, 2048, 4, 2), [8, 2, 5]),
+                                            (2056, (4, 2, 2048, 0, 0), [8, 3]), (4096, (5, 5, 2056, 0, 0), [7, 8, 2]), (3080, (4, 3, 2120, 0, 0), [4, 6]),
+                                            (256, (48, 6, 2048, 4, 2), [8, 6]), (64, (48, 16, 2048, 0, 0), [3, 4]), (128, (16, 8, 4104, 0, 0), [8, 8]),
+                                            (4096, (8, 8, 168, 0, 0), [8])])
 def test_routed_layers_of_few_rows(width, moe, cuts):
     cfg = P.config([P.attention(mlp=P.moe(*moe), **ATT), P.attention(mlp=P.moe(*moe), kv_from=0, **ATT)], width=width, vocab=50)
     check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)
@@ -130,7 +131,7 @@ def test_routed_layers_of_few_rows(width, moe, cuts):
 @pytest.mark.parametrize("rows", [2, 5, 8, 40])
 @pytest.mark.parametrize("over", [dict(identity=5), dict(scale_input=True)])
 def test_routed_forms(rows, over):
-    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.moe(6, 3, 64, 0, 0))], width=64, vocab=50)
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.moe(6, 3, 2048, 0, 0))], width=64, vocab=50)
     base = kazozen.config_from_dict(cfg)
     layer = base.layers[-1]
     d = dataclasses.replace(base, layers=[*base.layers[:-1], dataclasses.replace(layer, moe=dataclasses.replace(layer.moe, **over))])
@@ -168,7 +169,7 @@ def test_window_attention(heads, kv, dim, page, window, keep, cuts):
 # ... and of several requests beside each other
 @pytest.mark.parametrize("requests,cuts", [(2, [33, 4, 1]), (5, [70, 1, 2]), (8, [20, 1])])
 def test_window_attention_of_requests(requests, cuts):
-    cfg = P.config([P.attention(heads=8, kv_heads=2, dim=128, vdim=128, size=40, keep=3, mlp=P.moe(8, 2, 64, 4, 2)),
+    cfg = P.config([P.attention(heads=8, kv_heads=2, dim=128, vdim=128, size=40, keep=3, mlp=P.moe(8, 2, 2048, 4, 2)),
                     P.attention(heads=8, kv_heads=2, dim=128, vdim=128, size=40, keep=3, mlp=P.dense(96), kv_from=0)], width=256, vocab=50)
     check(cfg, P.random_checkpoint(cfg, seed=requests), sum(cuts) + 2, cuts, requests=requests)
 

@@ -5197,6 +5197,7 @@ __global__ __launch_bounds__(256) void k_hb_moe_up_rows(const float* h, long ldh
     auto load = [&](int c0) {
 #pragma unroll
         for (int c = 0; c < NC; ++c) {
+            if (512 * (c0 + c) >= W) break;
             const int k = lane * 8 + 512 * (c0 + c), o = k < W ? 512 * (c0 + c) : 0;
 #pragma unroll
             for (int r = 0; r < 4; ++r) wr[c][r] = *(const uint4*)(w[r] + (k < W || lane * 8 < W ? o : -lane * 8));
@@ -5231,6 +5232,7 @@ __global__ __launch_bounds__(256) void k_hb_moe_up_rows(const float* h, long ldh
             if (c0 > 0) load(c0);
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
+                if (512 * (c0 + c) >= W) break;
                 const int k = lane * 8 + 512 * (c0 + c);
                 if (k >= W) break;
                 float wf[4][8];
@@ -5273,7 +5275,7 @@ __global__ __launch_bounds__(256) void k_hb_moe_up_rows(const float* h, long ldh
 // x joins sum_k wgt_k * (identity ? h : down_{e_k} . act_k), k ascending: k_hb_moe_down_combine's sums, a wave per (row, column) like there, of activations that
 // are bf16 already (rounding them was most of that kernel's arithmetic).  The rows' blocks of four columns follow each other on one XCD, so an
 // expert's rows come from memory once and from that L2 for its other entries; a wave asks for two entries' rows at a time.
-// 8 rows, 2048 x 2048, 16 choices among 8 experts (67 MB of distinct rows): 22.0 -> 20.4 us.  Taken once per block, for all entries from LDS: 23.3 with one
+// 8 rows, 2048 x 2048, 16 choices among 8 experts (67 MB of distinct rows): 22.0 -> 18.3 us.  Taken once per block, for all entries from LDS: 23.3 with one
 // column a wave, 25.1 with two; that leaves too few waves for the sums, whose order keeps them off the matrix cores.
 __global__ __launch_bounds__(256) void k_hb_moe_down_rows(const bf16_t* act, const bf16_t* w_down, const float* h, long ldh, float* C, long ldc, int M, int N, int K,
                                                           hb_join join, hb_entries en) {
@@ -5290,21 +5292,26 @@ __global__ __launch_bounds__(256) void k_hb_moe_down_rows(const bf16_t* act, con
         const bf16_t *p0 = w_down + ((size_t)(e0 < en.experts ? e0 : 0) * N + c) * K, *p1 = w_down + ((size_t)(e1 < en.experts ? e1 : 0) * N + c) * K;
         const bf16_t *x0 = act + (size_t)i0 * K, *x1 = act + (size_t)i1 * K;
         float a0 = 0.f, a1 = 0.f;
-        for (int b = lane * 8; b < K; b += 512 * NC) {
+        for (int b = 0; b < K; b += 512 * NC) {      // (pieces and a second entry that are not there are not asked for)
             uint4 u0[NC], u1[NC], v0[NC], v1[NC];
 #pragma unroll
             for (int i = 0; i < NC; ++i) {
-                const int k = b + 512 * i < K ? b + 512 * i : b;
+                if (b + 512 * i >= K) break;
+                const int k = b + 512 * i + lane * 8 < K ? b + 512 * i + lane * 8 : 0;
                 u0[i] = *(const uint4*)(p0 + k);
                 v0[i] = *(const uint4*)(x0 + k);
-                u1[i] = *(const uint4*)(p1 + k);
-                v1[i] = *(const uint4*)(x1 + k);
+                if (k0 + 1 < en.top) {
+                    u1[i] = *(const uint4*)(p1 + k);
+                    v1[i] = *(const uint4*)(x1 + k);
+                }
             }
 #pragma unroll
             for (int i = 0; i < NC; ++i) {
                 if (b + 512 * i >= K) break;
-                a0 = hb_dot8(u0[i], v0[i], a0);
-                a1 = hb_dot8(u1[i], v1[i], a1);
+                if (b + 512 * i + lane * 8 < K) {
+                    a0 = hb_dot8(u0[i], v0[i], a0);
+                    if (k0 + 1 < en.top) a1 = hb_dot8(u1[i], v1[i], a1);
+                }
             }
         }
         float v = (b5 ? a1 : a0) + __shfl_xor(b5 ? a0 : a1, 32, 64);      // (hb_wave_sum's tree: its first step leaves an entry to each half of the wave)
@@ -5325,7 +5332,9 @@ static bool hb_glu_rows_ok(const float* A, long lda, const bf16_t* W, int M, int
 // Columns up to which a dense down product takes eight a block: a block to each CU (with the halves of K in the halves of a tile, k_hb_gemm_rows16 and
 // this, us: 2560 x 6912 18.9, 20.3; 3072 x 8192 19.4, 21.3; 4096 x 11008 34.1, 34.8).
 #define HB_DOWN8_COLS 2048
-// Dense unit of a few rows; false: its shape is the general launches'.  *done: the down product is in it too.
+// Dense unit of a few rows; false: its shape is the general launches'.  *done: the down product is in it too.  Whole steps of four such layers of 2, 8 and 16
+// rows, us, general launches and these (width, inner width): 512, 1408 184, 154; 203, 171; 230, 202; 2048, 5632 288, 256; 328, 294; 370, 359; 4096, 11008 577, 563;
+// 668, 664; 781, 770; 1024, 1000 187, 170; 223, 203; 256, 233.
 static bool hb_try_ff_rows(hipStream_t st, const float* A, long lda, const bf16_t* w_up, const float* b_up, const bf16_t* w_down, const float* b_down, float* act,
                            float* C, long ldc, int M, int W, int ff, hb_glu_args glu, const hb_join& join, bool* done) {
     if (!hb_glu_rows_ok(A, lda, w_up, M, W)) return false;
@@ -5337,13 +5346,20 @@ static bool hb_try_ff_rows(hipStream_t st, const float* A, long lda, const bf16_
 }
 static bool hb_try_ff_rows(hipStream_t, const float*, long, const float*, const float*, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args,
                            const hb_join&, bool*) { return false; }
-// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.  Both products, us,
-// entry by entry and this: 8 rows of 1024 18.6, 18.2; of 2048 60.7, 52.2; of 4096 231, 137; 4 rows of 2048 32.6, 29.1; 2 rows of 2048 24.2, 22.2, of 4096 67.4, 55.4.
+// Routed layer of 2 to 8 rows (no shared expert, no residual gate, gated experts); false: its shape is the entry-by-entry launches'.  What these save is
+// an expert's rows read once for all its entries; what they cost is a trip and a barrier for the entries' rows in LDS.  So: wide experts, two choices and more
+// (one: wider ones), or many weights in all.  Whole steps of three and four such layers, us, entry by entry and this (width, experts, choices, inner width): 8 rows:
+// 2048, 8, 2, 2048 288, 262; 3072, 8, 2, 4096 691, 473; 2048, 4, 1, 8192 472, 358; 2048, 64, 8, 1024 694, 576; 2048, 64, 8, 512 480, 476; 2 rows: 2048, 8, 2, 2048
+// 198, 196; 1024, 8, 4, 2048 193, 183; 2048, 8, 1, 4096 194, 193.  Left out: 8 rows of 512, 16, 2, 512 198, 212; 1024, 8, 2, 1024 234, 239; 2048, 4, 1, 2048 314,
+// 322; 2048, 64, 8, 256 410, 421; 4 rows of 2048, 64, 8, 512 389, 400; 2 rows of 2048, 8, 2, 1536 182, 190.
+static bool hb_moe_rows_pay(int M, int W, int ff, int top) {
+    return top >= 2 ? ff >= 2048 || (size_t)M * top * W * ff >= 40u << 20 : ff >= 4096;
+}
 static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16_t* w_gate_up, const bf16_t* w_down, float* act, float* C, long ldc, int M, int W,
                             int ff, hb_glu_args glu, const hb_join& join, hb_entries en) {
     const size_t lds = (size_t)HB_MOE_UP_ROWS * W * 2;
     if (M < 2 || M * en.top > 64 || en.experts < 1 || (W & 7) || (ldh & 3) || ((size_t)h & 15) || ((size_t)w_gate_up & 15) || (ff & 7) || ((size_t)w_down & 15) ||
-        lds > 64 * 1024) return false;
+        lds > 64 * 1024 || !hb_moe_rows_pay(M, W, ff, en.top)) return false;
     hipLaunchKernelGGL(k_hb_moe_up_rows, dim3((ff + 7) / 8, M * en.top), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
     hipLaunchKernelGGL(k_hb_moe_down_rows, dim3((W + 31) / 32 * 8 * M), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
     return true;
