@@ -1744,8 +1744,8 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
         // column tiles per block: one while the call is a handful of row tiles (latency: more blocks in flight), two from 256 tiles on
         // once there are >= 16 row tiles (every block re-loads and re-splits its A rows: at 448+ rows that traffic and VALU work
         // outweigh the extra blocks — CosyVoice2 chunk 49.7 -> 46.6 ms at B=8, 36.6 -> 35.2 at B=4, unchanged at B=1), four above 512
-        // (above 2048, and this: 8 requests of 28 tokens, 896 rows, 28.61 and 28.16 ms; 4 of 20 22.60, 22.54; 1 of 28 20.58 both), but above
-        // 2048 below those 16 row tiles and from 1025 rows on (GLM-4-Voice's flow with 512 there too, 1032 rows 53.7 and 54.2 ms, 1376 rows 57.3, 57.8)
+        // (above 2048, and this: 8 requests of 28 tokens, 896 rows, 28.61 and 28.16 ms; 4 of 20 22.60, 22.54; 1 of 28 20.58 both; nowhere
+        // slower at 40 shapes of CosyVoice2's flow and 24 of GLM-4-Voice's), but above 2048 below those 16 row tiles and from 1025 rows on (GLM-4-Voice's flow with 512 there too, 1032 rows 53.7 and 54.2 ms, 1376 rows 57.3, 57.8)
         const int four = rows_nt_tiles(1) ? rows_nt_tiles(1) : a.M >= 256 && a.M <= 1024 ? 512 : 2048;
         int nt = tiles > four ? 4 : tiles > (a.M >= 256 ? rows_nt_tiles(0) : 1024) ? 2 : 1;
         while (nt > 1 && nt * kb > 16) nt >>= 1;
