@@ -93,11 +93,11 @@ def test_routed_products(rows, width, ff, top, up, down):
     check(cfg, P.random_checkpoint(cfg, seed=ff), rows, [rows], tiles, page=64)
 
 
-# Sums that join two gated residual streams (closing products of the mixer and of the dense unit, K = 640), and routed ones
-@pytest.mark.parametrize("rows,width,tile", [(33, 512, (32, 32)), (520, 2432, (64, 32)), (193, 3520, (64, 64)), (520, 3648, (128, 128))])
-def test_products_that_join_streams(rows, width, tile):
-    cfg = GU.config([GU.attention(heads=10, kv_heads=5, dim=32, vdim=64, size=64, bias_max=40, rows=16, mlp=GU.dense(640))], width=width, vocab=50)
-    check(cfg, GU.random_checkpoint(cfg, seed=rows), rows, [rows], [(JOIN, rows, width, 640, 1, *tile)], page=64)
+# Sums that join two gated residual streams (closing products of the mixer and of the dense unit), and routed ones
+@pytest.mark.parametrize("rows,width,k,tile", [(33, 512, 640, (32, 32)), (520, 2432, 640, (64, 32)), (850, 1856, 640, (64, 64)), (850, 2368, 1280, (128, 128))])
+def test_products_that_join_streams(rows, width, k, tile):
+    cfg = GU.config([GU.attention(heads=k // 64, kv_heads=k // 128, dim=32, vdim=64, size=64, bias_max=40, rows=16, mlp=GU.dense(k))], width=width, vocab=50)
+    check(cfg, GU.random_checkpoint(cfg, seed=rows), rows, [rows], [(JOIN, rows, width, k, 1, *tile)], page=64)
 
 
 @pytest.mark.parametrize("streams,width", [(2, 512), (2, 70), (3, 96), (4, 128)])

@@ -1336,11 +1336,10 @@ static const hb_tile HB_TILES[3][9] = {
      {192, 128, 625.f, 5800.f, 1.f}, {256, 128, 710.f, 7500.f, 1.f}, {256, 192, 1120.f, 7000.f, 1.f}, {256, 160, 780.f, 9500.f, 1.f}},
     {{32, 64, 190.f, 2600.f, 0.7f}, {64, 32, 0.f, 0.f, 0.f}, {64, 64, 290.f, 2300.f, 0.72f}, {128, 64, 420.f, 2400.f, 0.84f}, {128, 128, 527.f, 5300.f, 1.f},
      {192, 128, 625.f, 5800.f, 1.f}, {256, 128, 710.f, 7500.f, 1.f}, {256, 192, 1120.f, 7000.f, 1.f}, {256, 160, 0.f, 0.f, 0.f}},
-    // HB_EPI_JOIN: its epilogue, which waits for what it reads, is most of a block's time (costs fitted to whole steps); over 128 x 128 it would keep 208 to
-    // 400 bytes of scratch a lane.  Prompt steps of four Gaparax layers, us, all sums that join in 32 x 32, 64 x 32, 64 x 64, 128 x 64, 128 x 128: width 1024,
-    // 200 rows 464, 493, 537, 635, 662; 1024 rows 1031, 995, 1016, 1136, 1156; 2048 rows 1788, 1721, 1672, 1764, 1773; width 2048, 700 rows 1536, 1506, 1472,
-    // 1543, 1575; 2048 rows 3604, 3361, 3204, 3131, 3110.
-    {{32, 32, 160.f, 6400.f, 0.52f}, {64, 32, 195.f, 11900.f, 0.46f}, {64, 64, 290.f, 17300.f, 0.36f}, {128, 64, 0.f, 0.f, 0.f}, {128, 128, 527.f, 28700.f, 0.7f},
+    // HB_EPI_JOIN: its epilogue, which waits for what it reads, is most of a block's time; over 128 x 128 it would keep 208 to 400 bytes of scratch a lane.
+    // Two gated streams, us, 32 x 32, 64 x 32, 64 x 64, 128 x 128 (M, N x K): 256, 1024 x 1024 8.8, 12.3, 20.6, 39.4; 700, 1024 x 1024 16.8, 14.6, 21.4, 38.7; 1300, 1024 x
+    // 4096 59.2, 46.8, 37.7, 57.3; 700, 2048 x 2048 37.9, 36.8, 31.2, 53.7; 1600, 2048 x 8192 239, 180, 134, 91.
+    {{32, 32, 152.f, 5300.f, 0.56f}, {64, 32, 184.f, 8900.f, 0.6f}, {64, 64, 230.f, 16500.f, 0.56f}, {128, 64, 0.f, 0.f, 0.f}, {128, 128, 404.f, 32700.f, 0.5f},
      {192, 128, 0.f, 0.f, 0.f}, {256, 128, 0.f, 0.f, 0.f}, {256, 192, 0.f, 0.f, 0.f}, {256, 160, 0.f, 0.f, 0.f}}};
 // The tile whose blocks are through first by that measure, `rows` being the rows of a product as far as the host knows (a gathered one has fewer
 // than M): a wide tile moves fewer bytes per product, but a last round that is nearly empty costs as much as a full one.  Rows, N x K: tile
