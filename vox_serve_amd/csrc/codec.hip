@@ -4039,6 +4039,20 @@ __device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
     for (int i = 1; i < TB_PARTS; ++i) v[0] = tb_add(v[0], v[i]);
     return tb_add(v[TB_PARTS], tb_add(v[0], b2));
 }
+// exp(d), d <= 0 (or NaN), to the last bit or two of fp32: 2^(d log2 e) with what the product's rounding drops; below the smallest denormal 0, also for -inf
+__device__ __forceinline__ float exp_below(float d) {
+    const float t = d * 1.44269504088896340736f;
+    const float e = __fmaf_rn(d, 1.925963033500e-8f, __fmaf_rn(d, 1.44269504088896340736f, -t));
+    const float x = __builtin_amdgcn_exp2f(t);
+    return d < -104.0f ? 0.0f : __fmaf_rn(x, e * 0.693147180559945f, x);
+}
+// The largest value of a lane's row of 16 lanes (a maximum does not see the order it is taken in)
+__device__ __forceinline__ float row16_max(float s) {
+    s = fmaxf(s, vox_dpp<0x128, 0xF>(s, s));      // row_ror:8, 4, 2, 1
+    s = fmaxf(s, vox_dpp<0x124, 0xF>(s, s));
+    s = fmaxf(s, vox_dpp<0x122, 0xF>(s, s));
+    return fmaxf(s, vox_dpp<0x121, 0xF>(s, s));
+}
 // The estimators' attention on the matrix cores (no relative-position term, dk = 64, at most 256 keys: every CosyVoice2 / GLM estimator
 // call).  A block owns 16 consecutive queries of one (request, head); its WV (8) waves take the 16-key tiles w, w + WV for
 // BOTH products, so nothing but the row maxima, the row sums and the 16 x 64 partial outputs crosses a wave:
@@ -4054,15 +4068,17 @@ __device__ __forceinline__ float4 tb_sum(const float* p, size_t ps, float4 b2) {
 // weights), one of that product's eight runs of K: the feed-forward launch adds the heads' planes in order and has the product's bits without
 // its 256 KB of weights a block.  896 rows: 11.4 -> 13.0 us here, 13.0 -> 10.8 there and 9.1 -> 8.3 in the next q | k | v.  (Two query
 // tiles a block, which read each key once for both: 15.2.)
+// Four waves share a SIMD, so what a wave issues counts: 184 keys, 13.6 us -> 11.8 with a tile's rows addressed together and clamped (each row had its own
+// branches, a division among them, and a wait between the tiles), DPP in the place of LDS permutes and exp_below in the place of expf (2.6 are its fp32 MFMA).
 template <int DK, int WV, bool OUT>
 __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
     static_assert(DK == 64, "operand layout below is written for 64-dim heads");
     constexpr int KT = 16 / WV, PS = KT * 16 + 4, OS = DK + 4;      // WV waves x KT key tiles of 16: at most 256 keys
-    __shared__ float red_mx[WV][16], red_sum[WV][16];
+    __shared__ __attribute__((aligned(16))) float red_mx[WV][16], red_sum[WV][16];
     __shared__ __attribute__((aligned(16))) float Ps[WV][16][PS];
     __shared__ __attribute__((aligned(16))) float Os[WV][16][OS];
     __shared__ uint4 pl[OUT ? 3 * 2 * 64 : 1];
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, fr = lane & 15, kq = lane >> 4;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, fr = lane & 15, kq = lane >> 4;
     int i0 = blockIdx.x * 16, h = blockIdx.y, n = blockIdx.z;
     if constexpr (OUT) {
         const int qt = (a.T + 15) >> 4, item = tb_item(tb_share{a.per, a.rest});
@@ -4072,43 +4088,48 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
         i0 = (nh - h * qt) * 16;
     }
     const int HD = a.H * DK, ld = 3 * HD, S = a.Tc + a.T, nt = (S + 15) >> 4;
-    const float* cache = a.cache ? a.cache + (a.cidx ? (size_t)a.cidx[n] * a.cache_half_stride : a.B > 0 ? (size_t)(n / a.B) * a.cache_half_stride : 0) +
+    const float* const cache = a.cache ? a.cache + (a.cidx ? (size_t)a.cidx[n] * a.cache_half_stride : a.B > 0 ? (size_t)(n / a.B) * a.cache_half_stride : 0) +
                                        (size_t)h * a.Tcap * 2 * DK : nullptr;
-    auto krow = [&](int j) -> const float* {      // K row of key j (its V row: + DK in the cache, + HD in qkv)
-        return j < a.Tc ? cache + (size_t)flow_cache_row(j, a.prefix, a.ring_head, a.Tcap) * 2 * DK
-                        : a.qkv + ((size_t)n * a.T + (j - a.Tc)) * ld + HD + h * DK;
-    };
+    // Keys at or beyond S read key S - 1, whose products are dropped: no load stands behind a branch of its own
+    const float* const fresh = a.qkv + ((ptrdiff_t)n * a.T - a.Tc) * ld + HD + h * DK;      // key j's K row: + j ld, its V row HD behind it
     const int iq = i0 + fr < a.T ? i0 + fr : a.T - 1;
-    const float* qrow = a.qkv + ((size_t)n * a.T + iq) * ld + h * DK + 4 * kq;
+    const float* qrow = a.qkv + (size_t)n * a.T * ld + h * DK;
     float4 q[4], k[KT][4], v[KT][4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) q[c] = *reinterpret_cast<const float4*>(qrow + 16 * c);
+    for (int c = 0; c < 4; ++c) q[c] = *reinterpret_cast<const float4*>(qrow + (unsigned)(iq * ld + 4 * kq + 16 * c));
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
-        const int kt = t * WV + wave;
+        const int j0 = (t * WV + wave) * 16, last = S - 1 - j0;
+        if (last < 0) continue;
+        const float *pk, *pv[4];      // B operand of P V: key j0 + 4 s4 + kq, dims 4 fr .. 4 fr + 3
+        if (j0 >= a.Tc || (j0 + 16 <= a.Tc && a.ring_head == 0)) {      // the tile's keys lie one behind the other
+            const bool old = j0 < a.Tc;
+            const float* const base = old ? cache + j0 * 2 * DK : fresh + (ptrdiff_t)j0 * ld;
+            const int step = old ? 2 * DK : ld, vo = old ? DK : HD;
+            pk = base + (unsigned)((fr < last ? fr : last) * step + 4 * kq);
 #pragma unroll
-        for (int c = 0; c < 4; ++c) { k[t][c] = make_float4(0.f, 0.f, 0.f, 0.f); v[t][c] = make_float4(0.f, 0.f, 0.f, 0.f); }
-        if (kt < nt) {
-            const int j = kt * 16 + fr;
-            if (j < S) {
-                const float* kr = krow(j) + 4 * kq;
+            for (int s4 = 0; s4 < 4; ++s4) pv[s4] = base + (unsigned)((4 * s4 + kq < last ? 4 * s4 + kq : last) * step + vo + 4 * fr);
+        } else {
+            auto row = [&](int j, int is_v) -> const float* {
+                j = j < S ? j : S - 1;
+                return j < a.Tc ? cache + (flow_cache_row(j, a.prefix, a.ring_head, a.Tcap) * 2 + is_v) * DK : fresh + (ptrdiff_t)j * ld + is_v * HD;
+            };
+            pk = row(j0 + fr, 0) + 4 * kq;
 #pragma unroll
-                for (int c = 0; c < 4; ++c) k[t][c] = *reinterpret_cast<const float4*>(kr + 16 * c);
-            }
-#pragma unroll
-            for (int s4 = 0; s4 < 4; ++s4) {      // B operand of P V: key 16 kt + 4 s4 + kq, dims 4 fr .. 4 fr + 3
-                const int jv = kt * 16 + 4 * s4 + kq;
-                if (jv < S) v[t][s4] = *reinterpret_cast<const float4*>(krow(jv) + (jv < a.Tc ? DK : HD) + 4 * fr);
-            }
+            for (int s4 = 0; s4 < 4; ++s4) pv[s4] = row(j0 + 4 * s4 + kq, 1) + 4 * fr;
         }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) k[t][c] = ldg_f4(pk + 16 * c);
+#pragma unroll
+        for (int s4 = 0; s4 < 4; ++s4) v[t][s4] = ldg_f4(pv[s4]);
     }
     f32x4 sc[KT];
     float mx[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
     for (int t = 0; t < KT; ++t) {
         const int kt = t * WV + wave;
-        sc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
         if (kt < nt) {
+            sc[t] = (f32x4){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int c = 0; c < 4; ++c) {
                 sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[c].x, k[t][c].x, sc[t], 0, 0, 0);
@@ -4116,45 +4137,48 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
                 sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[c].z, k[t][c].z, sc[t], 0, 0, 0);
                 sc[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[c].w, k[t][c].w, sc[t], 0, 0, 0);
             }
-        }
-        const int j = kt * 16 + fr;      // accumulator r: query i0 + 4 kq + r, key j
+            const int j = kt * 16 + fr;      // accumulator r: query i0 + 4 kq + r, key j
+            const bool in = j < S;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int i = i0 + 4 * kq + r;
-            float s = sc[t][r] * a.scale;
-            if (kt >= nt || j >= S || (a.mask_block > 0 && j > i && j / a.mask_block != i / a.mask_block)) s = -INFINITY;
-            sc[t][r] = s;
-            mx[r] = fmaxf(mx[r], s);
+            for (int r = 0; r < 4; ++r) sc[t][r] = in ? sc[t][r] * a.scale : -INFINITY;
+            if (a.mask_block > 0) {
+                const int jb = j / a.mask_block;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const int i = i0 + 4 * kq + r;
+                    if (j > i && jb != i / a.mask_block) sc[t][r] = -INFINITY;
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) mx[r] = fmaxf(mx[r], sc[t][r]);
         }
     }
     uint4 wf[OUT ? 2 : 1][2];      // (in flight while the outputs are formed)
     if constexpr (OUT) tb_weights<2, 2>(wf, a.wo, wave * 2, 16, h * 2, lane);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) mx[r] = fmaxf(mx[r], __shfl_xor(mx[r], off, 64));
-        if (fr == 0) red_mx[wave][4 * kq + r] = mx[r];
-    }
+    for (int r = 0; r < 4; ++r) mx[r] = row16_max(mx[r]);
+    if (fr == 0) *reinterpret_cast<float4*>(&red_mx[wave][4 * kq]) = make_float4(mx[0], mx[1], mx[2], mx[3]);
     __syncthreads();
-    float sum[4];
+    float4 gm = *reinterpret_cast<const float4*>(&red_mx[0][4 * kq]);
 #pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int qi = 4 * kq + r;
-        float gm = red_mx[0][qi];
-#pragma unroll
-        for (int w = 1; w < WV; ++w) gm = fmaxf(gm, red_mx[w][qi]);
-        float sm = 0.0f;
-#pragma unroll
-        for (int t = 0; t < KT; ++t) {
-            const float p = sc[t][r] == -INFINITY ? 0.0f : expf(sc[t][r] - gm);
-            Ps[wave][qi][16 * t + fr] = p;
-            sm += p;
-        }
-#pragma unroll
-        for (int off = 8; off >= 1; off >>= 1) sm += __shfl_xor(sm, off, 64);
-        sum[r] = sm;
-        if (fr == 0) red_sum[wave][qi] = sm;
+    for (int w = 1; w < WV; ++w) {
+        const float4 m = *reinterpret_cast<const float4*>(&red_mx[w][4 * kq]);
+        gm = make_float4(fmaxf(gm.x, m.x), fmaxf(gm.y, m.y), fmaxf(gm.z, m.z), fmaxf(gm.w, m.w));
     }
+    const float top[4] = {gm.x, gm.y, gm.z, gm.w};
+    float sum[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int t = 0; t < KT; ++t)
+        if (t * WV + wave < nt)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                const float p = exp_below(sc[t][r] - top[r]);
+                Ps[wave][4 * kq + r][16 * t + fr] = p;
+                sum[r] += p;
+            }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) sum[r] = butterfly<16>(sum[r]);
+    if (fr == 0) *reinterpret_cast<float4*>(&red_sum[wave][4 * kq]) = make_float4(sum[0], sum[1], sum[2], sum[3]);
     __builtin_amdgcn_wave_barrier();      // the wave's own p tile: written in accumulator layout, read back as A operands
     f32x4 o[4];
 #pragma unroll
@@ -4176,25 +4200,39 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
     for (int r = 0; r < 4; ++r)      // o[d][r] = out[query 4 kq + r][dim 4 fr + d]
         *reinterpret_cast<float4*>(&Os[wave][4 * kq + r][4 * fr]) = make_float4(o[0][r], o[1][r], o[2][r], o[3][r]);
     __syncthreads();
-    const int qi = tid >> 4, c4 = (tid & 15) * 4;
-    if (tid < 256 && (OUT || i0 + qi < a.T)) {
+    if constexpr (OUT) {      // two columns to a thread of the eight waves
+        const int qi = tid >> 5, c2 = (tid & 31) * 2, g = c2 >> 3;
         float l = red_sum[0][qi];
-        float4 o4 = *reinterpret_cast<const float4*>(&Os[0][qi][c4]);
+        float2 o2 = *reinterpret_cast<const float2*>(&Os[0][qi][c2]);
 #pragma unroll
         for (int w = 1; w < WV; ++w) {
             l += red_sum[w][qi];
-            const float4 pw = *reinterpret_cast<const float4*>(&Os[w][qi][c4]);
-            o4.x += pw.x; o4.y += pw.y; o4.z += pw.z; o4.w += pw.w;
+            const float2 pw = *reinterpret_cast<const float2*>(&Os[w][qi][c2]);
+            o2.x += pw.x; o2.y += pw.y;
         }
         const float inv = 1.0f / l;
-        o4 = make_float4(o4.x * inv, o4.y * inv, o4.z * inv, o4.w * inv);
-        if constexpr (OUT) {      // (wave = rows 4 wave .. + 3, columns 4 (lane % 16) ..)
-            const tb_split s = tb_split3(o4);
-            const int g = (tid & 15) >> 1;
-            uint2* d = reinterpret_cast<uint2*>(pl + (g >> 2) * 64 + (g & 3) * 16 + tb_turn(g >> 2, g & 3, qi)) + (tid & 1);
+        o2 = make_float2(o2.x * inv, o2.y * inv);
+        u32* d = reinterpret_cast<u32*>(pl + (g >> 2) * 64 + (g & 3) * 16 + tb_turn(g >> 2, g & 3, qi)) + (tid & 3);
 #pragma unroll
-            for (int p = 0; p < 3; ++p) d[p * 2 * 128] = s.t[p];
-        } else *reinterpret_cast<float4*>(a.out + ((size_t)n * a.T + i0 + qi) * HD + h * DK + c4) = o4;
+        for (int p = 0; p < 3; ++p) {
+            const u32 term = pack_bf2(o2.x, o2.y);
+            d[p * 2 * 256] = term;
+            o2 = make_float2(o2.x - bflo(term), o2.y - bfhi(term));
+        }
+    } else {
+        const int qi = tid >> 4, c4 = (tid & 15) * 4;
+        if (tid < 256 && i0 + qi < a.T) {
+            float l = red_sum[0][qi];
+            float4 o4 = *reinterpret_cast<const float4*>(&Os[0][qi][c4]);
+#pragma unroll
+            for (int w = 1; w < WV; ++w) {
+                l += red_sum[w][qi];
+                const float4 pw = *reinterpret_cast<const float4*>(&Os[w][qi][c4]);
+                o4.x += pw.x; o4.y += pw.y; o4.z += pw.z; o4.w += pw.w;
+            }
+            const float inv = 1.0f / l;
+            *reinterpret_cast<float4*>(a.out + ((size_t)n * a.T + i0 + qi) * HD + h * DK + c4) = make_float4(o4.x * inv, o4.y * inv, o4.z * inv, o4.w * inv);
+        }
     }
     if constexpr (OUT) {
         __syncthreads();

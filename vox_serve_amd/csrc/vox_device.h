@@ -154,6 +154,10 @@ __device__ __forceinline__ uint4 ldg(const uint4* p) {
     const u32x4_t v = *(const VOX_GLOBAL_AS u32x4_t*)p;
     return make_uint4(v.x, v.y, v.z, v.w);
 }
+__device__ __forceinline__ float4 ldg_f4(const float* p) {
+    const u32x4_t v = *(const VOX_GLOBAL_AS u32x4_t*)p;
+    return make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
+}
 
 // ---- sampler pieces shared by sampler.hip and the persistent depth step's fused pick (kernels_lm.hip) ----
 // sortable key of a bf16 value (value order == unsigned key order; -0 == +0) and its inverse; Philox4x32-10 word 0 of (seed, offset, row)
