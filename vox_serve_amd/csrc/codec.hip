@@ -77,6 +77,8 @@ struct ConvGemmArgs {
     // split of fp32 rows made the many-row decoder convs VALU-bound (MFMA 16 % busy).
     // NP = 3: "S3" rows, [h][m][l], 6 * Cin bytes, the value itself.
     int out2_s2;
+    // k_rows_gemm: x / (Cin / 32) and x / L as the high word of a product (div_inverse); 0: by division
+    unsigned kpt_inv, len_inv;
     int dev;               // development builds (-DVOX_DEV_KNOBS, VOX_CODEC_DEV): 1 skip the K loop, 2 no out2 stores, 4 no out stores, 8 no residual loads
 };
 #ifdef VOX_DEV_KNOBS
@@ -1097,36 +1099,62 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
     float4 av[MT][KB][2];
     uint4 bv[NT][KB];
     float4 lw[LN ? KB : 1][2], lb[LN ? KB : 1][2];
+    // No load stands behind a branch of its own: rows and columns beyond the last read that one (nothing stores them), rows outside a request read the
+    // lane's own row and are zeroed in the registers (`out_of`).  The history's slot is asked for by the waves that have such a row, ahead of everything.
+    int col[KB], off[KB], tap_of[KB];
+    {
+        int tap = a.kpt_inv ? (int)__umulhi((unsigned)(wave * KB), a.kpt_inv) : wave * KB / kpt, kc = wave * KB - tap * kpt;
 #pragma unroll
-    for (int j = 0; j < KB; ++j) {
-        const int kbi = wave * KB + j, tap = kbi / kpt, c0 = (kbi - tap * kpt) * 32 + kq * 8;
-#pragma unroll
-        for (int mt = 0; mt < MT; ++mt) {
-            const int am = m0 + mt * 16 + fr;
-            const float* arow = nullptr;
-            if (am < a.M) {
-                const int ab = am / a.L, st = am % a.L - a.off[tap];
-                if (st >= a.L) arow = nullptr;
-                else if (st >= 0) arow = a.x + ((size_t)ab * a.L + st) * a.Cin;
-                else if (a.state && a.P + st >= 0) arow = a.state + ((size_t)a.slots[ab] * a.P + (a.P + st)) * a.Cin;
-            }
-            av[mt][j][0] = av[mt][j][1] = make_float4(0.f, 0.f, 0.f, 0.f);
-            if (arow) {
-                av[mt][j][0] = *reinterpret_cast<const float4*>(arow + c0);
-                av[mt][j][1] = *reinterpret_cast<const float4*>(arow + c0 + 4);
-            }
+        for (int j = 0; j < KB; ++j) {
+            tap_of[j] = tap; col[j] = kc * 32; off[j] = a.off[tap];
+            if (++kc == kpt) { kc = 0; ++tap; }
         }
+    }
+    int back = off[0];
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int bn = n0 + t * 16 + fr;
-            bv[t][j] = make_uint4(0, 0, 0, 0);
-            if (bn < a.N) bv[t][j] = *reinterpret_cast<const uint4*>(a.w + ((size_t)tap * a.N + bn) * a.Cin + c0);
-        }
-        if (LN) {
+    for (int j = 1; j < KB; ++j) back = back > off[j] ? back : off[j];
+    const int first = a.state ? -a.P : 0;      // rows of a request and its history: first .. L - 1
+    const unsigned span = (unsigned)(a.L - first);
+    const float *row[MT], *hist[MT];
+    int al[MT];
+    unsigned out_of = 0;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        const int m = m0 + mt * 16 + fr, am = m < a.M ? m : a.M - 1, ab = a.len_inv ? (int)__umulhi((unsigned)am, a.len_inv) : am / a.L;
+        al[mt] = am - ab * a.L;
+        row[mt] = hist[mt] = a.x + (size_t)am * a.Cin + kq * 8;
+        if (a.state && __ballot(al[mt] < back)) hist[mt] = a.state + ((size_t)a.slots[ab] * a.P + (a.P + al[mt])) * a.Cin + kq * 8;
+    }
+    auto load_rows = [&] {
+#pragma unroll
+        for (int j = 0; j < KB; ++j)
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt) {
+                const int st = al[mt] - off[j];
+                const bool none = (unsigned)(st - first) >= span;
+                out_of |= none ? 1u << (mt * KB + j) : 0u;
+                const float* p = (st < 0 ? hist[mt] : row[mt]) + (none ? (ptrdiff_t)col[j] : (ptrdiff_t)col[j] - (ptrdiff_t)off[j] * a.Cin);
+                av[mt][j][0] = ldg_f4(p);
+                av[mt][j][1] = ldg_f4(p + 4);
+            }
+    };
+    if (LN) load_rows();      // (their statistics come first)
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        const int n = n0 + t * 16 + fr;
+        const unsigned wo = (unsigned)(n < a.N ? n : a.N - 1) * (unsigned)a.Cin + kq * 8;
+#pragma unroll
+        for (int j = 0; j < KB; ++j) bv[t][j] = *reinterpret_cast<const uint4*>(a.w + ((size_t)tap_of[j] * a.N * a.Cin + col[j]) + wo);
+    }
+    if (LN)
+#pragma unroll
+        for (int j = 0; j < KB; ++j) {
+            const int c0 = col[j] + kq * 8;
             lw[j][0] = *reinterpret_cast<const float4*>(a.ln_w + c0); lw[j][1] = *reinterpret_cast<const float4*>(a.ln_w + c0 + 4);
             lb[j][0] = *reinterpret_cast<const float4*>(a.ln_b + c0); lb[j][1] = *reinterpret_cast<const float4*>(a.ln_b + c0 + 4);
         }
-    }
+    else load_rows();
+    const bool zeroes = __ballot(out_of != 0);
     float mean[MT], rstd[MT];
 #pragma unroll
     for (int mt = 0; mt < MT; ++mt) mean[mt] = rstd[mt] = 0.0f;
@@ -1185,23 +1213,24 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) x8[e] = (x8[e] - mean[mt]) * rstd[mt] * w8[e] + b8[e];
             }
-            unsigned short hb[8], mb[8], lbb[8];
+            if (zeroes) {
+                const bool z = out_of >> (mt * KB + j) & 1;
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                hb[e] = f2bf(x8[e]);
-                const float r1 = x8[e] - bf2f(hb[e]);
-                mb[e] = f2bf(r1);
-                lbb[e] = f2bf(r1 - bf2f(mb[e]));
+                for (int e = 0; e < 8; ++e) x8[e] = z ? 0.0f : x8[e];
             }
-            const uint4 ah = make_uint4(hb[0] | (unsigned)hb[1] << 16, hb[2] | (unsigned)hb[3] << 16, hb[4] | (unsigned)hb[5] << 16, hb[6] | (unsigned)hb[7] << 16);
-            const uint4 amid = make_uint4(mb[0] | (unsigned)mb[1] << 16, mb[2] | (unsigned)mb[3] << 16, mb[4] | (unsigned)mb[5] << 16, mb[6] | (unsigned)mb[7] << 16);
-            const uint4 al = make_uint4(lbb[0] | (unsigned)lbb[1] << 16, lbb[2] | (unsigned)lbb[3] << 16, lbb[4] | (unsigned)lbb[5] << 16, lbb[6] | (unsigned)lbb[7] << 16);
+            u32 h[3][4];
 #pragma unroll
-            for (int t = 0; t < NT; ++t) {      // plane order of the staged kernels: low terms first
-                if (a.planes >= 3) acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(al), as_cbf8(bv[t][j]), acc[mt][t], 0, 0, 0);
-                if (a.planes >= 2) acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(amid), as_cbf8(bv[t][j]), acc[mt][t], 0, 0, 0);
-                acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(ah), as_cbf8(bv[t][j]), acc[mt][t], 0, 0, 0);
-            }
+            for (int p = 0; p < 3; ++p)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    h[p][e] = pack_bf2(x8[2 * e], x8[2 * e + 1]);
+                    if (p < 2) { x8[2 * e] -= bflo(h[p][e]); x8[2 * e + 1] -= bfhi(h[p][e]); }
+                }
+#pragma unroll
+            for (int t = 0; t < NT; ++t)      // plane order of the staged kernels: low terms first
+#pragma unroll
+                for (int p = 2; p >= 0; --p)
+                    acc[mt][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_cbf8(make_uint4(h[p][0], h[p][1], h[p][2], h[p][3])), as_cbf8(bv[t][j]), acc[mt][t], 0, 0, 0);
         }
     }
 #pragma unroll
@@ -1224,7 +1253,7 @@ __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
         const int e = wave + i * WV, tile = (e >> 2) < MT * NT ? (e >> 2) : 0, r = e & 3, mt = tile / NT, t = tile - mt * NT;
         int m = m0 + mt * 16 + kq * 4 + r, n = n0 + t * 16 + fr;
         m = m < Mc ? m : Mc; n = n < Nc ? n : Nc;
-        e_b[i] = a.bias ? a.bias[n % a.bias_mod] : 0.0f;
+        e_b[i] = a.bias ? a.bias[a.bias_mod >= a.N ? n : n % a.bias_mod] : 0.0f;
         e_s[i] = a.scale ? a.scale[n] : 1.0f;
         e_rs[i] = a.rscale ? a.rscale[m] : 1.0f;
         e_res[i] = a.res ? a.res[(size_t)m * a.N + n] : 0.0f;
@@ -1741,6 +1770,10 @@ static int rows_nt_tiles(int which) {
     static const int v4 = [] { const char* e = getenv("VOX_ROWS_NT4"); return e ? atoi(e) : 0; }();
     return which ? v4 : v2;
 }
+// x / d = umulhi(x, inverse) for 0 <= x < n: with inverse = (2^32 + r) / d, 0 <= r < d, exact while x r < 2^32.  0 where that does not hold (and for d = 1)
+static unsigned div_inverse(int d, int n) {
+    return d > 1 && (uint64_t)d * (uint64_t)n < 1ull << 32 ? (unsigned)(((1ull << 32) + (unsigned)d - 1) / (unsigned)d) : 0u;
+}
 static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const float* state, const int* slots, int n,
                      int L, int P, const int* offs, float* out, const float* res, const float* scale, int gelu,
                      float* out2 = nullptr, const vox_snake_w* sn = nullptr, int sn_mod = 0, const float* rscale = nullptr,
@@ -1757,7 +1790,7 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
     a.bias_mod = w.bias_mod > 0 ? w.bias_mod : w.n; a.gelu = gelu;
     if (out2 && sn) { a.out2 = out2; a.sn_alpha = sn->alpha; a.sn_invb = sn->inv_beta; a.sn_mod = sn_mod > 0 ? sn_mod : w.n; }
     for (int k = 0; k < w.n_taps; ++k) a.off[k] = offs ? offs[k] : 0;
-    if (g_conv_rows_gemm && rows_gemm_on() && out && !out2 && a.M <= g_conv_skinny_rows && w.cin % 32 == 0 && (w.n_taps * w.cin) % 128 == 0 && (!ln_w || (w.n_taps == 1 && a.off[0] == 0))) {
+    if (g_conv_rows_gemm && a.planes == 3 && rows_gemm_on() && out && !out2 && a.M <= g_conv_skinny_rows && w.cin % 32 == 0 && (long)w.n * w.cin < 1l << 31 && (w.n_taps * w.cin) % 128 == 0 && (!ln_w || (w.n_taps == 1 && a.off[0] == 0))) {
         // every operand requested up front, K split over the block's waves (k_rows_gemm): 8 waves from K = 512 on
         const int K = w.n_taps * w.cin, wv = (K >= 512 && K % 256 == 0 && rows_wv8_on()) ? 8 : 4, kb = K / (32 * wv);
         const int tiles = ((w.n + 15) / 16) * ((a.M + 15) / 16);
@@ -1771,6 +1804,8 @@ static int conv_gemm(hipStream_t st, const vox_conv_w& w, const float* x, const 
         while (nt > 1 && nt * kb > 16) nt >>= 1;
         const int mt = (tiles / nt >= rows_mt2_blocks() && kb <= 4 && (wv == 4 || nt <= 2)) ? 2 : 1;      // (the 8-wave sum buffer: MT NT <= 4)
         if (ln_w) { a.ln_w = ln_w; a.ln_b = ln_b; a.ln_eps = ln_eps; }
+        a.kpt_inv = div_inverse(w.cin / 32, K / 32);
+        a.len_inv = div_inverse(L, a.M);
         const dim3 g((w.n + 16 * nt - 1) / (16 * nt), (a.M + 16 * mt - 1) / (16 * mt));
 #define VOX_ROWS1(KB_, NT_, MT_, WV_)                                                                              \
         if (kb == KB_ && nt == NT_ && mt == MT_ && wv == WV_) {                                                        \
