@@ -34,3 +34,10 @@ def test_linear_rows_bit_exact(dev, B, N_, K):  # noqa: F811
                                          (75, (4096, 2, 1, 384))])
 def test_stack_rows_with_norms(dev, n_rows, dims):  # noqa: F811
     stack_rows_case(Tape(), dev, n_rows, dims=dims)
+
+
+@pytest.mark.parametrize("n_rows,dims", [(3, (4096, 2, 1, 8224)), (8, (4096, 32, 2, 4128)), (9, (4096, 32, 2, 4128)), (16, (4096, 2, 1, 4160))])
+def test_stack_few_rows_more_column_tiles_than_cus(dev, n_rows, dims):  # noqa: F811
+    """Up to 16 rows of 4096 values whose norm runs inside k_gemm_tiles: one and two rows a wave, 257 .. 514 column tiles (the last round of blocks nearly
+    empty), and the down projection behind them on k_linear_mfma_stream with its input fragment-major, waves with a k-step more than others among them."""
+    stack_rows_case(Tape(), dev, n_rows, dims=dims)

@@ -252,7 +252,7 @@ static int stack_layers(vox_stack* s, hipStream_t st, void* x, void* kv, int64_t
         if (o_fk && !(decode_rows && c.max_kvlen <= 16 && vox_attn1_linear_supported(ac, o))) { ac.out_frag = s->afrag; o.x_frag = s->afrag; }
         xf_ready = o_fk && g_fk;
         if (xf_ready) { o.y_frag = s->xfrag; g.x_frag = s->xfrag; }
-        if (g_fk && d_fk) { g.y_frag = s->hfrag; g.y_rowmajor = 0; d.x_frag = s->hfrag; }
+        if (g_fk && (d_fk || vox_linear_is_stream(d))) { g.y_frag = s->hfrag; g.y_rowmajor = 0; d.x_frag = s->hfrag; }
         if (decode_rows && c.max_kvlen <= 16 && !(ablate() & 256) && vox_attn1_linear_supported(ac, o)) {
             VOX_TRY(vox_launch_attn1_linear(st, ac, o));     // short context: attention recomputed inside o_proj
         } else {

@@ -30,6 +30,7 @@ struct LinArgs {
     int y_rowmajor;
     int row_tiles;       // k_gemv only: > 1 = that many row tiles of BT rows, one block per (column group, row tile)
     int rt_rows;         // k_gemm_fullk<.., ROWSPLIT>: rows per row tile (0 = 16 * MT); 8 or 4: SUB-TILE row split for <= 16 rows (below)
+    int cus;             // compute units of the device
     int no_one_seg;      // k_linear_mfma A/B knob (VOX_MFMA_ONESEG=0): row statistics by the separate pass even when K fits one segment
 };
 
@@ -884,11 +885,12 @@ static int launch_linear_mfma_t(hipStream_t st, const LinArgs& a) {
 // added in wave order: bit-identical to k_linear_mfma (oracle: VR_ORD_MFMA4), which keeps the calls this form does not cover
 // (17+ rows, x_out, a norm prologue with K > 1024).
 //   k_linear_mfma_small   K <= 1024: every operand of the call is requested before anything waits (CosyVoice2's 896-wide linears)
-//   k_linear_mfma_stream  K  > 1024, copy prologue: two register buffers of H k-steps per wave; a buffer is refilled as soon as it has
+//   k_linear_mfma_stream  K  > 1024, copy prologue: four register buffers of four k-steps per wave; a buffer is refilled as soon as it has
 //                         been multiplied, the loop body has no conditional load (the in-order vmcnt accounting stays exact), steps
-//                         past the end re-request the last real step (cache hits) and are not multiplied.  CosyVoice2's 4864-wide down
-//                         projection has 56 column tiles: all of a block's 155 KB are in flight after two groups; GLM-4-Voice's
-//                         13 696-wide one keeps 128 KB per CU in flight with no barrier in the walk.
+//                         past the end re-request the last real step (cache hits) and are not multiplied.  The rows come fragment-major where
+//                         the gate / up launch in front writes them so: row-major, a request touches 16 lines and they cost what the weights do.
+//                         Alone, us, two buffers of 16 / four of four / those with fragment-major rows: GLM-4-Voice's 13 696 x 4096
+//                         26.7 / 22.1 / 19.4 (no rows at all 19.9), CosyVoice2's 4864 x 896 11.1 / 8.7 / 6.9; four of eight 11.4.
 // ================================================================================================
 template <int PRO, int EPI>
 __global__ __launch_bounds__(256) void k_linear_mfma_small(LinArgs a) {
@@ -1001,8 +1003,9 @@ __global__ __launch_bounds__(256) void k_linear_mfma_small(LinArgs a) {
     }
 }
 
-template <int EPI, int H>
+template <int EPI>
 __global__ __launch_bounds__(256) void k_linear_mfma_stream(LinArgs a) {
+    constexpr int H = 4, NBUF = 4;
     static_assert(EPI == EPI_STORE || EPI == EPI_SILU, "copy prologue, plain epilogues");
     __shared__ f32x4_t red[3][64];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1012,7 +1015,10 @@ __global__ __launch_bounds__(256) void k_linear_mfma_stream(LinArgs a) {
     const int bt = a.B;                                     // <= 16
     const int T = (a.K - 32 * wave + 127) >> 7;             // this wave's k-steps (K > 1024: at least 8)
     const int G = (T + H - 1) / H;
-    const uint4* xrow = x_row_ptr(a, fr < bt ? fr : bt - 1) + ((32 * wave + fk) >> 3);     // step t: 16 chunks further
+    const int arow = fr < bt ? fr : bt - 1;
+    const uint4* xrow = a.x_frag ? reinterpret_cast<const uint4*>(a.x_frag) + (size_t)wave * 64 + arow + (lane & 48)     // step t: four fragments further
+                                 : x_row_ptr(a, arow) + ((32 * wave + fk) >> 3);                                         // ... or 16 chunks
+    const int xstep = a.x_frag ? 256 : 16;
     // row-major: lane (fr, g) reads 16 B of weight row n0 + fr per step (16 rows x 64 B per wave request), step t 16 chunks further;
     // fragment-major (the decoder stack's copy, N % 16 == 0): the same register contents from ONE contiguous 1 KiB request — k-step
     // wave + 4 t of column tile blockIdx.x, four fragments further per step
@@ -1020,7 +1026,7 @@ __global__ __launch_bounds__(256) void k_linear_mfma_stream(LinArgs a) {
     const int wstep = wf ? 256 : 16;
     const uint4* wrow = wf ? reinterpret_cast<const uint4*>(a.W_frag) + ((size_t)blockIdx.x * (a.K >> 5) + wave) * 64 + lane
                            : reinterpret_cast<const uint4*>(a.W + (size_t)nrow * a.K + 32 * wave + fk);
-    uint4 xb[2][H], wb[2][H];
+    uint4 xb[NBUF][H], wb[NBUF][H];
     f32x4_t acc = (f32x4_t){0.f, 0.f, 0.f, 0.f};
     auto issue = [&](auto BUF, int g) {
         constexpr int b = decltype(BUF)::value;
@@ -1028,30 +1034,30 @@ __global__ __launch_bounds__(256) void k_linear_mfma_stream(LinArgs a) {
         for (int i = 0; i < H; ++i) {
             int t = g * H + i;
             t = t < T ? t : T - 1;                  // past the end: the last real step again (a cache hit; never multiplied)
-            xb[b][i] = xrow[16 * t];
+            xb[b][i] = xrow[xstep * t];
             wb[b][i] = ldg_nt(wrow + (size_t)wstep * t);
         }
     };
-    auto consume = [&](auto BUF, auto GUARD, int g) {      // GUARD: the group may reach past the wave's last step
+    auto consume = [&](auto BUF, int g) {
         constexpr int b = decltype(BUF)::value;
 #pragma unroll
         for (int i = 0; i < H; ++i)
-            if (!decltype(GUARD)::value || g * H + i < T)
-                acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(xb[b][i]), as_bf8(wb[b][i]), acc, 0, 0, 0);
+            if (g * H + i < T) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(xb[b][i]), as_bf8(wb[b][i]), acc, 0, 0, 0);
     };
     issue(vox_ic<0>{}, 0);
-    issue(vox_ic<1>{}, G > 1 ? 1 : 0);
-    int g = 0;
-    for (; g + 4 <= G; g += 2) {                    // steady state: every group multiplied here is complete, every one requested exists
-        consume(vox_ic<0>{}, vox_ic<0>{}, g);
-        issue(vox_ic<0>{}, g + 2);
-        consume(vox_ic<1>{}, vox_ic<0>{}, g + 1);
-        issue(vox_ic<1>{}, g + 3);
+    issue(vox_ic<1>{}, 1);
+    issue(vox_ic<2>{}, 2);
+    issue(vox_ic<3>{}, 3);
+    for (int g = 0; g < G; g += NBUF) {      // (requests without a condition: behind one, the compiler waits for everything)
+        consume(vox_ic<0>{}, g);
+        issue(vox_ic<0>{}, g + NBUF);
+        consume(vox_ic<1>{}, g + 1);
+        issue(vox_ic<1>{}, g + NBUF + 1);
+        consume(vox_ic<2>{}, g + 2);
+        issue(vox_ic<2>{}, g + NBUF + 2);
+        consume(vox_ic<3>{}, g + 3);
+        issue(vox_ic<3>{}, g + NBUF + 3);
     }
-    consume(vox_ic<0>{}, vox_ic<1>{}, g);           // one to three groups left; buffer 1 holds g + 1 (if it exists)
-    issue(vox_ic<0>{}, g + 2 < G ? g + 2 : G - 1);
-    consume(vox_ic<1>{}, vox_ic<1>{}, g + 1);
-    consume(vox_ic<0>{}, vox_ic<1>{}, g + 2);
     float res_pre[4] = {0.f, 0.f, 0.f, 0.f};
     const int n = n0 + fr;
     if (a.residual && wave == 0 && n < a.N) {
@@ -1105,7 +1111,7 @@ static int launch_linear_mfma_pe(hipStream_t st, const LinArgs& a_in) {
             return VOX_OK;
         }
         if constexpr (PRO == PRO_COPY && (EPI == EPI_STORE || EPI == EPI_SILU)) {
-            hipLaunchKernelGGL((k_linear_mfma_stream<EPI, 16>), grid, dim3(256), 0, st, a);
+            hipLaunchKernelGGL(k_linear_mfma_stream<EPI>, grid, dim3(256), 0, st, a);
             return VOX_OK;
         }
     }
@@ -1514,6 +1520,164 @@ __global__ __launch_bounds__(512) void k_gemm_fullk(LinArgs a) {
 }
 
 // ================================================================================================
+// The same linear for up to 16 rows of 4096 values behind a norm and more column tiles than CUs (GLM-4-Voice's q | k | v, gate / up and head): a
+// block per CU walks the tiles blockIdx.x, + gridDim.x, ...  The first weights are requested before anything waits; under them the block normalises
+// the rows (a wave a row, k_rmsnorm's sums, through LDS) and its waves take their K ranges of them into registers for all tiles, where a block per tile asked
+// for them again each time (half as many bytes as its weights) and a launch in front had normalised them.  Then a wave has one tile's fragments in flight
+// while it multiplies the other's; a tile's sums cross the waves through one of two LDS buffers, and four waves finish one output a thread.
+// Same k-steps, same sums: the same bits as k_rmsnorm and k_gemm_fullk.
+// Bound by the weight stream (6.6 TB/s is what loads alone reach).  8 rows, us, with the norm's launch before -> here: 13 696 gate / up (224 MB)
+// 44.3 + 4.7 -> 37.6, 4608 q | k | v (38 MB; 288 blocks on 256 CUs) 12.3 + 4.7 -> 10.8, head of 168 960 (1.38 GB, row-major) 293 + 4.7 -> 263.
+// ================================================================================================
+template <int KSTEPS, int EPI, int ROWS>
+__global__ __launch_bounds__(512) void k_gemm_tiles(LinArgs a) {
+    constexpr bool SM = EPI == EPI_SILU_MUL;
+    constexpr int NB = SM ? 2 : 1, NCH = KSTEPS * 32;      // 16-byte pieces of a row
+    extern __shared__ __attribute__((aligned(16))) char tiles_smem[];
+    float (*const red)[NB][8][256] = reinterpret_cast<float (*)[NB][8][256]>(tiles_smem);      // two buffers, where the rows have been
+    uint4* const xs = reinterpret_cast<uint4*>(tiles_smem);                                    // piece c of row r at c * 16 + (r ^ (c & 15))
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15;
+    const int tiles = (a.N + 15) >> 4, step = gridDim.x, kbase = wave * (KSTEPS * 32) + (lane >> 4) * 8, row = fr < a.B ? fr : a.B - 1;
+    uint4 xa[KSTEPS], w0[KSTEPS], w1[KSTEPS];
+    uint4 nx[ROWS][NCH / 64], ng[NCH / 64];      // wave w: rows w and (ROWS = 2) w + 8; a row less: the last one again
+#pragma unroll
+    for (int i = 0; i < ROWS; ++i) {
+        const int r = wave + 8 * i;
+        const uint4* xr = x_row_ptr(a, r < a.B ? r : a.B - 1) + lane;
+#pragma unroll
+        for (int u = 0; u < NCH / 64; ++u) nx[i][u] = ldg(xr + 64 * u);
+    }
+#pragma unroll
+    for (int u = 0; u < NCH / 64; ++u) ng[u] = reinterpret_cast<const uint4*>(a.nw)[lane + 64 * u];
+    __builtin_amdgcn_sched_barrier(0);
+    // the rows normalised as k_rmsnorm does it, a wave a row, while the first weights travel
+    auto rows_ready = [&] {
+#pragma unroll
+        for (int i = 0; i < ROWS; ++i) {
+            const int r = wave + 8 * i;
+            float ss = 0.0f;
+#pragma unroll
+            for (int u = 0; u < NCH / 64; ++u) ss = sq8(nx[i][u], ss);
+            ss = butterfly<64>(ss);
+            const float rinv = 1.0f / sqrtf(ss / (float)a.K + a.eps);
+#pragma unroll
+            for (int u = 0; u < NCH / 64; ++u) nx[i][u] = norm_chunk(nx[i][u], ng[u], rinv);
+            if (r < a.B)
+#pragma unroll
+                for (int u = 0; u < NCH / 64; ++u) {
+                    const int c = lane + 64 * u;
+                    xs[c * 16 + (r ^ (c & 15))] = nx[i][u];
+                }
+        }
+        __syncthreads();
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) {
+            const int c = wave * (KSTEPS * 4) + s * 4 + (lane >> 4);
+            xa[s] = xs[c * 16 + (row ^ (c & 15))];
+        }
+        __syncthreads();
+    };
+    auto load = [&](uint4 (&v)[KSTEPS], const bf16_t* frag, const bf16_t* w, int t) {
+        if (frag) {
+            const uint4* p = reinterpret_cast<const uint4*>(frag) + ((size_t)t * (a.K >> 5) + wave * KSTEPS) * 64 + lane;
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) v[s] = ldg_nt(p + s * 64);
+        } else {
+            const int n = t * 16 + fr;
+            const uint4* p = reinterpret_cast<const uint4*>(w + (size_t)(n < a.N ? n : a.N - 1) * a.K + kbase);
+#pragma unroll
+            for (int s = 0; s < KSTEPS; ++s) v[s] = ldg_nt(p + s * 4);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto multiply = [&](const uint4 (&v)[KSTEPS]) {
+        f32x4_t c = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KSTEPS; ++s) c = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf8(xa[s]), as_bf8(v[s]), c, 0, 0, 0);
+        return c;
+    };
+    // thread e < 256 finishes output e of a tile: accumulator r = e % 4 of lane e / 4
+    const int eb = (tid >> 6) * 4 + (tid & 3), en = (tid >> 2) & 15;      // its row and column
+    u32 res_raw = 0, bias_raw = 0;
+    auto request = [&](int t) {      // (ahead of the next tile's weights: loads return in order)
+        if (!SM && wave < 4) {
+            const int n = t * 16 + en, nc = n < a.N ? n : a.N - 1;
+            if (a.residual) res_raw = a.residual[(size_t)(eb < a.B ? eb : a.B - 1) * a.N + nc];
+            if (a.bias) bias_raw = a.bias[nc];
+        }
+    };
+    auto finish = [&](int t, int par, f32x4_t c0, f32x4_t c1) {
+        *reinterpret_cast<f32x4_t*>(&red[par][0][wave][lane * 4]) = c0;
+        if (SM) *reinterpret_cast<f32x4_t*>(&red[par][NB - 1][wave][lane * 4]) = c1;
+        __syncthreads();      // (the other buffer's readers have passed the barrier of their tile before this one is written again)
+        const int n = t * 16 + en;
+        if (wave < 4 && eb < a.B && n < a.N) {
+            float v = red[par][0][0][tid], u = SM ? red[par][NB - 1][0][tid] : 0.0f;
+#pragma unroll
+            for (int w = 1; w < 8; ++w) {
+                v += red[par][0][w][tid];
+                if (SM) u += red[par][NB - 1][w][tid];
+            }
+            bf16_t o;
+            if (SM) {
+                o = f2bf(bfround(silu_c(bfround(v))) * bfround(u));
+            } else {
+                if (a.bias) v = v + bf2f((bf16_t)bias_raw);
+                o = f2bf(v);
+                if (EPI == EPI_SILU) o = f2bf(silu_c(bf2f(o)));
+                if (a.residual) o = f2bf(bf2f((bf16_t)res_raw) + bf2f(o));
+            }
+            if (a.y_rowmajor) a.y[(size_t)eb * a.N + n] = o;
+            if (a.y_frag) a.y_frag[frag_off(eb, n, a.N)] = o;
+        }
+    };
+    // (the loops request without a condition, and end before there is nothing to request: behind a conditional request the compiler waits for everything)
+    const f32x4_t none = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    int t = blockIdx.x;
+    load(w0, a.W_frag, a.W, t);
+    if constexpr (SM) {
+        if (ROWS == 1) load(w1, a.W2_frag, a.W2, t);
+        rows_ready();
+        if (ROWS != 1) load(w1, a.W2_frag, a.W2, t);      // (two rows' pieces and both tiles do not fit the registers)
+        int par = 0;
+        for (; t + step < tiles; t += step, par ^= 1) {
+            const f32x4_t c0 = multiply(w0);
+            load(w0, a.W_frag, a.W, t + step);
+            const f32x4_t c1 = multiply(w1);
+            load(w1, a.W2_frag, a.W2, t + step);
+            finish(t, par, c0, c1);
+        }
+        const f32x4_t c0 = multiply(w0), c1 = multiply(w1);
+        finish(t, par, c0, c1);
+    } else {
+        rows_ready();
+        if (t + step < tiles) load(w1, a.W_frag, a.W, t + step);
+        for (; t + 3 * step < tiles; t += 2 * step) {
+            request(t);
+            const f32x4_t c0 = multiply(w0);
+            load(w0, a.W_frag, a.W, t + 2 * step);
+            finish(t, 0, c0, none);
+            request(t + step);
+            const f32x4_t c1 = multiply(w1);
+            load(w1, a.W_frag, a.W, t + 3 * step);
+            finish(t + step, 1, c1, none);
+        }
+        request(t);
+        const f32x4_t c0 = multiply(w0);
+        if (t + 2 * step < tiles) load(w0, a.W_frag, a.W, t + 2 * step);
+        finish(t, 0, c0, none);
+        if (t + step < tiles) {
+            request(t + step);
+            finish(t + step, 1, multiply(w1), none);
+        }
+        if (t + 2 * step < tiles) {
+            request(t + 2 * step);
+            finish(t + 2 * step, 0, multiply(w0), none);
+        }
+    }
+}
+
+// ================================================================================================
 // linear for 33..128 rows with K >= 2048 (prefills): the arithmetic of k_gemm_fullk (eight contiguous K ranges, a wave each, MFMA k-steps
 // ascending, partial sums added in wave order: the same bits), the operands through LDS.  k_gemm_fullk runs its 32-row form once per row
 // tile: every block waits out the latency of its weights, and the row tiles of a column fetch them again.  Here a block has NT column
@@ -1723,6 +1887,20 @@ static bool fullk_prenorm_ok(const LinearCall& c) {
     return !c.fixed_order && !c.x_out && !c.x_rows && c.norm_scratch && c.pro == PRO_RMSNORM && (c.K == 4096 || (c.K == 2048 && c.B > 16 && dev_prenorm2048())) &&
            (c.epi == EPI_STORE || c.epi == EPI_SILU_MUL) && fullk_shape_ok(c.B, c.N, c.K, PRO_COPY, c.epi == EPI_SILU_MUL ? EPI_SILU_MUL : EPI_STORE, c.exact_rows);
 }
+// a linear of up to 16 rows whose norm prologue k_gemm_tiles takes: more column tiles than CUs (its blocks then hide the rows' trip and the norm behind weights in
+// flight, which a block per tile cannot)
+static bool gemm_tiles_ok(const LinArgs& a) {
+    const size_t at = (size_t)a.x | (size_t)(a.x_stride * 2) | (size_t)a.nw | (size_t)a.W | (size_t)a.W2;
+    return a.B <= 16 && a.K == 4096 && (at & 15) == 0 && (a.N + 15) / 16 > a.cus;
+}
+template <int EPI>
+static int launch_gemm_tiles(hipStream_t st, const LinArgs& a) {
+    constexpr int lds = 16 * 4096 * 2;
+    const auto kern = a.B <= 8 ? k_gemm_tiles<16, EPI, 1> : k_gemm_tiles<16, EPI, 2>;
+    VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    hipLaunchKernelGGL(kern, dim3(a.cus), dim3(512), lds, st, a);
+    return VOX_OK;
+}
 template <int MT, int KSTEPS, int PRO, int EPI>
 static int launch_gemm_fullk_t(hipStream_t st, const LinArgs& a0) {
     LinArgs a = a0;
@@ -1840,6 +2018,11 @@ bool vox_fullk_weight_ok(int N, int K) {
     const int ks = K / 256;
     return N % 16 == 0 && K % 256 == 0 && (ks == 4 || ks == 8 || ks == 12 || ks == 16 || ks == 24 || ks == 32);
 }
+// true when vox_launch_linear gives this call to k_linear_mfma_stream, which takes a fragment-major input too
+bool vox_linear_is_stream(const LinearCall& c) {
+    return !linear_is_fullk(c) && !vox_linear_is_rows_gemm(c) && !c.fixed_order && !c.x_out && c.B > c.exact_rows && c.B <= 16 && c.K % 32 == 0 && c.K > 1024 &&
+           c.pro == PRO_COPY && (c.epi == EPI_STORE || c.epi == EPI_SILU) && mfma_direct();
+}
 // ... and for k_linear_mfma_stream (<= 16 rows, copy prologue, K > 1024 off the full-K shapes: GLM-4-Voice's / CosyVoice2's down projection)
 bool vox_stream_weight_ok(int N, int K) { return !vox_fullk_weight_ok(N, K) && N % 16 == 0 && K % 32 == 0 && K > 1024; }
 
@@ -1870,6 +2053,7 @@ int vox_launch_linear(vox_ctx* ctx, hipStream_t st, const LinearCall& call) {
     a.x_out_stride = c.x_out_stride ? c.x_out_stride : c.K; a.eps = c.eps; a.B = c.B; a.N = c.N; a.K = c.K; a.Hq = c.Hq; a.D = c.D;
     a.max_chunks = c.max_chunks;
     a.keep = c.keep_weights;
+    a.cus = ctx->n_cu;
     a.post_nw = (const bf16_t*)c.post_norm_w; a.post_out = (bf16_t*)c.post_norm_out; a.post_eps = c.eps;
     a.y_rowmajor = 1;
     if (linear_is_fullk(c)) {
@@ -1877,8 +2061,10 @@ int vox_launch_linear(vox_ctx* ctx, hipStream_t st, const LinearCall& call) {
         a.y_frag = (bf16_t*)c.y_frag; a.y_rowmajor = c.y_rowmajor || !c.y_frag;
         if (c.epi == EPI_SILU_MUL && (a.W_frag == nullptr) != (a.W2_frag == nullptr))
             return vox_fail(VOX_ERR_INVALID, "linear: W_frag and W2_frag must be given together");
+    } else if (c.x_frag && vox_linear_is_stream(c)) {
+        a.x_frag = (const bf16_t*)c.x_frag;
     } else if (c.x_frag && !c.x) {
-        return vox_fail(VOX_ERR_INVALID, "linear: fragment-major input outside the 9..32 rows path");
+        return vox_fail(VOX_ERR_INVALID, "linear: fragment-major input outside the paths that read it");
     }
     const int ncu = ctx->n_cu;
     int pro = c.pro, epi = c.epi;
@@ -1901,6 +2087,7 @@ int vox_launch_linear(vox_ctx* ctx, hipStream_t st, const LinearCall& call) {
             return launch_gemm_fullk<PRO_COPY, EPI_STORE>(st, a);
         }
 #endif
+        if (gemm_tiles_ok(a)) return epi == EPI_SILU_MUL ? launch_gemm_tiles<EPI_SILU_MUL>(st, a) : launch_gemm_tiles<EPI_STORE>(st, a);
         hipLaunchKernelGGL(k_rmsnorm, dim3((c.B + 3) / 4), dim3(256), 0, st, a.x, a.nw, (bf16_t*)c.norm_scratch, c.B, c.K, c.eps);
         a.x = (const bf16_t*)c.norm_scratch; a.x_stride = c.K; a.x_frag = nullptr;
         if (c.B > 32 && gemm_rows_ok(c)) return epi == EPI_SILU_MUL ? launch_gemm_rows<EPI_SILU_MUL>(st, a) : launch_gemm_rows<EPI_STORE>(st, a);

@@ -74,6 +74,7 @@ enum { VOX_PRO_COPY = 0, VOX_PRO_RMSNORM = 1, VOX_PRO_ATTN = 2 };
 enum { VOX_EPI_STORE = 0, VOX_EPI_SILU = 1, VOX_EPI_SILU_MUL = 2 };
 bool vox_linear_is_rows_gemm(const LinearCall& c);
 bool vox_linear_is_fullk(const LinearCall& c);      // true: the call takes the 9..32 rows path that honours *_frag
+bool vox_linear_is_stream(const LinearCall& c);     // true: a copy-prologue linear of <= 16 rows that reads x_frag if given
 bool vox_fullk_weight_ok(int N, int K);
 bool vox_stream_weight_ok(int N, int K);             // a weight of this shape can be used fragment-major
 int vox_launch_swizzle_frag(hipStream_t st, const void* src, void* dst, int rows, int K);   // rows % 16 == 0, K % 32 == 0
