@@ -116,12 +116,20 @@ def test_dense_units_of_few_rows(width, ff, cuts):
     check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)
 
 
+# Products of 2 to 16 rows whose columns make more tiles than there are CUs (a head's, and gate and up): one tile more, whole rounds, a last round of one block,
+# a last tile of one column; every K that a wave's registers hold, with the rows' requests of several requests a step
+@pytest.mark.parametrize("width,vocab,ff,cuts", [(512, 4097, 2056, [8, 16, 2]), (1024, 8192, 4096, [3, 9]), (1536, 8193, 64, [16, 5]), (2048, 12305, 2064, [7, 2, 16])])
+def test_more_column_tiles_than_cus(width, vocab, ff, cuts):
+    cfg = P.config([P.attention(mlp=P.dense(ff), **ATT)], width=width, vocab=vocab, bigram=None)
+    check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)
+
+
 # 2 to 8 rows, routed layers of wide experts (inner widths of 2048 and more, or many weights in all): rows of one piece, of a few columns into the next, of
 # two whole rounds; one to 64 entries, an odd one at the end; inner widths of one round, a few columns into the next, two rounds, and less than one piece
 @pytest.mark.parametrize("width,moe,cuts", [(64, (2, 2, 2048, 0, 0), [2, 8, 3]), (512, (3, 1, 4096, 0, 0), [8, 7]), (2048, (8, 2, 2048, 4, 2), [8, 2, 5]),
                                             (2056, (4, 2, 2048, 0, 0), [8, 3]), (4096, (5, 5, 2056, 0, 0), [7, 8, 2]), (3080, (4, 3, 2120, 0, 0), [4, 6]),
                                             (256, (48, 6, 2048, 4, 2), [8, 6]), (64, (48, 16, 2048, 0, 0), [3, 4]), (128, (16, 8, 4104, 0, 0), [8, 8]),
-                                            (4096, (8, 8, 168, 0, 0), [8])])
+                                            (4096, (8, 8, 168, 0, 0), [8]), (4096, (4, 1, 2048, 0, 0), [8, 3]), (2052, (8, 2, 2048, 0, 0), [6, 8])])
 def test_routed_layers_of_few_rows(width, moe, cuts):
     cfg = P.config([P.attention(mlp=P.moe(*moe), **ATT), P.attention(mlp=P.moe(*moe), kv_from=0, **ATT)], width=width, vocab=50)
     check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)

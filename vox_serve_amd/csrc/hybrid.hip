@@ -1285,6 +1285,123 @@ __global__ __launch_bounds__(512) void k_hb_gemm_rows16(const float* A, long lda
         else hb_finish<EPI>(rm, C, ldc, orow, n0 + ocol, sum, bz);
     }
 }
+// The same product for K = 256 U where there are more column tiles than CUs: a block per CU walks the tiles blockIdx.x, + gridDim.x, ...  Its waves keep
+// their steps of the rows in registers as bf16 (a block per tile reads them again each time, twice the bytes of its weights), and the next tile's weights are in
+// flight while this one's are multiplied and summed.  The sums are the kernel's above: same bits.
+// GLU: a tile is eight gate and the same eight up columns (column c + 8 of the tile is up column c; N = the inner width), the activation is in the
+// epilogue, and out16 stores bf16.
+// Bound by the weights' way from memory.  8 rows, a block per tile -> here, us: gate and up 11264 x 2048 (46 MB) 15.4 -> 12.1, q | k | v 5120 x 2048 10.4 -> 8.9, a head of 32000 x
+// 2048 (131 MB) 36.2 -> 26.9.  Whole steps of 2 to 16 rows, K = 512, 1024, 1536, 2048 with 257 to 2000 column tiles: 0.2 to 17 % faster, none slower.
+struct hb_glu_out {
+    hb_glu_args glu;
+    int out16;
+};
+template <int EPI, int U, bool GLU>
+__global__ __launch_bounds__(512) void k_hb_rows_walk(const float* A, long lda, const bf16_t* Wt, const float* bias, float* C, long ldc, int M, int N,
+                                                      hb_rowmap rm, hb_glu_out go) {
+    constexpr int TC = GLU ? 8 : 16;      // output columns of a tile
+    __shared__ float red[2][8][16][17];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 15, kb = lane >> 4;
+    const int tiles = (N + TC - 1) / TC, step = gridDim.x;
+    const float* arow = A + (size_t)(col < M ? col : M - 1) * lda + wv * 32 + kb * 8;
+    uint4 af[U], w0[U], w1[U];
+    float4 a0[U], a1[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        a0[u] = *(const float4*)(arow + 256 * u);
+        a1[u] = *(const float4*)(arow + 256 * u + 4);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    auto load = [&](uint4 (&w)[U], int t) {
+        int n;
+        if (GLU) {
+            n = t * 8 + (col & 7);
+            n = (col >> 3) * N + (n < N ? n : N - 1);
+        } else {
+            n = t * 16 + col;
+            n = n < N ? n : N - 1;
+        }
+        const bf16_t* wrow = Wt + (size_t)n * (256 * U) + wv * 32 + kb * 8;
+#pragma unroll
+        for (int u = 0; u < U; ++u) w[u] = ldg_nt((const uint4*)(wrow + 256 * u));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    int t = blockIdx.x, par = 0;
+    load(w0, t);
+    const bool rowok = col < M;
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        const uint4 v = make_uint4(pack_bf2(a0[u].x, a0[u].y), pack_bf2(a0[u].z, a0[u].w), pack_bf2(a1[u].x, a1[u].y), pack_bf2(a1[u].z, a1[u].w));
+        af[u] = rowok ? v : make_uint4(0, 0, 0, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    const int orow = GLU ? threadIdx.x >> 3 : threadIdx.x >> 4, ocol = threadIdx.x & (TC - 1);
+    const bool mine = threadIdx.x < 16 * TC && orow < M;
+    // the tile's biases, asked for ahead of the next tile's weights (loads return in order) and, where there are none, from the weights: a value that only
+    // some paths load is waited for with everything in flight
+    const float* const bp = bias ? bias : (const float*)Wt;
+    const int blast = bias ? N - 1 : 0;
+    auto request = [&](int t) {
+        const int n = t * TC + ocol < blast ? t * TC + ocol : blast;
+        return make_float2(bp[n], GLU ? bp[bias ? N + n : 0] : 0.f);
+    };
+    auto tile = [&](const uint4 (&w)[U], int t, float2 b2) {
+        hb_f32x4 acc = hb_f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            union { uint4 q; hb_bf16x8 b; } a, b;
+            a.q = af[u];
+            b.q = w[u];
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a.b, b.b, acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) red[par][wv][kb * 4 + r][col] = acc[r];
+        __syncthreads();      // (this buffer's readers of two tiles ago have passed the barrier of the tile between)
+        const float (*const p)[16][17] = red[par];
+        par ^= 1;
+        const int n = t * TC + ocol;
+        if (mine && n < N) {
+            float sum = p[0][orow][ocol], up = GLU ? p[0][orow][8 + ocol] : 0.f;
+#pragma unroll
+            for (int v = 1; v < 8; ++v) {
+                sum += p[v][orow][ocol];
+                if (GLU) up += p[v][orow][8 + ocol];
+            }
+            const float bz = bias ? b2.x : 0.f, bu = bias ? b2.y : 0.f;
+            if (GLU) {
+                const float y = hb_glu(sum + bz, up + bu, go.glu.limit, go.glu.alpha, go.glu.up_offset, go.glu.gelu);
+                const size_t o = (size_t)orow * ldc + n;
+                if (go.out16) ((bf16_t*)C)[o] = f2bf(y);
+                else C[o] = y;
+            } else hb_finish<EPI>(rm, C, ldc, orow, n, sum, bz);
+        }
+    };
+    while (true) {      // (the request for the next tile and the one that is multiplied lie in one path: the waits stay exact)
+        const float2 b0 = request(t);
+        if (t + step >= tiles) { tile(w0, t, b0); break; }
+        load(w1, t + step);
+        tile(w0, t, b0);
+        t += step;
+        const float2 b1 = request(t);
+        if (t + step >= tiles) { tile(w1, t, b1); break; }
+        load(w0, t + step);
+        tile(w1, t, b1);
+        t += step;
+    }
+}
+#define HB_WALK_BLOCKS 256
+template <int EPI, bool GLU>
+static bool hb_rows_walk(hipStream_t st, const float* A, long lda, const bf16_t* W, const float* bias, float* C, long ldc, int M, int N, int K, const hb_rowmap& rm,
+                         hb_glu_out go) {
+    if (M < 2 || M > 16 || K > 2048 || (K & 255) || (lda & 3) || ((size_t)A & 15) || ((size_t)W & 15) || (N + (GLU ? 7 : 15)) / (GLU ? 8 : 16) <= HB_WALK_BLOCKS) return false;
+#define HB_WALK(U_) \
+    case U_: hipLaunchKernelGGL((k_hb_rows_walk<EPI, U_, GLU>), dim3(HB_WALK_BLOCKS), dim3(512), 0, st, A, lda, W, bias, C, ldc, M, N, rm, go); break;
+    switch (K >> 8) { HB_WALK(2) HB_WALK(4) HB_WALK(6) HB_WALK(8) default: return false; }
+#undef HB_WALK
+    return true;
+}
+template <int EPI, bool GLU>
+static bool hb_rows_walk(hipStream_t, const float*, long, const float*, const float*, float*, long, int, int, int, const hb_rowmap&, hb_glu_out) { return false; }
 // every operand of every product of a strided batch is 16-byte aligned
 static inline bool hb_batch_aligned(const hb_rowmap& rm, int nz, size_t wsize) {
     return nz == 1 || ((rm.w_stride * wsize) % 16 == 0 && (rm.a_stride * 4) % 16 == 0);
@@ -1458,7 +1575,9 @@ int hb_gemm_epi(hb_ws16 ws, hipStream_t st, const float* A, long lda, const T* W
         if (wide) hipLaunchKernelGGL((k_hb_gemv<T, MR_, EPI, 4>), g, b, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm); \
         else hipLaunchKernelGGL((k_hb_gemv<T, MR_, EPI, 1>), g, b, 0, st, A, lda, W, bias, C, ldc, M, N, K, rm); \
     } while (0)
-    if (hb_try_rows16<EPI>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz)) {}
+    bool done = false;
+    if constexpr (EPI != HB_EPI_JOIN) done = !ws.general && nz == 1 && hb_rows_walk<EPI, false>(st, A, lda, W, bias, C, ldc, M, N, K, rm, hb_glu_out{});
+    if (done || hb_try_rows16<EPI>(st, A, lda, W, bias, C, ldc, M, N, K, rm, nz)) {}
     else if (M == 1) HB_GEMV(1);
     else if (M == 2) HB_GEMV(2);
     else if (M <= 4) HB_GEMV(4);
@@ -5068,6 +5187,7 @@ __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, cons
 // activation is in its epilogue.  out: rows of ldo elements, bf16 where out16.
 // Bound by the weights' way from memory.  8 rows, 11264 x 2048 (46 MB): 15.4 us + 4.8 for the activation's own launch -> 16.0.  Column tiles walked by one
 // block, with the next tile's weights asked for ahead and the rows kept: 22 - 28, the registers leave too few blocks.
+template <bool FULL>
 __global__ __launch_bounds__(512) void k_hb_glu_rows(const float* A, long lda, const bf16_t* Wt, const float* bias, void* out, long ldo, int out16, int M, int ff,
                                                      int K, hb_glu_args glu) {
     __shared__ float red[8][16][17];
@@ -5082,14 +5202,15 @@ __global__ __launch_bounds__(512) void k_hb_glu_rows(const float* A, long lda, c
         float4 a0[U], a1[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const int k = (s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5;
+            const int k = (FULL || s0 + 8 * u < nsteps ? s0 + 8 * u : s0) << 5;
             wf[u] = *(const uint4*)(wrow + k);
             a0[u] = *(const float4*)(arow + k);
             a1[u] = *(const float4*)(arow + k + 4);
         }
+        if (FULL) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            if (s0 + 8 * u >= nsteps) break;
+            if (!FULL && s0 + 8 * u >= nsteps) break;
             union { uint4 q; hb_bf16x8 b; } af, bfv;
             af.q.x = pack_bf2(a0[u].x, a0[u].y); af.q.y = pack_bf2(a0[u].z, a0[u].w);
             af.q.z = pack_bf2(a1[u].x, a1[u].y); af.q.w = pack_bf2(a1[u].z, a1[u].w);
@@ -5170,103 +5291,122 @@ __device__ __forceinline__ float hb_dot8(uint4 u, uint4 v, float a) {
     a = fmaf(bflo(u.x), bflo(v.x), a); a = fmaf(bfhi(u.x), bfhi(v.x), a); a = fmaf(bflo(u.y), bflo(v.y), a); a = fmaf(bfhi(u.y), bfhi(v.y), a);
     a = fmaf(bflo(u.z), bflo(v.z), a); a = fmaf(bfhi(u.z), bfhi(v.z), a); a = fmaf(bflo(u.w), bflo(v.w), a); return fmaf(bfhi(u.w), bfhi(v.w), a);
 }
-// Gate and up rows of the routed entries with their activation, k_hb_moe_gate_up's sums (hb_dot_wave).  Block (columns, entry): the first entry of an expert
-// takes all of that expert's, the blocks of the others end at once, so a weight is read and widened once a step, not once an entry.  The
+// Gate and up rows of the routed entries with their activation, k_hb_moe_gate_up's sums (hb_dot_wave).  The blocks are shared out among the distinct experts and walk
+// their columns eight at a time, for all of an expert's entries, so a weight is read and widened once a step, not once an entry.  The
 // entries' rows lie in LDS as the bf16 that the products see; a wave has two gate and two up rows and multiplies a piece of them by all entries.
 // Bound by the weights' way from memory and the products on the vector units, which keep the order of the sums (on the matrix cores 27.8).  8 rows, 16
 // choices among 8 experts of 2048 x 2048 (up to 134 MB of distinct rows, 268 with each entry reading
-// its own): 38.7 -> 31.8 us.
+// its own): 38.7 -> 29.9 us (31.8 with a block for each group of columns and entry, most of which ended at once, and no weights in flight while others are multiplied).
 #define HB_MOE_UP_ROWS 8
-__global__ __launch_bounds__(256) void k_hb_moe_up_rows(const float* h, long ldh, const bf16_t* w_gate_up, bf16_t* act, int W, int ff, int M, hb_glu_args glu,
+// Two blocks to a CU, or one for every unit that there can be (eight columns of an entry's expert) while that is few: 2 rows, 3 choices among 8 experts of 2048 x
+// 1024, a step of three such layers 184 us with a block each and 189 with 512 that walk.
+static int hb_moe_up_blocks(int entries, int ff) {
+    const int units = entries * ((ff + 7) / 8);
+    return units <= 1280 ? units : 512;
+}
+// the entries that share this lane's expert with an earlier one left out: one bit for each routed expert (ne <= 64 entries, one a lane)
+__device__ __forceinline__ unsigned long long hb_moe_leaders(int sel, int ne, int experts, int lane) {
+    bool first = lane < ne && sel < experts;
+    for (int j = 0; j + 1 < ne; ++j) first = first && !(j < lane && __builtin_amdgcn_readlane(sel, j) == sel);
+    return __ballot(first);
+}
+__global__ __launch_bounds__(256, 2) void k_hb_moe_up_rows(const float* h, long ldh, const bf16_t* w_gate_up, bf16_t* act, int W, int ff, int M, hb_glu_args glu,
                                                         hb_entries en) {
     extern __shared__ __attribute__((aligned(16))) bf16_t rows[];      // [HB_MOE_UP_ROWS][W]
     constexpr int NC = 4, NE = HB_MOE_UP_ROWS;
-    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ne = M * en.top, e = en.sel[blockIdx.y];
-    if (e >= en.experts) return;
-    unsigned long long left = __ballot(lane < ne && en.sel[lane < ne ? lane : 0] == e);
-    if (__builtin_ctzll(left) != (int)blockIdx.y) return;
-    const int n0 = blockIdx.x * 8 + wv * 2;
-    const bf16_t* w[4];      // gate, gate, up, up
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-        const int n = n0 + (r & 1) < ff ? n0 + (r & 1) : ff - 1;
-        w[r] = w_gate_up + ((size_t)e * 2 * ff + (size_t)(r >> 1) * ff + n) * W + lane * 8;
-    }
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6), ne = M * en.top, groups = (ff + 7) >> 3;
+    const int mine = en.sel[lane < ne ? lane : 0];
+    unsigned long long lead = hb_moe_leaders(mine, ne, en.experts, lane);
+    const int nd = (int)__popcll(lead);
+    if (nd == 0) return;
+    // blocks slot, slot + nd, ... walk the columns of the slot-th expert
+    const int slot = (int)blockIdx.x % nd, x0 = (int)blockIdx.x / nd, nx = ((int)gridDim.x - slot + nd - 1) / nd;
+    if (x0 >= groups) return;
+    for (int i = 0; i < slot; ++i) lead &= lead - 1;
+    const int e = __builtin_amdgcn_readlane(mine, __builtin_ctzll(lead));
+    unsigned long long left = __ballot(lane < ne && mine == e);
+    const bf16_t* const we = w_gate_up + (size_t)e * 2 * ff * W + lane * 8;
+    const int nch = (W + 512 * NC - 1) / (512 * NC), units = ((groups - x0 + nx - 1) / nx) * nch;      // a unit: a group of columns, 512 NC elements of K
+    // Each piece's registers take the next unit's as soon as they have been multiplied (behind the last unit: the expert's first piece, which nobody multiplies).
     uint4 wr[NC][4];
-    auto load = [&](int c0) {
+    auto load = [&](int c, int u) {
+        const bool more = u < units;
+        const int n0 = more ? (x0 + u / nch * nx) * 8 + wv * 2 : 0, k = more ? u % nch * (512 * NC) + 512 * c : 0;
+        const int kl = k + lane * 8 < W ? k : -lane * 8;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-            if (512 * (c0 + c) >= W) break;
-            const int k = lane * 8 + 512 * (c0 + c), o = k < W ? 512 * (c0 + c) : 0;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) wr[c][r] = *(const uint4*)(w[r] + (k < W || lane * 8 < W ? o : -lane * 8));
+        for (int r = 0; r < 4; ++r) {      // gate, gate, up, up
+            const int n = n0 + (r & 1) < ff ? n0 + (r & 1) : ff - 1;
+            wr[c][r] = ldg((const uint4*)(we + (size_t)(more ? (r >> 1) * ff + n : 0) * W + kl));
         }
     };
     while (left) {      // (an expert has an entry of a row once; more than 8 only where scores are no numbers)
         int nb = 0, ent[NE];
 #pragma unroll
         for (int j = 0; j < NE; ++j) {
-            ent[j] = left ? __builtin_ctzll(left) : 0;
+            ent[j] = left ? __builtin_ctzll(left) : ent[0];
             nb += left ? 1 : 0;
             left &= left - 1;
         }
-        load(0);
 #pragma unroll
-        for (int j = 0; j < NE; ++j) {
-            if (j >= nb) break;
-            const float* x = h + (size_t)(ent[j] / en.top) * ldh;
-            const float xs = en.scale_input ? en.wgt[ent[j]] : 1.0f;
+        for (int c = 0; c < NC; ++c) load(c, 0);
+        for (int j0 = 0; j0 < nb; j0 += 2) {
+            const int ea = j0 == 0 ? ent[0] : j0 == 2 ? ent[2] : j0 == 4 ? ent[4] : ent[6], eb = j0 == 0 ? ent[1] : j0 == 2 ? ent[3] : j0 == 4 ? ent[5] : ent[7];
+            const float *xa = h + (size_t)(ea / en.top) * ldh, *xb = h + (size_t)(eb / en.top) * ldh;
+            const float sa = en.scale_input ? en.wgt[ea] : 1.0f, sb = en.scale_input ? en.wgt[eb] : 1.0f;
             for (int k = tid * 4; k < W; k += 1024) {
-                const float4 v = *(const float4*)(x + k);
-                *(uint2*)(rows + (size_t)j * W + k) = make_uint2(pack_bf2(v.x * xs, v.y * xs), pack_bf2(v.z * xs, v.w * xs));
+                const float4 v = *(const float4*)(xa + k), w = *(const float4*)(xb + k);
+                *(uint2*)(rows + (size_t)j0 * W + k) = make_uint2(pack_bf2(v.x * sa, v.y * sa), pack_bf2(v.z * sa, v.w * sa));
+                *(uint2*)(rows + (size_t)(j0 + 1) * W + k) = make_uint2(pack_bf2(w.x * sb, w.y * sb), pack_bf2(w.z * sb, w.w * sb));
             }
         }
         __syncthreads();
         float acc[NE][4];
+        for (int u = 0; u < units; ++u) {
+            const int c0 = u % nch * NC, n0 = (x0 + u / nch * nx) * 8 + wv * 2;
+            if (c0 == 0)
 #pragma unroll
-        for (int j = 0; j < NE; ++j)
+                for (int j = 0; j < NE; ++j)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) acc[j][r] = 0.f;
-        for (int c0 = 0; c0 * 512 < W; c0 += NC) {
-            if (c0 > 0) load(c0);
+                    for (int r = 0; r < 4; ++r) acc[j][r] = 0.f;
 #pragma unroll
             for (int c = 0; c < NC; ++c) {
-                if (512 * (c0 + c) >= W) break;
-                const int k = lane * 8 + 512 * (c0 + c);
-                if (k >= W) break;
+                const int k = lane * 8 + 512 * (c0 + c), kc = k < W ? k : 0;
                 float wf[4][8];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    const uint4 u = wr[c][r];
-                    wf[r][0] = bflo(u.x); wf[r][1] = bfhi(u.x); wf[r][2] = bflo(u.y); wf[r][3] = bfhi(u.y);
-                    wf[r][4] = bflo(u.z); wf[r][5] = bfhi(u.z); wf[r][6] = bflo(u.w); wf[r][7] = bfhi(u.w);
+                    const uint4 q = wr[c][r];
+                    wf[r][0] = bflo(q.x); wf[r][1] = bfhi(q.x); wf[r][2] = bflo(q.y); wf[r][3] = bfhi(q.y);
+                    wf[r][4] = bflo(q.z); wf[r][5] = bfhi(q.z); wf[r][6] = bflo(q.w); wf[r][7] = bfhi(q.w);
                 }
+                load(c, u + 1);
+                __builtin_amdgcn_sched_barrier(0);
+                if (k < W)
 #pragma unroll
-                for (int j = 0; j < NE; ++j) {
-                    if (j >= nb) break;
-                    const uint4 u = *(const uint4*)(rows + (size_t)j * W + k);
-                    const float xf[8] = {bflo(u.x), bfhi(u.x), bflo(u.y), bfhi(u.y), bflo(u.z), bfhi(u.z), bflo(u.w), bfhi(u.w)};
+                    for (int j = 0; j < NE; ++j) {
+                        if (j >= nb) break;
+                        const uint4 q = *(const uint4*)(rows + (size_t)j * W + kc);
+                        const float xf[8] = {bflo(q.x), bfhi(q.x), bflo(q.y), bfhi(q.y), bflo(q.z), bfhi(q.z), bflo(q.w), bfhi(q.w)};
 #pragma unroll
-                    for (int i = 0; i < 8; ++i)
+                        for (int i = 0; i < 8; ++i)
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(wf[r][i], xf[i], acc[j][r]);
-                }
+                            for (int r = 0; r < 4; ++r) acc[j][r] = fmaf(wf[r][i], xf[i], acc[j][r]);
+                    }
             }
-        }
-        // hb_wave_sum's tree, with the values spread over the lanes at its first two steps: lanes 0, 16, 32, 48 are left with row 0, 1, 2, 3
-        const bool b5 = lane & 32, b4 = lane & 16;
+            if (u % nch != nch - 1) continue;
+            // hb_wave_sum's tree, with the values spread over the lanes at its first two steps: lanes 0, 16, 32, 48 are left with row 0, 1, 2, 3
+            const bool b5 = lane & 32, b4 = lane & 16;
 #pragma unroll
-        for (int j = 0; j < NE; ++j) {
-            if (j >= nb) break;
-            const float v0 = (b5 ? acc[j][2] : acc[j][0]) + __shfl_xor(b5 ? acc[j][0] : acc[j][2], 32, 64);
-            const float v1 = (b5 ? acc[j][3] : acc[j][1]) + __shfl_xor(b5 ? acc[j][1] : acc[j][3], 32, 64);
-            float v = (b4 ? v1 : v0) + __shfl_xor(b4 ? v0 : v1, 16, 64);
-#pragma unroll
-            for (int o = 8; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
-            const float up = __shfl_xor(v, 32, 64);
-            const int n = n0 + (lane >> 4);
-            if (lane < 32 && (lane & 15) == 0 && n < ff)
-                act[(size_t)ent[j] * ff + n] = f2bf(hb_glu(v, up, glu.limit, glu.alpha, glu.up_offset, glu.gelu));
+            for (int j = 0; j < NE; ++j) {
+                if (j >= nb) break;
+                const float v0 = (b5 ? acc[j][2] : acc[j][0]) + __shfl_xor(b5 ? acc[j][0] : acc[j][2], 32, 64);
+                const float v1 = (b5 ? acc[j][3] : acc[j][1]) + __shfl_xor(b5 ? acc[j][1] : acc[j][3], 32, 64);
+                float v = (b4 ? v1 : v0) + __shfl_xor(b4 ? v0 : v1, 16, 64);
+                v = butterfly<16>(v);
+                const float up = __shfl_xor(v, 32, 64);
+                const int n = n0 + (lane >> 4);
+                if (lane < 32 && (lane & 15) == 0 && n < ff)
+                    act[(size_t)ent[j] * ff + n] = f2bf(hb_glu(v, up, glu.limit, glu.alpha, glu.up_offset, glu.gelu));
+            }
         }
         if (left) __syncthreads();
     }
@@ -5325,6 +5465,93 @@ __global__ __launch_bounds__(256) void k_hb_moe_down_rows(const bf16_t* act, con
     }
     if (lane == 0) hb_join_apply(join, jin, C + (size_t)row * ldc, row, c, acc);
 }
+// The same for one or two choices and K <= 2048: 64 blocks of each XCD are shared out among the rows, and a block's waves walk that XCD's columns, the row's
+// activations in registers, the next column's weights in flight while this one's are multiplied.
+// 8 rows, 2048 x 2048, 16 choices among 8 experts: 18.4 -> 16.2 us.
+#define HB_MOE_DOWN_BLOCKS 512      // two to a CU, 64 to an XCD
+template <bool TWO>
+__global__ __launch_bounds__(256, 2) void k_hb_moe_down_walk(const bf16_t* act, const bf16_t* w_down, const float* h, long ldh, float* C, long ldc, int M, int N, int K,
+                                                             hb_join join, hb_entries en) {
+    constexpr int NC = 4, NE = TWO ? 2 : 1;
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), in_xcd = (int)blockIdx.x >> 3;
+    const int row = in_xcd % M, at = in_xcd / M, step = (HB_MOE_DOWN_BLOCKS / 8 / M) * 32, i0 = row * en.top;
+    if (at >= HB_MOE_DOWN_BLOCKS / 8 / M) return;
+    int c = (at * 8 + ((int)blockIdx.x & 7)) * 4 + wv;
+    const bool b5 = lane & 32;
+    int e[NE];
+    float wg[NE];
+    const bf16_t* p[NE];
+    uint4 v[NE][NC], ua[NE][NC], ub[NE][NC];
+    int ko[NC];
+#pragma unroll
+    for (int i = 0; i < NC; ++i) ko[i] = 512 * i + lane * 8 < K ? 512 * i + lane * 8 : 0;
+#pragma unroll
+    for (int j = 0; j < NE; ++j) {
+        e[j] = en.sel[i0 + j];
+        wg[j] = en.wgt[i0 + j];
+        p[j] = w_down + (size_t)(e[j] < en.experts ? e[j] : 0) * N * K;
+#pragma unroll
+        for (int i = 0; i < NC; ++i) v[j][i] = ldg((const uint4*)(act + (size_t)(i0 + j) * K + ko[i]));
+    }
+    auto load = [&](uint4 (&u)[NE][NC], int c) {
+#pragma unroll
+        for (int j = 0; j < NE; ++j)
+#pragma unroll
+            for (int i = 0; i < NC; ++i) u[j][i] = ldg((const uint4*)(p[j] + (size_t)c * K + ko[i]));
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    float s0 = 0.f, s1 = 0.f;      // lane t: the sums of the wave's t-th column
+    int t = 0;
+    auto column = [&](const uint4 (&u)[NE][NC]) {
+        float a[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < NC; ++i) {
+            if (512 * i >= K) break;
+            if (512 * i + lane * 8 < K)
+#pragma unroll
+                for (int j = 0; j < NE; ++j) a[j] = hb_dot8(u[j][i], v[j][i], a[j]);
+        }
+        float d = (b5 ? a[1] : a[0]) + __shfl_xor(b5 ? a[0] : a[1], 32, 64);      // (hb_wave_sum's tree, an entry to each half of the wave)
+        d = butterfly<32>(d);
+        const float d0 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(d), 0)), d1 = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(d), 32));
+        s0 = lane == t ? d0 : s0;
+        s1 = lane == t ? d1 : s1;
+        ++t;
+    };
+    // 64 columns at most between two of these: their joins together, a lane a column
+    auto finish = [&](int first) {
+        const int cl = first + lane * step;
+        if (lane < t) {
+            const hb_join_in jin = hb_join_load(join, C + (size_t)row * ldc, row, cl);
+            const float hv = e[0] >= en.experts || e[NE - 1] >= en.experts ? h[(size_t)row * ldh + cl] : 0.f;
+            float acc = 0.f;
+            if (e[0] >= en.experts) acc = fmaf(wg[0], hv, acc);
+            else acc = fmaf(en.scale_input ? 1.0f : wg[0], s0, acc);
+            if (TWO) {
+                if (e[NE - 1] >= en.experts) acc = fmaf(wg[NE - 1], hv, acc);
+                else acc = fmaf(en.scale_input ? 1.0f : wg[NE - 1], s1, acc);
+            }
+            hb_join_apply(join, jin, C + (size_t)row * ldc, row, cl, acc);
+        }
+        t = 0;
+    };
+    while (c < N) {
+        const int first = c, end = N - c > 64 * step ? c + 64 * step : N;
+        load(ua, c);
+        while (true) {      // (a column's weights and the next one's lie in one path: the waits stay exact)
+            if (c + step >= end) { column(ua); break; }
+            load(ub, c + step);
+            column(ua);
+            c += step;
+            if (c + step >= end) { column(ub); break; }
+            load(ua, c + step);
+            column(ub);
+            c += step;
+        }
+        c += step;
+        finish(first);
+    }
+}
 static bool hb_glu_rows_ok(const float* A, long lda, const bf16_t* W, int M, int K) {
     return M >= 2 && M <= 16 && !(K & 31) && !(lda & 3) && !((size_t)A & 15) && !((size_t)W & 15);
 }
@@ -5338,7 +5565,13 @@ static bool hb_try_ff_rows(hipStream_t st, const float* A, long lda, const bf16_
                            float* C, long ldc, int M, int W, int ff, hb_glu_args glu, const hb_join& join, bool* done) {
     if (!hb_glu_rows_ok(A, lda, w_up, M, W)) return false;
     *done = M <= 8 && W <= HB_DOWN8_COLS && !(ff & 31) && !((size_t)w_down & 15);
-    hipLaunchKernelGGL(k_hb_glu_rows, dim3((ff + 7) / 8), dim3(512), 0, st, A, lda, w_up, b_up, (void*)act, (long)ff, *done ? 1 : 0, M, ff, W, glu);
+    if (!hb_rows_walk<HB_EPI_STORE, true>(st, A, lda, w_up, b_up, act, ff, M, ff, W, hb_plain(), hb_glu_out{glu, *done ? 1 : 0}))
+    {
+        // whole rounds of requests: all of a round in flight (4096 wide, 11008: steps 1 - 2 % faster, 2048 wide, 2048: 3 - 6 %); else a step at a time by more blocks to a CU
+        // (with zero rows for the steps that are not there 2560 wide, 6912: 10 % slower, 512 wide, 1408: 7 %)
+        if (W % 2048 == 0) hipLaunchKernelGGL(k_hb_glu_rows<true>, dim3((ff + 7) / 8), dim3(512), 0, st, A, lda, w_up, b_up, (void*)act, (long)ff, *done ? 1 : 0, M, ff, W, glu);
+        else hipLaunchKernelGGL(k_hb_glu_rows<false>, dim3((ff + 7) / 8), dim3(512), 0, st, A, lda, w_up, b_up, (void*)act, (long)ff, *done ? 1 : 0, M, ff, W, glu);
+    }
     if (*done)
         hipLaunchKernelGGL(k_hb_down_rows8, dim3((W + 7) / 8), dim3(256), 0, st, (const bf16_t*)act, (long)ff, w_down, b_down, C, ldc, M, W, ff, join);
     return true;
@@ -5359,8 +5592,12 @@ static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16
     const size_t lds = (size_t)HB_MOE_UP_ROWS * W * 2;
     if (M < 2 || M * en.top > 64 || en.experts < 1 || (W & 7) || (ldh & 3) || ((size_t)h & 15) || ((size_t)w_gate_up & 15) || (ff & 7) || ((size_t)w_down & 15) ||
         lds > 64 * 1024 || !hb_moe_rows_pay(M, W, ff, en.top)) return false;
-    hipLaunchKernelGGL(k_hb_moe_up_rows, dim3((ff + 7) / 8, M * en.top), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
-    hipLaunchKernelGGL(k_hb_moe_down_rows, dim3((W + 31) / 32 * 8 * M), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
+    hipLaunchKernelGGL(k_hb_moe_up_rows, dim3(hb_moe_up_blocks(M * en.top, ff)), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
+    if (en.top == 2 && ff <= 2048)
+        hipLaunchKernelGGL(k_hb_moe_down_walk<true>, dim3(HB_MOE_DOWN_BLOCKS), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
+    else if (en.top == 1 && ff <= 2048)
+        hipLaunchKernelGGL(k_hb_moe_down_walk<false>, dim3(HB_MOE_DOWN_BLOCKS), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
+    else hipLaunchKernelGGL(k_hb_moe_down_rows, dim3((W + 31) / 32 * 8 * M), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
     return true;
 }
 static bool hb_try_moe_rows(hipStream_t, const float*, long, const float*, const float*, float*, float*, long, int, int, int, hb_glu_args, const hb_join&, hb_entries) {
