@@ -191,6 +191,7 @@ __device__ __forceinline__ void conv_epilogue(const ConvGemmArgs& a, f32x4 (&acc
 // 64 x 64 grid would leave most of the 256 CUs idle (the mid-size decoder stages are MFMA-bound per CU).
 template <int BK, int WM, int WN, bool UNR = false>
 __global__ __launch_bounds__(256, (WM * WN > 12 ? 3 : 4)) void k_conv_gemm(ConvGemmArgs a) {
+    touch_args(a);
     constexpr int BM = 32 * WM, BN = 32 * WN;
     constexpr int LD = BK + 8;          // LDS row stride in bf16 elements (+16 B: the 16 rows of a fragment read hit distinct banks)
     constexpr int SEG = BK / 8;         // 8-element segments per row
@@ -364,18 +365,27 @@ __device__ __forceinline__ void conv_job(const ConvJob& j, const int* slots, int
     if (conv_job_whole(j)) {
         const float4* src = reinterpret_cast<const float4*>(x + (size_t)(j.L - j.P) * j.C);
         const int n4 = j.P * (j.C / 4);
+        const int e1 = e0 * 4 * threads + (int)threadIdx.x;
+        float4 v[4];      // (requested together: a condition around each would make four trips of them)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int e = (e0 * 4 + i) * threads + (int)threadIdx.x;
-            if (e < n4) reinterpret_cast<float4*>(s)[e] = src[e];
-        }
+        for (int i = 0; i < 4; ++i) v[i] = ldg_f4(reinterpret_cast<const float*>(src + (e1 + i * threads < n4 ? e1 + i * threads : n4 - 1)));
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            if (e1 + i * threads < n4) reinterpret_cast<float4*>(s)[e1 + i * threads] = v[i];
         return;
     }
     const int c = e0 * threads + (int)threadIdx.x;
     if (c >= j.C) return;
-    for (int i = 0; i < j.P; ++i) {
-        const int e = j.L + i;
-        s[(size_t)i * j.C + c] = e < j.P ? s[(size_t)e * j.C + c] : x[(size_t)(e - j.P) * j.C + c];
+    for (int i0 = 0; i0 < j.P; i0 += 8) {      // (rows are read ahead of where they are written: L > 0)
+        float v[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int e = j.L + (i0 + i < j.P ? i0 + i : j.P - 1);
+            v[i] = ldg(e < j.P ? s + (size_t)e * j.C + c : x + (size_t)(e - j.P) * j.C + c);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            if (i0 + i < j.P) s[(size_t)(i0 + i) * j.C + c] = v[i];
     }
 }
 static int conv_job_blocks(const ConvJob& j, int threads) { return j.state ? j.n * conv_job_per(j, threads) : 0; }
@@ -389,6 +399,8 @@ __global__ __launch_bounds__(256) void k_conv_jobs(ConvJob a, ConvJob b, int na,
 }
 struct ConvDmaArgs : ConvGemmArgs {
     int tm, tn, tiles8, mfast;      // tiles along M and N; their number rounded up to 8; 1: the blocks of an XCD walk the rows first
+    int tdiv;              // tiles of the direction walked first, and div_inverse of it
+    unsigned tdiv_inv;
     const float* rms_x;    // fp32 rows [M, Cin] whose 1 / rms scales the sums of row m (the rows' RMSNorm, its weight already in x), or NULL
     float rms_eps;
     const float* nw;       // out2 <- terms of v * nw[n] (no activation), or NULL
@@ -423,11 +435,14 @@ __device__ __forceinline__ void conv_put_terms(bf16_t* row, int width, int c, co
 #define CONV_SINE 4        // 0, with snake_exact for SnakeBeta
 // The epilogue of W neighbouring channels (n ..) of MT rows (m, m + 16, ..) that one lane holds: constants once, every row's residual
 // requested ahead of the first store, 16-byte accesses throughout.
-template <int T, int EPI, int W, int MT>
-__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n,
-                                             const f32x4* res_ready = nullptr) {
-    if (n >= a.N) return;          // (N and the group width are multiples of W)
+template <int W, int MT>
+struct conv_consts {
     float b[W], s[W], al[W], ib[W], nw[W], rs[MT][W];
+    int cj, cc;      // (a transposed conv's N = r * sn_mod outputs: r consumer rows)
+};
+template <int W, int MT>
+__device__ __forceinline__ void conv_fetch(conv_consts<W, MT>& k, const ConvDmaArgs& a, int m, int n, const f32x4* res_ready = nullptr) {
+    if (n >= a.N) return;
     const auto fetch = [](float (&d)[W], const float* p) {
 #pragma unroll
         for (int q = 0; q < W / 4; ++q) {
@@ -436,20 +451,26 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
             for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
         }
     };
-    const int cj = a.out2 ? n / a.sn_mod : 0, cc = n - cj * a.sn_mod;      // (a transposed conv's N = r * sn_mod outputs: r consumer rows)
-    if (a.bias) fetch(b, a.bias + n % a.bias_mod);
-    if (a.scale) fetch(s, a.scale + n);
-    if (a.sn_alpha) { fetch(al, a.sn_alpha + cc); fetch(ib, a.sn_invb + cc); }
-    if (a.nw) fetch(nw, a.nw + n);
+    k.cj = a.out2 ? (a.sn_mod >= a.N ? 0 : n / a.sn_mod) : 0;
+    k.cc = n - k.cj * a.sn_mod;
+    if (a.bias) fetch(k.b, a.bias + (a.bias_mod >= a.N ? n : n % a.bias_mod));
+    if (a.scale) fetch(k.s, a.scale + n);
+    if (a.sn_alpha) { fetch(k.al, a.sn_alpha + k.cc); fetch(k.ib, a.sn_invb + k.cc); }
+    if (a.nw) fetch(k.nw, a.nw + n);
     if (res_ready) {
 #pragma unroll
         for (int i = 0; i < MT; ++i)
 #pragma unroll
-            for (int e = 0; e < W; ++e) rs[i][e] = res_ready[i * (W / 4) + e / 4][e % 4];
+            for (int e = 0; e < W; ++e) k.rs[i][e] = res_ready[i * (W / 4) + e / 4][e % 4];
     } else if (a.res)
 #pragma unroll
-        for (int i = 0; i < MT; ++i)
-            if (m + 16 * i < a.M) fetch(rs[i], a.res + (size_t)(m + 16 * i) * a.N + n);
+        for (int i = 0; i < MT; ++i) fetch(k.rs[i], a.res + (size_t)(m + 16 * i < a.M ? m + 16 * i : a.M - 1) * a.N + n);
+}
+template <int T, int EPI, int W, int MT>
+__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n, const conv_consts<W, MT>& k) {
+    if (n >= a.N) return;          // (N and the group width are multiples of W)
+    const float (&b)[W] = k.b, (&s)[W] = k.s, (&al)[W] = k.al, (&ib)[W] = k.ib, (&nw)[W] = k.nw, (&rs)[MT][W] = k.rs;
+    const int cj = k.cj, cc = k.cc;
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const size_t o = (size_t)(m + 16 * i) * a.N + n;
@@ -493,6 +514,10 @@ __device__ __forceinline__ void conv_dma_glu(const ConvDmaArgs& a, f32x4 g, f32x
     }
     conv_put_terms<2>(reinterpret_cast<bf16_t*>(a.out2) + (size_t)m * a.N * 2, a.N, n, v);
 }
+// A conv of few rows is one dependent chain, 4 - 6 us of it for 1 - 2 us of bytes, so what stands in front of the first request and behind the
+// last product counts as much as the products: arguments in one trip (touch_args), tile and request numbers by host-made inverses, the
+// slots of all of a wave's rows and the epilogue's constants asked for together and early.  us a launch, one request of 2 frames, before / so:
+// 3072 x 512 (16 x 32 tiles) 6.8 / 5.4, 512 x 1024 5.4 / 4.9; the decoder's 84 launches 665 / 594, of 10 frames 829 / 795.
 template <int BM, int BN, int WM, int WN, int WK, int BK, int S, int NP, int EPI, int WP = 1>
 __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     constexpr int NWV = WM * WN * WK, MT = BM / WM / 16, NT = BN / WN / 16, KS = BK / 32, PPR = BK / 8, KW = WP == 2 ? WK : 1;
@@ -506,15 +531,26 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     extern __shared__ __attribute__((aligned(1024))) char conv_lds[];
     __shared__ float rms_s[BM];
     const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    touch_args(a);
     if ((int)blockIdx.x >= a.tiles8) {
         conv_job(a.job, a.slots, (int)blockIdx.x - a.tiles8, 64 * NWV);
         return;
     }
     const int t = ((int)blockIdx.x & 7) * (a.tiles8 >> 3) + ((int)blockIdx.x >> 3);
     if (t >= a.tm * a.tn) return;
-    const int m0 = (a.mfast ? t % a.tm : t / a.tn) * BM, n0 = (a.mfast ? t / a.tm : t % a.tn) * BN;      // (glu: n0 counts gate and up columns)
+    const int tq = a.tdiv_inv ? (int)__umulhi((unsigned)t, a.tdiv_inv) : a.tdiv == 1 ? t : t / a.tdiv, tr = t - tq * a.tdiv;
+    const int m0 = (a.mfast ? tr : tq) * BM, n0 = (a.mfast ? tq : tr) * BN;      // (glu: n0 counts gate and up columns)
     const int wk = wv / NC, wmn = wv % NC, wm = wmn / WN, wn = wmn % WN, fr = lane & 15, fk = lane >> 4, lw = NLD < NWV ? wv - NC : wv;
     const bool loads = NLD == NWV || lw >= 0, multiplies = NLD == NWV || lw < 0;
+    const int rl = wm * MT * 16 + fr, nl = n0 + wn * NT * 16;
+    // Waves that only multiply have nothing in flight: they ask for the epilogue's constants and residual now, not in a trip of their own behind the last step
+    constexpr int P = PAIR ? 2 : 1;
+    constexpr bool EARLY = NLD < NWV && EPI != CONV_GLU;
+    conv_consts<4 * P, MT> kc[EARLY ? NT / P : 1];
+    if constexpr (EARLY)
+        if (multiplies)
+#pragma unroll
+            for (int j = 0; j < NT; j += P) conv_fetch(kc[j / P], a, m0 + rl, nl + j * 16 + fk * 4 * P);
     const int rb = a.Cin * (NP == 3 ? 6 : 4);
     // The weights are the first operand of the MFMA: a lane's four sums are neighbouring channels of one row.  PAIR: tiles j and j + 1 take the
     // weight rows 8 q + 0..3 and 8 q + 4..7 (q = 0..3), so that they hold eight neighbouring channels together.
@@ -528,17 +564,23 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
     bool half_a = false, half_b[EPI == CONV_CHUNKS ? NB : 1];      // (the lane's piece is of the step's second slice)
     static_assert(EPI != CONV_CHUNKS || BK == 64, "two slices a step");
     if (loads) {
+        int slot[NA];      // (asked for together, in front of everything else)
+#pragma unroll
+        for (int i = 0; i < NA; ++i) {
+            int m = m0 + ((i * NLD + lw) % CA * 64 + lane) / PPR % BM;
+            m = m < a.M ? m : a.M - 1;                  // (rows past the end repeat the last one: nothing of them is stored)
+            const int b = a.len_inv ? (int)__umulhi((unsigned)m, a.len_inv) : a.L == 1 ? m : m / a.L;
+            ts[i] = m - b * a.L;
+            slot[i] = ldg(a.state ? a.slots + b : reinterpret_cast<const int*>(g_conv_zero_row));
+        }
 #pragma unroll
         for (int i = 0; i < NA; ++i) {
             const int q = (i * NLD + lw) % CA * 64 + lane, pl = q / (BM * PPR), r = q / PPR % BM, pc8 = (q % PPR) ^ (BK == 32 ? (r >> 1) & 3 : r & 7);
             const int pc = EPI == CONV_CHUNKS ? pc8 & 3 : pc8;
             if (EPI == CONV_CHUNKS) half_a = pc8 > 3;      // (the same for every i: whole rows of eight pieces apart)
-            int m = m0 + r;
-            m = m < a.M ? m : a.M - 1;                  // (rows past the end repeat the last one: nothing of them is stored)
-            const int b = m / a.L;
-            ts[i] = m - b * a.L;
+            const int m = m0 + r < a.M ? m0 + r : a.M - 1;
             xp[i] = reinterpret_cast<const char*>(a.x) + (size_t)m * rb + pl * a.Cin * 2 + pc * 16;
-            sp[i] = a.state ? reinterpret_cast<const char*>(a.state) + ((size_t)a.slots[b] * a.P + a.P + ts[i]) * rb + pl * a.Cin * 2 + pc * 16 : nullptr;
+            sp[i] = reinterpret_cast<const char*>(a.state) + ((size_t)slot[i] * a.P + a.P + ts[i]) * rb + pl * a.Cin * 2 + pc * 16;      // (read where there is a state)
         }
 #pragma unroll
         for (int i = 0; i < NB; ++i) {
@@ -617,14 +659,19 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
 #pragma unroll
         for (int s = 0; s < S - 1; ++s) request(s);
     }
-    if (a.rms_x) {
-        for (int r = wv; r < BM; r += NWV) {
-            const int m = m0 + r < a.M ? m0 + r : a.M - 1;
-            const float4* x4 = reinterpret_cast<const float4*>(a.rms_x + (size_t)m * a.Cin);
+    if (EPI != CONV_CHUNKS && a.rms_x) {      // (CONV_CHUNKS has no such rows)
+        for (int r = wv; r < BM && m0 + r < a.M; r += NWV) {
+            const float* x = a.rms_x + (size_t)(m0 + r) * a.Cin;
             float s = 0.0f;
-            for (int c = lane; c < a.Cin / 4; c += 64) {
-                const float4 v = x4[c];
-                s += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+            for (int c0 = lane * 4; c0 < a.Cin; c0 += 1024) {      // (four requests together; what is past the end adds nothing)
+                float4 v[4];
+#pragma unroll
+                for (int k = 0; k < 4; ++k) v[k] = ldg_f4(x + (c0 + k * 256 < a.Cin ? c0 + k * 256 : c0));
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    const float q = v[k].x * v[k].x + v[k].y * v[k].y + v[k].z * v[k].z + v[k].w * v[k].w;
+                    s += c0 + k * 256 < a.Cin ? q : 0.0f;
+                }
             }
             for (int o = 32; o >= 1; o >>= 1) s += __shfl_xor(s, o, 64);
             if (lane == 0) rms_s[r] = rsqrtf(s / (float)a.Cin + a.rms_eps);
@@ -716,14 +763,12 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
         for (int k = 1; k < KW; ++k) v += part[(k * FR + f) * 64];
         return v;
     };
-    const int rl = wm * MT * 16 + fr, nl = n0 + wn * NT * 16;
     if constexpr (EPI == CONV_GLU) {
 #pragma unroll
         for (int f = 0; f < FR; f += 2)
             if (KW == 1 || (f / 2) % KW == wk)
                 conv_dma_glu(a, sum(f), sum(f + 1), rms_s[rl + f / NT * 16], m0 + rl + f / NT * 16, (nl >> 1) + f % NT * 8 + fk * 4);
     } else {
-        constexpr int P = PAIR ? 2 : 1;
         const float* rms = a.rms_x ? rms_s + rl : nullptr;
 #pragma unroll
         for (int j = 0; j < NT; j += P) {
@@ -734,7 +779,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
                     for (int q = 0; q < P; ++q) v[i][q] = acc[i][j + q];
-                conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, MT>(a, v, rms, m0 + rl, n);
+                if constexpr (!EARLY) conv_fetch(kc[0], a, m0 + rl, n);
+                conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, MT>(a, v, rms, m0 + rl, n, kc[EARLY ? j / P : 0]);
             } else {
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
@@ -742,7 +788,9 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                         f32x4 v[1][P];
 #pragma unroll
                         for (int q = 0; q < P; ++q) v[0][q] = sum(i * NT + j + q);
-                        conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
+                        conv_consts<4 * P, 1> k1;
+                        conv_fetch(k1, a, m0 + rl + i * 16, n);
+                        conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n, k1);
                     }
             }
         }
@@ -761,6 +809,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
 // timed alone: 326 with the residual asked for in the epilogue, 311 - 332 with four stages or 64-row blocks.)
 template <int C, int CH, int TAPS, int T, int HP, int NW, int MT, int S>
 __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_conv_unit(ConvDmaArgs a1, ConvDmaArgs a2, int H) {
+    touch_args(a1);
+    touch_args(a2);
     constexpr int BM = 16 * MT * NW, R = BM + HP, NT = CH / 16, NP = CH / 32, NT2 = C / 16, NCK = C / 32;
     constexpr int SA = T * R * 64, CA = SA / 1024, NA = (CA + NW - 1) / NW, CW1 = CH / 16, CW2 = C / 16, SW = (C > CH ? C : CH) * 64;
     constexpr int NB = ((C > CH ? CW2 : CW1) + NW - 1) / NW;       // requests of a wave per slice (the smaller kind repeats some)
@@ -948,7 +998,9 @@ __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_co
         f32x4 v[MT][2];
 #pragma unroll
         for (int i = 0; i < MT; ++i) { v[i][0] = out[i][2 * p]; v[i][1] = out[i][2 * p + 1]; }
-        conv_dma_out<T, 0, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
+        conv_consts<8, MT> k;
+        conv_fetch(k, a2, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
+        conv_dma_out<T, 0, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, k);
     }
 }
 
@@ -957,6 +1009,7 @@ __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_co
 // register prefetch.  These stages run a handful of blocks: time = number of dependent K steps, so the steps are wide.
 template <int BK, bool LN = false>
 __global__ __launch_bounds__(256) void k_conv_gemm_skinny(ConvGemmArgs a) {
+    touch_args(a);
     constexpr int LD = BK + 8;                      // bf16 elements
     constexpr int NA = (16 * BK / 4 + 255) / 256;   // float4 per thread (activations)
     constexpr int NB = 64 * BK / 8 / 256;           // uint4 per thread (weights)
@@ -1086,6 +1139,7 @@ __global__ __launch_bounds__(256) void k_conv_gemm_skinny(ConvGemmArgs a) {
 // alone (8 waves from K = 512 on: half the serial work per wave), so a request's output does not depend on what shares its batch.
 template <int KB, int NT, bool LN, int MT, int WV>
 __global__ __launch_bounds__(64 * WV) void k_rows_gemm(ConvGemmArgs a) {
+    touch_args(a);
     __shared__ float red[WV][MT * NT][256];
     __shared__ float ln_stat[LN ? 2 * WV * 16 * MT : 1];
     // (the wave index provably uniform: the tap of a k-block, and with it a.off[tap], is then a scalar — read per lane from the argument
@@ -1886,6 +1940,8 @@ static int conv_dma_launch(hipStream_t st, ConvDmaArgs& a) {
     a.tn = ((EPI == CONV_GLU ? 2 * a.N : a.N) + BN - 1) / BN;
     a.tiles8 = (a.tm * a.tn + 7) & ~7;
     a.mfast = (size_t)a.n_taps * a.N > (size_t)a.M * 2;      // weights larger than rows: each XCD reads its own columns of them
+    a.tdiv = a.mfast ? a.tm : a.tn;
+    a.tdiv_inv = div_inverse(a.tdiv, a.tiles8);
     hipLaunchKernelGGL(kern, dim3(a.tiles8 + conv_job_blocks(a.job, threads)), dim3(threads), lds, st, a);
     return VOX_OK;
 }
@@ -1998,6 +2054,7 @@ static int conv_s2(hipStream_t st, ConvDmaArgs& a, int epi = 0) {
     if (a.n_taps > CG_MAXTAPS) return vox_fail(VOX_ERR_INVALID, "codec conv: too many taps");
     if (a.N % 16 || a.sn_mod % 8 || a.bias_mod % 8) return vox_fail(VOX_ERR_INVALID, "codec conv: %d channels (groups of %d)", a.N, a.sn_mod);
     a.planes = g_conv_planes;
+    a.len_inv = div_inverse(a.L, a.M);
     if (epi == CONV_GLU) {
         a.N /= 2;
         a.sn_mod = a.N;
@@ -3748,6 +3805,7 @@ __device__ __forceinline__ int flow_cache_row(int j, int prefix, int head, int c
 }
 #define FLOW_MAXKEYS 1024
 __global__ __launch_bounds__(256) void k_flow_attn(FlowAttn a) {
+    touch_args(a);
     __shared__ float ps[4][FLOW_MAXKEYS];
     __shared__ __attribute__((aligned(16))) float qs[4][2][128];
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
