@@ -359,6 +359,7 @@ __global__ __launch_bounds__(256) void k_linear(LinArgs a) {
 // bit for bit, as k_linear.
 template <int BT, int KC, int R, int PRO, int EPI>
 __global__ __launch_bounds__(256) void k_gemv(LinArgs a) {
+    touch_args(a);
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     constexpr int OUT = (EPI == EPI_SILU_MUL) ? R / 2 : R;
     // 3..8 rows: the same kernel per row tile.  Block id = (x / 8) * 8T + tile * 8 + x % 8: the T blocks that stream the same
@@ -634,6 +635,7 @@ __device__ __forceinline__ bf16x8_t as_bf8(uint4 v) {
 template <int B_> struct vox_ic { static constexpr int value = B_; };
 template <int MT, int PRO, int EPI, bool FULL, int KSEG, int DEPTH = 1>
 __global__ __launch_bounds__(256) void k_linear_mfma(LinArgs a) {
+    touch_args(a);
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int BT = 16 * MT;
     constexpr int LDK = KSEG + 8;                  // padded row stride (elements)
@@ -1005,6 +1007,7 @@ __global__ __launch_bounds__(256) void k_linear_mfma_small(LinArgs a) {
 
 template <int EPI>
 __global__ __launch_bounds__(256) void k_linear_mfma_stream(LinArgs a) {
+    touch_args(a);
     constexpr int H = 4, NBUF = 4;
     static_assert(EPI == EPI_STORE || EPI == EPI_SILU, "copy prologue, plain epilogues");
     __shared__ f32x4_t red[3][64];
@@ -1324,6 +1327,7 @@ static int launch_gemm_splitk(hipStream_t st, const LinArgs& a, float* ws, size_
 // epilogue.  Every output keeps its K split and summation order, so the results are bit-identical to CT = 1.
 template <int MT, int KSTEPS, int PRO, int EPI, bool ROWSPLIT, int CT = 1>
 __global__ __launch_bounds__(512) void k_gemm_fullk(LinArgs a) {
+    touch_args(a);
     static_assert(CT == 1 || (EPI == EPI_SILU_MUL && !ROWSPLIT), "two column tiles per block: the SiLU*up form only");
     constexpr bool SM = (EPI == EPI_SILU_MUL);
     constexpr int NB = SM ? 2 : 1;
@@ -1531,6 +1535,7 @@ __global__ __launch_bounds__(512) void k_gemm_fullk(LinArgs a) {
 // ================================================================================================
 template <int KSTEPS, int EPI, int ROWS>
 __global__ __launch_bounds__(512) void k_gemm_tiles(LinArgs a) {
+    touch_args(a);
     constexpr bool SM = EPI == EPI_SILU_MUL;
     constexpr int NB = SM ? 2 : 1, NCH = KSTEPS * 32;      // 16-byte pieces of a row
     extern __shared__ __attribute__((aligned(16))) char tiles_smem[];
@@ -1693,6 +1698,7 @@ __global__ __launch_bounds__(512) void k_gemm_tiles(LinArgs a) {
 // ================================================================================================
 template <int MT, int NT, int EPI, int S>
 __global__ __launch_bounds__(512) void k_gemm_rows(LinArgs a) {
+    touch_args(a);
     constexpr bool SM = (EPI == EPI_SILU_MUL);
     constexpr int NB = SM ? 2 : 1, NW = NB * NT, STAGE = (NW + MT) * 1024;
     extern __shared__ __attribute__((aligned(1024))) char rows_lds[];
@@ -1818,6 +1824,7 @@ __global__ __launch_bounds__(512) void k_gemm_rows(LinArgs a) {
 // (range, sequence), which keep their KS chunks for the product.  y: fragment-major (rows rounded up to 16).
 template <int KS>
 __global__ __launch_bounds__(256) void k_norm_rows(LinArgs a, bf16_t* y) {
+    touch_args(a);
     const int lane = threadIdx.x & 31, row = blockIdx.x * 8 + (threadIdx.x >> 5);
     const int r = row < a.B ? row : a.B - 1;
     const uint4 *x = x_row_ptr(a, r) + (lane >> 2) * (KS * 4) + (lane & 3), *w = reinterpret_cast<const uint4*>(a.nw) + (lane >> 2) * (KS * 4) + (lane & 3);
@@ -2237,6 +2244,7 @@ struct HeadArgs {
 };
 
 __global__ __launch_bounds__(64) void k_head_prepare(HeadArgs a) {
+    touch_args(a);
     __shared__ float sh[512];
     __shared__ __attribute__((aligned(16))) bf16_t so[512];
     const int head = blockIdx.x, n = blockIdx.y, lane = threadIdx.x;
@@ -2461,6 +2469,7 @@ __device__ __forceinline__ void prep_head(const bf16_t* src, const bf16_t* nw, f
 
 template <int D, bool FUSED>
 __global__ __launch_bounds__(256) void k_attn_partial(AttnArgs a) {
+    touch_args(a);
     constexpr int LPT = D / 8;        // lanes per token
     constexpr int TPW = 64 / LPT;     // tokens per wave pass
     constexpr int GMAX = 16;
@@ -2728,6 +2737,7 @@ _Pragma("unroll") \
 // (An earlier one-launch variant gave each chunk ONE wave and lost: a 32-token chunk is too long a serial chain for a wave.)
 template <int D, int GMAX, int NG, int NCH = 8>
 __global__ __launch_bounds__(1024) void k_attn_decode8(AttnArgs a) {
+    touch_args(a);
     // NCH = 16 (CPG = 2 chunks per group): contexts of up to 512 tokens — the second chunk's tile is requested when the first one has been
     // parked, so its HBM latency runs under the first chunk's scores / softmax / P.V (one tile's registers at a time)
     constexpr int LPT = D / 8, TPW = 64 / LPT, GT = 1024 / NG, GW = GT / 64, CPG = NCH / NG;
@@ -3462,6 +3472,7 @@ __device__ __forceinline__ void attn_short_wave(const AttnArgs& at, int row, int
 // head's cached K / V itself (L2 hits), the first one appends the new token.
 template <int NT>
 __global__ __launch_bounds__(256) void k_attn_short(AttnArgs at, int n_pairs) {
+    touch_args(at);
     VOX_TR_DECL
     const int pi = blockIdx.x * 4 + (threadIdx.x >> 6);
     if (pi >= n_pairs) return;

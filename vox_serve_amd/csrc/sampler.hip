@@ -95,6 +95,7 @@ __device__ __forceinline__ void preprocess_part(const SampArgs& a, bf16_t* lg, i
 __device__ __forceinline__ void preprocess_row(const SampArgs& a, bf16_t* lg, int b, int tid, int nthr) { preprocess_part(a, lg, b, 0, a.V, tid, nthr); }
 
 __global__ __launch_bounds__(256) void k_sample(SampArgs a) {
+    touch_args(a);
     extern __shared__ __attribute__((aligned(16))) char smem[];
     __shared__ unsigned long long red[4];
     __shared__ int hist[256];
@@ -285,6 +286,7 @@ __global__ __launch_bounds__(256) void k_sample(SampArgs a) {
 // per frame, 23 -> ~8 us each.
 template <int EPT>
 __global__ __launch_bounds__(256) void k_sample_topk(SampArgs a) {
+    touch_args(a);
     __shared__ int wsum[2][4];
     __shared__ int sh_i[8];
     __shared__ u32 cand_key[SAMP_KMAX], srt_key[SAMP_KMAX];
@@ -615,6 +617,7 @@ __global__ __launch_bounds__(512) void k_bucket_coarse(SampArgs a) {
 // PARTS: keys, histogram and coarse masses have been left by the two launches above
 template <bool PARTS>
 __global__ __launch_bounds__(1024) void k_sample_bucket(SampArgs a) {
+    touch_args(a);
     __shared__ u32 tile[PARTS ? 1 : 256][33];      // the coarse pass's staging tile
     __shared__ BKShared S;
     __shared__ u32 wred[16];
