@@ -740,8 +740,21 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_hb_gemm_dma(const bf16_t* A
 #pragma unroll
     for (int s = 0; s < S; ++s) request(s, s * BK < klast ? s * BK : klast);
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * (NA + NW)) : "memory");
-    read(smem, p0, a0, w0);
     int stage = 0;
+    // A wave whose rows all lie past the end (the last rows of an expert's list fill a tenth of a 256-row tile as often as all of it) only
+    // loads: its share of the matrix cores goes to the wave beside it on the SIMD, whose rows lie 128 further up.  A prefill of 2048 tokens over eight
+    // experts, 4214 -> 4177 us.
+    if (m0 + wm * MT * 16 >= M) {
+        for (int kt = 0; kt < nt; ++kt) {
+            asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
+            const int kn = (kt + S) * BK;
+            request(stage, kn < klast ? kn : klast);
+            stage = stage == S - 1 ? 0 : stage + 1;
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        return;
+    }
+    read(smem, p0, a0, w0);
     for (int kt = 0; kt < nt; ++kt) {
         __builtin_amdgcn_sched_barrier(0);
         read(smem + stage * STAGE, p1, a1, w1);
