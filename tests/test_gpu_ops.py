@@ -493,6 +493,42 @@ def test_stack_forward_small_batches_both_settings(dev, n_rows):
         N.set_exact_rows(2)
 
 
+@pytest.mark.parametrize("n_rows,heads,kvh", [(3, 4, 2), (12, 8, 2), (128, 8, 4), (129, 8, 4), (64, 16, 4), (65, 16, 4)])
+def test_short_attention_of_a_fixed_length(dev, n_rows, heads, kvh):
+    """The depth loops' form (identity pages, length and position known when launched) against the one that reads the plan: the same hidden
+    states and the same new K/V, bit for bit.  Up to 512 (row, pair of heads) products four waves share one, above that a wave has each."""
+    import ctypes
+    from vox_serve_amd import _native as N
+    from vox_serve_amd.engine import StackCfg, _stack_config, rope_table
+    L, ctx = N.lib(), N.ctx()
+    H, F, D, page = 256, 256, 128, 16
+    rng = np.random.default_rng(n_rows)
+    w = lambda *s_, sd=0.05: T(vr.f2bf(rng.standard_normal(s_, dtype=np.float32) * np.float32(sd)), dev)
+    ec = StackCfg(H, 1, heads, kvh, D, F, 1e-6, 1e6, 1.0, None, False, None, True, False)
+    ts = dict(wqkv=w((heads + 2 * kvh) * D, H), wo=w(H, heads * D), wgate=w(F, H), wup=w(F, H), wdown=w(H, F), ln1=1 + w(H), ln2=1 + w(H), qnorm=1 + w(D), knorm=1 + w(D))
+    arr = (N.LayerWeights * 1)()
+    for k, v in ts.items():
+        setattr(arr[0], k, v.data_ptr())
+    fn, rope = 1 + w(H), rope_table(64, ec, dev)
+    sc = _stack_config(ec, page, 144, page)
+    h = ctypes.c_void_p()
+    N.check(L.vox_stack_create(ctx, ctypes.byref(sc), arr, fn.data_ptr(), rope.data_ptr(), 64, ctypes.byref(h)))
+    i32 = lambda v: torch.tensor(v, dtype=torch.int32, device=dev)
+    ids = list(range(n_rows))
+    for nt in (2, 5, 8, 9, 15, 16):
+        x, kv0 = w(n_rows, H, sd=1.0), w(1, n_rows, 2, page, kvh, D, sd=0.5)
+        tens = [i32(v) for v in ([nt - 1] * n_rows, ids, [nt] * n_rows, ids, [nt - 1] * n_rows, ids + [n_rows], ids)]
+        ptab, out = i32([[r] for r in ids]), []
+        for fixed in (False, True):
+            kv, xi, y = kv0.clone(), x.clone(), torch.empty(n_rows, H, dtype=torch.bfloat16, device=dev)
+            rows = N.Rows(*[t.data_ptr() for t in tens], n_rows, nt, ptab.data_ptr(), 1, nt if fixed else 0, nt - 1 if fixed else -1, int(fixed))
+            N.check(L.vox_stack_forward(h, N.stream(), xi.data_ptr(), y.data_ptr(), kv.data_ptr(), kv[0].numel(), ctypes.byref(rows)))
+            torch.cuda.synchronize()
+            out.append((Bits(y), Bits(kv)))
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1]), nt
+    L.vox_stack_destroy(h)
+
+
 @pytest.mark.parametrize("n_rows", [12, 32])
 def test_stack_forward_batched_rows_k4096(dev, n_rows):
     """The same three attention routes at GLM-4-Voice width (hidden 4096 = 16 k-steps per wave): copy-prologue linears on the

@@ -3329,22 +3329,14 @@ __device__ __forceinline__ void attn_short_prefetch(const AttnArgs& at, int row,
     }
 }
 
-// v: this lane's 16-byte chunk of its group's head row (grp 0 / 1: the two q heads, 2: the new k, 3: the new v);
-// vnew: the new token's V row in the P.V layout (dims 4 dq .. 4 dq + 3).
-template <int NT>
-__device__ __forceinline__ void attn_short_compute(const AttnArgs& at, int row, int hk, int lane, const uint4 v, const uint2 vnew,
-                                                   const AttnShortPre<NT>& pf, bf16_t* out_row, bool do_append, int hq0 = -1) {
-    if (hq0 < 0) hq0 = hk * 2;           // the wave's two q heads: hq0, hq0 + 1 (two q heads per kv head: 2 hk; four: 4 hk + 2 pair)
-    constexpr int D = 128, TMAX = AttnShortPre<NT>::TMAX, UMAX = AttnShortPre<NT>::UMAX;
-    const int grp = lane >> 4, j = lane & 15;
-    const int g = lane >> 5, dq = lane & 31;      // P.V / output layout: lane = (q head g, dims 4 dq .. 4 dq + 3)
-    const size_t ps = (size_t)2 * at.page_size * at.Hkv * D;
-    const int L = pf.L, nt = pf.nt;
+// v: this lane's 16-byte chunk of its group's head row (grp 0 / 1: the two q heads, 2: the new k, 3: the new v), normed (where its head has
+// a norm) and rotated; v itself in grp 3.
+__device__ __forceinline__ uint4 attn_short_head(const AttnArgs& at, int grp, int j, const uint4 v, const uint4 gw4, const float4 (&cs4)[4]) {
+    constexpr int D = 128;
     // (two uniform conditions selected by lane group: a lane-indexed select of the two POINTERS goes through a scratch array, and
     // the wait behind that scratch load waits for every K/V request in flight)
     const bool qn_ok = at.qn != nullptr, kn_ok = at.kn != nullptr;
     const bool has_nw = grp < 2 ? qn_ok : (grp == 2 && kn_ok);
-    const uint4 gw4 = pf.gw4;
     // per-head RMSNorm (prep_head: butterfly<64> over a head's 16 non-zero lanes == butterfly<16>)
     float e[8] = {bflo(v.x), bfhi(v.x), bflo(v.y), bfhi(v.y), bflo(v.z), bfhi(v.z), bflo(v.w), bfhi(v.w)};
     {
@@ -3359,24 +3351,33 @@ __device__ __forceinline__ void attn_short_compute(const AttnArgs& at, int row, 
     }
     // NeoX RoPE over the full head: element i < 64 pairs with i + 64, i.e. with the same slot of lane ^ 8 (a rotation by 8 inside
     // the 16-lane row: one DPP move)
-    uint4 hq;
-    {
-        const float cc[8] = {pf.cs4[0].x, pf.cs4[0].z, pf.cs4[1].x, pf.cs4[1].z, pf.cs4[2].x, pf.cs4[2].z, pf.cs4[3].x, pf.cs4[3].z};
-        const float sn[8] = {pf.cs4[0].y, pf.cs4[0].w, pf.cs4[1].y, pf.cs4[1].w, pf.cs4[2].y, pf.cs4[2].w, pf.cs4[3].y, pf.cs4[3].w};
-        float r[8];
+    const float cc[8] = {cs4[0].x, cs4[0].z, cs4[1].x, cs4[1].z, cs4[2].x, cs4[2].z, cs4[3].x, cs4[3].z};
+    const float sn[8] = {cs4[0].y, cs4[0].w, cs4[1].y, cs4[1].w, cs4[2].y, cs4[2].w, cs4[3].y, cs4[3].w};
+    float r[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
+    for (int i = 0; i < 8; ++i) {
 #if VOX_DPP_BUTTERFLY
-            const float o = vox_dpp<0x128, 0xF>(e[i], e[i]);        // row_ror:8
+        const float o = vox_dpp<0x128, 0xF>(e[i], e[i]);        // row_ror:8
 #else
-            const float o = __shfl_xor(e[i], 8, VOX_WAVE);
+        const float o = __shfl_xor(e[i], 8, VOX_WAVE);
 #endif
-            const float mc = e[i] * cc[i];
-            r[i] = (j < 8) ? __fmaf_rn(-o, sn[i], mc) : __fmaf_rn(o, sn[i], mc);
-        }
-        hq.x = pack_bf2(r[0], r[1]); hq.y = pack_bf2(r[2], r[3]); hq.z = pack_bf2(r[4], r[5]); hq.w = pack_bf2(r[6], r[7]);
-        if (grp == 3) hq = v;
+        const float mc = e[i] * cc[i];
+        r[i] = (j < 8) ? __fmaf_rn(-o, sn[i], mc) : __fmaf_rn(o, sn[i], mc);
     }
+    if (grp == 3) return v;
+    return make_uint4(pack_bf2(r[0], r[1]), pack_bf2(r[2], r[3]), pack_bf2(r[4], r[5]), pack_bf2(r[6], r[7]));
+}
+// vnew: the new token's V row in the P.V layout (dims 4 dq .. 4 dq + 3).
+template <int NT>
+__device__ __forceinline__ void attn_short_compute(const AttnArgs& at, int row, int hk, int lane, const uint4 v, const uint2 vnew,
+                                                   const AttnShortPre<NT>& pf, bf16_t* out_row, bool do_append, int hq0 = -1) {
+    if (hq0 < 0) hq0 = hk * 2;           // the wave's two q heads: hq0, hq0 + 1 (two q heads per kv head: 2 hk; four: 4 hk + 2 pair)
+    constexpr int D = 128, TMAX = AttnShortPre<NT>::TMAX, UMAX = AttnShortPre<NT>::UMAX;
+    const int grp = lane >> 4, j = lane & 15;
+    const int g = lane >> 5, dq = lane & 31;      // P.V / output layout: lane = (q head g, dims 4 dq .. 4 dq + 3)
+    const size_t ps = (size_t)2 * at.page_size * at.Hkv * D;
+    const int L = pf.L, nt = pf.nt;
+    const uint4 hq = attn_short_head(at, grp, j, v, pf.gw4, pf.cs4);
     const uint4 q0c = shfl4(hq, j), q1c = shfl4(hq, 16 + j), knc = shfl4(hq, 32 + j);
     if (do_append) {
         const int pg = (NT > 0 || at.identity_pages) ? row : at.page[row];
@@ -3479,6 +3480,96 @@ __global__ __launch_bounds__(256) void k_attn_short(AttnArgs at, int n_pairs) {
     const int PP = at.Hq / (2 * at.Hkv), per_row = at.Hkv * PP;
     const int row = pi / per_row, rem = pi - row * per_row, hk = rem / PP, pp = rem - hk * PP;
     attn_short_wave<NT>(at, row, hk, threadIdx.x & 63, at.out + (size_t)row * at.Hq * 128, pp == 0, hk * 2 * PP + 2 * pp);
+    VOX_TR_END(2, NT)
+}
+
+// Few pairs (two blocks a CU at most): four waves share one.  A wave alone on its SIMD issues an instruction every four cycles at best, and a pair
+// of 32 tokens is 1415 of them; here each wave norms and rotates the heads for itself, takes every fourth group of four tokens' scores, all
+// probabilities (one a lane) and 32 of the 128 output dims: 2 x 32 chains over the tokens, one a lane.  The arithmetic of every score,
+// sum and output is attn_short_compute's chain: the same bits.  One more wait than there (the scores go through LDS).
+// us a launch, one wave a pair / four: 64 pairs of 32 tokens 7.3 / 3.2, of 16 4.9 / 3.2; 256 pairs of 16 5.3 / 4.0, of 8 4.8 / 3.9.
+// Beyond two blocks a CU the four-fold norm and rotation cost more than the shorter chain gives.  us a Qwen3-TTS frame: 512 pairs 4993 / 4963, 768
+// 6764 / 6773, 1024 7660 / 7693; a CSM frame of 384 pairs 10 150 / 10 025.
+template <int NT>
+__global__ __launch_bounds__(256) void k_attn_short4(AttnArgs at) {
+    touch_args(at);
+    VOX_TR_DECL
+    constexpr int D = 128, UMAX = (NT + 3) / 4, UW = (UMAX + 3) / 4, NP = (NT + 3) & ~3;
+    __shared__ __attribute__((aligned(16))) float s_sc[2][32], s_p[4][2][32];
+    const int lane = threadIdx.x & 63, w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), grp = lane >> 4, j = lane & 15, g = lane >> 5;
+    const int PP = at.Hq / (2 * at.Hkv), per_row = at.Hkv * PP, pi = blockIdx.x;
+    const int row = pi / per_row, rem = pi - row * per_row, hk = rem / PP, pp = rem - hk * PP, hq0 = hk * 2 * PP + 2 * pp;
+    const bf16_t* raw = at.qkv + (size_t)row * (at.Hq + 2 * at.Hkv) * D;
+    const bf16_t* src = raw + (size_t)(grp < 2 ? hq0 + grp : grp == 2 ? at.Hq + hk : at.Hq + at.Hkv + hk) * D;
+    const size_t ps = (size_t)2 * at.page_size * at.Hkv * D, ts = (size_t)at.Hkv * D;
+    const bf16_t* kb = at.kv + (size_t)row * ps + (size_t)hk * D;
+    const int vd = w * 32 + (lane & 31);
+    const bf16_t* vb = kb + (size_t)at.page_size * at.Hkv * D + vd;
+    // everything is asked for at once (attn_short_prefetch's identity form: page = row, slot = token, position = fixed_pos)
+    const uint4 v = ldg(reinterpret_cast<const uint4*>(src) + j);
+    uint4 gw4 = make_uint4(0, 0, 0, 0);
+    if (at.qn && at.kn) gw4 = ldg(reinterpret_cast<const uint4*>(grp < 2 ? at.qn : at.kn) + j);
+    int p = at.fixed_pos;
+    p = p < 0 ? 0 : (p >= at.table_max_pos ? at.table_max_pos - 1 : p);
+    const float* cp = at.cs + (size_t)p * D + (j & 7) * 16;   // row = D/2 (c,s) pairs
+    const float4 cs4[4] = {ldg_f4(cp), ldg_f4(cp + 4), ldg_f4(cp + 8), ldg_f4(cp + 12)};
+    uint4 kr[UW];
+#pragma unroll
+    for (int i = 0; i < UW; ++i) {
+        const int t = (i * 4 + w) * 4 + grp;      // (past the cached tokens: the last of them, its score is not used)
+        kr[i] = ldg(reinterpret_cast<const uint4*>(kb + (size_t)(t < NT - 1 ? t : NT - 2) * ts) + j);
+    }
+    __builtin_amdgcn_sched_barrier(0);      // (K in front of V: the scores wait for nothing behind them)
+    bf16_t vr[NT];
+#pragma unroll
+    for (int t = 0; t < NT - 1; ++t) vr[t] = *(const VOX_GLOBAL_AS bf16_t*)(vb + (size_t)t * ts);
+    vr[NT - 1] = *(const VOX_GLOBAL_AS bf16_t*)(raw + (size_t)(at.Hq + at.Hkv + hk) * D + vd);
+    const uint4 hq = attn_short_head(at, grp, j, v, gw4, cs4);
+    const uint4 q0c = shfl4(hq, j), q1c = shfl4(hq, 16 + j), knc = shfl4(hq, 32 + j);
+    if (pp == 0 && w == 0 && grp >= 2) {
+        bf16_t* base = at.kv_w + (size_t)row * ps + ((size_t)(NT - 1) * at.Hkv + hk) * D;
+        if (grp == 3) base += (size_t)at.page_size * at.Hkv * D;
+        reinterpret_cast<uint4*>(base)[j] = hq;
+    }
+    const float q0f[8] = {bflo(q0c.x), bfhi(q0c.x), bflo(q0c.y), bfhi(q0c.y), bflo(q0c.z), bfhi(q0c.z), bflo(q0c.w), bfhi(q0c.w)};
+    const float q1f[8] = {bflo(q1c.x), bfhi(q1c.x), bflo(q1c.y), bfhi(q1c.y), bflo(q1c.z), bfhi(q1c.z), bflo(q1c.w), bfhi(q1c.w)};
+#pragma unroll
+    for (int i = 0; i < UW; ++i) {
+        const int t = (i * 4 + w) * 4 + grp;
+        const uint4 kx = t == NT - 1 ? knc : kr[i];
+        const float kf[8] = {bflo(kx.x), bfhi(kx.x), bflo(kx.y), bfhi(kx.y), bflo(kx.z), bfhi(kx.z), bflo(kx.w), bfhi(kx.w)};
+        float d0 = 0.0f, d1 = 0.0f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { d0 = __fmaf_rn(q0f[e], kf[e], d0); d1 = __fmaf_rn(q1f[e], kf[e], d1); }
+        d0 = butterfly<16>(d0) * at.scale;
+        d1 = butterfly<16>(d1) * at.scale;
+        if (j < 2 && t < 32) s_sc[j][t] = t < NT ? (j ? d1 : d0) : -INFINITY;
+    }
+    __syncthreads();
+    // lane (head g, token lane & 31)
+    const float sv = (lane & 31) < NT ? s_sc[g][lane & 31] : -INFINITY;
+    float m = sv;
+#pragma unroll
+    for (int off = 16; off >= 1; off >>= 1) m = fmaxf(m, __shfl_xor(m, off, VOX_WAVE));
+    s_p[w][g][lane & 31] = (lane & 31) < NT ? exp2_c((sv - m) * VOX_LOG2E) : 0.0f;
+    __builtin_amdgcn_wave_barrier();
+    __threadfence_block();
+    float o = 0.0f, l = 0.0f;
+#pragma unroll
+    for (int t0 = 0; t0 < NP; t0 += 4) {
+        const float4 p4 = *reinterpret_cast<const float4*>(&s_p[w][g][t0]);
+        const float pt[4] = {p4.x, p4.y, p4.z, p4.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+            if (t0 + e < NT) {
+                l = l + pt[e];
+                o = __fmaf_rn(pt[e], bf2f(vr[t0 + e < NT ? t0 + e : 0]), o);
+            }
+    }
+    const bf16_t r = f2bf(o / l);
+    const int col = (hq0 + g) * D + vd;
+    at.out[(size_t)row * at.Hq * D + col] = r;
+    if (at.out_frag) at.out_frag[frag_off(row, col, at.Hq * D)] = r;
     VOX_TR_END(2, NT)
 }
 
@@ -5010,6 +5101,7 @@ static void fill_attn_args(AttnArgs& a, const AttnCall& c) {
     a.out = nullptr;
 }
 
+#define ATTN_SHORT4_PAIRS 512      // (row, pair of heads) products up to which four waves share one: two blocks a CU
 // which compile-time token count a short-attention launch may take: NT > 0 assumes identity pages, a fixed position and a page that
 // holds all NT tokens (attn_short_prefetch); anything else reads the plan arrays (NT = 0)
 static inline int attn_short_nt(const AttnArgs& at) {
@@ -5031,7 +5123,10 @@ int vox_launch_attn_short(hipStream_t st, const AttnCall& c) {
     const int n_pairs = c.Nq * c.Hkv * (c.Hq / (2 * c.Hkv));
     // NT > 0 = the depth-loop form: identity pages, fixed position, the page holds every visible token (attn_short_prefetch)
     switch (attn_short_nt(at)) {      // depth loop: the visible length is part of the captured graph
-#define VOX_AS(NT_) case NT_: hipLaunchKernelGGL(k_attn_short<NT_>, dim3((n_pairs + 3) / 4), dim3(256), 0, st, at, n_pairs); return VOX_OK;
+#define VOX_AS(NT_) case NT_: \
+            if (n_pairs <= ATTN_SHORT4_PAIRS) hipLaunchKernelGGL(k_attn_short4<NT_>, dim3(n_pairs), dim3(256), 0, st, at); \
+            else hipLaunchKernelGGL(k_attn_short<NT_>, dim3((n_pairs + 3) / 4), dim3(256), 0, st, at, n_pairs); \
+            return VOX_OK;
         VOX_AS(2) VOX_AS(3) VOX_AS(4) VOX_AS(5) VOX_AS(6) VOX_AS(7) VOX_AS(8) VOX_AS(9) VOX_AS(10) VOX_AS(11) VOX_AS(12)
         VOX_AS(13) VOX_AS(14) VOX_AS(15) VOX_AS(16) VOX_AS(17) VOX_AS(18) VOX_AS(19) VOX_AS(20) VOX_AS(21) VOX_AS(22) VOX_AS(23) VOX_AS(24)
         VOX_AS(25) VOX_AS(26) VOX_AS(27) VOX_AS(28) VOX_AS(29) VOX_AS(30) VOX_AS(31) VOX_AS(32)
