@@ -440,8 +440,10 @@ struct conv_consts {
     float b[W], s[W], al[W], ib[W], nw[W], rs[MT][W];
     int cj, cc;      // (a transposed conv's N = r * sn_mod outputs: r consumer rows)
 };
+// What the epilogue reads, asked for ahead of the K loop.  (Kernels whose waves have no registers for it read it in the epilogue: through this
+// struct the 256 x 192 tile spilled 36 bytes a lane there, 73 -> 82 us at 51 200 rows of 384 channels.)
 template <int W, int MT>
-__device__ __forceinline__ void conv_fetch(conv_consts<W, MT>& k, const ConvDmaArgs& a, int m, int n, const f32x4* res_ready = nullptr) {
+__device__ __forceinline__ void conv_fetch(conv_consts<W, MT>& k, const ConvDmaArgs& a, int m, int n) {
     if (n >= a.N) return;
     const auto fetch = [](float (&d)[W], const float* p) {
 #pragma unroll
@@ -457,20 +459,50 @@ __device__ __forceinline__ void conv_fetch(conv_consts<W, MT>& k, const ConvDmaA
     if (a.scale) fetch(k.s, a.scale + n);
     if (a.sn_alpha) { fetch(k.al, a.sn_alpha + k.cc); fetch(k.ib, a.sn_invb + k.cc); }
     if (a.nw) fetch(k.nw, a.nw + n);
-    if (res_ready) {
-#pragma unroll
-        for (int i = 0; i < MT; ++i)
-#pragma unroll
-            for (int e = 0; e < W; ++e) k.rs[i][e] = res_ready[i * (W / 4) + e / 4][e % 4];
-    } else if (a.res)
+    if (a.res)
 #pragma unroll
         for (int i = 0; i < MT; ++i) fetch(k.rs[i], a.res + (size_t)(m + 16 * i < a.M ? m + 16 * i : a.M - 1) * a.N + n);
 }
-template <int T, int EPI, int W, int MT>
-__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n, const conv_consts<W, MT>& k) {
+template <int T, int EPI, int W, int MT, bool FETCHED = false>
+__device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n,
+                                             const f32x4* res_ready = nullptr, const conv_consts<W, MT>& early = conv_consts<W, MT>{}) {
     if (n >= a.N) return;          // (N and the group width are multiples of W)
-    const float (&b)[W] = k.b, (&s)[W] = k.s, (&al)[W] = k.al, (&ib)[W] = k.ib, (&nw)[W] = k.nw, (&rs)[MT][W] = k.rs;
-    const int cj = k.cj, cc = k.cc;
+    float b[W], s[W], al[W], ib[W], nw[W], rs[MT][W];
+    int cj, cc;      // (a transposed conv's N = r * sn_mod outputs: r consumer rows)
+    if constexpr (FETCHED) {
+        cj = early.cj;
+        cc = early.cc;
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+            b[e] = early.b[e]; s[e] = early.s[e]; al[e] = early.al[e]; ib[e] = early.ib[e]; nw[e] = early.nw[e];
+#pragma unroll
+            for (int i = 0; i < MT; ++i) rs[i][e] = early.rs[i][e];
+        }
+    } else {
+        cj = a.out2 ? n / a.sn_mod : 0;
+        cc = n - cj * a.sn_mod;
+        const auto fetch = [](float (&d)[W], const float* p) {
+#pragma unroll
+            for (int q = 0; q < W / 4; ++q) {
+                const f32x4 t = *reinterpret_cast<const f32x4_a4*>(p + 4 * q);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
+            }
+        };
+        if (a.bias) fetch(b, a.bias + n % a.bias_mod);
+        if (a.scale) fetch(s, a.scale + n);
+        if (a.sn_alpha) { fetch(al, a.sn_alpha + cc); fetch(ib, a.sn_invb + cc); }
+        if (a.nw) fetch(nw, a.nw + n);
+        if (res_ready) {
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+                for (int e = 0; e < W; ++e) rs[i][e] = res_ready[i * (W / 4) + e / 4][e % 4];
+        } else if (a.res)
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+                if (m + 16 * i < a.M) fetch(rs[i], a.res + (size_t)(m + 16 * i) * a.N + n);
+    }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
         const size_t o = (size_t)(m + 16 * i) * a.N + n;
@@ -779,8 +811,8 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                 for (int i = 0; i < MT; ++i)
 #pragma unroll
                     for (int q = 0; q < P; ++q) v[i][q] = acc[i][j + q];
-                if constexpr (!EARLY) conv_fetch(kc[0], a, m0 + rl, n);
-                conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, MT>(a, v, rms, m0 + rl, n, kc[EARLY ? j / P : 0]);
+                if constexpr (EARLY) conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, MT, true>(a, v, rms, m0 + rl, n, nullptr, kc[j / P]);
+                else conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, MT>(a, v, rms, m0 + rl, n);
             } else {
 #pragma unroll
                 for (int i = 0; i < MT; ++i)
@@ -788,9 +820,7 @@ __global__ __launch_bounds__(64 * WM * WN * WK) void k_conv_dma(ConvDmaArgs a) {
                         f32x4 v[1][P];
 #pragma unroll
                         for (int q = 0; q < P; ++q) v[0][q] = sum(i * NT + j + q);
-                        conv_consts<4 * P, 1> k1;
-                        conv_fetch(k1, a, m0 + rl + i * 16, n);
-                        conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n, k1);
+                        conv_dma_out<NP == 3 ? 3 : 2, EPI, 4 * P, 1>(a, v, rms ? rms + i * 16 : nullptr, m0 + rl + i * 16, n);
                     }
             }
         }
@@ -998,9 +1028,7 @@ __global__ __launch_bounds__(64 * NW, C == 192 ? 2 : C == 128 ? 3 : 4) void k_co
         f32x4 v[MT][2];
 #pragma unroll
         for (int i = 0; i < MT; ++i) { v[i][0] = out[i][2 * p]; v[i][1] = out[i][2 * p + 1]; }
-        conv_consts<8, MT> k;
-        conv_fetch(k, a2, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
-        conv_dma_out<T, 0, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, k);
+        conv_dma_out<T, 0, 8, MT>(a2, v, nullptr, m0 + wv * MT * 16 + fr, p * 32 + fk * 8, EARLY ? res[EARLY ? p : 0] : nullptr);
     }
 }
 
