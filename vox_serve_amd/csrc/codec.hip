@@ -441,7 +441,7 @@ struct conv_consts {
     int cj, cc;      // (a transposed conv's N = r * sn_mod outputs: r consumer rows)
 };
 // What the epilogue reads, asked for ahead of the K loop.  (Kernels whose waves have no registers for it read it in the epilogue: through this
-// struct the 256 x 192 tile spilled 36 bytes a lane there, 73 -> 82 us at 51 200 rows of 384 channels.)
+// struct the 256 x 192 tile spilled 36 bytes a lane there, 146 -> 165 us at 51 200 rows of 384 channels, 7 taps.)
 template <int W, int MT>
 __device__ __forceinline__ void conv_fetch(conv_consts<W, MT>& k, const ConvDmaArgs& a, int m, int n) {
     if (n >= a.N) return;
