@@ -859,6 +859,9 @@ int vox_flow_decode_chunk_slots(vox_flow* m, void* stream, const int32_t* tokens
 int vox_fade_in_out(void* stream, float* wav, int n, int L, const float* prev_tail, const double* window, int fade);
 /* z [mel][frames] = the seeded CFM start noise vox_flow_* draw when `noise` is NULL (for callers that replay captured graphs) */
 int vox_flow_fill_noise(void* stream, uint64_t seed, uint32_t noise_stream, int mel, int frames, float* z);
+/* y[i] = f(x[i]), n device floats: the scalar functions of the codecs' and flows' kernels (0 GELU, 1 Mish, 2 the attention's exponential, for
+ * checks of each by itself; x <= 0 for the last) */
+int vox_flow_function(void* stream, int which, const float* x, float* y, int n);
 
 /* ---- GLM-4-Voice flow: speech tokens -> mel ---------------------------------------------------------------------------
  * Replaces GLMFlowModel.inference (/root/reference/vox_serve/tokenizer/glm.py:2065-2112: BlockConformerEncoder :1005-1112 with

@@ -3766,17 +3766,13 @@ int vox_hift_decode(vox_hift* m, void* stream, const float* mel, int n, int T, c
 // ====================================================================================================================
 // CosyVoice2 flow (speech tokens -> mel): conformer encoder + conditional flow matching.  See include/voxhip.h for the contract.
 // ====================================================================================================================
-// exp(d) for d <= 88 (or NaN), to the last bit or two of fp32: 2^(d log2 e) with what the product's rounding drops; below the smallest denormal 0, also for -inf
-__device__ __forceinline__ float exp_below(float d) {
-    const float t = d * 1.44269504088896340736f;
-    const float e = __fmaf_rn(d, 1.925963033500e-8f, __fmaf_rn(d, 1.44269504088896340736f, -t));
-    const float x = __builtin_amdgcn_exp2f(t);
-    return d < -104.0f ? 0.0f : __fmaf_rn(x, e * 0.693147180559945f, x);
-}
+// The exponential of the attention's scores: libm's, within one unit of the last place (0.82 at worst over -10 .. 0, 0.30 in the mean square), denormal results
+// included.  exp2 of the unreduced product with a correction behind it was 1.24 and 0.41, and 0 below 2^-126 (k_flow_attn_mfma, 184 keys: 11.7 us for 12.0).
+__device__ __forceinline__ float flow_exp(float d) { return expf(d); }
 // v tanh(log(1 + e^v)) = v n / (n + 2) with n = e^v (e^v + 2): sums of positive terms only, where log1p and tanh took some 250 instructions (k_flow_ln, 896 rows of
 // 256: 4.75 us a launch, now 4.5, which is what a launch takes); error over normal inputs, relative 2-norm, 3.6e-8 (with libm's three steps rounded right: 3.4e-8)
 __device__ __forceinline__ float mish_f(float v) {
-    const float e = exp_below(v > 20.0f ? 20.0f : v), n = __fmaf_rn(e, e, e + e), d = n + 2.0f;
+    const float e = flow_exp(v > 20.0f ? 20.0f : v), n = __fmaf_rn(e, e, e + e), d = n + 2.0f;
     const float r = __builtin_amdgcn_rcpf(d), q = n * r;
     return v * __fmaf_rn(__fmaf_rn(-q, d, n), r, q);
 }
@@ -4281,8 +4277,8 @@ __device__ __forceinline__ float row16_max(float s) {
 // weights), one of that product's eight runs of K: the feed-forward launch adds the heads' planes in order and has the product's bits without
 // its 256 KB of weights a block.  896 rows: 11.4 -> 13.0 us here, 13.0 -> 10.8 there and 9.1 -> 8.3 in the next q | k | v.  (Two query
 // tiles a block, which read each key once for both: 15.2.)
-// Four waves share a SIMD, so what a wave issues counts: 184 keys, 13.6 us -> 11.8 with a tile's rows addressed together and clamped (each row had its own
-// branches, a division among them, and a wait between the tiles), DPP in the place of LDS permutes and exp_below in the place of expf (2.6 are its fp32 MFMA).
+// Four waves share a SIMD, so what a wave issues counts: 184 keys, 13.6 us -> 12.0 with a tile's rows addressed together and clamped (each row had its own
+// branches, a division among them, and a wait between the tiles) and DPP in the place of LDS permutes (2.6 are its fp32 MFMA).
 template <int DK, int WV, bool OUT>
 __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
     static_assert(DK == 64, "operand layout below is written for 64-dim heads");
@@ -4385,7 +4381,7 @@ __global__ __launch_bounds__(64 * WV) void k_flow_attn_mfma(FlowAttn a) {
         if (t * WV + wave < nt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-                const float p = exp_below(sc[t][r] - top[r]);
+                const float p = flow_exp(sc[t][r] - top[r]);
                 Ps[wave][4 * kq + r][16 * t + fr] = p;
                 sum[r] += p;
             }
@@ -5366,6 +5362,17 @@ __global__ __launch_bounds__(256) void k_flow_noise_z(uint64_t seed, uint32_t st
 extern "C" int vox_flow_fill_noise(void* stream, uint64_t seed, uint32_t noise_stream, int mel, int frames, float* z) {
     if (!z || mel < 1 || frames < 1) return vox_fail(VOX_ERR_INVALID, "flow_fill_noise: bad arguments");
     hipLaunchKernelGGL(k_flow_noise_z, dim3(ew_grid((size_t)mel * frames)), dim3(256), 0, (hipStream_t)stream, seed, noise_stream, z, (size_t)mel * frames);
+    return VOX_OK;
+}
+
+// y = the function that the codecs' and flows' kernels use, one value a thread
+__global__ __launch_bounds__(256) void k_flow_function(int which, const float* x, float* y, size_t n) {
+    const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
+    if (i < n) y[i] = which == 0 ? gelu_f(x[i]) : which == 1 ? mish_f(x[i]) : flow_exp(x[i]);
+}
+extern "C" int vox_flow_function(void* stream, int which, const float* x, float* y, int n) {
+    if (which < 0 || which > 2 || !x || !y || n < 1) return vox_fail(VOX_ERR_INVALID, "flow_function: bad arguments");
+    hipLaunchKernelGGL(k_flow_function, dim3(((size_t)n + 255) / 256), dim3(256), 0, (hipStream_t)stream, which, x, y, (size_t)n);
     return VOX_OK;
 }
 
