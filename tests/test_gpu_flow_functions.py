@@ -45,3 +45,13 @@ def test_exponential_of_the_attention():
     x, y = call(EXP, torch.cat([torch.linspace(-110, 0, 1_000_003), torch.tensor([v for v in SPECIAL if not v > 0])]))
     assert same_bits(y, torch.exp(x))
     assert (y[(x < -88) & (x > -103)] > 0).all() and y[x == float("-inf")].eq(0).all()
+
+
+def test_mish():
+    x, y = call(MISH, torch.cat([torch.randn(4_000_000, generator=torch.Generator().manual_seed(0)), torch.linspace(-120, 120, 100_001), torch.tensor(SPECIAL)]))
+    assert same_bits(y, x * torch.tanh(torch.where(x > 20, x, torch.log1p(torch.exp(x)))))
+    n = slice(0, 4_000_000)
+    w = x[n].double() * torch.tanh(torch.log1p(torch.exp(x[n].double())))
+    e = (y[n].double() - w).norm() / w.norm()
+    print("mish", e.item())
+    assert e < 3.5e-8
