@@ -55,3 +55,13 @@ def test_mish():
     e = (y[n].double() - w).norm() / w.norm()
     print("mish", e.item())
     assert e < 3.5e-8
+
+
+def test_gelu():
+    x, y = call(GELU, torch.cat([torch.randn(4_000_000, generator=torch.Generator().manual_seed(0)), torch.linspace(-120, 120, 100_001), torch.tensor(SPECIAL)]))
+    n = slice(0, 4_000_000)
+    w = x[n].double() * 0.5 * (1 + torch.erf(x[n].double() * 0.5 ** 0.5))
+    e = (y[n].double() - w).norm() / w.norm()
+    print("gelu", e.item())
+    assert same_bits(y, 0.5 * x * (1 + torch.erf(x * 0.70710678118654752440)))
+    assert e < 4e-8

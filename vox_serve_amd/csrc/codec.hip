@@ -113,25 +113,9 @@ __device__ __forceinline__ float snake_exact(float v, float alpha, float invb) {
     return v + invb * (s_ * s_);
 }
 
-// GELU (its exact form) = v Phi(v).  Phi(-a) = 2^-(1 + a P(a)) for a = |v|: P of degree 9 fitted to (-log2 Phi(-a) - 1) / a on [0, 6] (weighted least squares,
-// reweighted towards equal errors of a Phi(-a)); beyond, P goes on rising and the power is below 1e-9.  No branch: with libm's erff, whose two
-// ranges a wave runs both, k_tb_ff took 10.9 us for 9.9 (896 rows, eight values a lane; row sums by DPP with it).  Error over normal inputs, relative 2-norm: 3.4e-8 (0.5 v (1 + erf), erf rounded right:
-// 3.8e-8, which for v < 0 loses what 1 + erf cancels: 1.1e-5 of the value at -3; here 1e-6).
-__device__ __forceinline__ float gelu_f(float v) {
-    const float a = fabsf(v);
-    float p = 3.89322242e-8f;
-    p = __fmaf_rn(p, a, -1.08436791e-6f);
-    p = __fmaf_rn(p, a, 1.30051358e-5f);
-    p = __fmaf_rn(p, a, -8.60596701e-5f);
-    p = __fmaf_rn(p, a, 3.05078225e-4f);
-    p = __fmaf_rn(p, a, -3.79670673e-5f);
-    p = __fmaf_rn(p, a, -6.91637117e-3f);
-    p = __fmaf_rn(p, a, 5.24296537e-2f);
-    p = __fmaf_rn(p, a, 4.59222287e-1f);
-    p = __fmaf_rn(p, a, 1.15110421f);
-    const float t = __builtin_amdgcn_exp2f(-__fmaf_rn(p, a, 1.0f));
-    return v * (v < 0.0f ? t : 1.0f - t);
-}
+// GELU in its exact form.  (As v Phi(v) with log2 Phi by a polynomial and no branch: k_tb_ff, 896 rows, 9.9 us for 10.5, and 3.4e-8 from 64 bits over normal inputs
+// for 3.9e-8, relative 2-norm; but every codec's samples move by it, a flow's by 4e-4 once ten solver steps and the vocoder's source phase have carried it on.)
+__device__ __forceinline__ float gelu_f(float v) { return 0.5f * v * (1.0f + erff(v * 0.70710678118654752440f)); }
 
 // Epilogue of the tiled conv GEMMs (2 x 2 waves, WM x WN 16x16 tiles per wave)
 template <int WM, int WN>
