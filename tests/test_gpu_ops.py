@@ -156,11 +156,12 @@ def test_paged_decode_attention_bit_exact(dev, Hq, Hkv, D, page, lens):
     assert np.array_equal(Bits(out), ref)
 
 
-def test_paged_prefill_attention_bit_exact(dev):
+# (grids of up to 4096 blocks ask for their arguments at once, larger ones do not: 2784 and 7320)
+@pytest.mark.parametrize("q_lens,kv_lens", [([40, 1, 75], [40, 90, 75]), ([150, 3, 30], [150, 90, 33])])
+def test_paged_prefill_attention_bit_exact(dev, q_lens, kv_lens):
     from vox_serve_amd.flashinfer_utils import FlashInferPrefillWrapper
     rng = np.random.default_rng(5)
     Hq, Hkv, D, page = 16, 8, 128, 16
-    q_lens, kv_lens = [40, 1, 75], [40, 90, 75]
     npages = [(n + page - 1) // page for n in kv_lens]
     P = sum(npages) + 2
     indptr = np.concatenate([[0], np.cumsum(npages)]).astype(np.int32)

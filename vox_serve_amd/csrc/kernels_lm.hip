@@ -2244,7 +2244,6 @@ struct HeadArgs {
 };
 
 __global__ __launch_bounds__(64) void k_head_prepare(HeadArgs a) {
-    touch_args(a);
     __shared__ float sh[512];
     __shared__ __attribute__((aligned(16))) bf16_t so[512];
     const int head = blockIdx.x, n = blockIdx.y, lane = threadIdx.x;
@@ -2467,9 +2466,11 @@ __device__ __forceinline__ void prep_head(const bf16_t* src, const bf16_t* nw, f
     prep_head_apply<D>(o, nw, eps, cs_row, rot, interleave, sh, out, lane);
 }
 
-template <int D, bool FUSED>
+// TOUCH: every block waits for all of its arguments first, also those past their row's end, which a causal prompt has about half of.  That pays while the
+// first blocks' trip is what a launch takes; behind the first blocks of a CU the lines are in its scalar cache and the wait only holds the slot (figures at the launch).
+template <int D, bool FUSED, bool TOUCH>
 __global__ __launch_bounds__(256) void k_attn_partial(AttnArgs a) {
-    touch_args(a);
+    if (TOUCH) touch_args(a);
     constexpr int LPT = D / 8;        // lanes per token
     constexpr int TPW = 64 / LPT;     // tokens per wave pass
     constexpr int GMAX = 16;
@@ -2637,11 +2638,16 @@ int vox_launch_attn_partial(hipStream_t st, const AttnCall& c) {
     if (nchunk == 1) { a.out = (bf16_t*)c.out; a.out_frag = (bf16_t*)c.out_frag; }
     dim3 grid(nchunk, c.Hkv, c.Nq);
     const bool fused = c.qkv != nullptr;
-#define VOX_ATT(D_)                                                                           \
-    if (c.D == D_) {                                                                          \
-        if (fused) hipLaunchKernelGGL((k_attn_partial<D_, true>), grid, dim3(256), 0, st, a); \
-        else hipLaunchKernelGGL((k_attn_partial<D_, false>), grid, dim3(256), 0, st, a);      \
-        return VOX_OK;                                                                        \
+    // Arguments at once (TOUCH) where a prompt's grid is about two rounds of blocks.  us a Qwen3-TTS prompt, without / with it: 16 rows 2369 / 2359, 40 (640 blocks)
+    // 3060 / 3040, 75 (1800) 3312 / 3304, 128 (4096) 4139 / 4132; 200 (11 200) 9735 / 9770, 450 20 776 / 21 003, 1000 (256 000) 58 150 / 59 750.  The fused form's
+    // prologue has loads enough in front: frames of 8 requests of 600 tokens (1280 blocks) 3395 / 3421, of 32 of 2000 5932 / 6297.
+    const bool touch = (size_t)nchunk * c.Hkv * c.Nq <= 4096;
+#define VOX_ATT(D_)                                                                                             \
+    if (c.D == D_) {                                                                                            \
+        if (fused) hipLaunchKernelGGL((k_attn_partial<D_, true, false>), grid, dim3(256), 0, st, a);            \
+        else if (touch) hipLaunchKernelGGL((k_attn_partial<D_, false, true>), grid, dim3(256), 0, st, a);       \
+        else hipLaunchKernelGGL((k_attn_partial<D_, false, false>), grid, dim3(256), 0, st, a);                 \
+        return VOX_OK;                                                                                          \
     }
     VOX_ATT(128) VOX_ATT(64) VOX_ATT(16)
 #undef VOX_ATT

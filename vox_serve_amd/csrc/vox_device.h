@@ -163,7 +163,7 @@ __device__ __forceinline__ float4 ldg_f4(const float* p) {
 // A kernel's arguments are read where they are first used, and each 64-byte line of them that the scalar cache has not seen yet is a trip to
 // L2: a chain of them in front of the first load of a kernel whose arguments are many.  This asks for all lines at once.
 // (us of a whole call, without / with it in the kernels that take LinArgs, AttnArgs or SampArgs: a Qwen3-TTS frame of 32 requests 4031 / 3921, a
-// CSM frame of 16 4694 / 4575, a prefill of 75 tokens 3322 / 3299)
+// CSM frame of 16 4694 / 4575, a prefill of 75 tokens 3322 / 3299; grids of many rounds of blocks lose by it: k_attn_partial's launch)
 template <class A>
 __device__ __forceinline__ void touch_args(const A& a) {
     int v = 0;
