@@ -129,17 +129,18 @@ def test_more_column_tiles_than_cus(width, vocab, ff, cuts):
 @pytest.mark.parametrize("width,moe,cuts", [(64, (2, 2, 2048, 0, 0), [2, 8, 3]), (512, (3, 1, 4096, 0, 0), [8, 7]), (2048, (8, 2, 2048, 4, 2), [8, 2, 5]),
                                             (2056, (4, 2, 2048, 0, 0), [8, 3]), (4096, (5, 5, 2056, 0, 0), [7, 8, 2]), (3080, (4, 3, 2120, 0, 0), [4, 6]),
                                             (256, (48, 6, 2048, 4, 2), [8, 6]), (64, (48, 16, 2048, 0, 0), [3, 4]), (128, (16, 8, 4104, 0, 0), [8, 8]),
-                                            (4096, (8, 8, 168, 0, 0), [8]), (4096, (4, 1, 2048, 0, 0), [8, 3]), (2052, (8, 2, 2048, 0, 0), [6, 8])])
+                                            (4096, (8, 8, 168, 0, 0), [8]), (4096, (4, 1, 2048, 0, 0), [8, 3]), (4096, (4, 2, 1032, 0, 0), [8, 5]), (2052, (8, 2, 2048, 0, 0), [6, 8])])
 def test_routed_layers_of_few_rows(width, moe, cuts):
     cfg = P.config([P.attention(mlp=P.moe(*moe), **ATT), P.attention(mlp=P.moe(*moe), kv_from=0, **ATT)], width=width, vocab=50)
     check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)
 
 
-# ... with outputs that have no expert, and with weights that multiply an expert's input
+# ... with outputs that have no expert, and with weights that multiply an expert's input; two choices take the walk of the down rows
 @pytest.mark.parametrize("rows", [2, 5, 8, 40])
-@pytest.mark.parametrize("over", [dict(identity=5), dict(scale_input=True)])
-def test_routed_forms(rows, over):
-    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.moe(6, 3, 2048, 0, 0))], width=64, vocab=50)
+@pytest.mark.parametrize("over", [dict(identity=5), dict(scale_input=True), dict(identity=5, scale_input=True)])
+@pytest.mark.parametrize("width,top,ff", [(64, 3, 2048), (2056, 2, 2048), (64, 2, 2048)])
+def test_routed_forms(rows, over, width, top, ff):
+    cfg = P.config([P.attention(heads=2, kv_heads=1, dim=32, vdim=32, size=50, keep=2, mlp=P.moe(6, top, ff, 0, 0))], width=width, vocab=50)
     base = kazozen.config_from_dict(cfg)
     layer = base.layers[-1]
     d = dataclasses.replace(base, layers=[*base.layers[:-1], dataclasses.replace(layer, moe=dataclasses.replace(layer.moe, **over))])

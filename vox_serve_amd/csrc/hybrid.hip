@@ -5478,51 +5478,52 @@ __global__ __launch_bounds__(256) void k_hb_moe_down_rows(const bf16_t* act, con
     }
     if (lane == 0) hb_join_apply(join, jin, C + (size_t)row * ldc, row, c, acc);
 }
-// The same for one or two choices and K <= 2048: 64 blocks of each XCD are shared out among the rows, and a block's waves walk that XCD's columns, the row's
-// activations in registers, the next column's weights in flight while this one's are multiplied.
+// The same for two choices and K <= 2048: 64 blocks of each XCD are shared out among the rows, and a block's waves walk that XCD's columns, the row's
+// activations in registers, the next column's weights in flight while this one's are multiplied.  A wave takes 64 columns at most.
 // 8 rows, 2048 x 2048, 16 choices among 8 experts: 18.4 -> 16.2 us.
 #define HB_MOE_DOWN_BLOCKS 512      // two to a CU, 64 to an XCD
-template <bool TWO>
+static bool hb_moe_down_walks(int M, int N, int K, int top) { return top == 2 && K <= 2048 && N <= 64 * 32 * (HB_MOE_DOWN_BLOCKS / 8 / M); }
 __global__ __launch_bounds__(256, 2) void k_hb_moe_down_walk(const bf16_t* act, const bf16_t* w_down, const float* h, long ldh, float* C, long ldc, int M, int N, int K,
                                                              hb_join join, hb_entries en) {
-    constexpr int NC = 4, NE = TWO ? 2 : 1;
+    constexpr int NC = 4;
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), in_xcd = (int)blockIdx.x >> 3;
-    const int row = in_xcd % M, at = in_xcd / M, step = (HB_MOE_DOWN_BLOCKS / 8 / M) * 32, i0 = row * en.top;
+    const int row = in_xcd % M, at = in_xcd / M, step = (HB_MOE_DOWN_BLOCKS / 8 / M) * 32, i0 = row * 2;
     if (at >= HB_MOE_DOWN_BLOCKS / 8 / M) return;
-    int c = (at * 8 + ((int)blockIdx.x & 7)) * 4 + wv;
+    const int first = (at * 8 + ((int)blockIdx.x & 7)) * 4 + wv;
+    if (first >= N) return;
     const bool b5 = lane & 32;
-    int e[NE];
-    float wg[NE];
-    const bf16_t* p[NE];
-    uint4 v[NE][NC], ua[NE][NC], ub[NE][NC];
+    int e[2];
+    float wg[2];
+    const bf16_t* p[2];
+    uint4 v[2][NC], ua[2][NC], ub[2][NC];
     int ko[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) ko[i] = 512 * i + lane * 8 < K ? 512 * i + lane * 8 : 0;
 #pragma unroll
-    for (int j = 0; j < NE; ++j) {
+    for (int j = 0; j < 2; ++j) {
         e[j] = en.sel[i0 + j];
         wg[j] = en.wgt[i0 + j];
         p[j] = w_down + (size_t)(e[j] < en.experts ? e[j] : 0) * N * K;
 #pragma unroll
         for (int i = 0; i < NC; ++i) v[j][i] = ldg((const uint4*)(act + (size_t)(i0 + j) * K + ko[i]));
     }
-    auto load = [&](uint4 (&u)[NE][NC], int c) {
+    auto load = [&](uint4 (&u)[2][NC], int c) {
 #pragma unroll
-        for (int j = 0; j < NE; ++j)
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
             for (int i = 0; i < NC; ++i) u[j][i] = ldg((const uint4*)(p[j] + (size_t)c * K + ko[i]));
         __builtin_amdgcn_sched_barrier(0);
     };
     float s0 = 0.f, s1 = 0.f;      // lane t: the sums of the wave's t-th column
     int t = 0;
-    auto column = [&](const uint4 (&u)[NE][NC]) {
+    auto column = [&](const uint4 (&u)[2][NC]) {
         float a[2] = {0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < NC; ++i) {
             if (512 * i >= K) break;
             if (512 * i + lane * 8 < K)
 #pragma unroll
-                for (int j = 0; j < NE; ++j) a[j] = hb_dot8(u[j][i], v[j][i], a[j]);
+                for (int j = 0; j < 2; ++j) a[j] = hb_dot8(u[j][i], v[j][i], a[j]);
         }
         float d = (b5 ? a[1] : a[0]) + __shfl_xor(b5 ? a[0] : a[1], 32, 64);      // (hb_wave_sum's tree, an entry to each half of the wave)
         d = butterfly<32>(d);
@@ -5531,39 +5532,28 @@ __global__ __launch_bounds__(256, 2) void k_hb_moe_down_walk(const bf16_t* act, 
         s1 = lane == t ? d1 : s1;
         ++t;
     };
-    // 64 columns at most between two of these: their joins together, a lane a column
-    auto finish = [&](int first) {
-        const int cl = first + lane * step;
-        if (lane < t) {
-            const hb_join_in jin = hb_join_load(join, C + (size_t)row * ldc, row, cl);
-            const float hv = e[0] >= en.experts || e[NE - 1] >= en.experts ? h[(size_t)row * ldh + cl] : 0.f;
-            float acc = 0.f;
-            if (e[0] >= en.experts) acc = fmaf(wg[0], hv, acc);
-            else acc = fmaf(en.scale_input ? 1.0f : wg[0], s0, acc);
-            if (TWO) {
-                if (e[NE - 1] >= en.experts) acc = fmaf(wg[NE - 1], hv, acc);
-                else acc = fmaf(en.scale_input ? 1.0f : wg[NE - 1], s1, acc);
-            }
-            hb_join_apply(join, jin, C + (size_t)row * ldc, row, cl, acc);
-        }
-        t = 0;
-    };
-    while (c < N) {
-        const int first = c, end = N - c > 64 * step ? c + 64 * step : N;
-        load(ua, c);
-        while (true) {      // (a column's weights and the next one's lie in one path: the waits stay exact)
-            if (c + step >= end) { column(ua); break; }
-            load(ub, c + step);
-            column(ua);
-            c += step;
-            if (c + step >= end) { column(ub); break; }
-            load(ua, c + step);
-            column(ub);
-            c += step;
-        }
+    int c = first;
+    load(ua, c);
+    while (true) {      // (a column's weights and the next one's lie in one path: the waits stay exact)
+        if (c + step >= N) { column(ua); break; }
+        load(ub, c + step);
+        column(ua);
         c += step;
-        finish(first);
+        if (c + step >= N) { column(ub); break; }
+        load(ua, c + step);
+        column(ub);
+        c += step;
     }
+    if (lane >= t) return;      // the joins together, a lane a column
+    const int cl = first + lane * step;
+    const hb_join_in jin = hb_join_load(join, C + (size_t)row * ldc, row, cl);
+    const float hv = e[0] >= en.experts || e[1] >= en.experts ? h[(size_t)row * ldh + cl] : 0.f;
+    float acc = 0.f;
+    if (e[0] >= en.experts) acc = fmaf(wg[0], hv, acc);
+    else acc = fmaf(en.scale_input ? 1.0f : wg[0], s0, acc);
+    if (e[1] >= en.experts) acc = fmaf(wg[1], hv, acc);
+    else acc = fmaf(en.scale_input ? 1.0f : wg[1], s1, acc);
+    hb_join_apply(join, jin, C + (size_t)row * ldc, row, cl, acc);
 }
 static bool hb_glu_rows_ok(const float* A, long lda, const bf16_t* W, int M, int K) {
     return M >= 2 && M <= 16 && !(K & 31) && !(lda & 3) && !((size_t)A & 15) && !((size_t)W & 15);
@@ -5606,10 +5596,8 @@ static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16
     if (M < 2 || M * en.top > 64 || en.experts < 1 || (W & 7) || (ldh & 3) || ((size_t)h & 15) || ((size_t)w_gate_up & 15) || (ff & 7) || ((size_t)w_down & 15) ||
         lds > 64 * 1024 || !hb_moe_rows_pay(M, W, ff, en.top)) return false;
     hipLaunchKernelGGL(k_hb_moe_up_rows, dim3(hb_moe_up_blocks(M * en.top, ff)), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
-    if (en.top == 2 && ff <= 2048)
-        hipLaunchKernelGGL(k_hb_moe_down_walk<true>, dim3(HB_MOE_DOWN_BLOCKS), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
-    else if (en.top == 1 && ff <= 2048)
-        hipLaunchKernelGGL(k_hb_moe_down_walk<false>, dim3(HB_MOE_DOWN_BLOCKS), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
+    if (hb_moe_down_walks(M, W, ff, en.top))
+        hipLaunchKernelGGL(k_hb_moe_down_walk, dim3(HB_MOE_DOWN_BLOCKS), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
     else hipLaunchKernelGGL(k_hb_moe_down_rows, dim3((W + 31) / 32 * 8 * M), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
     return true;
 }
