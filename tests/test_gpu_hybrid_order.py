@@ -135,7 +135,7 @@ def test_routed_layers_of_few_rows(width, moe, cuts):
     check(cfg, P.random_checkpoint(cfg, seed=width), sum(cuts) + 2, cuts)
 
 
-# ... with outputs that have no expert, and with weights that multiply an expert's input; two choices take the walk of the down rows
+# ... with outputs that have no expert, and with weights that multiply an expert's input; two choices and 8192 sums and more take the walk of the down rows
 @pytest.mark.parametrize("rows", [2, 5, 8, 40])
 @pytest.mark.parametrize("over", [dict(identity=5), dict(scale_input=True), dict(identity=5, scale_input=True)])
 @pytest.mark.parametrize("width,top,ff", [(64, 3, 2048), (2056, 2, 2048), (64, 2, 2048)])

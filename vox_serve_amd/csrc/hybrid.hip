@@ -742,8 +742,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_hb_gemm_dma(const bf16_t* A
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * (NA + NW)) : "memory");
     int stage = 0;
     // A wave whose rows all lie past the end (the last rows of an expert's list fill a tenth of a 256-row tile as often as all of it) only
-    // loads: its share of the matrix cores goes to the wave beside it on the SIMD, whose rows lie 128 further up.  A prefill of 2048 tokens over eight
-    // experts, 4214 -> 4177 us.
+    // loads: its share of the matrix cores goes to the wave beside it on the SIMD, whose rows lie 128 further up.  Prefills over eight experts, multiplying those rows / so, four
+    // runs of each in turn that differ by 0.3 %, us: 700 tokens 2356 / 2328, 1000 2739 / 2705, 1500 3516 / 3468, 1800 3896 / 3795, 2048 4073 / 4023; 100 and 400 the same.
     if (m0 + wm * MT * 16 >= M) {
         for (int kt = 0; kt < nt; ++kt) {
             asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
@@ -5198,8 +5198,8 @@ __global__ __launch_bounds__(256) void k_hb_moe_combine(float* x, long ldx, cons
 //
 // y = hb_glu(A . Wg^T + b, A . Wu^T + b): k_hb_gemm_rows16's product and sums on a tile of eight gate and the same eight up columns, so the
 // activation is in its epilogue.  out: rows of ldo elements, bf16 where out16.
-// Bound by the weights' way from memory.  8 rows, 11264 x 2048 (46 MB): 15.4 us + 4.8 for the activation's own launch -> 16.0.  Column tiles walked by one
-// block, with the next tile's weights asked for ahead and the rows kept: 22 - 28, the registers leave too few blocks.
+// Bound by the weights' way from memory.  8 rows, 11264 x 2048 (46 MB): 15.4 us + 4.8 for the activation's own launch -> 16.0.  Where there are more tiles than CUs and
+// K fills a wave's registers k_hb_rows_walk takes the product (12.1; a first form of that walk, whose registers left too few blocks, 22 - 28).
 template <bool FULL>
 __global__ __launch_bounds__(512) void k_hb_glu_rows(const float* A, long lda, const bf16_t* Wt, const float* bias, void* out, long ldo, int out16, int M, int ff,
                                                      int K, hb_glu_args glu) {
@@ -5311,12 +5311,9 @@ __device__ __forceinline__ float hb_dot8(uint4 u, uint4 v, float a) {
 // choices among 8 experts of 2048 x 2048 (up to 134 MB of distinct rows, 268 with each entry reading
 // its own): 38.7 -> 29.9 us (31.8 with a block for each group of columns and entry, most of which ended at once, and no weights in flight while others are multiplied).
 #define HB_MOE_UP_ROWS 8
-// Two blocks to a CU, or one for every unit that there can be (eight columns of an entry's expert) while that is few: 2 rows, 3 choices among 8 experts of 2048 x
-// 1024, a step of three such layers 184 us with a block each and 189 with 512 that walk.
-static int hb_moe_up_blocks(int entries, int ff) {
-    const int units = entries * ((ff + 7) / 8);
-    return units <= 1280 ? units : 512;
-}
+// What the registers leave room for, two to a CU.  (A block for every eight columns of an entry's expert instead, us a step of three such layers, 512 / those: 2 rows
+// of 2048, 8 experts, 2 choices, 2048 wide (1024 of them) 208 / 218, of 4096 300 / 316, of 1024 170 / 176; 8 rows of 2048 307 / 344.)
+#define HB_MOE_UP_BLOCKS 512
 // the entries that share this lane's expert with an earlier one left out: one bit for each routed expert (ne <= 64 entries, one a lane)
 __device__ __forceinline__ unsigned long long hb_moe_leaders(int sel, int ne, int experts, int lane) {
     bool first = lane < ne && sel < experts;
@@ -5480,9 +5477,11 @@ __global__ __launch_bounds__(256) void k_hb_moe_down_rows(const bf16_t* act, con
 }
 // The same for two choices and K <= 2048: 64 blocks of each XCD are shared out among the rows, and a block's waves walk that XCD's columns, the row's
 // activations in registers, the next column's weights in flight while this one's are multiplied.  A wave takes 64 columns at most.
-// 8 rows, 2048 x 2048, 16 choices among 8 experts: 18.4 -> 16.2 us.
+// 8 rows, 2048 x 2048, 16 choices among 8 experts: 18.4 -> 16.2 us.  Few waves have a few columns each, so it pays from four rows and 8192 sums on; us a step of three such
+// layers, this / the kernel above: 4096 x 2048, 8, 6, 4 rows 426 / 442, 405 / 411, 362 / 364, 3 and 2 rows 336 / 336, 301 / 299; 2048 x 2048, 8, 4 rows 306 / 311, 249 / 250, 3 and 2 rows 246 /
+// 243, 207 / 206; 1024 x 2048, 8 rows 225 / 227, 6 and 4 rows 204 / 204, 190 / 188.
 #define HB_MOE_DOWN_BLOCKS 512      // two to a CU, 64 to an XCD
-static bool hb_moe_down_walks(int M, int N, int K, int top) { return top == 2 && K <= 2048 && N <= 64 * 32 * (HB_MOE_DOWN_BLOCKS / 8 / M); }
+static bool hb_moe_down_walks(int M, int N, int K, int top) { return top == 2 && K <= 2048 && M >= 4 && M * N >= 8192 && N <= 64 * 32 * (HB_MOE_DOWN_BLOCKS / 8 / M); }
 __global__ __launch_bounds__(256, 2) void k_hb_moe_down_walk(const bf16_t* act, const bf16_t* w_down, const float* h, long ldh, float* C, long ldc, int M, int N, int K,
                                                              hb_join join, hb_entries en) {
     constexpr int NC = 4;
@@ -5595,7 +5594,7 @@ static bool hb_try_moe_rows(hipStream_t st, const float* h, long ldh, const bf16
     const size_t lds = (size_t)HB_MOE_UP_ROWS * W * 2;
     if (M < 2 || M * en.top > 64 || en.experts < 1 || (W & 7) || (ldh & 3) || ((size_t)h & 15) || ((size_t)w_gate_up & 15) || (ff & 7) || ((size_t)w_down & 15) ||
         lds > 64 * 1024 || !hb_moe_rows_pay(M, W, ff, en.top)) return false;
-    hipLaunchKernelGGL(k_hb_moe_up_rows, dim3(hb_moe_up_blocks(M * en.top, ff)), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
+    hipLaunchKernelGGL(k_hb_moe_up_rows, dim3(HB_MOE_UP_BLOCKS), dim3(256), lds, st, h, ldh, w_gate_up, (bf16_t*)act, W, ff, M, glu, en);
     if (hb_moe_down_walks(M, W, ff, en.top))
         hipLaunchKernelGGL(k_hb_moe_down_walk, dim3(HB_MOE_DOWN_BLOCKS), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
     else hipLaunchKernelGGL(k_hb_moe_down_rows, dim3((W + 31) / 32 * 8 * M), dim3(256), 0, st, (const bf16_t*)act, w_down, h, ldh, C, ldc, M, W, ff, join, en);
