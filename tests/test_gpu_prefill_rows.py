@@ -41,3 +41,28 @@ def test_stack_few_rows_more_column_tiles_than_cus(dev, n_rows, dims):  # noqa: 
     """Up to 16 rows of 4096 values whose norm runs inside k_gemm_tiles: one and two rows a wave, 257 .. 514 column tiles (the last round of blocks nearly
     empty), and the down projection behind them on k_linear_mfma_stream with its input fragment-major, waves with a k-step more than others among them."""
     stack_rows_case(Tape(), dev, n_rows, dims=dims)
+
+
+@pytest.mark.parametrize("B,V", [(8, 12305), (9, 8192), (9, 8197), (9, 12288), (16, 12305), (16, 16400), (3, 20487), (16, 20480)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_head_of_few_rows_walks_column_tiles(dev, B, V, bias):  # noqa: F811
+    """A 4096-wide model's head (k_gemm_tiles, plain outputs): two to five rounds of a block per CU and one tile more, a last tile of a few columns, one and two rows
+    a wave.  The layer's outputs are zero, so the head reads the embeddings: rmsnorm and linear on them, in launches of their own, have the same bits."""
+    from vox_serve_amd import _native as N
+    from vox_serve_amd.engine import LMCfg, LMEngine, StackCfg
+    H, D, F = 4096, 128, 64
+    rng = np.random.default_rng(B + V)
+    w = lambda *s, m=0.0, sd=0.05: T(vr.f2bf(m + rng.standard_normal(s, dtype=np.float32) * np.float32(sd)), dev)
+    zero = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=dev)
+    layer = dict(wqkv=w(4 * D, H), wo=zero(H, 2 * D), wgate=w(F, H), wup=w(F, H), wdown=zero(H, F), ln1=w(H, m=1.0), ln2=w(H, m=1.0))
+    norm, emb, head, b = w(H, m=1.0), w(B, H, sd=1.0), w(V, H), w(V, sd=1.0) if bias else None
+    eng = LMEngine(LMCfg(StackCfg(H, 1, 2, 1, D, F, qk_norm=False), B, V, max_pos=64), [layer], norm, emb, head, b, max_batch=B, page_size=16, max_pages=B, max_seq_len=16,
+                   max_prefill_rows=16, device=dev)
+    eng.input_ids[:, 0] = torch.arange(B, dtype=torch.int32, device=dev)
+    eng.upload_plan(pos=[0] * B, kvlen=[1] * B, page=range(B), slot=[0] * B, indptr=range(B + 1), indices=range(B))
+    eng.frame(B, 1, eng.sampling_cfg(greedy=True), feedback=False)
+    xn, want = torch.empty_like(emb), torch.empty(B, V, dtype=torch.bfloat16, device=dev)
+    N.check(N.lib().vox_rmsnorm(N.ctx(), N.stream(), N.ptr(emb), N.ptr(norm), N.ptr(xn), B, H, 1e-6))
+    N.check(N.lib().vox_linear(N.ctx(), N.stream(), N.ptr(head), N.ptr(b) if bias else None, N.ptr(xn), None, N.ptr(want), B, V, H, 0))
+    got = eng.out_logits[:B]
+    assert want.float().std() > 0 and np.array_equal(Bits(got), Bits(want)), (got != want).nonzero()[:4].tolist()
