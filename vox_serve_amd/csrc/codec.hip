@@ -2294,9 +2294,10 @@ static int codec_attention(vox_codec* m, hipStream_t st, int l, const int32_t* s
     bf16_t* ring = m->ring + (size_t)l * m->max_slots * c.window * 2 * HD;
     // (VOX_CODEC_ATTN2=0: RoPE / ring write and the attention as two launches — A/B timing; bit-identical)
     static const bool attn2 = [] { const char* e = getenv("VOX_CODEC_ATTN2"); return !(e && e[0] == '0'); }();
-    const size_t lds2 = (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + L * c.window) * 4;
-    if (attn2 && c.head_dim == 64 && L <= c.window && lds2 <= 64 * 1024) {
-        const size_t lds = (size_t)(c.window * (2 * c.head_dim + 4) + L * c.head_dim + L * ((c.window + 3) & ~3)) * 4;
+    // One launch up to a tile of 64 KB; with its rows on 16 bytes it takes up to 2 % more, two blocks of which still share a CU's LDS
+    const size_t tile = (size_t)(2 * c.window * (c.head_dim + 1) + L * c.head_dim + L * c.window) * 4;
+    if (attn2 && c.head_dim == 64 && L <= c.window && tile <= 64 * 1024) {
+        const size_t lds = tile + (size_t)(2 * c.window + L * (-c.window & 3)) * 4;
         if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_codec_attn2<64>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
         hipLaunchKernelGGL(k_codec_attn2<64>, dim3(c.num_heads, n), dim3(attn_threads(L)), lds, st, qkv, ring, slots, m->pos, out, L, c.num_heads, c.window,
                            m->w.inv_freq, terms);
