@@ -419,6 +419,18 @@ __device__ __forceinline__ void conv_put_terms(bf16_t* row, int width, int c, co
 #define CONV_SINE 4        // 0, with snake_exact for SnakeBeta
 // The epilogue of W neighbouring channels (n ..) of MT rows (m, m + 16, ..) that one lane holds: constants once, every row's residual
 // requested ahead of the first store, 16-byte accesses throughout.
+template <int W>
+__device__ __forceinline__ void conv_get(float (&d)[W], const float* p) {
+#pragma unroll
+    for (int q = 0; q < W / 4; ++q) {
+        const f32x4 t = *reinterpret_cast<const f32x4_a4*>(p + 4 * q);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
+    }
+}
+// the consumer row and the bias of channel n (no division where there is one row, one bias a channel)
+__device__ __forceinline__ int conv_row_of(const ConvDmaArgs& a, int n) { return !a.out2 || a.sn_mod >= a.N ? 0 : n / a.sn_mod; }
+__device__ __forceinline__ int conv_bias_at(const ConvDmaArgs& a, int n) { return a.bias_mod >= a.N ? n : n % a.bias_mod; }
 template <int W, int MT>
 struct conv_consts {
     float b[W], s[W], al[W], ib[W], nw[W], rs[MT][W];
@@ -429,23 +441,15 @@ struct conv_consts {
 template <int W, int MT>
 __device__ __forceinline__ void conv_fetch(conv_consts<W, MT>& k, const ConvDmaArgs& a, int m, int n) {
     if (n >= a.N) return;
-    const auto fetch = [](float (&d)[W], const float* p) {
-#pragma unroll
-        for (int q = 0; q < W / 4; ++q) {
-            const f32x4 t = *reinterpret_cast<const f32x4_a4*>(p + 4 * q);
-#pragma unroll
-            for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
-        }
-    };
-    k.cj = a.out2 ? (a.sn_mod >= a.N ? 0 : n / a.sn_mod) : 0;
+    k.cj = conv_row_of(a, n);
     k.cc = n - k.cj * a.sn_mod;
-    if (a.bias) fetch(k.b, a.bias + (a.bias_mod >= a.N ? n : n % a.bias_mod));
-    if (a.scale) fetch(k.s, a.scale + n);
-    if (a.sn_alpha) { fetch(k.al, a.sn_alpha + k.cc); fetch(k.ib, a.sn_invb + k.cc); }
-    if (a.nw) fetch(k.nw, a.nw + n);
+    if (a.bias) conv_get<W>(k.b, a.bias + conv_bias_at(a, n));
+    if (a.scale) conv_get<W>(k.s, a.scale + n);
+    if (a.sn_alpha) { conv_get<W>(k.al, a.sn_alpha + k.cc); conv_get<W>(k.ib, a.sn_invb + k.cc); }
+    if (a.nw) conv_get<W>(k.nw, a.nw + n);
     if (a.res)
 #pragma unroll
-        for (int i = 0; i < MT; ++i) fetch(k.rs[i], a.res + (size_t)(m + 16 * i < a.M ? m + 16 * i : a.M - 1) * a.N + n);
+        for (int i = 0; i < MT; ++i) conv_get<W>(k.rs[i], a.res + (size_t)(m + 16 * i < a.M ? m + 16 * i : a.M - 1) * a.N + n);
 }
 template <int T, int EPI, int W, int MT, bool FETCHED = false>
 __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (&acc)[MT][W / 4], const float* rms, int m, int n,
@@ -463,20 +467,12 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
             for (int i = 0; i < MT; ++i) rs[i][e] = early.rs[i][e];
         }
     } else {
-        cj = a.out2 ? n / a.sn_mod : 0;
+        cj = conv_row_of(a, n);
         cc = n - cj * a.sn_mod;
-        const auto fetch = [](float (&d)[W], const float* p) {
-#pragma unroll
-            for (int q = 0; q < W / 4; ++q) {
-                const f32x4 t = *reinterpret_cast<const f32x4_a4*>(p + 4 * q);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) d[4 * q + e] = t[e];
-            }
-        };
-        if (a.bias) fetch(b, a.bias + n % a.bias_mod);
-        if (a.scale) fetch(s, a.scale + n);
-        if (a.sn_alpha) { fetch(al, a.sn_alpha + cc); fetch(ib, a.sn_invb + cc); }
-        if (a.nw) fetch(nw, a.nw + n);
+        if (a.bias) conv_get<W>(b, a.bias + conv_bias_at(a, n));
+        if (a.scale) conv_get<W>(s, a.scale + n);
+        if (a.sn_alpha) { conv_get<W>(al, a.sn_alpha + cc); conv_get<W>(ib, a.sn_invb + cc); }
+        if (a.nw) conv_get<W>(nw, a.nw + n);
         if (res_ready) {
 #pragma unroll
             for (int i = 0; i < MT; ++i)
@@ -485,7 +481,7 @@ __device__ __forceinline__ void conv_dma_out(const ConvDmaArgs& a, const f32x4 (
         } else if (a.res)
 #pragma unroll
             for (int i = 0; i < MT; ++i)
-                if (m + 16 * i < a.M) fetch(rs[i], a.res + (size_t)(m + 16 * i) * a.N + n);
+                if (m + 16 * i < a.M) conv_get<W>(rs[i], a.res + (size_t)(m + 16 * i) * a.N + n);
     }
 #pragma unroll
     for (int i = 0; i < MT; ++i) {
