@@ -1276,6 +1276,185 @@ __global__ __launch_bounds__(1024) void k_splitk_reduce_rows(const float* part, 
     }
 }
 
+// The same product for many rows (prompts of more than 128 tokens) in one launch: k_gemm_splitk's sums to the bit — a chain of MFMA k-steps per 256 columns of K,
+// those sums added in ascending order — with both kept in registers, so that no partial sum goes through memory (a 200-row Qwen3 layer wrote and read back
+// 8 x 200 x 12288 x 4 bytes for gate and up alone) and a weight is read once per BM rows, not once per 128 and launch.  BM x BN outputs per block, WM x WN waves.
+// k-tiles of 64 go from memory straight into LDS (1 KB per wave instruction = eight 128-byte rows), S stages of them in flight; the 16-byte pieces of a row
+// lie at piece ^ (row & 7), so the fragment reads of 16 rows do not meet in a bank.  A wave's fragments are read half a k-tile before they are multiplied; one
+// wait + barrier per k-tile, in its middle: it says that every wave's part of tile t + 1 has landed and that every wave holds the second half of tile t in
+// registers, so tile t's stage may be requested anew.  The weights are the first operand (a lane then holds four neighbouring columns of a row).  Blocks of one
+// XCD (block id modulo 8) take neighbouring tiles, 1024 rows deep, so that its L2 holds what they share.
+// EPI_SILU_MUL: the block's columns are BN / 2 gate rows and the BN / 2 up rows beside them, interleaved by U so that a lane owns both.
+template <int BM, int BN, int WM, int WN, int S, int EPI>
+__global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
+    touch_args(a);
+    constexpr bool SM = EPI == EPI_SILU_MUL;
+    constexpr int BK = 64, NWV = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16, CN = SM ? BN / 2 : BN, NA = BM / 8 / NWV, NW = BN / 8 / NWV;
+    constexpr int STAGE = (BM + BN) * BK, U = NT * 8;       // U: gate (up) columns of a wave
+    static_assert(BM % (8 * NWV) == 0 && BN % (8 * NWV) == 0 && (!SM || NT % 2 == 0) && S > 2 && (S - 1) * (NA + NW) < 64, "whole wave instructions");
+    extern __shared__ __attribute__((aligned(1024))) bf16_t slab_lds[];
+    const int tid = threadIdx.x, lane = tid & 63, wv = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tm = (a.B + BM - 1) / BM, tn = (a.N + CN - 1) / CN, total = tm * tn, per = (total + 7) >> 3;
+    const int in_xcd = (int)blockIdx.x >> 3, t = ((int)blockIdx.x & 7) * per + in_xcd;
+    if (in_xcd >= per || t >= total) return;
+    constexpr int GM = 1024 / BM;
+    const int g0 = t / (GM * tn) * GM, gh = tm - g0 < GM ? tm - g0 : GM, tg = t - g0 * tn;
+    const int m0 = (g0 + tg % gh) * BM, n0 = tg / gh * CN;
+    const int wm = wv / WN, wn = wv % WN, fr = lane & 15, fk = lane >> 4;
+    // byte offsets of this lane's 16 bytes of each of its rows (rows and columns past the end repeat the last one: nothing of them is stored)
+    const unsigned pc = ((lane & 7) ^ (lane >> 3)) * 16;
+    unsigned ao[NA], wo[NW];
+#pragma unroll
+    for (int i = 0; i < NA; ++i) {
+        const int gm = m0 + (wv + i * NWV) * 8 + (lane >> 3);
+        ao[i] = (unsigned)(gm < a.B ? gm : a.B - 1) * (unsigned)(a.x_stride * 2) + pc;
+    }
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        const int r = (wv + i * NWV) * 8 + (lane >> 3), gn = SM ? n0 + r / (2 * U) * U + r % U : n0 + r;
+        wo[i] = (unsigned)(gn < a.N ? gn : a.N - 1) * (unsigned)(a.K * 2) + pc;
+    }
+    const unsigned sbase = (unsigned)(size_t)(__attribute__((address_space(3))) bf16_t*)slab_lds;
+    auto request = [&](int stage, int k0) {
+        const unsigned ls = __builtin_amdgcn_readfirstlane(sbase + stage * (STAGE * 2));
+#pragma unroll
+        for (int i = 0; i < NA; ++i) lds_dma16(a.x + k0, ao[i], ls + (wv + i * NWV) * 1024);
+#pragma unroll
+        for (int i = 0; i < NW; ++i) lds_dma16((SM && (wv + i * NWV) * 8 % (2 * U) >= U ? a.W2 : a.W) + k0, wo[i], ls + BM * 128 + (wv + i * NWV) * 1024);
+    };
+    f32x4_t acc[MT][NT], sum[MT][NT];
+#pragma unroll
+    for (int i = 0; i < MT; ++i)
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+    bf16x8_t a0[MT], w0[NT], a1[MT], w1[NT];
+    const int p0 = (fk ^ (fr & 7)) << 3, p1 = ((4 + fk) ^ (fr & 7)) << 3;
+    const int arow = (wm * MT * 16 + fr) * BK, wrow = BM * BK + (wn * NT * 16 + fr) * BK;
+    auto read = [&](const bf16_t* sp, int piece, bf16x8_t (&af)[MT], bf16x8_t (&wf)[NT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j) wf[j] = *(const bf16x8_t*)(sp + wrow + j * 16 * BK + piece);
+#pragma unroll
+        for (int i = 0; i < MT; ++i) af[i] = *(const bf16x8_t*)(sp + arow + i * 16 * BK + piece);
+    };
+    // the products of one half tile, the reads of the next one (issued in front) spread between them
+    auto multiply = [&](const bf16x8_t (&af)[MT], const bf16x8_t (&wf)[NT]) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+        constexpr int G = MT * NT / (MT + NT);
+        if constexpr (G > 0) {
+#pragma unroll
+            for (int g = 0; g < MT + NT; ++g) {
+                __builtin_amdgcn_sched_group_barrier(0x8, G, 0);        // G products,
+                __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);      // one LDS read
+            }
+            __builtin_amdgcn_sched_group_barrier(0x8, MT * NT - G * (MT + NT), 0);
+        }
+    };
+    auto fold = [&]() {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) {
+                sum[i][j] += acc[i][j];
+                acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+            }
+    };
+    const int nt = a.K / BK, klast = a.K - BK;
+#pragma unroll
+    for (int s = 0; s < S; ++s) request(s, s * BK < klast ? s * BK : klast);
+    asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * (NA + NW)) : "memory");
+    int stage = 0;
+    read(slab_lds, p0, a0, w0);
+    for (int kt = 0; kt < nt; ++kt) {
+        __builtin_amdgcn_sched_barrier(0);
+        read(slab_lds + stage * STAGE, p1, a1, w1);
+        multiply(a0, w0);
+        __builtin_amdgcn_sched_barrier(0);
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
+        const int kn = (kt + S) * BK;
+        request(stage, kn < klast ? kn : klast);
+        stage = stage == S - 1 ? 0 : stage + 1;
+        __builtin_amdgcn_sched_barrier(0);
+        read(slab_lds + stage * STAGE, p0, a0, w0);
+        multiply(a1, w1);
+        if ((kt & 3) == 3) fold();
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (the repeated last tiles: nothing may land after the block has ended)
+    if (nt & 3) fold();
+    // sum[i][j][r]: column fk * 4 + r of tile j, row fr of tile i
+    const bool vec = (a.N & 3) == 0 && (((size_t)a.y | (size_t)a.residual) & 7) == 0;
+#pragma unroll
+    for (int i = 0; i < MT; ++i) {
+        const int gm = m0 + (wm * MT + i) * 16 + fr;
+        if (gm >= a.B) continue;
+#pragma unroll
+        for (int j = 0; j < (SM ? NT / 2 : NT); ++j) {
+            const int gn = SM ? n0 + wn * U + j * 16 + fk * 4 : n0 + (wn * NT + j) * 16 + fk * 4;
+            if (gn >= a.N) continue;
+            const size_t oi = (size_t)gm * a.N + gn;
+            uint2 rs = make_uint2(0, 0);
+            if (!SM && a.residual && vec) rs = *reinterpret_cast<const uint2*>(a.residual + oi);
+            bf16_t o[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if constexpr (SM) {
+                    o[r] = f2bf(bfround(silu_c(bfround(sum[i][j][r]))) * bfround(sum[i][j + NT / 2][r]));
+                } else {
+                    float v = sum[i][j][r];
+                    const int c = gn + r < a.N ? r : 0;
+                    if (a.bias) v = v + bf2f(a.bias[gn + c]);
+                    o[r] = f2bf(v);
+                    if (EPI == EPI_SILU) o[r] = f2bf(silu_c(bf2f(o[r])));
+                    if (a.residual) {
+                        const u32 w = r < 2 ? rs.x : rs.y;
+                        o[r] = f2bf((vec ? (r & 1 ? bfhi(w) : bflo(w)) : bf2f(a.residual[oi + c])) + bf2f(o[r]));
+                    }
+                }
+            }
+            if (vec) *reinterpret_cast<uint2*>(a.y + oi) = make_uint2((u32)o[0] | ((u32)o[1] << 16), (u32)o[2] | ((u32)o[3] << 16));
+            else
+#pragma unroll
+                for (int r = 0; r < 4; ++r)
+                    if (gn + r < a.N) a.y[oi + r] = o[r];
+        }
+    }
+}
+// The norm k_splitk_reduce_rows applies to its rows, for k_gemm_slabs' outputs: its 1024 chains (column n belongs to chain n mod 1024) eight to a thread, its
+// sums in its order.  One block of two waves per row.
+__global__ __launch_bounds__(128) void k_post_norm_rows(const bf16_t* y, const bf16_t* w, bf16_t* out, int N, float eps) {
+    __shared__ float red[16];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const uint4* yr = reinterpret_cast<const uint4*>(y + (size_t)blockIdx.x * N);
+    const int nch = N >> 3;
+    float ss[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    for (int c = tid; c < nch; c += 128) {
+        const uint4 v = yr[c];
+        const u32 d[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            ss[2 * e] = fmaf(bflo(d[e]), bflo(d[e]), ss[2 * e]);
+            ss[2 * e + 1] = fmaf(bfhi(d[e]), bfhi(d[e]), ss[2 * e + 1]);
+        }
+    }
+    // butterfly over 64 chains = eight threads x eight: partners 32, 16, 8 in other threads, 4, 2, 1 in this one
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        ss[e] += __shfl_xor(ss[e], 4);
+        ss[e] += __shfl_xor(ss[e], 2);
+        ss[e] += __shfl_xor(ss[e], 1);
+    }
+    const float s4[4] = {ss[0] + ss[4], ss[1] + ss[5], ss[2] + ss[6], ss[3] + ss[7]};
+    if ((lane & 7) == 0) red[tid >> 3] = (s4[0] + s4[2]) + (s4[1] + s4[3]);
+    __syncthreads();
+    float tot = 0.0f;
+#pragma unroll
+    for (int k = 0; k < 16; ++k) tot = tot + red[k];
+    const float rinv = 1.0f / sqrtf(tot / (float)N + eps);
+    for (int c = tid; c < nch; c += 128) reinterpret_cast<uint4*>(out + (size_t)blockIdx.x * N)[c] = norm_chunk(yr[c], reinterpret_cast<const uint4*>(w)[c], rinv);
+}
+
 template <int MT, int KS, bool SM>
 static void launch_gemm_splitk_t(hipStream_t st, const LinArgs& a, float* ws, int b0, int bt, int rs, dim3 grid) {
     const size_t smem = (size_t)(16 * MT + 64) * (KS + 8) * 2;
@@ -1287,10 +1466,67 @@ static void launch_gemm_splitk_t(hipStream_t st, const LinArgs& a, float* ws, in
     }
     hipLaunchKernelGGL(kern, grid, dim3(256), smem, st, a, ws, b0, bt, rs);
 }
+// A tile of k_gemm_slabs: its size, what a block of it takes in ns (K / 64 steps of `step` beside `fixed`), and what share of that another round of blocks adds
+// (less than one where several blocks fit a CU).  us, measured inside prompts, tiles in this order (32 x 32 never was the fastest):
+// 200 rows: 4096 x 2048 13.5 11.6 16.9 20.0 31.4, 2048 x 2048 9.2 12.2 18.8 21.6 35.2, gate + up 12288 x 2048 35.7 26.7 26.7 22.4 33.5, 2048 x 6144 20.5 27.7 43 54 84;
+// 450 rows: 24.4 17.5 17.3 20.4 31.9, 14.2 12.7 19.2 22.0 35.8, 67.5 46.4 38.7 42.3 36.0, 32.8 28.4 43.2 52.4 84.1;
+// 1000 rows: 49.2 35.6 28.0 23.8 33.5, 27.5 20.4 20.6 23.9 36.8, 141 98.0 74.5 67.6 71.4, 71.0 51.0 46.3 59.4 86.5.
+struct slab_tile {
+    int bm, bn;
+    float step, fixed, next;
+};
+static const slab_tile SLAB_TILES[5] = {{64, 32, 172.f, 4000.f, 0.6f}, {64, 64, 245.f, 4700.f, 0.6f}, {128, 64, 400.f, 4600.f, 0.68f}, {128, 128, 500.f, 6000.f, 1.f},
+                                        {256, 128, 800.f, 8500.f, 1.f}};
+// the tile whose blocks are through first by that measure
+static int pick_slab_tile(int B, int Ntot, int K) {
+    int best = 0;
+    float ns = 0.f;
+    for (int i = 0; i < 5; ++i) {
+        const slab_tile& t = SLAB_TILES[i];
+        const int blocks = ((B + t.bm - 1) / t.bm) * ((Ntot + t.bn - 1) / t.bn), rounds = (blocks + 255) / 256;
+        const float v = (K / 64 * t.step + t.fixed) * (1.0f + (rounds - 1) * t.next);
+        if (i == 0 || v < ns) { best = i; ns = v; }
+    }
+    return best;
+}
+template <int BM, int BN, int WM, int WN, int S, int EPI>
+static int launch_gemm_slabs_t(hipStream_t st, const LinArgs& a) {
+    constexpr int lds = S * (BM + BN) * 128, CN = EPI == EPI_SILU_MUL ? BN / 2 : BN;
+    static_assert(lds <= 160 * 1024, "LDS of a CU");
+    const auto kern = k_gemm_slabs<BM, BN, WM, WN, S, EPI>;
+    if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
+    const int tiles = ((a.B + BM - 1) / BM) * ((a.N + CN - 1) / CN);
+    hipLaunchKernelGGL(kern, dim3((tiles + 7) & ~7), dim3(WM * WN * 64), lds, st, a);
+    return VOX_OK;
+}
+template <int EPI>
+static int launch_gemm_slabs(hipStream_t st, const LinArgs& a) {
+    switch (pick_slab_tile(a.B, EPI == EPI_SILU_MUL ? 2 * a.N : a.N, a.K)) {
+    case 0: VOX_TRY((launch_gemm_slabs_t<64, 32, 4, 1, 6, EPI>(st, a))); break;
+    case 1: VOX_TRY((launch_gemm_slabs_t<64, 64, 2, 2, 4, EPI>(st, a))); break;
+    case 2: VOX_TRY((launch_gemm_slabs_t<128, 64, 2, 2, 3, EPI>(st, a))); break;
+    case 3: VOX_TRY((launch_gemm_slabs_t<128, 128, 4, 2, 4, EPI>(st, a))); break;
+    default: VOX_TRY((launch_gemm_slabs_t<256, 128, 4, 2, 3, EPI>(st, a))); break;
+    }
+    if (EPI == EPI_STORE && a.post_nw && a.post_out)
+        hipLaunchKernelGGL(k_post_norm_rows, dim3(a.B), dim3(128), 0, st, a.y, a.post_nw, a.post_out, a.N, a.post_eps);
+    return VOX_OK;
+}
+// what k_gemm_slabs reads in whole 16-byte pieces and addresses in 32 bits, its output apart from its input (the blocks of its one launch do not wait for each other)
+template <int EPI>
+static bool gemm_slabs_ok(const LinArgs& a) {
+    const size_t at = (size_t)a.x | (size_t)a.W | (size_t)a.W2 | (size_t)(a.x_stride * 2);
+    const size_t xn = ((size_t)a.B - 1) * a.x_stride + a.K, yn = (size_t)a.B * a.N;
+    if (a.B <= 128 || a.K % 64 || (at & 15) || a.x_rows || a.x_stride < 0 || xn >= (1ull << 31) || (size_t)a.N * a.K >= (1ull << 31)) return false;
+    if (a.x < a.y + yn && a.y < a.x + xn) return false;
+    if (EPI == EPI_STORE && a.post_nw && a.post_out) return a.N % 8 == 0 && (((size_t)a.y | (size_t)a.post_nw | (size_t)a.post_out) & 15) == 0;
+    return true;
+}
 template <int EPI>
 static int launch_gemm_splitk(hipStream_t st, const LinArgs& a, float* ws, size_t ws_bytes) {
     constexpr bool SM = (EPI == EPI_SILU_MUL);
     const int Ntot = SM ? 2 * a.N : a.N;
+    if (gemm_slabs_ok<EPI>(a)) return launch_gemm_slabs<EPI>(st, a);
     for (int b0 = 0; b0 < a.B; b0 += 128) {
         const int bt = (a.B - b0) < 128 ? (a.B - b0) : 128;
         const int mt = bt <= 16 ? 1 : bt <= 32 ? 2 : bt <= 64 ? 4 : bt <= 80 ? 5 : 8;
