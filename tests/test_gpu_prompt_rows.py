@@ -1,4 +1,4 @@
-"""Prompts of more than 128 tokens: their linears (k_gemm_slabs, k_post_norm_rows) against the launches that serve fewer rows, bit for bit."""
+"""Prompts of more than 128 tokens: their linears (k_gemm_slabs, k_post_norm_rows) and attention (k_attn_prompt) against the launches that serve fewer rows, bit for bit."""
 import ctypes
 
 import numpy as np
@@ -69,3 +69,55 @@ def test_prompt_in_one_portion_and_in_many(dev, rows, H, heads, kvh, D, F, bias)
     N.lib().vox_stack_destroy(h)
     assert np.array_equal(Bits(got[0][0]), Bits(got[1][0])) and np.array_equal(Bits(got[0][1]), Bits(got[1][1]))
     assert torch.isfinite(got[0][0].float()).all()
+
+
+def attend(dev, q, kv, q_req, kvlen, indptr, indices, Hkv, page, one_by_one):  # noqa: F811
+    """vox_paged_attention on all rows at once, or on one row at a time (k_attn_partial and k_attn_merge)."""
+    from vox_serve_amd import _native as N
+    i32 = lambda v: torch.as_tensor(np.asarray(v), dtype=torch.int32).to(dev)
+    n, Hq, D = q.shape
+    out, top = torch.full_like(q, 7.0), int(max(kvlen))
+    ip, ix = i32(indptr), i32(indices)
+    ws = torch.empty(N.lib().vox_attn_workspace_bytes(n, Hq, D, top) // 4, dtype=torch.float32, device=dev)
+    for i, j in ([(0, n)] if not one_by_one else [(i, i + 1) for i in range(n)]):
+        qr, kl = i32(q_req[i:j]), i32(kvlen[i:j])
+        N.check(N.lib().vox_paged_attention(N.ctx(), N.stream(), q[i:j].data_ptr(), N.ptr(kv), N.ptr(qr), N.ptr(kl), N.ptr(ip), N.ptr(ix), out[i:j].data_ptr(), N.ptr(ws), j - i, Hq, Hkv, D,
+                                            page, top, float(D ** -0.5)))
+    torch.cuda.synchronize()
+    return out
+
+
+def prompt_case(seed, lens, ctx, page):
+    """Rows of requests behind one another: (q_req, kvlen, indptr, indices)."""
+    rng = np.random.default_rng(seed)
+    q_req, kvlen, indptr, total = [], [], [0], 0
+    for r, (n, c) in enumerate(zip(lens, ctx)):
+        q_req += [r] * n
+        kvlen += list(range(c + 1, c + n + 1))
+        total += -(-(c + n) // page)
+        indptr.append(total)
+    return q_req, kvlen, indptr, list(rng.permutation(total + 3)[:total])
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,page,lens,ctx", [(16, 8, 128, 128, [200], [0]), (4, 2, 128, 32, [1, 97, 3, 160, 33], [0, 300, 31, 7, 64]), (8, 2, 64, 24, [130, 5, 140], [11, 290, 0]),
+                                                    (6, 2, 128, 16, [170], [100]), (3, 3, 64, 8, [257], [0]), (32, 2, 128, 128, [70], [200]), (32, 8, 64, 128, [290], [0]),
+                                                    (8, 8, 128, 128, [1031], [0])])
+def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special):  # noqa: F811
+    """Several requests in a tile, tiles of 16, 8, 5, 4 and 1 rows, ragged chunks, pages that no power of two divides, four and eight waves; with infinities and NaN among keys and
+    values (single rows never read the tokens behind them), and a row without tokens in between."""
+    g = torch.Generator(device=dev).manual_seed(sum(lens))
+    q_req, kvlen, indptr, indices = prompt_case(sum(lens), lens, ctx, page)
+    q = torch.randn(len(q_req), Hq, D, generator=g, device=dev).bfloat16()
+    kv = torch.randn(max(indices) + 1, 2, page, Hkv, D, generator=g, device=dev).bfloat16()
+    if special:
+        kvlen[len(kvlen) // 2] = 0
+        for page_id in indices[:: max(1, len(indices) // 5)]:
+            kv[page_id, 1, page // 3, 0, 1] = float("inf")
+            kv[page_id, 1, page // 2, Hkv - 1, D - 2] = float("nan")
+            kv[page_id, 0, page - 1, 0, 3] = float("-inf")
+    a, b = (attend(dev, q, kv, q_req, kvlen, indptr, indices, Hkv, page, one) for one in (False, True))
+    nan = torch.isnan(a.float()) & torch.isnan(b.float())
+    same = (a.view(torch.int16) == b.view(torch.int16)) | nan
+    assert same.all(), (~same).nonzero()[:4].tolist()
+    assert special or not nan.any()

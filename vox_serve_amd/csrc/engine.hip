@@ -74,6 +74,9 @@ int vox_paged_attention(vox_ctx* ctx, void* stream, const void* q, const void* k
     c.q = q; c.kv = kv; c.q_req = q_req; c.q_kvlen = q_kvlen; c.indptr = indptr; c.indices = indices;
     c.part_o = (float*)ws; c.part_ml = (float*)ws + (size_t)Nq * Hq * mc * D; c.scale = scale; c.Nq = Nq;
     c.Hq = Hq; c.Hkv = Hkv; c.D = D; c.page_size = page_size; c.max_chunks = mc; c.max_kvlen = max_kvlen;
+    c.out = out;
+    if (vox_attn_prompt_supported(c)) return vox_launch_attn_prompt((hipStream_t)stream, c);
+    c.out = nullptr;
     VOX_TRY(vox_launch_attn_partial((hipStream_t)stream, c));
     return vox_launch_attn_merge((hipStream_t)stream, c.part_o, c.part_ml, q_kvlen, out, Nq, Hq, D, mc);
 }
@@ -263,6 +266,8 @@ static int stack_layers(vox_stack* s, hipStream_t st, void* x, void* kv, int64_t
                 VOX_TRY(vox_launch_attn_short(st, ac));      // one wave per (row, kv head), registers only
             } else if (decode_rows && !(ablate() & 1024) && vox_attn_decode8_supported(ac)) {
                 VOX_TRY(vox_launch_attn_decode8(st, ac));    // <= 256 visible tokens: every chunk and the merge in one launch
+            } else if (vox_attn_prompt_supported(ac)) {
+                VOX_TRY(vox_launch_attn_prompt(st, ac));     // prompts of more than one chunk, merge included
             } else {
                 VOX_TRY(vox_launch_attn_partial(st, ac));
                 if (mc > 1) VOX_TRY(vox_launch_attn_merge(st, part_o, part_ml, r->q_kvlen, s->attn_out, n, c.heads, c.head_dim, mc, ac.out_frag));
