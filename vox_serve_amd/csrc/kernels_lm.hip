@@ -498,30 +498,160 @@ __global__ __launch_bounds__(256) void k_gemv(LinArgs a) {
         }
 }
 
+// k_gemv for one or two rows: a block of eight waves per CU, whose waves keep the normed rows in registers and walk the columns, the next column's weights in flight under this
+// one's products.  k_gemv's waves fetch and norm the rows anew for each one or two columns: two rows at K = 4096 are 24 KB and 700 instructions beside 16 KB of weights
+// and 500.  The same sums in the same order.  A step is a column, with EPI_SILU_MUL its gate row and its up row, from K = 3072 on (PAIR false) one after the other: both
+// at once beside the next ones do not fit the registers (52 us for 38).  Bound by memory (6.0 - 6.2 TB/s where there are many columns).  us, k_gemv and now: two rows: gate / up
+// 13696 x 4096 75.5, 38.2, 8192 x 2048 15.6, 13.5, 8192 x 1024 10.4, 8.8, 3072 x 1024 6.1, 5.6; head 168960 x 4096 365, 222; q | k | v 4608 x 4096 16.1, 11.5, 4096 x 1024 5.1, 4.4;
+// 1024 x 3072 4.2, 3.8; one row: 40.4, 36.6 (13696 x 4096), 11.0, 8.9 (4608 x 4096), 7.7, 7.4 (4096 x 4096), 233, 221 (head).
+template <int BT, int KC, int PRO, int EPI>
+__global__ __launch_bounds__(512, 2) void k_gemv_walk(LinArgs a) {
+    touch_args(a);
+    constexpr bool SM = EPI == EPI_SILU_MUL, PAIR = SM && KC < 6;
+    constexpr int R = PAIR ? 2 : 1;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int step = gridDim.x * 8, pb = BT == 2 ? lane & 1 : 0;      // lanes 0 and 1 finish the two rows
+    int n = blockIdx.x * 8 + wave;
+    if (n >= a.N) return;
+    struct Step { uint4 w[R][KC]; u32 res, bias; };
+    Step s0, s1;
+    auto request = [&](Step& s, const bf16_t* W, int n) {
+#pragma unroll
+        for (int r = 0; r < R; ++r) {
+            const uint4* wr = reinterpret_cast<const uint4*>((r ? a.W2 : W) + (size_t)n * a.K);
+            if (a.keep) {
+#pragma unroll
+                for (int j = 0; j < KC; ++j) s.w[r][j] = wr[lane + 64 * j];
+            } else {
+#pragma unroll
+                for (int j = 0; j < KC; ++j) s.w[r][j] = ldg_nt(wr + lane + 64 * j);
+            }
+        }
+        if (!SM && a.residual) s.res = a.residual[(size_t)pb * a.N + n];
+        if (!SM && a.bias) s.bias = a.bias[n];
+    };
+    uint4 xv[BT][KC], nwv[KC];
+#pragma unroll
+    for (int b = 0; b < BT; ++b) {
+        const uint4* xr = x_row_ptr(a, b);
+#pragma unroll
+        for (int j = 0; j < KC; ++j) xv[b][j] = xr[lane + 64 * j];
+    }
+    if (PRO == PRO_RMSNORM) {
+        const uint4* nwp = reinterpret_cast<const uint4*>(a.nw);
+#pragma unroll
+        for (int j = 0; j < KC; ++j) nwv[j] = nwp[lane + 64 * j];
+    }
+    request(s0, a.W, n);
+    if (PRO == PRO_RMSNORM) {
+#pragma unroll
+        for (int b = 0; b < BT; ++b) {
+            float s = 0.0f;
+#pragma unroll
+            for (int j = 0; j < KC; ++j) s = sq8(xv[b][j], s);
+            s = butterfly<64>(s);
+            const float rinv = 1.0f / sqrtf(s / (float)a.K + a.eps);
+#pragma unroll
+            for (int j = 0; j < KC; ++j) {
+                xv[b][j] = norm_chunk(xv[b][j], nwv[j], rinv);
+                if (a.x_out && blockIdx.x == 0 && wave == 0) reinterpret_cast<uint4*>(a.x_out + (size_t)b * a.x_out_stride)[lane + 64 * j] = xv[b][j];
+            }
+        }
+    }
+    // the rows' products with one weight row: this lane's row (pb)
+    auto dot = [&](const uint4 (&w)[KC]) {
+        if constexpr (KC == 8)      // (opaque: unpacked ahead of the loop, the rows would take 128 registers and the weights in flight would be spilled)
+#pragma unroll
+            for (int b = 0; b < BT; ++b)
+#pragma unroll
+                for (int j = 0; j < KC; ++j) asm volatile("" : "+v"(xv[b][j].x), "+v"(xv[b][j].y), "+v"(xv[b][j].z), "+v"(xv[b][j].w));
+        float s[BT];
+#pragma unroll
+        for (int b = 0; b < BT; ++b) s[b] = 0.0f;
+#pragma unroll
+        for (int j = 0; j < KC; ++j)
+#pragma unroll
+            for (int b = 0; b < BT; ++b) s[b] = dot8(w[j], xv[b][j], s[b]);
+#pragma unroll
+        for (int b = 0; b < BT; ++b) s[b] = butterfly<64>(s[b]);
+        return pb ? s[BT - 1] : s[0];
+    };
+    auto store = [&](int n, bf16_t r) {
+        if (lane < BT) a.y[(size_t)pb * a.N + n] = r;
+    };
+    auto glu = [&](int n, float g, float u) { store(n, f2bf(bfround(silu_c(bfround(g))) * bfround(u))); };
+    auto finish = [&](const Step& s, int n) {
+        if constexpr (PAIR) {
+            const float g = dot(s.w[0]);
+            glu(n, g, dot(s.w[R - 1]));
+        } else {
+            float v = dot(s.w[0]);
+            if (a.bias) v = v + bf2f((bf16_t)s.bias);
+            bf16_t r = f2bf(v);
+            if (EPI == EPI_SILU) r = f2bf(silu_c(bf2f(r)));
+            if (a.residual) r = f2bf(bf2f((bf16_t)s.res) + bf2f(r));
+            store(n, r);
+        }
+    };
+    // (the request for the next weights and the ones that are multiplied lie in one path: the waits stay exact)
+    if constexpr (SM && !PAIR) {
+        for (; n + step < a.N; n += step) {
+            request(s1, a.W2, n);
+            const float g = dot(s0.w[0]);
+            request(s0, a.W, n + step);
+            glu(n, g, dot(s1.w[0]));
+        }
+        request(s1, a.W2, n);
+        const float g = dot(s0.w[0]);
+        glu(n, g, dot(s1.w[0]));
+    } else {
+        while (true) {
+            if (n + step >= a.N) { finish(s0, n); break; }
+            request(s1, a.W, n + step);
+            finish(s0, n);
+            n += step;
+            if (n + step >= a.N) { finish(s1, n); break; }
+            request(s0, a.W, n + step);
+            finish(s1, n);
+            n += step;
+        }
+    }
+}
+
 #ifndef VOX_GEMV_COLS      // output columns per wave (development knob; 0 = heuristic)
 #define VOX_GEMV_COLS 0
 #endif
 template <int BT, int KC, int PRO, int EPI>
 static int launch_gemv_k(hipStream_t st, const LinArgs& a) {
     constexpr bool SM = (EPI == EPI_SILU_MUL);
-    // columns per wave: enough waves to cover the 1024 SIMDs a few times over, as many bytes in flight per wave
-    // as the register file allows (R*KC 16-byte loads per lane)
-    int cols = VOX_GEMV_COLS;
-    if (cols == 0) cols = (a.N / (SM ? 1 : 1) >= 4096 && KC <= 4) ? 2 : 1;
-    if (SM) cols = cols > 2 ? 2 : cols;
-    while (cols > 1 && cols * (SM ? 2 : 1) * KC > 24) cols >>= 1;
-    if (BT >= 4 && !SM && a.N >= 2048) cols = 2;          // share the unpacked activation pairs between two weight rows
-    if (BT >= 4) while (cols > 1 && cols * (SM ? 2 : 1) * KC > 8) cols >>= 1;
-#define VOX_GV(C_)                                                                                       \
-    if (cols == C_) {                                                                                    \
-        const int gx = (a.N + 4 * C_ - 1) / (4 * C_);                                                    \
-        if (a.row_tiles > 1 && gx % 8) return vox_fail(VOX_ERR_INVALID, "gemv: row tiles need N/(4 cols) %% 8 == 0"); \
-        hipLaunchKernelGGL((k_gemv<BT, KC, (SM ? 2 * C_ : C_), PRO, EPI>), dim3(gx * (a.row_tiles > 1 ? a.row_tiles : 1)), \
-                           dim3(256), 0, st, a);                                                         \
-        return VOX_OK;                                                                                   \
+    if constexpr (BT <= 2 && KC <= 8) {
+        if (a.row_tiles <= 1) {
+            // as few steps as it takes with a block on every CU, and no more blocks than those steps need (K of more than 4096 does not fit the registers twice)
+            const int per = (a.N + 8 * a.cus - 1) / (8 * a.cus);
+            hipLaunchKernelGGL((k_gemv_walk<BT, KC, PRO, EPI>), dim3((a.N + 8 * per - 1) / (8 * per)), dim3(512), 0, st, a);
+            return VOX_OK;
+        }
     }
-    VOX_GV(1) VOX_GV(2) VOX_GV(4)
+    if constexpr (BT > 1 || KC > 8) {
+        // columns per wave: enough waves to cover the 1024 SIMDs a few times over, as many bytes in flight per wave
+        // as the register file allows (R*KC 16-byte loads per lane)
+        int cols = VOX_GEMV_COLS;
+        if (cols == 0) cols = (a.N / (SM ? 1 : 1) >= 4096 && KC <= 4) ? 2 : 1;
+        if (SM) cols = cols > 2 ? 2 : cols;
+        while (cols > 1 && cols * (SM ? 2 : 1) * KC > 24) cols >>= 1;
+        if (BT >= 4 && !SM && a.N >= 2048) cols = 2;          // share the unpacked activation pairs between two weight rows
+        if (BT >= 4) while (cols > 1 && cols * (SM ? 2 : 1) * KC > 8) cols >>= 1;
+#define VOX_GV(C_)                                                                                       \
+        if (cols == C_) {                                                                                    \
+            const int gx = (a.N + 4 * C_ - 1) / (4 * C_);                                                    \
+            if (a.row_tiles > 1 && gx % 8) return vox_fail(VOX_ERR_INVALID, "gemv: row tiles need N/(4 cols) %% 8 == 0"); \
+            hipLaunchKernelGGL((k_gemv<BT, KC, (SM ? 2 * C_ : C_), PRO, EPI>), dim3(gx * (a.row_tiles > 1 ? a.row_tiles : 1)), \
+                               dim3(256), 0, st, a);                                                         \
+            return VOX_OK;                                                                                   \
+        }
+        VOX_GV(1) VOX_GV(2) VOX_GV(4)
 #undef VOX_GV
+    }
     return vox_fail(VOX_ERR_INVALID, "gemv: no variant");
 }
 template <int PRO, int EPI>
