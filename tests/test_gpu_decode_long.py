@@ -1,0 +1,54 @@
+"""Decode attention over more than 256 tokens by a wave per chunk (k_attn_decode) against k_attn_partial and k_attn_merge, which take pages that are no multiple of 32 tokens: the
+same tokens in pages of both kinds, bit for bit.  Rows of one chunk to many, chunks that end at every kind of place, one and two heads a block, NaN in every slot that holds no token."""
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+from oracle import voxref as vr
+
+from .test_gpu_ops import Bits, T, dev  # noqa: F401  (dev: fixture)
+from .test_gpu_prompt_rows import stack
+
+pytestmark = pytest.mark.gpu
+
+LENS = [700, 1, 31, 32, 33, 257, 288, 289, 300, 511, 512, 513, 64, 95, 543, 544]
+
+
+@pytest.mark.parametrize("heads,kvh,D,rows,top,page", [(16, 8, 128, 16, 700, 32), (16, 8, 128, 17, 700, 96), (4, 2, 128, 40, 513, 128), (32, 8, 64, 8, 700, 64), (32, 8, 64, 9, 513, 32),
+                                                       (32, 2, 128, 3, 700, 128), (32, 2, 128, 9, 1000, 32)])
+def test_long_contexts_against_pages_of_sixteen(dev, heads, kvh, D, rows, top, page):  # noqa: F811
+    from vox_serve_amd import _native as N
+    H, F = 256, 512
+    lens = [top] + [min(LENS[i % len(LENS)], top) for i in range(1, rows)]
+    rng = np.random.default_rng(rows)
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x0 = T(vr.f2bf(rng.standard_normal((rows, H), dtype=np.float32)), dev)
+    past = [torch.randn(2, 2, n, kvh, D, generator=g, device=dev).bfloat16() for n in lens]      # [layer][K | V][token]
+    i32 = lambda v: torch.as_tensor(np.asarray(v), dtype=torch.int32).to(dev)
+    got = []
+    for size in (16, page):
+        per = -(-top // size)
+        perm = rng.permutation(rows * per)
+        table = perm.reshape(rows, per)
+        h, keep = stack(dev, H, heads, kvh, D, F, rows, top + 8, size, 5, False)
+        kv = torch.full((2, rows * per, 2, size, kvh, D), float("nan"), dtype=torch.bfloat16, device=dev)
+        for r, n in enumerate(lens):
+            tok = torch.arange(n - 1)
+            kv[:, torch.as_tensor(table[r])[tok // size], :, tok % size] = past[r][:, :, : n - 1].permute(2, 0, 1, 3, 4)
+        last = [n - 1 for n in lens]
+        tens = [i32(last), i32(range(rows)), i32(lens), i32([table[r][n // size] for r, n in enumerate(last)]), i32([n % size for n in last]),
+                i32(np.arange(rows + 1) * per), i32(table.reshape(-1))]
+        ptab = i32(table)
+        rs = N.Rows(*[t.data_ptr() for t in tens], rows, top, ptab.data_ptr(), per, 0, -1, 0)
+        x, y = x0.clone(), torch.empty(rows, H, dtype=torch.bfloat16, device=dev)
+        N.check(N.lib().vox_stack_forward(h, N.stream(), x.data_ptr(), y.data_ptr(), kv.data_ptr(), kv[0].numel(), ctypes.byref(rs)))
+        torch.cuda.synchronize()
+        N.lib().vox_stack_destroy(h)
+        new = torch.stack([kv[:, int(table[r][n // size]), :, n % size] for r, n in enumerate(last)])
+        assert torch.isfinite(y.float()).all() and torch.isfinite(new.float()).all()
+        got.append((Bits(y), Bits(new), int(torch.isnan(kv.float()).sum()) + sum(lens) * 4 * kvh * D == kv.numel()))
+    for a, b in zip(*got):
+        assert np.array_equal(a, b)
+    assert got[0][2]

@@ -6,7 +6,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libvoxhip.so")
-SOURCES = ["core.hip", "kernels_lm.hip", "attn_prompt.hip", "sampler.hip", "engine.hip", "codec.hip", "hybrid.hip"]
+SOURCES = ["core.hip", "kernels_lm.hip", "attn_prompt.hip", "attn_decode.hip", "sampler.hip", "engine.hip", "codec.hip", "hybrid.hip"]
 # the hybrid-mixer engine alone (context, sampler, its own kernels): what a process that only serves such a model has to compile
 HYBRID_SOURCES = ["core.hip", "sampler.hip", "hybrid.hip"]
 HYBRID_LIB = os.path.join(HERE, "libvoxhip_hybrid.so")

@@ -1,6 +1,6 @@
 // Prompt attention: many query rows of a request against the request's K / V pages.
-#include "vox_device.h"
 #include "vox_internal.h"
+#include "vox_attn.h"
 
 typedef float f32x16_t __attribute__((ext_vector_type(16)));
 
@@ -13,20 +13,6 @@ struct PromptAttnArgs {
     int Nq, Hq, Hkv, G, rows, page_size, page_shift, max_chunks;      // G: q heads per kv head; rows: query rows of a tile (16 / G)
 };
 
-// exp2_c without its branches (a lane has 8 or 16 of them, whose chains then run beside each other): the same value for every x
-__device__ __forceinline__ float exp2_flat(float x) {
-    const float n = __builtin_rintf(x), f = x - n;
-    float p = 1.52527338e-5f;
-    p = __fmaf_rn(p, f, 1.54035304e-4f);
-    p = __fmaf_rn(p, f, 1.33335581e-3f);
-    p = __fmaf_rn(p, f, 9.61812911e-3f);
-    p = __fmaf_rn(p, f, 5.55041087e-2f);
-    p = __fmaf_rn(p, f, 2.40226507e-1f);
-    p = __fmaf_rn(p, f, 6.93147181e-1f);
-    p = __fmaf_rn(p, f, 1.0f);
-    const float r = __uint_as_float(__float_as_uint(p) + ((u32)(int)n << 23));
-    return !(x > -125.0f) ? 0.0f : x >= 128.0f ? __uint_as_float(0x7f800000u) : r;
-}
 // One block per (16 columns = `rows` query rows x G heads of a kv head), NWV waves, over the rows' whole context: the outputs of k_attn_partial and k_attn_merge to
 // the bit.  Their sums are chains of fp32 fused multiply-adds, and an MFMA with K = 1 is exactly one link of such a chain for a whole tile: D[i][j] = fma(A[i], B[j],
 // C[i][j]) (rounding, denormals and infinities as v_fma_f32: 524 288 chains of 32 compared).  v_mfma_f32_16x16x1_4b takes four tiles at once (lane = tile and row or
@@ -99,7 +85,7 @@ __global__ __launch_bounds__(64 * NWV, 2) void k_attn_prompt(PromptAttnArgs a, i
     auto store = [&](int u, uint2 y) {
         const int d = mhead * D + (md + u * TC) * 4, K = a.Hq * D;
         *reinterpret_cast<uint2*>(a.out + (size_t)mrow * K + d) = y;
-        if (a.out_frag) *reinterpret_cast<uint2*>(a.out_frag + ((size_t)(mrow >> 4) * (K >> 5) + (d >> 5)) * 512 + (size_t)((mrow & 15) + 16 * ((d & 31) >> 3)) * 8 + (d & 7)) = y;
+        if (a.out_frag) *reinterpret_cast<uint2*>(a.out_frag + frag_off(mrow, d, K)) = y;
     };
     bool todo = L > 0;
     for (unsigned long long open; (open = __ballot(todo)) != 0;) {      // (the same in every wave)

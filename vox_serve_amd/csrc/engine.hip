@@ -264,6 +264,8 @@ static int stack_layers(vox_stack* s, hipStream_t st, void* x, void* kv, int64_t
             if ((ablate() & 1) || attn_in) {
             } else if (decode_rows && c.max_kvlen <= 32 && !(ablate() & 512) && vox_attn_short_supported(ac)) {
                 VOX_TRY(vox_launch_attn_short(st, ac));      // one wave per (row, kv head), registers only
+            } else if (decode_rows && !(ablate() & 1024) && vox_attn_decode_supported(ac)) {
+                VOX_TRY(vox_launch_attn_decode(st, ac));     // a wave per chunk, merge included
             } else if (decode_rows && !(ablate() & 1024) && vox_attn_decode8_supported(ac)) {
                 VOX_TRY(vox_launch_attn_decode8(st, ac));    // <= 256 visible tokens: every chunk and the merge in one launch
             } else if (vox_attn_prompt_supported(ac)) {

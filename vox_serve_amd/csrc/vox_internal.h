@@ -167,6 +167,8 @@ int vox_launch_talker_mlp(hipStream_t st, const TalkerMlpCall& c);
 bool vox_depth_step_supported(const DepthStepCall& c);
 int vox_launch_depth_step(hipStream_t st, const DepthStepCall& c);
 int vox_launch_attn_partial(hipStream_t st, const AttnCall& c);
+bool vox_attn_decode_supported(const AttnCall& c);       // decode rows, one launch for chunks and merge (attn_decode.hip)
+int vox_launch_attn_decode(hipStream_t st, const AttnCall& c);
 bool vox_attn_prompt_supported(const AttnCall& c);       // many rows that read q and their pages, merge included: out is written, the partial outputs are not (attn_prompt.hip)
 int vox_launch_attn_prompt(hipStream_t st, const AttnCall& c);
 bool vox_attn_decode8_supported(const AttnCall& c);      // decode rows, 2..8 chunks: every chunk + the merge in one launch
