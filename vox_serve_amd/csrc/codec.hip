@@ -2801,6 +2801,124 @@ void vox_mimi_destroy(vox_mimi* m) {
 }
 }  // extern "C"
 
+// LayerNorm of 512-wide fp32 rows and the linear behind it (one tap, three-term rows, EPI as k_conv_dma's) in one launch: k_layernorm_f32's sums and k_conv_dma's products to the
+// bit.  The launch between them wrote three terms of every row for 12 to 16 column blocks to read back; here each of those norms its 16 rows itself (a wave
+// per row: two of k_layernorm_f32's four waves in the halves of the wave, the other two behind them), while the weights of its columns, all of K, are on their way into
+// registers: one trip, one barrier, no step behind another.  W of the eight waves multiply, 16 columns each.  us, both launches
+// before and now: 8 rows, q | k | v 3.9 + 4.8, 6.9, with GELU 3.9 + 6.0, 8.2 (eight waves); 320 rows 4.9 + 7.8, 9.2 and 4.9 + 11.4, 14.8.
+template <int W, int EPI>
+__global__ __launch_bounds__(512) void k_ln_linear(ConvDmaArgs a, const float* x, const float* lw, const float* lb, float eps) {
+    touch_args(a);
+    constexpr int C = 512, KS = C / 32;
+    __shared__ uint4 lnl_rows[3 * 16 * (C / 8)];      // [3 terms][16 rows][C / 8 pieces], piece c of row r at c ^ (r & 7)
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), fr = lane & 15, fk = lane >> 4;
+    const int t = (int)blockIdx.x, m0 = t / a.tn * 16, n0 = (t % a.tn * W + wave) * 16;
+    const bool multiplies = W == 8 || wave < W;
+    const int j = lane & 31, hw = lane >> 5;
+    float2 v[2][2][2], w2[2][2], b2[2][2];      // [row of the wave][wave hw or hw + 2 of the norm][first or second of its two columns]
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int m = m0 + wave * 2 + i;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) v[i][p][u] = *reinterpret_cast<const float2*>(x + (size_t)(m < a.M ? m : a.M - 1) * C + 256 * u + 64 * (hw + 2 * p) + 2 * j);
+    }
+#pragma unroll
+    for (int p = 0; p < 2; ++p)
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            w2[p][u] = *reinterpret_cast<const float2*>(lw + 256 * u + 64 * (hw + 2 * p) + 2 * j);
+            b2[p][u] = *reinterpret_cast<const float2*>(lb + 256 * u + 64 * (hw + 2 * p) + 2 * j);
+        }
+    uint4 wf[KS];
+    if (multiplies) {
+        const int n = n0 + fr;
+        const uint4* wr = reinterpret_cast<const uint4*>(a.w + (size_t)(n < a.N ? n : a.N - 1) * C) + fk;
+#pragma unroll
+        for (int k = 0; k < KS; ++k) wf[k] = ldg(wr + k * 4);
+    }
+    // the sum of one of the four waves' 64 values, two to a lane: partners 32 .. 2 in other lanes, 1 in this one
+    auto wave_sum = [](float s0, float s1) {
+        s0 = xor_add<1>(xor_add<2>(xor_add<4>(xor_add<8>(xor_add<16>(s0)))));
+        s1 = xor_add<1>(xor_add<2>(xor_add<4>(xor_add<8>(xor_add<16>(s1)))));
+        return s0 + s1;
+    };
+    auto four = [&](float r0, float r1) {       // waves hw, hw + 2 -> ((0 + 1) + 2) + 3
+        const vox_u2 a0 = __builtin_amdgcn_permlane32_swap(__float_as_uint(r0), __float_as_uint(r0), false, false);
+        const vox_u2 a1 = __builtin_amdgcn_permlane32_swap(__float_as_uint(r1), __float_as_uint(r1), false, false);
+        return __uint_as_float(a0.x) + __uint_as_float(a0.y) + __uint_as_float(a1.x) + __uint_as_float(a1.y);
+    };
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        float r[2];
+#pragma unroll
+        for (int p = 0; p < 2; ++p) r[p] = wave_sum(v[i][p][0].x + v[i][p][1].x, v[i][p][0].y + v[i][p][1].y);
+        const float mean = four(r[0], r[1]) / (float)C;
+#pragma unroll
+        for (int p = 0; p < 2; ++p) {
+            float s[2] = {0.0f, 0.0f};
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                v[i][p][u].x -= mean;
+                v[i][p][u].y -= mean;
+                s[0] += v[i][p][u].x * v[i][p][u].x;
+                s[1] += v[i][p][u].y * v[i][p][u].y;
+            }
+            r[p] = wave_sum(s[0], s[1]);
+        }
+        const float rstd = rsqrtf(four(r[0], r[1]) / (float)C + eps);
+        const int row = wave * 2 + i;
+#pragma unroll
+        for (int p = 0; p < 2; ++p)
+#pragma unroll
+            for (int u = 0; u < 2; ++u) {
+                float y0 = v[i][p][u].x * rstd * w2[p][u].x + b2[p][u].x, y1 = v[i][p][u].y * rstd * w2[p][u].y + b2[p][u].y;
+                const int c = 256 * u + 64 * (hw + 2 * p) + 2 * j;
+                u32* const d = reinterpret_cast<u32*>(lnl_rows + row * (C / 8) + ((c >> 3) ^ (row & 7))) + (j & 3);
+#pragma unroll
+                for (int q = 0; q < 3; ++q) {
+                    const u32 h = pack_bf2(y0, y1);
+                    d[q * (16 * C / 2)] = h;
+                    y0 -= bflo(h);
+                    y1 -= bfhi(h);
+                }
+            }
+    }
+    __syncthreads();
+    if (!multiplies) return;
+    f32x4 acc[1][1] = {{(f32x4){0.f, 0.f, 0.f, 0.f}}};
+#pragma unroll
+    for (int k = 0; k < KS; ++k)
+#pragma unroll
+        for (int p = 2; p >= 0; --p) {
+            union { uint4 u; cbf16x8 b; } wa, xa;
+            wa.u = wf[k];
+            xa.u = lnl_rows[(p * 16 + fr) * (C / 8) + ((k * 4 + fk) ^ (fr & 7))];
+            acc[0][0] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wa.b, xa.b, acc[0][0], 0, 0, 0);
+        }
+    conv_dma_out<3, EPI, 4, 1>(a, acc, nullptr, m0 + fr, n0 + fk * 4);
+}
+template <int W, int EPI>
+static int ln_linear_launch(hipStream_t st, ConvDmaArgs& a, const float* x, const float* lw, const float* lb, float eps) {
+    a.tn = (a.N + 16 * W - 1) / (16 * W);
+    hipLaunchKernelGGL((k_ln_linear<W, EPI>), dim3((a.M + 15) / 16 * a.tn), dim3(512), 0, st, a, x, lw, lb, eps);
+    return VOX_OK;
+}
+// a: the linear's arguments, whose rows are LayerNorm(x); buf: rows for the two launches where the one does not apply
+template <int EPI>
+static int ln_linear(hipStream_t st, ConvDmaArgs& a, const float* x, const float* lw, const float* lb, float eps, float* buf) {
+    const size_t at = (size_t)a.w | (size_t)x, at8 = (size_t)lw | (size_t)lb;
+    if (a.Cin == 512 && a.n_taps == 1 && !a.state && !a.job.state && a.N % 16 == 0 && a.sn_mod % 8 == 0 && a.bias_mod % 8 == 0 && (at & 15) == 0 && (at8 & 7) == 0) {
+        // Up to 64 rows two waves multiply (all eight norm): four times the CUs fetch the weights.  Mimi chunks, us, rows of the transformer, launch pairs / two / eight waves:
+        // 2 371 / 344 / 349, 20 429 / 396 / 408, 32 422 / 389 / 401, 64 460 / 423 / 433, 80 514 / 494 / 487, 128 529 / 523 / 497, 160 627 / 638 / 583, 320 916 / 983 / 877
+        return a.M <= 64 ? ln_linear_launch<2, EPI>(st, a, x, lw, lb, eps) : ln_linear_launch<8, EPI>(st, a, x, lw, lb, eps);
+    }
+    hipLaunchKernelGGL(k_layernorm_f32, dim3(a.M), dim3(256), 0, st, x, lw, lb, buf, a.Cin, eps, 3);
+    return conv_s2(st, a, EPI);
+}
+
+
 // slots == NULL: stateless chunk (fresh state: the reference's MimiDecoder.decode); else streaming on the given state slots.
 // Activations that only convs read are S3 rows (three bf16 terms: the fp32 value), written by whatever produces them; ELU is in the
 // epilogue of the conv in front of it, a conv's history in extra blocks of the next launch (as in codec_chunk_s2).
@@ -2840,8 +2958,7 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
     L *= 2;
     for (int l = 0; l < c.num_layers; ++l) {                                                                 // h = A
         const vox_mimi_layer_w& lw = w.layers[l];
-        hipLaunchKernelGGL(k_layernorm_f32, dim3(n * L), dim3(256), 0, st, A, lw.ln1_w, lw.ln1_b, Cb, C, c.ln_eps, 3);
-        { ConvDmaArgs a = conv(lw.qkv, Cb, nullptr, 0, nullptr); a.out = Db; VOX_TRY(run(a)); }              // Db [nL, 3*dim]
+        { ConvDmaArgs a = conv(lw.qkv, Cb, nullptr, 0, nullptr); a.out = Db; VOX_TRY(ln_linear<0>(st, a, A, lw.ln1_w, lw.ln1_b, c.ln_eps, Cb)); }              // Db [nL, 3*dim]
         if (S) {
             const size_t ring = (size_t)m->max_slots * m->ring_cap * C;
             const size_t smem = ((size_t)L * D + (size_t)(c.context + L) * (D + 1) + 4 * (size_t)(c.context + L)) * 4;
@@ -2852,8 +2969,7 @@ static int mimi_run(vox_mimi* m, hipStream_t st, const int32_t* codes, int code_
                                c.context, c.max_period);
         }
         { ConvDmaArgs a = conv(lw.o, Cb, nullptr, 0, nullptr); a.res = a.out = A; a.scale = lw.scale1; VOX_TRY(run(a)); }   // h += s1 * o(attn)
-        hipLaunchKernelGGL(k_layernorm_f32, dim3(n * L), dim3(256), 0, st, A, lw.ln2_w, lw.ln2_b, Cb, C, c.ln_eps, 3);
-        { ConvDmaArgs a = conv(lw.fc1, Cb, nullptr, 0, nullptr); terms(a, Db); VOX_TRY(run(a, CONV_GELU)); }
+        { ConvDmaArgs a = conv(lw.fc1, Cb, nullptr, 0, nullptr); terms(a, Db); VOX_TRY(ln_linear<CONV_GELU>(st, a, A, lw.ln2_w, lw.ln2_b, c.ln_eps, Cb)); }
         { ConvDmaArgs a = conv(lw.fc2, Db, nullptr, 0, nullptr); a.res = a.out = A; a.scale = lw.scale2;                    // h += s2 * mlp
           if (l == c.num_layers - 1) terms(a, Cb);
           VOX_TRY(run(a)); }
