@@ -4606,9 +4606,12 @@ __global__ __launch_bounds__(256) void k_hb_win_attn_mfma(const float* q, long l
 // dims).  Pieces of a row are swizzled through the address a lane loads from, so neither operand's reads meet in a bank.  Products, weights and
 // their order are those of the form above, and so are the tiles (the kept tokens and the window's start of the 64 rows around the block's): the
 // same bits.
-// Bound by the vector work of the softmax, the products (query and weights in two terms: 64 a wave and tile) and the operand reads, about 1000 clocks
-// each per wave and tile, and by the imbalance of the first rows (up to 34 tiles a CU, 26.5 on average).  2048 rows, 16 heads of 128 over 4, window
-// 1024 + 4: 100 us staged through registers per head, 55 here (63 with page arithmetic by division and 64-bit addresses).
+// A wave asks for all of a tile's keys before its first product and for the first 32 keys' values before the softmax, whose masks are one branch a tile: it waits for
+// LDS twice a tile and not eight times.
+// Bound by the vector work of the softmax (320 instructions a wave and tile, 1280 clocks) and the products (query and weights in two terms: 64 a wave and tile, 1024
+// clocks), two waves a SIMD at most, and by the imbalance of the first rows (up to 34 tiles a CU, 26.5 on average).  2048 rows, 16 heads of 128 over 4, window 1024 + 4:
+// 100 us staged through registers per head, 55 here with page arithmetic by shifts and 32-bit addresses (63 without), 50.6 with a block's arguments read late, and 46.7
+// so (operands asked for four at a time and a branch per masked score before).
 // the larger of a column's four lanes (l ^ 16, l ^ 32)
 __device__ __forceinline__ float hb_col_max(float v) {
     const vox_u2 r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
@@ -4718,35 +4721,56 @@ __global__ __launch_bounds__(256, 2) void k_hb_win_attn_dma(const float* q, long
         if (!active || (!early && (base > wp_hi || (base + 63 < wlo_first && base >= w.keep)))) continue;
         const char *kt_s = smem_w + (c & 1) * 2 * TILE, *vt_s = kt_s + TILE;
         hb_f32x4 st[4];
+        uint4 ka[KS][4], va[CT];
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt) st[kt] = hb_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            uint4 a[4];
+        for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
             for (int kt = 0; kt < 4; ++kt)
-                a[kt] = *(const uint4*)(kt_s + (kt * 16 + col) * RB + 16 * ((ks * 4 + g4) ^ (D == 128 ? col : col >> 1)));
+                ka[ks][kt] = *(const uint4*)(kt_s + (kt * 16 + col) * RB + 16 * ((ks * 4 + g4) ^ (D == 128 ? col : col >> 1)));
+        __builtin_amdgcn_sched_barrier(0);       // (every key operand is asked for before the first product)
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) st[kt] = hb_mfma_bf16(a[kt], qh[ks], st[kt]);
+        for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
-            for (int kt = 0; kt < 4; ++kt) st[kt] = hb_mfma_bf16(a[kt], ql[ks], st[kt]);
+            for (int kt = 0; kt < 4; ++kt) st[kt] = hb_mfma_bf16(ka[ks][kt], qh[ks], st[kt]);
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt) st[kt] = hb_mfma_bf16(ka[ks][kt], ql[ks], st[kt]);
         }
+        // V^T of 32 keys: keys kk*32 + g4*4 + 0..3 and 16 above, in the order in which a lane holds its weights
+        auto values = [&](int kk, int ct) {
+            const int key = kk * 32 + g4 * 4 + (col >> 2);
+            const char* v0 = vt_s + key * RB + (col & 3) * 8 + 32 * (ct ^ (D == 128 ? key & 7 : (key >> 1) & 3));      // (the same for key + 16)
+            union { hb_i16x4 v[2]; uint4 u; } x;
+            x.v[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) hb_i16x4*)v0);
+            x.v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) hb_i16x4*)(v0 + 16 * RB));
+            return x.u;
+        };
+#pragma unroll
+        for (int ct = 0; ct < CT; ++ct) va[ct] = values(0, ct);
+        __builtin_amdgcn_sched_barrier(0);       // (and the first 32 keys' values before the softmax)
         // lane (col, g4) holds the scores of column `col` against keys base + kt*16 + g4*4 + i
         const bool full = early ? base + 63 < kept : (base + 63 <= wp_first && base >= wlo_hi);     // every row of the wave sees the whole tile
         float z[4][4], top = LOWEST;
 #pragma unroll
         for (int kt = 0; kt < 4; ++kt)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                float s = st[kt][i] * zmul;
-                if (!full) {
-                    const int key = base + kt * 16 + g4 * 4 + i;
-                    const bool see = early ? key < kept : key <= p && (key >= lo_r || key < w.keep);
-                    s = see ? s : -INFINITY;
+            for (int i = 0; i < 4; ++i) z[kt][i] = st[kt][i] * zmul;
+        if (!full) {
+            // one branch for the tile: keys of from .. last, and those below `below`
+            const int k0 = base + g4 * 4, last = (early ? kept - 1 : p) - k0, from = (early ? 0 : lo_r) - k0, below = w.keep - k0;
+#pragma unroll
+            for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int key = kt * 16 + i;
+                    z[kt][i] = (key <= last) & ((key >= from) | (key < below)) ? z[kt][i] : -INFINITY;
                 }
-                z[kt][i] = s;
-                top = fmaxf(top, s);
-            }
+        }
+#pragma unroll
+        for (int kt = 0; kt < 4; ++kt)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) top = fmaxf(top, z[kt][i]);
         top = hb_col_max(top);
         if (__ballot(top > m)) {
             const float mn = fmaxf(m, top), alpha = __builtin_amdgcn_exp2f(m - mn);
@@ -4773,27 +4797,18 @@ __global__ __launch_bounds__(256, 2) void k_hb_win_attn_dma(const float* q, long
                                 z[2 * kk + 1][3]};
             hb_split_bf16x8(v, ph[kk], plo[kk]);
         }
-        // O^T[dim][column] += V^T[dim][key] P[key][column]: keys kk*32 + g4*4 + 0..3 and 16 above, in the order in which a lane holds its weights
+        // O^T[dim][column] += V^T[dim][key] P[key][column]
 #pragma unroll
         for (int kk = 0; kk < 2; ++kk) {
-            const int key = kk * 32 + g4 * 4 + (col >> 2);
-            const char* vr = vt_s + key * RB + (col & 3) * 8;
-            const int sw0 = D == 128 ? key & 7 : (key >> 1) & 3;      // (the same for key + 16)
 #pragma unroll
-            for (int half_ct = 0; half_ct < CT; half_ct += 4) {
-                uint4 a[4];
+            for (int c0 = 0; c0 < CT; c0 += 4) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) oacc[c0 + e] = hb_mfma_bf16(va[c0 + e], ph[kk], oacc[c0 + e]);
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
-                    const char* v0 = vr + 32 * ((half_ct + e) ^ sw0);
-                    union { hb_i16x4 v[2]; uint4 u; } x;
-                    x.v[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) hb_i16x4*)v0);
-                    x.v[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) hb_i16x4*)(v0 + 16 * RB));
-                    a[e] = x.u;
+                    oacc[c0 + e] = hb_mfma_bf16(va[c0 + e], plo[kk], oacc[c0 + e]);
+                    if (kk == 0) va[c0 + e] = values(1, c0 + e);
                 }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) oacc[half_ct + e] = hb_mfma_bf16(a[e], ph[kk], oacc[half_ct + e]);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) oacc[half_ct + e] = hb_mfma_bf16(a[e], plo[kk], oacc[half_ct + e]);
             }
         }
     }
