@@ -121,3 +121,13 @@ def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, 
     same = (a.view(torch.int16) == b.view(torch.int16)) | nan
     assert same.all(), (~same).nonzero()[:4].tolist()
     assert special or not nan.any()
+
+
+@pytest.mark.parametrize("special", [False, True])
+@pytest.mark.parametrize("Hq,Hkv,D,page,lens,ctx", [(16, 8, 128, 128, [75], [0]), (4, 2, 128, 32, [5, 33, 1, 20], [0, 30, 95, 60]), (16, 8, 128, 96, [9, 16], [191, 240]),
+                                                    (32, 8, 64, 64, [20, 2], [76, 31]), (32, 8, 64, 32, [2, 12], [254, 128]), (32, 2, 128, 128, [24], [190]),
+                                                    (6, 1, 128, 32, [40], [0]), (2, 1, 64, 32, [2], [31])])
+def test_short_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special):  # noqa: F811
+    """A wave per chunk, four and eight waves: rows of one chunk to eight that end at and around a chunk's last token, several requests; with infinities and NaN, also behind
+    the last token of a row, and a row without tokens."""
+    test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special)

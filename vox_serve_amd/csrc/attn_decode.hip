@@ -1,4 +1,5 @@
-// Decode attention over long contexts: one query row per request, its new token's K / V among the rows it sees.
+// Decode attention over long contexts: one query row per request, its new token's K / V among the rows it sees.  Rows of short prompts: the same with q prepared and every
+// token's K / V in the pages.
 #include "vox_internal.h"
 #include "vox_attn.h"
 
@@ -24,8 +25,9 @@ __device__ __forceinline__ float xor_max(float s) {
 //  - V: a lane has two dims (D = 64: one) of every token; p comes by v_readlane as a scalar operand.
 // The next chunk's K rows are in flight under the softmax and P.V, its V rows under the next scores.  us a Qwen3-TTS layer of 32 rows, before and now: 2000 tokens (262 MB) 91, 55.8
 // (4.7 TB/s), 325 tokens (43 MB) 18.3, 14.8 (one chunk of a wave: the trip of its rows, 750 vector instructions, the merge).
-template <int D, int G, int NWV>
-__global__ __launch_bounds__(64 * NWV) void k_attn_decode(AttnArgs a, int nchunk) {
+// PREP: a decode row, whose q and newest k and v come from the projection (norm, RoPE and append here); else a.q and the pages hold them.
+template <int D, int G, int NWV, bool PREP>
+__global__ __launch_bounds__(64 * NWV, PREP ? 1 : 4) void k_attn_decode(AttnArgs a, int nchunk) {
     touch_args(a);
     constexpr int LPT = D / 8, TPW = 64 / LPT, NP = VOX_TC / TPW, NS = G * NP, E = (G + 1) / 2;
     extern __shared__ __attribute__((aligned(16))) char dec_lds[];      // partial outputs [nchunk][G][D] | (m, l) [nchunk][G] | weights [nchunk][G]
@@ -39,11 +41,11 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode(AttnArgs a, int nchunk
     const int HS = gridDim.x / a.Hkv, hk = blockIdx.x / HS, hs = blockIdx.x - hk * HS, row = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane % LPT, tg = lane / LPT;
     const int* const pages = a.ptab ? a.ptab + (size_t)row * a.pt_stride : a.indices + a.indptr[a.q_req[row]];
-    const int L = a.q_kvlen[row], pg_new = a.page[row], sl_new = a.slot[row];
-    const int nc = (L + VOX_TC - 1) / VOX_TC, Gf = a.Hq / a.Hkv, h0 = hk * Gf + hs * G;
+    const int L = a.q_kvlen[row], pg_new = PREP ? a.page[row] : -1, sl_new = PREP ? a.slot[row] : 0;
+    const int ncl = (L + VOX_TC - 1) / VOX_TC, nc = PREP || ncl < nchunk ? ncl : nchunk, Gf = a.Hq / a.Hkv, h0 = hk * Gf + hs * G;
     const size_t trow = (size_t)a.Hkv * D, ps = (size_t)2 * a.page_size * trow;
-    const bf16_t* const raw = a.qkv + (size_t)row * (a.Hq + 2 * a.Hkv) * D;
-    const bf16_t* const vnew = raw + (size_t)(a.Hq + a.Hkv + hk) * D;
+    const bf16_t* const raw = PREP ? a.qkv + (size_t)row * (a.Hq + 2 * a.Hkv) * D : a.q + ((size_t)row * a.Hq + h0) * D;
+    const bf16_t* const vnew = PREP ? raw + (size_t)(a.Hq + a.Hkv + hk) * D : nullptr;
     uint4 k[NP];
     u32 v[VOX_TC];                // D = 128: dims 2 lane, 2 lane + 1 of token t; D = 64: dim lane
     const u32 k_at = tg * (u32)trow + j * 8, v_at = lane * (D / 64);      // elements
@@ -65,36 +67,40 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode(AttnArgs a, int nchunk
         } else {                  // the newest token's row is the projection's, zeros behind it
             const int last = L - 1 - c * VOX_TC;
 #pragma unroll
-            for (int t = 0; t < VOX_TC; ++t, vb += trow) v[t] = dims(t < last ? vb : t == last ? vnew : reinterpret_cast<const bf16_t*>(dec_zero_row));
+            for (int t = 0; t < VOX_TC; ++t, vb += trow) v[t] = dims(t < last + !PREP ? vb : PREP && t == last ? vnew : reinterpret_cast<const bf16_t*>(dec_zero_row));
         }
     };
     float* const Sw = S[wave];
     int c = wave;
     PrepOps po;
-    int p = a.pos[row];
+    uint4 qv[G];
+    int p = PREP ? a.pos[row] : 0;
     p = p < 0 ? 0 : (p >= a.table_max_pos ? a.table_max_pos - 1 : p);
-    const float* const cs_row = a.cs ? a.cs + (size_t)p * (a.rot >> 1) * 2 : nullptr;
+    const float* const cs_row = PREP && a.cs ? a.cs + (size_t)p * (a.rot >> 1) * 2 : nullptr;
     const bf16_t* const nw = wave == G ? a.kn : a.qn;
-    if (wave <= G) po = prep_head_load<D>(wave == G ? raw + (size_t)(a.Hq + hk) * D : raw + (size_t)(h0 + wave) * D, nw, cs_row, a.rot, lane);
+    if (!PREP) {
+#pragma unroll
+        for (int g = 0; g < G; ++g) qv[g] = reinterpret_cast<const uint4*>(raw)[g * LPT + j];
+    } else if (wave <= G) po = prep_head_load<D>(wave == G ? raw + (size_t)(a.Hq + hk) * D : raw + (size_t)(h0 + wave) * D, nw, cs_row, a.rot, lane);
     const bf16_t* kb = a.kv;
     if (c < nc) {
         kb = k_rows(c);
         fetch_k(kb);
         fetch_v(c, kb);
     }
-    if (wave <= G) prep_head_apply<D>(po, nw, a.eps, cs_row, a.rot, a.interleave, Sh + wave * D, wave == G ? Knew : reinterpret_cast<bf16_t*>(Qs) + (size_t)wave * D, lane);
-    __syncthreads();
+    if (PREP && wave <= G) prep_head_apply<D>(po, nw, a.eps, cs_row, a.rot, a.interleave, Sh + wave * D, wave == G ? Knew : reinterpret_cast<bf16_t*>(Qs) + (size_t)wave * D, lane);
+    if (PREP) __syncthreads();
     float qf[G][8];
 #pragma unroll
     for (int g = 0; g < G; ++g) {
-        const uint4 q = Qs[g * LPT + j];
+        const uint4 q = PREP ? Qs[g * LPT + j] : qv[g];
         const u32 w[4] = {q.x, q.y, q.z, q.w};
 #pragma unroll
         for (int e = 0; e < 4; ++e) { qf[g][2 * e] = bflo(w[e]); qf[g][2 * e + 1] = bfhi(w[e]); }
     }
     while (c < nc) {
         const int nt = L - c * VOX_TC < VOX_TC ? L - c * VOX_TC : VOX_TC;
-        if (c == nc - 1) {        // the row's newest token is the last one
+        if (PREP && c == nc - 1) {        // the row's newest token is the last one
             const uint4 kn = reinterpret_cast<const uint4*>(Knew)[j];
 #pragma unroll
             for (int n = 0; n < NP; ++n)
@@ -130,7 +136,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode(AttnArgs a, int nchunk
         }
         const int cc = c;
         c += NWV;
-        if (c < nc) {             // (the next chunk's K rows under this one's outputs, its V rows under its scores)
+        if (PREP && c < nc) {     // (the next chunk's K rows under this one's outputs, its V rows under its scores)
             kb = k_rows(c);
             fetch_k(kb);
         }
@@ -166,7 +172,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode(AttnArgs a, int nchunk
                 if constexpr (D == 128) o1[g] = __fmaf_rn(pt, v1, o1[g]);
             }
         }
-        if (c < nc) fetch_v(c, kb);
+        if (PREP && c < nc) fetch_v(c, kb);
 #pragma unroll
         for (int g = 0; g < G; ++g) {
             float* const o = Po + ((size_t)cc * G + g) * D;
@@ -174,6 +180,7 @@ __global__ __launch_bounds__(64 * NWV) void k_attn_decode(AttnArgs a, int nchunk
             else o[lane] = o0[g];
             if (lane == (g & 1) * 32) Pml[cc * G + g] = make_float2(m[g / 2], l[g]);
         }
+        if (!PREP) break;         // (a chunk a wave)
     }
     __syncthreads();
     if (wave < G) {               // the chunks' weights against the largest of their maxima
@@ -214,10 +221,10 @@ static int decode_heads(const AttnCall& c) {
     return c.Hq * c.Nq <= 256 ? 1 : 2;
 }
 bool vox_attn_decode_supported(const AttnCall& c) { return decode_heads(c) > 0; }
-template <int D, int G, int NWV>
+template <int D, int G, int NWV, bool PREP>
 static int launch_decode(hipStream_t st, const AttnArgs& a, int Nq, int nchunk) {
     const int lds = nchunk * G * (D * 4 + 8 + 4);
-    const auto kern = k_attn_decode<D, G, NWV>;
+    const auto kern = k_attn_decode<D, G, NWV, PREP>;
     if (lds > 60 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, 150 * 1024));
     hipLaunchKernelGGL(kern, dim3(a.Hq / G, Nq), dim3(64 * NWV), lds, st, a, nchunk);
     return VOX_OK;
@@ -230,6 +237,36 @@ int vox_launch_attn_decode(hipStream_t st, const AttnCall& c) {
     a.pos = c.pos; a.page = c.page; a.slot = c.slot; a.eps = c.eps; a.rot = c.rot; a.interleave = c.interleave; a.table_max_pos = c.table_max_pos;
     a.ptab = c.ptab; a.pt_stride = c.pt_stride; a.out = (bf16_t*)c.out; a.out_frag = (bf16_t*)c.out_frag;
     const int G = decode_heads(c), nchunk = (c.max_kvlen + VOX_TC - 1) / VOX_TC;
-    if (c.D == 128) return G == 1 ? launch_decode<128, 1, 16>(st, a, c.Nq, nchunk) : launch_decode<128, 2, 8>(st, a, c.Nq, nchunk);
-    return G == 1 ? launch_decode<64, 1, 16>(st, a, c.Nq, nchunk) : launch_decode<64, 2, 8>(st, a, c.Nq, nchunk);
+    if (c.D == 128) return G == 1 ? launch_decode<128, 1, 16, true>(st, a, c.Nq, nchunk) : launch_decode<128, 2, 8, true>(st, a, c.Nq, nchunk);
+    return G == 1 ? launch_decode<64, 1, 16, true>(st, a, c.Nq, nchunk) : launch_decode<64, 2, 8, true>(st, a, c.Nq, nchunk);
+}
+
+// Rows of up to eight chunks that read q and their pages, a wave per chunk (108 registers, D = 64: 90, since no wave goes on to a next chunk), four waves a block for up to four
+// chunks.  One launch of short trips instead of k_attn_partial's barriers and a merge, but every row fetches its own K and V, where k_attn_prompt's tiles share them: by estimates
+// fitted to 2 to 250 rows behind 0 to 190 tokens.  us, k_attn_partial + merge or k_attn_prompt / this kernel, 16 heads on 8, D = 128, no context: 33 rows 7.4 / 5.1, 64 8.4 / 5.2,
+// 75 9.4 / 6.5, 96 11.6 / 6.5, 128 11.0 / 8.1, 144 13.1 / 13.5 (eight waves), 250 14.1 / 21.8; behind 100: 8 rows 7.4 / 5.1, 64 13.4 / 7.7, 128 14.1 / 14.5; 32 heads on 8, D = 64:
+// 48 7.2 / 4.7, 96 9.4 / 8.5, 128 9.7 / 9.8; 32 heads on 2: 48 10.5 / 5.4, 96 11.0 / 10.7, behind 190 24 13.6 / 9.2, 64 13.9 / 15.2.
+static bool rows_pay(const AttnCall& c, int nchunk) {
+    const float own = (float)c.Nq / (64.0f * nchunk), seen = own < 0.5f ? 1.0f - own : 0.5f;
+    const int blocks = c.Nq * c.Hq / 2, slots = nchunk > 4 ? 512 : c.D == 64 ? 1280 : 1024, rounds = (blocks + slots - 1) / slots;
+    const float waves = (float)blocks * nchunk * seen, round = c.D == 64 ? 1.7f : nchunk > 4 ? 1.9f : 2.0f;
+    const float wave = nchunk > 4 ? (c.D == 64 ? 0.0008f : 0.00105f) : c.D == 64 ? 0.00135f : 0.00155f, base = nchunk > 4 ? (c.D == 64 ? 3.2f : 4.0f) : c.D == 64 ? 1.8f : 2.1f;
+    float parts, prompt;
+    vox_attn_prompt_us(c, nchunk, parts, prompt);
+    return base + round * rounds + wave * waves < (parts < prompt ? parts : prompt);
+}
+// (one row is no prompt: it stays with k_attn_partial, the form that tests hold this one and k_attn_prompt to)
+bool vox_attn_rows_supported(const AttnCall& c) {
+    const int G = c.Hkv > 0 ? c.Hq / c.Hkv : 0, nchunk = (c.max_kvlen + VOX_TC - 1) / VOX_TC;
+    const size_t at = (size_t)c.q | (size_t)c.kv;
+    return c.q && !c.qkv && c.out && !c.ptab && !c.identity_pages && c.fixed_kvlen <= 0 && c.Nq > 1 && c.Hq == G * c.Hkv && G >= 2 && G <= 16 && G % 2 == 0 && (c.D == 128 || c.D == 64) &&
+           c.page_size % VOX_TC == 0 && nchunk > 1 && nchunk <= 8 && (at & 15) == 0 && rows_pay(c, nchunk);
+}
+int vox_launch_attn_rows(hipStream_t st, const AttnCall& c) {
+    AttnArgs a{};
+    a.q = (const bf16_t*)c.q; a.q_req = c.q_req; a.q_kvlen = c.q_kvlen; a.indptr = c.indptr; a.indices = c.indices; a.scale = c.scale; a.kv = (const bf16_t*)c.kv;
+    a.Hq = c.Hq; a.Hkv = c.Hkv; set_page_size(a, c.page_size); a.max_chunks = c.max_chunks; a.out = (bf16_t*)c.out; a.out_frag = (bf16_t*)c.out_frag;
+    const int nchunk = (c.max_kvlen + VOX_TC - 1) / VOX_TC;
+    if (c.D == 128) return nchunk <= 4 ? launch_decode<128, 2, 4, false>(st, a, c.Nq, nchunk) : launch_decode<128, 2, 8, false>(st, a, c.Nq, nchunk);
+    return nchunk <= 4 ? launch_decode<64, 2, 4, false>(st, a, c.Nq, nchunk) : launch_decode<64, 2, 8, false>(st, a, c.Nq, nchunk);
 }

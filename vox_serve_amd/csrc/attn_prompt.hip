@@ -310,11 +310,16 @@ static int prompt_blocks(const AttnCall& c) {
 // former by blocks (row, kv head, chunk; a prompt's rows see half of it), the latter by rounds of eight chunks, of which a tile's block goes through one after the other
 // while the chip may be idle.  Measured, former / latter: 16 heads on 8, D = 128, no context: 64 rows 8.6 / 10.8, 96 12.0 / 11.0; behind 1500 tokens: 2 rows 12 / 59,
 // 32 48 / 60, 64 84 / 65, 128 152 / 67; 32 heads on 8, D = 64, behind 700: 16 rows 17 / 24, 48 35 / 25; 32 heads on 2: 48 rows 14.0 / 9.5, behind 1500: 32 48 / 60, 64 81 / 65.
-static bool prompt_pays(const AttnCall& c, int nchunk) {
+void vox_attn_prompt_us(const AttnCall& c, int nchunk, float& parts, float& prompt) {
     const float G = (float)(c.Hq / c.Hkv), own = (float)c.Nq / (64.0f * nchunk), seen = own < 0.5f ? 1.0f - own : 0.5f;
-    const float former = 7.3f + 0.35f * G * c.D / 128 + (float)c.Nq * c.Hkv * nchunk * seen * (0.0018f + 0.0000038f * G * c.D);
+    parts = 7.3f + 0.35f * G * c.D / 128 + (float)c.Nq * c.Hkv * nchunk * seen * (0.0018f + 0.0000038f * G * c.D);
     const float longest = (float)((nchunk + 7) / 8), all = prompt_blocks(c) * seen * nchunk / 2048.0f;
-    return 3.0f + (4.0f + 0.04f * c.D) * (longest > all ? longest : all) < former;
+    prompt = 3.0f + (4.0f + 0.04f * c.D) * (longest > all ? longest : all);
+}
+static bool prompt_pays(const AttnCall& c, int nchunk) {
+    float parts, prompt;
+    vox_attn_prompt_us(c, nchunk, parts, prompt);
+    return prompt < parts;
 }
 bool vox_attn_prompt_supported(const AttnCall& c) {
     const int G = c.Hkv > 0 ? c.Hq / c.Hkv : 0, nchunk = (c.max_kvlen + VOX_TC - 1) / VOX_TC;

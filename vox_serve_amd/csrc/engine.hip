@@ -75,6 +75,7 @@ int vox_paged_attention(vox_ctx* ctx, void* stream, const void* q, const void* k
     c.part_o = (float*)ws; c.part_ml = (float*)ws + (size_t)Nq * Hq * mc * D; c.scale = scale; c.Nq = Nq;
     c.Hq = Hq; c.Hkv = Hkv; c.D = D; c.page_size = page_size; c.max_chunks = mc; c.max_kvlen = max_kvlen;
     c.out = out;
+    if (vox_attn_rows_supported(c)) return vox_launch_attn_rows((hipStream_t)stream, c);
     if (vox_attn_prompt_supported(c)) return vox_launch_attn_prompt((hipStream_t)stream, c);
     c.out = nullptr;
     VOX_TRY(vox_launch_attn_partial((hipStream_t)stream, c));
@@ -268,6 +269,8 @@ static int stack_layers(vox_stack* s, hipStream_t st, void* x, void* kv, int64_t
                 VOX_TRY(vox_launch_attn_decode(st, ac));     // a wave per chunk, merge included
             } else if (decode_rows && !(ablate() & 1024) && vox_attn_decode8_supported(ac)) {
                 VOX_TRY(vox_launch_attn_decode8(st, ac));    // <= 256 visible tokens: every chunk and the merge in one launch
+            } else if (vox_attn_rows_supported(ac)) {
+                VOX_TRY(vox_launch_attn_rows(st, ac));       // few rows of more than one chunk, merge included
             } else if (vox_attn_prompt_supported(ac)) {
                 VOX_TRY(vox_launch_attn_prompt(st, ac));     // prompts of more than one chunk, merge included
             } else {

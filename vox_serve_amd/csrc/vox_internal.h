@@ -169,6 +169,9 @@ int vox_launch_depth_step(hipStream_t st, const DepthStepCall& c);
 int vox_launch_attn_partial(hipStream_t st, const AttnCall& c);
 bool vox_attn_decode_supported(const AttnCall& c);       // decode rows, one launch for chunks and merge (attn_decode.hip)
 int vox_launch_attn_decode(hipStream_t st, const AttnCall& c);
+bool vox_attn_rows_supported(const AttnCall& c);         // few rows that read q and their pages, 2..8 chunks, merge included (attn_decode.hip)
+int vox_launch_attn_rows(hipStream_t st, const AttnCall& c);
+void vox_attn_prompt_us(const AttnCall& c, int nchunk, float& parts, float& prompt);      // estimates: k_attn_partial with its merge, and k_attn_prompt
 bool vox_attn_prompt_supported(const AttnCall& c);       // many rows that read q and their pages, merge included: out is written, the partial outputs are not (attn_prompt.hip)
 int vox_launch_attn_prompt(hipStream_t st, const AttnCall& c);
 bool vox_attn_decode8_supported(const AttnCall& c);      // decode rows, 2..8 chunks: every chunk + the merge in one launch
