@@ -1,4 +1,4 @@
-"""Prompts of more than 128 tokens: their linears (k_gemm_slabs, k_post_norm_rows) and attention (k_attn_prompt) against the launches that serve fewer rows, bit for bit."""
+"""Prompts: their linears (k_gemm_slabs, k_post_norm_rows) and attention (k_attn_prompt, k_attn_decode) against the launches that serve fewer rows, bit for bit."""
 import ctypes
 
 import numpy as np
@@ -131,3 +131,25 @@ def test_short_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens,
     """A wave per chunk, four and eight waves: rows of one chunk to eight that end at and around a chunk's last token, several requests; with infinities and NaN, also behind
     the last token of a row, and a row without tokens."""
     test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special)
+
+
+@pytest.mark.parametrize("rows,N,K,tile", [(33, 151, 1152, 0), (65, 130, 640, 0), (129, 2048, 128, 0), (300, 2050, 1152, 1), (450, 2050, 1152, 2), (1000, 2048, 640, 2), (520, 4100, 640, 3),
+                                           (257, 6000, 384, 3)])
+def test_linears_of_many_rows_against_portions(dev, rows, N, K, tile):  # noqa: F811
+    """vox_linear on all rows (k_gemm_slabs with four chains, every tile) and on portions of at most 24 (k_linear_mfma): ragged rows and columns, one k-tile pair to many, with and
+    without SiLU, bias and residual."""
+    from vox_serve_amd import _native as NV
+    g = torch.Generator(device=dev).manual_seed(rows + tile)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
+    W, b, x, res = rnd(N, K), rnd(N), rnd(rows, K), rnd(rows, N)
+    cuts = np.cumsum([0] + [len(p) for p in np.array_split(np.arange(rows), -(-rows // 24))])
+    for act, bias, residual in [(0, b, res), (1, b, None), (1, None, res), (0, None, None)]:
+        ys = []
+        for bounds in ([0, rows], list(cuts)):
+            y = torch.full((rows, N), 7.0, dtype=torch.bfloat16, device=dev)
+            for i, j in zip(bounds, bounds[1:]):
+                NV.check(NV.lib().vox_linear(NV.ctx(), NV.stream(), NV.ptr(W), NV.ptr(bias) if bias is not None else None, x[i:j].data_ptr(),
+                                             residual[i:j].data_ptr() if residual is not None else None, y[i:j].data_ptr(), j - i, N, K, act))
+            torch.cuda.synchronize()
+            ys.append(Bits(y))
+        assert np.array_equal(*ys), (act, bias is not None, residual is not None)

@@ -1411,9 +1411,13 @@ __global__ __launch_bounds__(1024) void k_splitk_reduce_rows(const float* part, 
 // registers, so tile t's stage may be requested anew.  The weights are the first operand (a lane then holds four neighbouring columns of a row).  Blocks of one
 // XCD (block id modulo 8) take neighbouring tiles, 1024 rows deep, so that its L2 holds what they share.
 // EPI_SILU_MUL: the block's columns are BN / 2 gate rows and the BN / 2 up rows beside them, interleaved by U so that a lane owns both.
-template <int BM, int BN, int WM, int WN, int S, int EPI>
+// FOUR: k_linear_mfma's sums instead (step s of K belongs to chain s % 4, the chains added in order; K a multiple of 128), every chain in registers.  k_linear_mfma walks
+// its rows 32 at a time in a block per 16 columns.  us a linear of 2048 x 2048 with SiLU, before and now: 33 rows 11.7, 9.6, 75 19.5, 9.9,
+// 129 29.6, 9.9, 400 82, 13.0, 1000 241, 21.5 (an eighth of a Qwen3-TTS prompt of 1000 tokens was the two of its text projection).
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool FOUR>
 __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
     touch_args(a);
+    static_assert(!FOUR || EPI != EPI_SILU_MUL, "plain outputs");
     constexpr bool SM = EPI == EPI_SILU_MUL;
     constexpr int BK = 64, NWV = WM * WN, MT = BM / WM / 16, NT = BN / WN / 16, CN = SM ? BN / 2 : BN, NA = BM / 8 / NWV, NW = BN / 8 / NWV;
     constexpr int STAGE = (BM + BN) * BK, U = NT * 8;       // U: gate (up) columns of a wave
@@ -1448,11 +1452,16 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
 #pragma unroll
         for (int i = 0; i < NW; ++i) lds_dma16((SM && (wv + i * NWV) * 8 % (2 * U) >= U ? a.W2 : a.W) + k0, wo[i], ls + BM * 128 + (wv + i * NWV) * 1024);
     };
-    f32x4_t acc[MT][NT], sum[MT][NT];
+    constexpr int CH = FOUR ? 4 : 1;
+    f32x4_t acc[CH][MT][NT], sum[MT][NT];
 #pragma unroll
     for (int i = 0; i < MT; ++i)
 #pragma unroll
-        for (int j = 0; j < NT; ++j) acc[i][j] = sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < NT; ++j) {
+            sum[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int c = 0; c < CH; ++c) acc[c][i][j] = sum[i][j];
+        }
     bf16x8_t a0[MT], w0[NT], a1[MT], w1[NT];
     const int p0 = (fk ^ (fr & 7)) << 3, p1 = ((4 + fk) ^ (fr & 7)) << 3;
     const int arow = (wm * MT * 16 + fr) * BK, wrow = BM * BK + (wn * NT * 16 + fr) * BK;
@@ -1463,11 +1472,11 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
         for (int i = 0; i < MT; ++i) af[i] = *(const bf16x8_t*)(sp + arow + i * 16 * BK + piece);
     };
     // the products of one half tile, the reads of the next one (issued in front) spread between them
-    auto multiply = [&](const bf16x8_t (&af)[MT], const bf16x8_t (&wf)[NT]) {
+    auto multiply = [&](const bf16x8_t (&af)[MT], const bf16x8_t (&wf)[NT], f32x4_t (&sums)[MT][NT]) {
 #pragma unroll
         for (int j = 0; j < NT; ++j)
 #pragma unroll
-            for (int i = 0; i < MT; ++i) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], acc[i][j], 0, 0, 0);
+            for (int i = 0; i < MT; ++i) sums[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[j], af[i], sums[i][j], 0, 0, 0);
         constexpr int G = MT * NT / (MT + NT);
         if constexpr (G > 0) {
 #pragma unroll
@@ -1483,8 +1492,8 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
         for (int j = 0; j < NT; ++j)
 #pragma unroll
             for (int i = 0; i < MT; ++i) {
-                sum[i][j] += acc[i][j];
-                acc[i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
+                sum[i][j] += acc[0][i][j];
+                acc[0][i][j] = (f32x4_t){0.f, 0.f, 0.f, 0.f};
             }
     };
     const int nt = a.K / BK, klast = a.K - BK;
@@ -1493,10 +1502,11 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
     asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"((S - 1) * (NA + NW)) : "memory");
     int stage = 0;
     read(slab_lds, p0, a0, w0);
-    for (int kt = 0; kt < nt; ++kt) {
+    auto step = [&](auto CHAIN, int kt) {
+        constexpr int c0 = decltype(CHAIN)::value, c1 = FOUR ? c0 + 1 : 0;
         __builtin_amdgcn_sched_barrier(0);
         read(slab_lds + stage * STAGE, p1, a1, w1);
-        multiply(a0, w0);
+        multiply(a0, w0, acc[c0]);
         __builtin_amdgcn_sched_barrier(0);
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"((S - 2) * (NA + NW)) : "memory");
         const int kn = (kt + S) * BK;
@@ -1504,11 +1514,28 @@ __global__ __launch_bounds__(WM * WN * 64, 2) void k_gemm_slabs(LinArgs a) {
         stage = stage == S - 1 ? 0 : stage + 1;
         __builtin_amdgcn_sched_barrier(0);
         read(slab_lds + stage * STAGE, p0, a0, w0);
-        multiply(a1, w1);
-        if ((kt & 3) == 3) fold();
+        multiply(a1, w1, acc[c1]);
+    };
+    if constexpr (FOUR) {
+        for (int kt = 0; kt < nt; kt += 2) {
+            step(vox_ic<0>{}, kt);
+            step(vox_ic<2>{}, kt + 1);
+        }
+    } else {
+        for (int kt = 0; kt < nt; ++kt) {
+            step(vox_ic<0>{}, kt);
+            if ((kt & 3) == 3) fold();
+        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // (the repeated last tiles: nothing may land after the block has ended)
-    if (nt & 3) fold();
+    if constexpr (FOUR) {
+#pragma unroll
+        for (int j = 0; j < NT; ++j)
+#pragma unroll
+            for (int i = 0; i < MT; ++i) sum[i][j] = ((acc[0][i][j] + acc[1][i][j]) + acc[2][i][j]) + acc[CH - 1][i][j];
+    } else if (nt & 3) {
+        fold();
+    }
     // sum[i][j][r]: column fk * 4 + r of tile j, row fr of tile i
     const bool vec = (a.N & 3) == 0 && (((size_t)a.y | (size_t)a.residual) & 7) == 0;
 #pragma unroll
@@ -1604,10 +1631,10 @@ struct slab_tile {
 static const slab_tile SLAB_TILES[5] = {{64, 32, 172.f, 4000.f, 0.6f}, {64, 64, 245.f, 4700.f, 0.6f}, {128, 64, 400.f, 4600.f, 0.68f}, {128, 128, 500.f, 6000.f, 1.f},
                                         {256, 128, 800.f, 8500.f, 1.f}};
 // the tile whose blocks are through first by that measure
-static int pick_slab_tile(int B, int Ntot, int K) {
+static int pick_slab_tile(int B, int Ntot, int K, int tiles = 5) {
     int best = 0;
     float ns = 0.f;
-    for (int i = 0; i < 5; ++i) {
+    for (int i = 0; i < tiles; ++i) {
         const slab_tile& t = SLAB_TILES[i];
         const int blocks = ((B + t.bm - 1) / t.bm) * ((Ntot + t.bn - 1) / t.bn), rounds = (blocks + 255) / 256;
         const float v = (K / 64 * t.step + t.fixed) * (1.0f + (rounds - 1) * t.next);
@@ -1615,11 +1642,11 @@ static int pick_slab_tile(int B, int Ntot, int K) {
     }
     return best;
 }
-template <int BM, int BN, int WM, int WN, int S, int EPI>
+template <int BM, int BN, int WM, int WN, int S, int EPI, bool FOUR = false>
 static int launch_gemm_slabs_t(hipStream_t st, const LinArgs& a) {
     constexpr int lds = S * (BM + BN) * 128, CN = EPI == EPI_SILU_MUL ? BN / 2 : BN;
     static_assert(lds <= 160 * 1024, "LDS of a CU");
-    const auto kern = k_gemm_slabs<BM, BN, WM, WN, S, EPI>;
+    const auto kern = k_gemm_slabs<BM, BN, WM, WN, S, EPI, FOUR>;
     if (lds > 64 * 1024) VOX_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds));
     const int tiles = ((a.B + BM - 1) / BM) * ((a.N + CN - 1) / CN);
     hipLaunchKernelGGL(kern, dim3((tiles + 7) & ~7), dim3(WM * WN * 64), lds, st, a);
@@ -1639,14 +1666,29 @@ static int launch_gemm_slabs(hipStream_t st, const LinArgs& a) {
     return VOX_OK;
 }
 // what k_gemm_slabs reads in whole 16-byte pieces and addresses in 32 bits, its output apart from its input (the blocks of its one launch do not wait for each other)
-template <int EPI>
-static bool gemm_slabs_ok(const LinArgs& a) {
+static bool slab_operands_ok(const LinArgs& a) {
     const size_t at = (size_t)a.x | (size_t)a.W | (size_t)a.W2 | (size_t)(a.x_stride * 2);
     const size_t xn = ((size_t)a.B - 1) * a.x_stride + a.K, yn = (size_t)a.B * a.N;
-    if (a.B <= 128 || a.K % 64 || (at & 15) || a.x_rows || a.x_stride < 0 || xn >= (1ull << 31) || (size_t)a.N * a.K >= (1ull << 31)) return false;
-    if (a.x < a.y + yn && a.y < a.x + xn) return false;
+    if (a.K % 64 || (at & 15) || a.x_rows || a.x_stride < 0 || xn >= (1ull << 31) || (size_t)a.N * a.K >= (1ull << 31)) return false;
+    return !(a.x < a.y + yn && a.y < a.x + xn);
+}
+template <int EPI>
+static bool gemm_slabs_ok(const LinArgs& a) {
+    if (a.B <= 128 || !slab_operands_ok(a)) return false;
     if (EPI == EPI_STORE && a.post_nw && a.post_out) return a.N % 8 == 0 && (((size_t)a.y | (size_t)a.post_nw | (size_t)a.post_out) & 15) == 0;
     return true;
+}
+// The same tiles with k_linear_mfma's sums (all but the largest, whose four chains the registers do not hold), where that kernel would go over its weights more than once (2048 x 2048
+// with SiLU, us, that kernel and this one: 17 rows 7.8, 9.5, 32 8.2, 9.5, 33 11.7, 9.6; 4096 x 4096 32 15.1, 14.9, 33 25.4, 15.0).
+static bool gemm_chains_ok(const LinArgs& a) { return a.B > 32 && a.K % 128 == 0 && !a.x_out && slab_operands_ok(a); }
+template <int EPI>
+static int launch_gemm_chains(hipStream_t st, const LinArgs& a) {
+    switch (pick_slab_tile(a.B, a.N, a.K, 4)) {
+    case 0: return launch_gemm_slabs_t<64, 32, 4, 1, 6, EPI, true>(st, a);
+    case 1: return launch_gemm_slabs_t<64, 64, 2, 2, 4, EPI, true>(st, a);
+    case 2: return launch_gemm_slabs_t<128, 64, 2, 2, 3, EPI, true>(st, a);
+    default: return launch_gemm_slabs_t<128, 128, 4, 2, 4, EPI, true>(st, a);
+    }
 }
 template <int EPI>
 static int launch_gemm_splitk(hipStream_t st, const LinArgs& a, float* ws, size_t ws_bytes) {
@@ -2494,6 +2536,8 @@ int vox_launch_linear(vox_ctx* ctx, hipStream_t st, const LinearCall& call) {
     if (c.B > c.exact_rows && !c.fixed_order && c.pro != PRO_ATTN && c.K % 32 == 0) {   // above exact_rows: MFMA path (weights streamed once per 32-row tile)
         static const bool stream_frag = [] { const char* e = getenv("VOX_STREAM_FRAG"); return !(e && e[0] == '0'); }();     // (=0: row-major weights, A/B timing)
         if (stream_frag && c.W_frag && c.B <= 16 && c.pro == PRO_COPY && c.epi != EPI_SILU_MUL && vox_stream_weight_ok(c.N, c.K)) a.W_frag = (const bf16_t*)c.W_frag;
+        if (c.pro == PRO_COPY && (c.epi == EPI_STORE || c.epi == EPI_SILU) && gemm_chains_ok(a))
+            return c.epi == EPI_SILU ? launch_gemm_chains<EPI_SILU>(st, a) : launch_gemm_chains<EPI_STORE>(st, a);
 #define VOX_PM(P, E) if (c.pro == P && c.epi == E) return launch_linear_mfma_pe<P, E>(st, a);
         VOX_PM(PRO_COPY, EPI_STORE) VOX_PM(PRO_COPY, EPI_SILU) VOX_PM(PRO_COPY, EPI_SILU_MUL)
         VOX_PM(PRO_RMSNORM, EPI_STORE) VOX_PM(PRO_RMSNORM, EPI_SILU_MUL)
