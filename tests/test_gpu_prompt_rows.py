@@ -12,22 +12,26 @@ from .test_gpu_ops import Bits, T, dev  # noqa: F401  (dev: fixture)
 pytestmark = pytest.mark.gpu
 
 
-def stack(dev, H, heads, kvh, D, F, rows, tokens, page, seed, bias):  # noqa: F811
+def stack(dev, H, heads, kvh, D, F, rows, tokens, page, seed, bias, norm=False, skew=0):  # noqa: F811
     from vox_serve_amd import _native as N
     from vox_serve_amd.engine import StackCfg, _stack_config, rope_table
     rng = np.random.default_rng(seed)
     w = lambda *s: T(vr.f2bf(rng.standard_normal(s, dtype=np.float32) * np.float32(0.05)), dev)
     g = lambda n: T(vr.f2bf(1 + 0.1 * rng.standard_normal(n).astype(np.float32)), dev)
-    c = StackCfg(H, 2, heads, kvh, D, F, 1e-6, 1e6, 1.0, None, False, None, False, bias)
+    c = StackCfg(H, 2, heads, kvh, D, F, 1e-6, 1e6, 1.0, None, norm, None, False, bias)
     arr, keep = (N.LayerWeights * 2)(), []
     for l in range(2):
         ts = dict(wqkv=w((heads + 2 * kvh) * D, H), wo=w(H, heads * D), wgate=w(F, H), wup=w(F, H), wdown=w(H, F), ln1=g(H), ln2=g(H))
         if bias:
             ts["bqkv"] = w((heads + 2 * kvh) * D)
+        if norm:
+            ts.update(qnorm=g(D), knorm=g(D))
         for k, v in ts.items():
             keep.append(v)
             setattr(arr[l], k, v.data_ptr())
     fn, rope = g(H), rope_table(tokens, c, dev)
+    if skew:      # the table `skew` floats off a 16-byte boundary
+        rope = torch.cat([rope.new_zeros(skew), rope.reshape(-1)])[skew:]
     sc, h = _stack_config(c, page, rows, tokens), ctypes.c_void_p()
     N.check(N.lib().vox_stack_create(N.ctx(), ctypes.byref(sc), arr, fn.data_ptr(), rope.data_ptr(), tokens, ctypes.byref(h)))
     return h, keep + [fn, rope]
@@ -153,3 +157,19 @@ def test_linears_of_many_rows_against_portions(dev, rows, N, K, tile):  # noqa: 
             torch.cuda.synchronize()
             ys.append(Bits(y))
         assert np.array_equal(*ys), (act, bias is not None, residual is not None)
+
+
+@pytest.mark.parametrize("heads,kvh,D,norm,bias", [(16, 8, 128, True, False), (3, 1, 128, False, True), (14, 2, 64, False, True), (32, 8, 64, True, False)])
+def test_heads_of_a_row_together(dev, heads, kvh, D, norm, bias):  # noqa: F811
+    """k_head_rows against k_head_prepare, which takes RoPE tables that lie on no 16 bytes: hidden rows and cache bit for bit; heads that fill a block and that do not."""
+    rows, H, page = 40, 256, 32
+    x = T(vr.f2bf(np.random.default_rng(3).standard_normal((rows, H), dtype=np.float32)), dev)
+    got = []
+    for skew in (0, 2):
+        h, keep = stack(dev, H, heads, kvh, D, 512, rows, 64, page, 9, bias, norm, skew)
+        kv = torch.zeros(2, 3, 2, page, kvh, D, dtype=torch.bfloat16, device=dev)
+        got.append((Bits(forward(dev, h, x, kv, page, kvh, D, [rows], [2, 0])), Bits(kv)))
+        from vox_serve_amd import _native as N
+        N.lib().vox_stack_destroy(h)
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+    assert np.abs(vr.bf2f(got[0][1])).max() > 0.01
