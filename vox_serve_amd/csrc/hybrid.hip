@@ -323,21 +323,39 @@ struct hb_post {
     float eps;
     int rms;
     bf16_t* x16;            // the new rows as bf16 too, at the stride of x (register form), or NULL
+    // the output is still in parts: y[row] = sum_k wgt[row * top + k] * eo[row * top + k] (register form; y only says that there is one)
+    const float *eo, *wgt;
+    int top, unweighted;
 };
 // NC > 0: rows of at most 1024 * NC columns whose operands lie on 16-byte boundaries; thread t owns the columns 4t .. 4t+3 of every 1024,
 // everything is requested at the start and the new row stays in its registers (out) as well as in xo (NULL: not written)
-template <int NC> __device__ __forceinline__ void hb_post_row(const hb_post& p, int row, const float* xr, float* xo, long ldx, int W, float (*red)[4], float4 (&out)[NC]) {
+template <int NC, bool PARTS = false> __device__ __forceinline__ void hb_post_row(const hb_post& p, int row, const float* xr, float* xo, long ldx, int W, float (*red)[4], float4 (&out)[NC]) {
     const float* yr = p.y + (size_t)row * p.ldy;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     float4 y[NC], g[NC], b[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         const int k = threadIdx.x * 4 + 1024 * i, kc = k < W ? k : 0;
-        y[i] = *(const float4*)(yr + kc);
+        y[i] = PARTS ? make_float4(0.f, 0.f, 0.f, 0.f) : *(const float4*)(yr + kc);
         out[i] = *(const float4*)(xr + kc);
         g[i] = *(const float4*)(p.w + kc);
         b[i] = p.b ? *(const float4*)(p.b + kc) : make_float4(0.f, 0.f, 0.f, 0.f);
         if (k >= W) y[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    if constexpr (PARTS) {      // k_hb_moe_combine's sums
+#pragma unroll 2
+        for (int e = 0; e < p.top; ++e) {
+            const size_t en = (size_t)row * p.top + e;
+            const float w = p.unweighted ? 1.0f : p.wgt[en];
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                const int k = threadIdx.x * 4 + 1024 * i;
+                const float4 v = *(const float4*)(p.eo + en * W + (k < W ? k : 0));
+                if (k < W) y[i] = make_float4(fmaf(w, v.x, y[i].x), fmaf(w, v.y, y[i].y), fmaf(w, v.z, y[i].z), fmaf(w, v.w, y[i].w));
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < NC; ++i) y[i] = make_float4(0.f + y[i].x, 0.f + y[i].y, 0.f + y[i].z, 0.f + y[i].w);
     }
     float mean = 0.f;
     if (!p.rms) {
@@ -400,17 +418,19 @@ static int hb_post_pieces(const hb_post& p, const float* x, long ldx, int W) {
     if ((W & 3) || (ldx & 3) || (p.ldy & 3) || W > 4096 || (((size_t)p.y | (size_t)x | (size_t)p.w | (size_t)p.b) & 15)) return 0;
     return W <= 1024 ? 1 : (W <= 2048 ? 2 : 4);
 }
-template <int NC> __global__ __launch_bounds__(256) void k_hb_post_norm(hb_post p, float* x, long ldx, int W) {
+// PARTS: the routed sum in front of the norm (k_hb_moe_combine's, which wrote 4 bytes a value for this launch to read).  2048 rows of 2048, two choices, us: 12.0 + 12.0 apart, 14.3 so.
+template <int NC, bool PARTS = false> __global__ __launch_bounds__(256) void k_hb_post_norm(hb_post p, float* x, long ldx, int W) {
     __shared__ float red[2][4];
     float* xr = x + (size_t)blockIdx.x * ldx;
     if constexpr (NC > 0) {
         float4 out[NC];
-        hb_post_row<NC>(p, blockIdx.x, xr, xr, ldx, W, red, out);
+        hb_post_row<NC, PARTS>(p, blockIdx.x, xr, xr, ldx, W, red, out);
     } else hb_post_row_any(p, blockIdx.x, xr, W, red);
 }
 static void hb_post_norm(hipStream_t st, int n, const hb_post& p, float* x, long ldx, int W) {
     const int nc = hb_post_pieces(p, x, ldx, W);
     auto kern = nc == 1 ? k_hb_post_norm<1> : nc == 2 ? k_hb_post_norm<2> : nc == 4 ? k_hb_post_norm<4> : k_hb_post_norm<0>;
+    if (p.eo) kern = nc == 1 ? k_hb_post_norm<1, true> : nc == 2 ? k_hb_post_norm<2, true> : k_hb_post_norm<4, true>;      // (hb_moe: nc > 0)
     hipLaunchKernelGGL(kern, dim3(n), dim3(256), 0, st, p, x, ldx, W);
 }
 
@@ -1234,6 +1254,7 @@ static void hb_settle(hipStream_t st, hb_pending& pd, int n, int W) {
     hb_post_norm(st, n, pd.p, pd.x, pd.ldx, W);
     pd.x16 = pd.p.x16;
     pd.p.y = nullptr;
+    pd.p.eo = nullptr;
 }
 
 // 2..16 rows, bf16: one MFMA row tile; a block owns 16 output columns and its eight waves take the 32-wide k-steps w, w + 8, ...
@@ -6331,9 +6352,11 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
 }
 
 // Routed feed-forward of the rows h2 (first completed by `post` when it names a sublayer's output), added to cur.  Few rows: one GEMV pair per routed entry; more: the entries are
-// listed per expert and every expert multiplies its own rows in one tile launch.
+// listed per expert and every expert multiplies its own rows in one tile launch.  parts != NULL: the norm that alone reads the result (rows h2, stride ldh, are its stream); where
+// it can add the routed outputs itself they stay in parts, and it says so.
 template <typename T>
-static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, const float* h2, long ldh, hb_post post, float* cur, long ldx, int n, hb_join jn) {
+static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, const float* h2, long ldh, hb_post post, float* cur, long ldx, int n, hb_join jn,
+                  hb_post* parts) {
     const vox_hybrid_moe& E = *L.moe;
     jn.scale = L.ls2;
     if (L.res_gate) { jn.gate = m->rgate; jn.ldg = m->cfg.width; }
@@ -6380,6 +6403,13 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
         VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(m->ws16, st, m->moe_act, (long)ff, (const T*)E.w_down, nullptr, m->moe_out, (long)W, n, W, ff, down, E.experts, rows, ne));
     }
     const int vec = !m->ws16.general && !(W & 3) && !(ldx & 3) && !(ldh & 3) && !(((size_t)cur | (size_t)h2 | (size_t)m->moe_out) & 15) ? 1 : 0;
+    if (parts && vec && top > 0 && E.identity == 0 && E.shared_ff == 0 && jn.store && !jn.gate && !jn.scale && jn.streams == 0 && hb_post_pieces(*parts, h2, ldh, W) > 0) {
+        parts->eo = m->moe_out;
+        parts->wgt = m->moe_wgt;
+        parts->top = top;
+        parts->unweighted = E.scale_input;
+        return VOX_OK;
+    }
     hipLaunchKernelGGL(k_hb_moe_combine, dim3(n), dim3(256), 0, st, cur, ldx, h2, ldh, m->moe_out, m->moe_sel, m->moe_wgt, top, E.experts, W,
                        E.scale_input, jn, vec);
     if (E.shared_ff > 0) {
@@ -6467,12 +6497,15 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
         if (L.sibling >= 0)
             VOX_TRY(hb_mixer<T>(m, st, io, m->layers[L.sibling], run.side_cache, run.side_pool, run.side_state, hn, W, src, lds_x, cur, ldx, n, n_req,
                                 max_kvlen, j1));
+        hb_post parts{};      // the second sublayer's norm, its routed outputs perhaps still apart
         if (L.moe) {
             if (!parallel && !post) hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h2, nullptr, nullptr, (long)W, L.norm2_b);
             hb_post p1 = pd.p;
             if (p1.y) { p1.x16 = pd.buf16; pd.x16 = nullptr; }
             pd.p.y = nullptr;
-            VOX_TRY(hb_moe<T>(m, st, L, post ? pd.x : hf, ldf, post ? p1 : none, dst, ldd, n, j2));
+            hb_post p2 = post2;
+            VOX_TRY(hb_moe<T>(m, st, L, post ? pd.x : hf, ldf, post ? p1 : none, dst, ldd, n, j2, post && n > 1 ? &p2 : nullptr));
+            parts = p2;
         } else if (L.ff > 0 && L.ff_kind == VOX_FF_GATED) {
             // down(act(gate h + b) * (up h + b)) + b: gate and up rows in one product, the activation in place behind it
             if (!parallel && !post) hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h2, nullptr, nullptr, (long)W, L.norm2_b);
@@ -6525,7 +6558,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->ff, nf, (const T*)L.w_down, nullptr, dst, ldd, n, W, L.ff, j2));
         }
         if (post) {
-            if (has_ff) pd.p = post2;
+            if (has_ff) pd.p = L.moe ? parts : post2;
             if (io->trace) hb_settle(st, pd, n, W);
             cur = pd.x;
             other = pd.x_next;
