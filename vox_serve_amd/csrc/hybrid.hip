@@ -323,20 +323,25 @@ struct hb_post {
     float eps;
     int rms;
     bf16_t* x16;            // the new rows as bf16 too, at the stride of x (register form), or NULL
-    // the output is still in parts: y[row] = sum_k wgt[row * top + k] * eo[row * top + k] (register form; y only says that there is one)
+};
+// The output still in parts: y[row] = sum_k wgt[row * top + k] * eo[row * top + k] (register form; hb_post's y then only says that there is one).
+// (apart from hb_post, which the kernels of a step of few rows take by value)
+struct hb_parts {
     const float *eo, *wgt;
     int top, unweighted;
 };
 // NC > 0: rows of at most 1024 * NC columns whose operands lie on 16-byte boundaries; thread t owns the columns 4t .. 4t+3 of every 1024,
 // everything is requested at the start and the new row stays in its registers (out) as well as in xo (NULL: not written)
-template <int NC, bool PARTS = false> __device__ __forceinline__ void hb_post_row(const hb_post& p, int row, const float* xr, float* xo, long ldx, int W, float (*red)[4], float4 (&out)[NC]) {
+template <int NC, bool PARTS = false> __device__ __forceinline__ void hb_post_row(const hb_post& p, int row, const float* xr, float* xo, long ldx, int W, float (*red)[4], float4 (&out)[NC],
+                                                                                         const hb_parts& q = hb_parts{}) {
     const float* yr = p.y + (size_t)row * p.ldy;
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     float4 y[NC], g[NC], b[NC];
 #pragma unroll
     for (int i = 0; i < NC; ++i) {
         const int k = threadIdx.x * 4 + 1024 * i, kc = k < W ? k : 0;
-        y[i] = PARTS ? make_float4(0.f, 0.f, 0.f, 0.f) : *(const float4*)(yr + kc);
+        if constexpr (PARTS) y[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+        else y[i] = *(const float4*)(yr + kc);
         out[i] = *(const float4*)(xr + kc);
         g[i] = *(const float4*)(p.w + kc);
         b[i] = p.b ? *(const float4*)(p.b + kc) : make_float4(0.f, 0.f, 0.f, 0.f);
@@ -344,13 +349,13 @@ template <int NC, bool PARTS = false> __device__ __forceinline__ void hb_post_ro
     }
     if constexpr (PARTS) {      // k_hb_moe_combine's sums
 #pragma unroll 2
-        for (int e = 0; e < p.top; ++e) {
-            const size_t en = (size_t)row * p.top + e;
-            const float w = p.unweighted ? 1.0f : p.wgt[en];
+        for (int e = 0; e < q.top; ++e) {
+            const size_t en = (size_t)row * q.top + e;
+            const float w = q.unweighted ? 1.0f : q.wgt[en];
 #pragma unroll
             for (int i = 0; i < NC; ++i) {
                 const int k = threadIdx.x * 4 + 1024 * i;
-                const float4 v = *(const float4*)(p.eo + en * W + (k < W ? k : 0));
+                const float4 v = *(const float4*)(q.eo + en * W + (k < W ? k : 0));
                 if (k < W) y[i] = make_float4(fmaf(w, v.x, y[i].x), fmaf(w, v.y, y[i].y), fmaf(w, v.z, y[i].z), fmaf(w, v.w, y[i].w));
             }
         }
@@ -367,15 +372,15 @@ template <int NC, bool PARTS = false> __device__ __forceinline__ void hb_post_ro
         __syncthreads();
         mean = (((red[0][0] + red[0][1]) + red[0][2]) + red[0][3]) / (float)W;
     }
-    float q = 0.f;
+    float sq = 0.f;
 #pragma unroll
     for (int i = 0; i < NC; ++i)
         if ((int)threadIdx.x * 4 + 1024 * i < W) {
             y[i].x -= mean; y[i].y -= mean; y[i].z -= mean; y[i].w -= mean;
-            q += y[i].x * y[i].x; q += y[i].y * y[i].y; q += y[i].z * y[i].z; q += y[i].w * y[i].w;
+            sq += y[i].x * y[i].x; sq += y[i].y * y[i].y; sq += y[i].z * y[i].z; sq += y[i].w * y[i].w;
         }
-    q = hb_wave_sum(q);
-    if (lane == 0) red[1][wv] = q;
+    sq = hb_wave_sum(sq);
+    if (lane == 0) red[1][wv] = sq;
     __syncthreads();
     const float inv = 1.0f / sqrtf((((red[1][0] + red[1][1]) + red[1][2]) + red[1][3]) / (float)W + p.eps);
 #pragma unroll
@@ -418,21 +423,20 @@ static int hb_post_pieces(const hb_post& p, const float* x, long ldx, int W) {
     if ((W & 3) || (ldx & 3) || (p.ldy & 3) || W > 4096 || (((size_t)p.y | (size_t)x | (size_t)p.w | (size_t)p.b) & 15)) return 0;
     return W <= 1024 ? 1 : (W <= 2048 ? 2 : 4);
 }
-// PARTS: the routed sum in front of the norm (k_hb_moe_combine's, which wrote 4 bytes a value for this launch to read).  2048 rows of 2048, two choices, us: 12.0 + 12.0 apart, 14.3 so.
-template <int NC, bool PARTS = false> __global__ __launch_bounds__(256) void k_hb_post_norm(hb_post p, float* x, long ldx, int W) {
+template <int NC> __global__ __launch_bounds__(256) void k_hb_post_norm(hb_post p, float* x, long ldx, int W) {
     __shared__ float red[2][4];
     float* xr = x + (size_t)blockIdx.x * ldx;
     if constexpr (NC > 0) {
         float4 out[NC];
-        hb_post_row<NC, PARTS>(p, blockIdx.x, xr, xr, ldx, W, red, out);
+        hb_post_row<NC>(p, blockIdx.x, xr, xr, ldx, W, red, out);
     } else hb_post_row_any(p, blockIdx.x, xr, W, red);
 }
 static void hb_post_norm(hipStream_t st, int n, const hb_post& p, float* x, long ldx, int W) {
     const int nc = hb_post_pieces(p, x, ldx, W);
     auto kern = nc == 1 ? k_hb_post_norm<1> : nc == 2 ? k_hb_post_norm<2> : nc == 4 ? k_hb_post_norm<4> : k_hb_post_norm<0>;
-    if (p.eo) kern = nc == 1 ? k_hb_post_norm<1, true> : nc == 2 ? k_hb_post_norm<2, true> : k_hb_post_norm<4, true>;      // (hb_moe: nc > 0)
     hipLaunchKernelGGL(kern, dim3(n), dim3(256), 0, st, p, x, ldx, W);
 }
+static void hb_post_parts(hipStream_t st, int n, const hb_post& p, const hb_parts& q, float* x, long ldx, int W);
 
 // ---- RMS norm over `groups` equal consecutive slices of the row, fp32; optional row gather; one or two weights --------------
 // Every slice is divided by its own sqrt(mean square + eps); y1 = that * w1 and (w2 != NULL) y2 = that * w2: the two norms of a
@@ -1227,6 +1231,7 @@ __global__ __launch_bounds__(256) void k_hb_post_gemv(hb_post p, const float* x,
 // reader has it completed in place first.
 struct hb_pending {
     hb_post p;          // p.y NULL: nothing pending
+    hb_parts parts;     // eo NULL: p.y holds the output
     float *x, *x_next;
     long ldx;
     bf16_t* buf16;      // room for the rows of x as bf16 at its stride, when the products that read x would round all of them, else NULL
@@ -1251,10 +1256,11 @@ static bool hb_try_post_gemv(hipStream_t st, hb_pending& pd, bool glu, const T* 
 static void hb_settle(hipStream_t st, hb_pending& pd, int n, int W) {
     if (!pd.p.y) return;
     pd.p.x16 = hb_post_pieces(pd.p, pd.x, pd.ldx, W) ? pd.buf16 : nullptr;
-    hb_post_norm(st, n, pd.p, pd.x, pd.ldx, W);
+    if (pd.parts.eo) hb_post_parts(st, n, pd.p, pd.parts, pd.x, pd.ldx, W);
+    else hb_post_norm(st, n, pd.p, pd.x, pd.ldx, W);
     pd.x16 = pd.p.x16;
     pd.p.y = nullptr;
-    pd.p.eo = nullptr;
+    pd.parts.eo = nullptr;
 }
 
 // 2..16 rows, bf16: one MFMA row tile; a block owns 16 output columns and its eight waves take the 32-wide k-steps w, w + 8, ...
@@ -5695,6 +5701,20 @@ __global__ void k_hb_feedback(const int* out_ids, int* input_ids, uint64_t* rng,
     if (b == 0 && rng) *rng += 1;
 }
 
+// k_hb_post_norm with the routed sum in front of it (k_hb_moe_combine's, which wrote 4 bytes a value for that launch to read).  2048 rows of 2048, two choices, us: 12.0 + 12.0
+// apart, 14.2 so.
+template <int NC> __global__ __launch_bounds__(256) void k_hb_post_parts(hb_post p, hb_parts q, float* x, long ldx, int W) {
+    __shared__ float red[2][4];
+    float* xr = x + (size_t)blockIdx.x * ldx;
+    float4 out[NC];
+    hb_post_row<NC, true>(p, blockIdx.x, xr, xr, ldx, W, red, out, q);
+}
+static void hb_post_parts(hipStream_t st, int n, const hb_post& p, const hb_parts& q, float* x, long ldx, int W) {      // (hb_moe asks for the register form)
+    const int nc = hb_post_pieces(p, x, ldx, W);
+    auto kern = nc == 1 ? k_hb_post_parts<1> : nc == 2 ? k_hb_post_parts<2> : k_hb_post_parts<4>;
+    hipLaunchKernelGGL(kern, dim3(n), dim3(256), 0, st, p, q, x, ldx, W);
+}
+
 }  // namespace
 
 #define HB_LAT_MAX_SEG 64     // blocks that share the keys of one row in the few-row latent attention
@@ -6352,11 +6372,11 @@ static int hb_mixer(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, cons
 }
 
 // Routed feed-forward of the rows h2 (first completed by `post` when it names a sublayer's output), added to cur.  Few rows: one GEMV pair per routed entry; more: the entries are
-// listed per expert and every expert multiplies its own rows in one tile launch.  parts != NULL: the norm that alone reads the result (rows h2, stride ldh, are its stream); where
-// it can add the routed outputs itself they stay in parts, and it says so.
+// listed per expert and every expert multiplies its own rows in one tile launch.  next != NULL: the norm that alone reads the result (rows h2, stride ldh, are its stream); where it
+// can add the routed outputs itself they stay in parts.
 template <typename T>
 static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, const float* h2, long ldh, hb_post post, float* cur, long ldx, int n, hb_join jn,
-                  hb_post* parts) {
+                  const hb_post* next, hb_parts* parts) {
     const vox_hybrid_moe& E = *L.moe;
     jn.scale = L.ls2;
     if (L.res_gate) { jn.gate = m->rgate; jn.ldg = m->cfg.width; }
@@ -6403,7 +6423,7 @@ static int hb_moe(vox_hybrid* m, hipStream_t st, const vox_hybrid_layer& L, cons
         VOX_TRY(hb_gemm_tiles<HB_EPI_STORE>(m->ws16, st, m->moe_act, (long)ff, (const T*)E.w_down, nullptr, m->moe_out, (long)W, n, W, ff, down, E.experts, rows, ne));
     }
     const int vec = !m->ws16.general && !(W & 3) && !(ldx & 3) && !(ldh & 3) && !(((size_t)cur | (size_t)h2 | (size_t)m->moe_out) & 15) ? 1 : 0;
-    if (parts && vec && top > 0 && E.identity == 0 && E.shared_ff == 0 && jn.store && !jn.gate && !jn.scale && jn.streams == 0 && hb_post_pieces(*parts, h2, ldh, W) > 0) {
+    if (next && vec && top > 0 && E.identity == 0 && E.shared_ff == 0 && jn.store && !jn.gate && !jn.scale && jn.streams == 0 && hb_post_pieces(*next, h2, ldh, W) > 0) {
         parts->eo = m->moe_out;
         parts->wgt = m->moe_wgt;
         parts->top = top;
@@ -6497,15 +6517,12 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
         if (L.sibling >= 0)
             VOX_TRY(hb_mixer<T>(m, st, io, m->layers[L.sibling], run.side_cache, run.side_pool, run.side_state, hn, W, src, lds_x, cur, ldx, n, n_req,
                                 max_kvlen, j1));
-        hb_post parts{};      // the second sublayer's norm, its routed outputs perhaps still apart
         if (L.moe) {
             if (!parallel && !post) hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h2, nullptr, nullptr, (long)W, L.norm2_b);
             hb_post p1 = pd.p;
             if (p1.y) { p1.x16 = pd.buf16; pd.x16 = nullptr; }
             pd.p.y = nullptr;
-            hb_post p2 = post2;
-            VOX_TRY(hb_moe<T>(m, st, L, post ? pd.x : hf, ldf, post ? p1 : none, dst, ldd, n, j2, post && n > 1 ? &p2 : nullptr));
-            parts = p2;
+            VOX_TRY(hb_moe<T>(m, st, L, post ? pd.x : hf, ldf, post ? p1 : none, dst, ldd, n, j2, post && n > 1 ? &post2 : nullptr, &pd.parts));
         } else if (L.ff > 0 && L.ff_kind == VOX_FF_GATED) {
             // down(act(gate h + b) * (up h + b)) + b: gate and up rows in one product, the activation in place behind it
             if (!parallel && !post) hb_norm(m, st, n, src, lds_x, nullptr, L.norm2, m->h2, nullptr, nullptr, (long)W, L.norm2_b);
@@ -6558,7 +6575,7 @@ static int hb_step(vox_hybrid* m, hipStream_t st, const vox_hybrid_io* io, const
             VOX_TRY(hb_gemm_resid<T>(m->ws16, st, m->ff, nf, (const T*)L.w_down, nullptr, dst, ldd, n, W, L.ff, j2));
         }
         if (post) {
-            if (has_ff) pd.p = L.moe ? parts : post2;
+            if (has_ff) pd.p = post2;
             if (io->trace) hb_settle(st, pd, n, W);
             cur = pd.x;
             other = pd.x_next;
