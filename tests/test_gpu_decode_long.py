@@ -52,3 +52,40 @@ def test_long_contexts_against_pages_of_sixteen(dev, heads, kvh, D, rows, top, p
     for a, b in zip(*got):
         assert np.array_equal(a, b)
     assert got[0][2]
+
+
+def decode(dev, h, x0, kv, lens, pos, page, slot, table, top):  # noqa: F811
+    """Decode rows with a page table: their hidden rows; kv holds their new tokens."""
+    from vox_serve_amd import _native as N
+    rows, per = len(lens), len(table[0])
+    i32 = lambda v: torch.as_tensor(np.asarray(v), dtype=torch.int32).to(dev)
+    ptab = i32(table)
+    tens = [i32(pos), i32(range(rows)), i32(lens), i32(page), i32(slot), i32(np.arange(rows + 1) * per), ptab.reshape(-1)]
+    rs = N.Rows(*[t.data_ptr() for t in tens], rows, top, ptab.data_ptr(), per, 0, -1, 0)
+    x, y = x0.clone(), torch.empty_like(x0)
+    N.check(N.lib().vox_stack_forward(h, N.stream(), x.data_ptr(), y.data_ptr(), kv.data_ptr(), kv[0].numel(), ctypes.byref(rs)))
+    torch.cuda.synchronize()
+    return y
+
+
+@pytest.mark.parametrize("heads,kvh,D,rows", [(16, 8, 128, 16), (16, 8, 128, 17), (32, 8, 64, 8), (32, 8, 64, 9)])
+def test_rows_longer_than_their_call_says(dev, heads, kvh, D, rows):  # noqa: F811
+    """Rows of 321 to 400 tokens in a call of up to 320: what the block keeps of a row ends with the call's ten chunks, so that such a row is one of 320 tokens (its newest is the last of
+    them), and its neighbours are untouched by it."""
+    from vox_serve_amd import _native as N
+    H, page, per, top = 256, 32, 13, 320
+    lens = [(400, 320, 321, 33, 352, 319, 385)[r % 7] for r in range(rows)]
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x0 = torch.randn(rows, H, generator=g, device=dev).bfloat16()
+    kv0 = torch.randn(2, rows * per, 2, page, kvh, D, generator=g, device=dev).bfloat16()
+    table = np.random.default_rng(rows).permutation(rows * per).reshape(rows, per)
+    last = [n - 1 for n in lens]
+    at = dict(pos=last, page=[table[r][n // page] for r, n in enumerate(last)], slot=[n % page for n in last], table=table, top=top)
+    h, keep = stack(dev, H, heads, kvh, D, 512, rows, per * page, page, 5, False)
+    got = []
+    for said in (lens, [min(n, top) for n in lens]):
+        kv = kv0.clone()
+        got.append((Bits(decode(dev, h, x0, kv, said, **at)), Bits(kv)))
+    N.lib().vox_stack_destroy(h)
+    assert np.isfinite(vr.bf2f(got[0][0])).all()
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])

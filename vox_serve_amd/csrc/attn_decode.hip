@@ -41,8 +41,9 @@ __global__ __launch_bounds__(64 * NWV, PREP ? 1 : 4) void k_attn_decode(AttnArgs
     const int HS = gridDim.x / a.Hkv, hk = blockIdx.x / HS, hs = blockIdx.x - hk * HS, row = blockIdx.y;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), j = lane % LPT, tg = lane / LPT;
     const int* const pages = a.ptab ? a.ptab + (size_t)row * a.pt_stride : a.indices + a.indptr[a.q_req[row]];
-    const int L = a.q_kvlen[row], pg_new = PREP ? a.page[row] : -1, sl_new = PREP ? a.slot[row] : 0;
-    const int ncl = (L + VOX_TC - 1) / VOX_TC, nc = PREP || ncl < nchunk ? ncl : nchunk, Gf = a.Hq / a.Hkv, h0 = hk * Gf + hs * G;
+    // (a row longer than its call says ends with the chunks that LDS was asked for)
+    const int Lr = a.q_kvlen[row], L = Lr < nchunk * VOX_TC ? Lr : nchunk * VOX_TC, pg_new = PREP ? a.page[row] : -1, sl_new = PREP ? a.slot[row] : 0;
+    const int nc = (L + VOX_TC - 1) / VOX_TC, Gf = a.Hq / a.Hkv, h0 = hk * Gf + hs * G;
     const size_t trow = (size_t)a.Hkv * D, ps = (size_t)2 * a.page_size * trow;
     const bf16_t* const raw = PREP ? a.qkv + (size_t)row * (a.Hq + 2 * a.Hkv) * D : a.q + ((size_t)row * a.Hq + h0) * D;
     const bf16_t* const vnew = PREP ? raw + (size_t)(a.Hq + a.Hkv + hk) * D : nullptr;
