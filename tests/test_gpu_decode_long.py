@@ -89,3 +89,32 @@ def test_rows_longer_than_their_call_says(dev, heads, kvh, D, rows):  # noqa: F8
     N.lib().vox_stack_destroy(h)
     assert np.isfinite(vr.bf2f(got[0][0])).all()
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
+
+
+@pytest.mark.parametrize("heads,kvh,D,rows", [(16, 8, 128, 16), (16, 8, 128, 17), (32, 8, 64, 9)])
+def test_table_entries_without_cached_tokens_are_not_used(dev, heads, kvh, D, rows):  # noqa: F811
+    """Padding rows (one token, page -1) and rows whose newest token opens a page that their table does not list yet: -1 in the table wherever a page holds no cached token, against
+    pages of 16 tokens (k_attn_partial, which never asks for those).  The page in front of the cache belongs to the same allocation."""
+    from vox_serve_amd import _native as N
+    H, top = 256, 513
+    lens = [(513, 1, 33, 129, 385, 1, 289, 130)[r % 8] for r in range(rows)]
+    g = torch.Generator(device=dev).manual_seed(rows)
+    x0 = torch.randn(rows, H, generator=g, device=dev).bfloat16()
+    past = [torch.randn(2, 2, n, kvh, D, generator=g, device=dev).bfloat16() for n in lens]
+    got = []
+    for size in (16, 32):
+        per = -(-top // size)
+        table = np.random.default_rng(rows).permutation(rows * per).reshape(rows, per)
+        h, keep = stack(dev, H, heads, kvh, D, 512, rows, per * size, size, 5, False)
+        room = torch.zeros(1 + 2 * rows * per, 2, size, kvh, D, dtype=torch.bfloat16, device=dev)
+        kv = room[1:].view(2, rows * per, 2, size, kvh, D)
+        for r, n in enumerate(lens):
+            tok = torch.arange(n - 1)
+            kv[:, torch.as_tensor(table[r])[tok // size], :, tok % size] = past[r][:, :, : n - 1].permute(2, 0, 1, 3, 4)
+        page = [-1 if n == 1 else int(table[r][(n - 1) // size]) for r, n in enumerate(lens)]
+        bare = np.array([[table[r][j] if j * size < n - 1 else -1 for j in range(per)] for r, n in enumerate(lens)])
+        y = decode(dev, h, x0, kv, lens, [n - 1 for n in lens], page, [(n - 1) % size for n in lens], bare, top)
+        N.lib().vox_stack_destroy(h)
+        got.append((Bits(y), Bits(torch.stack([kv[:, p, :, (n - 1) % size] for p, n in zip(page, lens) if n > 1])), float(room[0].abs().max())))
+    assert np.isfinite(vr.bf2f(got[0][0])).all() and got[0][2] == got[1][2] == 0
+    assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])

@@ -53,7 +53,9 @@ __global__ __launch_bounds__(64 * NWV, PREP ? 1 : 4) void k_attn_decode(AttnArgs
     // (a chunk lies in one page; what the page holds behind the row's cached tokens is read and not used.  Scalar bases, one 32-bit offset a lane)
     auto k_rows = [&](int c) {
         const int tok = c * VOX_TC, pi = page_of(a, tok);
-        return a.kv + (size_t)__builtin_amdgcn_readfirstlane(pages[pi]) * ps + ((size_t)(tok - pi * a.page_size) * a.Hkv + hk) * D;
+        // (a chunk of the newest token alone reads page 0 for nothing: its entry of the table may not be there yet, and a padding row has none)
+        const int pg = !PREP || tok < L - 1 ? __builtin_amdgcn_readfirstlane(pages[pi]) : 0;
+        return a.kv + (size_t)pg * ps + ((size_t)(tok - pi * a.page_size) * a.Hkv + hk) * D;
     };
     auto fetch_k = [&](const bf16_t* kb) {
 #pragma unroll
