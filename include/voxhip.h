@@ -93,6 +93,15 @@ int64_t vox_attn_workspace_bytes(int Nq, int Hq, int D, int max_kvlen);
 int vox_paged_attention(vox_ctx* ctx, void* stream, const void* q, const void* kv_layer, const int32_t* q_req,
                         const int32_t* q_kvlen, const int32_t* kv_indptr, const int32_t* kv_indices, void* out,
                         void* workspace, int Nq, int Hq, int Hkv, int D, int page_size, int max_kvlen, float scale);
+/* The same, told how many requests the rows belong to: the launches differ in what they share between the rows of a request
+ * (0: not known, as vox_paged_attention; the outputs are the same). */
+int vox_paged_attention_of(vox_ctx* ctx, void* stream, const void* q, const void* kv_layer, const int32_t* q_req,
+                           const int32_t* q_kvlen, const int32_t* kv_indptr, const int32_t* kv_indices, void* out,
+                           void* workspace, int Nq, int Hq, int Hkv, int D, int page_size, int max_kvlen, float scale, int n_req);
+/* Which attention launch serves n_rows rows of n_req requests (operands on 16 bytes), decided on the host: 0 a block per chunk and a merge, 1 a wave per
+ * chunk, 2 tiles of rows and heads, 3 (decode) a block per row for up to 16 chunks.  decode: rows with their new token beside them (a stack's decode rows of
+ * more than 32 tokens with a page table), else rows that read q and their pages. */
+int vox_attention_form(int decode, int n_rows, int n_req, int Hq, int Hkv, int D, int page_size, int max_kvlen);
 
 /* nn.Linear on bf16 (qwen3_tts.py:562-601): y[b,n] = bf16(dot(W[n,:],x[b,:]) + bias[n]);
  * residual != NULL: y = bf16(residual + y).  act: 0 none, 1 SiLU applied to the rounded output. */
@@ -164,6 +173,7 @@ typedef struct { /* device int32 arrays describing one ragged forward (FlashInfe
     int32_t fixed_kvlen;       /* > 0: every row attends to exactly this many tokens */
     int32_t fixed_pos;         /* >= 0 with fixed_kvlen: every row's position id */
     int32_t identity_pages;    /* request r owns the single page r and row i belongs to request i */
+    int32_t n_req;             /* requests that the rows belong to (prompts: which attention launch is the faster one) */
 } vox_rows;
 
 /* x [n_rows,hidden] bf16 is updated in place layer by layer; y (may alias x) = final RMSNorm(x).

@@ -45,7 +45,7 @@ def forward(dev, h, x, kv, page, kvh, D, parts, pages):  # noqa: F811
     for n in parts:
         pos = np.arange(at, at + n)
         tens = [i32(pos), i32(np.zeros(n)), i32(pos + 1), i32(np.asarray(pages)[pos // page]), i32(pos % page), i32([0, len(pages)]), i32(pages)]
-        rows = N.Rows(*[t.data_ptr() for t in tens], n, at + n, None, 0, 0, -1, 0)
+        rows = N.Rows(*[t.data_ptr() for t in tens], n, at + n, None, 0, 0, -1, 0, 1)
         xi, y = x[at: at + n].clone(), torch.empty(n, x.shape[1], dtype=torch.bfloat16, device=dev)
         N.check(N.lib().vox_stack_forward(h, N.stream(), xi.data_ptr(), y.data_ptr(), kv.data_ptr(), kv[0].numel(), ctypes.byref(rows)))
         torch.cuda.synchronize()
@@ -75,18 +75,21 @@ def test_prompt_in_one_portion_and_in_many(dev, rows, H, heads, kvh, D, F, bias)
     assert torch.isfinite(got[0][0].float()).all()
 
 
-def attend(dev, q, kv, q_req, kvlen, indptr, indices, Hkv, page, one_by_one):  # noqa: F811
-    """vox_paged_attention on all rows at once, or on one row at a time (k_attn_partial and k_attn_merge)."""
+def attend(dev, q, kv, q_req, kvlen, indptr, indices, Hkv, page, top, one_by_one, form):  # noqa: F811
+    """vox_paged_attention_of on all rows at once, which the launch `form` serves, or on one row at a time (k_attn_partial and k_attn_merge: 300 tokens are more than any group's single
+    row leaves to the others)."""
     from vox_serve_amd import _native as N
     i32 = lambda v: torch.as_tensor(np.asarray(v), dtype=torch.int32).to(dev)
     n, Hq, D = q.shape
-    out, top = torch.full_like(q, 7.0), int(max(kvlen))
+    top, n_req = (max(top, 300), 1) if one_by_one else (top, len(indptr) - 1)
+    assert N.lib().vox_attention_form(0, 1 if one_by_one else n, n_req, Hq, Hkv, D, page, top) == (0 if one_by_one else form)
+    out = torch.full_like(q, 7.0)
     ip, ix = i32(indptr), i32(indices)
     ws = torch.empty(N.lib().vox_attn_workspace_bytes(n, Hq, D, top) // 4, dtype=torch.float32, device=dev)
     for i, j in ([(0, n)] if not one_by_one else [(i, i + 1) for i in range(n)]):
         qr, kl = i32(q_req[i:j]), i32(kvlen[i:j])
-        N.check(N.lib().vox_paged_attention(N.ctx(), N.stream(), q[i:j].data_ptr(), N.ptr(kv), N.ptr(qr), N.ptr(kl), N.ptr(ip), N.ptr(ix), out[i:j].data_ptr(), N.ptr(ws), j - i, Hq, Hkv, D,
-                                            page, top, float(D ** -0.5)))
+        N.check(N.lib().vox_paged_attention_of(N.ctx(), N.stream(), q[i:j].data_ptr(), N.ptr(kv), N.ptr(qr), N.ptr(kl), N.ptr(ip), N.ptr(ix), out[i:j].data_ptr(), N.ptr(ws), j - i, Hq, Hkv,
+                                               D, page, top, float(D ** -0.5), n_req))
     torch.cuda.synchronize()
     return out
 
@@ -104,14 +107,16 @@ def prompt_case(seed, lens, ctx, page):
 
 
 @pytest.mark.parametrize("special", [False, True])
-@pytest.mark.parametrize("Hq,Hkv,D,page,lens,ctx", [(16, 8, 128, 128, [200], [0]), (4, 2, 128, 32, [1, 97, 3, 160, 33], [0, 300, 31, 7, 64]), (8, 2, 64, 24, [130, 5, 140], [11, 290, 0]),
-                                                    (6, 2, 128, 16, [170], [100]), (3, 3, 64, 8, [257], [0]), (32, 2, 128, 128, [70], [200]), (32, 8, 64, 128, [290], [0]),
-                                                    (8, 8, 128, 128, [1031], [0])])
-def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special):  # noqa: F811
-    """Several requests in a tile, tiles of 16, 8, 5, 4 and 1 rows, ragged chunks, pages that no power of two divides, four and eight waves; with infinities and NaN among keys and
-    values (single rows never read the tokens behind them), and a row without tokens in between."""
+@pytest.mark.parametrize("Hq,Hkv,D,page,lens,ctx", [(16, 8, 128, 128, [200], [0]), (16, 8, 128, 32, [1, 197, 3, 2, 260, 33], [0, 300, 31, 5, 7, 64]),
+                                                    (32, 8, 64, 24, [330, 240, 5, 7], [11, 0, 90, 40]), (8, 8, 64, 24, [130, 5, 140], [11, 290, 0]), (18, 6, 128, 16, [170, 90], [100, 0]),
+                                                    (15, 5, 64, 8, [257], [0]), (12, 12, 64, 8, [257], [0]), (14, 2, 64, 16, [150, 60], [60, 9]), (32, 2, 128, 128, [70], [200]),
+                                                    (32, 8, 64, 128, [290], [0]), (8, 8, 128, 128, [1031], [0])])
+def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special, form=2):  # noqa: F811
+    """Several requests in a tile, tiles of 16, 8, 5 (a column of the 16 idle), 4, 2 (two idle) and 1 rows, ragged chunks, pages that no power of two divides, four and eight waves; with
+    infinities and NaN among keys and values (single rows never read the tokens behind them), and a row without tokens in between."""
     g = torch.Generator(device=dev).manual_seed(sum(lens))
     q_req, kvlen, indptr, indices = prompt_case(sum(lens), lens, ctx, page)
+    top = max(kvlen)
     q = torch.randn(len(q_req), Hq, D, generator=g, device=dev).bfloat16()
     kv = torch.randn(max(indices) + 1, 2, page, Hkv, D, generator=g, device=dev).bfloat16()
     if special:
@@ -120,7 +125,7 @@ def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, 
             kv[page_id, 1, page // 3, 0, 1] = float("inf")
             kv[page_id, 1, page // 2, Hkv - 1, D - 2] = float("nan")
             kv[page_id, 0, page - 1, 0, 3] = float("-inf")
-    a, b = (attend(dev, q, kv, q_req, kvlen, indptr, indices, Hkv, page, one) for one in (False, True))
+    a, b = (attend(dev, q, kv, q_req, kvlen, indptr, indices, Hkv, page, top, one, form) for one in (False, True))
     nan = torch.isnan(a.float()) & torch.isnan(b.float())
     same = (a.view(torch.int16) == b.view(torch.int16)) | nan
     assert same.all(), (~same).nonzero()[:4].tolist()
@@ -134,7 +139,7 @@ def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, 
 def test_short_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special):  # noqa: F811
     """A wave per chunk, four and eight waves: rows of one chunk to eight that end at and around a chunk's last token, several requests; with infinities and NaN, also behind
     the last token of a row, and a row without tokens."""
-    test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special)
+    test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special, form=1)
 
 
 @pytest.mark.parametrize("rows,N,K,tile", [(33, 151, 1152, 0), (65, 130, 640, 0), (129, 2048, 128, 0), (300, 2050, 1152, 1), (450, 2050, 1152, 2), (1000, 2048, 640, 2), (520, 4100, 640, 3),

@@ -1,6 +1,7 @@
 """CPU tests of the host side: worker bookkeeping + scheduler policy against traces captured from the reference's own
 ModelWorker / Scheduler (tests/golden/g6_host_traces.json), the wire format, the C-ABI export table, the DP pool over
 gloo (world_size 2), DecoderCache semantics and the Qwen3 prompt layout."""
+import ctypes
 import hashlib
 import json
 import os
@@ -142,11 +143,24 @@ def test_c_abi_exports_every_declared_symbol():
     out = subprocess.check_output(["nm", "-D", "--defined-only", so]).decode()
     exported = set(re.findall(r"\bT (vox_[a-z0-9_]+)", out))
     assert declared and declared <= exported, sorted(declared - exported)
-    import ctypes
     L = ctypes.CDLL(so)                 # loads without a GPU; no compute entry point is called here
     assert L.vox_abi_version() == 1
     from vox_serve_amd import _native
     assert set(_native._SIGS) <= exported
+
+
+@pytest.mark.parametrize("heads,kvh,D,page,rows,top", [(16, 8, 128, 128, 64, 1500), (16, 8, 128, 128, 48, 1000), (16, 8, 128, 16, 32, 256), (16, 8, 128, 16, 128, 128), (32, 8, 64, 128, 128, 600),
+                                                       (32, 8, 64, 16, 32, 250), (8, 8, 128, 128, 64, 1500), (8, 8, 128, 16, 128, 250)])
+def test_attention_tiles_are_not_for_rows_of_different_requests(heads, kvh, D, page, rows, top):
+    """A tile of the prompt attention takes its rows' requests one after the other: one row a request goes to a block per chunk (measured 1.3 to 9 times as fast at these sizes), also
+    where the number of requests is not known; the rows of one request go to tiles."""
+    from vox_serve_amd import _native
+    form = ctypes.CDLL(_native.LIB_PATH).vox_attention_form
+    assert form(0, rows, rows, heads, kvh, D, page, top) == form(0, rows, 0, heads, kvh, D, page, top) == 0
+    assert form(0, 450, 1, heads, kvh, D, page, 450) == 2 and form(0, 1000, 1, heads, kvh, D, page, 1000) == 2
+    # a prompt beside rows of other requests, and prompts together
+    assert form(0, 75 + 31, 32, heads, kvh, D, page, 301) == 0
+    assert form(0, 1024, 8, heads, kvh, D, page, 128) == form(0, 1000, 4, heads, kvh, D, page, 250) == form(0, 900, 2, heads, kvh, D, page, 450) == 2
 
 
 def test_product_never_imports_the_oracle():

@@ -34,7 +34,7 @@ class LayerWeights(Structure):
 class Rows(Structure):
     _fields_ = [(n, c_void_p) for n in ("pos", "q_req", "q_kvlen", "page", "slot", "kv_indptr", "kv_indices")] + \
                [("n_rows", c_int32), ("max_kvlen", c_int32), ("page_table", c_void_p), ("pt_stride", c_int32),
-                ("fixed_kvlen", c_int32), ("fixed_pos", c_int32), ("identity_pages", c_int32)]
+                ("fixed_kvlen", c_int32), ("fixed_pos", c_int32), ("identity_pages", c_int32), ("n_req", c_int32)]
 
 
 class Qwen3Config(Structure):
@@ -80,6 +80,9 @@ _SIGS = {
     "vox_attn_workspace_bytes": (c_int64, [c_int, c_int, c_int, c_int]),
     "vox_paged_attention": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                     c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float]),
+    "vox_paged_attention_of": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+                                       c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int]),
+    "vox_attention_form": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
     "vox_linear": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                            c_int]),
     "vox_linear_silu_mul": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int]),

@@ -250,7 +250,7 @@ int vox_launch_attn_decode(hipStream_t st, const AttnCall& c) {
 // 75 9.4 / 6.5, 96 11.6 / 6.5, 128 11.0 / 8.1, 144 13.1 / 13.5 (eight waves), 250 14.1 / 21.8; behind 100: 8 rows 7.4 / 5.1, 64 13.4 / 7.7, 128 14.1 / 14.5; 32 heads on 8, D = 64:
 // 48 7.2 / 4.7, 96 9.4 / 8.5, 128 9.7 / 9.8; 32 heads on 2: 48 10.5 / 5.4, 96 11.0 / 10.7, behind 190 24 13.6 / 9.2, 64 13.9 / 15.2.
 static bool rows_pay(const AttnCall& c, int nchunk) {
-    const float own = (float)c.Nq / (64.0f * nchunk), seen = own < 0.5f ? 1.0f - own : 0.5f;
+    const float seen = vox_attn_seen(c, nchunk);
     const int blocks = c.Nq * c.Hq / 2, slots = nchunk > 4 ? 512 : c.D == 64 ? 1280 : 1024, rounds = (blocks + slots - 1) / slots;
     const float waves = (float)blocks * nchunk * seen, round = c.D == 64 ? 1.7f : nchunk > 4 ? 1.9f : 2.0f;
     const float wave = nchunk > 4 ? (c.D == 64 ? 0.0008f : 0.00105f) : c.D == 64 ? 0.00135f : 0.00155f, base = nchunk > 4 ? (c.D == 64 ? 3.2f : 4.0f) : c.D == 64 ? 1.8f : 2.1f;

@@ -306,14 +306,32 @@ static int prompt_blocks(const AttnCall& c) {
     const int rows = 16 / (c.Hq / c.Hkv);
     return c.Hkv * ((c.Nq + rows - 1) / rows);
 }
+static int requests(const AttnCall& c) { return c.n_req < 1 || c.n_req > c.Nq ? c.Nq : c.n_req; }
+float vox_attn_seen(const AttnCall& c, int nchunk) {      // (a prompt's rows alone see half of it on average)
+    const float own = (float)c.Nq / (64.0f * nchunk * requests(c));
+    return own < 0.5f ? 1.0f - own : 0.5f;
+}
+static bool four_waves(const AttnCall& c) { return prompt_blocks(c) > (c.D == 64 ? 256 : 512); }
 // What k_attn_partial and k_attn_merge take and what this kernel takes, us, fitted to 2 to 1000 rows behind 0 to 3000 tokens, 2 and 8 kv heads of 2, 4 and 16 q heads.  The
 // former by blocks (row, kv head, chunk; a prompt's rows see half of it), the latter by rounds of eight chunks, of which a tile's block goes through one after the other
-// while the chip may be idle.  Measured, former / latter: 16 heads on 8, D = 128, no context: 64 rows 8.6 / 10.8, 96 12.0 / 11.0; behind 1500 tokens: 2 rows 12 / 59,
+// while the chip may be idle.  A tile takes its rows' requests one after the other: at most as many as it has rows, and since no request has more rows than the call
+// has tokens, at most two beyond those that the call's rows leave over.  Measured, former / latter: 16 heads on 8, D = 128, no context: 64 rows 8.6 / 10.8, 96 12.0 / 11.0; behind 1500 tokens: 2 rows 12 / 59,
 // 32 48 / 60, 64 84 / 65, 128 152 / 67; 32 heads on 8, D = 64, behind 700: 16 rows 17 / 24, 48 35 / 25; 32 heads on 2: 48 rows 14.0 / 9.5, behind 1500: 32 48 / 60, 64 81 / 65.
+// One row a request (one per tile and pass), 16 heads on 8, D = 128: 64 rows of 1500 tokens 115 / 516, 128 of 600 93 / 234; 32 heads on 8, D = 64: 128 of 600 71 / 93; 32 heads on 2 (a row
+// a tile) 65 / 37.  16 heads on 8: a prompt of 75 rows beside 31 of one row behind 300 tokens 25 / 149, eight prompts of 128 rows 105 / 28, four of 250 189 / 44.
 void vox_attn_prompt_us(const AttnCall& c, int nchunk, float& parts, float& prompt) {
-    const float G = (float)(c.Hq / c.Hkv), own = (float)c.Nq / (64.0f * nchunk), seen = own < 0.5f ? 1.0f - own : 0.5f;
+    const float G = (float)(c.Hq / c.Hkv), seen = vox_attn_seen(c, nchunk);
     parts = 7.3f + 0.35f * G * c.D / 128 + (float)c.Nq * c.Hkv * nchunk * seen * (0.0018f + 0.0000038f * G * c.D);
-    const float longest = (float)((nchunk + 7) / 8), all = prompt_blocks(c) * seen * nchunk / 2048.0f;
+    const int req = requests(c), rows = 16 / (c.Hq / c.Hkv), tiles = (c.Nq + rows - 1) / rows;
+    int passes = 1;
+    if (req > 1) {
+        const int whole = c.Nq > rows ? (c.Nq - rows + c.max_kvlen - 1) / c.max_kvlen : 0, left = req - whole + 2;
+        passes = left < 1 ? 1 : left;
+        if (passes > rows) passes = rows;
+        if (passes > req) passes = req;
+    }
+    const int round = passes > 1 && four_waves(c) ? 4 : 8;
+    const float longest = (float)passes * ((nchunk + round - 1) / round), all = (float)c.Hkv * (tiles + req - 1) * seen * nchunk / 2048.0f;
     prompt = 3.0f + (4.0f + 0.04f * c.D) * (longest > all ? longest : all);
 }
 static bool prompt_pays(const AttnCall& c, int nchunk) {
@@ -337,7 +355,7 @@ int vox_launch_attn_prompt(hipStream_t st, const AttnCall& c) {
     // four waves and two blocks to a CU where there are blocks for it (one's trips behind the other's products, shorter last rounds), else eight.  us, eight / four: 16 heads on
     // 8, D = 128: 256 rows (256 blocks) 14.3 / 18.2, 450 (456) 32.7 / 34.3, 640 (640) 52.2 / 42.8, 1000 101 / 91; 32 heads on 8, D = 64: 128 rows (256) 10.7 / 10.9, 160 (320)
     // 17.2 / 14.1, 1000 148 / 120
-    const bool four = prompt_blocks(c) > (c.D == 64 ? 256 : 512);
+    const bool four = four_waves(c);
     if (c.D == 128) return four ? launch_prompt_t<128, 4>(st, a, nchunk) : launch_prompt_t<128, 8>(st, a, nchunk);
     return four ? launch_prompt_t<64, 4>(st, a, nchunk) : launch_prompt_t<64, 8>(st, a, nchunk);
 }

@@ -65,9 +65,9 @@ int64_t vox_attn_workspace_bytes(int Nq, int Hq, int D, int max_kvlen) {
     return (int64_t)Nq * Hq * n_chunks(max_kvlen) * (D + 2) * 4;
 }
 
-int vox_paged_attention(vox_ctx* ctx, void* stream, const void* q, const void* kv, const int32_t* q_req,
-                        const int32_t* q_kvlen, const int32_t* indptr, const int32_t* indices, void* out, void* ws,
-                        int Nq, int Hq, int Hkv, int D, int page_size, int max_kvlen, float scale) {
+int vox_paged_attention_of(vox_ctx* ctx, void* stream, const void* q, const void* kv, const int32_t* q_req,
+                           const int32_t* q_kvlen, const int32_t* indptr, const int32_t* indices, void* out, void* ws,
+                           int Nq, int Hq, int Hkv, int D, int page_size, int max_kvlen, float scale, int n_req) {
     (void)ctx;
     const int mc = n_chunks(max_kvlen);
     AttnCall c;
@@ -75,11 +75,26 @@ int vox_paged_attention(vox_ctx* ctx, void* stream, const void* q, const void* k
     c.part_o = (float*)ws; c.part_ml = (float*)ws + (size_t)Nq * Hq * mc * D; c.scale = scale; c.Nq = Nq;
     c.Hq = Hq; c.Hkv = Hkv; c.D = D; c.page_size = page_size; c.max_chunks = mc; c.max_kvlen = max_kvlen;
     c.out = out;
+    c.n_req = n_req;
     if (vox_attn_rows_supported(c)) return vox_launch_attn_rows((hipStream_t)stream, c);
     if (vox_attn_prompt_supported(c)) return vox_launch_attn_prompt((hipStream_t)stream, c);
     c.out = nullptr;
     VOX_TRY(vox_launch_attn_partial((hipStream_t)stream, c));
     return vox_launch_attn_merge((hipStream_t)stream, c.part_o, c.part_ml, q_kvlen, out, Nq, Hq, D, mc);
+}
+int vox_paged_attention(vox_ctx* ctx, void* stream, const void* q, const void* kv, const int32_t* q_req,
+                        const int32_t* q_kvlen, const int32_t* indptr, const int32_t* indices, void* out, void* ws,
+                        int Nq, int Hq, int Hkv, int D, int page_size, int max_kvlen, float scale) {
+    return vox_paged_attention_of(ctx, stream, q, kv, q_req, q_kvlen, indptr, indices, out, ws, Nq, Hq, Hkv, D, page_size, max_kvlen, scale, 0);
+}
+int vox_attention_form(int decode, int n_rows, int n_req, int Hq, int Hkv, int D, int page_size, int max_kvlen) {
+    alignas(16) static char at[16];      // (an address for the rules to look at)
+    AttnCall c;
+    c.q = c.kv = c.out = at; c.part_o = (float*)at; c.Nq = n_rows; c.n_req = n_req; c.Hq = Hq; c.Hkv = Hkv; c.D = D; c.page_size = page_size; c.max_kvlen = max_kvlen;
+    c.max_chunks = n_chunks(max_kvlen);
+    if (!decode) return vox_attn_rows_supported(c) ? 1 : vox_attn_prompt_supported(c) ? 2 : 0;
+    c.qkv = at; c.ptab = c.page = c.slot = (const int*)at; c.cs = (const float*)at;
+    return vox_attn_decode_supported(c) ? 1 : vox_attn_decode8_supported(c) ? 3 : 0;
 }
 
 int vox_linear(vox_ctx* ctx, void* stream, const void* W, const void* bias, const void* x, const void* residual,
@@ -233,7 +248,7 @@ static int stack_layers(vox_stack* s, hipStream_t st, void* x, void* kv, int64_t
         ac.q = s->q; ac.kv = kvl; ac.q_req = r->q_req; ac.q_kvlen = r->q_kvlen; ac.indptr = r->kv_indptr;
         ac.indices = r->kv_indices; ac.part_o = part_o; ac.part_ml = part_ml; ac.scale = scale; ac.Nq = n;
         ac.Hq = c.heads; ac.Hkv = c.kv_heads; ac.D = c.head_dim; ac.page_size = c.page_size; ac.max_chunks = mc;
-        ac.max_kvlen = r->max_kvlen;
+        ac.max_kvlen = r->max_kvlen; ac.n_req = r->n_req;
         ac.out = s->attn_out;
         LinearCall o;  // o_proj + residual
         o.W = w.wo; o.x = s->attn_out; o.residual = x; o.y = x; o.B = n; o.N = c.hidden; o.K = nq;
@@ -955,6 +970,7 @@ int vox_qwen3_prefill(vox_qwen3* m, void* stream, const vox_qwen3_io* io, const 
     vox_rows r{};
     r.pos = io->pos; r.q_req = q_req; r.q_kvlen = io->kvlen; r.page = io->page; r.slot = io->slot;
     r.kv_indptr = io->kv_indptr; r.kv_indices = io->kv_indices; r.n_rows = n_rows; r.max_kvlen = max_kvlen;
+    r.n_req = n_req > 0 ? n_req : 1;
     VOX_TRY(stack_layers(m->talker, st, m->x, io->kv, io->kv_layer_stride, &r));
     if (n_req == 0) return VOX_OK;      // context chunk of a long prompt: K/V appended, nothing sampled
     VOX_TRY(qwen3_head(m, st, io, n_req, last_rows));
@@ -1213,6 +1229,7 @@ int vox_csm_prefill(vox_csm* m, void* stream, const vox_csm_io* io, const int32_
     vox_rows r{};
     r.pos = io->pos; r.q_req = q_req; r.q_kvlen = io->kvlen; r.page = io->page; r.slot = io->slot;
     r.kv_indptr = io->kv_indptr; r.kv_indices = io->kv_indices; r.n_rows = n_rows; r.max_kvlen = max_kvlen;
+    r.n_req = n_req > 0 ? n_req : 1;
     VOX_TRY(stack_layers(m->backbone, st, m->x, io->kv, io->kv_layer_stride, &r, false, n_rows <= m->ctx->exact_rows));
     if (n_req == 0) return VOX_OK;      // context chunk of a long prompt
     VOX_TRY(csm_head(m, st, io, n_req, last_rows));
@@ -1325,6 +1342,7 @@ int vox_lm_prefill(vox_lm* m, void* stream, const vox_lm_io* io, const int32_t* 
     vox_rows r{};
     r.pos = io->pos; r.q_req = q_req; r.q_kvlen = io->kvlen; r.page = io->page; r.slot = io->slot;
     r.kv_indptr = io->kv_indptr; r.kv_indices = io->kv_indices; r.n_rows = n_rows; r.max_kvlen = max_kvlen;
+    r.n_req = n_req > 0 ? n_req : 1;
     return lm_run(m, (hipStream_t)stream, io, row_ids, row_masks, row_features, r, false, last_rows, n_req, sc, seed, feedback);
 }
 

@@ -109,6 +109,7 @@ struct AttnCall {
     void* out_frag = nullptr;   // optional: the same output ALSO in fragment-major form (A operand of a 9..32 rows o_proj)
     const int* ptab = nullptr;
     int pt_stride = 0, fixed_kvlen = 0, fixed_pos = -1, identity_pages = 0;
+    int n_req = 0;         // requests that the rows belong to (0: not known, as many as rows)
 };
 // Persistent depth step (one request): 5 layers + the codebook head of one depth-loop step in one launch (kernels_lm.hip).
 struct DepthStepCall {
@@ -171,6 +172,7 @@ bool vox_attn_decode_supported(const AttnCall& c);       // decode rows, one lau
 int vox_launch_attn_decode(hipStream_t st, const AttnCall& c);
 bool vox_attn_rows_supported(const AttnCall& c);         // few rows that read q and their pages, 2..8 chunks, merge included (attn_decode.hip)
 int vox_launch_attn_rows(hipStream_t st, const AttnCall& c);
+float vox_attn_seen(const AttnCall& c, int nchunk);       // share of the call's chunks that a row sees on average
 void vox_attn_prompt_us(const AttnCall& c, int nchunk, float& parts, float& prompt);      // estimates: k_attn_partial with its merge, and k_attn_prompt
 bool vox_attn_prompt_supported(const AttnCall& c);       // many rows that read q and their pages, merge included: out is written, the partial outputs are not (attn_prompt.hip)
 int vox_launch_attn_prompt(hipStream_t st, const AttnCall& c);

@@ -84,10 +84,10 @@ class _PagedBase:
         m = self._meta
         out = torch.empty_like(q)
         ws = self._workspace(q.shape[0], m["max_kvlen"])
-        N.check(N.lib().vox_paged_attention(
+        N.check(N.lib().vox_paged_attention_of(
             N.ctx(), N.stream(), N.ptr(q), N.ptr(kv_cache), N.ptr(m["q_req"]), N.ptr(m["q_kvlen"]), N.ptr(m["indptr"]),
             N.ptr(m["indices"]), N.ptr(out), N.ptr(ws), q.shape[0], self.n_qo_head, self.n_kv_head, self.head_dim,
-            kv_cache.shape[2], m["max_kvlen"], float(self.head_dim) ** -0.5))
+            kv_cache.shape[2], m["max_kvlen"], float(self.head_dim) ** -0.5, m["n_req"]))
         return out
 
     def _append(self, kv_cache, k, v, page, slot):
@@ -143,7 +143,7 @@ class FlashInferPrefillWrapper(_PagedBase):
         self._meta = dict(q_req=q_req.to(dev), q_kvlen=q_kvlen.to(dev), page=page32, slot=slot32,
                           indptr=paged_kv_indptr.to(device=dev, dtype=torch.int32),
                           indices=paged_kv_indices.to(device=dev, dtype=torch.int32),
-                          max_kvlen=int(kv_len.max()) if n_req else 1)
+                          max_kvlen=int(kv_len.max()) if n_req else 1, n_req=n_req)
 
     def run(self, q, kv_cache):
         return self._run(q, kv_cache)
@@ -181,7 +181,7 @@ class FlashInferDecodeWrapper(_PagedBase):
                           page=page_idx.to(device=dev, dtype=torch.int32), slot=pos_idx.to(device=dev, dtype=torch.int32),
                           indptr=paged_kv_indptr.to(device=dev, dtype=torch.int32),
                           indices=paged_kv_indices.to(device=dev, dtype=torch.int32),
-                          max_kvlen=int(kv_len.max()) if b else 1)
+                          max_kvlen=int(kv_len.max()) if b else 1, n_req=b)
 
     def run(self, q, kv_cache):
         return self._run(q, kv_cache)
