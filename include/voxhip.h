@@ -142,6 +142,11 @@ int vox_rep_update_mc(vox_ctx* ctx, void* stream, uint8_t* cache, const int32_t*
 int vox_sample(vox_ctx* ctx, void* stream, const void* logits, int B, int V, const vox_sampling_config* cfg,
                uint64_t seed, uint64_t offset, int32_t* out_ids);
 
+/* Which launch serves a linear (operands on 16 bytes), decided on the host.  rows 1 and 2, k = 1024, 2048, 3072, 4096: 0 a wave per column or two, 1 waves that
+ * walk the columns.  More than 128 rows of a stack's linear (split_k) or 32 of any other: 16 + the tile, 0 64 x 32, 1 64 x 64, 2 128 x 64, 3 128 x 128, 4 256 x 128 (rows x
+ * weight rows).  Else -1.  norm: a norm in front; glu: gate and up rows, n of each. */
+int vox_linear_form(int cus, int rows, int n, int k, int norm, int glu, int split_k);
+
 /* ---- decoder stack engine: replaces vox_serve/model/<family>.py decoder layers --------------------- */
 typedef struct {
     int32_t hidden, layers, heads, kv_heads, head_dim, ffn;

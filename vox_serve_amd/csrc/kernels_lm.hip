@@ -499,7 +499,7 @@ __global__ __launch_bounds__(256) void k_gemv(LinArgs a) {
 // and 500.  The same sums in the same order.  A step is a column, with EPI_SILU_MUL its gate row and its up row, from K = 3072 on (PAIR false) one after the other: both
 // at once beside the next ones do not fit the registers (52 us for 38).  Bound by memory (6.0 - 6.2 TB/s where there are many columns).  us, k_gemv and now: two rows: gate / up
 // 13696 x 4096 75.5, 38.2, 8192 x 2048 15.6, 13.5, 8192 x 1024 10.4, 8.8, 3072 x 1024 6.1, 5.6; head 168960 x 4096 365, 222; q | k | v 4608 x 4096 16.1, 11.5, 4096 x 1024 5.1, 4.4;
-// 1024 x 3072 4.2, 3.8; one row: 40.4, 36.6 (13696 x 4096), 11.0, 8.9 (4608 x 4096), 7.7, 7.4 (4096 x 4096), 233, 221 (head).
+// 1024 x 3072 4.2, 3.8; one row: 40.4, 36.6 (13696 x 4096), 11.0, 8.9 (4608 x 4096), 7.7, 7.4 (4096 x 4096), 233, 221 (head).  (Where: walk_pays.)
 template <int BT, int KC, int PRO, int EPI>
 __global__ __launch_bounds__(512, 2) void k_gemv_walk(LinArgs a) {
     touch_args(a);
@@ -617,37 +617,52 @@ __global__ __launch_bounds__(512, 2) void k_gemv_walk(LinArgs a) {
 #ifndef VOX_GEMV_COLS      // output columns per wave (development knob; 0 = heuristic)
 #define VOX_GEMV_COLS 0
 #endif
+// k_gemv_walk or k_gemv: the same sums, measured on 64 to 131072 columns (k_gemv's time = 1).  Fewer columns than the chip's waves leave nothing to walk (1.0 - 1.4).  From there on the walk
+// saves what k_gemv does per column, above all the norm: with one it takes 0.8 - 1.0 (two rows 0.5 - 1.0), but for narrow K (1024 and, one row, 2048) behind 16384 and 32768 weight rows,
+// where more loads in flight per CU count (1.03 - 1.08; two rows, gate and up: 0.9).  Two rows without a norm: 0.65 - 1.02 as well, at K = 1024 plain outputs 1.02 - 1.43, at K = 4096 1.02 - 1.2 where less than seven eighths of the waves have a column in every step (0.94 - 1.0 else).  One row without a norm: 1.0 - 1.12, but 0.94 - 1.0 where every wave
+// has one or two whole columns; gate and up together at K = 3072 0.95 - 1.01, elsewhere to 1.09.
+template <int BT, int KC, int PRO, int EPI>
+static bool walk_pays(int N, int cus) {
+    constexpr bool SM = EPI == EPI_SILU_MUL;
+    const int waves = 8 * cus;
+    if (N < waves) return false;
+    if (BT == 2 && PRO == PRO_COPY && !SM && KC == 8) {
+        const int per = (N + waves - 1) / waves;
+        return 8 * ((N + per - 1) / per) >= 7 * waves;
+    }
+    if (PRO == PRO_RMSNORM || (BT == 2 && (SM || KC > 2))) return KC >= 6 || (BT == 2 && (KC == 4 || (SM && PRO == PRO_RMSNORM))) || (SM ? 2 * N : N) <= 4 * KC * waves;
+    if (SM) return KC == 6;
+    return N <= 2 * waves && N % waves == 0;
+}
 template <int BT, int KC, int PRO, int EPI>
 static int launch_gemv_k(hipStream_t st, const LinArgs& a) {
     constexpr bool SM = (EPI == EPI_SILU_MUL);
     if constexpr (BT <= 2 && KC <= 8) {
-        if (a.row_tiles <= 1) {
+        if (a.row_tiles <= 1 && walk_pays<BT, KC, PRO, EPI>(a.N, a.cus)) {
             // as few steps as it takes with a block on every CU, and no more blocks than those steps need (K of more than 4096 does not fit the registers twice)
             const int per = (a.N + 8 * a.cus - 1) / (8 * a.cus);
             hipLaunchKernelGGL((k_gemv_walk<BT, KC, PRO, EPI>), dim3((a.N + 8 * per - 1) / (8 * per)), dim3(512), 0, st, a);
             return VOX_OK;
         }
     }
-    if constexpr (BT > 1 || KC > 8) {
-        // columns per wave: enough waves to cover the 1024 SIMDs a few times over, as many bytes in flight per wave
-        // as the register file allows (R*KC 16-byte loads per lane)
-        int cols = VOX_GEMV_COLS;
-        if (cols == 0) cols = (a.N / (SM ? 1 : 1) >= 4096 && KC <= 4) ? 2 : 1;
-        if (SM) cols = cols > 2 ? 2 : cols;
-        while (cols > 1 && cols * (SM ? 2 : 1) * KC > 24) cols >>= 1;
-        if (BT >= 4 && !SM && a.N >= 2048) cols = 2;          // share the unpacked activation pairs between two weight rows
-        if (BT >= 4) while (cols > 1 && cols * (SM ? 2 : 1) * KC > 8) cols >>= 1;
+    // columns per wave: enough waves to cover the 1024 SIMDs a few times over, as many bytes in flight per wave
+    // as the register file allows (R*KC 16-byte loads per lane)
+    int cols = VOX_GEMV_COLS;
+    if (cols == 0) cols = (a.N / (SM ? 1 : 1) >= 4096 && KC <= 4) ? 2 : 1;
+    if (SM) cols = cols > 2 ? 2 : cols;
+    while (cols > 1 && cols * (SM ? 2 : 1) * KC > 24) cols >>= 1;
+    if (BT >= 4 && !SM && a.N >= 2048) cols = 2;          // share the unpacked activation pairs between two weight rows
+    if (BT >= 4) while (cols > 1 && cols * (SM ? 2 : 1) * KC > 8) cols >>= 1;
 #define VOX_GV(C_)                                                                                       \
-        if (cols == C_) {                                                                                    \
-            const int gx = (a.N + 4 * C_ - 1) / (4 * C_);                                                    \
-            if (a.row_tiles > 1 && gx % 8) return vox_fail(VOX_ERR_INVALID, "gemv: row tiles need N/(4 cols) %% 8 == 0"); \
-            hipLaunchKernelGGL((k_gemv<BT, KC, (SM ? 2 * C_ : C_), PRO, EPI>), dim3(gx * (a.row_tiles > 1 ? a.row_tiles : 1)), \
-                               dim3(256), 0, st, a);                                                         \
-            return VOX_OK;                                                                                   \
-        }
-        VOX_GV(1) VOX_GV(2) VOX_GV(4)
-#undef VOX_GV
+    if (cols == C_) {                                                                                    \
+        const int gx = (a.N + 4 * C_ - 1) / (4 * C_);                                                    \
+        if (a.row_tiles > 1 && gx % 8) return vox_fail(VOX_ERR_INVALID, "gemv: row tiles need N/(4 cols) %% 8 == 0"); \
+        hipLaunchKernelGGL((k_gemv<BT, KC, (SM ? 2 * C_ : C_), PRO, EPI>), dim3(gx * (a.row_tiles > 1 ? a.row_tiles : 1)), \
+                           dim3(256), 0, st, a);                                                         \
+        return VOX_OK;                                                                                   \
     }
+    VOX_GV(1) VOX_GV(2) VOX_GV(4)
+#undef VOX_GV
     return vox_fail(VOX_ERR_INVALID, "gemv: no variant");
 }
 template <int PRO, int EPI>
@@ -2549,6 +2564,25 @@ int vox_launch_linear(vox_ctx* ctx, hipStream_t st, const LinearCall& call) {
     VOX_PE(PRO_RMSNORM, EPI_STORE) VOX_PE(PRO_RMSNORM, EPI_SILU_MUL) VOX_PE(PRO_ATTN, EPI_STORE)
 #undef VOX_PE
     return vox_fail(VOX_ERR_INVALID, "linear: unsupported prologue/epilogue combination");
+}
+
+template <int BT, int PRO, int EPI>
+static int gemv_form(int n, int k, int cus) {
+    switch (k) {
+    case 1024: return walk_pays<BT, 2, PRO, EPI>(n, cus);
+    case 2048: return walk_pays<BT, 4, PRO, EPI>(n, cus);
+    case 3072: return walk_pays<BT, 6, PRO, EPI>(n, cus);
+    case 4096: return walk_pays<BT, 8, PRO, EPI>(n, cus);
+    default: return -1;
+    }
+}
+extern "C" int vox_linear_form(int cus, int rows, int n, int k, int norm, int glu, int split_k) {
+    if (rows == 1) return norm ? (glu ? gemv_form<1, PRO_RMSNORM, EPI_SILU_MUL>(n, k, cus) : gemv_form<1, PRO_RMSNORM, EPI_STORE>(n, k, cus))
+                               : (glu ? gemv_form<1, PRO_COPY, EPI_SILU_MUL>(n, k, cus) : gemv_form<1, PRO_COPY, EPI_STORE>(n, k, cus));
+    if (rows == 2) return norm ? (glu ? gemv_form<2, PRO_RMSNORM, EPI_SILU_MUL>(n, k, cus) : gemv_form<2, PRO_RMSNORM, EPI_STORE>(n, k, cus))
+                               : (glu ? gemv_form<2, PRO_COPY, EPI_SILU_MUL>(n, k, cus) : gemv_form<2, PRO_COPY, EPI_STORE>(n, k, cus));
+    if (split_k) return rows > 128 && k % 64 == 0 ? 16 + pick_slab_tile(rows, glu ? 2 * n : n, k) : -1;
+    return rows > 32 && k % 128 == 0 && !glu && !norm ? 16 + pick_slab_tile(rows, n, k, 4) : -1;
 }
 
 // ================================================================================================
