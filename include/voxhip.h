@@ -146,6 +146,8 @@ int vox_sample(vox_ctx* ctx, void* stream, const void* logits, int B, int V, con
  * walk the columns.  More than 128 rows of a stack's linear (split_k) or 32 of any other: 16 + the tile, 0 64 x 32, 1 64 x 64, 2 128 x 64, 3 128 x 128, 4 256 x 128 (rows x
  * weight rows).  Else -1.  norm: a norm in front; glu: gate and up rows, n of each. */
 int vox_linear_form(int cus, int rows, int n, int k, int norm, int glu, int split_k);
+/* Which launch norms, turns and stores the heads of `rows` rows (q, k and v heads of a row in all; RoPE over whole heads in halves, or none): 0 a wave per head, 1 several heads a wave. */
+int vox_heads_form(int rows, int heads, int D, int norm);
 
 /* ---- decoder stack engine: replaces vox_serve/model/<family>.py decoder layers --------------------- */
 typedef struct {

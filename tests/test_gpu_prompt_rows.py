@@ -164,17 +164,20 @@ def test_linears_of_many_rows_against_portions(dev, rows, N, K, tile):  # noqa: 
         assert np.array_equal(*ys), (act, bias is not None, residual is not None)
 
 
-@pytest.mark.parametrize("heads,kvh,D,norm,bias", [(16, 8, 128, True, False), (3, 1, 128, False, True), (14, 2, 64, False, True), (32, 8, 64, True, False)])
-def test_heads_of_a_row_together(dev, heads, kvh, D, norm, bias):  # noqa: F811
+@pytest.mark.parametrize("heads,kvh,D,norm,bias,rows", [(16, 8, 128, True, False, 40), (3, 1, 128, False, True, 361), (14, 2, 64, False, True, 101), (32, 8, 64, True, False, 40),
+                                                        (32, 8, 64, False, False, 38)])
+def test_heads_of_a_row_together(dev, heads, kvh, D, norm, bias, rows):  # noqa: F811
     """k_head_rows against k_head_prepare, which takes RoPE tables that lie on no 16 bytes: hidden rows and cache bit for bit; heads that fill a block and that do not."""
-    rows, H, page = 40, 256, 32
+    from vox_serve_amd import _native as N
+    H, page = 256, 32
+    pages = list(np.random.default_rng(rows).permutation(-(-rows // page) + 1)[: -(-rows // page)])
+    assert N.lib().vox_heads_form(rows, heads + 2 * kvh, D, norm) == 1 and (norm or N.lib().vox_heads_form(20, heads + 2 * kvh, D, 0) == 0)
     x = T(vr.f2bf(np.random.default_rng(3).standard_normal((rows, H), dtype=np.float32)), dev)
     got = []
     for skew in (0, 2):
-        h, keep = stack(dev, H, heads, kvh, D, 512, rows, 64, page, 9, bias, norm, skew)
-        kv = torch.zeros(2, 3, 2, page, kvh, D, dtype=torch.bfloat16, device=dev)
-        got.append((Bits(forward(dev, h, x, kv, page, kvh, D, [rows], [2, 0])), Bits(kv)))
-        from vox_serve_amd import _native as N
+        h, keep = stack(dev, H, heads, kvh, D, 512, rows, page * len(pages), page, 9, bias, norm, skew)
+        kv = torch.zeros(2, len(pages) + 1, 2, page, kvh, D, dtype=torch.bfloat16, device=dev)
+        got.append((Bits(forward(dev, h, x, kv, page, kvh, D, [rows], pages)), Bits(kv)))
         N.lib().vox_stack_destroy(h)
     assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
     assert np.abs(vr.bf2f(got[0][1])).max() > 0.01

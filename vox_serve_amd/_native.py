@@ -86,6 +86,7 @@ _SIGS = {
     "vox_linear": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int,
                            c_int]),
     "vox_linear_form": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int]),
+    "vox_heads_form": (c_int, [c_int, c_int, c_int, c_int]),
     "vox_linear_silu_mul": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int]),
     "vox_suppress": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_void_p, c_int]),
     "vox_rep_penalty": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_float]),

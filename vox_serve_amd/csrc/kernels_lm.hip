@@ -2748,7 +2748,7 @@ __global__ __launch_bounds__(64) void k_head_prepare(HeadArgs a) {
 
 // The same for head dims 8 LPT = 64 and 128 whose RoPE, if there is one, pairs the halves of the whole head: LPT lanes hold a head, 256 / LPT heads of a row a block, and the
 // pairs meet by a DPP move (LPT = 16: row_ror:8 is lane ^ 8; LPT = 8: lane ^ 4), not in LDS.  Everything that does not turn on the position is asked for at once, so a launch is three trips to
-// memory and not six.  us, 32 heads of 128, before and now: 75 rows 4.7, 4.0, 640 8.7, 5.5; 20 rows 3.9, 3.8.
+// memory and not six.  us, 32 heads of 128, before and now: 75 rows 4.7, 4.0, 640 8.7, 5.5.
 template <int LPT>
 __global__ __launch_bounds__(256) void k_head_rows(HeadArgs a) {
     constexpr int D = 8 * LPT;
@@ -2801,6 +2801,11 @@ __global__ __launch_bounds__(256) void k_head_rows(HeadArgs a) {
     if (dst) reinterpret_cast<uint4*>(dst)[l] = make_uint4((u32)o[0] | ((u32)o[1] << 16), (u32)o[2] | ((u32)o[3] << 16), (u32)o[4] | ((u32)o[5] << 16), (u32)o[6] | ((u32)o[7] << 16));
 }
 
+// Few heads without norms are through sooner with a wave each, whose loads per lane are fewer.  us a launch, k_head_prepare and k_head_rows, heads in all: 14 + 2 of 64 (vox_rope) 8 rows
+// 2.13, 2.43, 75 (1200) 2.39, 2.52, 150 (2400) 2.71, 2.58; 16 + 8 of 128 32 rows (768) 2.19, 2.36, 48 (1152) 2.33, 2.36, 75 (1800) 2.52, 2.41, 300 3.90, 3.02; 32 + 8 of 64 24 rows (960)
+// 2.21, 2.50, 40 (1600) 2.42, 2.51, 64 (2560) 2.64, 2.53.  With norms k_head_rows is nowhere behind (1 to 600 rows).
+static bool head_rows_pay(int rows, int heads, bool norm) { return norm || (long)rows * heads >= 1800; }
+extern "C" int vox_heads_form(int rows, int heads, int D, int norm) { return (D == 64 || D == 128) && head_rows_pay(rows, heads, norm != 0); }
 int vox_launch_head_prepare(hipStream_t st, const HeadCall& c) {
     if (c.D % 8 || c.D > 512 || c.N <= 0) return c.N <= 0 ? VOX_OK : vox_fail(VOX_ERR_INVALID, "head_prepare: bad D");
     HeadArgs a{};
@@ -2811,7 +2816,7 @@ int vox_launch_head_prepare(hipStream_t st, const HeadCall& c) {
     a.slot = c.slot; a.eps = c.eps; a.Hq = c.Hq; a.Hkv = c.Hkv; a.D = c.D; a.rot = c.rot;
     a.interleave = c.interleave; a.page_size = c.page_size; a.table_max_pos = c.table_max_pos;
     const int heads = c.Hq + c.Hkv + (c.v_src ? c.Hkv : 0);
-    if ((c.D == 64 || c.D == 128) && (!c.cs || (c.rot == c.D && !c.interleave)) && ((size_t)c.cs & 15) == 0) {
+    if ((c.D == 64 || c.D == 128) && (!c.cs || (c.rot == c.D && !c.interleave)) && ((size_t)c.cs & 15) == 0 && head_rows_pay(c.N, heads, c.qn || c.kn)) {
         const int per = 2048 / c.D;
         if (c.D == 128) hipLaunchKernelGGL((k_head_rows<16>), dim3((heads + per - 1) / per, c.N), dim3(256), 0, st, a);
         else hipLaunchKernelGGL((k_head_rows<8>), dim3((heads + per - 1) / per, c.N), dim3(256), 0, st, a);
