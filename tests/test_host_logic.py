@@ -163,6 +163,15 @@ def test_attention_tiles_are_not_for_rows_of_different_requests(heads, kvh, D, p
     assert form(0, 1024, 8, heads, kvh, D, page, 128) == form(0, 1000, 4, heads, kvh, D, page, 250) == form(0, 900, 2, heads, kvh, D, page, 450) == 2
 
 
+# (heads, kv heads, D, rows, tokens of the call): one launch (1) or a block per chunk and a merge (0), the line on both sides
+@pytest.mark.parametrize("heads,kvh,D,rows,top,form", [(16, 8, 128, 32, 4096, 1), (16, 8, 128, 24, 4096, 1), (16, 8, 128, 23, 4096, 0), (16, 8, 128, 32, 4097, 0), (32, 2, 128, 1, 1024, 1),
+                                                       (32, 2, 128, 16, 1024, 1), (32, 2, 128, 17, 1024, 0), (32, 2, 128, 16, 1025, 0), (32, 2, 128, 64, 2048, 0), (32, 8, 64, 6, 1024, 1),
+                                                       (32, 8, 64, 5, 1024, 0)])
+def test_where_a_wave_takes_a_chunk_of_a_decode_row(heads, kvh, D, rows, top, form):
+    from vox_serve_amd import _native
+    assert ctypes.CDLL(_native.LIB_PATH).vox_attention_form(1, rows, rows, heads, kvh, D, 128, top) == form
+
+
 def test_product_never_imports_the_oracle():
     for dp, _, files in os.walk(os.path.join(ROOT, "vox_serve_amd")):
         for f in files:

@@ -214,13 +214,16 @@ __global__ __launch_bounds__(64 * NWV, PREP ? 1 : 4) void k_attn_decode(AttnArgs
 // k_attn_partial + merge (up to 512 tokens from 16 rows on k_attn_decode8) and this kernel, rows x tokens, Qwen3-TTS: 2 x 300 2799 / 2838, 4 x 300 3137 / 3092, 4 x 1000 3217 / 3317,
 // 8 x 600 3382 / 3231, 8 x 2000 3765 / 3818, 12 x 1400 3957 / 3607, 16 x 2000 4327 / 4137, 32 x 325 3749 / 3646, 32 x 600 4552 / 3822, 32 x 2000 5742 / 4766; CSM 4 x 1000 4335 / 4363,
 // 8 x 600 4490 / 4419, 16 x 1000 4701 / 4631; sixteen heads on a kv head (GLM-4-Voice), whose chunk blocks are long: 1 x 300 3897 / 3591, 1 x 1000 3954 / 3783, 8 x 1000 4261 / 4169.
+// LDS and the estimate go by the call's bound, which a graph's rows may be far below: a layer of 32 rows of Qwen3-TTS in calls of 2048 with 2000 / 1030 tokens 118 / 87, 106 / 65, of 4096 with 4000
+// / 2100 196 / 138, 151 / 93 (134 KB of LDS: a block to a CU); 24 rows of 4000 157 / 120, 12 of 1000 42 / 39, of 2000 58 / 54.  Sixteen heads: a chunk's K and V are fetched by eight blocks of two
+// heads here and by one there, which pays while no CU has two of them: a layer of 16 rows of 300 38.8 / 33.2, of 1000 46.2 / 46.1, 24 of 300 53.0 / 53.3, of 1000 69 / 78, 64 of 2000 157 / 208.
 static int decode_heads(const AttnCall& c) {
     const int G = c.Hkv > 0 ? c.Hq / c.Hkv : 0, nchunk = (c.max_kvlen + VOX_TC - 1) / VOX_TC;
     const size_t at = (size_t)c.qkv | (size_t)c.kv | (size_t)c.qn | (size_t)c.kn;
     if (!c.qkv || !c.out || c.identity_pages || c.fixed_kvlen > 0 || !c.page || !c.slot || c.Nq < 1 || c.Hq != G * c.Hkv || c.page_size % VOX_TC || nchunk <= 8 ||
         nchunk > 128 || (at & 15) || ((size_t)c.cs & 7)) return 0;
     if (!((c.D == 128 && (G == 2 || G == 16)) || (c.D == 64 && G == 4))) return 0;
-    if (2 * c.Nq * c.Hkv < 3 * nchunk && !(G == 16 && nchunk <= 32)) return 0;
+    if (G == 16 ? nchunk > 32 || c.Nq * c.Hkv > 32 : 2 * c.Nq * c.Hkv < 3 * nchunk) return 0;
     return c.Hq * c.Nq <= 256 ? 1 : 2;
 }
 bool vox_attn_decode_supported(const AttnCall& c) { return decode_heads(c) > 0; }
