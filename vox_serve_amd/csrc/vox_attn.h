@@ -120,18 +120,3 @@ __device__ __forceinline__ void prep_head(const bf16_t* src, const bf16_t* nw, f
     const PrepOps o = prep_head_load<D>(src, nw, cs_row, rot, lane);
     prep_head_apply<D>(o, nw, eps, cs_row, rot, interleave, sh, out, lane);
 }
-
-// exp2_c without its branches (for lanes with several of them, whose chains then run beside each other): the same value for every x
-__device__ __forceinline__ float exp2_flat(float x) {
-    const float n = __builtin_rintf(x), f = x - n;
-    float p = 1.52527338e-5f;
-    p = __fmaf_rn(p, f, 1.54035304e-4f);
-    p = __fmaf_rn(p, f, 1.33335581e-3f);
-    p = __fmaf_rn(p, f, 9.61812911e-3f);
-    p = __fmaf_rn(p, f, 5.55041087e-2f);
-    p = __fmaf_rn(p, f, 2.40226507e-1f);
-    p = __fmaf_rn(p, f, 6.93147181e-1f);
-    p = __fmaf_rn(p, f, 1.0f);
-    const float r = __uint_as_float(__float_as_uint(p) + ((u32)(int)n << 23));
-    return !(x > -125.0f) ? 0.0f : x >= 128.0f ? __uint_as_float(0x7f800000u) : r;
-}

@@ -118,9 +118,8 @@ __device__ __forceinline__ float butterfly(float s) {
 }
 #endif
 
-__device__ __forceinline__ float exp2_c(float x) {
-    if (!(x > -125.0f)) return 0.0f;
-    if (x >= 128.0f) return __uint_as_float(0x7f800000u);
+// 2^x for -125 < x < 128
+__device__ __forceinline__ float exp2_core(float x) {
     float n = __builtin_rintf(x);
     float f = x - n;
     float p = 1.52527338e-5f;
@@ -132,6 +131,16 @@ __device__ __forceinline__ float exp2_c(float x) {
     p = __fmaf_rn(p, f, 6.93147181e-1f);
     p = __fmaf_rn(p, f, 1.0f);
     return __uint_as_float(__float_as_uint(p) + (((u32)(int)n) << 23));
+}
+__device__ __forceinline__ float exp2_c(float x) {
+    if (!(x > -125.0f)) return 0.0f;
+    if (x >= 128.0f) return __uint_as_float(0x7f800000u);
+    return exp2_core(x);
+}
+// the same without branches (for lanes with several of them, whose chains then run beside each other)
+__device__ __forceinline__ float exp2_flat(float x) {
+    const float r = exp2_core(x);
+    return !(x > -125.0f) ? 0.0f : x >= 128.0f ? __uint_as_float(0x7f800000u) : r;
 }
 __device__ __forceinline__ float silu_c(float g) {
     float e = exp2_c((-g) * VOX_LOG2E);
