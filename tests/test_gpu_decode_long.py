@@ -19,10 +19,11 @@ LENS = [700, 1, 31, 32, 33, 257, 288, 289, 300, 511, 512, 513, 64, 95, 543, 544]
 @pytest.mark.parametrize("heads,kvh,D,rows,top,page", [(16, 8, 128, 16, 700, 32), (16, 8, 128, 17, 700, 96), (4, 2, 128, 40, 513, 128), (32, 8, 64, 8, 700, 64), (32, 8, 64, 9, 513, 32),
                                                        (32, 2, 128, 3, 700, 128), (32, 2, 128, 9, 1000, 32),
                                                        (16, 8, 128, 12, 1900, 128), (16, 8, 128, 24, 1900, 128), (16, 8, 128, 14, 2304, 96), (16, 8, 128, 24, 2304, 32), (16, 8, 128, 24, 4096, 128),
-                                                       (32, 8, 64, 8, 1300, 32), (32, 8, 64, 24, 4096, 128)])
+                                                       (32, 8, 64, 8, 1300, 32), (32, 8, 64, 24, 4096, 128), (16, 8, 128, 17, 512, 32), (32, 8, 64, 16, 480, 96)])
 def test_long_contexts_against_pages_of_sixteen(dev, heads, kvh, D, rows, top, page):  # noqa: F811
+    """(16 rows and more of up to 512 tokens in pages of 16: k_attn_decode8 with two chunks a group.)"""
     from vox_serve_amd import _native as N
-    assert [N.lib().vox_attention_form(1, rows, rows, heads, kvh, D, size, top) for size in (16, page)] == [0, 1]
+    assert [N.lib().vox_attention_form(1, rows, rows, heads, kvh, D, size, top) for size in (16, page)] == [3 if rows >= 16 and top <= 512 else 0, 1]
     H, F = 256, 512
     lens = [top] + [min(LENS[i % len(LENS)], top) for i in range(1, rows)]
     rng = np.random.default_rng(rows)

@@ -55,12 +55,18 @@ def forward(dev, h, x, kv, page, kvh, D, parts, pages):  # noqa: F811
 
 
 # K = 320: one 256-column sum and a quarter; 1088: four and a quarter; 704: two and three quarters.  Rows behind a tile of 64, 128 and 256, one row in the last tile.  The
-# wide ones reach the tiles of 128 and 256 rows.
-@pytest.mark.parametrize("rows,H,heads,kvh,D,F,bias", [(129, 320, 4, 2, 64, 704, True), (193, 320, 4, 2, 64, 704, False), (257, 1088, 4, 4, 128, 448, True), (300, 320, 2, 1, 64, 6208, False),
-                                                       (520, 320, 3, 1, 128, 12352, False), (1000, 1088, 2, 2, 64, 2112, True)])
-def test_prompt_in_one_portion_and_in_many(dev, rows, H, heads, kvh, D, F, bias):  # noqa: F811
+# tiles: those of q | k | v (a norm in front, bias), o (residual, the next norm behind), gate and up, down.
+@pytest.mark.parametrize("rows,H,heads,kvh,D,F,bias,tiles", [(129, 320, 4, 2, 64, 704, True, (0, 0, 0, 0)), (193, 320, 4, 2, 64, 704, False, (0, 0, 0, 0)), (257, 1088, 4, 4, 128, 448, True, (0, 0, 0, 0)),
+                                                             (300, 320, 2, 1, 64, 6208, False, (0, 0, 4, 0)), (520, 320, 3, 1, 128, 12352, False, (0, 0, 3, 0)),
+                                                             (1000, 1088, 2, 2, 64, 2112, True, (0, 2, 4, 2)), (233, 320, 33, 11, 64, 1088, True, (1, 0, 1, 0)),
+                                                             (233, 320, 33, 33, 64, 2112, True, (2, 0, 2, 0)), (233, 320, 33, 33, 128, 4160, True, (3, 0, 3, 0)),
+                                                             (450, 320, 33, 33, 128, 6208, True, (4, 0, 4, 0)), (450, 1088, 4, 2, 64, 448, False, (0, 1, 0, 1)),
+                                                             (1000, 2112, 4, 2, 64, 448, False, (0, 3, 1, 3))])
+def test_prompt_in_one_portion_and_in_many(dev, rows, H, heads, kvh, D, F, bias, tiles):  # noqa: F811
     """Portions of at most 100 rows take k_gemm_splitk (no width here is one of k_gemm_fullk's)."""
     from vox_serve_amd import _native as N
+    form = N.lib().vox_linear_form
+    assert tuple(form(256, rows, n, k, norm, glu, 1) - 16 for n, k, norm, glu in (((heads + 2 * kvh) * D, H, 1, 0), (H, heads * D, 0, 0), (F, H, 1, 1), (H, F, 0, 0))) == tiles
     page, n = 32, -(-rows // 32)
     rng = np.random.default_rng(rows)
     h, keep = stack(dev, H, heads, kvh, D, F, rows, n * page, page, rows, bias)
@@ -148,6 +154,7 @@ def test_linears_of_many_rows_against_portions(dev, rows, N, K, tile):  # noqa: 
     """vox_linear on all rows (k_gemm_slabs with four chains, every tile) and on portions of at most 24 (k_linear_mfma): ragged rows and columns, one k-tile pair to many, with and
     without SiLU, bias and residual."""
     from vox_serve_amd import _native as NV
+    assert NV.lib().vox_linear_form(256, rows, N, K, 0, 0, 0) == 16 + tile
     g = torch.Generator(device=dev).manual_seed(rows + tile)
     rnd = lambda *s: torch.randn(*s, generator=g, device=dev).bfloat16()
     W, b, x, res = rnd(N, K), rnd(N), rnd(rows, K), rnd(rows, N)

@@ -839,15 +839,17 @@ def test_decode_attention_for_257_to_512_tokens_is_bit_identical_to_partial_plus
     """Contexts of 257..512 visible tokens: the one-launch decode attention with two chunks per group (k_attn_decode8<.., NCH = 16>, the
     second tile in flight under the first chunk's arithmetic) against the chunked partial + merge launches it replaces — same chunk
     arithmetic, same merge order: ids, logits, fed-back features and the K/V cache identical over free-running eager frames that cross
-    page and chunk boundaries (ragged lengths per row)."""
+    page and chunk boundaries (ragged lengths per row).  Pages of 16 tokens: in pages of 128 several rows take k_attn_decode."""
+    from vox_serve_amd import _native as N
     from vox_serve_amd.engine import Qwen3Cfg, Qwen3Engine
     from vox_serve_amd.synth import synth_qwen3_weights
     cfg = Qwen3Cfg()
     W = synth_qwen3_weights(cfg, dev, seed=0)
-    ps, ppr = 128, 5
+    ps, ppr = 16, 40
     outs = []
     for on in ("0", "1"):      # 0: never, 1: from one row on
         monkeypatch.setenv("VOX_ATTN_DECODE16", on)
+        assert N.lib().vox_attention_form(1, B, B, 16, 8, 128, ps, 512) == (3 if on == "1" else 0)
         e = Qwen3Engine(cfg, W, max_batch=B, page_size=ps, max_pages=B * ppr + 1, max_seq_len=640, max_prefill_rows=64)
         e.keep_hidden = False
         g = torch.Generator(device=dev).manual_seed(9)

@@ -3136,7 +3136,7 @@ _Pragma("unroll") \
 template <int D, int GMAX, int NG, int NCH = 8>
 __global__ __launch_bounds__(1024) void k_attn_decode8(AttnArgs a) {
     touch_args(a);
-    // NCH = 16 (CPG = 2 chunks per group): contexts of up to 512 tokens — the second chunk's tile is requested when the first one has been
+    // NCH = 16 (CPG = 2 chunks per group): contexts of up to 512 tokens (where: decode16_min_rows) — the second chunk's tile is requested when the first one has been
     // parked, so its HBM latency runs under the first chunk's scores / softmax / P.V (one tile's registers at a time)
     constexpr int LPT = D / 8, TPW = 64 / LPT, GT = 1024 / NG, GW = GT / 64, CPG = NCH / NG;
     constexpr int KVL = (VOX_TC * LPT + GT - 1) / GT;
@@ -3543,8 +3543,8 @@ __global__ __launch_bounds__(1024) void k_attn_decode8_v1(AttnArgs a) {
 
 #endif
 
-// rows from which contexts of 257..512 tokens take the one-launch form (below: partial + merge — at one row 8 blocks running two
-// rounds lose to 88 chunk blocks: 2.79 vs 2.59 ms per frame; at 32 rows 4.09 vs 4.27).  VOX_ATTN_DECODE16 = 0 never, n = from n rows
+// rows from which contexts of 257..512 tokens that k_attn_decode does not take (pages that are no multiple of 32 tokens, a single kv head, operands on no 16 bytes) have the one-launch
+// form (below: partial + merge — at one row 8 blocks running two rounds lose to 88 chunk blocks: 2.79 vs 2.59 ms per frame; at 32 rows 4.09 vs 4.27, in pages of 128 before k_attn_decode).  VOX_ATTN_DECODE16 = 0 never, n = from n rows
 // (read per call — launches are captured into graphs, this is not a hot path — so that a test can A/B it)
 static int decode16_min_rows() {
     const char* e = getenv("VOX_ATTN_DECODE16");
