@@ -98,10 +98,10 @@ def test_mimi_does_not_depend_on_its_batch(dev, n, T):  # noqa: F811
     dec.close()
 
 
-@pytest.mark.parametrize("n", [1, 8, 9, 32, 33])
+@pytest.mark.parametrize("n", [1, 8, 9, 32, 33, 320, 321])
 def test_mimi_norm_and_linear_in_one_launch(dev, n):  # noqa: F811
     """Two transformer rows a request and frame: two rows, a whole tile of 16, two into the next, 64 (the last of the two-wave form), 66 (the
-    eight-wave form, two rows in its last tile).  The last request alone takes the two-wave form, bit for bit the same; against the oracle in
+    eight-wave form, two rows in its last tile), 640 (the last of it), 642 (two launches).  The last request alone takes the two-wave form, bit for bit the same; against the oracle in
     fp32 with the bar of the test above (relative 1e-5, fp32 rounding through eight layers: 2^-24 * sqrt(500 launches' roundings) = 1.3e-6)."""
     from oracle import mimi_ref as MR
     from vox_serve_amd.tokenizer.mimi import MimiConfig, MimiDecoder
@@ -112,8 +112,8 @@ def test_mimi_norm_and_linear_in_one_launch(dev, n):  # noqa: F811
     codes = torch.randint(0, cfg.bins, (n, cfg.n_q, 1), generator=torch.Generator().manual_seed(n))
     got = dec.decode(codes).cpu().clone()
     assert torch.equal(dec.decode(codes[-1:]).cpu()[0], got[-1])
-    ref = MR.MimiRef(cfg, W).decode(codes).numpy()
-    assert rms(ref) > 1e-4 and rms(got.numpy() - ref) < 1e-5 * max(1.0, rms(ref))
+    ref = MR.MimiRef(cfg, W).decode(codes[-33:]).numpy()
+    assert rms(ref) > 1e-4 and rms(got[-33:].numpy() - ref) < 1e-5 * max(1.0, rms(ref))
     dec.close()
 
 

@@ -2909,8 +2909,9 @@ static int ln_linear_launch(hipStream_t st, ConvDmaArgs& a, const float* x, cons
 template <int EPI>
 static int ln_linear(hipStream_t st, ConvDmaArgs& a, const float* x, const float* lw, const float* lb, float eps, float* buf) {
     const size_t at = (size_t)a.w | (size_t)x, at8 = (size_t)lw | (size_t)lb;
-    if (a.Cin == 512 && a.n_taps == 1 && !a.state && !a.job.state && a.N % 16 == 0 && a.sn_mod % 8 == 0 && a.bias_mod % 8 == 0 && (at & 15) == 0 && (at8 & 7) == 0) {
-        // Up to 64 rows two waves multiply (all eight norm): four times the CUs fetch the weights.  Mimi chunks, us, rows of the transformer, launch pairs / two / eight waves:
+    if (a.M <= 640 && a.Cin == 512 && a.n_taps == 1 && !a.state && !a.job.state && a.N % 16 == 0 && a.sn_mod % 8 == 0 && a.bias_mod % 8 == 0 && (at & 15) == 0 && (at8 & 7) == 0) {
+        // (More than 640 rows fill the chip with larger tiles, and these norm and fetch weights too often: launch pairs / eight waves 400 1078 / 1079, 640 1476 / 1466, 960 1935 / 1961,
+        // 1280 2465 / 2515.)  Up to 64 rows two waves multiply (all eight norm): four times the CUs fetch the weights.  Mimi chunks, us, rows of the transformer, launch pairs / two / eight waves:
         // 2 371 / 344 / 349, 20 429 / 396 / 408, 32 422 / 389 / 401, 64 460 / 423 / 433, 80 514 / 494 / 487, 128 529 / 523 / 497, 160 627 / 638 / 583, 320 916 / 983 / 877
         return a.M <= 64 ? ln_linear_launch<2, EPI>(st, a, x, lw, lb, eps) : ln_linear_launch<8, EPI>(st, a, x, lw, lb, eps);
     }
