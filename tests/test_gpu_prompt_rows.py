@@ -115,7 +115,7 @@ def prompt_case(seed, lens, ctx, page):
 @pytest.mark.parametrize("special", [False, True])
 @pytest.mark.parametrize("Hq,Hkv,D,page,lens,ctx", [(16, 8, 128, 128, [200], [0]), (16, 8, 128, 32, [1, 197, 3, 2, 260, 33], [0, 300, 31, 5, 7, 64]),
                                                     (32, 8, 64, 24, [330, 240, 5, 7], [11, 0, 90, 40]), (8, 8, 64, 24, [130, 5, 140], [11, 290, 0]), (18, 6, 128, 16, [170, 90], [100, 0]),
-                                                    (15, 5, 64, 8, [257], [0]), (12, 12, 64, 8, [257], [0]), (14, 2, 64, 16, [150, 60], [60, 9]), (32, 2, 128, 128, [70], [200]),
+                                                    (15, 5, 64, 8, [257], [0]), (12, 12, 64, 8, [257], [0]), (56, 8, 64, 16, [121, 90], [0, 9]), (32, 2, 128, 128, [70], [200]),
                                                     (32, 8, 64, 128, [290], [0]), (8, 8, 128, 128, [1031], [0])])
 def test_prompt_attention_against_single_rows(dev, Hq, Hkv, D, page, lens, ctx, special, form=2):  # noqa: F811
     """Several requests in a tile, tiles of 16, 8, 5 (a column of the 16 idle), 4, 2 (two idle) and 1 rows, ragged chunks, pages that no power of two divides, four and eight waves; with

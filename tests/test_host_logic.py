@@ -163,6 +163,14 @@ def test_attention_tiles_are_not_for_rows_of_different_requests(heads, kvh, D, p
     assert form(0, 1024, 8, heads, kvh, D, page, 128) == form(0, 1000, 4, heads, kvh, D, page, 250) == form(0, 900, 2, heads, kvh, D, page, 450) == 2
 
 
+@pytest.mark.parametrize("heads,kvh,D,rows,top,form", [(14, 2, 64, 30, 230, 0), (14, 2, 64, 48, 148, 0), (14, 2, 64, 300, 300, 2), (24, 8, 64, 16, 216, 0), (8, 8, 64, 30, 130, 0),
+                                                       (24, 8, 128, 96, 96, 2), (24, 8, 128, 30, 130, 0), (32, 2, 128, 70, 270, 2)])
+def test_attention_tiles_of_few_rows(heads, kvh, D, rows, top, form):
+    """One request's rows that end at `top` tokens: tiles only where their one round of chunks is the faster launch (measured 1.1 to 1.4 times at these sizes)."""
+    from vox_serve_amd import _native
+    assert ctypes.CDLL(_native.LIB_PATH).vox_attention_form(0, rows, 1, heads, kvh, D, 128, top) == form
+
+
 # (heads, kv heads, D, rows, tokens of the call): one launch (1) or a block per chunk and a merge (0), the line on both sides
 @pytest.mark.parametrize("heads,kvh,D,rows,top,form", [(16, 8, 128, 32, 4096, 1), (16, 8, 128, 24, 4096, 1), (16, 8, 128, 23, 4096, 0), (16, 8, 128, 32, 4097, 0), (32, 2, 128, 1, 1024, 1),
                                                        (32, 2, 128, 16, 1024, 1), (32, 2, 128, 17, 1024, 0), (32, 2, 128, 16, 1025, 0), (32, 2, 128, 64, 2048, 0), (32, 8, 64, 6, 1024, 1),

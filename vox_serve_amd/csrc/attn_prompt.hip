@@ -312,16 +312,17 @@ float vox_attn_seen(const AttnCall& c, int nchunk) {      // (a prompt's rows al
     return own < 0.5f ? 1.0f - own : 0.5f;
 }
 static bool four_waves(const AttnCall& c) { return prompt_blocks(c) > (c.D == 64 ? 256 : 512); }
-// What k_attn_partial and k_attn_merge take and what this kernel takes, us, fitted to 2 to 1000 rows behind 0 to 3000 tokens, 2 and 8 kv heads of 2, 4 and 16 q heads.  The
-// former by blocks (row, kv head, chunk; a prompt's rows see half of it), the latter by rounds of eight chunks, of which a tile's block goes through one after the other
-// while the chip may be idle.  A tile takes its rows' requests one after the other: at most as many as it has rows, and since no request has more rows than the call
+// What k_attn_partial and k_attn_merge take and what this kernel takes, us, fitted to 2 to 1000 rows behind 0 to 1500 tokens, 1 to 8 kv heads of 1 to 16 q heads.  The
+// former by blocks (row, kv head, chunk; a prompt's rows see half of it), the latter by rounds of eight chunks (a last one of up to four is shorter), of which a tile's block goes
+// through one after the other while the chip may be idle.  A tile takes its rows' requests one after the other: at most as many as it has rows, and since no request has more rows than the call
 // has tokens, at most two beyond those that the call's rows leave over.  Measured, former / latter: 16 heads on 8, D = 128, no context: 64 rows 8.6 / 10.8, 96 12.0 / 11.0; behind 1500 tokens: 2 rows 12 / 59,
-// 32 48 / 60, 64 84 / 65, 128 152 / 67; 32 heads on 8, D = 64, behind 700: 16 rows 17 / 24, 48 35 / 25; 32 heads on 2: 48 rows 14.0 / 9.5, behind 1500: 32 48 / 60, 64 81 / 65.
+// 32 48 / 60, 64 84 / 65, 128 152 / 67; 32 heads on 8, D = 64, behind 700: 16 rows 17 / 24, 48 35 / 25; 32 heads on 2: 48 rows 14.0 / 9.5, behind 1500: 32 48 / 60, 64 81 / 65; 14 on 2, D = 64, behind 200:
+// 30 rows 8.6 / 11.4, 128 17.1 / 15.8; 24 on 8, D = 128: 96 rows 13.4 / 11.4.
 // One row a request (one per tile and pass), 16 heads on 8, D = 128: 64 rows of 1500 tokens 115 / 516, 128 of 600 93 / 234; 32 heads on 8, D = 64: 128 of 600 71 / 93; 32 heads on 2 (a row
 // a tile) 65 / 37.  16 heads on 8: a prompt of 75 rows beside 31 of one row behind 300 tokens 25 / 149, eight prompts of 128 rows 105 / 28, four of 250 189 / 44.
 void vox_attn_prompt_us(const AttnCall& c, int nchunk, float& parts, float& prompt) {
     const float G = (float)(c.Hq / c.Hkv), seen = vox_attn_seen(c, nchunk);
-    parts = 7.3f + 0.35f * G * c.D / 128 + (float)c.Nq * c.Hkv * nchunk * seen * (0.0018f + 0.0000038f * G * c.D);
+    parts = 6.3f + 0.3f * G * c.D / 128 + (float)c.Nq * c.Hkv * nchunk * seen * (0.00195f + 0.0000053f * G * c.D);
     const int req = requests(c), rows = 16 / (c.Hq / c.Hkv), tiles = (c.Nq + rows - 1) / rows;
     int passes = 1;
     if (req > 1) {
@@ -330,9 +331,11 @@ void vox_attn_prompt_us(const AttnCall& c, int nchunk, float& parts, float& prom
         if (passes > rows) passes = rows;
         if (passes > req) passes = req;
     }
-    const int round = passes > 1 && four_waves(c) ? 4 : 8;
-    const float longest = (float)passes * ((nchunk + round - 1) / round), all = (float)c.Hkv * (tiles + req - 1) * seen * nchunk / 2048.0f;
-    prompt = 3.0f + (4.0f + 0.04f * c.D) * (longest > all ? longest : all);
+    const bool four = passes > 1 && four_waves(c);
+    const float round = c.D == 64 ? 6.8f : 9.5f, half = c.D == 64 ? 2.1f : 3.2f;
+    const float pass = four ? round * ((nchunk + 3) / 4) : round * ((nchunk + 7) / 8) - ((nchunk - 1) % 8 < 4 ? half : 0.0f);
+    const float longest = passes * pass, all = round * c.Hkv * (tiles + req - 1) * seen * nchunk / 2048.0f;
+    prompt = 4.7f + (longest > all ? longest : all);
 }
 static bool prompt_pays(const AttnCall& c, int nchunk) {
     float parts, prompt;
